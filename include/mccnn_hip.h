@@ -141,6 +141,37 @@ int mccnn_gather_i32(mccnn_stream_t stream, int64_t count, const int32_t *src,
 int mccnn_gather_rows(mccnn_stream_t stream, int64_t num_rows, int num_cols, const float *src,
                       const int32_t *indices, float *out);
 
+/* out[i, c] = src[rows[i] * src_stride + first_col + c] for c < num_cols and 0 for num_cols <=
+ * c < num_cols_out (rows NULL: row i): rows of features or gradients brought into another
+ * order and padded to a channel count of the layer kernels. */
+int mccnn_gather_rows_padded(mccnn_stream_t stream, int64_t num_rows, const int32_t *rows,
+                             const float *src, int64_t src_stride, int first_col, int num_cols,
+                             int num_cols_out, float *out);
+
+/* The weights of a convolution layer as its kernels read them, one launch: from the final
+ * weights [L, num_features * hidden, group_features] (MCConv.py:180-187; L = 1 for
+ * kernel-point convolutions) the kernel MLPs first_mlp .. first_mlp + num_mlps - 1 as a dense
+ * matrix over padded sizes, zero outside the diagonal blocks, with c < padded_features, k <
+ * num_mlps * padded_hidden, f < num_mlps * padded_group: w [(c,k), f], wt [f, (c,k)],
+ * w2 [(f,k), c], w2t [c, (f,k)] (each NULL to skip), and from kernel_weights [L, D, hidden],
+ * kernel_biases [L * hidden] the padded [num_mlps, D, padded_hidden] and its biases (NULL to
+ * skip).  _unpack_: the gradients of the same parameters back in the caller's shapes, from
+ * dense_grads [padded_features, (f,k)] and the padded kernel gradients (NULL to skip either).
+ * No counterpart among the reference's ops. */
+int mccnn_pack_layer_weights(mccnn_stream_t stream, int num_dims, int num_features, int hidden,
+                             int group_features, int first_mlp, int num_mlps,
+                             int padded_features, int padded_hidden, int padded_group,
+                             const float *final_weights, const float *kernel_weights,
+                             const float *kernel_biases, float *w_out, float *wt_out,
+                             float *w2_out, float *w2t_out, float *kernel_weights_out,
+                             float *kernel_biases_out);
+int mccnn_unpack_layer_grads(mccnn_stream_t stream, int num_dims, int num_features, int hidden,
+                             int group_features, int first_mlp, int num_mlps,
+                             int padded_features, int padded_hidden, int padded_group,
+                             const float *dense_grads, const float *kernel_weight_grads,
+                             const float *kernel_bias_grads, float *final_grads_out,
+                             float *weight_grads_out, float *bias_grads_out);
+
 /* BuildGridDs: build_grid_ds/cc/ops/build_grid_ds_ops.cpp:27-115.
  * ds_out is int32 [batch_size, num_cells[0], num_cells[1], 2]: (first, last+1)
  * index of each column in the sorted arrays, (0,0) when empty.  num_cells is

@@ -4,7 +4,6 @@ built, or a tensor is not a contiguous GPU tensor of the right dtype, the call
 raises."""
 import ctypes
 import os
-import threading
 import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -13,6 +12,7 @@ LIB_PATH = os.environ.get("MCCNN_HIP_LIBRARY") or os.path.join(_HERE, "libmccnn_
 CSRC_DIR = os.path.join(_HERE, "csrc")
 
 _lib = None
+_host = None
 
 i64 = ctypes.c_int64
 cint = ctypes.c_int
@@ -41,7 +41,8 @@ def lib():
             raise RuntimeError(
                 "libmccnn_hip.so is not built (expected at %s); run "
                 "`make -C %s` or __graft_entry__.build()" % (LIB_PATH, CSRC_DIR))
-        handle = ctypes.CDLL(LIB_PATH)
+        # global symbols: the host extension (_host.so) resolves the C ABI against this library
+        handle = ctypes.CDLL(LIB_PATH, mode=ctypes.RTLD_GLOBAL)
         handle.mccnn_last_error.restype = ctypes.c_char_p
         for name in ("mccnn_build_grid_workspace_bytes",
                      "mccnn_find_neighbors_workspace_bytes",
@@ -57,6 +58,22 @@ def lib():
             getattr(handle, name).restype = csize
         _lib = handle
     return _lib
+
+
+def host():
+    """The host extension (csrc/host.cpp): sequences of C-ABI calls issued from C++."""
+    global _host
+    if _host is None:
+        import torch  # noqa: F401  (the extension links against torch's libraries)
+        lib()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError("_host.so is not built; run `make -C %s` or "
+                               "__graft_entry__.build()" % CSRC_DIR) from e
+        module.set_error_class(InvalidArgumentError)
+        _host = module
+    return _host
 
 
 def check(rc):
@@ -90,23 +107,6 @@ def ptr(t, dtype=None):
     return vptr(t.data_ptr())
 
 
-_host_counts = threading.local()
-
-
-def host_count():
-    """One int64 in pinned host memory per thread: the `_count` halves of the
-    dynamic-size ops copy their total there, and a device-to-host copy into pinned
-    memory completes without the staging a pageable destination needs.
-    -> (tensor [1], pointer)."""
-    import torch
-    t = getattr(_host_counts, "tensor", None)
-    if t is None:
-        # [0] the count; [1], [2] the two facts mccnn_find_neighbors_count_facts reports
-        t = torch.zeros(4, dtype=torch.int64, pin_memory=True)
-        _host_counts.tensor = t
-    return t, vptr(t.data_ptr())
-
-
 def workspace(nbytes, device):
     import torch
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
@@ -124,6 +124,7 @@ _timing = None
 def start_timing():
     global _timing
     _timing = {}
+    host().start_timing()
 
 
 class region:
@@ -150,6 +151,8 @@ def collect_timing():
     import torch
     torch.cuda.synchronize()
     out = {k: [a.elapsed_time(b) for a, b in v] for k, v in (_timing or {}).items()}
+    for name, ms in host().collect_timing():
+        out.setdefault(name, []).append(ms)
     _timing = None
     return out
 

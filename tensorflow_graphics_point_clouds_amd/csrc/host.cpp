@@ -1,0 +1,974 @@
+// Host path of the layers and of the point-cloud structures: the sequences of C-ABI calls
+// that make up a grid, a neighbour search or a layer pass, issued from C++ on tensors.
+//
+// A pass over a few thousand points is bound by what happens between the kernels: with every
+// C-ABI call made through ctypes (6 to 8 us each with its argument objects) and every
+// intermediate tensor, pad and permutation made in Python, a forward call on 2 x 1024 points
+// took 375 us for 109 us of kernels.  The functions here allocate with the caching allocator,
+// run on the current stream of the current device, release the interpreter lock, and keep no
+// state between calls but a pool of pinned 256-byte blocks (as many as threads were ever
+// waiting for a device count at the same time).
+#include <torch/extension.h>
+
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime.h>
+
+#include <mutex>
+#include <utility>
+#include <vector>
+
+#include "../../include/mccnn_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// ------------------------------------------------------------------ errors, pointers ----
+
+struct InvalidArgument : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
+void check(int rc) {
+  if (rc == MCCNN_OK) return;
+  const std::string msg = mccnn_last_error();
+  if (rc == MCCNN_INVALID_ARGUMENT) throw InvalidArgument(msg);
+  throw std::runtime_error("HIP error in libmccnn_hip: " + msg);
+}
+
+void hip_check(hipError_t e) {
+  if (e != hipSuccess) throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e));
+}
+
+void *raw(const Tensor &t, at::ScalarType type) {
+  if (!t.defined()) return nullptr;
+  TORCH_CHECK_TYPE(t.is_cuda(), "expected a GPU tensor, got one on ", t.device());
+  TORCH_CHECK_TYPE(t.scalar_type() == type, "expected dtype ", type, ", got ", t.scalar_type());
+  TORCH_CHECK_TYPE(t.is_contiguous(), "expected a contiguous tensor");
+  return t.data_ptr();
+}
+float *f32(const Tensor &t) { return static_cast<float *>(raw(t, at::kFloat)); }
+int32_t *i32(const Tensor &t) { return static_cast<int32_t *>(raw(t, at::kInt)); }
+int64_t *i64(const Tensor &t) { return static_cast<int64_t *>(raw(t, at::kLong)); }
+Tensor opt(const OptTensor &t) { return t.has_value() ? *t : Tensor(); }
+
+hipStream_t current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+Tensor empty_f32(at::IntArrayRef sizes, const Tensor &like) {
+  return at::empty(sizes, like.options().dtype(at::kFloat).requires_grad(false));
+}
+Tensor empty_i32(at::IntArrayRef sizes, const Tensor &like) {
+  return at::empty(sizes, like.options().dtype(at::kInt).requires_grad(false));
+}
+Tensor empty_i64(at::IntArrayRef sizes, const Tensor &like) {
+  return at::empty(sizes, like.options().dtype(at::kLong).requires_grad(false));
+}
+Tensor workspace(size_t bytes, const Tensor &like) {
+  return at::empty({(int64_t)(bytes ? bytes : 1)},
+                   like.options().dtype(at::kByte).requires_grad(false));
+}
+
+int64_t dim(const Tensor &t, int64_t axis) { return t.dim() > axis ? t.size(axis) : -1; }
+
+int compute_units() {
+  static thread_local int device = -1, cus = 0;
+  int d = 0;
+  hip_check(hipGetDevice(&d));
+  if (d != device) {
+    hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, d));
+    device = d;
+  }
+  return cus;
+}
+
+// A block of pinned host memory for the counts a call waits for, taken from a pool.
+class PinnedBlock {
+ public:
+  PinnedBlock() {
+    {
+      std::lock_guard<std::mutex> lock(mutex());
+      if (!pool().empty()) {
+        p_ = pool().back();
+        pool().pop_back();
+      }
+    }
+    if (!p_) hip_check(hipHostMalloc(&p_, 256, hipHostMallocDefault));
+  }
+  ~PinnedBlock() {
+    std::lock_guard<std::mutex> lock(mutex());
+    pool().push_back(p_);
+  }
+  PinnedBlock(const PinnedBlock &) = delete;
+  int64_t *words() { return static_cast<int64_t *>(p_); }
+  int32_t *ints() { return static_cast<int32_t *>(p_); }
+
+ private:
+  static std::mutex &mutex() { static std::mutex *m = new std::mutex; return *m; }
+  static std::vector<void *> &pool() { static auto *v = new std::vector<void *>; return *v; }
+  void *p_ = nullptr;
+};
+
+// ------------------------------------------------------------------------- timing ----
+// The counterpart of the regions of _lib.py for the calls made here: a pair of events
+// around every call while timing is on.
+
+struct TimedCall {
+  const char *name;
+  hipEvent_t start, end;
+};
+std::mutex g_timing_mutex;
+std::atomic<bool> g_timing{false};
+std::vector<TimedCall> g_timed;
+
+class Region {
+ public:
+  Region(const char *name, hipStream_t s) : on_(g_timing.load(std::memory_order_relaxed)), s_(s) {
+    if (!on_) return;
+    c_.name = name;
+    hip_check(hipEventCreate(&c_.start));
+    hip_check(hipEventCreate(&c_.end));
+    hip_check(hipEventRecord(c_.start, s_));
+  }
+  ~Region() {
+    if (!on_) return;
+    (void)hipEventRecord(c_.end, s_);
+    std::lock_guard<std::mutex> lock(g_timing_mutex);
+    g_timed.push_back(c_);
+  }
+
+ private:
+  bool on_;
+  hipStream_t s_;
+  TimedCall c_{};
+};
+
+void start_timing() {
+  std::lock_guard<std::mutex> lock(g_timing_mutex);
+  g_timed.clear();
+  g_timing = true;
+}
+
+std::vector<std::pair<std::string, double>> collect_timing() {
+  g_timing = false;
+  hip_check(hipDeviceSynchronize());
+  std::vector<std::pair<std::string, double>> out;
+  std::lock_guard<std::mutex> lock(g_timing_mutex);
+  for (auto &c : g_timed) {
+    float ms = 0.0f;
+    hip_check(hipEventElapsedTime(&ms, c.start, c.end));
+    out.emplace_back(c.name, ms);
+    (void)hipEventDestroy(c.start);
+    (void)hipEventDestroy(c.end);
+  }
+  g_timed.clear();
+  return out;
+}
+
+// --------------------------------------------------------------------------- grid ----
+
+Tensor compute_keys(const Tensor &points, const Tensor &bids, const Tensor &smin,
+                    const Tensor &num_cells, const Tensor &inv_cell) {
+  Tensor keys = empty_i64({points.size(0)}, points);
+  hipStream_t s = current_stream();
+  Region r("compute_keys", s);
+  check(mccnn_compute_keys(s, points.size(0), (int)dim(points, 1), f32(points), bids.size(0),
+                           i32(bids), smin.size(0), (int)dim(smin, 1), f32(smin),
+                           (int)num_cells.size(0), i32(num_cells), (int)inv_cell.size(0),
+                           f32(inv_cell), i64(keys)));
+  return keys;
+}
+
+std::pair<Tensor, Tensor> sort_keys(const Tensor &keys, int64_t bits) {
+  const int64_t n = keys.size(0);
+  Tensor sorted = empty_i64({n}, keys), order = empty_i32({n}, keys);
+  Tensor ws = workspace(mccnn_sort_keys_workspace_bytes(n), keys);
+  hipStream_t s = current_stream();
+  Region r("sort_keys_descending", s);
+  check(mccnn_sort_keys_descending(s, n, (int)bits, i64(keys), i64(sorted), i32(order),
+                                   ws.data_ptr(), ws.numel()));
+  return {sorted, order};
+}
+
+struct GridTensors {
+  Tensor aabb_min, aabb_max, num_cells, smin, inv_cell, keys, sorted_keys, sorted_indices,
+      sorted_points, sorted_bids;
+  std::vector<int64_t> cells_host;
+  int64_t key_bits = 0;
+};
+
+// The grid of a point cloud (pylib/pc/Grid.py:32-84).
+GridTensors build_grid(const Tensor &points, const Tensor &bids, int64_t batch,
+                       const Tensor &cell_sizes) {
+  const int64_t n = points.size(0), d = points.size(1);
+  GridTensors g;
+  g.aabb_min = empty_f32({batch, d}, points);
+  g.aabb_max = empty_f32({batch, d}, points);
+  g.num_cells = empty_i32({d}, points);
+  g.smin = empty_f32({batch, d}, points);
+  g.inv_cell = empty_f32({d}, points);
+  g.keys = empty_i64({n}, points);
+  g.sorted_keys = empty_i64({n}, points);
+  g.sorted_indices = empty_i32({n}, points);
+  g.sorted_points = empty_f32({n, d}, points);
+  g.sorted_bids = empty_i32({n}, points);
+  Tensor ws = workspace(mccnn_build_grid_workspace_bytes(n), points);
+  hipStream_t s = current_stream();
+  PinnedBlock host;
+  int bits = 1;
+  Region r("build_grid", s);
+  check(mccnn_build_grid(s, n, (int)d, f32(points), i32(bids), (int)batch, f32(cell_sizes),
+                         f32(g.aabb_min), f32(g.aabb_max), i32(g.num_cells), f32(g.smin),
+                         f32(g.inv_cell), i64(g.keys), i64(g.sorted_keys), i32(g.sorted_indices),
+                         f32(g.sorted_points), i32(g.sorted_bids), ws.data_ptr(), ws.numel(),
+                         host.ints(), &bits));
+  for (int64_t i = 0; i < d; ++i) g.cells_host.push_back(host.ints()[i]);
+  g.key_bits = bits;
+  return g;
+}
+
+Tensor build_grid_ds(const Tensor &sorted_keys, const Tensor &num_cells,
+                     const std::vector<int32_t> &host, int64_t batch) {
+  if (batch <= 0) throw InvalidArgument("BuildGridDs requires a positive batch size");
+  if (host.size() < 2) throw InvalidArgument("BuildGridDs expects a valid number of dimensions");
+  hipStream_t s = current_stream();
+  Tensor ds = empty_i32({batch, std::max(host[0], 0), std::max(host[1], 0), 2}, sorted_keys);
+  Region r("build_grid_ds", s);
+  check(mccnn_build_grid_ds(s, sorted_keys.size(0), i64(sorted_keys), (int)num_cells.size(0),
+                            i32(num_cells), (int)host.size(), host.data(), (int)batch, i32(ds)));
+  return ds;
+}
+
+// ---------------------------------------------------------------------- neighbours ----
+
+// -> (ranges, neighbors, whether the table is an untruncated self-neighbourhood)
+std::tuple<Tensor, Tensor, bool> find_neighbors(const Tensor &samples, const Tensor &sbids,
+                                                const Tensor &points, const Tensor &keys,
+                                                const Tensor &ds, const Tensor &num_cells,
+                                                const Tensor &smin, const Tensor &inv_cell,
+                                                const Tensor &inv_radii, int64_t max_neighs) {
+  const int64_t ns = samples.size(0);
+  const int nd = (int)dim(samples, 1);
+  Tensor ws = workspace(mccnn_find_neighbors_workspace_bytes(nd, ns), samples);
+  Tensor ranges = empty_i32({ns}, samples);
+  hipStream_t s = current_stream();
+  PinnedBlock host;
+  int64_t *total = host.words();
+  total[0] = total[1] = total[2] = 0;
+  {
+    Region r("find_neighbors_count", s);
+    check(mccnn_find_neighbors_count_facts(
+        s, ns, nd, f32(samples), sbids.size(0), i32(sbids), points.size(0), (int)dim(points, 1),
+        f32(points), keys.size(0), i64(keys), (int)ds.dim(), (int)dim(ds, 0), (int)dim(ds, 1),
+        (int)dim(ds, 2), (int)dim(ds, 3), i32(ds), (int)num_cells.size(0), i32(num_cells),
+        (int)dim(smin, 1), f32(smin), (int)inv_cell.size(0), f32(inv_cell),
+        (int)inv_radii.size(0), f32(inv_radii), (int)max_neighs, ws.data_ptr(), ws.numel(),
+        i32(ranges), total, total + 1));
+  }
+  const int64_t m = total[0];
+  const bool symmetric = total[1] == 0 && total[2] == 1;
+  Tensor neighbors = empty_i32({m, 2}, samples);
+  Region r("find_neighbors_fill", s);
+  check(mccnn_find_neighbors_fill(s, ns, nd, f32(samples), i32(sbids), points.size(0), f32(points),
+                                  i64(keys), i32(ds), i32(num_cells), f32(smin), f32(inv_cell),
+                                  f32(inv_radii), (int)max_neighs, ws.data_ptr(), ws.numel(),
+                                  i32(ranges), m, i32(neighbors)));
+  return {ranges, neighbors, symmetric};
+}
+
+// The pair table regrouped for centres in the order `order` -> (ranges, neighbors).
+std::pair<Tensor, Tensor> reorder_neighbors(const Tensor &ranges, const Tensor &neighbors,
+                                            const Tensor &order) {
+  const int64_t n = ranges.size(0);
+  Tensor ws = workspace(mccnn_reorder_neighbors_workspace_bytes(n), neighbors);
+  Tensor ranges_out = empty_i32({n}, ranges), out = empty_i32(neighbors.sizes(), neighbors);
+  hipStream_t s = current_stream();
+  Region r("reorder_neighbors", s);
+  check(mccnn_reorder_neighbors(s, n, i32(ranges), neighbors.size(0), i32(neighbors), i32(order),
+                                ws.data_ptr(), ws.numel(), i32(ranges_out), i32(out)));
+  return {ranges_out, out};
+}
+
+Tensor original_neighbor_ids(const Tensor &neighbors, const Tensor &sorted_indices) {
+  Tensor out = empty_i32(neighbors.sizes(), neighbors);
+  hipStream_t s = current_stream();
+  Region r("original_neighbor_ids", s);
+  check(mccnn_original_neighbor_ids(s, neighbors.size(0), i32(neighbors), i32(sorted_indices),
+                                    i32(out)));
+  return out;
+}
+
+// -> (point_ranges, pair_order)
+std::pair<Tensor, Tensor> transpose_neighbors(const Tensor &neighbors, int64_t num_pts) {
+  const int64_t m = neighbors.size(0);
+  Tensor ws = workspace(mccnn_transpose_neighbors_workspace_bytes(m, num_pts), neighbors);
+  Tensor ranges = empty_i32({num_pts}, neighbors), order = empty_i32({m}, neighbors);
+  hipStream_t s = current_stream();
+  Region r("transpose_neighbors", s);
+  check(mccnn_transpose_neighbors(s, m, i32(neighbors), num_pts, ws.data_ptr(), ws.numel(),
+                                  i32(ranges), i32(order)));
+  return {ranges, order};
+}
+
+Tensor swapped_pairs(const Tensor &neighbors, const Tensor &order) {
+  Tensor out = empty_i32(neighbors.sizes(), neighbors);
+  hipStream_t s = current_stream();
+  Region r("swapped_pairs", s);
+  check(mccnn_swapped_pairs(s, neighbors.size(0), i32(neighbors), i32(order), i32(out)));
+  return out;
+}
+
+Tensor gather_pdf(const Tensor &neighbors, int64_t column, const Tensor &pdf) {
+  Tensor out = empty_f32({neighbors.size(0)}, neighbors);
+  hipStream_t s = current_stream();
+  Region r("gather_pdf", s);
+  check(mccnn_gather_pdf_column(s, neighbors.size(0), i32(neighbors), (int)column, f32(pdf),
+                                f32(out)));
+  return out;
+}
+
+Tensor gather_i32(const Tensor &src, const Tensor &indices) {
+  Tensor out = empty_i32({indices.size(0)}, indices);
+  hipStream_t s = current_stream();
+  Region r("gather_i32", s);
+  check(mccnn_gather_i32(s, indices.size(0), i32(src), i32(indices), i32(out)));
+  return out;
+}
+
+Tensor compute_pdf(const Tensor &points, const Tensor &neighbors, const Tensor &ranges,
+                   const Tensor &inv_bandwidth, const Tensor &inv_radii, int64_t mode) {
+  Tensor pdf = empty_f32({ranges.size(0)}, points);
+  hipStream_t s = current_stream();
+  Region r("compute_pdf", s);
+  check(mccnn_compute_pdf(s, points.size(0), (int)dim(points, 1), f32(points), neighbors.size(0),
+                          (int)neighbors.dim(), (int)dim(neighbors, 1), i32(neighbors),
+                          ranges.size(0), i32(ranges), (int)inv_bandwidth.size(0),
+                          f32(inv_bandwidth), (int)inv_radii.size(0), f32(inv_radii), (int)mode,
+                          f32(pdf)));
+  return pdf;
+}
+
+// -> (points, batch ids, indices)
+std::tuple<Tensor, Tensor, Tensor> sampling(const Tensor &points, const Tensor &bids,
+                                            const Tensor &keys, const Tensor &num_cells,
+                                            const Tensor &neighbors, const Tensor &ranges,
+                                            int64_t mode) {
+  const int64_t n = points.size(0);
+  const int nd = (int)dim(points, 1);
+  Tensor ws = workspace(mccnn_sampling_workspace_bytes(n), points);
+  hipStream_t s = current_stream();
+  PinnedBlock host;
+  host.words()[0] = 0;
+  {
+    Region r("sampling_count", s);
+    check(mccnn_sampling_count(s, (int)mode, n, nd, f32(points), bids.size(0), i32(bids),
+                               keys.size(0), i64(keys), (int)num_cells.size(0), i32(num_cells),
+                               neighbors.size(0), (int)neighbors.dim(), (int)dim(neighbors, 1),
+                               i32(neighbors), ranges.size(0), i32(ranges), ws.data_ptr(),
+                               ws.numel(), host.words()));
+  }
+  const int64_t k = host.words()[0];
+  Tensor pts = empty_f32({k, nd}, points), out_bids = empty_i32({k}, points),
+         idx = empty_i32({k}, points);
+  Region r("sampling_fill", s);
+  check(mccnn_sampling_fill(s, (int)mode, n, nd, f32(points), i32(bids), i64(keys),
+                            i32(num_cells), ws.data_ptr(), ws.numel(), k, f32(pts), i32(out_bids),
+                            i32(idx)));
+  return {pts, out_bids, idx};
+}
+
+// ------------------------------------------------------------------ dense products ----
+
+Tensor gather_rows(const Tensor &src, const Tensor &rows, int64_t first_col, int64_t cols,
+                   int64_t out_cols) {
+  const int64_t n = rows.defined() ? rows.size(0) : src.size(0);
+  Tensor out = empty_f32({n, out_cols}, src);
+  hipStream_t s = current_stream();
+  Region r("gather_rows", s);
+  check(mccnn_gather_rows_padded(s, n, i32(rows), f32(src), src.size(1), (int)first_col, (int)cols,
+                                 (int)out_cols, f32(out)));
+  return out;
+}
+
+int64_t product_tiles(int64_t n, int64_t f) {   // 128 x 128 tiles, 256 x 64 for odd multiples of 64
+  return f % 128 == 0 ? (n + 127) / 128 * (f / 128) : (n + 255) / 256 * (f / 64);
+}
+
+enum class Product { kTiled, kRegisters, kLibrary };
+
+// Which kernel multiplies [n, r] by [r, f].  Weights beyond the registers of a block of
+// wavefronts (r f > 65536) take the tiled product, whose weights are handed over transposed,
+// once its tiles give every compute unit one; smaller inputs take the register-resident
+// product in blocks of w.  On the bf16 pipe the tiled kernel is also the faster one for
+// smaller weights once there are one and a half tiles per compute unit ([763 063, 1024] x
+// [1024, 64]: 0.82 against 0.93 ms inside the layer step; [30 000, 1024] x [1024, 64]: 0.087
+// against 0.049 ms).
+Product product_kind(int64_t n, int64_t r, int64_t f) {
+  const int64_t tiles = f % 64 == 0 ? product_tiles(n, f) : 0, units = compute_units();
+  if (mccnn_final_product_wt_supported((int)r, (int)f) &&
+      ((r * f > 65536 && tiles >= units) ||
+       (mccnn_split_products_enabled() && 2 * tiles >= 3 * units)))
+    return Product::kTiled;
+  return mccnn_final_product_supported((int)r, (int)f) ? Product::kRegisters : Product::kLibrary;
+}
+
+// x w for x [n, r]; `w` [r, f] and `wt` [f, r]: the one `kind` needs.  Rows of the result go
+// to out_rows if given.
+Tensor run_product(Product kind, const Tensor &x, const Tensor &w, const Tensor &wt,
+                   const Tensor &out_rows) {
+  const int64_t n = x.size(0), r = x.size(1);
+  hipStream_t s = current_stream();
+  if (kind == Product::kLibrary) {
+    Region t("gemm_final", s);
+    Tensor out = at::matmul(x, w);
+    return out_rows.defined() ? at::empty_like(out).index_copy_(0, out_rows.to(at::kLong), out)
+                              : out;
+  }
+  const int64_t f = kind == Product::kTiled ? wt.size(0) : w.size(1);
+  Tensor out = empty_f32({n, f}, x);
+  Region t("final_product", s);
+  if (kind == Product::kTiled)
+    check(mccnn_final_product_wt(s, n, (int)r, f32(x), (int)f, f32(wt), i32(out_rows), f32(out)));
+  else
+    check(mccnn_final_product(s, n, (int)r, f32(x), (int)f, f32(w), i32(out_rows), f32(out)));
+  return out;
+}
+
+Tensor final_product(const Tensor &x, const Tensor &w) {
+  const Product kind = product_kind(x.size(0), w.size(0), w.size(1));
+  if (kind == Product::kTiled) return run_product(kind, x, Tensor(), w.t().contiguous(), Tensor());
+  return run_product(kind, x, w.contiguous(), Tensor(), Tensor());
+}
+
+Tensor weight_grad_product(const Tensor &x, const Tensor &y) {
+  const int64_t c = x.size(1), r = y.size(1);
+  hipStream_t s = current_stream();
+  if (!mccnn_weight_grad_product_supported((int)c, (int)r)) {
+    Region t("gemm_dfinal", s);
+    return at::matmul(x.t(), y);
+  }
+  Tensor ws = workspace(mccnn_weight_grad_product_workspace_bytes((int)c, (int)r), x);
+  Tensor out = empty_f32({c, r}, x);
+  Region t("weight_grad_product", s);
+  check(mccnn_weight_grad_product(s, x.size(0), (int)c, f32(x), (int)r, f32(y), ws.data_ptr(),
+                                  ws.numel(), f32(out)));
+  return out;
+}
+
+Tensor projection_grad_product(const Tensor &x, const Tensor &w) {
+  const int64_t f = x.size(1), r = w.size(0);
+  hipStream_t s = current_stream();
+  if (!mccnn_projection_grad_product_supported((int)f, (int)r)) {
+    Region t("gemm_dproj", s);
+    return at::matmul(x, w.t());
+  }
+  Tensor out = empty_f32({x.size(0), r}, x);
+  Region t("projection_grad_product", s);
+  check(mccnn_projection_grad_product(s, x.size(0), (int)f, f32(x), (int)r, f32(w), f32(out)));
+  return out;
+}
+
+// --------------------------------------------------------------------- convolutions ----
+
+// The neighbourhood of a layer pass in grid order (`_SortedView` of pc.py), and how its pairs
+// are weighted.  The transposed half is only there when a gradient will be asked for.
+struct Geometry : torch::CustomClassHolder {
+  Tensor points_in, points_out, table, ranges, table_t, ranges_t, point_rows, centre_rows;
+  Tensor pdf, pdf_t, inv_radii, neg_inv_radii;
+};
+
+// Sizes of a layer: of its weights, and as the kernels run it.  A layer of several kernel
+// MLPs runs as mlps / per independent convolutions of per * hidden_pad basis columns: kernel
+// MLPs share no final weights (MCConv.py:180-194), so the dense products then cost that many
+// times less than on the block-diagonal matrix.
+struct Plan {
+  int64_t dims, c, h, g, mlps;
+  int64_t c_pad, h_pad, g_pad, per;
+  int64_t act;
+  int64_t k() const { return per * h_pad; }
+  int64_t f() const { return per * g_pad; }
+  bool padded() const { return c_pad != c || h_pad != h || g_pad != g || per != 1; }
+};
+
+// What the kernels read of one sub-layer's weights.
+struct Packed : torch::CustomClassHolder {
+  Tensor w, wt, w2, w2t, kw, kb;
+  Product forward = Product::kRegisters, transposed = Product::kRegisters;
+};
+
+c10::intrusive_ptr<Packed> pack(const Plan &p, int64_t first, const Tensor &final_weights,
+                                const Tensor &kw, const Tensor &kb, int64_t n_out, int64_t n_in,
+                                bool need_w, bool need_transposed) {
+  auto out = c10::make_intrusive<Packed>();
+  const int64_t k = p.k(), f = p.f(), r = p.c_pad * k;
+  out->forward = product_kind(n_out, r, f);
+  out->transposed = product_kind(n_in, f * k, p.c_pad);
+  const bool plain = !p.padded();
+  if (need_w || out->forward != Product::kTiled)
+    out->w = plain && p.mlps == 1 ? final_weights.view({r, f}) : empty_f32({r, f}, final_weights);
+  if (out->forward == Product::kTiled) out->wt = empty_f32({f, r}, final_weights);
+  if (need_transposed) {
+    if (out->transposed == Product::kTiled) out->w2t = empty_f32({p.c_pad, f * k}, final_weights);
+    else out->w2 = empty_f32({f * k, p.c_pad}, final_weights);
+  }
+  const bool kernel = kw.defined();
+  if (kernel) {
+    if (plain && p.mlps == 1) {
+      out->kw = kw;
+      out->kb = kb;
+    } else {
+      out->kw = empty_f32({p.per, p.dims, p.h_pad}, kw);
+      out->kb = empty_f32({k}, kb);
+    }
+  }
+  const bool pack_w = out->w.defined() && !(plain && p.mlps == 1);
+  const bool pack_kernel = kernel && !(plain && p.mlps == 1);
+  if (pack_w || out->wt.defined() || out->w2.defined() || out->w2t.defined() || pack_kernel) {
+    hipStream_t s = current_stream();
+    Region t("pack_layer_weights", s);
+    check(mccnn_pack_layer_weights(
+        s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, (int)first, (int)p.per, (int)p.c_pad,
+        (int)p.h_pad, (int)p.g_pad, f32(final_weights), f32(kw), f32(kb),
+        pack_w ? f32(out->w) : nullptr, f32(out->wt), f32(out->w2), f32(out->w2t),
+        pack_kernel ? f32(out->kw) : nullptr, pack_kernel ? f32(out->kb) : nullptr));
+  }
+  return out;
+}
+
+Tensor mc_project(const Plan &p, const Packed &w, const Tensor &feats, const Tensor &pin,
+                  const Tensor &pout, const Tensor &table, const Tensor &ranges,
+                  const Tensor &inv_radii, const Tensor &pdf) {
+  const int64_t k = p.k(), c = feats.size(1);
+  Tensor out = empty_f32({ranges.size(0), c * k}, feats);
+  hipStream_t s = current_stream();
+  Region t("mc_conv_project", s);
+  check(mccnn_mc_conv_project(s, (int)p.dims, feats.size(0), f32(pin), (int)c, f32(feats),
+                              ranges.size(0), f32(pout), table.size(0), i32(table), i32(ranges),
+                              f32(inv_radii), (int)k, (int)p.per, (int)p.act, f32(w.kw),
+                              f32(w.kb), f32(pdf), nullptr, f32(out)));
+  return out;
+}
+
+// Columns [first, first + cols) of the caller's rows cut out of a padded sub-layer result and
+// joined: [n, mlps * g] from the sub-layers' [n, per * g_pad].
+Tensor join_outputs(const Plan &p, std::vector<Tensor> &outs) {
+  if (p.g_pad != p.g)
+    for (auto &o : outs)
+      o = o.view({o.size(0), p.per, p.g_pad}).slice(2, 0, p.g).reshape({o.size(0), p.per * p.g});
+  return outs.size() == 1 ? outs[0] : at::cat(outs, 1);
+}
+
+// The rows of the upstream gradient that belong to sub-layer `first`, in the view's centre
+// order and padded to its columns.
+Tensor gather_upstream(const Plan &p, const Tensor &dout, const Tensor &rows, int64_t first) {
+  if (p.g_pad == p.g) return gather_rows(dout, rows, first * p.g, p.per * p.g, p.per * p.g);
+  if (p.per == 1) return gather_rows(dout, rows, first * p.g, p.g, p.g_pad);
+  Tensor cols = dout.slice(1, first * p.g, (first + p.per) * p.g)
+                    .reshape({dout.size(0), p.per, p.g});
+  cols = at::constant_pad_nd(cols, {0, p.g_pad - p.g}, 0).view({dout.size(0), p.f()});
+  return rows.defined() ? gather_rows(cols, rows, 0, p.f(), p.f()) : cols;
+}
+
+Tensor cut_columns(const Tensor &x, int64_t cols) {
+  return x.size(1) == cols ? x : x.slice(1, 0, cols).contiguous();
+}
+
+// The whole Monte-Carlo convolution (MCConv.py:137-194) on the grid-ordered view.  Forward:
+// fused basis + projection, product with the final weights, rows written to the centres'
+// original positions by the product.  Backward: the feature gradient is the same convolution
+// run from the centres back to the points over the transposed pair table (no scatter),
+//     Q[j, f, k]  = sum_{i in T(j)} basis[ij, k] dout[i, f]
+//     dfeat[j, c] = sum_{f,k} Q[j, f, k] W[c, k, f]
+//     dW[c, k, f] = sum_j feat[j, c] Q[j, f, k]
+// and the kernel-MLP gradients come from dproj = dout W^T.
+struct McConv : torch::autograd::Function<McConv> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &features, const Tensor &kw,
+                        const Tensor &kb, const Tensor &final_weights,
+                        const c10::intrusive_ptr<Geometry> &geo, const Plan &p, bool grads) {
+    const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
+    const int64_t n_out = geo->ranges.size(0);
+    std::vector<Tensor> outs;
+    c10::List<c10::IValue> packs(c10::AnyType::get());
+    for (int64_t first = 0; first < p.mlps; first += p.per) {
+      auto w = pack(p, first, final_weights, kw, kb, n_out, feats.size(0), grads,
+                    grads);
+      const Tensor proj = mc_project(p, *w, feats, geo->points_in, geo->points_out, geo->table,
+                                     geo->ranges, geo->inv_radii, geo->pdf);
+      outs.push_back(run_product(w->forward, proj, w->w, w->wt, geo->centre_rows));
+      if (grads) packs.push_back(c10::IValue::make_capsule(w));
+    }
+    if (grads) {
+      ctx->save_for_backward({feats, kw, kb, final_weights});
+      ctx->saved_data["geo"] = c10::IValue::make_capsule(geo);
+      ctx->saved_data["packs"] = packs;
+      ctx->saved_data["plan"] = std::vector<int64_t>{p.dims, p.c, p.h, p.g, p.mlps, p.c_pad,
+                                                     p.h_pad, p.g_pad, p.per, p.act};
+    }
+    return join_outputs(p, outs);
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grad_out) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &feats = saved[0], &kw = saved[1], &kb = saved[2], &fw = saved[3];
+    const auto v = ctx->saved_data["plan"].toIntVector();
+    const Plan p{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9]};
+    const auto geo = c10::static_intrusive_pointer_cast<Geometry>(
+        ctx->saved_data["geo"].toCapsule());
+    const auto packs = ctx->saved_data["packs"].toList();
+    const Tensor dout = grad_out[0].contiguous();
+    const int64_t n_out = geo->ranges.size(0), k = p.k();
+    const bool want_feat = ctx->needs_input_grad(0), want_kernel = ctx->needs_input_grad(1) ||
+                                                                   ctx->needs_input_grad(2);
+    const bool want_final = ctx->needs_input_grad(3);
+    Tensor dfeat, dkw, dkb, dfinal;
+    if (want_kernel) {
+      dkw = at::empty_like(kw);
+      dkb = at::empty_like(kb);
+    }
+    if (want_final) dfinal = at::empty_like(fw);
+    hipStream_t s = current_stream();
+    for (int64_t first = 0, i = 0; first < p.mlps; first += p.per, ++i) {
+      const auto w = c10::static_intrusive_pointer_cast<Packed>(
+          packs.get(i).toCapsule());
+      const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g || p.per != p.mlps
+                            ? gather_upstream(p, dout, geo->centre_rows, first) : dout;
+      const bool direct = !p.padded() && p.mlps == 1;      // gradients land in the caller's shapes
+      Tensor dkw_pad, dkb_pad, ddense;
+      if (want_kernel) {
+        const Tensor dproj = projection_grad_product(up, w->w);
+        Tensor ws = workspace(mccnn_mc_conv_project_grads_workspace_bytes((int)p.dims, (int)k,
+                                                                          n_out), feats);
+        dkw_pad = direct ? dkw : empty_f32({p.per, p.dims, p.h_pad}, feats);
+        dkb_pad = direct ? dkb : empty_f32({k}, feats);
+        Region t("mc_conv_project_grads", s);
+        check(mccnn_mc_conv_project_grads(
+            s, (int)p.dims, feats.size(0), f32(geo->points_in), (int)p.c_pad, f32(feats), n_out,
+            f32(geo->points_out), geo->table.size(0), i32(geo->table), i32(geo->ranges),
+            f32(geo->inv_radii), (int)k, (int)p.per, (int)p.act, f32(w->kw), f32(w->kb),
+            f32(geo->pdf), f32(dproj), ws.data_ptr(), ws.numel(), nullptr, nullptr, nullptr,
+            nullptr, f32(dkw_pad), f32(dkb_pad)));
+      }
+      if (want_feat || want_final) {
+        const Tensor q = mc_project(p, *w, up, geo->points_out, geo->points_in, geo->table_t,
+                                    geo->ranges_t, geo->neg_inv_radii, geo->pdf_t);
+        if (want_feat) {
+          Tensor d = run_product(w->transposed, q, w->w2, w->w2t, geo->point_rows);
+          if (dfeat.defined()) dfeat.add_(d);
+          else dfeat = d;
+        }
+        if (want_final) ddense = weight_grad_product(feats, q);
+      }
+      if (want_final || (want_kernel && !direct)) {
+        const bool kernel = want_kernel && !direct;
+        Region t("unpack_layer_grads", s);
+        check(mccnn_unpack_layer_grads(
+            s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, (int)first, (int)p.per, (int)p.c_pad,
+            (int)p.h_pad, (int)p.g_pad, f32(ddense), kernel ? f32(dkw_pad) : nullptr,
+            kernel ? f32(dkb_pad) : nullptr, f32(dfinal), kernel ? f32(dkw) : nullptr,
+            kernel ? f32(dkb) : nullptr));
+      }
+    }
+    if (dfeat.defined()) dfeat = cut_columns(dfeat, p.c);
+    return {dfeat, dkw, dkb, dfinal, Tensor(), Tensor(), Tensor()};
+  }
+};
+
+// Rigid kernel-point convolution (KPConv.py:165-232) on the same view: the basis are the
+// correlations with the kernel points, which need no gradient.
+struct KpShape {
+  int64_t num_kp, kind;
+  double sigma;
+};
+
+Tensor kp_project(const KpShape &kp, const Tensor &kernel_points, int64_t k, const Tensor &feats,
+                  const Tensor &pin, const Tensor &pout, const Tensor &table, const Tensor &ranges,
+                  const Tensor &inv_radii) {
+  const int64_t c = feats.size(1);
+  Tensor out = empty_f32({ranges.size(0), c * k}, feats);
+  hipStream_t s = current_stream();
+  Region t("kp_conv_project", s);
+  check(mccnn_kp_conv_project(s, (int)kernel_points.size(1), feats.size(0), f32(pin), (int)c,
+                              f32(feats), ranges.size(0), f32(pout), table.size(0), i32(table),
+                              i32(ranges), f32(inv_radii), (int)kp.num_kp, f32(kernel_points),
+                              (int)kp.kind, (float)kp.sigma, nullptr, f32(out)));
+  return out;
+}
+
+struct KpConv : torch::autograd::Function<KpConv> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &features, const Tensor &weights,
+                        const Tensor &kernel_points, const c10::intrusive_ptr<Geometry> &geo,
+                        const Plan &p, const KpShape &kp, bool grads) {
+    const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
+    auto w = pack(p, 0, weights, Tensor(), Tensor(), geo->ranges.size(0), feats.size(0), false,
+                  grads);
+    const Tensor proj = kp_project(kp, kernel_points, p.k(), feats, geo->points_in,
+                                   geo->points_out, geo->table, geo->ranges, geo->inv_radii);
+    Tensor out = run_product(w->forward, proj, w->w, w->wt, geo->centre_rows);
+    if (grads) {
+      ctx->save_for_backward({feats, weights, kernel_points});
+      ctx->saved_data["geo"] = c10::IValue::make_capsule(geo);
+      ctx->saved_data["pack"] = c10::IValue::make_capsule(w);
+      ctx->saved_data["plan"] = std::vector<int64_t>{p.dims, p.c, p.h, p.g, p.mlps, p.c_pad,
+                                                     p.h_pad, p.g_pad, p.per, p.act, kp.num_kp,
+                                                     kp.kind};
+      ctx->saved_data["sigma"] = kp.sigma;
+    }
+    return cut_columns(out, p.g);
+  }
+
+  static variable_list backward(AutogradContext *ctx, variable_list grad_out) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &feats = saved[0], &weights = saved[1], &kernel_points = saved[2];
+    const auto v = ctx->saved_data["plan"].toIntVector();
+    const Plan p{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9]};
+    const KpShape kp{v[10], v[11], ctx->saved_data["sigma"].toDouble()};
+    const auto geo = c10::static_intrusive_pointer_cast<Geometry>(
+        ctx->saved_data["geo"].toCapsule());
+    const auto w = c10::static_intrusive_pointer_cast<Packed>(ctx->saved_data["pack"].toCapsule());
+    const Tensor dout = grad_out[0].contiguous();
+    const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g
+                          ? gather_upstream(p, dout, geo->centre_rows, 0) : dout;
+    Tensor dfeat, dweights;
+    if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1)) {
+      const Tensor q = kp_project(kp, kernel_points, p.k(), up, geo->points_out, geo->points_in,
+                                  geo->table_t, geo->ranges_t, geo->neg_inv_radii);
+      if (ctx->needs_input_grad(0))
+        dfeat = cut_columns(run_product(w->transposed, q, w->w2, w->w2t, geo->point_rows), p.c);
+      if (ctx->needs_input_grad(1)) {
+        const Tensor ddense = weight_grad_product(feats, q);
+        dweights = at::empty_like(weights);
+        hipStream_t s = current_stream();
+        Region t("unpack_layer_grads", s);
+        check(mccnn_unpack_layer_grads(s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, 0, 1,
+                                       (int)p.c_pad, (int)p.h_pad, (int)p.g_pad, f32(ddense),
+                                       nullptr, nullptr, f32(dweights), nullptr, nullptr));
+      }
+    }
+    return {dfeat, dweights, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+c10::intrusive_ptr<Geometry> make_geometry(
+    const Tensor &points_in, const Tensor &points_out, const Tensor &table, const Tensor &ranges,
+    const OptTensor &table_t, const OptTensor &ranges_t, const Tensor &point_rows,
+    const OptTensor &centre_rows, const OptTensor &pdf, const OptTensor &pdf_t,
+    const Tensor &inv_radii, const OptTensor &neg_inv_radii) {
+  auto g = c10::make_intrusive<Geometry>();
+  g->points_in = points_in;
+  g->points_out = points_out;
+  g->table = table;
+  g->ranges = ranges;
+  g->table_t = opt(table_t);
+  g->ranges_t = opt(ranges_t);
+  g->point_rows = point_rows;
+  g->centre_rows = opt(centre_rows);
+  g->pdf = opt(pdf);
+  g->pdf_t = opt(pdf_t);
+  g->inv_radii = inv_radii;
+  g->neg_inv_radii = opt(neg_inv_radii);
+  return g;
+}
+
+Plan plan_of(const std::vector<int64_t> &v) {
+  return {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9]};
+}
+
+Tensor mc_conv(const Tensor &features, const Tensor &kw, const Tensor &kb, const Tensor &fw,
+               const std::vector<int64_t> &plan, bool grads, const Tensor &points_in,
+               const Tensor &points_out, const Tensor &table, const Tensor &ranges,
+               const OptTensor &table_t, const OptTensor &ranges_t, const Tensor &point_rows,
+               const OptTensor &centre_rows, const Tensor &pdf, const OptTensor &pdf_t,
+               const Tensor &inv_radii, const OptTensor &neg_inv_radii) {
+  return McConv::apply(features.contiguous(), kw.contiguous(), kb.contiguous(), fw.contiguous(),
+                       make_geometry(points_in, points_out, table, ranges, table_t, ranges_t,
+                                     point_rows, centre_rows, pdf, pdf_t, inv_radii,
+                                     neg_inv_radii),
+                       plan_of(plan), grads);
+}
+
+Tensor kp_conv(const Tensor &features, const Tensor &weights, const Tensor &kernel_points,
+               const std::vector<int64_t> &plan, int64_t kind, double sigma, bool grads,
+               const Tensor &points_in, const Tensor &points_out, const Tensor &table,
+               const Tensor &ranges, const OptTensor &table_t, const OptTensor &ranges_t,
+               const Tensor &point_rows, const OptTensor &centre_rows, const Tensor &inv_radii,
+               const OptTensor &neg_inv_radii) {
+  return KpConv::apply(features.contiguous(), weights.contiguous(), kernel_points,
+                       make_geometry(points_in, points_out, table, ranges, table_t, ranges_t,
+                                     point_rows, centre_rows, OptTensor(), OptTensor(), inv_radii,
+                                     neg_inv_radii),
+                       plan_of(plan), KpShape{kernel_points.size(0), kind, sigma}, grads);
+}
+
+// -------------------------------------------------------------------------- pooling ----
+
+struct LocalPool : torch::autograd::Function<LocalPool> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &features, const Tensor &neighbors,
+                        const Tensor &ranges, int64_t kind) {
+    Tensor out = empty_f32({ranges.size(0), features.size(1)}, features);
+    hipStream_t s = current_stream();
+    {
+      Region t("local_pool", s);
+      check(mccnn_local_pool(s, (int)kind, features.size(0), (int)features.size(1), f32(features),
+                             neighbors.size(0), i32(neighbors), ranges.size(0), i32(ranges),
+                             f32(out)));
+    }
+    ctx->save_for_backward({features, neighbors, ranges, out});
+    ctx->saved_data["kind"] = kind;
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grad_out) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &features = saved[0], &neighbors = saved[1], &ranges = saved[2], &out = saved[3];
+    Tensor dfeat = at::empty_like(features);
+    const Tensor grad = grad_out[0].contiguous();
+    hipStream_t s = current_stream();
+    Region t("local_pool_grads", s);
+    check(mccnn_local_pool_grads(s, (int)ctx->saved_data["kind"].toInt(), features.size(0),
+                                 (int)features.size(1), f32(features), neighbors.size(0),
+                                 i32(neighbors), ranges.size(0), i32(ranges), f32(out), f32(grad),
+                                 f32(dfeat)));
+    return {dfeat, Tensor(), Tensor(), Tensor()};
+  }
+};
+
+struct GlobalPool : torch::autograd::Function<GlobalPool> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &features, const Tensor &bids,
+                        int64_t batch, int64_t kind) {
+    Tensor out = empty_f32({batch, features.size(1)}, features);
+    Tensor counts = empty_i32({batch}, features);
+    hipStream_t s = current_stream();
+    {
+      Region t("global_pool", s);
+      check(mccnn_global_pool(s, (int)kind, features.size(0), (int)features.size(1), f32(features),
+                              i32(bids), (int)batch, f32(out), i32(counts)));
+    }
+    ctx->save_for_backward({features, bids, out, counts});
+    ctx->saved_data["kind"] = kind;
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grad_out) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &features = saved[0], &bids = saved[1], &out = saved[2], &counts = saved[3];
+    const int64_t kind = ctx->saved_data["kind"].toInt();
+    Tensor dfeat = at::empty_like(features), tie;
+    if (kind == 0) tie = at::empty_like(out);
+    const Tensor grad = grad_out[0].contiguous();
+    hipStream_t s = current_stream();
+    Region t("global_pool_grads", s);
+    check(mccnn_global_pool_grads(s, (int)kind, features.size(0), (int)features.size(1),
+                                  f32(features), i32(bids), (int)out.size(0), f32(out),
+                                  i32(counts), f32(grad), f32(tie), f32(dfeat)));
+    return {dfeat, Tensor(), Tensor(), Tensor()};
+  }
+};
+
+Tensor local_pool(const Tensor &features, const Tensor &neighbors, const Tensor &ranges,
+                  int64_t kind) {
+  return LocalPool::apply(features.contiguous(), neighbors, ranges, kind);
+}
+Tensor global_pool(const Tensor &features, const Tensor &bids, int64_t batch, int64_t kind) {
+  return GlobalPool::apply(features.contiguous(), bids, batch, kind);
+}
+
+// ------------------------------------------------------------------------ basis_proj ----
+
+Tensor basis_proj_raw(const Tensor &basis, const Tensor &features, const Tensor &neighbors,
+                      const Tensor &ranges, const Tensor &order) {
+  Tensor out = empty_f32({ranges.size(0), std::max<int64_t>(dim(features, 1), 0),
+                          std::max<int64_t>(dim(basis, 1), 0)}, features);
+  hipStream_t s = current_stream();
+  Region t("basis_proj_ordered", s);
+  check(mccnn_basis_proj_ordered(s, basis.size(0), (int)dim(basis, 1), f32(basis),
+                                 features.size(0), (int)dim(features, 1), f32(features),
+                                 neighbors.size(0), (int)neighbors.dim(), (int)dim(neighbors, 1),
+                                 i32(neighbors), ranges.size(0), i32(ranges), i32(order),
+                                 f32(out)));
+  return out;
+}
+
+Tensor basis_proj_raw_opt(const Tensor &basis, const Tensor &features, const Tensor &neighbors,
+                          const Tensor &ranges, const OptTensor &order) {
+  return basis_proj_raw(basis, features, neighbors, ranges, opt(order));
+}
+
+// -> (dbasis, dfeatures); with the transposed lists the feature gradient is summed per point
+// from per-pair rows, in a fixed order
+std::pair<Tensor, Tensor> basis_proj_grads(const Tensor &basis, const Tensor &features,
+                                           const Tensor &neighbors, const Tensor &ranges,
+                                           const Tensor &g, const OptTensor &order,
+                                           const OptTensor &point_ranges,
+                                           const OptTensor &pair_order) {
+  Tensor dbasis = at::empty_like(basis), dfeat = at::empty_like(features);
+  hipStream_t s = current_stream();
+  if (point_ranges.has_value()) {
+    Tensor rows = empty_f32({neighbors.size(0), features.size(1)}, features);
+    Region t("basis_proj_grads_gathered", s);
+    check(mccnn_basis_proj_grads_gathered(
+        s, basis.size(0), (int)dim(basis, 1), f32(basis), features.size(0), (int)dim(features, 1),
+        f32(features), neighbors.size(0), (int)neighbors.dim(), (int)dim(neighbors, 1),
+        i32(neighbors), ranges.size(0), i32(ranges), (int)g.dim(), dim(g, 0), dim(g, 1), dim(g, 2),
+        f32(g), i32(*point_ranges), i32(opt(pair_order)), f32(rows), f32(dbasis), f32(dfeat)));
+  } else {
+    Region t("basis_proj_grads_ordered", s);
+    check(mccnn_basis_proj_grads_ordered(
+        s, basis.size(0), (int)dim(basis, 1), f32(basis), features.size(0), (int)dim(features, 1),
+        f32(features), neighbors.size(0), (int)neighbors.dim(), (int)dim(neighbors, 1),
+        i32(neighbors), ranges.size(0), i32(ranges), i32(opt(order)), (int)g.dim(), dim(g, 0),
+        dim(g, 1), dim(g, 2), f32(g), f32(dbasis), f32(dfeat)));
+  }
+  return {dbasis, dfeat};
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  static py::object invalid_argument;
+  m.def("set_error_class", [](py::object cls) { invalid_argument = std::move(cls); });
+  py::register_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const InvalidArgument &e) {
+      PyErr_SetString(invalid_argument ? invalid_argument.ptr() : PyExc_ValueError, e.what());
+    }
+  });
+  py::class_<GridTensors>(m, "GridTensors")
+      .def_readonly("aabb_min", &GridTensors::aabb_min)
+      .def_readonly("aabb_max", &GridTensors::aabb_max)
+      .def_readonly("num_cells", &GridTensors::num_cells)
+      .def_readonly("scaled_aabb_min", &GridTensors::smin)
+      .def_readonly("inv_cell_sizes", &GridTensors::inv_cell)
+      .def_readonly("keys", &GridTensors::keys)
+      .def_readonly("sorted_keys", &GridTensors::sorted_keys)
+      .def_readonly("sorted_indices", &GridTensors::sorted_indices)
+      .def_readonly("sorted_points", &GridTensors::sorted_points)
+      .def_readonly("sorted_batch_ids", &GridTensors::sorted_bids)
+      .def_readonly("cells_host", &GridTensors::cells_host)
+      .def_readonly("key_bits", &GridTensors::key_bits);
+  using release = py::call_guard<py::gil_scoped_release>;
+  m.def("start_timing", &start_timing);
+  m.def("collect_timing", &collect_timing);
+  m.def("compute_keys", &compute_keys, release());
+  m.def("sort_keys", &sort_keys, release());
+  m.def("build_grid", &build_grid, release());
+  m.def("build_grid_ds", &build_grid_ds, release());
+  m.def("find_neighbors", &find_neighbors, release());
+  m.def("reorder_neighbors", &reorder_neighbors, release());
+  m.def("original_neighbor_ids", &original_neighbor_ids, release());
+  m.def("transpose_neighbors", &transpose_neighbors, release());
+  m.def("swapped_pairs", &swapped_pairs, release());
+  m.def("gather_pdf", &gather_pdf, release());
+  m.def("gather_i32", &gather_i32, release());
+  m.def("compute_pdf", &compute_pdf, release());
+  m.def("sampling", &sampling, release());
+  m.def("final_product", &final_product, release());
+  m.def("weight_grad_product", &weight_grad_product, release());
+  m.def("projection_grad_product", &projection_grad_product, release());
+  m.def("mc_conv", &mc_conv, release());
+  m.def("kp_conv", &kp_conv, release());
+  m.def("local_pool", &local_pool, release());
+  m.def("global_pool", &global_pool, release());
+  m.def("basis_proj", &basis_proj_raw_opt, release());
+  m.def("basis_proj_grads", &basis_proj_grads, release());
+}

@@ -149,83 +149,17 @@ def _gather_rows(x, rows):
 
 def _weight_grad_product(x, y):
     """x^T y for [N, C] and [N, R] operands with the long reduction over N."""
-    c, r = x.shape[1], y.shape[1]
-    L = _lib.lib()
-    if not L.mccnn_weight_grad_product_supported(cint(c), cint(r)):
-        with _lib.region("gemm_dfinal"):
-            return x.t() @ y
-    L.mccnn_weight_grad_product_workspace_bytes.restype = _lib.csize
-    ws = _lib.workspace(L.mccnn_weight_grad_product_workspace_bytes(cint(c), cint(r)), x.device)
-    out = torch.empty((c, r), dtype=_F32, device=x.device)
-    _lib.call("weight_grad_product", stream(), i64(x.shape[0]), cint(c), ptr(x, _F32), cint(r),
-              ptr(y, _F32), ptr(ws), _lib.csize(ws.numel()), ptr(out))
-    return out
+    return _lib.host().weight_grad_product(x, y)
 
 
 def _projection_grad_product(x, w):
     """x w^T for x [N, F] and w [R, F]."""
-    f, r = x.shape[1], w.shape[0]
-    if not _lib.lib().mccnn_projection_grad_product_supported(cint(f), cint(r)):
-        with _lib.region("gemm_dproj"):
-            return x @ w.t()
-    out = torch.empty((x.shape[0], r), dtype=_F32, device=x.device)
-    _lib.call("projection_grad_product", stream(), i64(x.shape[0]), cint(f), ptr(x, _F32),
-              cint(r), ptr(w.contiguous(), _F32), ptr(out))
-    return out
-
-
-_cu_count = {}
-
-
-def _compute_units(device):
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    if idx not in _cu_count:
-        _cu_count[idx] = torch.cuda.get_device_properties(idx).multi_processor_count
-    return _cu_count[idx]
-
-
-def _tiles(n, f):
-    """Blocks of the tiled product: 128 x 128 tiles, 256 x 64 for odd multiples of 64."""
-    return (n + 127) // 128 * (f // 128) if f % 128 == 0 else (n + 255) // 256 * (f // 64)
-
-
-def _padded_columns(cols):
-    """Output columns of a layer whose count the kernels do not cover, with zero columns
-    added: a multiple of 16, and of 64 beyond 32 (the tiled product and the 64-channel
-    kernels of the backward take 64 columns in less time than the blocked product takes 48:
-    [825 274, 2048] x [2048, 48] 3.4 ms, x [2048, 64] 1.9 ms)."""
-    return -(-cols // 64) * 64 if cols > 32 else -(-cols // 16) * 16
+    return _lib.host().projection_grad_product(x, w.contiguous())
 
 
 def _final_product(x, w):
     """x w for x [N, R] and the final weights w [R, F]."""
-    r, f = w.shape
-    L = _lib.lib()
-    out = torch.empty((x.shape[0], f), dtype=_F32, device=x.device)
-    # Weights beyond the registers of a block of wavefronts (R * F > 65536) take the tiled
-    # product, which reads both operands along the reduction: w is handed over transposed
-    # (a copy of at most a few MB).  Only when its 128-row tiles give every compute unit
-    # one; smaller inputs take the register-resident product in blocks of w.  With the dense
-    # products on the bf16 pipe the tiled kernel is also the faster one for smaller weights
-    # once there are one and a half tiles per compute unit ([763 063, 1024] x [1024, 64]:
-    # 0.82 against 0.93 ms inside the layer step; [30 000, 1024] x [1024, 64]: 0.087 against
-    # 0.049 ms, which is why the register-resident float32 kernel keeps the small inputs).
-    tiles, units = _tiles(x.shape[0], f), _compute_units(x.device)
-    if L.mccnn_final_product_wt_supported(cint(r), cint(f)) and (
-            (r * f > _TILED_ABOVE and tiles >= units) or
-            (L.mccnn_split_products_enabled() and 2 * tiles >= 3 * units)):
-        _lib.call("final_product_wt", stream(), i64(x.shape[0]), cint(r), ptr(x, _F32), cint(f),
-                  ptr(w.t().contiguous(), _F32), ptr(None), ptr(out), timed_as="final_product")
-        return out
-    if not L.mccnn_final_product_supported(cint(r), cint(f)):
-        with _lib.region("gemm_final"):
-            return x @ w
-    _lib.call("final_product", stream(), i64(x.shape[0]), cint(r), ptr(x, _F32), cint(f),
-              ptr(w.contiguous(), _F32), ptr(None), ptr(out))
-    return out
-
-
-_TILED_ABOVE = 65536      # weights that fit the registers of a block of wavefronts
+    return _lib.host().final_product(x, w)
 
 
 class _DenseProduct(torch.autograd.Function):
@@ -311,39 +245,21 @@ def _dense_final_weights(final_weights, c):
     return dense.reshape(c * l * h, l * g)
 
 
-class _MCConvLayer(torch.autograd.Function):
-    """The whole Monte-Carlo convolution (MCConv.py:137-194), run on the
-    neighbourhood's grid-ordered view (features and output gradients are permuted
-    into grid order once per pass so that the gathers of neighbouring centres hit
-    in L2).  Forward: fused basis + projection, product with the final weights
-    (inside the same kernel with `fuse_final`).  Backward: the feature gradient
-    is the same convolution run from the centres back to the points over the
-    transposed pair table (no scatter):
-        Q[j, f, k]  = sum_{i in T(j)} basis[ij, k] dout[i, f]
-        dfeat[j, c] = sum_{f,k} Q[j, f, k] W[c, k, f]
-        dW[c, k, f] = sum_j feat[j, c] Q[j, f, k]
-    and the kernel-MLP gradients come from dproj = dout W^T through the weight
-    half of the fused projection backward."""
+class _MCConvFusedLayer(torch.autograd.Function):
+    """The Monte-Carlo convolution (MCConv.py:137-194) with the product with the final weights
+    inside the projection kernel, in both directions (`fuse_final`); the same passes as
+    McConv of csrc/host.cpp, which runs the projection and the product as two kernels."""
 
     @staticmethod
-    def forward(ctx, weights, biases, final_weights, features, neighborhood, inv_radii, act,
-                fuse_final):
+    def forward(ctx, weights, biases, final_weights, features, neighborhood, inv_radii, act):
         view = neighborhood.sorted_view()
         pdf, _ = view.pair_pdf(neighborhood)
         feats = _gather_rows(features, view.point_rows)
         dense = _dense_final_weights(final_weights, features.shape[1])
-        if fuse_final:
-            out, _ = _mc_layer(weights, biases, feats, view.points_in, view.points_out,
-                               view.table, view.ranges, inv_radii, pdf, act, dense,
-                               view.centre_rows)
-        else:
-            # rows of the projection go straight to the centres' original positions
-            proj = _mc_project(weights, biases, feats, view.points_in, view.points_out,
-                               view.table, view.ranges, inv_radii, pdf, act,
-                               view.centre_rows)
-            out = _final_product(proj.reshape(proj.shape[0], -1), dense)
+        out, _ = _mc_layer(weights, biases, feats, view.points_in, view.points_out, view.table,
+                           view.ranges, inv_radii, pdf, act, dense, view.centre_rows)
         ctx.save_for_backward(weights, biases, final_weights, feats, features, inv_radii)
-        ctx.neighborhood, ctx.act, ctx.fuse_final = neighborhood, act, fuse_final
+        ctx.neighborhood, ctx.act = neighborhood, act
         return out
 
     @staticmethod
@@ -375,28 +291,20 @@ class _MCConvLayer(torch.autograd.Function):
                   ptr(ws), _lib.csize(ws.numel()), ptr(None), ptr(None), ptr(None), ptr(None),
                   ptr(dw), ptr(db))
         del dproj
-        # feature and final-weight gradients from the transposed convolution
+        # feature and final-weight gradients from the transposed convolution: rows of Q and of
+        # dfeat go straight to the points' original positions
         w2 = dense.reshape(c, k, f).permute(2, 1, 0).reshape(f * k, c)
-        neg = pc._negative(inv_radii)
-        if ctx.fuse_final:
-            # rows of Q and of dfeat go straight to the points' original positions
-            dfeat, q = _mc_layer(weights, biases, dout, view.points_out, view.points_in,
-                                 view.table_t, view.ranges_t, neg, pdf_t, ctx.act, w2,
-                                 view.point_rows, want_proj=True)
-            ddense = _weight_grad_product(features, q.reshape(features.shape[0], f * k))
-        else:
-            # rows of Q (and so of dfeat) go straight to the points' original positions
-            q = _mc_project(weights, biases, dout, view.points_out, view.points_in,
-                            view.table_t, view.ranges_t, neg, pdf_t, ctx.act, view.point_rows)
-            dfeat = _final_product(q.reshape(q.shape[0], f * k), w2)
-            ddense = _weight_grad_product(features, q.reshape(features.shape[0], f * k))
+        dfeat, q = _mc_layer(weights, biases, dout, view.points_out, view.points_in,
+                             view.table_t, view.ranges_t, pc._negative(inv_radii), pdf_t, ctx.act,
+                             w2, view.point_rows, want_proj=True)
+        ddense = _weight_grad_product(features, q.reshape(features.shape[0], f * k))
         ddense = ddense.reshape(c, f, k).permute(0, 2, 1)            # [C, K, F]
         if l == 1:
             dfinal = ddense.reshape(1, c * k, f)
         else:
             blocks = ddense.reshape(c, l, h, l, g)
             dfinal = torch.stack([blocks[:, i, :, i, :].reshape(c * h, g) for i in range(l)])
-        return dw, db, dfinal, dfeat, None, None, None, None
+        return dw, db, dfinal, dfeat, None, None, None
 
 
 def _truncated_normal(shape, std, generator, device):
@@ -456,6 +364,9 @@ class MCConv(torch.nn.Module):
         self.transposed_grads = transposed_grads
         # product with the final weights inside the projection kernel (out of LDS)
         self.fuse_final = fuse_final
+        # sizes of the layer as the grid-ordered kernels run it (None: not covered)
+        self._plan = _layer_plan(num_dims, num_features_in, num_features_out, num_mlps, hidden,
+                                 self._act)
 
     def forward(self, features, point_cloud_in, point_cloud_out, radius, neighborhood=None,
                 bandwidth=0.2, return_sorted=False, return_padded=False):
@@ -495,61 +406,30 @@ class MCConv(torch.nn.Module):
         return torch.cat([_dense_product(p[mlp].contiguous(), self.final_weights[mlp])
                           for mlp in range(l)], dim=1)
 
-    def _convolve_on_view(self, features, neighborhood, radii, biases, k):
-        """The fused path on the grid-ordered view; channel counts it does not cover
-        are zero-padded (features, rows / columns of the final weights) and the
-        result is cut back.  None if the shape is out of reach."""
-        d, c, f, l, h = (self._num_dims, self._num_features_in, self._num_features_out,
-                         self._num_mlps, self._hidden)
-        if d not in (2, 3):
-            return None
-        # hidden units per kernel MLP padded with zero columns until the layer has 16, 32 or
-        # 64 basis columns (every activation maps 0 to 0, and the rows of the final weights
-        # that meet the padding are zero too): `MCConv(c, f, 3, 1, [8])` then runs on the
-        # 16-column kernels
-        h_pad = next((v // l for v in (16, 32, 64) if v % l == 0 and v // l >= h), None)
-        pad = _layer_padding(c, f, l)
-        if pad is None or h_pad is None:
-            return None
-        c_pad, g_pad = pad
-        g = f // l
-        weights = self.weights
-        if h_pad != h:
-            weights = torch.nn.functional.pad(weights, (0, h_pad - h))
-            biases = torch.nn.functional.pad(biases, (0, h_pad - h))
-            k = l * h_pad
-        # the backward runs the same single-kernel layer transposed (output channels as its
-        # input channels), so both directions have to be covered
-        supported = _lib.lib().mccnn_mc_conv_layer_supported
-        fuse_final = (self.fuse_final
-                      and bool(supported(cint(d), cint(c_pad), cint(k), cint(g_pad * l)))
-                      and bool(supported(cint(d), cint(g_pad * l), cint(k), cint(c_pad))))
-        final = self.final_weights
-        if c_pad != c or g_pad != g or h_pad != h:
-            final = torch.nn.functional.pad(final.reshape(l, c, h, g),
-                                            (0, g_pad - g, 0, h_pad - h, 0, c_pad - c))
-            final = final.reshape(l, c_pad * h_pad, g_pad)
-            features = torch.nn.functional.pad(features, (0, c_pad - c))
-            h = h_pad
+    def _convolve_on_view(self, features, neighborhood, radii):
+        """The layer on the grid-ordered view (csrc/host.cpp); channel counts its kernels do
+        not cover are zero-padded on the way in and the result is cut back."""
         inv_radii = pc._reciprocal(radii)
-        per = 16 // h if h <= 16 and 16 % h == 0 else 0       # kernel MLPs per 16 basis columns
-        if k > 16 and per > 0 and l % per == 0 and (per * g_pad) % 16 == 0:
-            # Kernel MLPs do not share final weights (MCConv.py:180-194), so the layer is
-            # l / per independent convolutions of 16 basis columns, each with its own
-            # slice of the output: the dense products then cost l / per times less than on
-            # the block-diagonal [C*K, F] matrix (default constructor, 4 x 8: 16.5 -> 12 ms
-            # per step on the scene-scale batch).
-            outs = [_MCConvLayer.apply(weights[t:t + per].contiguous(),
-                                       biases[t:t + per].contiguous(), final[t:t + per],
-                                       features, neighborhood, inv_radii, self._act, False)
-                    for t in range(0, l, per)]
-            out = torch.cat(outs, dim=1)
-        else:
-            out = _MCConvLayer.apply(weights.contiguous(), biases.contiguous(), final, features,
-                                     neighborhood, inv_radii, self._act, fuse_final)
-        if g_pad != g:
-            out = out.reshape(-1, l, g_pad)[:, :, :g].reshape(-1, f)
-        return out
+        if self.fuse_final:
+            c, f, l, h = (self._num_features_in, self._num_features_out, self._num_mlps,
+                          self._hidden)
+            # the backward runs the same single-kernel layer transposed (output channels as its
+            # input channels), so both directions have to be covered
+            d, k, ok = self._num_dims, l * h, _lib.lib().mccnn_mc_conv_layer_supported
+            if ok(cint(d), cint(c), cint(k), cint(f)) and ok(cint(d), cint(f), cint(k), cint(c)):
+                return _MCConvFusedLayer.apply(self.weights, self.biases.reshape(l, h),
+                                               self.final_weights, features, neighborhood,
+                                               inv_radii, self._act)
+        grads = torch.is_grad_enabled() and (features.requires_grad or
+                                             self.weights.requires_grad or
+                                             self.final_weights.requires_grad or
+                                             self.biases.requires_grad)
+        view = neighborhood.sorted_view()
+        pdf, pdf_t = view.pair_pdf(neighborhood, grads)
+        return _lib.host().mc_conv(
+            features, self.weights, self.biases, self.final_weights, self._plan, grads,
+            *view.tensors(grads), pdf, pdf_t if grads else None, inv_radii,
+            pc._negative(inv_radii) if grads else None)
 
     def _convolve(self, features, point_cloud_in, point_cloud_out, radius, neighborhood,
                   bandwidth):
@@ -566,14 +446,12 @@ class MCConv(torch.nn.Module):
             pdf = _differentiable_pdf(neighborhood, bandwidth) if moving else None
             return self._convolve_deep(features, point_cloud_in, point_cloud_out, radii,
                                        neighborhood, pdf)
+        if self.fused and self.transposed_grads and self._plan is not None:
+            return self._convolve_on_view(features, neighborhood, radii)
         biases = self.biases.reshape(self._num_mlps, self._hidden)
         k = self._num_mlps * self._hidden
         fused = self.fused and _lib.lib().mccnn_mc_conv_supported(
             cint(d), cint(self._num_features_in), cint(k))
-        if self.fused and self.transposed_grads:
-            out = self._convolve_on_view(features, neighborhood, radii, biases, k)
-            if out is not None:
-                return out
         pdf = neighborhood.get_pdf()
         transposed = None
         if self.gathered_grads and features.requires_grad and \
@@ -641,17 +519,47 @@ def _activate(x, act):
     return torch.nn.functional.elu(x)
 
 
+def _padded_channels(c):
+    return next((v for v in (16, 32, 64, 128) if v >= c), None)
+
+
 def _layer_padding(c, f, num_mlps):
     """Channel counts the grid-ordered layer path runs on, or None: C rounded up to
-    16/32/64/128, and per kernel MLP as many output columns G' >= G as make the
-    total a multiple of 16 (at most 512)."""
-    c_pad = next((v for v in (16, 32, 64, 128) if v >= c), None)
-    step = 16 // math.gcd(16, num_mlps)
+    16/32/64/128, and per kernel MLP as many output columns G' >= G as make the total a column
+    count of the dense kernels (at most 512)."""
+    c_pad = _padded_channels(c)
     g = f // num_mlps
-    g_pad = -(-g // step) * step
-    if c_pad is None or g_pad * num_mlps > 512:
+    cols = next((v for v in [16, 32] + list(range(64, 513, 64))
+                 if v >= g * num_mlps and v % num_mlps == 0), None)
+    if c_pad is None or cols is None:
         return None
-    return c_pad, g_pad
+    return c_pad, cols // num_mlps
+
+
+def _layer_plan(d, c, f, mlps, hidden, act):
+    """Sizes of a Monte-Carlo layer for the host extension (`Plan` of csrc/host.cpp), or None
+    if its shape is out of reach: (dims, C, H, G, mlps, C', H', G', kernel MLPs per
+    sub-layer, activation).
+
+    Hidden units per kernel MLP are padded with zero columns until the layer has 16, 32 or 64
+    basis columns (every activation maps 0 to 0, and the rows of the final weights that meet
+    the padding are zero too).  Kernel MLPs do not share final weights (MCConv.py:180-194), so
+    a layer of several runs as independent convolutions of 16 basis columns where it divides
+    into them: the dense products then cost that many times less than on the block-diagonal
+    [C*K, F] matrix (default constructor, 4 x 8: 16.5 -> 12 ms per step on the scene-scale
+    batch)."""
+    if d not in (2, 3):
+        return None
+    h_pad = next((v // mlps for v in (16, 32, 64) if v % mlps == 0 and v // mlps >= hidden), None)
+    if h_pad is None:
+        return None
+    per = 16 // h_pad if h_pad <= 16 and 16 % h_pad == 0 else 0
+    if mlps * h_pad <= 16 or per == 0 or mlps % per != 0:
+        per = mlps
+    pad = _layer_padding(c, per * (f // mlps), per)
+    if pad is None:
+        return None
+    return [d, c, hidden, f // mlps, mlps, pad[0], h_pad, pad[1], per, act]
 
 
 class _PointConvLayer(torch.autograd.Function):
@@ -972,7 +880,8 @@ def _kp_project(features, points_in, points_out, neighbors, ranges, inv_radii, k
 
 class _KPConvRigidLayer(torch.autograd.Function):
     """Rigid kernel-point convolution (KPConv.py:165-232) on the neighbourhood's
-    grid-ordered view.  As for the Monte-Carlo convolution, the feature gradient is
+    grid-ordered view, for the shapes that KpConv of csrc/host.cpp does not cover (more than 32
+    kernel points, other dimensions or channel counts: through the op).  As for the Monte-Carlo convolution, the feature gradient is
     the same convolution run from the centres back to the points over the
     transposed pair table, with the kernel-point weights re-evaluated there
     (offset negated), and the weight gradient is feat^T Q; nothing is scattered and
@@ -980,18 +889,15 @@ class _KPConvRigidLayer(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, dense_weights, features, neighborhood, inv_radii, kernel_points, k, kind,
-                sigma, rows_in_view_order):
+                sigma):
         view = neighborhood.sorted_view()
         feats = _gather_rows(features, view.point_rows)
-        # rows of the projection go straight to the centres' original positions (or stay
-        # in the view's order, for a consumer that works on the view itself)
+        # rows of the projection go straight to the centres' original positions
         proj = _kp_project(feats, view.points_in, view.points_out, view.table, view.ranges,
-                           inv_radii, kernel_points, k, kind, sigma,
-                           None if rows_in_view_order else view.centre_rows)
+                           inv_radii, kernel_points, k, kind, sigma, view.centre_rows)
         out = _final_product(proj.reshape(proj.shape[0], -1), dense_weights)
         ctx.save_for_backward(dense_weights, feats, features, inv_radii, kernel_points)
         ctx.neighborhood, ctx.k, ctx.kind, ctx.sigma = neighborhood, k, kind, sigma
-        ctx.rows_in_view_order = rows_in_view_order
         return out
 
     @staticmethod
@@ -999,7 +905,7 @@ class _KPConvRigidLayer(torch.autograd.Function):
         dense, feats, features, inv_radii, kernel_points = ctx.saved_tensors
         view = ctx.neighborhood.sorted_view()
         k, c, f = ctx.k, feats.shape[1], dense.shape[1]
-        if view.centre_rows is not None and not ctx.rows_in_view_order:
+        if view.centre_rows is not None:
             dout = _gather_rows(dout, view.centre_rows)
         else:
             dout = dout.contiguous()
@@ -1015,7 +921,28 @@ class _KPConvRigidLayer(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             ddense = _weight_grad_product(features, q).reshape(c, f, k).permute(0, 2, 1)
             ddense = ddense.reshape(c * k, f)
-        return ddense, dfeat, None, None, None, None, None, None, None
+        return ddense, dfeat, None, None, None, None, None, None
+
+
+def _kp_plan(d, c, f, num_kp, k):
+    """Sizes of a kernel-point layer for the host extension, or None (see `_layer_plan`)."""
+    pad = _layer_padding(c, f, 1)
+    if d not in (2, 3) or k not in (16, 32) or pad is None:
+        return None
+    return [d, c, num_kp, f, 1, pad[0], k, pad[1], 1, 0]
+
+
+def _kp_rigid(weights, plan, features, neighborhood, inv_radii, kernel_points, k, kind, sigma):
+    """Rigid kernel-point convolution with weights [C*KP, F]."""
+    if plan is None:
+        c, kp = features.shape[1], kernel_points.shape[0]
+        dense = torch.nn.functional.pad(weights.reshape(c, kp, -1), (0, 0, 0, k - kp))
+        return _KPConvRigidLayer.apply(dense.reshape(c * k, -1), features, neighborhood, inv_radii,
+                                       kernel_points, k, kind, sigma)
+    grads = torch.is_grad_enabled() and (features.requires_grad or weights.requires_grad)
+    return _lib.host().kp_conv(features, weights, kernel_points, plan, kind, sigma, grads,
+                               *neighborhood.sorted_view().tensors(grads), inv_radii,
+                               pc._negative(inv_radii) if grads else None)
 
 
 def _kp_deform_project(features, points_in, points_out, neighbors, ranges, inv_radii,
@@ -1135,6 +1062,11 @@ class KPConv(torch.nn.Module):
             if offset_weights is None:
                 offset_weights = glorot(fan_in, self._num_kernel_points * num_dims)
             self.offset_weights = torch.nn.Parameter(offset_weights.to(_F32).contiguous())
+        self._plan = _kp_plan(num_dims, num_features_in, num_features_out,
+                              self._num_kernel_points, self._num_basis)
+        self._offset_plan = _kp_plan(num_dims, num_features_in,
+                                     self._num_kernel_points * num_dims,
+                                     self._num_kernel_points, self._num_basis)
         self.last_neighborhood = None
         self._last = None
         self.last_offsets = None      # [N_out, K, D] offsets of the last deformable call
@@ -1169,9 +1101,8 @@ class KPConv(torch.nn.Module):
             return self._convolve_moving(features, point_cloud_in, point_cloud_out, radii,
                                          neighborhood, sigma)
         if not self.deformable and self.transposed_grads:
-            return _KPConvRigidLayer.apply(self._padded(self.weights), features, neighborhood,
-                                           pc._reciprocal(radii), self._kernel_points, k,
-                                           self._kind, sigma, False)
+            return _kp_rigid(self.weights, self._plan, features, neighborhood,
+                             pc._reciprocal(radii), self._kernel_points, k, self._kind, sigma)
         if self.deformable and self.transposed_grads and k == 16 and d in (2, 3) and \
                 _lib.lib().mccnn_kp_deform_offset_grads_supported(cint(d), cint(c)):
             return self._convolve_deformed_on_view(features, neighborhood, radii, sigma)
@@ -1188,17 +1119,14 @@ class KPConv(torch.nn.Module):
 
         offsets = None
         if self.deformable:       # KPConv.py:317-392: offsets from a rigid convolution
-            w_off = self._padded(self.offset_weights)
             if self.transposed_grads and k in (16, 32):
-                # the rigid layer's kernels, output columns padded (45 -> 64)
-                cols = kp * d
-                w_off = torch.nn.functional.pad(w_off, (0, _padded_columns(cols) - cols))
-                offsets = _KPConvRigidLayer.apply(w_off, features, neighborhood,
-                                                  pc._reciprocal(radii), self._kernel_points, k,
-                                                  self._kind, sigma, False)[:, :cols]
+                offsets = _kp_rigid(self.offset_weights, self._offset_plan, features, neighborhood,
+                                    pc._reciprocal(radii), self._kernel_points, k, self._kind,
+                                    sigma)
             else:
                 rigid = _KPBasis.apply(None, *geometry, k, self._kind, sigma)
-                offsets = _dense_product(project(rigid).reshape(-1, c * k), w_off)
+                offsets = _dense_product(project(rigid).reshape(-1, c * k),
+                                         self._padded(self.offset_weights))
             offsets = offsets.reshape(-1, kp, d).contiguous()
         self._last = (offsets, geometry, sigma)
         self.last_offsets = offsets
@@ -1213,12 +1141,8 @@ class KPConv(torch.nn.Module):
         kp, k, d = self._num_kernel_points, self._num_basis, self._num_dims
         view = neighborhood.sorted_view()
         inv_radii = pc._reciprocal(radii)
-        cols = kp * d
-        w_off = torch.nn.functional.pad(self._padded(self.offset_weights),
-                                        (0, _padded_columns(cols) - cols))
-        offsets = _KPConvRigidLayer.apply(w_off, features, neighborhood, inv_radii,
-                                          self._kernel_points, k, self._kind, sigma,
-                                          False)[:, :cols]
+        offsets = _kp_rigid(self.offset_weights, self._offset_plan, features, neighborhood,
+                            inv_radii, self._kernel_points, k, self._kind, sigma)
         offsets = offsets.reshape(-1, kp, d)
         self.last_offsets = offsets
         on_view = offsets if view.centre_order is None else \
@@ -1280,29 +1204,6 @@ class KPConv(torch.nn.Module):
         return _KPRegularization.apply(offsets, *geometry, self._kind, sigma)
 
 
-class _LocalPool(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, features, neighbors, ranges, kind):
-        out = torch.empty((ranges.shape[0], features.shape[1]), dtype=_F32,
-                          device=features.device)
-        _lib.call("local_pool", stream(), cint(kind), i64(features.shape[0]), cint(features.shape[1]),
-            ptr(features, _F32), i64(neighbors.shape[0]), ptr(neighbors, _I32),
-            i64(ranges.shape[0]), ptr(ranges, _I32), ptr(out))
-        ctx.save_for_backward(features, neighbors, ranges, out)
-        ctx.kind = kind
-        return out
-
-    @staticmethod
-    def backward(ctx, grad):
-        features, neighbors, ranges, out = ctx.saved_tensors
-        dfeat = torch.empty_like(features)
-        _lib.call("local_pool_grads", stream(), cint(ctx.kind), i64(features.shape[0]), cint(features.shape[1]),
-            ptr(features, _F32), i64(neighbors.shape[0]), ptr(neighbors, _I32),
-            i64(ranges.shape[0]), ptr(ranges, _I32), ptr(out, _F32),
-            ptr(grad.contiguous(), _F32), ptr(dfeat))
-        return dfeat, None, None, None
-
-
 class _LocalPointPooling:
     kind = 0
 
@@ -1315,8 +1216,8 @@ class _LocalPointPooling:
             neighborhood = pc.Neighborhood(grid, radii, point_cloud_out)
         if point_cloud_out is None:          # centres of a self-neighbourhood: the sorted points
             point_cloud_out = neighborhood._point_cloud_sampled
-        out = _LocalPool.apply(features.contiguous(), neighborhood._original_neigh_ids,
-                               neighborhood._samples_neigh_ranges, self.kind)
+        out = _lib.host().local_pool(features, neighborhood._original_neigh_ids,
+                                     neighborhood._samples_neigh_ranges, self.kind)
         return point_cloud_out.format_output(out, return_sorted, return_padded)
 
 
@@ -1330,35 +1231,12 @@ class AveragePooling(_LocalPointPooling):
     kind = 1
 
 
-class _GlobalPool(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, features, batch_ids, batch_size, kind):
-        out = torch.empty((batch_size, features.shape[1]), dtype=_F32, device=features.device)
-        counts = torch.empty(batch_size, dtype=_I32, device=features.device)
-        _lib.call("global_pool", stream(), cint(kind), i64(features.shape[0]), cint(features.shape[1]),
-            ptr(features, _F32), ptr(batch_ids, _I32), cint(batch_size), ptr(out), ptr(counts))
-        ctx.save_for_backward(features, batch_ids, out, counts)
-        ctx.kind, ctx.batch_size = kind, batch_size
-        return out
-
-    @staticmethod
-    def backward(ctx, grad):
-        features, batch_ids, out, counts = ctx.saved_tensors
-        dfeat = torch.empty_like(features)
-        tie = torch.empty_like(out) if ctx.kind == 0 else None
-        _lib.call("global_pool_grads", stream(), cint(ctx.kind), i64(features.shape[0]), cint(features.shape[1]),
-            ptr(features, _F32), ptr(batch_ids, _I32), cint(ctx.batch_size), ptr(out, _F32),
-            ptr(counts, _I32), ptr(grad.contiguous(), _F32), ptr(tie), ptr(dfeat))
-        return dfeat, None, None, None
-
-
 class GlobalMaxPooling:
     """pylib/pc/layers/Pooling.py:25-61."""
 
     def __call__(self, features, point_cloud, return_padded=False):
         features = point_cloud.flatten_features(features)
-        out = _GlobalPool.apply(features.contiguous(), point_cloud._batch_ids,
-                                point_cloud._batch_size, 0)
+        out = _lib.host().global_pool(features, point_cloud._batch_ids, point_cloud._batch_size, 0)
         if return_padded and point_cloud._batch_shape is not None:   # Pooling.py:58-61
             out = out.reshape(tuple(point_cloud._batch_shape) + (-1,))
         return out
@@ -1369,8 +1247,7 @@ class GlobalAveragePooling:
 
     def __call__(self, features, point_cloud, return_padded=False):
         features = point_cloud.flatten_features(features)
-        out = _GlobalPool.apply(features.contiguous(), point_cloud._batch_ids,
-                                point_cloud._batch_size, 1)
+        out = _lib.host().global_pool(features, point_cloud._batch_ids, point_cloud._batch_size, 1)
         if return_padded and point_cloud._batch_shape is not None:   # Pooling.py:101-104
             out = out.reshape(tuple(point_cloud._batch_shape) + (-1,))
         return out

@@ -4,9 +4,7 @@ and `PointHierarchy` (pylib/pc/PointCloud.py, Grid.py, Neighborhood.py,
 sampling.py, PointHierarchy.py).  They only arrange arguments: bounding boxes,
 grid shape, sort and gathers are kernels of libmccnn_hip.so as well.
 """
-import ctypes
 import enum
-import threading
 import math
 
 import numpy as np
@@ -14,9 +12,7 @@ import numpy as np
 import torch
 
 from . import _lib, tfg_custom_ops
-from ._lib import cint, i64, ptr, stream
-
-_F32, _I32, _I64 = torch.float32, torch.int32, torch.int64
+_F32, _I32 = torch.float32, torch.int32
 
 
 class KDEMode(enum.Enum):
@@ -28,6 +24,7 @@ class KDEMode(enum.Enum):
 
 
 _vector_cache = {}       # (bytes of the host values, dims, device) -> shared device vector
+_scalar_cache = {}       # (float, dims, device) -> one of the vectors above
 _shared = {}             # id of a shared vector -> (the vector itself, its host values)
 _derived_cache = {}      # (operation, id of a shared vector) -> shared result
 
@@ -46,10 +43,16 @@ def _as_vector(value, dims, device):
     tensor is shared read-only afterwards: radii and cell sizes repeat in every
     layer of a network."""
     if isinstance(value, torch.Tensor):
+        if id(value) in _shared and value.shape[0] == dims and value.device == device:
+            return value                       # one of these vectors already
         t = value.to(dtype=_F32).reshape(-1)
         if t.numel() == 1:
             t = t.repeat(dims)
         return t.to(device).contiguous()
+    if type(value) is float:                   # the usual argument, without a trip through numpy
+        t = _scalar_cache.get((value, dims, device))
+        if t is not None:
+            return t
     host = np.asarray(value, dtype=np.float32).reshape(-1)
     key = (host.tobytes(), int(dims), str(device))
     t = _vector_cache.get(key)
@@ -60,6 +63,8 @@ def _as_vector(value, dims, device):
         t = t.to(device).contiguous()
         if len(_vector_cache) < 4096:
             _vector_cache[key] = _share(t, tuple(float(v) for v in t.tolist()))
+    if type(value) is float and len(_scalar_cache) < 4096 and id(t) in _shared:
+        _scalar_cache[(value, dims, device)] = t
     return t
 
 
@@ -135,6 +140,14 @@ class PointCloud:
         if points.dim() > 2:                                  # PointCloud.py:122-138
             self._batch_shape = tuple(points.shape[:-2])
             clouds, v = int(math.prod(self._batch_shape)), points.shape[-2]
+            if self._sizes is None and points.shape[-1] > 0:     # no padding: every row is a point
+                self._sizes = torch.full(self._batch_shape, v, dtype=_I32, device=dev)
+                self._points = points.reshape(clouds * v, -1).contiguous()
+                self._batch_ids = torch.arange(clouds, dtype=_I32, device=dev)[:, None] \
+                    .expand(clouds, v).reshape(-1)
+                self._batch_size = int(clouds if batch_size is None else batch_size)
+                self._dimension = self._points.shape[1]
+                return
             if self._sizes is None:
                 self._sizes = torch.full(self._batch_shape, v, dtype=_I32, device=dev)
             if tuple(self._sizes.shape) != self._batch_shape:
@@ -221,7 +234,9 @@ class PointCloud:
     def flatten_features(self, features):
         """Features [N, C] (returned unchanged) or padded [A1, ..., An, V, C] ->
         [N, C] in the order of the stored points (pylib/pc/utils.py:75-94)."""
-        features = torch.as_tensor(features, dtype=_F32, device=self._points.device)
+        if not isinstance(features, torch.Tensor) or features.dtype != _F32 or \
+                features.device != self._points.device:
+            features = torch.as_tensor(features, dtype=_F32, device=self._points.device)
         if features.dim() == 2:
             if features.shape[0] != self._points.shape[0]:
                 raise ValueError("expected one feature row per point")
@@ -257,21 +272,6 @@ class PointCloud:
         return self._points[self._batch_ids == id % self._batch_size]
 
 
-def _sort_keys(keys, key_bits):
-    """Stable descending sort -> (sorted keys, int32 permutation)."""
-    n, dev = keys.shape[0], keys.device
-    sorted_keys = torch.empty(n, dtype=_I64, device=dev)
-    sorted_indices = torch.empty(n, dtype=_I32, device=dev)
-    ws = _lib.workspace(_lib.lib().mccnn_sort_keys_workspace_bytes(i64(n)), dev)
-    _lib.call("sort_keys_descending", stream(), i64(n), cint(key_bits), ptr(keys, _I64),
-              ptr(sorted_keys), ptr(sorted_indices), ptr(ws), _lib.csize(ws.numel()))
-    return sorted_keys, sorted_indices
-
-
-_ONE_CALL_GRID = 16384     # points up to which a grid is built by the single-call entry point
-_pinned_shape = threading.local()
-
-
 class Grid:
     """Regular grid over a point cloud (pylib/pc/Grid.py:32-84): grid shape from
     the per-cloud bounding boxes, cell keys, stable descending sort, gathers."""
@@ -279,62 +279,23 @@ class Grid:
     def __init__(self, point_cloud, cell_sizes, aabb=None):
         # `aabb` is accepted for the reference's signature; like the reference
         # (Grid.py:42-44) the grid always takes the cloud's own bounding boxes
-        L = _lib.lib()
         pc = point_cloud
-        dev, n, d, b = pc._points.device, pc._points.shape[0], pc._dimension, pc._batch_size
         self._point_cloud = pc
-        self._batch_size = b
-        self._cell_sizes = _as_vector(cell_sizes, d, dev)
-        self._aabb_min = torch.empty((b, d), dtype=_F32, device=dev)
-        self._aabb_max = torch.empty((b, d), dtype=_F32, device=dev)
-        self._num_cells = torch.empty(d, dtype=_I32, device=dev)
-        self._scaled_aabb_min = torch.empty((b, d), dtype=_F32, device=dev)
-        self._inv_cell_sizes = torch.empty(d, dtype=_F32, device=dev)
+        self._batch_size = pc._batch_size
+        self._cell_sizes = _as_vector(cell_sizes, pc._dimension, pc._points.device)
+        g = _lib.host().build_grid(pc._points.detach(), pc._batch_ids, pc._batch_size,
+                                   self._cell_sizes)
+        self._aabb_min, self._aabb_max = g.aabb_min, g.aabb_max
+        self._num_cells = g.num_cells
+        self._scaled_aabb_min, self._inv_cell_sizes = g.scaled_aabb_min, g.inv_cell_sizes
+        self._cur_keys, self._sorted_keys = g.keys, g.sorted_keys
+        self._sorted_indices = g.sorted_indices
+        self._sorted_points, self._sorted_batch_ids = g.sorted_points, g.sorted_batch_ids
+        # host copy of the grid shape: sizes the key width and the column table
+        self._num_cells_host, self._key_bits = g.cells_host, g.key_bits
         self._fast_DS = None
         self._sorted_positions = None
         self._self_neighborhoods = {}
-        if 0 < n <= _ONE_CALL_GRID:
-            # small clouds are bound by calls and launches: the same five steps in one call
-            self._cur_keys = torch.empty(n, dtype=_I64, device=dev)
-            self._sorted_keys = torch.empty(n, dtype=_I64, device=dev)
-            self._sorted_indices = torch.empty(n, dtype=_I32, device=dev)
-            self._sorted_points = torch.empty_like(pc._points)
-            self._sorted_batch_ids = torch.empty_like(pc._batch_ids)
-            ws = _lib.workspace(L.mccnn_build_grid_workspace_bytes(i64(n)), dev)
-            # the grid shape comes back through pinned host memory (one allocation, reused)
-            # (per host thread: two threads may build grids at the same time)
-            pinned = getattr(_pinned_shape, "buffer", None)
-            if pinned is None:
-                pinned = _pinned_shape.buffer = torch.empty(16, dtype=_I32, pin_memory=True)
-            cells_host = (ctypes.c_int32 * d).from_address(pinned.data_ptr())
-            bits_host = ctypes.c_int.from_address(pinned.data_ptr() + 32)
-            _lib.call("build_grid", stream(), i64(n), cint(d), ptr(pc._points, _F32),
-                      ptr(pc._batch_ids, _I32), cint(b), ptr(self._cell_sizes),
-                      ptr(self._aabb_min), ptr(self._aabb_max), ptr(self._num_cells),
-                      ptr(self._scaled_aabb_min), ptr(self._inv_cell_sizes), ptr(self._cur_keys),
-                      ptr(self._sorted_keys), ptr(self._sorted_indices), ptr(self._sorted_points),
-                      ptr(self._sorted_batch_ids), ptr(ws), _lib.csize(ws.numel()), cells_host,
-                      ctypes.byref(bits_host))
-            self._num_cells_host = [int(v) for v in cells_host]
-            self._key_bits = int(bits_host.value)
-            return
-        _lib.call("grid_setup", stream(), i64(n), cint(d), ptr(pc._points, _F32), ptr(pc._batch_ids, _I32), cint(b),
-            ptr(self._cell_sizes), ptr(self._aabb_min), ptr(self._aabb_max),
-            ptr(self._num_cells), ptr(self._scaled_aabb_min), ptr(self._inv_cell_sizes))
-        self._cur_keys = tfg_custom_ops.compute_keys(
-            pc._points, pc._batch_ids, self._scaled_aabb_min, self._num_cells,
-            self._inv_cell_sizes)
-        # host copy of the grid shape: sizes the key width and the column table
-        self._num_cells_host = [int(v) for v in self._num_cells.tolist()]
-        total = b
-        for v in self._num_cells_host:
-            total *= v
-        self._key_bits = max(1, (total - 1).bit_length())
-        self._sorted_keys, self._sorted_indices = _sort_keys(self._cur_keys, self._key_bits)
-        self._sorted_points = torch.empty_like(pc._points)
-        self._sorted_batch_ids = torch.empty_like(pc._batch_ids)
-        _lib.call("gather_points", stream(), i64(n), cint(d), ptr(pc._points), ptr(pc._batch_ids),
-            ptr(self._sorted_indices), ptr(self._sorted_points), ptr(self._sorted_batch_ids))
 
     def sorted_positions(self):
         """Inverse of the sort: position of every original point in the sorted order."""
@@ -380,7 +341,6 @@ class _SortedView:
         self.points_in = grid._sorted_points
         self.point_rows = grid._sorted_indices           # int32, for kernels
         self._point_order = self._centre_order = None    # their int64 forms, on first use
-        n_out = samples._points.shape[0]
         if nbh._equal_samples:
             self.centre_rows = None
             self.points_out = grid._sorted_points
@@ -394,28 +354,14 @@ class _SortedView:
             order = nbh.compute_centre_order()
             self.centre_rows = order
             self.points_out = samples._points[self.centre_order].contiguous()
-            L = _lib.lib()
-            L.mccnn_reorder_neighbors_workspace_bytes.restype = _lib.csize
-            dev = nbh._neighbors.device
-            ws = _lib.workspace(L.mccnn_reorder_neighbors_workspace_bytes(i64(n_out)), dev)
-            self.ranges = torch.empty_like(nbh._samples_neigh_ranges)
-            self.table = torch.empty_like(nbh._neighbors)
-            _lib.call("reorder_neighbors", stream(), i64(n_out),
-                      ptr(nbh._samples_neigh_ranges, _I32), i64(nbh._neighbors.shape[0]),
-                      ptr(nbh._neighbors, _I32), ptr(order, _I32), ptr(ws),
-                      _lib.csize(ws.numel()), ptr(self.ranges), ptr(self.table))
-        if (nbh._equal_samples or nbh._self_neighborhood is not None) and nbh.max_neighbors == 0:
-            # An untruncated self-neighbourhood is symmetric (the distance test is exact
-            # under negation): the rows (x, p) of segment p are at once "x is a neighbour
-            # of centre p" and "p is a neighbour of centre x", so the table is its own
-            # transpose.
-            self.table_t, self.ranges_t = self.table, self.ranges
-        else:
-            self.ranges_t, pair_order = tfg_custom_ops.transpose_neighbors(
-                self.table, self.points_in.shape[0])
-            self.table_t = torch.empty_like(self.table)
-            _lib.call("swapped_pairs", stream(), i64(self.table.shape[0]), ptr(self.table, _I32),
-                      ptr(pair_order, _I32), ptr(self.table_t))
+            self.ranges, self.table = _lib.host().reorder_neighbors(
+                nbh._samples_neigh_ranges, nbh._neighbors, order)
+        # An untruncated self-neighbourhood is symmetric (the distance test is exact under
+        # negation): the rows (x, p) of segment p are at once "x is a neighbour of centre p"
+        # and "p is a neighbour of centre x", so the table is its own transpose.
+        self._symmetric = (nbh._equal_samples or nbh._self_neighborhood is not None) and \
+            nbh.max_neighbors == 0
+        self._transposed = (self.table, self.ranges) if self._symmetric else None
         self._pdf_key, self.pdf, self.pdf_t = None, None, None
 
     @property
@@ -432,33 +378,57 @@ class _SortedView:
             self._centre_order = self.centre_rows.long()
         return self._centre_order
 
-    def pair_pdf(self, nbh):
-        """Per-pair densities of `table` and `table_t` (the neighbour point's)."""
+    def _transpose(self):
+        """The pairs grouped by point: needed by gradients only, built on first use."""
+        if self._transposed is None:
+            ranges_t, pair_order = _lib.host().transpose_neighbors(self.table,
+                                                                   self.points_in.shape[0])
+            self._transposed = (_lib.host().swapped_pairs(self.table, pair_order), ranges_t)
+        return self._transposed
+
+    @property
+    def table_t(self):
+        return self._transpose()[0]
+
+    @property
+    def ranges_t(self):
+        return self._transpose()[1]
+
+    def tensors(self, transposed):
+        """(points_in, points_out, table, ranges, table_t, ranges_t, point_rows, centre_rows)
+        for the host extension; the transposed half is None unless asked for."""
+        table_t, ranges_t = self._transpose() if transposed else (None, None)
+        return (self.points_in, self.points_out, self.table, self.ranges, table_t, ranges_t,
+                self.point_rows, self.centre_rows)
+
+    def pair_pdf(self, nbh, transposed=True):
+        """Per-pair densities of `table` and (unless `transposed` is False) `table_t`, the
+        neighbour point's."""
         per_point = nbh._pdf_per_point
         # compute_pdf bumps the generation: a key made of the density tensor's address
         # could match a later tensor that the allocator put in the same place
         key = nbh._pdf_generation
-        if self.pdf is None or key != self._pdf_key:
-            m, dev = self.table.shape[0], self.table.device
-            if per_point is None:
-                self.pdf = self.pdf_t = torch.ones(m, dtype=_F32, device=dev)
-            else:
-                per_point = per_point.detach()
-                self.pdf = torch.empty(m, dtype=_F32, device=dev)
-                self.pdf_t = torch.empty(m, dtype=_F32, device=dev)
-                for out, table, column in ((self.pdf, self.table, 0), (self.pdf_t, self.table_t, 1)):
-                    _lib.call("gather_pdf_column", stream(), i64(m), ptr(table, _I32), cint(column),
-                              ptr(per_point, _F32), ptr(out))
-                if nbh._pdf_normalize:
-                    # Neighborhood.py:288-293: divided by the size of the pair's
-                    # neighbourhood, i.e. the pair count of its centre (column 1 of
-                    # `table`, column 0 of `table_t`)
-                    ends = self.ranges.long()
-                    counts = (ends - torch.cat([ends.new_zeros(1), ends[:-1]])).to(_F32)
-                    self.pdf = self.pdf / counts[self.table[:, 1].long()]
-                    self.pdf_t = self.pdf_t / counts[self.table_t[:, 0].long()]
-            self._pdf_key = key
+        if key != self._pdf_key:
+            self._pdf_key, self.pdf, self.pdf_t = key, None, None
+        if self.pdf is None:
+            self.pdf = self._pair_values(nbh, per_point, self.table, 0)
+        if transposed and self.pdf_t is None:
+            self.pdf_t = self.pdf if per_point is None else \
+                self._pair_values(nbh, per_point, self.table_t, 1)
         return self.pdf, self.pdf_t
+
+
+    def _pair_values(self, nbh, per_point, table, column):
+        if per_point is None:
+            return torch.ones(table.shape[0], dtype=_F32, device=table.device)
+        pdf = _lib.host().gather_pdf(table, column, per_point.detach())
+        if nbh._pdf_normalize:
+            # Neighborhood.py:288-293: divided by the size of the pair's neighbourhood, i.e.
+            # the pair count of its centre (column 1 of `table`, column 0 of `table_t`)
+            ends = self.ranges.long()
+            counts = (ends - torch.cat([ends.new_zeros(1), ends[:-1]])).to(_F32)
+            pdf = pdf / counts[table[:, 1 - column].long()]
+        return pdf
 
 
 class Neighborhood:
@@ -517,16 +487,8 @@ class Neighborhood:
         if self._self_neighborhood is None:      # a search that was put off
             return self._search()
         own, grid = self._self_neighborhood, self._grid
-        n = self._point_cloud_sampled._points.shape[0]
-        dev = own._neighbors.device
-        L = _lib.lib()
-        ws = _lib.workspace(L.mccnn_reorder_neighbors_workspace_bytes(i64(n)), dev)
-        self._ranges = torch.empty_like(own._samples_neigh_ranges)
-        self._table = torch.empty_like(own._neighbors)
-        _lib.call("reorder_neighbors", stream(), i64(n), ptr(own._samples_neigh_ranges, _I32),
-                  i64(own._neighbors.shape[0]), ptr(own._neighbors, _I32),
-                  ptr(grid.sorted_positions(), _I32), ptr(ws), _lib.csize(ws.numel()),
-                  ptr(self._ranges), ptr(self._table))
+        self._ranges, self._table = _lib.host().reorder_neighbors(
+            own._samples_neigh_ranges, own._neighbors, grid.sorted_positions())
 
     @property
     def _neighbors(self):
@@ -547,10 +509,8 @@ class Neighborhood:
         """The pairs addressed by original point ids (Neighborhood.py:246-250);
         built on first use."""
         if self._original is None:
-            nb = self._neighbors
-            self._original = torch.empty_like(nb)
-            _lib.call("original_neighbor_ids", stream(), i64(nb.shape[0]), ptr(nb, _I32),
-                      ptr(self._grid._sorted_indices, _I32), ptr(self._original))
+            self._original = _lib.host().original_neighbor_ids(self._neighbors,
+                                                               self._grid._sorted_indices)
         return self._original
 
     def transposed_pairs(self):
@@ -591,7 +551,7 @@ class Neighborhood:
         if not self._equal_samples and s._points.shape[0] > 0:
             keys = tfg_custom_ops.compute_keys(s._points, s._batch_ids, grid._scaled_aabb_min,
                                                grid._num_cells, grid._inv_cell_sizes)
-            self._centre_order = _sort_keys(keys, grid._key_bits)[1]
+            self._centre_order = _lib.host().sort_keys(keys, grid._key_bits)[1]
         return self._centre_order
 
     def compute_pdf(self, bandwidth=0.2, mode=KDEMode.constant, normalize=False):
@@ -629,9 +589,7 @@ class Neighborhood:
             if per_point is None:
                 self._pdf = torch.ones(nb.shape[0], dtype=_F32, device=nb.device)
             else:
-                self._pdf = torch.empty(nb.shape[0], dtype=_F32, device=nb.device)
-                _lib.call("gather_pdf", stream(), i64(nb.shape[0]), ptr(nb, _I32),
-                          ptr(per_point.detach(), _F32), ptr(self._pdf))
+                self._pdf = _lib.host().gather_pdf(nb, 0, per_point.detach())
             if self._pdf_normalize:       # divided by the size of the pair's neighbourhood
                 ends = self._samples_neigh_ranges.long()
                 counts = (ends - torch.cat([ends.new_zeros(1), ends[:-1]])).to(_F32)
@@ -659,9 +617,7 @@ def sample(neighborhood, sample_mode="poisson"):
         g._sorted_points, g._sorted_batch_ids, g._sorted_keys, g._num_cells, pairs, ranges, mode)
     original = None
     if mode == 0:
-        original = torch.empty_like(idx)
-        _lib.call("gather_i32", stream(), i64(idx.shape[0]), ptr(g._sorted_indices, _I32), ptr(idx, _I32),
-            ptr(original))
+        original = _lib.host().gather_i32(g._sorted_indices, idx)
     return PointCloud(pts, bids, g._batch_size), original
 
 

@@ -2,7 +2,8 @@
 (custom_ops/tfg_custom_ops/__init__.py:16-26), on torch GPU tensors, with the
 positional argument order of the reference's REGISTER_OP declarations.  Each
 function forwards to one or two C-ABI calls of libmccnn_hip.so on torch's
-current stream; nothing is computed in Python or torch.
+current stream (through the host extension, _host.so); nothing is computed in
+Python or torch.
 
 Gradients mirror custom_ops_wrapper.py:159-169 and :192-198: `basis_proj` and
 `compute_pdf_with_pt_grads` are differentiable (basis and features / points),
@@ -11,7 +12,7 @@ the other ops are not.
 import torch
 
 from .. import _lib
-from .._lib import InvalidArgumentError, cint, i64, ptr, stream, vptr
+from .._lib import InvalidArgumentError, cint, i64, ptr, stream
 
 __all__ = ["compute_keys", "build_grid_ds", "find_neighbors", "sampling",
            "compute_pdf_with_pt_grads", "compute_pdf_pt_grads", "basis_proj",
@@ -26,13 +27,7 @@ def _dim(t, axis, default=-1):
 
 def compute_keys(points, batch_ids, scaled_aabb_min, num_cells, inv_cell_sizes):
     """ComputeKeys (compute_keys_ops.cpp:29-41): int64 cell key per point."""
-    keys = torch.empty(points.shape[0], dtype=_I64, device=points.device)
-    _lib.call("compute_keys", stream(), i64(points.shape[0]), cint(_dim(points, 1)), ptr(points, _F32),
-        i64(batch_ids.shape[0]), ptr(batch_ids, _I32),
-        i64(scaled_aabb_min.shape[0]), cint(_dim(scaled_aabb_min, 1)),
-        ptr(scaled_aabb_min, _F32), cint(num_cells.shape[0]), ptr(num_cells, _I32),
-        cint(inv_cell_sizes.shape[0]), ptr(inv_cell_sizes, _F32), ptr(keys))
-    return keys
+    return _lib.host().compute_keys(points, batch_ids, scaled_aabb_min, num_cells, inv_cell_sizes)
 
 
 def build_grid_ds(sorted_keys, num_cells, num_cells_host, batch_size):
@@ -40,48 +35,16 @@ def build_grid_ds(sorted_keys, num_cells, num_cells_host, batch_size):
     `num_cells_host` is the host copy (list / CPU tensor / numpy) that sizes it."""
     host = [int(v) for v in (num_cells_host.tolist() if hasattr(num_cells_host, "tolist")
                              else num_cells_host)]
-    if batch_size <= 0:
-        raise InvalidArgumentError("BuildGridDs requires a positive batch size")
-    if len(host) < 2:
-        raise InvalidArgumentError("BuildGridDs expects a valid number of dimensions")
-    import ctypes
-    host_arr = (ctypes.c_int32 * len(host))(*host)
-    ds = torch.empty((batch_size, host[0], host[1], 2), dtype=_I32, device=sorted_keys.device)
-    _lib.call("build_grid_ds", stream(), i64(sorted_keys.shape[0]), ptr(sorted_keys, _I64), cint(num_cells.shape[0]),
-        ptr(num_cells, _I32), cint(len(host)), host_arr, cint(batch_size), ptr(ds))
-    return ds
+    return _lib.host().build_grid_ds(sorted_keys, num_cells, host, batch_size)
 
 
 def find_neighbors(samples, samples_batch_ids, points, point_keys, grid_acc_ds, num_cells,
                    scaled_aabb_min, inv_cell_sizes, inv_radii, max_neighs=0):
     """FindNeighbors (find_neighbors_ops.cpp:42-61) -> (ranges [N_out] inclusive
     end offsets, neighbors [M, 2] rows (sorted point index, centre index))."""
-    import ctypes
-    L = _lib.lib()
-    ns, nd = samples.shape[0], _dim(samples, 1)
-    dev = samples.device
-    ws_bytes = L.mccnn_find_neighbors_workspace_bytes(cint(nd), i64(ns))
-    ws = _lib.workspace(ws_bytes, dev)
-    ranges = torch.empty(ns, dtype=_I32, device=dev)
-    total, total_ptr = _lib.host_count()
-    dsr = grid_acc_ds.dim()
-    _lib.call("find_neighbors_count_facts", stream(), i64(ns), cint(nd), ptr(samples, _F32), i64(samples_batch_ids.shape[0]),
-        ptr(samples_batch_ids, _I32), i64(points.shape[0]), cint(_dim(points, 1)),
-        ptr(points, _F32), i64(point_keys.shape[0]), ptr(point_keys, _I64), cint(dsr),
-        cint(_dim(grid_acc_ds, 0)), cint(_dim(grid_acc_ds, 1)), cint(_dim(grid_acc_ds, 2)),
-        cint(_dim(grid_acc_ds, 3)), ptr(grid_acc_ds, _I32), cint(num_cells.shape[0]),
-        ptr(num_cells, _I32), cint(_dim(scaled_aabb_min, 1)), ptr(scaled_aabb_min, _F32),
-        cint(inv_cell_sizes.shape[0]), ptr(inv_cell_sizes, _F32), cint(inv_radii.shape[0]),
-        ptr(inv_radii, _F32), cint(max_neighs), ptr(ws), _lib.csize(ws.numel()), ptr(ranges),
-        total_ptr, _lib.vptr(total.data_ptr() + 8), timed_as="find_neighbors_count")
-    m = int(total[0])
-    symmetric = int(total[1]) == 0 and int(total[2]) == 1
-    neighbors = torch.empty((m, 2), dtype=_I32, device=dev)
-    _lib.call("find_neighbors_fill", stream(), i64(ns), cint(nd), ptr(samples, _F32), ptr(samples_batch_ids, _I32),
-        i64(points.shape[0]), ptr(points, _F32), ptr(point_keys, _I64), ptr(grid_acc_ds, _I32),
-        ptr(num_cells, _I32), ptr(scaled_aabb_min, _F32), ptr(inv_cell_sizes, _F32),
-        ptr(inv_radii, _F32), cint(max_neighs), ptr(ws), _lib.csize(ws.numel()), ptr(ranges),
-        i64(m), ptr(neighbors))
+    ranges, neighbors, symmetric = _lib.host().find_neighbors(
+        samples, samples_batch_ids, points, point_keys, grid_acc_ds, num_cells, scaled_aabb_min,
+        inv_cell_sizes, inv_radii, max_neighs)
     if symmetric:
         _remember_symmetric(neighbors)
     return ranges, neighbors
@@ -118,36 +81,12 @@ def find_neighbors_bounded(samples, samples_batch_ids, points, point_keys, grid_
 def sampling(points, batch_ids, point_keys, num_cells, neighbors, sample_neigh_indices, mode):
     """Sampling (sampling_ops.cpp:33-53): mode 0 Poisson disk, mode 1 cell average.
     -> (sample_pts [S, D], sample_batch_ids [S], sample_indices [S])."""
-    import ctypes
-    L = _lib.lib()
-    n, nd = points.shape[0], _dim(points, 1)
-    dev = points.device
-    ws = _lib.workspace(L.mccnn_sampling_workspace_bytes(i64(n)), dev)
-    total, total_ptr = _lib.host_count()
-    _lib.call("sampling_count", stream(), cint(mode), i64(n), cint(nd), ptr(points, _F32), i64(batch_ids.shape[0]),
-        ptr(batch_ids, _I32), i64(point_keys.shape[0]), ptr(point_keys, _I64),
-        cint(num_cells.shape[0]), ptr(num_cells, _I32), i64(neighbors.shape[0]),
-        cint(neighbors.dim()), cint(_dim(neighbors, 1)), ptr(neighbors, _I32),
-        i64(sample_neigh_indices.shape[0]), ptr(sample_neigh_indices, _I32), ptr(ws),
-        _lib.csize(ws.numel()), total_ptr)
-    s = int(total[0])
-    out_pts = torch.empty((s, nd), dtype=_F32, device=dev)
-    out_bids = torch.empty(s, dtype=_I32, device=dev)
-    out_idx = torch.empty(s, dtype=_I32, device=dev)
-    _lib.call("sampling_fill", stream(), cint(mode), i64(n), cint(nd), ptr(points, _F32), ptr(batch_ids, _I32),
-        ptr(point_keys, _I64), ptr(num_cells, _I32), ptr(ws), _lib.csize(ws.numel()), i64(s),
-        ptr(out_pts), ptr(out_bids), ptr(out_idx))
-    return out_pts, out_bids, out_idx
+    return _lib.host().sampling(points, batch_ids, point_keys, num_cells, neighbors,
+                                sample_neigh_indices, mode)
 
 
 def _compute_pdf_raw(points, neighbors, ranges, inv_bandwidth, inv_radii, mode):
-    pdf = torch.empty(ranges.shape[0], dtype=_F32, device=points.device)
-    _lib.call("compute_pdf", stream(), i64(points.shape[0]), cint(_dim(points, 1)), ptr(points, _F32),
-        i64(neighbors.shape[0]), cint(neighbors.dim()), cint(_dim(neighbors, 1)),
-        ptr(neighbors, _I32), i64(ranges.shape[0]), ptr(ranges, _I32),
-        cint(inv_bandwidth.shape[0]), ptr(inv_bandwidth, _F32), cint(inv_radii.shape[0]),
-        ptr(inv_radii, _F32), cint(mode), ptr(pdf))
-    return pdf
+    return _lib.host().compute_pdf(points, neighbors, ranges, inv_bandwidth, inv_radii, mode)
 
 
 # Pair tables that find_neighbors reported as untruncated self-neighbourhoods (symmetric:
@@ -210,20 +149,15 @@ def compute_pdf_with_pt_grads(points, neighbors, sample_neigh_indices, inv_bandw
     """ComputePdfWithPtGrads (compute_pdf_ops.cpp:43-56): Gaussian KDE per point
     over its neighbour list; differentiable with respect to `points`.
     `symmetric`: see `compute_pdf_pt_grads`."""
+    if not points.requires_grad:
+        return _compute_pdf_raw(points, neighbors, sample_neigh_indices, inv_bandwidth, inv_radii,
+                                mode)
     return _ComputePdf.apply(points, neighbors, sample_neigh_indices, inv_bandwidth,
                              inv_radii, mode, symmetric)
 
 
 def _basis_proj_raw(basis, features, neighbors, ranges, centre_order=None):
-    out = torch.empty((ranges.shape[0], _dim(features, 1), _dim(basis, 1)), dtype=_F32,
-                      device=features.device)
-    _lib.call("basis_proj_ordered", stream(), i64(basis.shape[0]), cint(_dim(basis, 1)),
-              ptr(basis, _F32), i64(features.shape[0]), cint(_dim(features, 1)),
-              ptr(features, _F32), i64(neighbors.shape[0]), cint(neighbors.dim()),
-              cint(_dim(neighbors, 1)), ptr(neighbors, _I32), i64(ranges.shape[0]),
-              ptr(ranges, _I32), ptr(centre_order, _I32 if centre_order is not None else None),
-              ptr(out))
-    return out
+    return _lib.host().basis_proj(basis, features, neighbors, ranges, centre_order)
 
 
 def gathered_grads_supported(num_features, num_basis):
@@ -241,40 +175,19 @@ def basis_proj_grads(basis_neighbors, pt_features, neighbors, sample_neigh_indic
     feat_gradients [N_in, C]).  `transposed` = (point_ranges, pair_order) from
     `transpose_neighbors` selects the atomic-free, bit-reproducible feature
     gradient (needs an [M, C] scratch tensor)."""
-    dbasis = torch.empty_like(basis_neighbors)
-    dfeat = torch.empty_like(pt_features)
-    g = in_gradients
-    head = (stream(), i64(basis_neighbors.shape[0]), cint(_dim(basis_neighbors, 1)),
-            ptr(basis_neighbors, _F32), i64(pt_features.shape[0]), cint(_dim(pt_features, 1)),
-            ptr(pt_features, _F32), i64(neighbors.shape[0]), cint(neighbors.dim()),
-            cint(_dim(neighbors, 1)), ptr(neighbors, _I32), i64(sample_neigh_indices.shape[0]),
-            ptr(sample_neigh_indices, _I32))
-    gdims = (cint(g.dim()), i64(_dim(g, 0)), i64(_dim(g, 1)), i64(_dim(g, 2)), ptr(g, _F32))
+    point_ranges = pair_order = None
     if transposed is not None and gathered_grads_supported(_dim(pt_features, 1),
                                                            _dim(basis_neighbors, 1)):
-        rows = torch.empty((neighbors.shape[0], pt_features.shape[1]), dtype=_F32,
-                           device=pt_features.device)
-        _lib.call("basis_proj_grads_gathered", *head, *gdims, ptr(transposed[0], _I32),
-                  ptr(transposed[1], _I32), ptr(rows), ptr(dbasis), ptr(dfeat))
-    else:
-        _lib.call("basis_proj_grads_ordered", *head,
-                  ptr(centre_order, _I32 if centre_order is not None else None), *gdims,
-                  ptr(dbasis), ptr(dfeat))
-    return dbasis, dfeat
+        point_ranges, pair_order = transposed
+    return _lib.host().basis_proj_grads(basis_neighbors, pt_features, neighbors,
+                                        sample_neigh_indices, in_gradients, centre_order,
+                                        point_ranges, pair_order)
 
 
 def transpose_neighbors(neighbors, num_pts):
     """Pair lists grouped by neighbour point: (point_ranges [num_pts] inclusive end
     offsets, pair_order [M] pair indices sorted by neighbors[:, 0], stable)."""
-    L = _lib.lib()
-    L.mccnn_transpose_neighbors_workspace_bytes.restype = _lib.csize
-    m, dev = neighbors.shape[0], neighbors.device
-    ws = _lib.workspace(L.mccnn_transpose_neighbors_workspace_bytes(i64(m), i64(num_pts)), dev)
-    point_ranges = torch.empty(num_pts, dtype=_I32, device=dev)
-    pair_order = torch.empty(m, dtype=_I32, device=dev)
-    _lib.call("transpose_neighbors", stream(), i64(m), ptr(neighbors, _I32), i64(num_pts),
-              ptr(ws), _lib.csize(ws.numel()), ptr(point_ranges), ptr(pair_order))
-    return point_ranges, pair_order
+    return _lib.host().transpose_neighbors(neighbors, num_pts)
 
 
 class _BasisProj(torch.autograd.Function):
