@@ -112,6 +112,35 @@ int mccnn_build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims,
                      void *workspace, size_t workspace_bytes,
                      int32_t *num_cells_out_host, int *key_bits_out_host);
 
+/* The same with the host copy of the shape written by the kernel itself into pinned host memory
+ * (hipHostMalloc) that stays valid until the call returns.  num_cells_out_pinned and
+ * key_bits_out_host may be NULL for up to mccnn_build_grid_single_launch_max() points: the
+ * whole grid is then one launch and the call does not wait for the device. */
+int64_t mccnn_build_grid_single_launch_max(void);
+int mccnn_build_grid_pinned(mccnn_stream_t stream, int64_t num_pts, int num_dims,
+                            const float *points, const int32_t *batch_ids, int batch_size,
+                            const float *cell_sizes, float *aabb_min_out, float *aabb_max_out,
+                            int32_t *num_cells_out, float *scaled_aabb_min_out,
+                            float *inv_cell_sizes_out, int64_t *keys_out,
+                            int64_t *sorted_keys_out, int32_t *sorted_indices_out,
+                            float *sorted_points_out, int32_t *sorted_batch_ids_out,
+                            void *workspace, size_t workspace_bytes,
+                            int32_t *num_cells_out_pinned, int *key_bits_out_host);
+
+/* Centres ordered by their cell keys in a grid that is there already (mccnn_compute_keys,
+ * mccnn_sort_keys_descending and mccnn_gather_points on the centres): order_out [N_out], and
+ * their coordinates and cloud ids in that order.  key_bits is only read beyond
+ * mccnn_build_grid_single_launch_max() centres.  _invert_order: inverse_out[order[i]] = i. */
+size_t mccnn_order_centres_workspace_bytes(int64_t num_samples);
+int mccnn_order_centres(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                        const float *samples, const int32_t *sample_batch_ids, int batch_size,
+                        const int32_t *num_cells, const float *scaled_aabb_min,
+                        const float *inv_cell_sizes, int key_bits, void *workspace,
+                        size_t workspace_bytes, int32_t *order_out, float *points_out,
+                        int32_t *batch_ids_out);
+int mccnn_invert_order(mccnn_stream_t stream, int64_t count, const int32_t *order,
+                       int32_t *inverse_out);
+
 /* Small gathers of the caller glue:
  *   original ids  out[m] = (sorted_indices[neighbors[m,0]], neighbors[m,1])
  *                 pylib/pc/Neighborhood.py:246-250
@@ -252,6 +281,31 @@ int mccnn_find_neighbors_fill(
 
 /* ------------------------------------------------------------------ pdf --- */
 
+/* The count half of a search by a caller with a grid in hand: mccnn_find_neighbors_count without
+ * the op's shape checks, grid_ds may be NULL (the whole key array is searched: no host copy of
+ * the grid's shape is needed, for clouds of a few thousand points), and result_pinned [2] is
+ * pinned host memory (hipHostMalloc) that the kernels write: the number of pairs, and 1 if some
+ * centre lost pairs to max_neighs.  Workspace: mccnn_find_neighbors_workspace_bytes; continued by
+ * mccnn_find_neighbors_fill. */
+int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                       const float *samples, const int32_t *sample_batch_ids, int64_t num_pts,
+                       const float *points, const int64_t *point_keys, const int32_t *grid_ds,
+                       const int32_t *num_cells, const float *scaled_aabb_min,
+                       const float *inv_cell_sizes, const float *inv_radii, int max_neighs,
+                       void *workspace, size_t workspace_bytes, int32_t *ranges_out,
+                       int64_t *result_pinned);
+
+/* Kernel density of a grid's own (sorted) points straight from the grid: mccnn_compute_pdf on the
+ * untruncated neighbourhood of the points among themselves, without its pair table.  grid_ds may
+ * be NULL as above. */
+size_t mccnn_grid_density_workspace_bytes(int num_dims, int64_t num_pts);
+int mccnn_grid_density(mccnn_stream_t stream, int64_t num_pts, int num_dims, const float *points,
+                       const int32_t *batch_ids, const int64_t *point_keys,
+                       const int32_t *grid_ds, const int32_t *num_cells,
+                       const float *scaled_aabb_min, const float *inv_cell_sizes,
+                       const float *inv_radii, const float *inv_bandwidth, int mode,
+                       void *workspace, size_t workspace_bytes, float *pdf_out);
+
 /* ComputePdf / ComputePdfWithPtGrads: compute_pdf/cc/ops/compute_pdf_ops.cpp:28-161.
  * pdf_out[i] = sum over the pairs of centre i of
  *   prod_d bw_d * exp(-0.5 * ((p_j - p_i)_d * bw_d * inv_radii_d)^2) * 0.39894228
@@ -373,6 +427,17 @@ int mccnn_reorder_neighbors(mccnn_stream_t stream, int64_t num_samples,
                             const int32_t *neighbors, const int32_t *centre_order,
                             void *workspace, size_t workspace_bytes,
                             int32_t *ranges_out, int32_t *neighbors_out);
+/* Its two halves: the end offsets alone, and single columns of the regrouped table (either
+ * output NULL to skip): the pairs with point_map (optional) applied to the point index, the
+ * density pdf[point] of every pair. */
+int mccnn_reorder_ranges(mccnn_stream_t stream, int64_t num_samples, const int32_t *ranges,
+                         const int32_t *centre_order, void *workspace, size_t workspace_bytes,
+                         int32_t *ranges_out);
+int mccnn_reorder_pairs(mccnn_stream_t stream, int64_t num_samples, const int32_t *ranges,
+                        int64_t num_neighbors, const int32_t *neighbors,
+                        const int32_t *centre_order, const int32_t *ranges_out,
+                        const int32_t *point_map, int32_t *neighbors_out, const float *pdf,
+                        float *pdf_per_pair_out);
 
 /* BasisProjGrads without atomics: the feature gradient of each pair is written
  * to pair_rows_workspace [M, C] and then summed per point over the lists of

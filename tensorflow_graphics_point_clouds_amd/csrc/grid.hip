@@ -7,6 +7,8 @@
 
 #include "common.h"
 #include "fill.h"
+#include "small_sort.h"
+#include "sort.h"
 
 namespace mccnn {
 
@@ -143,51 +145,75 @@ __global__ void aabb_init_kernel(int count, unsigned *mn, unsigned *mx) {
   }
 }
 
-// A wavefront walks a run of points (1024 for a large cloud, down to 64 for a small
-// one, so that a few thousand points still spread over many wavefronts).  While the 64 points of an
-// iteration belong to one cloud (the usual layout: clouds stored one after
-// another) the lanes keep running minima / maxima in registers; they are reduced
-// over the wavefront and sent as one atomic per dimension when the cloud changes
-// or the run ends.  Iterations that straddle two clouds use one atomic per lane.
-constexpr int kAabbRun = 1024;
-
-static int aabb_run(int64_t n) {
-  int64_t run = (n / 2048 + kWave - 1) / kWave * kWave;     // aim at ~2048 wavefronts
-  return (int)(run < kWave ? kWave : (run > kAabbRun ? kAabbRun : run));
-}
-
+// Running minima / maxima of one cloud over the lanes of a wavefront.
 template <int D>
-__device__ __forceinline__ void aabb_flush(int b, float *lo, float *hi, unsigned *mn,
-                                           unsigned *mx) {
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      lo[d] = fminf(lo[d], __shfl_xor(lo[d], off, kWave));
-      hi[d] = fmaxf(hi[d], __shfl_xor(hi[d], off, kWave));
-    }
-    if (lane_id() == 0) {
-      atomicMin(&mn[(int64_t)b * D + d], enc_float(lo[d]));
-      atomicMax(&mx[(int64_t)b * D + d], enc_float(hi[d]));
-    }
-    lo[d] = FLT_MAX;
-    hi[d] = -FLT_MAX;
-  }
-}
-
-template <int D>
-__global__ void __launch_bounds__(256) aabb_reduce_kernel(
-    int64_t n, int run, const float *__restrict__ pts, const int *__restrict__ bids,
-    unsigned *mn, unsigned *mx) {
-  const int64_t wave = blockIdx.x * (int64_t)(blockDim.x / kWave) + threadIdx.x / kWave;
-  const int64_t first = wave * run;
-  const int64_t last = first + run < n ? first + run : n;
+struct Bounds {
   float lo[D], hi[D];
+  __device__ __forceinline__ Bounds() { reset(); }
+  __device__ __forceinline__ void reset() {
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    lo[d] = FLT_MAX;
-    hi[d] = -FLT_MAX;
+    for (int d = 0; d < D; ++d) {
+      lo[d] = FLT_MAX;
+      hi[d] = -FLT_MAX;
+    }
   }
+  __device__ __forceinline__ void add(const float *p) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      lo[d] = fminf(lo[d], p[d]);
+      hi[d] = fmaxf(hi[d], p[d]);
+    }
+  }
+  // The wavefront's bounds into mn[0..D), mx[0..D) (encoded), then start over.
+  __device__ __forceinline__ void flush(unsigned *mn, unsigned *mx) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) {
+        lo[d] = fminf(lo[d], __shfl_xor(lo[d], off, kWave));
+        hi[d] = fmaxf(hi[d], __shfl_xor(hi[d], off, kWave));
+      }
+      if (lane_id() == 0) {
+        atomicMin(&mn[d], enc_float(lo[d]));
+        atomicMax(&mx[d], enc_float(hi[d]));
+      }
+    }
+    reset();
+  }
+};
+
+// Bounding boxes of all clouds.  A block takes one contiguous stretch of the points, each of
+// its wavefronts a quarter of it.  While the 64 points of an iteration belong to one cloud (the
+// usual layout: clouds stored one after another) the lanes keep running minima / maxima in
+// registers, reduced over the wavefront when the cloud changes or the stretch ends.  Results
+// meet in LDS for the first eight clouds of the stretch, and leave the block as one atomic per
+// cloud and dimension: thousands of wavefronts sending their own to the same few addresses
+// took 54 us on 763 k points in 8 clouds, the serial rate of an address.
+constexpr int kAabbThreads = 256;
+constexpr int kAabbLdsClouds = 8;
+
+template <int D>
+__global__ void __launch_bounds__(kAabbThreads) aabb_reduce_kernel(
+    int64_t n, int64_t per_block, const float *__restrict__ pts, const int *__restrict__ bids,
+    unsigned *mn, unsigned *mx) {
+  __shared__ unsigned lmn[kAabbLdsClouds * D], lmx[kAabbLdsClouds * D];
+  const unsigned none_lo = enc_float(FLT_MAX), none_hi = enc_float(-FLT_MAX);
+  for (int t = threadIdx.x; t < kAabbLdsClouds * D; t += kAabbThreads) {
+    lmn[t] = none_lo;
+    lmx[t] = none_hi;
+  }
+  __syncthreads();
+  const int64_t block_first = (int64_t)blockIdx.x * per_block;
+  const int b_first = block_first < n ? bids[block_first] : 0;
+  const int64_t per_wave = per_block / (kAabbThreads / kWave);
+  const int64_t first = block_first + (threadIdx.x / kWave) * per_wave;
+  const int64_t last = first + per_wave < n ? first + per_wave : n;
+  auto flush = [&](int b, Bounds<D> &box) {
+    const int e = b - b_first;
+    if (e >= 0 && e < kAabbLdsClouds) box.flush(lmn + e * D, lmx + e * D);
+    else box.flush(mn + (int64_t)b * D, mx + (int64_t)b * D);
+  };
+  Bounds<D> box;
   int cur = -1;                     // cloud of the running minima / maxima (wave-uniform)
   for (int64_t base = first; base < last; base += kWave) {
     const int64_t i = base + lane_id();
@@ -197,19 +223,12 @@ __global__ void __launch_bounds__(256) aabb_reduce_kernel(
 #pragma unroll
     for (int d = 0; d < D; ++d) p[d] = live ? pts[i * D + d] : 0.f;
     const int b0 = __shfl(b, 0, kWave);
-    const bool uniform = __all(b == b0 || !live) && b0 >= 0;
-    if (uniform) {
+    if (__all(b == b0 || !live)) {
       if (b0 != cur) {
-        if (cur >= 0) aabb_flush<D>(cur, lo, hi, mn, mx);
+        if (cur >= 0) flush(cur, box);
         cur = b0;
       }
-      if (live) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-          lo[d] = fminf(lo[d], p[d]);
-          hi[d] = fmaxf(hi[d], p[d]);
-        }
-      }
+      if (live) box.add(p);
     } else if (live) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
@@ -218,37 +237,282 @@ __global__ void __launch_bounds__(256) aabb_reduce_kernel(
       }
     }
   }
-  if (cur >= 0) aabb_flush<D>(cur, lo, hi, mn, mx);
+  if (cur >= 0) flush(cur, box);
+  __syncthreads();
+  for (int t = threadIdx.x; t < kAabbLdsClouds * D; t += kAabbThreads) {
+    const int64_t o = (int64_t)b_first * D + t;
+    if (lmn[t] != none_lo) atomicMin(&mn[o], lmn[t]);
+    if (lmx[t] != none_hi) atomicMax(&mx[o], lmx[t]);
+  }
 }
 
-// min - 1e-9f, max + 1e-9f, grid shape, scaled minimum and reciprocal cell size,
-// in the fp32 expressions of the reference's Python glue.
+// min - 1e-9f, max + 1e-9f, scaled minimum and cells of one (cloud, dimension), in the fp32
+// expressions of the reference's Python glue.
+struct CellExtent {
+  float lo, hi, smin;
+  int cells;
+};
+__device__ __forceinline__ CellExtent finalize_extent(unsigned mn, unsigned mx, float cell) {
+  CellExtent e;
+  e.lo = dec_float(mn) - 1e-9f;
+  e.hi = dec_float(mx) + 1e-9f;
+  const float size = e.hi - e.lo;
+  e.cells = (int)ceilf(size / cell);
+  e.smin = e.lo / cell;
+  return e;
+}
+
+// One block: boxes decoded in place, grid shape, scaled minima, reciprocal cell size.
 template <int D>
-__global__ void grid_finalize_kernel(int batch, const float *__restrict__ cell,
-                                     float *aabb_min, float *aabb_max, int *num_cells,
-                                     float *smin, float *inv_cell) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  int nc[D];
-#pragma unroll
-  for (int d = 0; d < D; ++d) nc[d] = 1;
-  for (int b = 0; b < batch; ++b) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const float lo = dec_float(reinterpret_cast<unsigned *>(aabb_min)[b * D + d]) - 1e-9f;
-      const float hi = dec_float(reinterpret_cast<unsigned *>(aabb_max)[b * D + d]) + 1e-9f;
-      aabb_min[b * D + d] = lo;
-      aabb_max[b * D + d] = hi;
-      const float size = hi - lo;
-      const int c = (int)ceilf(size / cell[d]);
-      nc[d] = c > nc[d] ? c : nc[d];
-      smin[b * D + d] = lo / cell[d];
+__global__ void __launch_bounds__(256) grid_finalize_kernel(int batch,
+                                                            const float *__restrict__ cell,
+                                                            float *aabb_min, float *aabb_max,
+                                                            int *num_cells, float *smin,
+                                                            float *inv_cell) {
+  __shared__ int nc[D];
+  if (threadIdx.x < D) nc[threadIdx.x] = 1;
+  __syncthreads();
+  for (int t = threadIdx.x; t < batch * D; t += blockDim.x) {
+    const int d = t % D;
+    const CellExtent e = finalize_extent(reinterpret_cast<unsigned *>(aabb_min)[t],
+                                         reinterpret_cast<unsigned *>(aabb_max)[t], cell[d]);
+    aabb_min[t] = e.lo;
+    aabb_max[t] = e.hi;
+    smin[t] = e.smin;
+    atomicMax(&nc[d], e.cells);
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    num_cells[threadIdx.x] = nc[threadIdx.x];
+    inv_cell[threadIdx.x] = 1.0f / cell[threadIdx.x];
+  }
+}
+
+// Largest batch * D whose extents a block keeps in LDS.
+constexpr int kGridLdsExtents = 512;
+
+// What a grid is made of; arrays of outputs in the caller's hands.
+struct GridArrays {
+  float *aabb_min, *aabb_max;
+  int *num_cells;
+  float *smin, *inv_cell;
+  int64_t *keys, *sorted_keys;
+  int *sorted_idx;
+  float *sorted_pts;
+  int *sorted_bids;
+};
+
+// Grid shape and keys in one launch, from the encoded boxes mn, mx: every block derives the
+// shape from the batch * D extents for itself (a few dozen values from L2), block 0 writes it
+// out (and to shape_host, pinned host memory the caller waits for).  Beside the 64-bit keys the
+// block stores their lower halves and the digit histogram of its tile for the sort.
+template <int D>
+__global__ void __launch_bounds__(kSortThreads) grid_keys_kernel(
+    int64_t n, int batch, int nb, const float *__restrict__ pts, const int *__restrict__ bids,
+    const float *__restrict__ cell, const unsigned *__restrict__ mn,
+    const unsigned *__restrict__ mx, GridArrays g, unsigned *__restrict__ keys32,
+    int *__restrict__ hist, int *shape_host) {
+  __shared__ int nc[D];
+  __shared__ float smin[kGridLdsExtents];
+  __shared__ int bins[kSortRadix];
+  bins[threadIdx.x] = 0;
+  if (threadIdx.x < D) nc[threadIdx.x] = 1;
+  __syncthreads();
+  for (int t = threadIdx.x; t < batch * D; t += kSortThreads) {
+    const CellExtent e = finalize_extent(mn[t], mx[t], cell[t % D]);
+    smin[t] = e.smin;
+    atomicMax(&nc[t % D], e.cells);
+    if (blockIdx.x == 0) {
+      g.aabb_min[t] = e.lo;
+      g.aabb_max[t] = e.hi;
+      g.smin[t] = e.smin;
     }
   }
+  __syncthreads();
+  GridShape<D> shape;
+  float ic[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    num_cells[d] = nc[d];
-    inv_cell[d] = 1.0f / cell[d];
+    shape.n[d] = nc[d];
+    ic[d] = 1.0f / cell[d];
   }
+  if (blockIdx.x == 0 && threadIdx.x < D) {
+    g.num_cells[threadIdx.x] = nc[threadIdx.x];
+    g.inv_cell[threadIdx.x] = ic[threadIdx.x];
+    if (shape_host) shape_host[threadIdx.x] = nc[threadIdx.x];
+  }
+  const int64_t base = (int64_t)blockIdx.x * kSortTile;
+#pragma unroll
+  for (int k = 0; k < kSortItems; ++k) {
+    const int64_t i = base + k * kSortThreads + threadIdx.x;
+    if (i < n) {
+      const int b = bids[i];
+      float p[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) p[d] = pts[i * D + d];
+      int c[D];
+      cell_of_point<D>(p, smin + b * D, ic, shape, c);
+      const int64_t key = key_of_cell<D>(c, shape, b);
+      g.keys[i] = key;
+      keys32[i] = (unsigned)key;
+      atomicAdd(&bins[(~(unsigned)key) & (kSortRadix - 1)], 1);
+    }
+  }
+  __syncthreads();
+  hist[(int64_t)threadIdx.x * nb + blockIdx.x] = bins[threadIdx.x];
+}
+
+// The whole grid of a small cloud (up to 16 384 points) in one launch of one block: boxes,
+// shape, keys, sort (small_sort.h), gathers.  As separate launches the same steps take 57 us of
+// kernels on 16 x 1024 points, plus the gaps between eight launches and a host round trip for
+// the grid shape.  kOrderOnly: the points are centres of a grid that is there already
+// (num_cells, smin, inv_cell given); their order by cell key, and coordinates and cloud ids in
+// that order.
+struct SmallGridLds {
+  SmallSortLds sort;
+  unsigned mn[kGridLdsExtents], mx[kGridLdsExtents];
+  float smin[kGridLdsExtents];
+  int nc[kMaxDims];
+};
+
+template <int D, bool kOrderOnly>
+__global__ void __launch_bounds__(kSmallThreads) grid_small_kernel(
+    int n, int batch, const float *__restrict__ pts, const int *__restrict__ bids,
+    const float *__restrict__ cell, GridArrays g) {
+  extern __shared__ __align__(16) char lds_raw[];
+  SmallGridLds &s = *reinterpret_cast<SmallGridLds *>(lds_raw);
+  const int t = threadIdx.x, lane = lane_id();
+  const int first = small_first(n), last = small_last(n);
+  GridShape<D> shape;
+  float ic[D];
+  if (kOrderOnly) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      shape.n[d] = g.num_cells[d];
+      ic[d] = g.inv_cell[d];
+    }
+  } else {
+    if (t < batch * D) {
+      s.mn[t] = enc_float(FLT_MAX);
+      s.mx[t] = enc_float(-FLT_MAX);
+    }
+    if (t < D) s.nc[t] = 1;
+    __syncthreads();
+    Bounds<D> box;
+    int cur = -1;
+    for (int base = first; base < last; base += kWave) {
+      const int i = base + lane;
+      const bool live = i < last;
+      const int b = live ? bids[i] : -1;
+      float p[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) p[d] = live ? pts[(int64_t)i * D + d] : 0.0f;
+      const int b0 = __shfl(b, 0, kWave);
+      if (__all(b == b0 || !live)) {
+        if (b0 != cur) {
+          if (cur >= 0) box.flush(s.mn + cur * D, s.mx + cur * D);
+          cur = b0;
+        }
+        if (live) box.add(p);
+      } else if (live) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+          atomicMin(&s.mn[b * D + d], enc_float(p[d]));
+          atomicMax(&s.mx[b * D + d], enc_float(p[d]));
+        }
+      }
+    }
+    if (cur >= 0) box.flush(s.mn + cur * D, s.mx + cur * D);
+    __syncthreads();
+    if (t < batch * D) {
+      const CellExtent e = finalize_extent(s.mn[t], s.mx[t], cell[t % D]);
+      g.aabb_min[t] = e.lo;
+      g.aabb_max[t] = e.hi;
+      g.smin[t] = e.smin;
+      s.smin[t] = e.smin;
+      atomicMax(&s.nc[t % D], e.cells);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      shape.n[d] = s.nc[d];
+      ic[d] = 1.0f / cell[d];
+    }
+    if (t < D) {
+      g.num_cells[t] = s.nc[t];
+      g.inv_cell[t] = 1.0f / cell[t];
+    }
+  }
+  uint64_t cells = (uint64_t)(batch > 0 ? batch : 1);
+#pragma unroll
+  for (int d = 0; d < D; ++d) cells *= (uint64_t)shape.n[d];
+  const int bits = cells > 1 ? 64 - __clzll((long long)(cells - 1)) : 1;
+  for (int r = 0; r < kSmallRounds; ++r) {
+    const int i = first + r * kWave + lane;
+    if (i < last) {
+      const int b = bids[i];
+      float p[D], m[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        p[d] = pts[(int64_t)i * D + d];
+        m[d] = kOrderOnly ? g.smin[(int64_t)b * D + d] : s.smin[b * D + d];
+      }
+      int c[D];
+      cell_of_point<D>(p, m, ic, shape, c);
+      g.keys[i] = key_of_cell<D>(c, shape, b);
+    }
+  }
+  __threadfence_block();
+  __syncthreads();                       // the keys are in memory for the whole block
+  int item[kSmallRounds];
+  small_sort(n, bits, g.keys, item, s.sort);
+#pragma unroll
+  for (int r = 0; r < kSmallRounds; ++r) {
+    const int i = first + r * kWave + lane;
+    if (i < last) {
+      const int from = item[r];
+      g.sorted_idx[i] = from;
+      if (!kOrderOnly) g.sorted_keys[i] = g.keys[from];
+#pragma unroll
+      for (int d = 0; d < D; ++d) g.sorted_pts[(int64_t)i * D + d] = pts[(int64_t)from * D + d];
+      g.sorted_bids[i] = bids[from];
+    }
+  }
+}
+
+// inverse[order[i]] = i
+__global__ void __launch_bounds__(256) invert_order_kernel(int64_t n, const int *__restrict__ order,
+                                                           int *__restrict__ inverse) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    inverse[order[i]] = (int)i;
+}
+
+template <class Kernel, class... Args>
+static int launch_small(Kernel kernel, hipStream_t s, Args... args) {
+  MCCNN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)sizeof(SmallGridLds)));
+  hipLaunchKernelGGL(kernel, dim3(1), dim3(kSmallThreads), sizeof(SmallGridLds), s, args...);
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
+static int reduce_boxes(hipStream_t s, int64_t n, int num_dims, const float *points,
+                        const int *batch_ids, int batch, unsigned *mn, unsigned *mx) {
+  const int count = batch * num_dims;
+  hipLaunchKernelGGL(aabb_init_kernel, dim3(blocks_for(count, 256)), dim3(256), 0, s, count, mn, mx);
+  MCCNN_LAUNCH_CHECK();
+  if (n == 0) return MCCNN_OK;
+  // stretches of at least 1024 points, at most 1024 blocks
+  int64_t per_block = (n + 1023) / 1024;
+  per_block = (per_block < 1024 ? 1024 : per_block + 255) / 256 * 256;
+  MCCNN_DIM_SWITCH(num_dims,
+                   hipLaunchKernelGGL(aabb_reduce_kernel<D>, dim3(blocks_for(n, (int)per_block)),
+                                      dim3(kAabbThreads), 0, s, n, per_block, points, batch_ids, mn,
+                                      mx));
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
 }
 
 }  // namespace mccnn
@@ -340,25 +604,15 @@ extern "C" int mccnn_grid_setup(mccnn_stream_t stream, int64_t num_pts, int num_
   MCCNN_REQUIRE(num_pts >= 0 && cell_sizes && aabb_min_out && aabb_max_out && num_cells_out &&
                     scaled_aabb_min_out && inv_cell_sizes_out,
                 "grid_setup received a null tensor");
-  const int count = batch_size * num_dims;
-  hipLaunchKernelGGL(aabb_init_kernel, dim3(blocks_for(count, 256)), dim3(256), 0,
-                     as_stream(stream), count, (unsigned *)aabb_min_out, (unsigned *)aabb_max_out);
-  MCCNN_LAUNCH_CHECK();
-  if (num_pts > 0) {
-    MCCNN_REQUIRE(points && batch_ids, "grid_setup received a null tensor");
-    const int run = aabb_run(num_pts);
-    MCCNN_DIM_SWITCH(num_dims, hipLaunchKernelGGL(aabb_reduce_kernel<D>,
-                                                  dim3(blocks_for(num_pts, 4 * run)),
-                                                  dim3(256), 0,
-                                                  as_stream(stream), num_pts, run, points, batch_ids,
-                                                  (unsigned *)aabb_min_out,
-                                                  (unsigned *)aabb_max_out));
-    MCCNN_LAUNCH_CHECK();
-  }
-  MCCNN_DIM_SWITCH(num_dims, hipLaunchKernelGGL(grid_finalize_kernel<D>, dim3(1), dim3(64), 0,
-                                                as_stream(stream), batch_size, cell_sizes,
-                                                aabb_min_out, aabb_max_out, num_cells_out,
-                                                scaled_aabb_min_out, inv_cell_sizes_out));
+  MCCNN_REQUIRE(num_pts == 0 || (points && batch_ids), "grid_setup received a null tensor");
+  hipStream_t s = as_stream(stream);
+  int rc = reduce_boxes(s, num_pts, num_dims, points, batch_ids, batch_size,
+                        (unsigned *)aabb_min_out, (unsigned *)aabb_max_out);
+  if (rc != MCCNN_OK) return rc;
+  MCCNN_DIM_SWITCH(num_dims, hipLaunchKernelGGL(grid_finalize_kernel<D>, dim3(1), dim3(256), 0, s,
+                                                batch_size, cell_sizes, aabb_min_out, aabb_max_out,
+                                                num_cells_out, scaled_aabb_min_out,
+                                                inv_cell_sizes_out));
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
@@ -442,13 +696,111 @@ extern "C" int mccnn_gather_i32(mccnn_stream_t stream, int64_t count, const int3
   return MCCNN_OK;
 }
 
-// The grid of pylib/pc/Grid.py:32-64 in one call: bounding boxes and grid shape, keys, the
-// host copy of the grid shape (the one synchronisation: it sizes the key width of the sort
-// and, for the caller, the grid table), stable descending sort, gathers.  The same
-// sequence a caller gets from the five entry points above; small clouds are bound by the
-// cost of making calls and launches, and this is one call instead of five.
+extern "C" int mccnn_invert_order(mccnn_stream_t stream, int64_t count, const int32_t *order,
+                                  int32_t *inverse_out) {
+  MCCNN_REQUIRE(count >= 0, "invert_order expects a non-negative size");
+  if (count == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(order && inverse_out, "invert_order received a null tensor");
+  hipLaunchKernelGGL(invert_order_kernel, dim3(capped_grid(count)), dim3(256), 0,
+                     as_stream(stream), count, order, inverse_out);
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
+// The grid of pylib/pc/Grid.py:32-64 in one call.  Up to 16 384 points: one launch, no host
+// round trip unless the caller asks for the shape.  Beyond that: boxes, shape and keys (three
+// launches), the host copy of the shape -- it sizes the key width of the sort and, for the
+// caller, the grid table --, three launches per digit of the sort, the last of which gathers
+// the points.
 extern "C" size_t mccnn_build_grid_workspace_bytes(int64_t num_pts) {
-  return mccnn_sort_keys_workspace_bytes(num_pts);
+  if (num_pts < 0) num_pts = 0;
+  return carve_sort_workspace(nullptr, num_pts).bytes + align256(sizeof(unsigned) * (size_t)num_pts) +
+         2 * align256(sizeof(unsigned) * kGridLdsExtents);
+}
+
+extern "C" int64_t mccnn_build_grid_single_launch_max(void) { return kSmallMax; }
+
+static int key_bits_for(int batch, int num_dims, const int32_t *cells) {
+  unsigned long long total = (unsigned long long)(batch > 0 ? batch : 1);
+  for (int d = 0; d < num_dims; ++d) total *= (unsigned long long)cells[d];
+  int bits = 1;
+  while (bits < 64 && (1ull << bits) < total) ++bits;
+  return bits;
+}
+
+static int build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims, const float *points,
+                      const int32_t *batch_ids, int batch_size, const float *cell_sizes,
+                      const GridArrays &g, void *workspace, size_t workspace_bytes,
+                      bool shape_is_pinned, int32_t *num_cells_out_host, int *key_bits_out_host) {
+  MCCNN_REQUIRE(valid_dims(num_dims), "build_grid expects a valid number of dimensions");
+  MCCNN_REQUIRE(num_pts >= 0 && num_pts < ((int64_t)1 << 31), "build_grid expects 0 <= num_pts < 2^31");
+  MCCNN_REQUIRE(workspace_bytes >= mccnn_build_grid_workspace_bytes(num_pts),
+                "build_grid workspace too small");
+  hipStream_t s = as_stream(stream);
+  const bool extents_fit = batch_size > 0 && batch_size * num_dims <= kGridLdsExtents;
+  const bool want_shape = num_cells_out_host != nullptr;
+  if (num_pts > 0 && extents_fit) {
+    MCCNN_REQUIRE(points && batch_ids && cell_sizes && g.aabb_min && g.aabb_max && g.num_cells &&
+                      g.smin && g.inv_cell && g.keys && g.sorted_keys && g.sorted_idx &&
+                      g.sorted_pts && g.sorted_bids && workspace,
+                  "build_grid received a null tensor");
+    if (num_pts <= kSmallMax) {
+      int rc = MCCNN_OK;
+      MCCNN_DIM_SWITCH(num_dims, rc = launch_small(grid_small_kernel<D, false>, s, (int)num_pts,
+                                                   batch_size, points, batch_ids, cell_sizes, g));
+      if (rc != MCCNN_OK || !want_shape) return rc;
+      MCCNN_HIP_CHECK(hipMemcpyAsync(num_cells_out_host, g.num_cells, sizeof(int32_t) * num_dims,
+                                     hipMemcpyDeviceToHost, s));
+      MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+      *key_bits_out_host = key_bits_for(batch_size, num_dims, num_cells_out_host);
+      return MCCNN_OK;
+    }
+    MCCNN_REQUIRE(want_shape, "build_grid needs host outputs for the grid shape and the key width");
+    const SortWorkspace w = carve_sort_workspace(workspace, num_pts);
+    char *p = (char *)workspace + w.bytes;
+    unsigned *keys32 = (unsigned *)p;
+    p += align256(sizeof(unsigned) * (size_t)num_pts);
+    unsigned *mn = (unsigned *)p, *mx = (unsigned *)(p + align256(sizeof(unsigned) * kGridLdsExtents));
+    int rc = reduce_boxes(s, num_pts, num_dims, points, batch_ids, batch_size, mn, mx);
+    if (rc != MCCNN_OK) return rc;
+    const int nb = (int)((num_pts + kSortTile - 1) / kSortTile);
+    MCCNN_DIM_SWITCH(num_dims,
+                     hipLaunchKernelGGL(grid_keys_kernel<D>, dim3(nb), dim3(kSortThreads), 0, s,
+                                        num_pts, batch_size, nb, points, batch_ids, cell_sizes, mn,
+                                        mx, g, keys32, w.hist,
+                                        shape_is_pinned ? num_cells_out_host : (int32_t *)nullptr));
+    MCCNN_LAUNCH_CHECK();
+    if (!shape_is_pinned)
+      MCCNN_HIP_CHECK(hipMemcpyAsync(num_cells_out_host, g.num_cells, sizeof(int32_t) * num_dims,
+                                     hipMemcpyDeviceToHost, s));
+    MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+    const int bits = key_bits_for(batch_size, num_dims, num_cells_out_host);
+    *key_bits_out_host = bits;
+    if (bits <= 32) {
+      const SortedPoints out = {points, batch_ids, g.sorted_pts, g.sorted_bids};
+      return sort_grid_keys(s, num_dims, num_pts, bits, keys32, w, g.sorted_keys, g.sorted_idx,
+                            out);
+    }
+  } else {
+    MCCNN_REQUIRE(num_cells_out_host && key_bits_out_host,
+                  "build_grid needs host outputs for the grid shape and the key width");
+    int rc = mccnn_grid_setup(stream, num_pts, num_dims, points, batch_ids, batch_size, cell_sizes,
+                              g.aabb_min, g.aabb_max, g.num_cells, g.smin, g.inv_cell);
+    if (rc != MCCNN_OK) return rc;
+    rc = mccnn_compute_keys(stream, num_pts, num_dims, points, num_pts, batch_ids, batch_size,
+                            num_dims, g.smin, num_dims, g.num_cells, num_dims, g.inv_cell, g.keys);
+    if (rc != MCCNN_OK) return rc;
+    MCCNN_HIP_CHECK(hipMemcpyAsync(num_cells_out_host, g.num_cells, sizeof(int32_t) * num_dims,
+                                   hipMemcpyDeviceToHost, s));
+    MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+    *key_bits_out_host = key_bits_for(batch_size, num_dims, num_cells_out_host);
+  }
+  // keys wider than 32 bits, or more clouds than a block keeps the extents of
+  int rc = mccnn_sort_keys_descending(stream, num_pts, *key_bits_out_host, g.keys, g.sorted_keys,
+                                      g.sorted_idx, workspace, workspace_bytes);
+  if (rc != MCCNN_OK) return rc;
+  return mccnn_gather_points(stream, num_pts, num_dims, points, batch_ids, g.sorted_idx,
+                             g.sorted_pts, g.sorted_bids);
 }
 
 extern "C" int mccnn_build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims,
@@ -461,29 +813,77 @@ extern "C" int mccnn_build_grid(mccnn_stream_t stream, int64_t num_pts, int num_
                                 int32_t *sorted_batch_ids_out, void *workspace,
                                 size_t workspace_bytes, int32_t *num_cells_out_host,
                                 int *key_bits_out_host) {
-  MCCNN_REQUIRE(valid_dims(num_dims), "build_grid expects a valid number of dimensions");
   MCCNN_REQUIRE(num_cells_out_host && key_bits_out_host,
                 "build_grid needs host outputs for the grid shape and the key width");
-  int rc = mccnn_grid_setup(stream, num_pts, num_dims, points, batch_ids, batch_size, cell_sizes,
-                            aabb_min_out, aabb_max_out, num_cells_out, scaled_aabb_min_out,
-                            inv_cell_sizes_out);
-  if (rc != MCCNN_OK) return rc;
-  rc = mccnn_compute_keys(stream, num_pts, num_dims, points, num_pts, batch_ids, batch_size,
-                          num_dims, scaled_aabb_min_out, num_dims, num_cells_out, num_dims,
-                          inv_cell_sizes_out, keys_out);
-  if (rc != MCCNN_OK) return rc;
+  const GridArrays g = {aabb_min_out, aabb_max_out, num_cells_out, scaled_aabb_min_out,
+                        inv_cell_sizes_out, keys_out, sorted_keys_out, sorted_indices_out,
+                        sorted_points_out, sorted_batch_ids_out};
+  return build_grid(stream, num_pts, num_dims, points, batch_ids, batch_size, cell_sizes, g,
+                    workspace, workspace_bytes, false, num_cells_out_host, key_bits_out_host);
+}
+
+extern "C" int mccnn_build_grid_pinned(mccnn_stream_t stream, int64_t num_pts, int num_dims,
+                                       const float *points, const int32_t *batch_ids,
+                                       int batch_size, const float *cell_sizes,
+                                       float *aabb_min_out, float *aabb_max_out,
+                                       int32_t *num_cells_out, float *scaled_aabb_min_out,
+                                       float *inv_cell_sizes_out, int64_t *keys_out,
+                                       int64_t *sorted_keys_out, int32_t *sorted_indices_out,
+                                       float *sorted_points_out, int32_t *sorted_batch_ids_out,
+                                       void *workspace, size_t workspace_bytes,
+                                       int32_t *num_cells_out_pinned, int *key_bits_out_host) {
+  const GridArrays g = {aabb_min_out, aabb_max_out, num_cells_out, scaled_aabb_min_out,
+                        inv_cell_sizes_out, keys_out, sorted_keys_out, sorted_indices_out,
+                        sorted_points_out, sorted_batch_ids_out};
+  return build_grid(stream, num_pts, num_dims, points, batch_ids, batch_size, cell_sizes, g,
+                    workspace, workspace_bytes, true, num_cells_out_pinned, key_bits_out_host);
+}
+
+// Centres in the order of their cells in a grid that is there already: order, coordinates and
+// cloud ids.  Up to 16 384 centres one launch; beyond that keys, sort and gather, for which the
+// key width of the grid is needed.
+extern "C" int mccnn_order_centres(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                                   const float *samples, const int32_t *sample_batch_ids,
+                                   int batch_size, const int32_t *num_cells,
+                                   const float *scaled_aabb_min, const float *inv_cell_sizes,
+                                   int key_bits, void *workspace, size_t workspace_bytes,
+                                   int32_t *order_out, float *points_out,
+                                   int32_t *batch_ids_out) {
+  MCCNN_REQUIRE(valid_dims(num_dims), "order_centres expects a valid number of dimensions");
+  MCCNN_REQUIRE(num_samples >= 0 && num_samples < ((int64_t)1 << 31) && batch_size > 0,
+                "order_centres expects 0 <= num_samples < 2^31 and a positive batch size");
+  if (num_samples == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(samples && sample_batch_ids && num_cells && scaled_aabb_min && inv_cell_sizes &&
+                    workspace && order_out && points_out && batch_ids_out,
+                "order_centres received a null tensor");
+  MCCNN_REQUIRE(workspace_bytes >= mccnn_order_centres_workspace_bytes(num_samples),
+                "order_centres workspace too small");
   hipStream_t s = as_stream(stream);
-  MCCNN_HIP_CHECK(hipMemcpyAsync(num_cells_out_host, num_cells_out, sizeof(int32_t) * num_dims,
-                                 hipMemcpyDeviceToHost, s));
-  MCCNN_HIP_CHECK(hipStreamSynchronize(s));
-  unsigned long long total = (unsigned long long)(batch_size > 0 ? batch_size : 1);
-  for (int d = 0; d < num_dims; ++d) total *= (unsigned long long)num_cells_out_host[d];
-  int bits = 1;
-  while (bits < 64 && (1ull << bits) < total) ++bits;
-  *key_bits_out_host = bits;
-  rc = mccnn_sort_keys_descending(stream, num_pts, bits, keys_out, sorted_keys_out,
-                                  sorted_indices_out, workspace, workspace_bytes);
+  if (num_samples <= kSmallMax) {
+    const GridArrays g = {nullptr, nullptr, (int *)num_cells, (float *)scaled_aabb_min,
+                          (float *)inv_cell_sizes, (int64_t *)workspace, nullptr, order_out,
+                          points_out, batch_ids_out};
+    int rc = MCCNN_OK;
+    MCCNN_DIM_SWITCH(num_dims, rc = launch_small(grid_small_kernel<D, true>, s, (int)num_samples,
+                                                 batch_size, samples, sample_batch_ids,
+                                                 (const float *)nullptr, g));
+    return rc;
+  }
+  char *p = (char *)workspace;
+  int64_t *keys = (int64_t *)p, *sorted = (int64_t *)(p + align256(8 * (size_t)num_samples));
+  void *ws = p + 2 * align256(8 * (size_t)num_samples);
+  int rc = mccnn_compute_keys(stream, num_samples, num_dims, samples, num_samples,
+                              sample_batch_ids, batch_size, num_dims, scaled_aabb_min, num_dims,
+                              num_cells, num_dims, inv_cell_sizes, keys);
   if (rc != MCCNN_OK) return rc;
-  return mccnn_gather_points(stream, num_pts, num_dims, points, batch_ids, sorted_indices_out,
-                             sorted_points_out, sorted_batch_ids_out);
+  rc = mccnn_sort_keys_descending(stream, num_samples, key_bits, keys, sorted, order_out, ws,
+                                  carve_sort_workspace(nullptr, num_samples).bytes);
+  if (rc != MCCNN_OK) return rc;
+  return mccnn_gather_points(stream, num_samples, num_dims, samples, sample_batch_ids, order_out,
+                             points_out, batch_ids_out);
+}
+
+extern "C" size_t mccnn_order_centres_workspace_bytes(int64_t num_samples) {
+  if (num_samples < 0) num_samples = 0;
+  return 2 * align256(8 * (size_t)num_samples) + carve_sort_workspace(nullptr, num_samples).bytes;
 }

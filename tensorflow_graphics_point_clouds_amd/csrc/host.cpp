@@ -181,21 +181,10 @@ Tensor compute_keys(const Tensor &points, const Tensor &bids, const Tensor &smin
   return keys;
 }
 
-std::pair<Tensor, Tensor> sort_keys(const Tensor &keys, int64_t bits) {
-  const int64_t n = keys.size(0);
-  Tensor sorted = empty_i64({n}, keys), order = empty_i32({n}, keys);
-  Tensor ws = workspace(mccnn_sort_keys_workspace_bytes(n), keys);
-  hipStream_t s = current_stream();
-  Region r("sort_keys_descending", s);
-  check(mccnn_sort_keys_descending(s, n, (int)bits, i64(keys), i64(sorted), i32(order),
-                                   ws.data_ptr(), ws.numel()));
-  return {sorted, order};
-}
-
 struct GridTensors {
   Tensor aabb_min, aabb_max, num_cells, smin, inv_cell, keys, sorted_keys, sorted_indices,
       sorted_points, sorted_bids;
-  std::vector<int64_t> cells_host;
+  std::vector<int64_t> cells_host;   // empty: the shape has not been waited for
   int64_t key_bits = 0;
 };
 
@@ -216,17 +205,49 @@ GridTensors build_grid(const Tensor &points, const Tensor &bids, int64_t batch,
   g.sorted_bids = empty_i32({n}, points);
   Tensor ws = workspace(mccnn_build_grid_workspace_bytes(n), points);
   hipStream_t s = current_stream();
+  Region r("build_grid", s);
+  auto call = [&](int32_t *cells, int *bits) {
+    check(mccnn_build_grid_pinned(s, n, (int)d, f32(points), i32(bids), (int)batch,
+                                  f32(cell_sizes), f32(g.aabb_min), f32(g.aabb_max),
+                                  i32(g.num_cells), f32(g.smin), f32(g.inv_cell), i64(g.keys),
+                                  i64(g.sorted_keys), i32(g.sorted_indices), f32(g.sorted_points),
+                                  i32(g.sorted_bids), ws.data_ptr(), ws.numel(), cells, bits));
+  };
+  if (n > 0 && n <= mccnn_build_grid_single_launch_max() && batch > 0 && batch * d <= 512) {
+    call(nullptr, nullptr);
+    return g;
+  }
   PinnedBlock host;
   int bits = 1;
-  Region r("build_grid", s);
-  check(mccnn_build_grid(s, n, (int)d, f32(points), i32(bids), (int)batch, f32(cell_sizes),
-                         f32(g.aabb_min), f32(g.aabb_max), i32(g.num_cells), f32(g.smin),
-                         f32(g.inv_cell), i64(g.keys), i64(g.sorted_keys), i32(g.sorted_indices),
-                         f32(g.sorted_points), i32(g.sorted_bids), ws.data_ptr(), ws.numel(),
-                         host.ints(), &bits));
+  call(host.ints(), &bits);
   for (int64_t i = 0; i < d; ++i) g.cells_host.push_back(host.ints()[i]);
   g.key_bits = bits;
   return g;
+}
+
+// Centres in the order of their cells in a grid -> (order, coordinates, cloud ids).
+std::tuple<Tensor, Tensor, Tensor> order_centres(const Tensor &samples, const Tensor &bids,
+                                                 int64_t batch, const Tensor &num_cells,
+                                                 const Tensor &smin, const Tensor &inv_cell,
+                                                 int64_t key_bits) {
+  const int64_t n = samples.size(0), d = samples.size(1);
+  Tensor order = empty_i32({n}, samples), pts = empty_f32({n, d}, samples),
+         out_bids = empty_i32({n}, samples);
+  Tensor ws = workspace(mccnn_order_centres_workspace_bytes(n), samples);
+  hipStream_t s = current_stream();
+  Region r("order_centres", s);
+  check(mccnn_order_centres(s, n, (int)d, f32(samples), i32(bids), (int)batch, i32(num_cells),
+                            f32(smin), f32(inv_cell), (int)key_bits, ws.data_ptr(), ws.numel(),
+                            i32(order), f32(pts), i32(out_bids)));
+  return {order, pts, out_bids};
+}
+
+Tensor invert_order(const Tensor &order) {
+  Tensor out = empty_i32({order.size(0)}, order);
+  hipStream_t s = current_stream();
+  Region r("invert_order", s);
+  check(mccnn_invert_order(s, order.size(0), i32(order), i32(out)));
+  return out;
 }
 
 Tensor build_grid_ds(const Tensor &sorted_keys, const Tensor &num_cells,
@@ -278,17 +299,85 @@ std::tuple<Tensor, Tensor, bool> find_neighbors(const Tensor &samples, const Ten
   return {ranges, neighbors, symmetric};
 }
 
-// The pair table regrouped for centres in the order `order` -> (ranges, neighbors).
-std::pair<Tensor, Tensor> reorder_neighbors(const Tensor &ranges, const Tensor &neighbors,
-                                            const Tensor &order) {
+// The same for the structures of pc.py, which hold the grid: its column table is optional (for
+// a small cloud it would need the grid's shape on the host first).
+// -> (ranges, neighbors, whether a neighbourhood was cut at max_neighs)
+std::tuple<Tensor, Tensor, bool> search(const Tensor &samples, const Tensor &sbids,
+                                        const Tensor &points, const Tensor &keys,
+                                        const OptTensor &ds, const Tensor &num_cells,
+                                        const Tensor &smin, const Tensor &inv_cell,
+                                        const Tensor &inv_radii, int64_t max_neighs) {
+  const int64_t ns = samples.size(0);
+  const int nd = (int)dim(samples, 1);
+  Tensor ws = workspace(mccnn_find_neighbors_workspace_bytes(nd, ns), samples);
+  Tensor ranges = empty_i32({ns}, samples);
+  hipStream_t s = current_stream();
+  PinnedBlock host;
+  {
+    Region r("find_neighbors_count", s);
+    check(mccnn_search_count(s, ns, nd, f32(samples), i32(sbids), points.size(0), f32(points),
+                             i64(keys), i32(opt(ds)), i32(num_cells), f32(smin), f32(inv_cell),
+                             f32(inv_radii), (int)max_neighs, ws.data_ptr(), ws.numel(),
+                             i32(ranges), host.words()));
+  }
+  const int64_t m = host.words()[0];
+  const bool cut = host.words()[1] != 0;
+  Tensor neighbors = empty_i32({m, 2}, samples);
+  Region r("find_neighbors_fill", s);
+  check(mccnn_find_neighbors_fill(s, ns, nd, f32(samples), i32(sbids), points.size(0), f32(points),
+                                  i64(keys), nullptr, i32(num_cells), f32(smin), f32(inv_cell),
+                                  f32(inv_radii), (int)max_neighs, ws.data_ptr(), ws.numel(),
+                                  i32(ranges), m, i32(neighbors)));
+  return {ranges, neighbors, cut};
+}
+
+Tensor grid_density(const Tensor &points, const Tensor &bids, const Tensor &keys,
+                    const OptTensor &ds, const Tensor &num_cells, const Tensor &smin,
+                    const Tensor &inv_cell, const Tensor &inv_radii, const Tensor &inv_bandwidth,
+                    int64_t mode) {
+  const int64_t n = points.size(0);
+  const int nd = (int)dim(points, 1);
+  Tensor ws = workspace(mccnn_grid_density_workspace_bytes(nd, n), points);
+  Tensor pdf = empty_f32({n}, points);
+  hipStream_t s = current_stream();
+  Region r("compute_pdf", s);
+  check(mccnn_grid_density(s, n, nd, f32(points), i32(bids), i64(keys), i32(opt(ds)),
+                           i32(num_cells), f32(smin), f32(inv_cell), f32(inv_radii),
+                           f32(inv_bandwidth), (int)mode, ws.data_ptr(), ws.numel(), f32(pdf)));
+  return pdf;
+}
+
+// Columns of the pair table regrouped for centres in the order `order`: the end offsets, the
+// pairs (point indices through `map` if given), the density of every pair's point.
+Tensor reorder_ranges(const Tensor &ranges, const Tensor &order) {
   const int64_t n = ranges.size(0);
-  Tensor ws = workspace(mccnn_reorder_neighbors_workspace_bytes(n), neighbors);
-  Tensor ranges_out = empty_i32({n}, ranges), out = empty_i32(neighbors.sizes(), neighbors);
+  Tensor ws = workspace(mccnn_reorder_neighbors_workspace_bytes(n), ranges);
+  Tensor out = empty_i32({n}, ranges);
   hipStream_t s = current_stream();
   Region r("reorder_neighbors", s);
-  check(mccnn_reorder_neighbors(s, n, i32(ranges), neighbors.size(0), i32(neighbors), i32(order),
-                                ws.data_ptr(), ws.numel(), i32(ranges_out), i32(out)));
-  return {ranges_out, out};
+  check(mccnn_reorder_ranges(s, n, i32(ranges), i32(order), ws.data_ptr(), ws.numel(), i32(out)));
+  return out;
+}
+
+Tensor reorder_pairs(const Tensor &ranges, const Tensor &neighbors, const Tensor &order,
+                     const Tensor &ranges_out, const OptTensor &map) {
+  Tensor out = empty_i32(neighbors.sizes(), neighbors);
+  hipStream_t s = current_stream();
+  Region r("reorder_neighbors", s);
+  check(mccnn_reorder_pairs(s, ranges.size(0), i32(ranges), neighbors.size(0), i32(neighbors),
+                            i32(order), i32(ranges_out), i32(opt(map)), i32(out), nullptr,
+                            nullptr));
+  return out;
+}
+
+Tensor reorder_pdf(const Tensor &ranges, const Tensor &neighbors, const Tensor &order,
+                   const Tensor &ranges_out, const Tensor &pdf) {
+  Tensor out = empty_f32({neighbors.size(0)}, neighbors);
+  hipStream_t s = current_stream();
+  Region r("gather_pdf", s);
+  check(mccnn_reorder_pairs(s, ranges.size(0), i32(ranges), neighbors.size(0), i32(neighbors),
+                            i32(order), i32(ranges_out), nullptr, nullptr, f32(pdf), f32(out)));
+  return out;
 }
 
 Tensor original_neighbor_ids(const Tensor &neighbors, const Tensor &sorted_indices) {
@@ -950,11 +1039,16 @@ PYBIND11_MODULE(_host, m) {
   m.def("start_timing", &start_timing);
   m.def("collect_timing", &collect_timing);
   m.def("compute_keys", &compute_keys, release());
-  m.def("sort_keys", &sort_keys, release());
+  m.def("order_centres", &order_centres, release());
+  m.def("invert_order", &invert_order, release());
   m.def("build_grid", &build_grid, release());
   m.def("build_grid_ds", &build_grid_ds, release());
   m.def("find_neighbors", &find_neighbors, release());
-  m.def("reorder_neighbors", &reorder_neighbors, release());
+  m.def("search", &search, release());
+  m.def("grid_density", &grid_density, release());
+  m.def("reorder_ranges", &reorder_ranges, release());
+  m.def("reorder_pairs", &reorder_pairs, release());
+  m.def("reorder_pdf", &reorder_pdf, release());
   m.def("original_neighbor_ids", &original_neighbor_ids, release());
   m.def("transpose_neighbors", &transpose_neighbors, release());
   m.def("swapped_pairs", &swapped_pairs, release());

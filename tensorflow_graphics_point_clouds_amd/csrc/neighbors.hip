@@ -16,9 +16,10 @@
 // (Keeping the count pass's hit masks for the fill pass, so that it need not load
 // and test the candidates again, was measured: what the count pass loses by
 // storing them is what the fill pass gains, and crowded centres, whose masks do
-// not fit a fixed budget, pay for both.  Letting the count pass find its slices
-// itself, 9 of a group's 16 lanes searching, saves a launch and was no faster
-// either.)
+// not fit a fixed budget, pay for both.)
+// Small inputs are bound by launches: there the count pass finds its slices itself (every
+// lane of a group searches one or two), and a grid without a column table, which would need
+// the grid's shape on the host first, is searched over all of its keys.
 // Compiled with -ffp-contract=off (the distance test decides integer output).
 #include "common.h"
 #include "fill.h"
@@ -44,116 +45,130 @@ struct OffsetInfo {
   }
 };
 
+// What a search needs of the grid, per dimension in registers.
+template <int D>
+struct SearchGrid {
+  GridShape<D> g;
+  float ic[D], rho[D];                 // rho: one cell in units of the radius
+  __device__ __forceinline__ SearchGrid(const int *__restrict__ num_cells,
+                                        const float *__restrict__ inv_cell,
+                                        const float *__restrict__ inv_radii)
+      : g(load_shape<D>(num_cells)) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      ic[d] = inv_cell[d];
+      rho[d] = inv_radii[d] / ic[d];
+    }
+  }
+};
+
+// The slice of sorted points in cell row r of the neighbourhood of point p (cloud b).  `ds` is
+// the column table, or null: then the whole key array [0, np) is searched.
+template <int D>
+__device__ __forceinline__ int2 cell_row_slice(const SearchGrid<D> &sg, const float *p, int b,
+                                               int r, int64_t np, const int64_t *__restrict__ keys,
+                                               const int2 *__restrict__ ds,
+                                               const float *__restrict__ smin) {
+  constexpr int OD = OffsetInfo<D>::kDims;
+  const GridShape<D> &g = sg.g;
+  float m[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) m[d] = smin[(int64_t)b * D + d];
+  int cell[D];
+  cell_of_point<D>(p, m, sg.ic, g, cell);
+  // The centre in cell units, as the keys were computed, and what rounding can have
+  // moved a point across a cell face: a point filed under cell x has a true
+  // coordinate within `slack` of [x, x + 1) (outermost cells: unbounded outwards).
+  float rel[D], slack[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const float prod = p[d] * sg.ic[d];
+    rel[d] = prod - m[d];
+    slack[d] = 9.6e-7f * (fabsf(prod) + fabsf(m[d]) + 1.0f);       // 8 float epsilons
+  }
+  // offset digits, most significant = dim 0, value 1 - digit (descending); g2 = lower
+  // bound of the squared scaled distance to any point of the offset cell row, taken
+  // over the offset dimensions
+  bool inside = true;
+  float g2 = 0.0f;
+#pragma unroll
+  for (int d = OD - 1; d >= 0; --d) {
+    const int off = 1 - (r % 3);
+    r /= 3;
+    float gap = off < 0 ? rel[d] - (float)cell[d]
+                        : (off > 0 ? (float)(cell[d] + 1) - rel[d] : 0.0f);
+    gap = fmaxf(gap - slack[d], 0.0f) * sg.rho[d];
+    g2 += gap * gap;
+    cell[d] += off;
+    inside = inside && cell[d] >= 0 && cell[d] < g.n[d];
+  }
+  // Cells that no pair of the exact test can come from are left out: every candidate
+  // dropped here has a scaled distance of at least sqrt(1 + 1e-5) > 1, whatever the
+  // rounding of the test itself (a few 1e-7), so the pairs found do not change.
+  g2 *= 0.99999f;
+  if (!inside || !(g2 < 1.0f)) return make_int2(0, 0);
+  int2 span = make_int2(0, (int)np);
+  if (ds) span = ds[((int64_t)b * g.n[0] + cell[0]) * g.n[1] + cell[1]];
+  if (span.y <= span.x) return make_int2(0, 0);
+  if (D == 2 && ds) return span;
+  const int64_t aux = key_of_cell<D>(cell, g, b);
+  int64_t maxk = aux, mink = aux;
+  if (D > 2) {
+    const int w = cell[D - 1], nw = g.n[D - 1];
+    // last dimension: the cells w - 1 .. w + 1 of the reference, cut to those the
+    // sphere can reach given the offset in the other dimensions (out-of-range
+    // coordinates belong to the outermost cells)
+    const float reach = sqrtf(1.0f - g2) / sg.rho[D - 1] * 1.00001f + slack[D - 1];
+    int wlo = (int)floorf(fmaxf(rel[D - 1] - reach, -1.0f));
+    int whi = (int)floorf(fminf(rel[D - 1] + reach, (float)nw));
+    wlo = wlo < 0 ? 0 : (wlo > nw - 1 ? nw - 1 : wlo);
+    whi = whi < 0 ? 0 : (whi > nw - 1 ? nw - 1 : whi);
+    wlo = wlo > w - 1 ? wlo : (w > 0 ? w - 1 : 0);
+    whi = whi < w + 1 ? whi : (w < nw - 1 ? w + 1 : nw - 1);
+    if (whi < wlo) return make_int2(0, 0);
+    maxk = aux + (whi - w);
+    mink = aux + (wlo - w);
+  }
+  int lo = span.x, hi = span.y;
+  while (lo < hi) {                       // first index with key <= maxk
+    const int mid = lo + ((hi - lo) >> 1);
+    if (keys[mid] > maxk) lo = mid + 1; else hi = mid;
+  }
+  const int first = lo;
+  hi = span.y;
+  while (lo < hi) {                       // first index with key < mink
+    const int mid = lo + ((hi - lo) >> 1);
+    if (keys[mid] >= mink) lo = mid + 1; else hi = mid;
+  }
+  return lo > first ? make_int2(first, lo) : make_int2(0, 0);
+}
+
 template <int D>
 __global__ void __launch_bounds__(256) nbr_ranges_kernel(
-    int64_t ns, const float *__restrict__ samples, const int *__restrict__ sbids,
+    int64_t ns, const float *__restrict__ samples, const int *__restrict__ sbids, int64_t np,
     const int64_t *__restrict__ keys, const int2 *__restrict__ ds,
     const int *__restrict__ num_cells, const float *__restrict__ smin,
     const float *__restrict__ inv_cell, const float *__restrict__ inv_radii,
     int2 *__restrict__ ranges) {
   constexpr int R = OffsetInfo<D>::count();
-  constexpr int OD = OffsetInfo<D>::kDims;
-  const GridShape<D> g = load_shape<D>(num_cells);
-  float ic[D], rho[D];                 // rho: one cell in units of the radius
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    ic[d] = inv_cell[d];
-    rho[d] = inv_radii[d] / ic[d];
-  }
+  const SearchGrid<D> sg(num_cells, inv_cell, inv_radii);
   const int64_t total = ns * R;
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
        t += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = t / R;
-    int r = (int)(t - c * R);
-    const int b = sbids[c];
-    float p[D], m[D];
+    float p[D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      p[d] = samples[c * D + d];
-      m[d] = smin[(int64_t)b * D + d];
-    }
-    int cell[D];
-    cell_of_point<D>(p, m, ic, g, cell);
-    // The centre in cell units, as the keys were computed, and what rounding can have
-    // moved a point across a cell face: a point filed under cell x has a true
-    // coordinate within `slack` of [x, x + 1) (outermost cells: unbounded outwards).
-    float rel[D], slack[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const float prod = p[d] * ic[d];
-      rel[d] = prod - m[d];
-      slack[d] = 9.6e-7f * (fabsf(prod) + fabsf(m[d]) + 1.0f);       // 8 float epsilons
-    }
-    // offset digits, most significant = dim 0, value 1 - digit (descending); g2 = lower
-    // bound of the squared scaled distance to any point of the offset cell row, taken
-    // over the offset dimensions
-    bool inside = true;
-    float g2 = 0.0f;
-#pragma unroll
-    for (int d = OD - 1; d >= 0; --d) {
-      const int off = 1 - (r % 3);
-      r /= 3;
-      float gap = off < 0 ? rel[d] - (float)cell[d]
-                          : (off > 0 ? (float)(cell[d] + 1) - rel[d] : 0.0f);
-      gap = fmaxf(gap - slack[d], 0.0f) * rho[d];
-      g2 += gap * gap;
-      cell[d] += off;
-      inside = inside && cell[d] >= 0 && cell[d] < g.n[d];
-    }
-    // Cells that no pair of the exact test can come from are left out: every candidate
-    // dropped here has a scaled distance of at least sqrt(1 + 1e-5) > 1, whatever the
-    // rounding of the test itself (a few 1e-7), so the pairs found do not change.
-    g2 *= 0.99999f;
-    inside = inside && g2 < 1.0f;
-    int2 out = make_int2(0, 0);
-    if (inside) {
-      const int64_t col = ((int64_t)b * g.n[0] + cell[0]) * g.n[1] + cell[1];
-      const int2 span = ds[col];
-      if (span.y > span.x) {
-        if (D == 2) {
-          out = span;
-        } else {
-          const int64_t aux = key_of_cell<D>(cell, g, b);
-          const int w = cell[D - 1], nw = g.n[D - 1];
-          // last dimension: the cells w - 1 .. w + 1 of the reference, cut to those the
-          // sphere can reach given the offset in the other dimensions (out-of-range
-          // coordinates belong to the outermost cells)
-          const float reach = sqrtf(1.0f - g2) / rho[D - 1] * 1.00001f + slack[D - 1];
-          int wlo = (int)floorf(fmaxf(rel[D - 1] - reach, -1.0f));
-          int whi = (int)floorf(fminf(rel[D - 1] + reach, (float)nw));
-          wlo = wlo < 0 ? 0 : (wlo > nw - 1 ? nw - 1 : wlo);
-          whi = whi < 0 ? 0 : (whi > nw - 1 ? nw - 1 : whi);
-          wlo = wlo > w - 1 ? wlo : (w > 0 ? w - 1 : 0);
-          whi = whi < w + 1 ? whi : (w < nw - 1 ? w + 1 : nw - 1);
-          const int64_t maxk = aux + (whi - w);
-          const int64_t mink = aux + (wlo - w);
-          int lo = span.x, hi = span.y;
-          while (lo < hi) {                       // first index with key <= maxk
-            const int mid = lo + ((hi - lo) >> 1);
-            if (keys[mid] > maxk) lo = mid + 1; else hi = mid;
-          }
-          const int first = lo;
-          hi = span.y;
-          while (lo < hi) {                       // first index with key < mink
-            const int mid = lo + ((hi - lo) >> 1);
-            if (keys[mid] >= mink) lo = mid + 1; else hi = mid;
-          }
-          if (lo > first && whi >= wlo) out = make_int2(first, lo);
-        }
-      }
-    }
-    ranges[t] = out;
+    for (int d = 0; d < D; ++d) p[d] = samples[c * D + d];
+    ranges[t] = cell_row_slice<D>(sg, p, sbids[c], (int)(t - c * R), np, keys, ds, smin);
   }
 }
 
 template <int D>
-__device__ __forceinline__ bool within_radius(const float *s, const float *__restrict__ pts,
-                                              int64_t j, const float *ir) {
+__device__ __forceinline__ bool within_radius(const float *diff, const float *ir) {
   float acc = 0.0f;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    const float diff = s[d] - pts[j * D + d];
-    const float sc = diff * ir[d];
+    const float sc = diff[d] * ir[d];
     const float sq = sc * sc;
     acc = acc + sq;
   }
@@ -165,14 +180,31 @@ __device__ __forceinline__ bool within_radius(const float *s, const float *__res
   return acc < 1.0f;
 }
 
-// kFill == false: counts[c] = number of hits (clamped to max_neighs when > 0).
-// kFill == true : writes the pairs of centre c starting at its start offset.
-template <int D, bool kFill>
+// What a visit of a centre's candidates produces.
+enum class Visit {
+  kCount,      // counts[c] = number of hits (clamped to max_neighs when > 0)
+  kFill,       // the pairs of centre c from its start offset on
+  kDensity,    // density[c]: the kernel density of centre c over its hits (compute_pdf)
+};
+
+struct VisitSearch {                  // for kSearch: the grid to find the slices in
+  const int *sbids;
+  int64_t np;
+  const int64_t *keys;
+  const int2 *ds;
+  const int *num_cells;
+  const float *smin, *inv_cell;
+};
+
+// kSearch: the lanes of a group find the centre's slices themselves (kCount also stores them
+// for the fill pass); otherwise `ranges` holds them.
+template <int D, Visit kVisit, bool kSearch>
 __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
     int64_t ns, const float *__restrict__ samples, const float *__restrict__ pts,
-    const int2 *__restrict__ ranges, const float *__restrict__ inv_radii, int max_neighs,
+    int2 *ranges, const float *__restrict__ inv_radii, int max_neighs, VisitSearch search,
     int *__restrict__ counts, const int *__restrict__ ends, int2 *__restrict__ nbrs,
-    int64_t *__restrict__ truncated = nullptr, int64_t capacity = ((int64_t)1 << 62)) {
+    int64_t *__restrict__ truncated, int64_t capacity, const float *__restrict__ inv_bandwidth,
+    int mode, float *__restrict__ density) {
   constexpr int R = OffsetInfo<D>::count();
   const int sub = threadIdx.x & (kGroup - 1);
   const int lane = lane_id();
@@ -189,30 +221,63 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
   const int limit = max_neighs > 0 ? max_neighs : 0x7fffffff;
   int found = 0;                                   // kFill: slots used so far
   int64_t start = 0;
-  if (kFill) start = c > 0 ? ends[c - 1] : 0;
-  // the slices of the centre, kGroup at a time: lane `sub` fetches one, the group then
-  // takes them in turn (one round trip to memory instead of one per slice)
+  if (kVisit == Visit::kFill) start = c > 0 ? ends[c - 1] : 0;
+  float scale[D], norm = 1.0f, sum = 0.0f;         // kDensity, as compute_pdf (pdf.hip)
+  if (kVisit == Visit::kDensity) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const float bw = mode == 0 ? inv_bandwidth[d] : sqrtf((float)ns);
+      scale[d] = bw * ir[d];
+      norm *= bw * 0.39894228f;
+    }
+  }
+  // the slices of the centre, kGroup at a time: lane `sub` fetches (or finds) one, the group
+  // then takes them in turn (one round trip to memory instead of one per slice)
   for (int r0 = 0; r0 < R; r0 += kGroup) {
-    const int2 mine = r0 + sub < R ? ranges[c * R + r0 + sub] : make_int2(0, 0);
+    int2 mine = make_int2(0, 0);
+    if (r0 + sub < R) {
+      if constexpr (kSearch) {
+        const SearchGrid<D> sg(search.num_cells, search.inv_cell, inv_radii);
+        mine = cell_row_slice<D>(sg, s, search.sbids[c], r0 + sub, search.np, search.keys,
+                                 search.ds, search.smin);
+        if (kVisit == Visit::kCount) ranges[c * R + r0 + sub] = mine;
+      } else {
+        mine = ranges[c * R + r0 + sub];
+      }
+    }
     const int lim = R - r0 < kGroup ? R - r0 : kGroup;
     for (int r = 0; r < lim; ++r) {
       const int2 span = make_int2(__shfl(mine.x, r, kGroup), __shfl(mine.y, r, kGroup));
       for (int j0 = span.x; j0 < span.y; j0 += kGroup) {
         const int j = j0 + sub;
-        const bool hit = j < span.y && within_radius<D>(s, pts, j, ir);
-        if (kFill) {
+        bool hit = false;
+        float diff[D];
+        if (j < span.y) {
+#pragma unroll
+          for (int d = 0; d < D; ++d) diff[d] = s[d] - pts[(int64_t)j * D + d];
+          hit = within_radius<D>(diff, ir);
+        }
+        if (kVisit == Visit::kFill) {
           const uint64_t hits = __ballot(hit) & group_mask;
           const int slot = found + __popcll(hits & below_mask);
           if (hit && slot < limit && start + slot < capacity)
             nbrs[start + slot] = make_int2(j, (int)c);
           found += __popcll(hits);
-        } else {
+        } else if (kVisit == Visit::kCount) {
           found += hit ? 1 : 0;
+        } else if (hit) {
+          float e = 0.0f;
+#pragma unroll
+          for (int d = 0; d < D; ++d) {
+            const float u = diff[d] * scale[d];
+            e += u * u;
+          }
+          sum += expf(-0.5f * e);
         }
       }
     }
   }
-  if (!kFill) {
+  if (kVisit == Visit::kCount) {
 #pragma unroll
     for (int off = kGroup / 2; off > 0; off >>= 1) found += __shfl_xor(found, off, kWave);
     if (sub == 0) {
@@ -221,7 +286,17 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
       if (truncated && found > limit) *truncated = 1;
     }
   }
+  if (kVisit == Visit::kDensity) {
+#pragma unroll
+    for (int off = kGroup / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
+    if (sub == 0) density[c] = sum * norm;
+  }
 }
+
+// Centres up to which the count pass finds its slices itself: 16 384 centres are 512 blocks,
+// one launch of latency; beyond that the searches of a group's lanes (nine slices, eight
+// lanes) cost more than a launch of one lane per slice (763 k centres: 88 us for the slices).
+constexpr int64_t kSearchInVisit = 16384;
 
 struct NbrWorkspace {
   int2 *ranges;
@@ -262,18 +337,24 @@ __global__ void __launch_bounds__(256) segment_counts_kernel(int64_t n, const in
   counts[q] = ranges[i] - (i > 0 ? ranges[i - 1] : 0);
 }
 
-__global__ void __launch_bounds__(256) segment_copy_kernel(int64_t n, const int *__restrict__ ranges,
-                                                           const int *__restrict__ order,
-                                                           const int2 *__restrict__ pairs,
-                                                           const int *__restrict__ ranges_out,
-                                                           int2 *__restrict__ pairs_out) {
+// `map` (optional) replaces the point index by map[index]; either output may be null, pdf_out
+// takes the density of the pair's point.
+__global__ void __launch_bounds__(256) segment_copy_kernel(
+    int64_t n, const int *__restrict__ ranges, const int *__restrict__ order,
+    const int2 *__restrict__ pairs, const int *__restrict__ ranges_out,
+    const int *__restrict__ map, int2 *__restrict__ pairs_out, const float *__restrict__ pdf,
+    float *__restrict__ pdf_out) {
   const int64_t q = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
   if (q >= n) return;
   const int sub = threadIdx.x & 15;
   const int i = order[q];
   const int src = i > 0 ? ranges[i - 1] : 0, cnt = ranges[i] - src;
   const int dst = ranges_out[q] - cnt;
-  for (int t = sub; t < cnt; t += 16) pairs_out[dst + t] = make_int2(pairs[src + t].x, (int)q);
+  for (int t = sub; t < cnt; t += 16) {
+    const int j = pairs[src + t].x;
+    if (pairs_out) pairs_out[dst + t] = make_int2(map ? map[j] : j, (int)q);
+    if (pdf_out) pdf_out[dst + t] = pdf[j];
+  }
 }
 
 }  // namespace mccnn
@@ -283,6 +364,42 @@ using namespace mccnn;
 extern "C" size_t mccnn_find_neighbors_workspace_bytes(int num_dims, int64_t num_samples) {
   if (!valid_dims(num_dims) || num_samples < 0) return 0;
   return carve_nbr_workspace(nullptr, num_dims, num_samples).bytes;
+}
+
+static int launch_count(hipStream_t s, int num_dims, int64_t ns, const float *samples,
+                        const float *points, int2 *slices, const float *inv_radii, int max_neighs,
+                        const VisitSearch *search, int *counts, int64_t *truncated) {
+  const dim3 grid(blocks_for(ns, kCentresPerBlock)), block(kNbrThreads);
+  if (search)
+    MCCNN_DIM_SWITCH(num_dims,
+                     hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kCount, true>), grid, block, 0,
+                                        s, ns, samples, points, slices, inv_radii, max_neighs,
+                                        *search, counts, (const int *)nullptr, (int2 *)nullptr,
+                                        truncated, (int64_t)0, (const float *)nullptr, 0,
+                                        (float *)nullptr))
+  else
+    MCCNN_DIM_SWITCH(num_dims,
+                     hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kCount, false>), grid, block,
+                                        0, s, ns, samples, points, slices, inv_radii, max_neighs,
+                                        VisitSearch{}, counts, (const int *)nullptr,
+                                        (int2 *)nullptr, truncated, (int64_t)0,
+                                        (const float *)nullptr, 0, (float *)nullptr))
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
+static int launch_fill(hipStream_t s, int num_dims, int64_t ns, const float *samples,
+                       const float *points, int2 *slices, const float *inv_radii, int max_neighs,
+                       const int *ends, int32_t *neighbors, int64_t capacity) {
+  MCCNN_DIM_SWITCH(num_dims,
+                   hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kFill, false>),
+                                      dim3(blocks_for(ns, kCentresPerBlock)), dim3(kNbrThreads), 0,
+                                      s, ns, samples, points, slices, inv_radii, max_neighs,
+                                      VisitSearch{}, (int *)nullptr, ends, (int2 *)neighbors,
+                                      (int64_t *)nullptr, capacity, (const float *)nullptr, 0,
+                                      (float *)nullptr));
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
 }
 
 // `facts_out_host` (optional, two values): [0] 1 if some centre lost pairs to max_neighs,
@@ -344,25 +461,21 @@ static int find_neighbors_count_impl(
   const int64_t work = num_samples * offsets_for(num_dims);
   MCCNN_DIM_SWITCH(num_dims,
                    hipLaunchKernelGGL(nbr_ranges_kernel<D>, dim3(blocks_for(work, 256)), dim3(256),
-                                      0, s, num_samples, samples, sample_batch_ids,
+                                      0, s, num_samples, samples, sample_batch_ids, num_pts,
                                       (const int64_t *)point_keys, (const int2 *)grid_ds,
                                       num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
                                       w.ranges));
   MCCNN_LAUNCH_CHECK();
-  const unsigned grid = blocks_for(num_samples, kCentresPerBlock);
   // truncation can only happen with max_neighs > 0: only then is the flag cleared and read
   int64_t *truncated = facts_out_host && max_neighs > 0 ? w.total + 1 : nullptr;
   if (truncated) {
     int rc0 = fill_zero(s, truncated, sizeof(int64_t));
     if (rc0 != MCCNN_OK) return rc0;
   }
-  MCCNN_DIM_SWITCH(num_dims, hipLaunchKernelGGL((nbr_visit_kernel<D, false>), dim3(grid),
-                                                dim3(kNbrThreads), 0, s, num_samples, samples,
-                                                points, (const int2 *)w.ranges, inv_radii,
-                                                max_neighs, ranges_out, (const int *)nullptr,
-                                                (int2 *)nullptr, truncated));
-  MCCNN_LAUNCH_CHECK();
-  int rc = inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, w.total);
+  int rc = launch_count(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
+                        nullptr, ranges_out, truncated);
+  if (rc != MCCNN_OK) return rc;
+  rc = inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, w.total);
   if (rc != MCCNN_OK) return rc;
   if (!to_host) return MCCNN_OK;
   MCCNN_HIP_CHECK(hipMemcpyAsync(num_neighbors_out_host, w.total, sizeof(int64_t),
@@ -431,14 +544,8 @@ extern "C" int mccnn_find_neighbors_fill(
   const NbrWorkspace w = carve_nbr_workspace(workspace, num_dims, num_samples);
   MCCNN_REQUIRE(workspace_bytes >= w.bytes, "FindNeighbors workspace too small (%zu < %zu)",
                 workspace_bytes, w.bytes);
-  const unsigned grid = blocks_for(num_samples, kCentresPerBlock);
-  MCCNN_DIM_SWITCH(num_dims, hipLaunchKernelGGL((nbr_visit_kernel<D, true>), dim3(grid),
-                                                dim3(kNbrThreads), 0, as_stream(stream),
-                                                num_samples, samples, points,
-                                                (const int2 *)w.ranges, inv_radii, max_neighs,
-                                                (int *)nullptr, ranges, (int2 *)neighbors_out));
-  MCCNN_LAUNCH_CHECK();
-  return MCCNN_OK;
+  return launch_fill(as_stream(stream), num_dims, num_samples, samples, points, w.ranges, inv_radii,
+                     max_neighs, ranges, neighbors_out, (int64_t)1 << 62);
 }
 
 // count_out[0] = pairs found, count_out[1] = 1 if they do not fit the capacity
@@ -474,13 +581,115 @@ extern "C" int mccnn_find_neighbors_bounded(
                      count_out_device);
   MCCNN_LAUNCH_CHECK();
   if (capacity == 0) return MCCNN_OK;
-  const unsigned grid = blocks_for(num_samples, kCentresPerBlock);
-  MCCNN_DIM_SWITCH(num_dims, hipLaunchKernelGGL((nbr_visit_kernel<D, true>), dim3(grid),
-                                                dim3(kNbrThreads), 0, s, num_samples, samples,
-                                                points, (const int2 *)w.ranges, inv_radii,
-                                                max_neighs, (int *)nullptr, ranges_out,
-                                                (int2 *)neighbors_out, (int64_t *)nullptr,
-                                                capacity));
+  return launch_fill(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
+                     ranges_out, neighbors_out, capacity);
+}
+
+// The count half of a search by a caller that has the grid in hand (no argument checks beyond
+// sizes and null pointers), with or without the grid's column table, and with the outcome in
+// pinned host memory.
+extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                                  const float *samples, const int32_t *sample_batch_ids,
+                                  int64_t num_pts, const float *points, const int64_t *point_keys,
+                                  const int32_t *grid_ds, const int32_t *num_cells,
+                                  const float *scaled_aabb_min, const float *inv_cell_sizes,
+                                  const float *inv_radii, int max_neighs, void *workspace,
+                                  size_t workspace_bytes, int32_t *ranges_out,
+                                  int64_t *result_pinned) {
+  MCCNN_REQUIRE(valid_dims(num_dims), "search_count expects a valid number of dimensions");
+  MCCNN_REQUIRE(num_samples >= 0 && num_pts >= 0 && num_samples < ((int64_t)1 << 31) &&
+                    num_pts < ((int64_t)1 << 31),
+                "search_count expects sizes in [0, 2^31)");
+  MCCNN_REQUIRE(result_pinned, "search_count received a null output");
+  result_pinned[0] = result_pinned[1] = 0;
+  if (num_samples == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(samples && sample_batch_ids && num_cells && scaled_aabb_min && inv_cell_sizes &&
+                    inv_radii && ranges_out && workspace && (num_pts == 0 || (points && point_keys)),
+                "search_count received a null tensor");
+  const NbrWorkspace w = carve_nbr_workspace(workspace, num_dims, num_samples);
+  MCCNN_REQUIRE(workspace_bytes >= w.bytes, "search_count workspace too small (%zu < %zu)",
+                workspace_bytes, w.bytes);
+  hipStream_t s = as_stream(stream);
+  const bool in_visit = num_samples <= kSearchInVisit;
+  const VisitSearch search = {sample_batch_ids, num_pts, (const int64_t *)point_keys,
+                              (const int2 *)grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes};
+  if (!in_visit) {
+    MCCNN_DIM_SWITCH(num_dims,
+                     hipLaunchKernelGGL(nbr_ranges_kernel<D>,
+                                        dim3(blocks_for(num_samples * offsets_for(num_dims), 256)),
+                                        dim3(256), 0, s, num_samples, samples, sample_batch_ids,
+                                        num_pts, (const int64_t *)point_keys, (const int2 *)grid_ds,
+                                        num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
+                                        w.ranges));
+    MCCNN_LAUNCH_CHECK();
+  }
+  int rc = launch_count(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
+                        in_visit ? &search : nullptr, ranges_out,
+                        max_neighs > 0 ? result_pinned + 1 : nullptr);
+  if (rc != MCCNN_OK) return rc;
+  rc = inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, result_pinned);
+  if (rc != MCCNN_OK) return rc;
+  MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+  MCCNN_REQUIRE(result_pinned[0] < (((int64_t)1 << 31) - 1),
+                "FindNeighbors found at least %lld pairs; the int32 offsets of the op contract "
+                "hold fewer than 2^31 - 1",
+                (long long)result_pinned[0]);
+  return MCCNN_OK;
+}
+
+extern "C" size_t mccnn_grid_density_workspace_bytes(int num_dims, int64_t num_pts) {
+  if (!valid_dims(num_dims) || num_pts < 0) return 0;
+  return num_pts <= kSearchInVisit ? 256
+                                   : align256(sizeof(int2) * (size_t)num_pts * offsets_for(num_dims));
+}
+
+// Kernel density of the grid's own points straight from the grid: what compute_pdf gives on the
+// pair table of the points among themselves, without the table (its count, the host round trip
+// for its size, the 8 bytes per pair written and read).
+extern "C" int mccnn_grid_density(mccnn_stream_t stream, int64_t num_pts, int num_dims,
+                                  const float *points, const int32_t *batch_ids,
+                                  const int64_t *point_keys, const int32_t *grid_ds,
+                                  const int32_t *num_cells, const float *scaled_aabb_min,
+                                  const float *inv_cell_sizes, const float *inv_radii,
+                                  const float *inv_bandwidth, int mode, void *workspace,
+                                  size_t workspace_bytes, float *pdf_out) {
+  MCCNN_REQUIRE(valid_dims(num_dims), "grid_density expects a valid number of dimensions");
+  MCCNN_REQUIRE(mode == 0 || mode == 1, "grid_density expects mode 0 or 1");
+  MCCNN_REQUIRE(num_pts >= 0 && num_pts < ((int64_t)1 << 31), "grid_density expects a size in [0, 2^31)");
+  if (num_pts == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(points && batch_ids && point_keys && num_cells && scaled_aabb_min &&
+                    inv_cell_sizes && inv_radii && inv_bandwidth && workspace && pdf_out,
+                "grid_density received a null tensor");
+  MCCNN_REQUIRE(workspace_bytes >= mccnn_grid_density_workspace_bytes(num_dims, num_pts),
+                "grid_density workspace too small");
+  hipStream_t s = as_stream(stream);
+  int2 *slices = (int2 *)workspace;
+  const VisitSearch search = {batch_ids, num_pts, (const int64_t *)point_keys,
+                              (const int2 *)grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes};
+  const dim3 grid(blocks_for(num_pts, kCentresPerBlock)), block(kNbrThreads);
+  if (num_pts <= kSearchInVisit) {
+    MCCNN_DIM_SWITCH(num_dims,
+                     hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kDensity, true>), grid, block,
+                                        0, s, num_pts, points, points, slices, inv_radii, 0, search,
+                                        (int *)nullptr, (const int *)nullptr, (int2 *)nullptr,
+                                        (int64_t *)nullptr, (int64_t)0, inv_bandwidth, mode,
+                                        pdf_out));
+    MCCNN_LAUNCH_CHECK();
+    return MCCNN_OK;
+  }
+  MCCNN_DIM_SWITCH(num_dims,
+                   hipLaunchKernelGGL(nbr_ranges_kernel<D>,
+                                      dim3(blocks_for(num_pts * offsets_for(num_dims), 256)),
+                                      dim3(256), 0, s, num_pts, points, batch_ids, num_pts,
+                                      (const int64_t *)point_keys, (const int2 *)grid_ds, num_cells,
+                                      scaled_aabb_min, inv_cell_sizes, inv_radii, slices));
+  MCCNN_LAUNCH_CHECK();
+  MCCNN_DIM_SWITCH(num_dims,
+                   hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kDensity, false>), grid, block, 0,
+                                      s, num_pts, points, points, slices, inv_radii, 0,
+                                      VisitSearch{}, (int *)nullptr, (const int *)nullptr,
+                                      (int2 *)nullptr, (int64_t *)nullptr, (int64_t)0,
+                                      inv_bandwidth, mode, pdf_out));
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
@@ -503,6 +712,26 @@ extern "C" int mccnn_reorder_neighbors(mccnn_stream_t stream, int64_t num_sample
                 "reorder_neighbors received a null tensor");
   MCCNN_REQUIRE(workspace_bytes >= mccnn_reorder_neighbors_workspace_bytes(num_samples),
                 "reorder_neighbors workspace too small");
+  int rc = mccnn_reorder_ranges(stream, num_samples, ranges, centre_order, workspace,
+                                workspace_bytes, ranges_out);
+  if (rc != MCCNN_OK) return rc;
+  return mccnn_reorder_pairs(stream, num_samples, ranges, num_neighbors, neighbors, centre_order,
+                             ranges_out, nullptr, neighbors_out, nullptr, nullptr);
+}
+
+// The two halves by themselves: the end offsets of the regrouped table, and any of its columns
+// -- the pairs, the pairs with original point ids, the per-pair densities -- without the
+// regrouped table in memory first.
+extern "C" int mccnn_reorder_ranges(mccnn_stream_t stream, int64_t num_samples,
+                                    const int32_t *ranges, const int32_t *centre_order,
+                                    void *workspace, size_t workspace_bytes,
+                                    int32_t *ranges_out) {
+  MCCNN_REQUIRE(num_samples >= 0, "reorder_ranges expects a non-negative size");
+  if (num_samples == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(ranges && centre_order && ranges_out && workspace,
+                "reorder_ranges received a null tensor");
+  MCCNN_REQUIRE(workspace_bytes >= mccnn_reorder_neighbors_workspace_bytes(num_samples),
+                "reorder_ranges workspace too small");
   hipStream_t s = as_stream(stream);
   int *scratch = (int *)workspace;
   int64_t *total = (int64_t *)((char *)workspace +
@@ -510,12 +739,25 @@ extern "C" int mccnn_reorder_neighbors(mccnn_stream_t stream, int64_t num_sample
   hipLaunchKernelGGL(segment_counts_kernel, dim3(blocks_for(num_samples, 256)), dim3(256), 0, s,
                      num_samples, ranges, centre_order, ranges_out);
   MCCNN_LAUNCH_CHECK();
-  int rc = inclusive_scan_i32(s, num_samples, ranges_out, scratch, total);
-  if (rc != MCCNN_OK) return rc;
-  if (num_neighbors == 0) return MCCNN_OK;
-  hipLaunchKernelGGL(segment_copy_kernel, dim3(blocks_for(num_samples * 16, 256)), dim3(256), 0, s,
-                     num_samples, ranges, centre_order, (const int2 *)neighbors, ranges_out,
-                     (int2 *)neighbors_out);
+  return inclusive_scan_i32(s, num_samples, ranges_out, scratch, total);
+}
+
+extern "C" int mccnn_reorder_pairs(mccnn_stream_t stream, int64_t num_samples,
+                                   const int32_t *ranges, int64_t num_neighbors,
+                                   const int32_t *neighbors, const int32_t *centre_order,
+                                   const int32_t *ranges_out, const int32_t *point_map,
+                                   int32_t *neighbors_out, const float *pdf,
+                                   float *pdf_per_pair_out) {
+  MCCNN_REQUIRE(num_samples >= 0 && num_neighbors >= 0 && num_neighbors < ((int64_t)1 << 31),
+                "reorder_pairs expects sizes in [0, 2^31)");
+  if (num_samples == 0 || num_neighbors == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(ranges && neighbors && centre_order && ranges_out &&
+                    (neighbors_out || pdf_per_pair_out) && (!pdf_per_pair_out || pdf),
+                "reorder_pairs received a null tensor");
+  hipLaunchKernelGGL(segment_copy_kernel, dim3(blocks_for(num_samples * 16, 256)), dim3(256), 0,
+                     as_stream(stream), num_samples, ranges, centre_order,
+                     (const int2 *)neighbors, ranges_out, point_map, (int2 *)neighbors_out, pdf,
+                     pdf_per_pair_out);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }

@@ -4,28 +4,34 @@
 //
 // LSD radix sort, 8-bit digits, on the complemented digit so that ascending
 // digit order is descending key order while stability keeps equal keys in input
-// order.  Per pass: (1) per-tile digit histogram in LDS, written digit-major,
-// (2) prefix sum over [256 digits x tiles], (3) stable scatter: ranks inside a
-// tile come from wavefront ballots (matching lanes with the same digit) plus
-// per-wave LDS counters, never from atomics, so the order is deterministic.
+// order.  Three launches per pass: (1) per-tile digit histogram in LDS, written
+// digit-major, (2) one block per digit scans its row over the tiles, (3) stable scatter:
+// every block adds up the 256 row totals in front of its digits, ranks the tile's items --
+// wavefront w owns the w-th quarter of the tile, the rank among lanes with the same digit
+// comes from ballots, never from atomics, so the order is deterministic --, orders the tile
+// by digit in LDS and writes it out in runs (a tile of 2048 items has runs of about eight;
+// written in input order every lane is a memory transaction of its own).
+// The grid's keys travel as 32-bit words where they fit (they nearly always do), its
+// histogram of the first pass comes with the keys, and its last pass also gathers the points:
+// 763 k keys of 21 bits took 90 us with 64-bit keys, a scan of three launches per pass and a
+// separate gather.
 #include "common.h"
 #include "fill.h"
+#include "small_sort.h"
+#include "sort.h"
 
 namespace mccnn {
 
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 8;
-constexpr int kSortTile = kSortThreads * kSortItems;
-constexpr int kSortWaves = kSortThreads / kWave;
-constexpr int kRadix = 256;
-
-__device__ __forceinline__ int digit_of(int64_t key, int shift) {
-  return (int)((~(uint64_t)key >> shift) & (kRadix - 1));
+template <class K>
+__device__ __forceinline__ int digit_of(K key, int shift) {
+  return (int)((~key >> shift) & (K)(kSortRadix - 1));
 }
 
-__global__ void __launch_bounds__(kSortThreads) sort_hist_kernel(
-    int64_t n, int shift, int nb, const int64_t *__restrict__ keys, int *__restrict__ hist) {
-  __shared__ int bins[kRadix];
+template <class K>
+__global__ void __launch_bounds__(kSortThreads) sort_hist_kernel(int64_t n, int shift, int nb,
+                                                                 const K *__restrict__ keys,
+                                                                 int *__restrict__ hist) {
+  __shared__ int bins[kSortRadix];
   bins[threadIdx.x] = 0;
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * kSortTile;
@@ -38,173 +44,147 @@ __global__ void __launch_bounds__(kSortThreads) sort_hist_kernel(
   hist[(int64_t)threadIdx.x * nb + blockIdx.x] = bins[threadIdx.x];
 }
 
-// hist holds the INCLUSIVE prefix sums of the digit-major histogram.
-template <bool kFirstPass>
-__global__ void __launch_bounds__(kSortThreads) sort_scatter_kernel(
-    int64_t n, int shift, int nb, const int64_t *__restrict__ keys_in,
-    const int *__restrict__ idx_in, const int *__restrict__ hist,
-    int64_t *__restrict__ keys_out, int *__restrict__ idx_out) {
-  __shared__ int running[kRadix];              // items of each digit seen in earlier rounds
-  __shared__ int wcount[kSortWaves][kRadix];   // per wave, this round
+// Exclusive scan of 256 per-thread values over the block.
+__device__ __forceinline__ int block_exclusive_256(int v, int *wave_sums, int *total) {
   const int lane = lane_id(), wave = threadIdx.x / kWave;
-  running[threadIdx.x] = 0;
-#pragma unroll
-  for (int w = 0; w < kSortWaves; ++w) wcount[w][threadIdx.x] = 0;
+  const int incl = wave_inclusive_scan(v);
+  if (lane == kWave - 1) wave_sums[wave] = incl;
   __syncthreads();
-
-  const int64_t base = (int64_t)blockIdx.x * kSortTile;
-  int64_t key[kSortItems];
-  int rank[kSortItems];
+  int carry = 0, sum = 0;
 #pragma unroll
-  for (int k = 0; k < kSortItems; ++k) {
-    const int64_t i = base + k * kSortThreads + threadIdx.x;
-    const bool live = i < n;
-    key[k] = live ? keys_in[i] : 0;
-    const int d = digit_of(key[k], shift);
-    // lanes of this wave holding the same digit (dead lanes match nothing)
-    uint64_t same = __ballot(live);
-#pragma unroll
-    for (int bit = 0; bit < 8; ++bit) {
-      const uint64_t b = __ballot((d >> bit) & 1);
-      same &= ((d >> bit) & 1) ? b : ~b;
-    }
-    const int below = __popcll(same & ((1ull << lane) - 1ull));
-    if (live && below == 0) wcount[wave][d] = __popcll(same);
-    __syncthreads();
-    int r = running[d] + below;
-#pragma unroll
-    for (int w = 0; w < kSortWaves; ++w)
-      if (w < wave) r += wcount[w][d];
-    rank[k] = r;
-    __syncthreads();
-    {
-      int add = 0;
-#pragma unroll
-      for (int w = 0; w < kSortWaves; ++w) {
-        add += wcount[w][threadIdx.x];
-        wcount[w][threadIdx.x] = 0;
-      }
-      running[threadIdx.x] += add;
-    }
-    __syncthreads();
+  for (int w = 0; w < kSortThreads / kWave; ++w) {
+    carry += w < wave ? wave_sums[w] : 0;
+    sum += wave_sums[w];
   }
-  // running[d] is now this tile's count of digit d: global start of the tile's
-  // run of digit d = inclusive prefix - count.
-  const int start = hist[(int64_t)threadIdx.x * nb + blockIdx.x] - running[threadIdx.x];
   __syncthreads();
-  running[threadIdx.x] = start;
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < kSortItems; ++k) {
-    const int64_t i = base + k * kSortThreads + threadIdx.x;
-    if (i < n) {
-      const int d = digit_of(key[k], shift);
-      const int64_t dst = (int64_t)running[d] + rank[k];
-      keys_out[dst] = key[k];
-      idx_out[dst] = kFirstPass ? (int)i : idx_in[i];
-    }
-  }
+  *total = sum;
+  return carry + incl - v;
 }
 
-// The whole sort in one launch for small inputs (a cloud of a few thousand points: the
-// multi-block passes above cost five launches each, 36 us for three passes of 16 k keys,
-// nearly all of it launch latency).  One block of 16 wavefronts runs every pass; wavefront
-// w owns the w-th sixteenth of the input, fetched into registers at the start of the pass.
-// Counting sweep: digit counts per wavefront with LDS atomics (counts do not depend on the
-// order).  Then 256 threads turn the [digit][wavefront] counts into start positions
-// (digits ascending, wavefronts ascending inside a digit).  Ranking sweep, without block
-// barriers: the wavefront walks its keys in rounds of 64 in input order, a lane's rank among
-// the lanes with its digit comes from ballots, the first such lane advances the
-// wavefront's start for the digit.  Same stable order as above.  The passes ping-pong
-// between two global buffers, which one block keeps coherent with its barriers.
-constexpr int kSmallSortThreads = 1024;
-constexpr int kSmallSortWaves = kSmallSortThreads / kWave;
-constexpr int kSmallSortRounds = 16;                 // keys per lane
-constexpr int64_t kSmallSortMax = (int64_t)kSmallSortThreads * kSmallSortRounds;
+// Block d: row d of the histogram becomes its exclusive prefix over the tiles, its total goes
+// to totals[d].
+__global__ void __launch_bounds__(kSortThreads) sort_row_scan_kernel(int nb, int *__restrict__ hist,
+                                                                     int *__restrict__ totals) {
+  __shared__ int wave_sums[kSortThreads / kWave];
+  int *row = hist + (int64_t)blockIdx.x * nb;
+  int carry = 0;
+  for (int base = 0; base < nb; base += kSortThreads) {
+    const int i = base + threadIdx.x;
+    const int v = i < nb ? row[i] : 0;
+    int total;
+    const int ex = block_exclusive_256(v, wave_sums, &total);
+    if (i < nb) row[i] = carry + ex;
+    carry += total;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
 
-__global__ void __launch_bounds__(kSmallSortThreads) sort_small_kernel(
-    int n, int passes, const int64_t *__restrict__ keys, int64_t *kbuf0, int *ibuf0,
-    int64_t *kbuf1, int *ibuf1) {
-  __shared__ int start[kSmallSortWaves][kRadix];     // counts, then next free positions
-  __shared__ int scan[kRadix];
+// kFirst: the index of an item is its position.  KO: type of the keys written.  D > 0: also
+// out_pts[rank] = pts[index], out_bids[rank] = bids[index] (the last pass of a grid).
+template <class KI, class KO, bool kFirst, int D>
+__global__ void __launch_bounds__(kSortThreads) sort_scatter_kernel(
+    int64_t n, int shift, int nb, const KI *__restrict__ keys_in, const int *__restrict__ idx_in,
+    const int *__restrict__ hist, const int *__restrict__ totals, KO *__restrict__ keys_out,
+    int *__restrict__ idx_out, const float *__restrict__ pts, const int *__restrict__ bids,
+    float *__restrict__ out_pts, int *__restrict__ out_bids) {
+  __shared__ int start[kSortWaves][kSortRadix];    // counts, then next free position in the tile
+  __shared__ int to_global[kSortRadix];            // position in the tile -> in the output
+  __shared__ int wave_sums[kSortThreads / kWave];
+  __shared__ KI tile_key[kSortTile];
+  __shared__ int tile_idx[kSortTile];
   const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
-  // the wavefront's chunk: a multiple of 64 keys, so that rounds are whole except the last
-  const int per_wave = ((n + kSmallSortWaves - 1) / kSmallSortWaves + kWave - 1) / kWave * kWave;
-  const int first = wave * per_wave;
-  const int last = first + per_wave < n ? first + per_wave : n;
-  const int64_t *kin = keys;
-  const int *iin = nullptr;
-  for (int p = 0; p < passes; ++p) {
-    const int shift = 8 * p;
-    int64_t *kout = (p & 1) ? kbuf1 : kbuf0;
-    int *iout = (p & 1) ? ibuf1 : ibuf0;
-    int64_t key[kSmallSortRounds];
-    int idx[kSmallSortRounds];
+  const int64_t base = (int64_t)blockIdx.x * kSortTile;
+  const int live_items = n - base < kSortTile ? (int)(n - base) : kSortTile;
+  const int first = wave * (kSortTile / kSortWaves);
+  KI key[kSortItems];
+  int idx[kSortItems];
 #pragma unroll
-    for (int r = 0; r < kSmallSortRounds; ++r) {
-      const int i = first + r * kWave + lane;
-      key[r] = i < last ? kin[i] : 0;
-      idx[r] = i < last ? (p == 0 ? i : iin[i]) : 0;
-    }
-    if (t < kRadix) {
+  for (int r = 0; r < kSortItems; ++r) {
+    const int i = first + r * kWave + lane;
+    key[r] = i < live_items ? keys_in[base + i] : (KI)0;
+    idx[r] = kFirst ? (int)(base + i) : (i < live_items ? idx_in[base + i] : 0);
+  }
 #pragma unroll
-      for (int w = 0; w < kSmallSortWaves; ++w) start[w][t] = 0;
-    }
-    __syncthreads();
+  for (int w = 0; w < kSortWaves; ++w) start[w][t] = 0;
+  const int row_prefix = hist[(int64_t)t * nb + blockIdx.x];
+  const int row_total = totals[t];
+  __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSmallSortRounds; ++r)
-      if (first + r * kWave + lane < last) atomicAdd(&start[wave][digit_of(key[r], shift)], 1);
-    __syncthreads();
-    // exclusive scan over (digit, wavefront): per-digit totals scanned over the digits
-    // (Hillis-Steele in LDS, every thread at every barrier), then spread over the wavefronts
-    int total = 0;
-    if (t < kRadix) {
+  for (int r = 0; r < kSortItems; ++r)
+    if (first + r * kWave + lane < live_items) atomicAdd(&start[wave][digit_of(key[r], shift)], 1);
+  __syncthreads();
+  int unused;
+  const int digit_base = block_exclusive_256(row_total, wave_sums, &unused) + row_prefix;
+  int count = 0;
 #pragma unroll
-      for (int w = 0; w < kSmallSortWaves; ++w) total += start[w][t];
-    }
-    int v = total;
-    for (int off = 1; off < kRadix; off <<= 1) {
-      if (t < kRadix) scan[t] = v;
-      __syncthreads();
-      if (t < kRadix && t >= off) v += scan[t - off];
-      __syncthreads();
-    }
-    if (t < kRadix) {
-      int run = v - total;
+  for (int w = 0; w < kSortWaves; ++w) count += start[w][t];
+  int run = block_exclusive_256(count, wave_sums, &unused);
+  to_global[t] = digit_base - run;
 #pragma unroll
-      for (int w = 0; w < kSmallSortWaves; ++w) {
-        const int c = start[w][t];
-        start[w][t] = run;
-        run += c;
-      }
-    }
-    __syncthreads();
+  for (int w = 0; w < kSortWaves; ++w) {
+    const int c = start[w][t];
+    start[w][t] = run;
+    run += c;
+  }
+  __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSmallSortRounds; ++r) {
-      if (first + r * kWave >= last) break;              // uniform in the wavefront
-      const bool live = first + r * kWave + lane < last;
+  for (int r = 0; r < kSortItems; ++r) {
+    if (first + r * kWave < live_items) {                // uniform in the wavefront
+      const bool live = first + r * kWave + lane < live_items;
       const int d = digit_of(key[r], shift);
-      uint64_t same = __ballot(live);
+      uint64_t same = __ballot(live);                    // lanes with this digit
 #pragma unroll
       for (int bit = 0; bit < 8; ++bit) {
         const uint64_t b = __ballot((d >> bit) & 1);
         same &= ((d >> bit) & 1) ? b : ~b;
       }
       const int below = __popcll(same & ((1ull << lane) - 1ull));
-      int dst = 0;
-      if (live) dst = start[wave][d] + below;
-      wave_lds_sync();                                   // every lane has read its start
-      if (live && below == 0) start[wave][d] = dst + __popcll(same);
+      int pos = 0;
+      if (live) pos = start[wave][d] + below;
+      wave_lds_sync();                                   // every lane has read its position
+      if (live && below == 0) start[wave][d] = pos + __popcll(same);
       wave_lds_sync();
       if (live) {
-        kout[dst] = key[r];
-        iout[dst] = idx[r];
+        tile_key[pos] = key[r];
+        tile_idx[pos] = idx[r];
       }
     }
-    __threadfence_block();
-    __syncthreads();               // the pass is in memory before the next one reads it
-    kin = kout;
-    iin = iout;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kSortItems; ++r) {
+    const int i = r * kSortThreads + t;
+    if (i < live_items) {
+      const KI k = tile_key[i];
+      const int id = tile_idx[i];
+      const int64_t dst = (int64_t)to_global[digit_of(k, shift)] + i;
+      keys_out[dst] = (KO)k;
+      idx_out[dst] = id;
+      if constexpr (D > 0) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) out_pts[dst * D + d] = pts[(int64_t)id * D + d];
+        out_bids[dst] = bids[id];
+      }
+    }
+  }
+}
+
+// The whole sort in one launch for up to 16 384 keys (small_sort.h).
+__global__ void __launch_bounds__(kSmallThreads) sort_small_kernel(
+    int n, int bits, const int64_t *__restrict__ keys, int64_t *__restrict__ keys_out,
+    int *__restrict__ idx_out) {
+  extern __shared__ __align__(16) char lds_raw[];
+  SmallSortLds &s = *reinterpret_cast<SmallSortLds *>(lds_raw);
+  const int first = small_first(n), last = small_last(n), lane = lane_id();
+  int item[kSmallRounds];
+  small_sort(n, bits, keys, item, s);
+#pragma unroll
+  for (int r = 0; r < kSmallRounds; ++r) {
+    const int i = first + r * kWave + lane;
+    if (i < last) {
+      keys_out[i] = keys[item[r]];
+      idx_out[i] = item[r];
+    }
   }
 }
 
@@ -222,16 +202,7 @@ __global__ void __launch_bounds__(256) transpose_keys_kernel(int64_t m_total, in
   }
 }
 
-struct SortWorkspace {
-  int64_t *keys_tmp;
-  int *idx_tmp;
-  int *hist;
-  int *scan_scratch;
-  int64_t *total;
-  size_t bytes;
-};
-
-static SortWorkspace carve_sort_workspace(void *ws, int64_t n) {
+SortWorkspace carve_sort_workspace(void *ws, int64_t n) {
   const int64_t nb = (n + kSortTile - 1) / kSortTile;
   char *p = (char *)ws;
   SortWorkspace w;
@@ -241,13 +212,71 @@ static SortWorkspace carve_sort_workspace(void *ws, int64_t n) {
   w.idx_tmp = (int *)(p + off);
   off += align256(sizeof(int) * (size_t)n);
   w.hist = (int *)(p + off);
-  off += align256(sizeof(int) * (size_t)(kRadix * nb));
-  w.scan_scratch = (int *)(p + off);
-  off += align256(sizeof(int) * scan_scratch_ints(kRadix * nb));
-  w.total = (int64_t *)(p + off);
-  off += 256;
+  off += align256(sizeof(int) * (size_t)(kSortRadix * nb));
+  w.totals = (int *)(p + off);
+  off += align256(sizeof(int) * kSortRadix);
   w.bytes = off;
   return w;
+}
+
+// One pass over 64-bit or 32-bit keys; the histogram of a first pass may be there already.
+template <class KI, class KO, bool kFirst, int D>
+static int sort_pass(hipStream_t s, int64_t n, int shift, bool have_hist, const KI *kin,
+                     const int *iin, KO *kout, int *iout, const SortWorkspace &w,
+                     const SortedPoints &g) {
+  const int nb = (int)((n + kSortTile - 1) / kSortTile);
+  if (!have_hist) {
+    hipLaunchKernelGGL((sort_hist_kernel<KI>), dim3(nb), dim3(kSortThreads), 0, s, n, shift, nb,
+                       kin, w.hist);
+    MCCNN_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(sort_row_scan_kernel, dim3(kSortRadix), dim3(kSortThreads), 0, s, nb, w.hist,
+                     w.totals);
+  MCCNN_LAUNCH_CHECK();
+  hipLaunchKernelGGL((sort_scatter_kernel<KI, KO, kFirst, D>), dim3(nb), dim3(kSortThreads), 0, s,
+                     n, shift, nb, kin, iin, w.hist, w.totals, kout, iout, g.points, g.batch_ids,
+                     g.points_out, g.batch_ids_out);
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
+template <int D>
+static int sort_grid_keys_d(hipStream_t s, int64_t n, int bits, unsigned *keys32,
+                            const SortWorkspace &w, int64_t *keys_out, int *idx_out,
+                            const SortedPoints &g) {
+  const int passes = (bits + 7) / 8;
+  // the 32-bit keys ping-pong between keys32 and the workspace, the indices between the
+  // workspace and the output so that the last pass lands there
+  unsigned *kbuf[2] = {(unsigned *)w.keys_tmp, keys32};
+  int *ibuf[2] = {passes % 2 ? idx_out : w.idx_tmp, passes % 2 ? w.idx_tmp : idx_out};
+  const unsigned *kin = keys32;
+  const int *iin = nullptr;
+  for (int p = 0; p < passes; ++p) {
+    const bool last = p == passes - 1;
+    unsigned *ko = kbuf[p & 1];
+    int *io = ibuf[p & 1];
+    int rc;
+    if (p == 0)
+      rc = last ? sort_pass<unsigned, int64_t, true, D>(s, n, 0, true, kin, iin, keys_out, io, w, g)
+                : sort_pass<unsigned, unsigned, true, 0>(s, n, 0, true, kin, iin, ko, io, w, g);
+    else
+      rc = last ? sort_pass<unsigned, int64_t, false, D>(s, n, 8 * p, false, kin, iin, keys_out,
+                                                         io, w, g)
+                : sort_pass<unsigned, unsigned, false, 0>(s, n, 8 * p, false, kin, iin, ko, io, w,
+                                                          g);
+    if (rc != MCCNN_OK) return rc;
+    kin = ko;
+    iin = io;
+  }
+  return MCCNN_OK;
+}
+
+int sort_grid_keys(hipStream_t s, int num_dims, int64_t n, int bits, unsigned *keys32,
+                   const SortWorkspace &w, int64_t *keys_out, int *idx_out,
+                   const SortedPoints &g) {
+  int rc = MCCNN_OK;
+  MCCNN_DIM_SWITCH(num_dims, rc = sort_grid_keys_d<D>(s, n, bits, keys32, w, keys_out, idx_out, g));
+  return rc;
 }
 
 }  // namespace mccnn
@@ -276,7 +305,6 @@ extern "C" int mccnn_sort_keys_descending(mccnn_stream_t stream, int64_t num_pts
                 workspace_bytes, w.bytes);
   hipStream_t s = as_stream(stream);
   const int passes = (key_bits + 7) / 8;
-  const int nb = (int)((num_pts + kSortTile - 1) / kSortTile);
   // Ping-pong so that the last pass lands in the caller's buffers.
   int64_t *kbuf[2];
   int *ibuf[2];
@@ -287,30 +315,27 @@ extern "C" int mccnn_sort_keys_descending(mccnn_stream_t stream, int64_t num_pts
     kbuf[0] = w.keys_tmp;                 ibuf[0] = w.idx_tmp;
     kbuf[1] = (int64_t *)sorted_keys_out; ibuf[1] = sorted_indices_out;
   }
-  if (num_pts <= kSmallSortMax) {
-    hipLaunchKernelGGL(sort_small_kernel, dim3(1), dim3(kSmallSortThreads), 0, s, (int)num_pts,
-                       passes, (const int64_t *)keys, kbuf[0], ibuf[0], kbuf[1], ibuf[1]);
+  if (num_pts <= kSmallMax) {
+    MCCNN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(sort_small_kernel),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        (int)sizeof(SmallSortLds)));
+    hipLaunchKernelGGL(sort_small_kernel, dim3(1), dim3(kSmallThreads), sizeof(SmallSortLds), s,
+                       (int)num_pts, key_bits, (const int64_t *)keys, (int64_t *)sorted_keys_out,
+                       sorted_indices_out);
     MCCNN_LAUNCH_CHECK();
     return MCCNN_OK;
   }
   const int64_t *kin = (const int64_t *)keys;
   const int *iin = nullptr;
+  const SortedPoints none = {};
   for (int p = 0; p < passes; ++p) {
-    const int shift = 8 * p;
     int64_t *kout = kbuf[p & 1];
     int *iout = ibuf[p & 1];
-    hipLaunchKernelGGL(sort_hist_kernel, dim3(nb), dim3(kSortThreads), 0, s, num_pts, shift, nb,
-                       kin, w.hist);
-    MCCNN_LAUNCH_CHECK();
-    int rc = inclusive_scan_i32(s, (int64_t)kRadix * nb, w.hist, w.scan_scratch, w.total);
+    int rc = p == 0 ? sort_pass<int64_t, int64_t, true, 0>(s, num_pts, 0, false, kin, iin, kout,
+                                                           iout, w, none)
+                    : sort_pass<int64_t, int64_t, false, 0>(s, num_pts, 8 * p, false, kin, iin,
+                                                            kout, iout, w, none);
     if (rc != MCCNN_OK) return rc;
-    if (p == 0)
-      hipLaunchKernelGGL(sort_scatter_kernel<true>, dim3(nb), dim3(kSortThreads), 0, s, num_pts,
-                         shift, nb, kin, iin, w.hist, kout, iout);
-    else
-      hipLaunchKernelGGL(sort_scatter_kernel<false>, dim3(nb), dim3(kSortThreads), 0, s, num_pts,
-                         shift, nb, kin, iin, w.hist, kout, iout);
-    MCCNN_LAUNCH_CHECK();
     kin = kout;
     iin = iout;
   }

@@ -33,36 +33,24 @@ int fill_zero(hipStream_t stream, void *ptr, size_t bytes) {
 }
 
 // ------------------------------------------------------------ prefix sum ----
-// Long inputs take three launches, no inter-block waiting: (1) each block of kScanTile items
-// writes its sum, (2) one block scans the block sums, (3) each block rescans its
-// tile with the carried-in offset.  The scanned values are int32 (pair counts are
-// int32 in the op contract); tile sums and the grand total are formed in 64 bits
-// and a tile sum that does not fit saturates, so that a total of 2^31 - 1 or more
-// is always reported as at least 2^31 - 1 and the callers can refuse it instead
-// of working on wrapped offsets.
+// Up to kScanSingleMax values: one launch, one block.  Up to 4 M values: two launches, no
+// inter-block waiting: (1) each block writes the sum of its tile, (2) each block adds up the
+// tile sums in front of its own (at most 2048 values, from L2) and rescans its tile.  Beyond
+// that a launch in between scans the tile sums.  A launch costs 2 to 4 us, as much as the
+// bytes of a million values, so the number of launches is what the short forms save (16 384
+// values: 9.1 us in rounds of 8 scalar loads per thread, 4 us with 16-byte loads; 100 000
+// values 11 us with three launches, 7 us with two).
+// The scanned values are int32 (pair counts are int32 in the op contract); tile sums and the
+// grand total are formed in 64 bits and a sum that does not fit saturates, so that a total of
+// 2^31 - 1 or more is always reported as at least 2^31 - 1 and the callers can refuse it
+// instead of working on wrapped offsets.
 
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
+constexpr int kScanMaxOwnPrefix = 2048;        // tile sums a block adds up by itself
 
 size_t scan_scratch_ints(int64_t n) { return (size_t)((n + kScanTile - 1) / kScanTile) + 1; }
-
-__device__ __forceinline__ int block_exclusive_scan(int v, int *total) {
-  __shared__ int wave_sums[kScanThreads / kWave];
-  const int lane = lane_id(), wave = threadIdx.x / kWave;
-  const int incl = wave_inclusive_scan(v);
-  if (lane == kWave - 1) wave_sums[wave] = incl;
-  __syncthreads();
-  int carry = 0, sum = 0;
-#pragma unroll
-  for (int w = 0; w < kScanThreads / kWave; ++w) {
-    if (w < wave) carry += wave_sums[w];
-    sum += wave_sums[w];
-  }
-  __syncthreads();
-  *total = sum;
-  return carry + incl - v;
-}
 
 constexpr long long kScanMax = 0x7fffffffLL;
 
@@ -70,8 +58,7 @@ __device__ __forceinline__ int saturate_i32(long long v) {
   return (int)(v > kScanMax ? kScanMax : v);
 }
 
-// 64-bit counterpart of block_exclusive_scan for the sums of whole tiles.
-template <int kThreads = kScanThreads>
+template <int kThreads>
 __device__ __forceinline__ long long block_exclusive_scan_i64(long long v, long long *total) {
   __shared__ long long wave_sums[kThreads / kWave];
   const int lane = lane_id(), wave = threadIdx.x / kWave;
@@ -94,15 +81,48 @@ __device__ __forceinline__ long long block_exclusive_scan_i64(long long v, long 
   return carry + incl - v;
 }
 
+// kItems values from `base` on, 0 past n; 16-byte loads where all of them exist and the array
+// is aligned to 16 bytes (`vec`).
+template <int kItems>
+__device__ __forceinline__ void load_items(const int *__restrict__ src, int64_t base, int64_t n,
+                                           bool vec, int *v) {
+  if (vec && base + kItems <= n) {
+#pragma unroll
+    for (int k = 0; k < kItems / 4; ++k) {
+      const int4 q = reinterpret_cast<const int4 *>(src + base)[k];
+      v[4 * k] = q.x; v[4 * k + 1] = q.y; v[4 * k + 2] = q.z; v[4 * k + 3] = q.w;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) v[k] = base + k < n ? src[base + k] : 0;
+  }
+}
+
+template <int kItems>
+__device__ __forceinline__ void store_items(int *__restrict__ dst, int64_t base, int64_t n,
+                                            bool vec, const int *v) {
+  if (vec && base + kItems <= n) {
+#pragma unroll
+    for (int k = 0; k < kItems / 4; ++k)
+      reinterpret_cast<int4 *>(dst + base)[k] =
+          make_int4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < kItems; ++k)
+      if (base + k < n) dst[base + k] = v[k];
+  }
+}
+
 __global__ void __launch_bounds__(kScanThreads) scan_tile_sums_kernel(
-    int64_t n, const int *__restrict__ counts, int *__restrict__ block_sums) {
+    int64_t n, bool vec, const int *__restrict__ counts, int *__restrict__ block_sums) {
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
+  int v[kScanItems];
+  load_items<kScanItems>(counts, base, n, vec, v);
   long long s = 0;
 #pragma unroll
-  for (int k = 0; k < kScanItems; ++k)
-    if (base + k < n) s += counts[base + k];
+  for (int k = 0; k < kScanItems; ++k) s += v[k];
   long long total;
-  block_exclusive_scan_i64(s, &total);
+  block_exclusive_scan_i64<kScanThreads>(s, &total);
   if (threadIdx.x == 0) block_sums[blockIdx.x] = saturate_i32(total);
 }
 
@@ -114,57 +134,67 @@ __global__ void __launch_bounds__(kScanThreads) scan_block_sums_kernel(int nb, i
     const int i = base + threadIdx.x;
     const long long v = i < nb ? block_sums[i] : 0;
     long long total;
-    const long long ex = block_exclusive_scan_i64(v, &total);
+    const long long ex = block_exclusive_scan_i64<kScanThreads>(v, &total);
     if (i < nb) block_sums[i] = saturate_i32(carry + ex);
     carry += total;
   }
   if (threadIdx.x == 0) *total_dev = carry;
 }
 
+// kOwnPrefix: block_sums are the tile sums themselves and the block adds up those in front of
+// it (the last block also writes the total); otherwise they have been scanned.
+template <bool kOwnPrefix>
 __global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(
-    int64_t n, int *__restrict__ counts, const int *__restrict__ block_sums) {
+    int64_t n, bool vec, int *__restrict__ counts, const int *__restrict__ block_sums,
+    int64_t *total_dev) {
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
   int v[kScanItems];
-  int s = 0;
+  load_items<kScanItems>(counts, base, n, vec, v);
+  long long s = 0;
 #pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    v[k] = base + k < n ? counts[base + k] : 0;
-    s += v[k];
+  for (int k = 0; k < kScanItems; ++k) s += v[k];
+  long long total, carry;
+  if (kOwnPrefix) {
+    long long before = 0;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanThreads) before += block_sums[i];
+    block_exclusive_scan_i64<kScanThreads>(before, &carry);
+  } else {
+    carry = block_sums[blockIdx.x];
   }
-  int total;
-  int run = block_exclusive_scan(s, &total) + block_sums[blockIdx.x];
+  long long run = carry + block_exclusive_scan_i64<kScanThreads>(s, &total);
+  if (kOwnPrefix && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total_dev = carry + total;
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
     run += v[k];
-    if (base + k < n) counts[base + k] = run;
+    v[k] = saturate_i32(run);
   }
+  store_items<kScanItems>(counts, base, n, vec, v);
 }
 
-// Short inputs: one block walks the tiles in order and carries the running total,
-// one launch instead of three (small clouds are bound by launches, not by bytes).
+// Short inputs: one block walks tiles of 16 values per thread and carries the running total.
 constexpr int kScanSingleThreads = 1024;
-constexpr int kScanSingleTile = kScanSingleThreads * kScanItems;
-constexpr int64_t kScanSingleBlockMax = 4 * kScanSingleTile;
+constexpr int kScanSingleItems = 16;
+constexpr int kScanSingleTile = kScanSingleThreads * kScanSingleItems;
+constexpr int64_t kScanSingleMax = 2 * kScanSingleTile;
 
 __global__ void __launch_bounds__(kScanSingleThreads) scan_single_block_kernel(
-    int64_t n, int *counts, int64_t *total_dev) {
+    int64_t n, bool vec, int *counts, int64_t *total_dev) {
   long long carry = 0;
   for (int64_t tile = 0; tile < n; tile += kScanSingleTile) {
-    const int64_t base = tile + (int64_t)threadIdx.x * kScanItems;
-    int v[kScanItems];
+    const int64_t base = tile + (int64_t)threadIdx.x * kScanSingleItems;
+    int v[kScanSingleItems];
+    load_items<kScanSingleItems>(counts, base, n, vec, v);
     long long s = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      v[k] = base + k < n ? counts[base + k] : 0;
-      s += v[k];
-    }
+    for (int k = 0; k < kScanSingleItems; ++k) s += v[k];
     long long total;
     long long run = carry + block_exclusive_scan_i64<kScanSingleThreads>(s, &total);
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
+    for (int k = 0; k < kScanSingleItems; ++k) {
       run += v[k];
-      if (base + k < n) counts[base + k] = saturate_i32(run);
+      v[k] = saturate_i32(run);
     }
+    store_items<kScanSingleItems>(counts, base, n, vec, v);
     carry += total;
   }
   if (threadIdx.x == 0) *total_dev = carry;
@@ -176,20 +206,27 @@ int inclusive_scan_i32(hipStream_t stream, int64_t n, int *counts, int *block_su
   if (nb == 0) {
     return fill_zero(stream, total_dev, sizeof(int64_t));
   }
-  if (n <= kScanSingleBlockMax) {
+  const bool vec = reinterpret_cast<uintptr_t>(counts) % 16 == 0;
+  if (n <= kScanSingleMax) {
     hipLaunchKernelGGL(scan_single_block_kernel, dim3(1), dim3(kScanSingleThreads), 0, stream, n,
-                       counts, total_dev);
+                       vec, counts, total_dev);
     MCCNN_LAUNCH_CHECK();
     return MCCNN_OK;
   }
-  hipLaunchKernelGGL(scan_tile_sums_kernel, dim3(nb), dim3(kScanThreads), 0, stream, n, counts,
-                     block_sums);
+  hipLaunchKernelGGL(scan_tile_sums_kernel, dim3(nb), dim3(kScanThreads), 0, stream, n, vec,
+                     counts, block_sums);
   MCCNN_LAUNCH_CHECK();
+  if (nb <= kScanMaxOwnPrefix) {
+    hipLaunchKernelGGL(scan_apply_kernel<true>, dim3(nb), dim3(kScanThreads), 0, stream, n, vec,
+                       counts, block_sums, total_dev);
+    MCCNN_LAUNCH_CHECK();
+    return MCCNN_OK;
+  }
   hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kScanThreads), 0, stream, nb,
                      block_sums, total_dev);
   MCCNN_LAUNCH_CHECK();
-  hipLaunchKernelGGL(scan_apply_kernel, dim3(nb), dim3(kScanThreads), 0, stream, n, counts,
-                     block_sums);
+  hipLaunchKernelGGL(scan_apply_kernel<false>, dim3(nb), dim3(kScanThreads), 0, stream, n, vec,
+                     counts, block_sums, total_dev);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }

@@ -13,6 +13,7 @@ import torch
 
 from . import _lib, tfg_custom_ops
 _F32, _I32 = torch.float32, torch.int32
+_SINGLE_LAUNCH = 16384     # points up to which a grid or an order of centres is one launch
 
 
 class KDEMode(enum.Enum):
@@ -291,19 +292,34 @@ class Grid:
         self._cur_keys, self._sorted_keys = g.keys, g.sorted_keys
         self._sorted_indices = g.sorted_indices
         self._sorted_points, self._sorted_batch_ids = g.sorted_points, g.sorted_batch_ids
-        # host copy of the grid shape: sizes the key width and the column table
-        self._num_cells_host, self._key_bits = g.cells_host, g.key_bits
+        # host copy of the grid shape: sizes the key width and the column table.  A small
+        # cloud's grid does not wait for it (None until somebody asks)
+        self._shape = (g.cells_host, g.key_bits) if g.cells_host else None
         self._fast_DS = None
         self._sorted_positions = None
         self._self_neighborhoods = {}
 
+    def _host_shape(self):
+        if self._shape is None:
+            cells = [int(v) for v in self._num_cells.tolist()]
+            total = self._batch_size
+            for v in cells:
+                total *= v
+            self._shape = (cells, max(1, (total - 1).bit_length()))
+        return self._shape
+
+    @property
+    def _num_cells_host(self):
+        return self._host_shape()[0]
+
+    @property
+    def _key_bits(self):
+        return self._host_shape()[1]
+
     def sorted_positions(self):
         """Inverse of the sort: position of every original point in the sorted order."""
         if self._sorted_positions is None:
-            n, dev = self._sorted_indices.shape[0], self._sorted_indices.device
-            inv = torch.empty(n, dtype=_I32, device=dev)
-            inv[self._sorted_indices.long()] = torch.arange(n, dtype=_I32, device=dev)
-            self._sorted_positions = inv
+            self._sorted_positions = _lib.host().invert_order(self._sorted_indices)
         return self._sorted_positions
 
     def self_neighborhood(self, radii, max_neighbors=0):
@@ -314,6 +330,19 @@ class Grid:
         if key not in self._self_neighborhoods:
             self._self_neighborhoods[key] = Neighborhood(self, radii, None, max_neighbors)
         return self._self_neighborhoods[key]
+
+    def known_self_neighborhood(self, radii):
+        """The untruncated self-neighbourhood if it has been built, else None."""
+        return self._self_neighborhoods.get((_host_values(radii), 0))
+
+    def search_tensors(self):
+        """(points, cloud ids, keys, column table or None, num_cells, scaled minimum, inverse
+        cell size) of the sorted grid for the host extension.  Small clouds are searched over
+        their keys, without the table and the host copy of the grid shape it needs."""
+        small = self._shape is None and self._fast_DS is None
+        return (self._sorted_points, self._sorted_batch_ids, self._sorted_keys,
+                None if small else self.get_DS(), self._num_cells, self._scaled_aabb_min,
+                self._inv_cell_sizes)
 
     def get_DS(self):
         if self._fast_DS is None:
@@ -337,7 +366,7 @@ class _SortedView:
     """
 
     def __init__(self, nbh):
-        grid, samples = nbh._grid, nbh._point_cloud_sampled
+        grid = nbh._grid
         self.points_in = grid._sorted_points
         self.point_rows = grid._sorted_indices           # int32, for kernels
         self._point_order = self._centre_order = None    # their int64 forms, on first use
@@ -345,17 +374,8 @@ class _SortedView:
             self.centre_rows = None
             self.points_out = grid._sorted_points
             self.table, self.ranges = nbh._neighbors, nbh._samples_neigh_ranges
-        elif nbh._self_neighborhood is not None:     # same cloud: the shared sorted search
-            own = nbh._self_neighborhood
-            self.centre_rows = grid._sorted_indices
-            self.points_out = grid._sorted_points
-            self.table, self.ranges = own._neighbors, own._samples_neigh_ranges
         else:
-            order = nbh.compute_centre_order()
-            self.centre_rows = order
-            self.points_out = samples._points[self.centre_order].contiguous()
-            self.ranges, self.table = _lib.host().reorder_neighbors(
-                nbh._samples_neigh_ranges, nbh._neighbors, order)
+            self.centre_rows, self.points_out, self.ranges, self.table = nbh._sorted_search()
         # An untruncated self-neighbourhood is symmetric (the distance test is exact under
         # negation): the rows (x, p) of segment p are at once "x is a neighbour of centre p"
         # and "p is a neighbour of centre x", so the table is its own transpose.
@@ -453,15 +473,10 @@ class Neighborhood:
         self._inv_radii = _reciprocal(self._radii)
         s = self._point_cloud_sampled
         self._self_neighborhood = None
-        self._table = self._ranges = self._original = None
+        self._table = self._ranges = self._original = self._sorted = None
         if point_cloud_sample is grid._point_cloud:
             # The centres are the grid's own points in the caller's order: search once
-            # from the sorted points (consecutive centres then walk the same cells;
-            # the same search also serves the densities and the grid-ordered view of
-            # the layers).  The table in the caller's centre order is the same
-            # segments regrouped (the pairs of a centre depend on its coordinates
-            # only); it is built when somebody asks for it, which the layers on the
-            # grid-ordered view never do.
+            # from the sorted points (the same search also serves the densities).
             self._self_neighborhood = grid.self_neighborhood(self._radii, max_neighbors)
         elif not lazy:
             self._search()
@@ -471,37 +486,73 @@ class Neighborhood:
         self._pdf_normalize = False
         self._pdf_generation = 0
         # optional visiting order of the centres for the projection kernels
-        self._centre_order = None
+        self._centre_order = self._centre_slots = None
         self._transposed_pairs = None
         self._sorted_view = None
         self._transposed = None
 
     def _search(self):
+        """The pair search.  Centres that are not the grid's sorted points are brought into
+        the order of their cells first: consecutive centres then walk the same cells, and the
+        table is the grid-ordered view the layers run on.  The table in the caller's centre
+        order is the same segments regrouped (the pairs of a centre depend on its coordinates
+        only), built column by column when somebody asks for it."""
         s, grid = self._point_cloud_sampled, self._grid
-        self._ranges, self._table = tfg_custom_ops.find_neighbors(
-            s._points, s._batch_ids, grid._sorted_points, grid._sorted_keys, grid.get_DS(),
-            grid._num_cells, grid._scaled_aabb_min, grid._inv_cell_sizes, self._inv_radii,
-            self.max_neighbors)
+        points, ids, keys, ds, num_cells, smin, inv_cell = grid.search_tensors()
+        if self._equal_samples:
+            self._ranges, self._table, cut = _lib.host().search(
+                points, ids, points, keys, ds, num_cells, smin, inv_cell, self._inv_radii,
+                self.max_neighbors)
+            if not cut:
+                tfg_custom_ops._remember_symmetric(self._table)
+            return
+        order, pts, bids = _lib.host().order_centres(
+            s._points.detach(), s._batch_ids, grid._batch_size, num_cells, smin, inv_cell,
+            0 if s._points.shape[0] <= _SINGLE_LAUNCH else grid._key_bits)
+        ranges, table, _ = _lib.host().search(pts, bids, points, keys, ds, num_cells, smin,
+                                              inv_cell, self._inv_radii, self.max_neighbors)
+        self._sorted = (order, pts, ranges, table)
 
-    def _regroup(self):
-        if self._self_neighborhood is None:      # a search that was put off
-            return self._search()
-        own, grid = self._self_neighborhood, self._grid
-        self._ranges, self._table = _lib.host().reorder_neighbors(
-            own._samples_neigh_ranges, own._neighbors, grid.sorted_positions())
+    def _sorted_search(self):
+        """(centre order, centres, ranges, pairs) with the centres in the order of their cells."""
+        if self._sorted is None:
+            own = self._self_neighborhood
+            if own is None:
+                self._search()                   # a search that was put off
+            else:
+                grid = self._grid
+                self._sorted = (grid._sorted_indices, grid._sorted_points,
+                                own._samples_neigh_ranges, own._neighbors)
+        return self._sorted
+
+    def _slots(self):
+        """Position of every centre in the cell order."""
+        if self._self_neighborhood is not None:
+            return self._grid.sorted_positions()
+        if self._centre_slots is None:
+            self._centre_slots = _lib.host().invert_order(self._sorted_search()[0])
+        return self._centre_slots
 
     @property
     def _neighbors(self):
         """[M, 2] pairs (sorted point index, centre index), grouped by centre."""
         if self._table is None:
-            self._regroup()
+            if self._equal_samples:
+                self._search()
+            else:
+                _, _, ranges, table = self._sorted_search()
+                self._table = _lib.host().reorder_pairs(ranges, table, self._slots(),
+                                                        self._samples_neigh_ranges, None)
         return self._table
 
     @property
     def _samples_neigh_ranges(self):
         """[N_out] inclusive end offset of every centre's pairs."""
         if self._ranges is None:
-            self._regroup()
+            if self._equal_samples:
+                self._search()
+            else:
+                self._ranges = _lib.host().reorder_ranges(self._sorted_search()[2], self._slots())
         return self._ranges
 
     @property
@@ -509,8 +560,14 @@ class Neighborhood:
         """The pairs addressed by original point ids (Neighborhood.py:246-250);
         built on first use."""
         if self._original is None:
-            self._original = _lib.host().original_neighbor_ids(self._neighbors,
-                                                               self._grid._sorted_indices)
+            if self._table is None and not self._equal_samples:
+                _, _, ranges, table = self._sorted_search()
+                self._original = _lib.host().reorder_pairs(ranges, table, self._slots(),
+                                                           self._samples_neigh_ranges,
+                                                           self._grid._sorted_indices)
+            else:
+                self._original = _lib.host().original_neighbor_ids(self._neighbors,
+                                                                   self._grid._sorted_indices)
         return self._original
 
     def transposed_pairs(self):
@@ -547,11 +604,8 @@ class Neighborhood:
     def compute_centre_order(self):
         """Rank the centres by their cell key in the grid (a scheduling hint for
         `basis_proj`; the grid's own sorted points already are in that order)."""
-        s, grid = self._point_cloud_sampled, self._grid
-        if not self._equal_samples and s._points.shape[0] > 0:
-            keys = tfg_custom_ops.compute_keys(s._points, s._batch_ids, grid._scaled_aabb_min,
-                                               grid._num_cells, grid._inv_cell_sizes)
-            self._centre_order = _lib.host().sort_keys(keys, grid._key_bits)[1]
+        if not self._equal_samples:
+            self._centre_order = self._sorted_search()[0]
         return self._centre_order
 
     def compute_pdf(self, bandwidth=0.2, mode=KDEMode.constant, normalize=False):
@@ -566,11 +620,18 @@ class Neighborhood:
         if mode == KDEMode.no_pdf:
             self._pdf_per_point = None
             return
-        nbh = self if self._equal_samples else self._grid.self_neighborhood(self._radii)
-        bw = _as_vector(bandwidth, d, dev)
+        grid = self._grid
+        inv_bw = _reciprocal(_as_vector(bandwidth, d, dev))
+        nbh = self if self._equal_samples else grid.known_self_neighborhood(self._radii)
+        if nbh is None:          # the points' own pairs are not at hand: densities from the grid
+            points, ids, keys, ds, num_cells, smin, inv_cell = grid.search_tensors()
+            self._pdf_per_point = _lib.host().grid_density(
+                points, ids, keys, ds, num_cells, smin, inv_cell, self._inv_radii, inv_bw,
+                mode.value)
+            return
         self._pdf_per_point = tfg_custom_ops.compute_pdf_with_pt_grads(
-            self._grid._sorted_points, nbh._neighbors, nbh._samples_neigh_ranges,
-            _reciprocal(bw), nbh._inv_radii, mode.value,
+            grid._sorted_points, nbh._neighbors, nbh._samples_neigh_ranges, inv_bw,
+            nbh._inv_radii, mode.value,
             symmetric=nbh._equal_samples and nbh.max_neighbors == 0)
 
     def point_pdf(self, **kwargs):
@@ -585,15 +646,20 @@ class Neighborhood:
         (Neighborhood.py:287)."""
         per_point = self.point_pdf(**kwargs)
         if self._pdf is None:
-            nb = self._neighbors
             if per_point is None:
-                self._pdf = torch.ones(nb.shape[0], dtype=_F32, device=nb.device)
+                self._pdf = torch.ones(self._neighbors.shape[0], dtype=_F32,
+                                       device=self._neighbors.device)
+            elif self._table is None and not self._equal_samples:
+                _, _, ranges, table = self._sorted_search()
+                self._pdf = _lib.host().reorder_pdf(ranges, table, self._slots(),
+                                                    self._samples_neigh_ranges,
+                                                    per_point.detach())
             else:
-                self._pdf = _lib.host().gather_pdf(nb, 0, per_point.detach())
+                self._pdf = _lib.host().gather_pdf(self._neighbors, 0, per_point.detach())
             if self._pdf_normalize:       # divided by the size of the pair's neighbourhood
                 ends = self._samples_neigh_ranges.long()
                 counts = (ends - torch.cat([ends.new_zeros(1), ends[:-1]])).to(_F32)
-                self._pdf = self._pdf / counts[nb[:, 1].long()]
+                self._pdf = self._pdf / counts[self._neighbors[:, 1].long()]
         return self._pdf
 
 

@@ -1,0 +1,99 @@
+"""The branches of the grid build and of the neighbour search at the sizes where they change:
+one launch / several, keys beyond 32 bits, clouds out of order, more clouds than a block keeps
+the extents of; searches with and without the column table; densities from the grid.  Integers
+against the oracle bit for bit, densities to 1e-5 of their (positive) terms."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    return torch.as_tensor(np.ascontiguousarray(a)).cuda()
+
+
+def _same(got, expect, what):
+    assert np.array_equal(got.cpu().numpy(), expect), what
+
+
+def _check_grid(grid, g):
+    _same(grid._aabb_min, g.aabb_min, "minimum")
+    _same(grid._aabb_max, g.aabb_max, "maximum")
+    _same(grid._scaled_aabb_min, g.scaled_aabb_min, "scaled minimum")
+    _same(grid._num_cells, g.num_cells, "shape")
+    assert grid._num_cells_host == [int(v) for v in g.num_cells]
+    _same(grid._cur_keys, g.keys, "keys")
+    _same(grid._sorted_keys, g.sorted_keys, "sorted keys")
+    _same(grid._sorted_indices, g.sorted_indices, "order")
+    _same(grid._sorted_points, g.sorted_points, "points")
+    _same(grid._sorted_batch_ids, g.sorted_batch_ids, "cloud ids")
+
+
+@pytest.mark.parametrize("n,d,batch,extent,cell,shuffled", [
+    (1, 3, 1, 1.0, 0.1, False), (65, 3, 2, 1.0, 0.2, True), (1025, 2, 3, 1.0, 0.05, False),
+    (16384, 3, 16, 1.0, 0.1, False), (16385, 3, 16, 1.0, 0.1, False),
+    (16384, 4, 5, 1.0, 0.2, True), (40000, 3, 20, 1.0, 0.05, True),
+    (3000, 3, 2, 9000.0, 0.5, False), (20000, 3, 2, 9000.0, 0.5, False),   # keys of 43 bits
+    (2000, 3, 300, 1.0, 0.3, False), (30000, 3, 300, 1.0, 0.3, True)])     # 900 extents
+def test_grid_build(oracle, n, d, batch, extent, cell, shuffled):
+    from tensorflow_graphics_point_clouds_amd import pc
+    rng = np.random.default_rng(n + d)
+    pts = (rng.random((n, d)) * extent).astype(np.float32)
+    bids = np.sort(np.arange(n) % batch).astype(np.int32)
+    if shuffled:
+        bids = rng.permutation(bids)
+    _check_grid(pc.Grid(pc.PointCloud(dev(pts), dev(bids), batch), cell),
+                oracle.Grid(pts, bids, batch, np.float32(cell)))
+
+
+@pytest.mark.parametrize("d", [2, 3, 4])
+@pytest.mark.parametrize("n,n_out,max_neighbors", [(700, 700, 0), (16384, 300, 0), (300, 16385, 0),
+                                                   (16385, 16384, 0), (5000, 4000, 3)])
+def test_search_with_and_without_column_table(oracle, d, n, n_out, max_neighbors):
+    """Centres scattered over twice the box, in the caller's order; the sorted search and the
+    regrouped columns against the oracle's table."""
+    from tensorflow_graphics_point_clouds_amd import pc
+    rng = np.random.default_rng(n + n_out + d)
+    batch, radius = 3, np.float32({2: 0.05, 3: 0.1, 4: 0.2}[d])
+    pts = rng.random((n, d), dtype=np.float32)
+    bids = np.sort(np.arange(n) % batch).astype(np.int32)
+    ctr = (2 * rng.random((n_out, d)) - 0.5).astype(np.float32)
+    cbids = np.sort(np.arange(n_out) % batch).astype(np.int32)
+    g = oracle.Grid(pts, bids, batch, radius)
+    on = oracle.Neighborhood(g, radius, ctr, cbids, max_neighbors)
+    grid = pc.Grid(pc.PointCloud(dev(pts), dev(bids), batch), float(radius))
+    nbh = pc.Neighborhood(grid, float(radius), pc.PointCloud(dev(ctr), dev(cbids), batch),
+                          max_neighbors)
+    _same(nbh._samples_neigh_ranges, on.ranges, "ranges")
+    _same(nbh._original_neigh_ids, on.original_neigh_ids, "original ids")
+    _same(nbh._neighbors, on.neighbors, "pairs")
+    own = pc.Neighborhood(grid, float(radius))
+    oown = oracle.Neighborhood(g, radius)
+    _same(own._samples_neigh_ranges, oown.ranges, "self ranges")
+    _same(own._neighbors, oown.neighbors, "self pairs")
+    if max_neighbors == 0:
+        # densities straight from the grid (no self-neighbourhood on this one) and per pair
+        grid2 = pc.Grid(grid._point_cloud, float(radius))
+        far = pc.Neighborhood(grid2, float(radius), nbh._point_cloud_sampled)
+        got = far.point_pdf(bandwidth=0.2).cpu().numpy().astype(np.float64)
+        bw = np.full(d, 5.0, np.float32)
+        expect = oracle.compute_pdf(g.sorted_points, oown.neighbors, oown.ranges, bw,
+                                    np.full(d, 1.0, np.float32) / radius)
+        assert np.abs(got / expect - 1).max() <= 1e-5
+        pair = far.get_pdf().cpu().numpy().astype(np.float64)
+        assert np.abs(pair / expect[on.neighbors[:, 0]] - 1).max(initial=0) <= 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 15, 16384, 16385, 32768, 32769, 2048 * 2048, 2048 * 2048 + 1])
+def test_prefix_sum_forms(n):
+    """Single block, two launches, three launches, through the regrouping of a table whose
+    centre lists have 0 to 3 pairs."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    counts = torch.randint(0, 4, (n,), device="cuda", generator=gen)
+    ranges = torch.cumsum(counts, 0).int()
+    order = torch.randperm(n, device="cuda", generator=gen).int()
+    got = _lib.host().reorder_ranges(ranges, order)
+    assert torch.equal(got, torch.cumsum(counts[order.long()], 0).int())
