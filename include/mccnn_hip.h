@@ -402,6 +402,27 @@ int mccnn_basis_proj_grads_ordered(
     int64_t in_grads_dim1, int64_t in_grads_dim2, const float *in_grads,
     float *basis_grads_out, float *feature_grads_out);
 
+/* BasisProjGrads with the scatter-add of the feature gradient gathered in LDS per group of
+ * consecutive centres of centre_order: every point a group lists is added to memory once per
+ * group instead of once per pair.  For any table and any order; pays where consecutive centres
+ * share their points, as in the order mccnn_neighbourhood_order finds from the table itself
+ * (centres by the smallest hashes of their points).  Float atomics: the order of the sums is not
+ * fixed, as for mccnn_basis_proj_grads.  Supported: up to 128 features; basis, in_grads and
+ * basis_grads_out aligned to 16 bytes, features too if their number is a multiple of 16.
+ * ..._pays: whether it is the faster one for a table of these sizes. */
+size_t mccnn_neighbourhood_order_workspace_bytes(int64_t num_samples);
+int mccnn_neighbourhood_order(mccnn_stream_t stream, int64_t num_samples, int64_t num_neighbors,
+                              const int32_t *neighbors, const int32_t *ranges, void *workspace,
+                              size_t workspace_bytes, int32_t *order_out);
+int mccnn_basis_proj_grads_grouped_pays(int num_features, int num_basis, int64_t num_samples,
+                                        int64_t num_neighbors);
+size_t mccnn_basis_proj_grads_grouped_workspace_bytes(int64_t num_samples, int64_t num_neighbors);
+int mccnn_basis_proj_grads_grouped(
+    mccnn_stream_t stream, int64_t num_pts, int num_basis, const float *basis, int num_features,
+    const float *features, int64_t num_neighbors, const int32_t *neighbors, int64_t num_samples,
+    const int32_t *ranges, const int32_t *centre_order, const float *in_grads, void *workspace,
+    size_t workspace_bytes, float *basis_grads_out, float *feature_grads_out);
+
 /* Pair lists grouped by neighbour point, the transposed view of a pair table:
  * point_ranges_out [num_pts] (inclusive end offsets) and pair_order_out [M], the
  * pair indices sorted by neighbours[:,0], ties in ascending pair index.  No

@@ -446,12 +446,6 @@ int launch_dfeat_gather(hipStream_t s, int64_t num_pts, int C, const int *point_
   return MCCNN_OK;
 }
 
-static bool mfma_grads_supported(int C, int K) {
-  if (K == 32) return C == 32 || C == 64 || C == 128;
-  if (K == 16) return C == 16 || C == 32 || C == 64 || C == 128;
-  return false;
-}
-
 // Channels per lane for the matrix-core path, 0 when the shape needs the generic
 // kernel.  Accumulator budget: at most 128 registers per lane.
 static int mfma_channels_per_lane(int C, int K) {

@@ -982,6 +982,47 @@ Tensor basis_proj_raw_opt(const Tensor &basis, const Tensor &features, const Ten
   return basis_proj_raw(basis, features, neighbors, ranges, opt(order));
 }
 
+Tensor neighbourhood_order(const Tensor &neighbors, const Tensor &ranges) {
+  const int64_t n = ranges.size(0);
+  Tensor order = empty_i32({n}, ranges);
+  Tensor ws = workspace(mccnn_neighbourhood_order_workspace_bytes(n), ranges);
+  hipStream_t s = current_stream();
+  Region t("neighbourhood_order", s);
+  check(mccnn_neighbourhood_order(s, n, neighbors.size(0), i32(neighbors), i32(ranges),
+                                  ws.data_ptr(), ws.numel(), i32(order)));
+  return order;
+}
+
+std::pair<Tensor, Tensor> basis_proj_grads_grouped(const Tensor &basis, const Tensor &features,
+                                                   const Tensor &neighbors, const Tensor &ranges,
+                                                   const Tensor &g, const Tensor &order) {
+  Tensor dbasis = at::empty_like(basis), dfeat = at::empty_like(features);
+  hipStream_t s = current_stream();
+  Tensor ws = workspace(mccnn_basis_proj_grads_grouped_workspace_bytes(ranges.size(0),
+                                                                       neighbors.size(0)), ranges);
+  Region t("basis_proj_grads_grouped", s);
+  check(mccnn_basis_proj_grads_grouped(s, features.size(0), (int)basis.size(1), f32(basis),
+                                       (int)features.size(1), f32(features), neighbors.size(0),
+                                       i32(neighbors), ranges.size(0), i32(ranges), i32(order),
+                                       f32(g), ws.data_ptr(), ws.numel(), f32(dbasis),
+                                       f32(dfeat)));
+  return {dbasis, dfeat};
+}
+
+bool aligned16(const Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// whether the grouped kernels take over (anything they cannot check is left to the others' errors)
+bool group_gradients(const Tensor &basis, const Tensor &features, const Tensor &neighbors,
+                     const Tensor &ranges, const Tensor &g) {
+  if (basis.dim() != 2 || features.dim() != 2 || neighbors.dim() != 2 || neighbors.size(1) != 2 ||
+      basis.size(0) != neighbors.size(0) || g.dim() != 3 || g.size(0) != ranges.size(0) ||
+      g.size(1) != features.size(1) || g.size(2) != basis.size(1))
+    return false;
+  return mccnn_basis_proj_grads_grouped_pays((int)features.size(1), (int)basis.size(1),
+                                             ranges.size(0), neighbors.size(0)) &&
+         aligned16(basis) && aligned16(features) && aligned16(g);
+}
+
 // -> (dbasis, dfeatures); with the transposed lists the feature gradient is summed per point
 // from per-pair rows, in a fixed order
 std::pair<Tensor, Tensor> basis_proj_grads(const Tensor &basis, const Tensor &features,
@@ -989,6 +1030,9 @@ std::pair<Tensor, Tensor> basis_proj_grads(const Tensor &basis, const Tensor &fe
                                            const Tensor &g, const OptTensor &order,
                                            const OptTensor &point_ranges,
                                            const OptTensor &pair_order) {
+  if (!point_ranges.has_value() && group_gradients(basis, features, neighbors, ranges, g))
+    return basis_proj_grads_grouped(basis, features, neighbors, ranges, g,
+                                    neighbourhood_order(neighbors, ranges));
   Tensor dbasis = at::empty_like(basis), dfeat = at::empty_like(features);
   hipStream_t s = current_stream();
   if (point_ranges.has_value()) {
@@ -1008,6 +1052,29 @@ std::pair<Tensor, Tensor> basis_proj_grads(const Tensor &basis, const Tensor &fe
         dim(g, 1), dim(g, 2), f32(g), f32(dbasis), f32(dfeat)));
   }
   return {dbasis, dfeat};
+}
+
+struct BasisProj : torch::autograd::Function<BasisProj> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &basis, const Tensor &features,
+                        const Tensor &neighbors, const Tensor &ranges, const OptTensor &order,
+                        const OptTensor &point_ranges, const OptTensor &pair_order) {
+    ctx->save_for_backward({basis, features, neighbors, ranges, opt(order), opt(point_ranges),
+                            opt(pair_order)});
+    return basis_proj_raw(basis, features, neighbors, ranges, opt(order));
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grad_out) {
+    const auto s = ctx->get_saved_variables();
+    auto given = [](const Tensor &t) { return t.defined() ? OptTensor(t) : OptTensor(); };
+    const auto grads = basis_proj_grads(s[0], s[1], s[2], s[3], grad_out[0].contiguous(),
+                                        given(s[4]), given(s[5]), given(s[6]));
+    return {grads.first, grads.second, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+  }
+};
+
+Tensor basis_proj_apply(const Tensor &basis, const Tensor &features, const Tensor &neighbors,
+                        const Tensor &ranges, const OptTensor &order,
+                        const OptTensor &point_ranges, const OptTensor &pair_order) {
+  return BasisProj::apply(basis, features, neighbors, ranges, order, point_ranges, pair_order);
 }
 
 }  // namespace
@@ -1064,5 +1131,8 @@ PYBIND11_MODULE(_host, m) {
   m.def("local_pool", &local_pool, release());
   m.def("global_pool", &global_pool, release());
   m.def("basis_proj", &basis_proj_raw_opt, release());
+  m.def("basis_proj_apply", &basis_proj_apply, release());
   m.def("basis_proj_grads", &basis_proj_grads, release());
+  m.def("basis_proj_grads_grouped", &basis_proj_grads_grouped, release());
+  m.def("neighbourhood_order", &neighbourhood_order, release());
 }

@@ -46,6 +46,13 @@ static unsigned wave_grid(int64_t waves) {
 }
 
 
+// Shapes with a matrix-core kernel for the gradients of the basis projection (basis_proj.hip).
+inline bool mfma_grads_supported(int C, int K) {
+  if (K == 32) return C == 32 || C == 64 || C == 128;
+  if (K == 16) return C == 16 || C == 32 || C == 64 || C == 128;
+  return false;
+}
+
 // dfeat[n, :] = sum over the pairs listed for point n of pair_rows[pair, :]
 // (defined in basis_proj.hip).
 int launch_dfeat_gather(hipStream_t s, int64_t num_pts, int C, const int *point_ranges,

@@ -33,4 +33,7 @@ struct SortedPoints {
 int sort_grid_keys(hipStream_t s, int num_dims, int64_t n, int bits, unsigned *keys32,
                    const SortWorkspace &w, int64_t *keys_out, int *idx_out, const SortedPoints &g);
 
+// Order of 32-bit keys, descending and stable; keys32 is overwritten.
+int sort_order32(hipStream_t s, int64_t n, unsigned *keys32, const SortWorkspace &w, int *idx_out);
+
 }  // namespace mccnn

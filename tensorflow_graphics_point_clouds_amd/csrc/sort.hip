@@ -279,6 +279,27 @@ int sort_grid_keys(hipStream_t s, int num_dims, int64_t n, int bits, unsigned *k
   return rc;
 }
 
+int sort_order32(hipStream_t s, int64_t n, unsigned *keys32, const SortWorkspace &w,
+                 int *idx_out) {
+  unsigned *kbuf[2] = {(unsigned *)w.keys_tmp, keys32};
+  int *ibuf[2] = {w.idx_tmp, idx_out};              // four passes: the last lands in idx_out
+  const unsigned *kin = keys32;
+  const int *iin = nullptr;
+  const SortedPoints none = {};
+  for (int p = 0; p < 4; ++p) {
+    unsigned *ko = kbuf[p & 1];
+    int *io = ibuf[p & 1];
+    int rc = p == 0 ? sort_pass<unsigned, unsigned, true, 0>(s, n, 0, false, kin, iin, ko, io, w,
+                                                             none)
+                    : sort_pass<unsigned, unsigned, false, 0>(s, n, 8 * p, false, kin, iin, ko, io,
+                                                              w, none);
+    if (rc != MCCNN_OK) return rc;
+    kin = ko;
+    iin = io;
+  }
+  return MCCNN_OK;
+}
+
 }  // namespace mccnn
 
 using namespace mccnn;

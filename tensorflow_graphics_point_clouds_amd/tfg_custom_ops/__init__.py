@@ -169,16 +169,19 @@ def gathered_grads_supported(num_features, num_basis):
     return False
 
 
+def _gathered_lists(basis, features, transposed):
+    if transposed is not None and gathered_grads_supported(_dim(features, 1), _dim(basis, 1)):
+        return transposed
+    return None, None
+
+
 def basis_proj_grads(basis_neighbors, pt_features, neighbors, sample_neigh_indices,
                      in_gradients, centre_order=None, transposed=None):
     """BasisProjGrads (basis_proj_ops.cpp:40-53) -> (basis_gradients [M, K],
     feat_gradients [N_in, C]).  `transposed` = (point_ranges, pair_order) from
     `transpose_neighbors` selects the atomic-free, bit-reproducible feature
     gradient (needs an [M, C] scratch tensor)."""
-    point_ranges = pair_order = None
-    if transposed is not None and gathered_grads_supported(_dim(pt_features, 1),
-                                                           _dim(basis_neighbors, 1)):
-        point_ranges, pair_order = transposed
+    point_ranges, pair_order = _gathered_lists(basis_neighbors, pt_features, transposed)
     return _lib.host().basis_proj_grads(basis_neighbors, pt_features, neighbors,
                                         sample_neigh_indices, in_gradients, centre_order,
                                         point_ranges, pair_order)
@@ -190,21 +193,6 @@ def transpose_neighbors(neighbors, num_pts):
     return _lib.host().transpose_neighbors(neighbors, num_pts)
 
 
-class _BasisProj(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, basis, features, neighbors, ranges, centre_order, transposed):
-        ctx.save_for_backward(basis, features, neighbors, ranges)
-        ctx.centre_order, ctx.transposed = centre_order, transposed
-        return _basis_proj_raw(basis, features, neighbors, ranges, centre_order)
-
-    @staticmethod
-    def backward(ctx, grad):
-        basis, features, neighbors, ranges = ctx.saved_tensors
-        dbasis, dfeat = basis_proj_grads(basis, features, neighbors, ranges, grad.contiguous(),
-                                         ctx.centre_order, ctx.transposed)
-        return dbasis, dfeat, None, None, None, None
-
-
 def basis_proj(basis_neighbors, pt_features, neighbors, sample_neigh_indices,
                centre_order=None, transposed=None):
     """BasisProj (basis_proj_ops.cpp:25-38): [N_out, C, K] sum over the pairs of
@@ -212,5 +200,7 @@ def basis_proj(basis_neighbors, pt_features, neighbors, sample_neigh_indices,
     `centre_order` (optional int32 permutation of the centres) only changes the
     order in which centres are processed; `transposed` (optional, see
     `basis_proj_grads`) selects the atomic-free backward."""
-    return _BasisProj.apply(basis_neighbors, pt_features, neighbors, sample_neigh_indices,
-                            centre_order, transposed)
+    point_ranges, pair_order = _gathered_lists(basis_neighbors, pt_features, transposed)
+    return _lib.host().basis_proj_apply(basis_neighbors, pt_features, neighbors,
+                                        sample_neigh_indices, centre_order, point_ranges,
+                                        pair_order)

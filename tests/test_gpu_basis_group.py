@@ -1,0 +1,50 @@
+"""Gradients of the basis projection by groups of centres, on tables made to hit the edges of the
+kernels: lists of 0, 1, 16, 17, 64, 65 and several hundred pairs, a point listed twice by a
+centre, and groups with more distinct points than the LDS table has rows."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [0, 1, 16, 17, 64, 65, 31, 33, 700, 5]
+
+
+@pytest.mark.parametrize("c,k,points,centres", [
+    (3, 8, 40, 1), (7, 64, 900, 37), (16, 16, 64, 10), (24, 32, 4000, 83), (64, 8, 300, 21),
+    (64, 64, 5000, 64), (96, 16, 500, 129), (104, 32, 2000, 50), (128, 64, 1000, 33),
+    (128, 32, 3000, 260)])
+def test_grouped_gradients(c, k, points, centres):
+    from tensorflow_graphics_point_clouds_amd import _lib
+    host = _lib.host()
+    rng = np.random.default_rng(c * 100 + k)
+    lengths = np.resize(LENGTHS, centres)
+    ranges = np.cumsum(lengths).astype(np.int32)
+    owner = np.repeat(np.arange(centres), lengths)
+    ids = np.concatenate([np.sort(rng.choice(points, n, replace=n > points))
+                          for n in lengths] + [np.zeros(0, np.int64)])
+    if len(ids) > 2:
+        ids[2] = ids[1]                                  # listed twice by its centre
+    pairs = np.stack([ids, owner], axis=1).astype(np.int32)
+    basis = rng.standard_normal((len(ids), k)).astype(np.float32)
+    feat = rng.standard_normal((points, c)).astype(np.float32)
+    up = rng.standard_normal((centres, c, k)).astype(np.float32)
+    args = [torch.from_numpy(x).cuda() for x in (basis, feat, pairs, ranges, up)]
+    order = host.neighbourhood_order(args[2], args[3])
+    assert np.array_equal(np.sort(order.cpu().numpy()), np.arange(centres))
+    dbasis, dfeat = (x.cpu().numpy() for x in host.basis_proj_grads_grouped(*args, order))
+
+    def reference(basis, feat, up):
+        db = np.einsum("mck,mc->mk", up[owner], feat[ids])
+        df = np.zeros_like(feat)
+        np.add.at(df, ids, np.einsum("mck,mk->mc", up[owner], basis))
+        return db, df
+    # A sum of n float32 products in any order is off by less than (n + 1) 2^-24 times the sum of
+    # their absolute values: n = c for dbasis, k times the pairs of a point for dfeat.
+    wide = [x.astype(np.float64) for x in (basis, feat, up)]
+    db, df = reference(*wide)
+    db_mag, df_mag = reference(*map(np.abs, wide))
+    terms = k * np.bincount(ids, minlength=points)[:, None]
+    assert np.all(np.abs(dbasis - db) <= (c + 1) * 2.0 ** -24 * db_mag)
+    assert np.all(np.abs(dfeat - df) <= (terms + 1) * 2.0 ** -24 * df_mag)
