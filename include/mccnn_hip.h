@@ -423,6 +423,32 @@ int mccnn_basis_proj_grads_grouped(
     const int32_t *ranges, const int32_t *centre_order, const float *in_grads, void *workspace,
     size_t workspace_bytes, float *basis_grads_out, float *feature_grads_out);
 
+/* Gradients of batch normalisation over the points followed by the leaky activation (slope 1:
+ * none, slope 0: ReLU), the BatchNormalization / LeakyReLU pairs of network_blocks.py:27-465 and
+ * modelnet40.py:128-260 (no op of the reference's: TensorFlow's).  x [num_pts, C] the input, y the
+ * activated output, mean and inv_std = 1/sqrt(variance + eps) what the forward pass used: the
+ * statistics of the points (training != 0) or given ones.  x_grads_out may be NULL. */
+size_t mccnn_norm_act_grads_workspace_bytes(int num_features);
+int mccnn_norm_act_grads(mccnn_stream_t stream, int64_t num_pts, int num_features, const float *x,
+                         const float *y, const float *in_grads, const float *mean,
+                         const float *inv_std, const float *weight, int training, float slope,
+                         void *workspace, size_t workspace_bytes, float *x_grads_out,
+                         float *weight_grads_out, float *bias_grads_out);
+
+/* Gradients of out = x w + bias for x [num_rows, num_cols_in], w [num_cols_in, num_cols_out], the
+ * per-point linear map of Conv1x1.py:24-101 (TensorFlow's matmul gradients): of the input, and of
+ * the weights and the bias (bias_grads_out may be NULL), summed in a fixed order.  float32 matrix
+ * instructions; any sizes. */
+int mccnn_linear_input_grads(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
+                             const float *weights, int num_cols_out, const float *in_grads,
+                             float *x_grads_out);
+size_t mccnn_linear_weight_grads_workspace_bytes(int64_t num_rows, int num_cols_in,
+                                                 int num_cols_out);
+int mccnn_linear_weight_grads(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
+                              const float *x, int num_cols_out, const float *in_grads,
+                              void *workspace, size_t workspace_bytes, float *weight_grads_out,
+                              float *bias_grads_out);
+
 /* Pair lists grouped by neighbour point, the transposed view of a pair table:
  * point_ranges_out [num_pts] (inclusive end offsets) and pair_order_out [M], the
  * pair indices sorted by neighbours[:,0], ties in ascending pair index.  No

@@ -1,19 +1,42 @@
 """Feature-space layers and residual blocks around the point convolutions
 (pylib/pc/layers/Conv1x1.py:24-101, pylib/pc/layers/network_blocks.py:27-465).
-Everything here is dense per-point work (a GEMM, batch normalisation, an
-activation) on stock torch; the spatial convolutions inside the blocks are the
-layers of `layers.py`."""
+Dense per-point work (a product, batch normalisation, an activation) on the
+kernels of csrc/point_dense.hip where they cover the input, else on stock torch;
+the spatial convolutions inside the blocks are the layers of `layers.py`."""
 import math
 
 import torch
 
-from . import layers, pc
+from . import _lib, layers, pc
 
 _F32 = torch.float32
 
 layer_types = {"mcconv": layers.MCConv, "mc": layers.MCConv, "mc_conv": layers.MCConv,
                "kpconv": layers.KPConv, "kp": layers.KPConv, "kp_conv": layers.KPConv,
                "pointconv": layers.PointConv, "point_conv": layers.PointConv}
+
+
+def _plain_rows(features):
+    """float32 rows on the GPU that the per-point kernels take."""
+    return (features.is_cuda and features.dtype == _F32 and features.dim() == 2 and
+            features.is_contiguous() and not torch.is_autocast_enabled("cuda"))
+
+
+def _leaky_slope(activation):
+    """The slope for negative inputs of a leaky activation (0: ReLU), else None."""
+    if activation is torch.relu or type(activation) is torch.nn.ReLU:
+        return 0.0
+    if type(activation) is torch.nn.LeakyReLU:
+        return activation.negative_slope
+    return None
+
+
+def _norm_act(norm, activation, features, training=None):
+    """activation(norm(features)), in the kernel of the normalisation if it can be."""
+    slope = _leaky_slope(activation)
+    if slope is None or not isinstance(norm, BatchNorm):
+        return activation(norm(features, training))
+    return norm(features, training, slope)
 
 
 def _identity(features, *args, **kwargs):
@@ -24,16 +47,32 @@ class BatchNorm(torch.nn.BatchNorm1d):
     """Batch normalisation over the points with Keras' defaults (moving-average
     momentum 0.99, epsilon 1e-3; torch counts the momentum from the other side).
     `training`, when given, overrides the module's train/eval mode, as the
-    reference passes it per call."""
+    reference passes it per call.  `negative_slope` applies a leaky ReLU of that
+    slope (0: ReLU) to the result."""
 
     def __init__(self, num_features, momentum=0.99, eps=1e-3, device="cuda"):
         super().__init__(num_features, eps=eps, momentum=1.0 - momentum, device=device)
 
-    def forward(self, features, training=None):
-        if training is None or bool(training) == self.training:
+    def forward(self, features, training=None, negative_slope=None):
+        training = self.training if training is None else bool(training)
+        if (_plain_rows(features) and features.shape[1] == self.num_features and
+                features.shape[0] > 1 and self.weight is not None and self.momentum is not None and
+                self.running_mean is not None and self.weight.dtype == _F32 and
+                self.running_mean.dtype == _F32 and self.weight.device == features.device):
+            return _lib.host().norm_act(features, self.weight, self.bias, self.running_mean,
+                                        self.running_var, self.num_batches_tracked, training,
+                                        self.momentum, self.eps,
+                                        1.0 if negative_slope is None else negative_slope)
+        out = self._forward(features, training)
+        if negative_slope is None:
+            return out
+        return torch.nn.functional.leaky_relu(out, negative_slope)
+
+    def _forward(self, features, training):
+        if training == self.training:
             return super().forward(features)
         mode = self.training
-        self.train(bool(training))
+        self.train(training)
         try:
             return super().forward(features)
         finally:
@@ -56,9 +95,14 @@ class Conv1x1(torch.nn.Module):
 
     def forward(self, features, point_cloud, return_sorted=False, return_padded=False):
         features = point_cloud.flatten_features(features)
-        out = features @ self.weights
-        if self.bias is not None:
-            out = out + self.bias
+        if (_plain_rows(features) and features.shape[1] == self.weights.shape[0] and
+                self.weights.dtype == _F32 and self.weights.device == features.device and
+                self.weights.is_contiguous()):
+            out = _lib.host().linear(features, self.weights, self.bias)
+        else:
+            out = features @ self.weights
+            if self.bias is not None:
+                out = out + self.bias
         return point_cloud.format_output(out, return_sorted, return_padded)
 
 
@@ -93,7 +137,7 @@ class PointResNet(torch.nn.Module):
         for i in range(self._num_blocks):
             skip = features
             for j in (2 * i, 2 * i + 1):
-                features = self._activation(self._batch_norm_layers[j](features, training))
+                features = _norm_act(self._batch_norm_layers[j], self._activation, features, training)
                 features = self._conv_layers[j](features, point_cloud, point_cloud, radius,
                                                 neighborhood, **kwargs)
             if self._projection_layers is not None:
@@ -136,12 +180,13 @@ class PointResNetBottleNeck(torch.nn.Module):
         bn, act = self._batch_norm_layers, self._activation
         for i in range(self._num_blocks):
             skip = features
-            features = self._downsampling_layers[i](act(bn[3 * i](features, training)),
-                                                    point_cloud)
-            features = self._conv_layers[i](act(bn[3 * i + 1](features, training)), point_cloud,
-                                            point_cloud, radius, neighborhood, **kwargs)
-            features = self._upsampling_layers[i](act(bn[3 * i + 2](features, training)),
-                                                  point_cloud)
+            features = self._downsampling_layers[i](
+                _norm_act(bn[3 * i], act, features, training), point_cloud)
+            features = self._conv_layers[i](_norm_act(bn[3 * i + 1], act, features, training),
+                                            point_cloud, point_cloud, radius, neighborhood,
+                                            **kwargs)
+            features = self._upsampling_layers[i](
+                _norm_act(bn[3 * i + 2], act, features, training), point_cloud)
             if self._projection_layers is not None:
                 skip = self._projection_layers[i](skip, point_cloud)
             features = features + skip
@@ -195,7 +240,7 @@ class PointResNetSpatialBottleNeck(torch.nn.Module):
             skip = features
             for stage in range(3):
                 j = 3 * i + stage
-                features = self._activation(self._batch_norm_layers[j](features, training))
+                features = _norm_act(self._batch_norm_layers[j], self._activation, features, training)
                 features = self._stage_layers[j](features, clouds[stage][0], clouds[stage][1],
                                                  radii[stage], neighborhoods[stage], **kwargs)
             if self._projection_layers is not None:

@@ -1077,6 +1077,129 @@ Tensor basis_proj_apply(const Tensor &basis, const Tensor &features, const Tenso
   return BasisProj::apply(basis, features, neighbors, ranges, order, point_ranges, pair_order);
 }
 
+// ----------------------------------------------------- layers between the convolutions ----
+
+bool recording_gradients() { return at::GradMode::is_enabled(); }
+
+// Batch normalisation over the points + leaky activation.
+struct NormAct : torch::autograd::Function<NormAct> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight,
+                        const Tensor &bias, const Tensor &running_mean, const Tensor &running_var,
+                        const OptTensor &batches, bool training, double momentum, double eps,
+                        double slope) {
+    auto norm = at::native_batch_norm(x, weight, bias, running_mean, running_var, training,
+                                      momentum, eps);
+    if (training && batches.has_value()) Tensor(*batches).add_(1);
+    Tensor out = std::get<0>(norm);
+    if (slope == 0.0) out.relu_();
+    else if (slope != 1.0) at::leaky_relu_(out, slope);
+    Tensor mean = std::get<1>(norm), inv = std::get<2>(norm);
+    if (!training) {
+      mean = running_mean.clone();
+      inv = (running_var + eps).rsqrt();
+    }
+    ctx->save_for_backward({x, weight, bias, mean, inv, slope == 1.0 ? x : out});
+    ctx->saved_data["training"] = training;
+    ctx->saved_data["eps"] = eps;
+    ctx->saved_data["slope"] = slope;
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grad_out) {
+    const auto v = ctx->get_saved_variables();
+    const Tensor &x = v[0], &weight = v[1], &bias = v[2], &out = v[5];
+    const bool training = ctx->saved_data["training"].toBool();
+    const double slope = ctx->saved_data["slope"].toDouble();
+    variable_list grads(10);
+    if (recording_gradients()) {          // gradients of gradients: through torch's operations
+      Tensor mean = v[3], inv = v[4];
+      if (training) {
+        mean = x.mean(0);
+        inv = (x.var(0, false) + ctx->saved_data["eps"].toDouble()).rsqrt();
+      }
+      const Tensor z = (x - mean) * inv * weight + bias, y = slope == 1.0 ? z : at::where(out > 0, z, z * slope);
+      variable_list wanted;
+      std::vector<size_t> slots;
+      for (size_t i = 0; i < 3; ++i)
+        if (v[i].requires_grad()) {
+          wanted.push_back(v[i]);
+          slots.push_back(i);
+        }
+      const auto g = torch::autograd::grad({y}, wanted, {grad_out[0]}, true, true);
+      for (size_t i = 0; i < slots.size(); ++i) grads[slots[i]] = g[i];
+      return grads;
+    }
+    const Tensor g = grad_out[0].contiguous();
+    if (ctx->needs_input_grad(0)) grads[0] = at::empty_like(x);
+    grads[1] = at::empty_like(weight);
+    grads[2] = at::empty_like(bias);
+    Tensor ws = workspace(mccnn_norm_act_grads_workspace_bytes((int)x.size(1)), x);
+    hipStream_t s = current_stream();
+    Region t("norm_act_grads", s);
+    check(mccnn_norm_act_grads(s, x.size(0), (int)x.size(1), f32(x), f32(out), f32(g), f32(v[3]),
+                               f32(v[4]), f32(weight), training, (float)slope, ws.data_ptr(),
+                               ws.numel(), f32(grads[0]), f32(grads[1]), f32(grads[2])));
+    return grads;
+  }
+};
+
+Tensor norm_act(const Tensor &x, const Tensor &weight, const Tensor &bias,
+                const Tensor &running_mean, const Tensor &running_var, const OptTensor &batches,
+                bool training, double momentum, double eps, double slope) {
+  return NormAct::apply(x, weight, bias, running_mean, running_var, batches, training, momentum,
+                        eps, slope);
+}
+
+// Per-point linear map with weights [R, F] and an optional bias of F elements.
+struct Linear : torch::autograd::Function<Linear> {
+  static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w,
+                        const OptTensor &bias) {
+    ctx->save_for_backward({x, w});
+    if (bias.has_value()) ctx->saved_data["bias"] = bias->sizes().vec();
+    Tensor out = x.mm(w);
+    if (bias.has_value()) out.add_(*bias);
+    return out;
+  }
+  static variable_list backward(AutogradContext *ctx, variable_list grad_out) {
+    const auto v = ctx->get_saved_variables();
+    const Tensor &x = v[0], &w = v[1];
+    const bool has_bias = ctx->saved_data.count("bias") > 0;
+    variable_list grads(3);
+    if (recording_gradients()) {          // gradients of gradients: through torch's operations
+      grads[0] = grad_out[0].mm(w.t());
+      grads[1] = x.t().mm(grad_out[0]);
+      if (has_bias)
+        grads[2] = grad_out[0].sum(0).view(ctx->saved_data["bias"].toIntVector());
+      return grads;
+    }
+    const Tensor g = grad_out[0].contiguous();
+    const int64_t n = x.size(0), r = w.size(0), f = w.size(1);
+    hipStream_t s = current_stream();
+    if (ctx->needs_input_grad(0)) {
+      grads[0] = at::empty_like(x);
+      Region t("linear_input_grads", s);
+      check(mccnn_linear_input_grads(s, n, (int)r, f32(w), (int)f, f32(g), f32(grads[0])));
+    }
+    if (ctx->needs_input_grad(1) || (has_bias && ctx->needs_input_grad(2))) {
+      grads[1] = at::empty_like(w);
+      if (has_bias) grads[2] = empty_f32(ctx->saved_data["bias"].toIntVector(), w);
+      if (n == 0) {
+        grads[1].zero_();
+        if (has_bias) grads[2].zero_();
+        return grads;
+      }
+      Tensor ws = workspace(mccnn_linear_weight_grads_workspace_bytes(n, (int)r, (int)f), x);
+      Region t("linear_weight_grads", s);
+      check(mccnn_linear_weight_grads(s, n, (int)r, f32(x), (int)f, f32(g), ws.data_ptr(),
+                                      ws.numel(), f32(grads[1]), f32(grads[2])));
+    }
+    return grads;
+  }
+};
+
+Tensor linear(const Tensor &x, const Tensor &w, const OptTensor &bias) {
+  return Linear::apply(x, w, bias);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -1131,6 +1254,8 @@ PYBIND11_MODULE(_host, m) {
   m.def("local_pool", &local_pool, release());
   m.def("global_pool", &global_pool, release());
   m.def("basis_proj", &basis_proj_raw_opt, release());
+  m.def("norm_act", &norm_act, release());
+  m.def("linear", &linear, release());
   m.def("basis_proj_apply", &basis_proj_apply, release());
   m.def("basis_proj_grads", &basis_proj_grads, release());
   m.def("basis_proj_grads_grouped", &basis_proj_grads_grouped, release());

@@ -53,15 +53,16 @@ class ConvBlock(torch.nn.Module):
                 float(conv_radius) == float(pool_radius):
             radii = pc._as_vector(conv_radius, 3, point_cloud_in._points.device)
             shared = pc.Neighborhood(pc.Grid(point_cloud_in, radii), radii, point_cloud_out)
-        res = self.reduce(self.act(self.norms[0](features, training)), point_cloud_in)
-        res = self.conv(self.act(self.norms[1](res, training)), point_cloud_in, point_cloud_out,
-                        conv_radius, shared)
-        res = self.expand(self.act(self.norms[2](res, training)), point_cloud_out)
+        norm_act = lambda norm, x: blocks._norm_act(norm, self.act, x, training)
+        res = self.reduce(norm_act(self.norms[0], features), point_cloud_in)
+        res = self.conv(norm_act(self.norms[1], res), point_cloud_in, point_cloud_out, conv_radius,
+                        shared)
+        res = self.expand(norm_act(self.norms[2], res), point_cloud_out)
         skip = features
         if self.pool is not None:
             skip = self.pool(skip, point_cloud_in, point_cloud_out, pool_radius, shared)
         if self.skip_conv is not None:
-            skip = self.skip_conv(self.act(self.skip_norm(skip, training)), point_cloud_out)
+            skip = self.skip_conv(norm_act(self.skip_norm, skip), point_cloud_out)
         return res + skip
 
 
@@ -120,6 +121,7 @@ class ClassificationNet(torch.nn.Module):
         features = self.global_pooling(features, hierarchy[-1])
         dropping = self.training if training is None else bool(training)
         drop = lambda x: torch.nn.functional.dropout(x, self.dropout_rate, dropping)
-        features = self.head_dense[0](drop(self.act(self.head_norms[0](features, training))))
+        features = self.head_dense[0](
+            drop(blocks._norm_act(self.head_norms[0], self.act, features, training)))
         features = self.act(drop(self.head_norms[1](features, training)))
         return self.head_dense[1](features)
