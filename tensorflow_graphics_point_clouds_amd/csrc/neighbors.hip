@@ -184,8 +184,58 @@ __device__ __forceinline__ bool within_radius(const float *diff, const float *ir
 enum class Visit {
   kCount,      // counts[c] = number of hits (clamped to max_neighs when > 0)
   kFill,       // the pairs of centre c from its start offset on
-  kDensity,    // density[c]: the kernel density of centre c over its hits (compute_pdf)
+  kDensity,    // density[c]: the kernel density of centre c over its hits (DensitySums)
 };
+
+// The kernel density of a centre, summed as compute_pdf_kernel (pdf.hip) sums it over the pair
+// table: there G lanes take the pairs of a centre in turn, and G goes by the mean length of a
+// list, which nobody knows before all centres are visited.  So the three sums are kept side by
+// side and grid_density_select_kernel takes the one that the table would have given: the same
+// bits whether a cloud's pairs are at hand or not (a difference in the last place moves a
+// network's activations across kinks: one classifier pass in ten had gradients off by 2e-4).
+// The eight lanes of a group hold one candidate each; a trip's hits go to the lane of their
+// number in the list modulo eight.  Against one plain sum per lane: 17.3 -> 20.6 us for 16 384
+// points of the three-level network, and 3.8 us of the selecting launch.
+struct DensitySums {
+  float four = 0.0f, eight = 0.0f, low = 0.0f, high = 0.0f;   // high: sixteenths 8..15
+  // value of this lane's hit (0 without one), the group's hits as bits, hits of earlier trips
+  __device__ __forceinline__ void add(float value, unsigned hits, int sub, int group, int found) {
+    const int rank = __popc(hits & ((1u << sub) - 1u)), count = __popc(hits);
+    const int slot = (hits >> sub) & 1u ? found + rank : found + count + (sub - rank);
+    const float w = __int_as_float(
+        __builtin_amdgcn_ds_permute(4 * (group + (slot & 7)), __float_as_int(value)));
+    eight += w;
+    if (((found + ((sub - found) & 7)) >> 3) & 1) high += w;
+    else low += w;
+    const int first = (found + ((sub - found) & 3)) & 7;
+    four += __shfl(w, first, 8);
+    four += __shfl(w, first ^ 4, 8);
+  }
+  __device__ __forceinline__ void finish() {
+#pragma unroll
+    for (int off = 2; off > 0; off >>= 1) four += __shfl_xor(four, off, kWave);
+    low += high;
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1) {
+      eight += __shfl_xor(eight, off, kWave);
+      low += __shfl_xor(low, off, kWave);
+    }
+  }
+};
+
+// One pair's part, with the contractions of pdf.hip (this file is built without any): those of
+// the sum of squares, and those inside the exponential.
+template <int D>
+__device__ __forceinline__ float density_term(const float *diff, const float *scale) {
+#pragma clang fp contract(fast)
+  float e = 0.0f;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const float u = diff[d] * scale[d];
+    e += u * u;
+  }
+  return expf(-0.5f * e);
+}
 
 struct VisitSearch {                  // for kSearch: the grid to find the slices in
   const int *sbids;
@@ -204,7 +254,7 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
     int2 *ranges, const float *__restrict__ inv_radii, int max_neighs, VisitSearch search,
     int *__restrict__ counts, const int *__restrict__ ends, int2 *__restrict__ nbrs,
     int64_t *__restrict__ truncated, int64_t capacity, const float *__restrict__ inv_bandwidth,
-    int mode, float *__restrict__ density) {
+    int mode, float *__restrict__ density /* kDensity: [3, ns], counts: hits per wavefront */) {
   constexpr int R = OffsetInfo<D>::count();
   const int sub = threadIdx.x & (kGroup - 1);
   const int lane = lane_id();
@@ -219,10 +269,11 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
 #pragma unroll
   for (int d = 0; d < D; ++d) s[d] = samples[c * D + d];
   const int limit = max_neighs > 0 ? max_neighs : 0x7fffffff;
-  int found = 0;                                   // kFill: slots used so far
+  int found = 0;                                   // hits so far (kCount: of this lane)
   int64_t start = 0;
   if (kVisit == Visit::kFill) start = c > 0 ? ends[c - 1] : 0;
-  float scale[D], norm = 1.0f, sum = 0.0f;         // kDensity, as compute_pdf (pdf.hip)
+  float scale[D], norm = 1.0f;                     // kDensity, as compute_pdf (pdf.hip)
+  DensitySums sums;
   if (kVisit == Visit::kDensity) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -265,14 +316,12 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
           found += __popcll(hits);
         } else if (kVisit == Visit::kCount) {
           found += hit ? 1 : 0;
-        } else if (hit) {
-          float e = 0.0f;
-#pragma unroll
-          for (int d = 0; d < D; ++d) {
-            const float u = diff[d] * scale[d];
-            e += u * u;
+        } else {
+          const unsigned hits = (unsigned)((__ballot(hit) & group_mask) >> (lane & ~(kGroup - 1)));
+          if (hits != 0) {                         // the same for the lanes of a group
+            sums.add(hit ? density_term<D>(diff, scale) : 0.0f, hits, sub, lane & ~(kGroup - 1), found);
+            found += __popc(hits);
           }
-          sum += expf(-0.5f * e);
         }
       }
     }
@@ -287,10 +336,42 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
     }
   }
   if (kVisit == Visit::kDensity) {
+    sums.finish();
+    if (sub == 0) {
+      density[c] = sums.four * norm;
+      density[ns + c] = sums.eight * norm;
+      density[2 * ns + c] = sums.low * norm;
+    }
+    int pairs = 0;                      // of the wavefront's centres (those past the end have left)
+    const int64_t first = c - lane / kGroup;
 #pragma unroll
-    for (int off = kGroup / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, kWave);
-    if (sub == 0) density[c] = sum * norm;
+    for (int g = 0; g < kWave / kGroup; ++g)
+      if (first + g < ns) pairs += __builtin_amdgcn_readlane(found, g * kGroup);
+    if (lane == 0) counts[first / (kWave / kGroup)] = pairs;
   }
+}
+
+// The sums that compute_pdf would have taken for lists of this mean length (the rule of
+// mccnn_compute_pdf).  Every block adds up all counts: 8 KB for 16 384 points, 400 KB from L2 for
+// 800 000, and few blocks do.
+constexpr int kSelectThreads = 1024, kSelectBlocks = 64;
+__global__ void __launch_bounds__(kSelectThreads) grid_density_select_kernel(
+    int64_t n, int64_t parts, const int *__restrict__ counts, const float *__restrict__ sums,
+    float *__restrict__ pdf) {
+  __shared__ int64_t part[kSelectThreads / kWave];
+  int64_t pairs = 0;
+  for (int64_t i = threadIdx.x; i < parts; i += blockDim.x) pairs += counts[i];
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) pairs += __shfl_xor(pairs, off, kWave);
+  if (lane_id() == 0) part[threadIdx.x / kWave] = pairs;
+  __syncthreads();
+  pairs = 0;
+  for (int w = 0; w < kSelectThreads / kWave; ++w) pairs += part[w];
+  const int64_t mean = pairs / n;
+  const float *from = sums + (mean <= 16 ? 0 : mean <= 96 ? n : 2 * n);
+  for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < n;
+       c += (int64_t)gridDim.x * blockDim.x)
+    pdf[c] = from[c];
 }
 
 // Centres up to which the count pass finds its slices itself: 16 384 centres are 512 blocks,
@@ -637,15 +718,37 @@ extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, in
   return MCCNN_OK;
 }
 
+struct DensityWorkspace {
+  int2 *slices;
+  float *sums;          // [3, n]
+  int *counts;          // pairs per wavefront of the visit
+  int64_t parts;
+  size_t bytes;
+};
+
+static DensityWorkspace carve_density_workspace(void *ws, int d, int64_t n) {
+  char *p = (char *)ws;
+  DensityWorkspace w;
+  size_t off = 0;
+  w.slices = (int2 *)(p + off);
+  off += n <= kSearchInVisit ? 256 : align256(sizeof(int2) * (size_t)n * offsets_for(d));
+  w.sums = (float *)(p + off);
+  off += align256(3 * sizeof(float) * (size_t)n);
+  w.parts = (n + kWave / kGroup - 1) / (kWave / kGroup);
+  w.counts = (int *)(p + off);
+  off += align256(sizeof(int) * (size_t)w.parts);
+  w.bytes = off;
+  return w;
+}
+
 extern "C" size_t mccnn_grid_density_workspace_bytes(int num_dims, int64_t num_pts) {
   if (!valid_dims(num_dims) || num_pts < 0) return 0;
-  return num_pts <= kSearchInVisit ? 256
-                                   : align256(sizeof(int2) * (size_t)num_pts * offsets_for(num_dims));
+  return carve_density_workspace(nullptr, num_dims, num_pts).bytes;
 }
 
 // Kernel density of the grid's own points straight from the grid: what compute_pdf gives on the
-// pair table of the points among themselves, without the table (its count, the host round trip
-// for its size, the 8 bytes per pair written and read).
+// pair table of the points among themselves, bit for bit, without the table (its count, the host
+// round trip for its size, the 8 bytes per pair written and read).
 extern "C" int mccnn_grid_density(mccnn_stream_t stream, int64_t num_pts, int num_dims,
                                   const float *points, const int32_t *batch_ids,
                                   const int64_t *point_keys, const int32_t *grid_ds,
@@ -663,33 +766,36 @@ extern "C" int mccnn_grid_density(mccnn_stream_t stream, int64_t num_pts, int nu
   MCCNN_REQUIRE(workspace_bytes >= mccnn_grid_density_workspace_bytes(num_dims, num_pts),
                 "grid_density workspace too small");
   hipStream_t s = as_stream(stream);
-  int2 *slices = (int2 *)workspace;
+  const DensityWorkspace w = carve_density_workspace(workspace, num_dims, num_pts);
   const VisitSearch search = {batch_ids, num_pts, (const int64_t *)point_keys,
                               (const int2 *)grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes};
   const dim3 grid(blocks_for(num_pts, kCentresPerBlock)), block(kNbrThreads);
+#define MCCNN_DENSITY_VISIT(kSearch_, search_)                                                  \
+  MCCNN_DIM_SWITCH(num_dims,                                                                    \
+                   hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kDensity, kSearch_>), grid,   \
+                                      block, 0, s, num_pts, points, points, w.slices, inv_radii, \
+                                      0, search_, w.counts, (const int *)nullptr,               \
+                                      (int2 *)nullptr, (int64_t *)nullptr, (int64_t)0,          \
+                                      inv_bandwidth, mode, w.sums))
   if (num_pts <= kSearchInVisit) {
+    MCCNN_DENSITY_VISIT(true, search);
+  } else {
     MCCNN_DIM_SWITCH(num_dims,
-                     hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kDensity, true>), grid, block,
-                                        0, s, num_pts, points, points, slices, inv_radii, 0, search,
-                                        (int *)nullptr, (const int *)nullptr, (int2 *)nullptr,
-                                        (int64_t *)nullptr, (int64_t)0, inv_bandwidth, mode,
-                                        pdf_out));
+                     hipLaunchKernelGGL(nbr_ranges_kernel<D>,
+                                        dim3(blocks_for(num_pts * offsets_for(num_dims), 256)),
+                                        dim3(256), 0, s, num_pts, points, batch_ids, num_pts,
+                                        (const int64_t *)point_keys, (const int2 *)grid_ds,
+                                        num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
+                                        w.slices));
     MCCNN_LAUNCH_CHECK();
-    return MCCNN_OK;
+    MCCNN_DENSITY_VISIT(false, VisitSearch{});
   }
-  MCCNN_DIM_SWITCH(num_dims,
-                   hipLaunchKernelGGL(nbr_ranges_kernel<D>,
-                                      dim3(blocks_for(num_pts * offsets_for(num_dims), 256)),
-                                      dim3(256), 0, s, num_pts, points, batch_ids, num_pts,
-                                      (const int64_t *)point_keys, (const int2 *)grid_ds, num_cells,
-                                      scaled_aabb_min, inv_cell_sizes, inv_radii, slices));
+#undef MCCNN_DENSITY_VISIT
   MCCNN_LAUNCH_CHECK();
-  MCCNN_DIM_SWITCH(num_dims,
-                   hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kDensity, false>), grid, block, 0,
-                                      s, num_pts, points, points, slices, inv_radii, 0,
-                                      VisitSearch{}, (int *)nullptr, (const int *)nullptr,
-                                      (int2 *)nullptr, (int64_t *)nullptr, (int64_t)0,
-                                      inv_bandwidth, mode, pdf_out));
+  const int64_t blocks = (num_pts + kSelectThreads - 1) / kSelectThreads;
+  hipLaunchKernelGGL(grid_density_select_kernel,
+                     dim3((unsigned)(blocks < kSelectBlocks ? blocks : kSelectBlocks)),
+                     dim3(kSelectThreads), 0, s, num_pts, w.parts, w.counts, w.sums, pdf_out);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }

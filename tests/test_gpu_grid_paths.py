@@ -86,6 +86,25 @@ def test_search_with_and_without_column_table(oracle, d, n, n_out, max_neighbors
         assert np.abs(pair / expect[on.neighbors[:, 0]] - 1).max(initial=0) <= 1e-5
 
 
+@pytest.mark.parametrize("d", [2, 3, 5])
+@pytest.mark.parametrize("n,mean", [(1, 1), (7, 5), (16384, 9), (16384, 60), (3000, 200),
+                                    (16385, 9), (20000, 60), (16390, 150)])
+def test_density_from_the_grid_is_that_of_the_table(n, d, mean):
+    """Bit for bit, for the three ways the table's kernel sums (4, 8 and 16 lanes)."""
+    from tensorflow_graphics_point_clouds_amd import pc
+    rng = np.random.default_rng(n + d)
+    ball = {2: np.pi, 3: 4.189, 5: 5.264}[d]
+    radius = float((mean / (max(n, 2) * ball)) ** (1.0 / d))
+    pts, bids = dev(rng.random((n, d), dtype=np.float32)), dev(np.zeros(n, np.int32))
+    cloud, centres = pc.PointCloud(pts, bids, 1), pc.PointCloud(pts[:5].clone(), bids[:5], 1)
+    for mode in (pc.KDEMode.constant, pc.KDEMode.num_points):
+        alone = pc.Neighborhood(pc.Grid(cloud, radius), radius, centres)
+        own = pc.Neighborhood(pc.Grid(cloud, radius), radius)
+        got = alone.point_pdf(bandwidth=0.2, mode=mode)
+        expect = own.point_pdf(bandwidth=0.2, mode=mode)
+        assert torch.equal(got, expect), float((got / expect - 1).abs().max())
+
+
 @pytest.mark.parametrize("n", [1, 15, 16384, 16385, 32768, 32769, 2048 * 2048, 2048 * 2048 + 1])
 def test_prefix_sum_forms(n):
     """Single block, two launches, three launches, through the regrouping of a table whose
