@@ -414,11 +414,19 @@ int launch_tile_split(hipStream_t s, int64_t n, int R, const float *x, int F, co
 // into four vectors of 8 points, splits them and parks them as [part][group of 8
 // points][column]; every matrix operand is then one 16-byte LDS read.  Per step of 32
 // points: C x 32 values of x and 128 x 32 of y.
+// A block alternates between fetching and splitting (memory, vector units) and multiplying
+// (matrix cores), so what counts is how many blocks a compute unit holds to do the one while
+// others do the other.  One patch per thread, of x or of y by wavefront, and its eight rows on
+// scalar addresses leave 158 (C = 128) and 124 registers: three and four blocks.  With a patch
+// of either operand per thread, addresses and end-of-input selects per load (and 256 columns per
+// block below C = 128) there were two: [825 274, 128]^T x [.., 2048] 2.92 -> 2.65 ms,
+// [763 063, 64]^T x [.., 1024] 0.98 -> 0.96, [200 003, 64]^T x [.., 1024] 0.253 -> 0.234,
+// [600 000, 32]^T x [.., 512] 0.327 -> 0.290, [20 000, 64]^T x [.., 1024] 0.058 -> 0.041.
 // Blocks are numbered so that the column groups of one slice run on the same XCD (the
 // hardware deals consecutive blocks to the eight XCDs in turn): the slice of x they all read
 // then comes from HBM once and from that XCD's L2 for the other groups.
-template <int C, int BN>
-__global__ void __launch_bounds__(kSplitThreads) tn_split_kernel(
+template <int C, int BN, int kBlocks>
+__global__ void __launch_bounds__(kSplitThreads, kBlocks) tn_split_kernel(
     int64_t n, int R, const float *__restrict__ x, const float *__restrict__ y, int slices,
     float *__restrict__ partials) {
   constexpr int kCT = C / 32;                                   // row tiles of the output
@@ -427,13 +435,12 @@ __global__ void __launch_bounds__(kSplitThreads) tn_split_kernel(
   constexpr int kLdA = C + 4, kLdB = BN + 4;
   constexpr int kAPatches = C * kSplitK / 32;                   // patches of 8 points x 4 columns
   constexpr int kBPatches = BN * kSplitK / 32;
-  constexpr int kAPer = (kAPatches + kSplitThreads - 1) / kSplitThreads;
-  constexpr int kBPer = (kBPatches + kSplitThreads - 1) / kSplitThreads;
-  // the patches of y go to the first threads, those of x to the last ones
-  constexpr int kAShift = kAPer * kSplitThreads - kAPatches;
+  static_assert(kAPatches + kBPatches <= kSplitThreads && kBPatches % kWave == 0,
+                "a patch per thread, whole wavefronts for y");
   __shared__ v8bf a_lds[3 * kSplitGroups * kLdA];
   __shared__ v8bf b_lds[3 * kSplitGroups * kLdB];
-  const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+  const int t = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
   const int p = lane & 31, h = lane >> 5;
   const int wm = wave / kWN, wn = wave % kWN;
   const int groups = R / BN;
@@ -454,58 +461,51 @@ __global__ void __launch_bounds__(kSplitThreads) tn_split_kernel(
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-  // patch idx of an operand with W columns: group g = idx / (W / 4), columns 4 c4 .. 4 c4 + 3
-  v4f xa[kAPer][8], yb[kBPer][8];
+  // The thread's patch: of y in the first wavefronts, of x in the others; group g of 8 points,
+  // columns 4 c4 .. 4 c4 + 3.  Eight rows on scalar addresses plus the lane's offset.
+  const bool of_y = wave < kBPatches / kWave;                   // the same for a wavefront
+  const int idx = of_y ? t : t - kBPatches;
+  const bool has = of_y || idx < kAPatches;
+  const int g = of_y ? idx / (BN / 4) : idx / (C / 4), c4 = of_y ? idx % (BN / 4) : idx % (C / 4);
+  const int ld = of_y ? R : C;
+  const char *from = reinterpret_cast<const char *>(of_y ? y + col0 : x) + s0 * kSplitK * 4 * ld;
+  const unsigned lane_bytes = has ? (8 * g * ld + 4 * c4) * 4u : 0u;
+  v4f patch[8];
   auto fetch = [&](int64_t step) {
     const int64_t p0 = step * kSplitK;
+    if (p0 + kSplitK <= n) {
+      if (of_y) {
 #pragma unroll
-    for (int i = 0; i < kAPer; ++i) {
-      const int idx = t + kSplitThreads * i - kAShift, g = idx / (C / 4), c4 = idx % (C / 4);
-      if (kAShift == 0 || idx >= 0) {
+        for (int r = 0; r < 8; ++r)
+          patch[r] = __builtin_nontemporal_load(
+              reinterpret_cast<const v4f *>(from + (int64_t)r * 4 * R + lane_bytes));
+      } else {
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const int64_t pt = p0 + 8 * g + r;        // points past the end count as zeros
-          const v4f v = *reinterpret_cast<const v4f *>(x + (pt < n ? pt : n - 1) * C + 4 * c4);
-          xa[i][r] = pt < n ? v : v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        }
+        for (int r = 0; r < 8; ++r)
+          patch[r] = *reinterpret_cast<const v4f *>(from + r * 4 * C + lane_bytes);
+      }
+    } else {                                                    // the last points
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const int64_t pt = p0 + 8 * g + r;                      // past the end: zeros
+        patch[r] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        if (pt < n) patch[r] = *reinterpret_cast<const v4f *>(from + (int64_t)r * 4 * ld + lane_bytes);
       }
     }
-#pragma unroll
-    for (int i = 0; i < kBPer; ++i) {
-      const int idx = t + kSplitThreads * i, g = idx / (BN / 4), c4 = idx % (BN / 4);
-      if (kBPatches % kSplitThreads == 0 || idx < kBPatches) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const int64_t pt = p0 + 8 * g + r;
-          const v4f v = __builtin_nontemporal_load(
-              reinterpret_cast<const v4f *>(y + (pt < n ? pt : n - 1) * R + col0 + 4 * c4));
-          yb[i][r] = pt < n ? v : v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-      }
-    }
+    from += (int64_t)kSplitK * 4 * ld;
   };
-  auto park_patch = [&](const v4f *patch, v8bf *lds, int ld, int g, int c4) {
+  auto park_patch = [&](v8bf *lds, int row) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const v4f lo = {patch[0][j], patch[1][j], patch[2][j], patch[3][j]};
       const v4f hi = {patch[4][j], patch[5][j], patch[6][j], patch[7][j]};
       const Split8 s = split8(lo, hi);
 #pragma unroll
-      for (int q = 0; q < 3; ++q) lds[(q * kSplitGroups + g) * ld + 4 * c4 + j] = s.p[q];
+      for (int q = 0; q < 3; ++q) lds[q * kSplitGroups * row + j] = s.p[q];
     }
   };
   auto park = [&]() {
-#pragma unroll
-    for (int i = 0; i < kAPer; ++i) {
-      const int idx = t + kSplitThreads * i - kAShift;
-      if (kAShift == 0 || idx >= 0) park_patch(xa[i], a_lds, kLdA, idx / (C / 4), idx % (C / 4));
-    }
-#pragma unroll
-    for (int i = 0; i < kBPer; ++i) {
-      const int idx = t + kSplitThreads * i;
-      if (kBPatches % kSplitThreads == 0 || idx < kBPatches)
-        park_patch(yb[i], b_lds, kLdB, idx / (BN / 4), idx % (BN / 4));
-    }
+    if (has) park_patch((of_y ? b_lds + g * kLdB : a_lds + g * kLdA) + 4 * c4, of_y ? kLdB : kLdA);
   };
 
   if (s0 < s1) fetch(s0);
@@ -544,31 +544,32 @@ __global__ void __launch_bounds__(kSplitThreads) tn_split_kernel(
     }
 }
 
-// Columns of y per block: 128 with all 128 rows of the output, 256 below that.
-static int tn_split_cols(int C) { return C == 128 ? 128 : 256; }
+constexpr int kTnCols = 128;          // columns of y per block
 
 bool tn_split_supported(int C, int R) {
   if (!(C == 32 || C == 64 || C == 128)) return false;
-  const int bn = tn_split_cols(C);
-  return R >= bn && R % bn == 0 && R <= 4096;
+  const int step = C == 128 ? 128 : 256;
+  return R >= step && R % step == 0 && R <= 4096;
 }
 
-// Slices of the point range for an output of C x R (also sizes the partial sums): a
-// multiple of 8, one eighth per XCD, about 1024 blocks in all.
+// Slices of the point range for an output of C x R (also sizes the partial sums): a multiple
+// of 8, one eighth per XCD, and about 1536 blocks in all with C = 128 (two full rounds of three
+// blocks per compute unit; 1024 blocks: 2.69 against 2.65 ms on [825 274, 128]^T x [.., 2048],
+// 0.214 against 0.204 ms on [100 000, 128]^T x [.., 1024]), 2048 below that (two rounds of four).
 int tn_split_slices(int C, int R) {
-  const int groups = R / tn_split_cols(C);
-  int s = 1024 / groups / 8 * 8;
+  const int groups = R / kTnCols;
+  int s = (C == 128 ? 1536 : 2048) / groups / 8 * 8;
   return s < 8 ? 8 : s;
 }
 
 int launch_tn_split(hipStream_t s, int64_t n, int C, const float *x, int R, const float *y,
                     int slices, float *partials) {
-  const int groups = R / tn_split_cols(C);
+  const int groups = R / kTnCols;
   const dim3 grid((unsigned)(groups * ((slices + 7) / 8) * 8)), block(kSplitThreads);
   switch (C) {
-    case 128: hipLaunchKernelGGL((tn_split_kernel<128, 128>), grid, block, 0, s, n, R, x, y, slices, partials); break;
-    case 64: hipLaunchKernelGGL((tn_split_kernel<64, 256>), grid, block, 0, s, n, R, x, y, slices, partials); break;
-    default: hipLaunchKernelGGL((tn_split_kernel<32, 256>), grid, block, 0, s, n, R, x, y, slices, partials); break;
+    case 128: hipLaunchKernelGGL((tn_split_kernel<128, kTnCols, 3>), grid, block, 0, s, n, R, x, y, slices, partials); break;
+    case 64: hipLaunchKernelGGL((tn_split_kernel<64, kTnCols, 4>), grid, block, 0, s, n, R, x, y, slices, partials); break;
+    default: hipLaunchKernelGGL((tn_split_kernel<32, kTnCols, 4>), grid, block, 0, s, n, R, x, y, slices, partials); break;
   }
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
