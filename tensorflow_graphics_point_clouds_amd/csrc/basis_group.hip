@@ -76,18 +76,21 @@ __global__ void __launch_bounds__(256) neighbourhood_key_kernel(int64_t n,
 // fetched in runs of consecutive lanes, one tile ahead, and turned in LDS (rows padded by one
 // 16-byte piece: reads of a column of pieces fall into different banks).  The reduction runs
 // over channels 16 j + 4 quarter + e (step 4 j + e), a 16-byte read per lane and j.
+// Centres go by `order` with neighbours on one XCD, so that most rows come from its L2
+// (800 k x 52 pairs, 128 x 32: 5.40 -> 5.29 ms).
 template <int CT, int K, bool kFull>
 __global__ void __launch_bounds__(256) basis_grads_kernel(
     int64_t n_out, int C, const float *__restrict__ feat, const int2 *__restrict__ nbrs,
-    const int *__restrict__ ranges, const float *__restrict__ in_grad,
-    float *__restrict__ dbasis) {
+    const int *__restrict__ ranges, const int *__restrict__ order,
+    const float *__restrict__ in_grad, float *__restrict__ dbasis) {
   constexpr int KT = K > 16 ? K / 16 : 1;
   constexpr int kPieces = 4 * CT, kLd = kPieces + 1;      // 16-byte pieces of a row
   __shared__ v4f tiles[kWavesPerBlock][16 * kLd];
   const int lane = lane_id(), quarter = lane >> 4, col = lane & 15;
   v4f *tile = tiles[threadIdx.x / kWave];
-  const int64_t centre = wave_slot();
-  if (centre >= n_out) return;
+  const int64_t slot = wave_slot_xcd();
+  if (slot >= n_out) return;
+  const int64_t centre = centre_of(slot, order);
   const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
   if (b <= a) return;
   auto pair_ids = [&](int m0) { return nbrs[m0 + lane < b ? m0 + lane : b - 1].x; };
@@ -479,7 +482,7 @@ static int launch_group(hipStream_t s, int64_t n, int64_t pairs, int C, int grou
   MCCNN_LAUNCH_CHECK();
   auto dbasis_kernel = full ? basis_grads_kernel<CT, K, true> : basis_grads_kernel<CT, K, false>;
   hipLaunchKernelGGL(dbasis_kernel, dim3(wave_grid(n)), dim3(256), 0, s, n, C, feat, nbrs, ranges,
-                     in_grad, dbasis);
+                     order, in_grad, dbasis);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
