@@ -43,9 +43,10 @@ __device__ __forceinline__ int small_last(int n) {
 }
 
 // item[r] of a lane becomes the index of the key with rank first + 64 r + lane.  `keys` must be
-// visible to the whole block (a barrier since they were written).
-__device__ __forceinline__ void small_sort(int n, int bits, const int64_t *keys, int *item,
-                                           SmallSortLds &s) {
+// visible to the whole block (a barrier since they were written); the lowest `bits` of keys less
+// `below` tell them apart.
+__device__ __forceinline__ void small_sort(int n, int bits, const int64_t *keys, int64_t below,
+                                           int *item, SmallSortLds &s) {
   const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
   const int first = small_first(n), last = small_last(n);
   const int passes = (bits + kSmallDigitBits - 1) / kSmallDigitBits;
@@ -59,7 +60,7 @@ __device__ __forceinline__ void small_sort(int n, int bits, const int64_t *keys,
 #pragma unroll
     for (int r = 0; r < kSmallRounds; ++r)
       digit[r] = first + r * kWave + lane < last
-                     ? (int)((~(uint64_t)keys[item[r]] >> shift) & (uint64_t)(radix - 1)) : 0;
+                     ? (int)((~(uint64_t)(keys[item[r]] - below) >> shift) & (uint64_t)(radix - 1)) : 0;
     for (int i = t; i < kSmallWaves * radix; i += kSmallThreads) s.start[i] = 0;
     __syncthreads();
     int *mine = s.start + wave * radix;

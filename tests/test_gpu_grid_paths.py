@@ -31,6 +31,37 @@ def _check_grid(grid, g):
     _same(grid._sorted_batch_ids, g.sorted_batch_ids, "cloud ids")
 
 
+@pytest.mark.parametrize("d", [2, 3])
+@pytest.mark.parametrize("sizes", [(1, 1), (700, 0, 33, 64, 65, 0), (0, 0, 5), (9000, 2, 1),
+                                   (16384, 0), (128,) * 128, (60,) * 129])
+@pytest.mark.parametrize("order", ["ascending", "descending", "one out of order"])
+def test_grid_build_cloud_by_cloud(oracle, d, sizes, order):
+    """Clouds of very different sizes, empty ones first, between and last; ids either way round."""
+    from tensorflow_graphics_point_clouds_amd import pc
+    rng = np.random.default_rng(sum(sizes) + d)
+    bids = np.repeat(np.arange(len(sizes)), sizes).astype(np.int32)
+    if order != "ascending":
+        bids = bids[::-1].copy()
+    if order == "one out of order":
+        bids[len(bids) // 2], bids[0] = bids[0], bids[len(bids) // 2]
+    pts = rng.random((len(bids), d), dtype=np.float32)
+    grid = pc.Grid(pc.PointCloud(dev(pts), dev(bids), len(sizes)), 0.07)
+    # with 200 clouds, the others empty, one block does it all (the oracle has no empty clouds)
+    whole = pc.Grid(pc.PointCloud(dev(pts), dev(bids), 200), 0.07)
+    for name in ("_num_cells", "_sorted_keys", "_sorted_indices", "_sorted_points",
+                 "_sorted_batch_ids"):
+        assert torch.equal(getattr(grid, name), getattr(whole, name)), name
+    centres = [pc.PointCloud(dev(pts[::2]), dev(bids[::2]), n) for n in (len(sizes), 200)]
+    search = [pc.Neighborhood(g, 0.07, c) for g, c in zip((grid, whole), centres)]
+    for name in ("_neighbors", "_samples_neigh_ranges", "_original_neigh_ids"):
+        assert torch.equal(getattr(search[0], name), getattr(search[1], name)), name
+    if min(sizes) > 0:
+        g = oracle.Grid(pts, bids, len(sizes), np.float32(0.07))
+        _check_grid(grid, g)
+        _same(search[0]._neighbors,
+              oracle.Neighborhood(g, np.float32(0.07), pts[::2], bids[::2], 0).neighbors, "pairs")
+
+
 @pytest.mark.parametrize("n,d,batch,extent,cell,shuffled", [
     (1, 3, 1, 1.0, 0.1, False), (65, 3, 2, 1.0, 0.2, True), (1025, 2, 3, 1.0, 0.05, False),
     (16384, 3, 16, 1.0, 0.1, False), (16385, 3, 16, 1.0, 0.1, False),
