@@ -819,6 +819,12 @@ int mccnn_final_product_supported(int num_cols_in, int num_cols_out);
 int mccnn_final_product(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
                         const float *x, int num_cols_out, const float *w,
                         const int32_t *out_rows, float *out);
+/* The same for weights whose columns from num_cols on (a multiple of 16) are padding: the first
+ * num_cols columns of out get the bits of the product without padding, the others may not be
+ * written. */
+int mccnn_final_product_padded(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
+                               const float *x, int num_cols_out, int num_cols, const float *w,
+                               const int32_t *out_rows, float *out);
 
 /* The same product with the weights handed over transposed, wt [F, R] (the rows of
  * wt run along the reduction, like the rows of x): the tiled product for weight

@@ -504,9 +504,9 @@ Product product_kind(int64_t n, int64_t r, int64_t f) {
 }
 
 // x w for x [n, r]; `w` [r, f] and `wt` [f, r]: the one `kind` needs.  Rows of the result go
-// to out_rows if given.
+// to out_rows if given; columns from `cols` on (if given) are padding and may be left unwritten.
 Tensor run_product(Product kind, const Tensor &x, const Tensor &w, const Tensor &wt,
-                   const Tensor &out_rows) {
+                   const Tensor &out_rows, int64_t cols = 0) {
   const int64_t n = x.size(0), r = x.size(1);
   hipStream_t s = current_stream();
   if (kind == Product::kLibrary) {
@@ -521,7 +521,8 @@ Tensor run_product(Product kind, const Tensor &x, const Tensor &w, const Tensor 
   if (kind == Product::kTiled)
     check(mccnn_final_product_wt(s, n, (int)r, f32(x), (int)f, f32(wt), i32(out_rows), f32(out)));
   else
-    check(mccnn_final_product(s, n, (int)r, f32(x), (int)f, f32(w), i32(out_rows), f32(out)));
+    check(mccnn_final_product_padded(s, n, (int)r, f32(x), (int)f, (int)(cols > 0 ? cols : f),
+                                     f32(w), i32(out_rows), f32(out)));
   return out;
 }
 
@@ -578,6 +579,8 @@ struct Plan {
   int64_t act;
   int64_t k() const { return per * h_pad; }
   int64_t f() const { return per * g_pad; }
+  // output columns without the padding that only follows them, in sixteens
+  int64_t cols() const { return per == 1 ? (g + 15) / 16 * 16 : f(); }
   bool padded() const { return c_pad != c || h_pad != h || g_pad != g || per != 1; }
 };
 
@@ -685,7 +688,7 @@ struct McConv : torch::autograd::Function<McConv> {
                     grads);
       const Tensor proj = mc_project(p, *w, feats, geo->points_in, geo->points_out, geo->table,
                                      geo->ranges, geo->inv_radii, geo->pdf);
-      outs.push_back(run_product(w->forward, proj, w->w, w->wt, geo->centre_rows));
+      outs.push_back(run_product(w->forward, proj, w->w, w->wt, geo->centre_rows, p.cols()));
       if (grads) packs.push_back(c10::IValue::make_capsule(w));
     }
     if (grads) {
@@ -794,7 +797,7 @@ struct KpConv : torch::autograd::Function<KpConv> {
                   grads);
     const Tensor proj = kp_project(kp, kernel_points, p.k(), feats, geo->points_in,
                                    geo->points_out, geo->table, geo->ranges, geo->inv_radii);
-    Tensor out = run_product(w->forward, proj, w->w, w->wt, geo->centre_rows);
+    Tensor out = run_product(w->forward, proj, w->w, w->wt, geo->centre_rows, p.cols());
     if (grads) {
       ctx->save_for_backward({feats, weights, kernel_points});
       ctx->saved_data["geo"] = c10::IValue::make_capsule(geo);

@@ -427,10 +427,23 @@ extern "C" int mccnn_final_product_supported(int num_cols_in, int num_cols_out) 
 extern "C" int mccnn_final_product(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
                                    const float *x, int num_cols_out, const float *w,
                                    const int32_t *out_rows, float *out) {
+  return mccnn_final_product_padded(stream, num_rows, num_cols_in, x, num_cols_out, num_cols_out, w,
+                                    out_rows, out);
+}
+
+// The blocks of columns and of the reduction, and with them the order of the sums, go by the
+// columns that count: 48 columns padded to 64 (for the tiled product of large inputs) would sum in
+// another order as one block of 64 than as three of 16, and a network's activations with it.
+extern "C" int mccnn_final_product_padded(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
+                                          const float *x, int num_cols_out, int num_cols,
+                                          const float *w, const int32_t *out_rows, float *out) {
   MCCNN_REQUIRE(mccnn_final_product_supported(num_cols_in, num_cols_out),
                 "final_product supports a multiple of 256 (at most 8192) input columns and a "
                 "multiple of 16 (at most 1024) output columns (got %d x %d)", num_cols_in,
                 num_cols_out);
+  MCCNN_REQUIRE(num_cols > 0 && num_cols <= num_cols_out && num_cols % 16 == 0,
+                "final_product expects a multiple of 16 of its columns to count (got %d of %d)",
+                num_cols, num_cols_out);
   MCCNN_REQUIRE(num_rows >= 0 && num_rows < ((int64_t)1 << 31),
                 "final_product expects a size in [0, 2^31)");
   if (num_rows == 0) return MCCNN_OK;
@@ -450,11 +463,13 @@ extern "C" int mccnn_final_product(mccnn_stream_t stream, int64_t num_rows, int 
               (F / (F % 128 == 0 ? 128 : 64)) >= cus)
     return launch_tile_product(s, num_rows, R, x, F, w, false, out_rows, out);
   int rb = 0, fb = 0;
-  product_blocks(R, F, &rb, &fb);
+  const bool fits = product_blocks(R, num_cols, &rb, &fb) && F % fb == 0;
+  const int cols = fits ? num_cols : F;
+  if (!fits) product_blocks(R, F, &rb, &fb);
   // A small input leaves compute units idle: narrower column blocks with longer reduction
   // blocks then give more blocks of threads, each walking fewer blocks of the reduction
   // (1500 rows x 4096 x 256: 8 visits of 512 rows of w per block of threads become 4 of 1024)
-  while (fb > 16 && rb < 1024 && R % (2 * rb) == 0 && tiles * (F / (fb / 2)) <= cus) {
+  while (fb > 16 && rb < 1024 && R % (2 * rb) == 0 && tiles * (cols / (fb / 2)) <= cus) {
     fb /= 2;
     rb *= 2;
   }
@@ -467,7 +482,7 @@ extern "C" int mccnn_final_product(mccnn_stream_t stream, int64_t num_rows, int 
   ld.ldo = F;
   ld.r_total = R;
   ld.f_block = fb;
-  const int col_blocks = F / fb;
+  const int col_blocks = cols / fb;
   // one block per compute unit in all (the register-resident weights and the LDS tile
   // fill it), shared among the column blocks; never more blocks than tiles
   int64_t per = cus / col_blocks < 1 ? 1 : cus / col_blocks;

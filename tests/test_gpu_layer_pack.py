@@ -69,3 +69,22 @@ def test_pack_and_unpack_layer_weights(abi, c, h, g, mlps, first, per, cp, hp, g
         assert torch.equal(got, d[:c, m, :g, m, :h].permute(0, 2, 1))
     assert torch.equal(dkw[first:first + per], kwp[:, :, :h])
     assert torch.equal(dkb[first:first + per], kbp.reshape(per, hp)[:, :h])
+
+
+@pytest.mark.parametrize("n,r,cols,padded", [(1, 256, 48, 64), (3000, 256, 48, 64), (700, 1024, 96, 128),
+                                             (5000, 1024, 160, 192), (33, 2048, 80, 128)])
+def test_padded_columns_leave_the_bits_alone(n, r, cols, padded):
+    """The product with zero columns behind the weights equals the one without, bit for bit."""
+    from ctypes import c_int64
+    from tensorflow_graphics_point_clouds_amd import _lib
+    from tensorflow_graphics_point_clouds_amd._lib import cint, ptr, stream
+    gen = torch.Generator(device="cuda").manual_seed(n + r)
+    x = torch.randn(n, r, device="cuda", generator=gen)
+    w = torch.randn(r, cols, device="cuda", generator=gen)
+    wide = torch.nn.functional.pad(w, (0, padded - cols)).contiguous()
+    expect, got = torch.empty(n, cols, device="cuda"), torch.empty(n, padded, device="cuda")
+    _lib.call("final_product", stream(), c_int64(n), cint(r), ptr(x), cint(cols), ptr(w),
+              ptr(None), ptr(expect))
+    _lib.call("final_product_padded", stream(), c_int64(n), cint(r), ptr(x), cint(padded),
+              cint(cols), ptr(wide), ptr(None), ptr(got))
+    assert torch.equal(got[:, :cols], expect)
