@@ -613,9 +613,12 @@ def isolated_basis_proj(torch, pc, synthetic, tfg, _lib, radius=0.04, steps=5, g
         for _ in range(steps):
             tfg._basis_proj_raw(basis, feat, ids, ranges, None)
             tfg.basis_proj_grads(basis, feat, ids, ranges, up, None)
-        t = {k.replace("_ordered", ""): v for k, v in _lib.collect_timing().items()}
+        t = {k.replace("_ordered", "").replace("_grouped", ""): v
+             for k, v in _lib.collect_timing().items()}
         for name in ("basis_proj", "basis_proj_grads"):
-            ms = sum(t[name]) / len(t[name])
+            ms = sum(t[name]) / steps
+            if name == "basis_proj_grads":        # the grouped form orders the centres first
+                ms += sum(t.get("neighbourhood_order", [])) / steps
             by = op_bytes(name, M, N, N, C, K, 3)
             entry = {"ms": ms}
             entry.update(roofline_entry(compulsory_bytes(name, M, N, N, C, K, 3), by, ms))
