@@ -424,7 +424,7 @@ int mccnn_basis_proj_grads_grouped(
     size_t workspace_bytes, float *basis_grads_out, float *feature_grads_out);
 
 /* Gradients of batch normalisation over the points followed by the leaky activation (slope 1:
- * none, slope 0: ReLU), the BatchNormalization / LeakyReLU pairs of network_blocks.py:27-465 and
+ * none, slope 0: ReLU; at least 0, since the side of 0 is read off y), the BatchNormalization / LeakyReLU pairs of network_blocks.py:27-465 and
  * modelnet40.py:128-260 (no op of the reference's: TensorFlow's).  x [num_pts, C] the input, y the
  * activated output, mean and inv_std = 1/sqrt(variance + eps) what the forward pass used: the
  * statistics of the points (training != 0) or given ones.  x_grads_out may be NULL. */

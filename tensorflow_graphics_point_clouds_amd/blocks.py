@@ -23,10 +23,11 @@ def _plain_rows(features):
 
 
 def _leaky_slope(activation):
-    """The slope for negative inputs of a leaky activation (0: ReLU), else None."""
+    """The slope for negative inputs of a leaky activation (0: ReLU) that keeps signs, as the
+    gradients of the kernels need it, else None."""
     if activation is torch.relu or type(activation) is torch.nn.ReLU:
         return 0.0
-    if type(activation) is torch.nn.LeakyReLU:
+    if type(activation) is torch.nn.LeakyReLU and activation.negative_slope >= 0:
         return activation.negative_slope
     return None
 
@@ -58,7 +59,8 @@ class BatchNorm(torch.nn.BatchNorm1d):
         if (_plain_rows(features) and features.shape[1] == self.num_features and
                 features.shape[0] > 1 and self.weight is not None and self.momentum is not None and
                 self.running_mean is not None and self.weight.dtype == _F32 and
-                self.running_mean.dtype == _F32 and self.weight.device == features.device):
+                self.running_mean.dtype == _F32 and self.weight.device == features.device and
+                (negative_slope is None or negative_slope >= 0)):
             return _lib.host().norm_act(features, self.weight, self.bias, self.running_mean,
                                         self.running_var, self.num_batches_tracked, training,
                                         self.momentum, self.eps,

@@ -1148,6 +1148,8 @@ struct NormAct : torch::autograd::Function<NormAct> {
 Tensor norm_act(const Tensor &x, const Tensor &weight, const Tensor &bias,
                 const Tensor &running_mean, const Tensor &running_var, const OptTensor &batches,
                 bool training, double momentum, double eps, double slope) {
+  // the gradients take the side of 0 from the result
+  if (!(slope >= 0.0)) throw InvalidArgument("norm_act expects a slope of at least 0");
   return NormAct::apply(x, weight, bias, running_mean, running_var, batches, training, momentum,
                         eps, slope);
 }

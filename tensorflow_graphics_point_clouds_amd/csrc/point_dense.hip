@@ -395,6 +395,7 @@ extern "C" int mccnn_norm_act_grads(mccnn_stream_t stream, int64_t num_pts, int 
                                     float *weight_grads_out, float *bias_grads_out) {
   MCCNN_REQUIRE(num_pts > 0 && num_features > 0 && num_features <= 65535 * 64,
                 "NormActGrads expects points and features");
+  MCCNN_REQUIRE(slope >= 0.0f, "NormActGrads expects a slope of at least 0 (got %g)", slope);
   MCCNN_REQUIRE(x && y && in_grads && mean && inv_std && weight && workspace && weight_grads_out &&
                     bias_grads_out,
                 "NormActGrads received a null tensor");

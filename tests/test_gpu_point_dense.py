@@ -91,3 +91,28 @@ def test_second_derivatives():
     second_expect, = torch.autograd.grad(expect.square().sum(), w)
     assert torch.allclose(first, expect, rtol=1e-4, atol=1e-4)
     assert torch.allclose(second, second_expect, rtol=1e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("slope", [-0.3, -1.0, 0.0, 0.3])
+def test_activation_of_any_slope(slope):
+    """An activation that does not keep signs (a negative slope) has its gradient taken from its
+    input: first and second derivatives against torch's operations in float64."""
+    from tensorflow_graphics_point_clouds_amd import blocks
+    x, g = _rand(300, 6, seed=1) * 2 + 1, _rand(300, 6, seed=2)
+    norm, act = blocks.BatchNorm(6), torch.nn.LeakyReLU(slope)
+    with torch.no_grad():
+        norm.weight.uniform_(0.5, 1.5)
+        norm.bias.normal_()
+
+    def derivatives(x, weight, bias, result):
+        first = torch.autograd.grad(result, (x, weight, bias), g.to(result.dtype),
+                                    create_graph=True)
+        return list(first) + list(torch.autograd.grad(first[0].square().sum(), (x, weight)))
+    a = x.clone().requires_grad_()
+    got = derivatives(a, norm.weight, norm.bias, blocks._norm_act(norm, act, a, True))
+    b, w, c = (t.detach().double().requires_grad_() for t in (x, norm.weight, norm.bias))
+    expect = derivatives(b, w, c, torch.nn.functional.leaky_relu(torch.nn.functional.batch_norm(
+        b, None, None, w, c, True, 0.0, norm.eps), slope))
+    for p, q in zip(got, expect):
+        # chains of some ten float32 roundings, the second derivatives of sums of 300 terms
+        assert (p.double() - q).norm() <= 1e-5 * q.norm()
