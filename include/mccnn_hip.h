@@ -821,7 +821,8 @@ int mccnn_final_product(mccnn_stream_t stream, int64_t num_rows, int num_cols_in
                         const int32_t *out_rows, float *out);
 /* The same for weights whose columns from num_cols on (a multiple of 16) are padding: the first
  * num_cols columns of out get the bits of the product without padding, the others may not be
- * written. */
+ * written.  Not so where num_cols_out columns take the tiled product (see below) and num_cols do
+ * not: its sums are in another order. */
 int mccnn_final_product_padded(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
                                const float *x, int num_cols_out, int num_cols, const float *w,
                                const int32_t *out_rows, float *out);

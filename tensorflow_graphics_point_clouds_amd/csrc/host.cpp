@@ -560,6 +560,20 @@ Tensor projection_grad_product(const Tensor &x, const Tensor &w) {
   return out;
 }
 
+// dout W^T for dout [n, f] and W [r, f] of a layer.  Column counts without a kernel take that of
+// the next multiple of 64 with zero columns in both operands where there is one: nearer to the
+// exact sums than the library's product (48 columns: 9.5e-8 against 1.25e-7 of the result; 96:
+// 1.4e-7 / 1.8e-7) and faster with the padding (400 000 x 48 x 1024: 309 against 590 us, x 96:
+// 569 / 823 us, plus 30 to 60 us for the padded rows).
+Tensor layer_projection_grad(const Tensor &dout, const Tensor &w) {
+  const int64_t f = dout.size(1), wide = (f + 63) / 64 * 64;
+  if (mccnn_projection_grad_product_supported((int)f, (int)w.size(0)) ||
+      !mccnn_projection_grad_product_supported((int)wide, (int)w.size(0)))
+    return projection_grad_product(dout, w);
+  return projection_grad_product(gather_rows(dout, Tensor(), 0, f, wide),
+                                 gather_rows(w, Tensor(), 0, f, wide));
+}
+
 // --------------------------------------------------------------------- convolutions ----
 
 // The neighbourhood of a layer pass in grid order (`_SortedView` of pc.py), and how its pairs
@@ -733,7 +747,7 @@ struct McConv : torch::autograd::Function<McConv> {
       const bool direct = !p.padded() && p.mlps == 1;      // gradients land in the caller's shapes
       Tensor dkw_pad, dkb_pad, ddense;
       if (want_kernel) {
-        const Tensor dproj = projection_grad_product(up, w->w);
+        const Tensor dproj = layer_projection_grad(up, w->w);
         Tensor ws = workspace(mccnn_mc_conv_project_grads_workspace_bytes((int)p.dims, (int)k,
                                                                           n_out), feats);
         dkw_pad = direct ? dkw : empty_f32({p.per, p.dims, p.h_pad}, feats);

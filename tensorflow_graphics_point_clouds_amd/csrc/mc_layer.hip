@@ -432,8 +432,8 @@ extern "C" int mccnn_final_product(mccnn_stream_t stream, int64_t num_rows, int 
 }
 
 // The blocks of columns and of the reduction, and with them the order of the sums, go by the
-// columns that count: 48 columns padded to 64 (for the tiled product of large inputs) would sum in
-// another order as one block of 64 than as three of 16, and a network's activations with it.
+// columns that count: 48 columns padded to 64 (for the tiled product of large inputs, which sums
+// in an order of its own) take three blocks of 16 and not one of 64.
 extern "C" int mccnn_final_product_padded(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
                                           const float *x, int num_cols_out, int num_cols,
                                           const float *w, const int32_t *out_rows, float *out) {
