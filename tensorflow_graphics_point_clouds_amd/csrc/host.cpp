@@ -893,17 +893,36 @@ Plan plan_of(const std::vector<int64_t> &v) {
   return {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9]};
 }
 
+// What the kernels take for granted about the operands of a layer.
+void check_layer(const char *op, const Plan &p, const Tensor &features, const Tensor &points_in,
+                 const Tensor &points_out, const Tensor &point_rows, const Tensor &final_weights,
+                 int64_t weights_in) {
+  auto require = [&](bool ok, const std::string &what) {
+    if (!ok) throw InvalidArgument(std::string(op) + " expects " + what);
+  };
+  require(features.dim() == 2 && features.size(1) == p.c,
+          std::to_string(p.c) + " input features (got " + std::to_string(dim(features, 1)) + ")");
+  require(features.size(0) >= point_rows.size(0), "a row of features per point");
+  require(dim(points_in, 1) == p.dims && dim(points_out, 1) == p.dims,
+          "points of " + std::to_string(p.dims) + " dimensions");
+  require(final_weights.numel() == weights_in * p.g, "weights of the layer's sizes");
+}
+
 Tensor mc_conv(const Tensor &features, const Tensor &kw, const Tensor &kb, const Tensor &fw,
                const std::vector<int64_t> &plan, bool grads, const Tensor &points_in,
                const Tensor &points_out, const Tensor &table, const Tensor &ranges,
                const OptTensor &table_t, const OptTensor &ranges_t, const Tensor &point_rows,
                const OptTensor &centre_rows, const Tensor &pdf, const OptTensor &pdf_t,
                const Tensor &inv_radii, const OptTensor &neg_inv_radii) {
+  const Plan p = plan_of(plan);
+  check_layer("MCConv", p, features, points_in, points_out, point_rows, fw, p.mlps * p.c * p.h);
+  if (kw.numel() != p.mlps * p.dims * p.h || kb.numel() != p.mlps * p.h)
+    throw InvalidArgument("MCConv expects kernel weights of the layer's sizes");
   return McConv::apply(features.contiguous(), kw.contiguous(), kb.contiguous(), fw.contiguous(),
                        make_geometry(points_in, points_out, table, ranges, table_t, ranges_t,
                                      point_rows, centre_rows, pdf, pdf_t, inv_radii,
                                      neg_inv_radii),
-                       plan_of(plan), grads);
+                       p, grads);
 }
 
 Tensor kp_conv(const Tensor &features, const Tensor &weights, const Tensor &kernel_points,
@@ -912,11 +931,15 @@ Tensor kp_conv(const Tensor &features, const Tensor &weights, const Tensor &kern
                const Tensor &ranges, const OptTensor &table_t, const OptTensor &ranges_t,
                const Tensor &point_rows, const OptTensor &centre_rows, const Tensor &inv_radii,
                const OptTensor &neg_inv_radii) {
+  const Plan p = plan_of(plan);
+  check_layer("KPConv", p, features, points_in, points_out, point_rows, weights, p.c * p.h);
+  if (dim(kernel_points, 0) != p.h || dim(kernel_points, 1) != p.dims)
+    throw InvalidArgument("KPConv expects kernel points of the layer's sizes");
   return KpConv::apply(features.contiguous(), weights.contiguous(), kernel_points,
                        make_geometry(points_in, points_out, table, ranges, table_t, ranges_t,
                                      point_rows, centre_rows, OptTensor(), OptTensor(), inv_radii,
                                      neg_inv_radii),
-                       plan_of(plan), KpShape{kernel_points.size(0), kind, sigma}, grads);
+                       p, KpShape{kernel_points.size(0), kind, sigma}, grads);
 }
 
 // -------------------------------------------------------------------------- pooling ----

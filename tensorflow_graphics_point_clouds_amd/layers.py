@@ -406,7 +406,15 @@ class MCConv(torch.nn.Module):
         return torch.cat([_dense_product(p[mlp].contiguous(), self.final_weights[mlp])
                           for mlp in range(l)], dim=1)
 
-    def _convolve_on_view(self, features, neighborhood, radii):
+    def _view_plan(self):
+        """The plan for the final weights as they are: they decide the output columns."""
+        g = self.final_weights.shape[-1]
+        if self._plan is None or self._plan[3] == g:
+            return self._plan
+        return _layer_plan(self._num_dims, self._num_features_in, g * self._num_mlps,
+                           self._num_mlps, self._hidden, self._act)
+
+    def _convolve_on_view(self, plan, features, neighborhood, radii):
         """The layer on the grid-ordered view (csrc/host.cpp); channel counts its kernels do
         not cover are zero-padded on the way in and the result is cut back."""
         inv_radii = pc._reciprocal(radii)
@@ -427,7 +435,7 @@ class MCConv(torch.nn.Module):
         view = neighborhood.sorted_view()
         pdf, pdf_t = view.pair_pdf(neighborhood, grads)
         return _lib.host().mc_conv(
-            features, self.weights, self.biases, self.final_weights, self._plan, grads,
+            features, self.weights, self.biases, self.final_weights, plan, grads,
             *view.tensors(grads), pdf, pdf_t if grads else None, inv_radii,
             pc._negative(inv_radii) if grads else None)
 
@@ -446,8 +454,9 @@ class MCConv(torch.nn.Module):
             pdf = _differentiable_pdf(neighborhood, bandwidth) if moving else None
             return self._convolve_deep(features, point_cloud_in, point_cloud_out, radii,
                                        neighborhood, pdf)
-        if self.fused and self.transposed_grads and self._plan is not None:
-            return self._convolve_on_view(features, neighborhood, radii)
+        plan = self._view_plan() if self.fused and self.transposed_grads else None
+        if plan is not None:
+            return self._convolve_on_view(plan, features, neighborhood, radii)
         biases = self.biases.reshape(self._num_mlps, self._hidden)
         k = self._num_mlps * self._hidden
         fused = self.fused and _lib.lib().mccnn_mc_conv_supported(
@@ -942,10 +951,13 @@ def _offset_columns(cols):
     return -(-cols // 64) * 64 if cols > 32 else -(-cols // 16) * 16
 
 
-def _kp_rigid(weights, plan, features, neighborhood, inv_radii, kernel_points, k, kind, sigma):
-    """Rigid kernel-point convolution with weights [C*KP, F]."""
+def _kp_rigid(weights, plan, c, features, neighborhood, inv_radii, kernel_points, k, kind, sigma):
+    """Rigid kernel-point convolution of features [N, C] with weights [C*KP, F]."""
     if plan is None:
-        c, kp = features.shape[1], kernel_points.shape[0]
+        if features.shape[1] != c:
+            raise _lib.InvalidArgumentError("KPConv expects %d input features (got %d)" %
+                                            (c, features.shape[1]))
+        kp = kernel_points.shape[0]
         dense = torch.nn.functional.pad(weights.reshape(c, kp, -1), (0, 0, 0, k - kp))
         return _KPConvRigidLayer.apply(dense.reshape(c * k, -1), features, neighborhood, inv_radii,
                                        kernel_points, k, kind, sigma)
@@ -1111,7 +1123,10 @@ class KPConv(torch.nn.Module):
             return self._convolve_moving(features, point_cloud_in, point_cloud_out, radii,
                                          neighborhood, sigma)
         if not self.deformable and self.transposed_grads:
-            return _kp_rigid(self.weights, self._plan, features, neighborhood,
+            plan, f = self._plan, self.weights.numel() // (c * kp)
+            if plan is not None and plan[3] != f:         # the weights decide the output columns
+                plan = _kp_plan(d, c, f, kp, k)
+            return _kp_rigid(self.weights, plan, c, features, neighborhood,
                              pc._reciprocal(radii), self._kernel_points, k, self._kind, sigma)
         if self.deformable and self.transposed_grads and k == 16 and d in (2, 3) and \
                 _lib.lib().mccnn_kp_deform_offset_grads_supported(cint(d), cint(c)):
@@ -1130,7 +1145,7 @@ class KPConv(torch.nn.Module):
         offsets = None
         if self.deformable:       # KPConv.py:317-392: offsets from a rigid convolution
             if self.transposed_grads and k in (16, 32):
-                offsets = _kp_rigid(self.offset_weights, self._offset_plan, features, neighborhood,
+                offsets = _kp_rigid(self.offset_weights, self._offset_plan, c, features, neighborhood,
                                     pc._reciprocal(radii), self._kernel_points, k, self._kind,
                                     sigma)
             else:
@@ -1151,8 +1166,8 @@ class KPConv(torch.nn.Module):
         kp, k, d = self._num_kernel_points, self._num_basis, self._num_dims
         view = neighborhood.sorted_view()
         inv_radii = pc._reciprocal(radii)
-        offsets = _kp_rigid(self.offset_weights, self._offset_plan, features, neighborhood,
-                            inv_radii, self._kernel_points, k, self._kind, sigma)
+        offsets = _kp_rigid(self.offset_weights, self._offset_plan, self._num_features_in, features,
+                            neighborhood, inv_radii, self._kernel_points, k, self._kind, sigma)
         offsets = offsets.reshape(-1, kp, d)
         self.last_offsets = offsets
         on_view = offsets if view.centre_order is None else \

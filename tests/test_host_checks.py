@@ -17,3 +17,39 @@ def test_norm_act_takes_only_activations_that_keep_signs():
         assert blocks._leaky_slope(torch.nn.LeakyReLU(slope)) is None
     assert blocks._leaky_slope(torch.nn.LeakyReLU(0.3)) == 0.3
     _lib.host().norm_act(x, *args, 0.3)
+
+
+def _layer_arguments(points=40, dims=3):
+    """Operands of a layer pass on host memory: what is checked is checked before the GPU."""
+    pts = torch.zeros(points, dims)
+    table, ranges = torch.zeros(4, 2, dtype=torch.int32), torch.zeros(points, dtype=torch.int32)
+    rows = torch.zeros(points, dtype=torch.int32)
+    return (pts, pts, table, ranges, None, None, rows, None), torch.ones(dims)
+
+
+@pytest.mark.parametrize("features,dims,kernel,final", [
+    ((40, 7), 3, (1, 3, 16), (1, 96, 32)), ((40, 5), 3, (1, 3, 16), (1, 96, 32)),
+    ((39, 6), 3, (1, 3, 16), (1, 96, 32)), ((40, 6), 2, (1, 3, 16), (1, 96, 32)),
+    ((40, 6), 3, (1, 3, 8), (1, 96, 32)), ((40, 6), 3, (1, 3, 16), (1, 96, 16))])
+def test_monte_carlo_layer_checks_its_operands(features, dims, kernel, final):
+    """Surplus feature columns are not dropped in silence, and no kernel reads past an operand."""
+    from tensorflow_graphics_point_clouds_amd import layers
+    geometry, inv_radii = _layer_arguments(dims=dims)
+    plan = layers._layer_plan(3, 6, 32, 1, 16, 0)
+    with pytest.raises(_lib.InvalidArgumentError):
+        _lib.host().mc_conv(torch.zeros(features), torch.zeros(kernel), torch.zeros(1, 16),
+                            torch.zeros(final), plan, False, *geometry, torch.zeros(4), None,
+                            inv_radii, None)
+
+
+@pytest.mark.parametrize("features,dims,weights,kernel_points", [
+    ((40, 7), 3, (90, 32), 15), ((40, 5), 3, (90, 32), 15), ((39, 6), 3, (90, 32), 15),
+    ((40, 6), 2, (90, 32), 15), ((40, 6), 3, (90, 16), 15), ((40, 6), 3, (90, 32), 14)])
+def test_kernel_point_layer_checks_its_operands(features, dims, weights, kernel_points):
+    from tensorflow_graphics_point_clouds_amd import layers
+    geometry, inv_radii = _layer_arguments(dims=dims)
+    plan = layers._kp_plan(3, 6, 32, 15, 16)
+    with pytest.raises(_lib.InvalidArgumentError):
+        _lib.host().kp_conv(torch.zeros(features), torch.zeros(weights),
+                            torch.zeros(kernel_points, 3), plan, 0, 1.0, False, *geometry,
+                            inv_radii, None)
