@@ -192,6 +192,10 @@ struct GridTensors {
 GridTensors build_grid(const Tensor &points, const Tensor &bids, int64_t batch,
                        const Tensor &cell_sizes) {
   const int64_t n = points.size(0), d = points.size(1);
+  if (cell_sizes.numel() < d)
+    throw InvalidArgument("BuildGrid expects a cell size for each of the points' dimensions");
+  if (bids.size(0) != n)
+    throw InvalidArgument("BuildGrid expects the same number of batch ids as number of points");
   GridTensors g;
   g.aabb_min = empty_f32({batch, d}, points);
   g.aabb_max = empty_f32({batch, d}, points);
@@ -225,11 +229,15 @@ GridTensors build_grid(const Tensor &points, const Tensor &bids, int64_t batch,
   return g;
 }
 
+void check_search(const Tensor &samples, const Tensor &sbids, const Tensor &num_cells,
+                  const Tensor &smin, const Tensor &inv_cell);
+
 // Centres in the order of their cells in a grid -> (order, coordinates, cloud ids).
 std::tuple<Tensor, Tensor, Tensor> order_centres(const Tensor &samples, const Tensor &bids,
                                                  int64_t batch, const Tensor &num_cells,
                                                  const Tensor &smin, const Tensor &inv_cell,
                                                  int64_t key_bits) {
+  check_search(samples, bids, num_cells, smin, inv_cell);
   const int64_t n = samples.size(0), d = samples.size(1);
   Tensor order = empty_i32({n}, samples), pts = empty_f32({n, d}, samples),
          out_bids = empty_i32({n}, samples);
@@ -299,6 +307,39 @@ std::tuple<Tensor, Tensor, bool> find_neighbors(const Tensor &samples, const Ten
   return {ranges, neighbors, symmetric};
 }
 
+// What find_neighbors asks of its arguments, for the entries below that skip its checks: a sample
+// cloud, radii or a grid of another number of dimensions would be read out of range.
+void check_search(const Tensor &samples, const Tensor &sbids, const Tensor &num_cells,
+                  const Tensor &smin, const Tensor &inv_cell) {
+  const int64_t d = dim(samples, 1);
+  auto require = [](bool ok, const char *what) {
+    if (!ok) throw InvalidArgument(std::string("FindNeighbors expects ") + what);
+  };
+  require(num_cells.numel() == d,
+          "a number of dimensions in num_cells equal to the number of dimensions in the samples");
+  require(dim(smin, 1) == d,
+          "a number of dimensions in scaled_aabb_min equal to the number of dimensions in the "
+          "samples");
+  require(inv_cell.numel() == d,
+          "a number of dimensions in inv_cell_sizes equal to the number of dimensions in the "
+          "samples");
+  require(sbids.size(0) == samples.size(0), "the same number of batch ids as samples");
+}
+
+void check_search(const Tensor &samples, const Tensor &sbids, const Tensor &points,
+                  const Tensor &keys, const Tensor &num_cells, const Tensor &smin,
+                  const Tensor &inv_cell, const Tensor &inv_radii) {
+  check_search(samples, sbids, num_cells, smin, inv_cell);
+  if (dim(points, 1) != dim(samples, 1))
+    throw InvalidArgument("FindNeighbors expects a number of dimensions in points equal to the "
+                          "number of dimensions in the samples");
+  if (inv_radii.numel() != dim(samples, 1))
+    throw InvalidArgument("FindNeighbors expects a number of dimensions in inv_radii equal to the "
+                          "number of dimensions in the input points");
+  if (keys.size(0) != points.size(0))
+    throw InvalidArgument("FindNeighbors expects the same number of keys as points");
+}
+
 // The same for the structures of pc.py, which hold the grid: its column table is optional (for
 // a small cloud it would need the grid's shape on the host first).
 // -> (ranges, neighbors, whether a neighbourhood was cut at max_neighs)
@@ -307,6 +348,7 @@ std::tuple<Tensor, Tensor, bool> search(const Tensor &samples, const Tensor &sbi
                                         const OptTensor &ds, const Tensor &num_cells,
                                         const Tensor &smin, const Tensor &inv_cell,
                                         const Tensor &inv_radii, int64_t max_neighs) {
+  check_search(samples, sbids, points, keys, num_cells, smin, inv_cell, inv_radii);
   const int64_t ns = samples.size(0);
   const int nd = (int)dim(samples, 1);
   Tensor ws = workspace(mccnn_find_neighbors_workspace_bytes(nd, ns), samples);
@@ -335,8 +377,12 @@ Tensor grid_density(const Tensor &points, const Tensor &bids, const Tensor &keys
                     const OptTensor &ds, const Tensor &num_cells, const Tensor &smin,
                     const Tensor &inv_cell, const Tensor &inv_radii, const Tensor &inv_bandwidth,
                     int64_t mode) {
+  check_search(points, bids, points, keys, num_cells, smin, inv_cell, inv_radii);
   const int64_t n = points.size(0);
   const int nd = (int)dim(points, 1);
+  if (inv_bandwidth.numel() != nd)
+    throw InvalidArgument("ComputePDF expects a number of dimensions in inv_bandwidth equal to the "
+                          "number of dimensions in the input points");
   Tensor ws = workspace(mccnn_grid_density_workspace_bytes(nd, n), points);
   Tensor pdf = empty_f32({n}, points);
   hipStream_t s = current_stream();

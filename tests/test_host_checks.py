@@ -53,3 +53,30 @@ def test_kernel_point_layer_checks_its_operands(features, dims, weights, kernel_
         _lib.host().kp_conv(torch.zeros(features), torch.zeros(weights),
                             torch.zeros(kernel_points, 3), plan, 0, 1.0, False, *geometry,
                             inv_radii, None)
+
+
+def _grid_arguments(dims, points=8):
+    """(points, cloud ids, keys, column table, num_cells, scaled minimum, inverse cell size)."""
+    return (torch.zeros(points, dims), torch.zeros(points, dtype=torch.int32),
+            torch.zeros(points, dtype=torch.int64), None, torch.ones(dims, dtype=torch.int32),
+            torch.zeros(1, dims), torch.ones(dims))
+
+
+@pytest.mark.parametrize("samples,grid,radii", [(2, 3, 3), (3, 2, 2), (3, 2, 3), (3, 3, 2), (2, 2, 3)])
+def test_searches_check_dimensions(samples, grid, radii):
+    """Centres, grid and radii of different dimensions are refused as find_neighbors refuses
+    them: the kernels would read past the shorter one."""
+    host = _lib.host()
+    centres, ids = torch.zeros(5, samples), torch.zeros(5, dtype=torch.int32)
+    args = _grid_arguments(grid)
+    with pytest.raises(_lib.InvalidArgumentError, match="dimensions"):
+        host.search(centres, ids, *args[:1], *args[2:], torch.ones(radii), 0)
+    with pytest.raises(_lib.InvalidArgumentError, match="dimensions"):
+        host.grid_density(*args, torch.ones(radii), torch.ones(5 - grid), 0)
+    if samples != grid:
+        with pytest.raises(_lib.InvalidArgumentError, match="dimensions"):
+            host.order_centres(centres, ids, 1, *args[4:], 0)
+    with pytest.raises(_lib.InvalidArgumentError, match="batch ids"):
+        host.search(torch.zeros(5, grid), ids[:4], *args[:1], *args[2:], torch.ones(grid), 0)
+    with pytest.raises(_lib.InvalidArgumentError, match="cell size"):
+        host.build_grid(torch.zeros(5, 3), ids, 1, torch.ones(2))
