@@ -143,9 +143,11 @@ class PointCloud:
             clouds, v = int(math.prod(self._batch_shape)), points.shape[-2]
             if self._sizes is None and points.shape[-1] > 0:     # no padding: every row is a point
                 self._sizes = torch.full(self._batch_shape, v, dtype=_I32, device=dev)
-                self._points = points.reshape(clouds * v, -1).contiguous()
+                # a copy, as with sizes: the caller may refill a padded buffer
+                self._points = points.reshape(clouds * v, -1).clone(
+                    memory_format=torch.contiguous_format)
                 self._batch_ids = torch.arange(clouds, dtype=_I32, device=dev)[:, None] \
-                    .expand(clouds, v).reshape(-1)
+                    .expand(clouds, v).reshape(-1).contiguous()    # (one cloud: still a view)
                 self._batch_size = int(clouds if batch_size is None else batch_size)
                 self._dimension = self._points.shape[1]
                 return

@@ -37,6 +37,22 @@ def test_padded_input_without_sizes_and_with_batch_shape():
     assert cloud.get_points(max_num_points=5).shape == (2, 2, 5, 2)
 
 
+@pytest.mark.parametrize("clouds", [1, 2])
+def test_padded_input_without_sizes_is_copied(clouds):
+    """A padded buffer that the caller refills leaves the cloud as it was; what kernels read is
+    contiguous, for a single cloud as well."""
+    pts = torch.rand(clouds, 5, 3, requires_grad=True)
+    before = pts.detach().clone().reshape(-1, 3)
+    cloud = pc.PointCloud(pts)
+    with torch.no_grad():
+        pts.zero_()
+    assert torch.equal(cloud._points.detach(), before)
+    assert cloud._points.is_contiguous() and cloud._batch_ids.is_contiguous()
+    assert cloud._batch_ids.tolist() == [b for b in range(clouds) for _ in range(5)]
+    cloud._points.sum().backward()
+    assert torch.equal(pts.grad, torch.ones_like(pts))
+
+
 def test_segmented_input_from_sizes_and_unsorted_batch_ids():
     rng = np.random.default_rng(1)
     pts = rng.random((7, 2)).astype(np.float32)
