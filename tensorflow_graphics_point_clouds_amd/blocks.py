@@ -6,6 +6,8 @@ the spatial convolutions inside the blocks are the layers of `layers.py`."""
 import math
 
 import torch
+from torch.autograd import forward_ad
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _lib, layers, pc
 
@@ -16,26 +18,46 @@ layer_types = {"mcconv": layers.MCConv, "mc": layers.MCConv, "mc_conv": layers.M
                "pointconv": layers.PointConv, "point_conv": layers.PointConv}
 
 
+def _eager():
+    """Whether nothing looks at the operations themselves: forward-mode derivatives, torch.func
+    transforms, tracing and compilation see torch's operations, not the kernels' nodes."""
+    return not (forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active() or
+                torch.compiler.is_compiling() or torch.jit.is_tracing())
+
+
 def _plain_rows(features):
     """float32 rows on the GPU that the per-point kernels take."""
     return (features.is_cuda and features.dtype == _F32 and features.dim() == 2 and
-            features.is_contiguous() and not torch.is_autocast_enabled("cuda"))
+            features.is_contiguous() and type(features) in (torch.Tensor, torch.nn.Parameter) and
+            not torch.is_autocast_enabled("cuda") and _eager())
+
+
+def _bare(module, kind):
+    """Whether calling the module is calling `kind`'s forward and nothing else: no hooks, no
+    forward of a subclass or of the instance's own."""
+    return (type(module).forward is kind.forward and "forward" not in module.__dict__ and
+            not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or
+                 module._backward_pre_hooks or _has_any_global_hook()))
 
 
 def _leaky_slope(activation):
     """The slope for negative inputs of a leaky activation (0: ReLU) that keeps signs, as the
     gradients of the kernels need it, else None."""
-    if activation is torch.relu or type(activation) is torch.nn.ReLU:
+    if activation is torch.relu:
         return 0.0
-    if type(activation) is torch.nn.LeakyReLU and activation.negative_slope >= 0:
+    if isinstance(activation, torch.nn.ReLU) and _bare(activation, torch.nn.ReLU):
+        return 0.0
+    if (isinstance(activation, torch.nn.LeakyReLU) and _bare(activation, torch.nn.LeakyReLU) and
+            activation.negative_slope >= 0):
         return activation.negative_slope
     return None
 
 
 def _norm_act(norm, activation, features, training=None):
-    """activation(norm(features)), in the kernel of the normalisation if it can be."""
+    """activation(norm(features)), in the kernel of the normalisation if nothing looks between
+    the two or at either of them."""
     slope = _leaky_slope(activation)
-    if slope is None or not isinstance(norm, BatchNorm):
+    if slope is None or not (isinstance(norm, BatchNorm) and _bare(norm, BatchNorm)):
         return activation(norm(features, training))
     return norm(features, training, slope)
 
