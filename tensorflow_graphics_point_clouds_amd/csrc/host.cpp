@@ -644,49 +644,64 @@ struct Plan {
   bool padded() const { return c_pad != c || h_pad != h || g_pad != g || per != 1; }
 };
 
-// What the kernels read of one sub-layer's weights.
-struct Packed : torch::CustomClassHolder {
+// What the kernels read of one sub-layer's weights.  Between the passes what the backward reads of
+// it rides among the saved tensors, so that autograd frees it afterwards.
+struct Packed {
   Tensor w, wt, w2, w2t, kw, kb;
-  Product forward = Product::kRegisters, transposed = Product::kRegisters;
+  Product forward = Product::kRegisters;
+  static constexpr size_t kTensors = 5;
+  void save(variable_list &to) const { to.insert(to.end(), {w, w2, w2t, kw, kb}); }
+  static Packed saved(const variable_list &from, size_t first) {
+    return {from[first],     Tensor(),        from[first + 1],
+            from[first + 2], from[first + 3], from[first + 4]};
+  }
 };
 
-c10::intrusive_ptr<Packed> pack(const Plan &p, int64_t first, const Tensor &final_weights,
-                                const Tensor &kw, const Tensor &kb, int64_t n_out, int64_t n_in,
-                                bool need_w, bool need_transposed) {
-  auto out = c10::make_intrusive<Packed>();
+Packed pack(const Plan &p, int64_t first, const Tensor &final_weights,
+            const Tensor &kw, const Tensor &kb, int64_t n_out, int64_t n_in, bool need_w,
+            bool need_transposed) {
+  Packed out;
   const int64_t k = p.k(), f = p.f(), r = p.c_pad * k;
-  out->forward = product_kind(n_out, r, f);
-  out->transposed = product_kind(n_in, f * k, p.c_pad);
+  out.forward = product_kind(n_out, r, f);
+  const Product transposed = product_kind(n_in, f * k, p.c_pad);
   const bool plain = !p.padded();
-  if (need_w || out->forward != Product::kTiled)
-    out->w = plain && p.mlps == 1 ? final_weights.view({r, f}) : empty_f32({r, f}, final_weights);
-  if (out->forward == Product::kTiled) out->wt = empty_f32({f, r}, final_weights);
+  if (need_w || out.forward != Product::kTiled)
+    out.w = plain && p.mlps == 1 ? final_weights.view({r, f}) : empty_f32({r, f}, final_weights);
+  if (out.forward == Product::kTiled) out.wt = empty_f32({f, r}, final_weights);
   if (need_transposed) {
-    if (out->transposed == Product::kTiled) out->w2t = empty_f32({p.c_pad, f * k}, final_weights);
-    else out->w2 = empty_f32({f * k, p.c_pad}, final_weights);
+    if (transposed == Product::kTiled) out.w2t = empty_f32({p.c_pad, f * k}, final_weights);
+    else out.w2 = empty_f32({f * k, p.c_pad}, final_weights);
   }
   const bool kernel = kw.defined();
   if (kernel) {
     if (plain && p.mlps == 1) {
-      out->kw = kw;
-      out->kb = kb;
+      out.kw = kw;
+      out.kb = kb;
     } else {
-      out->kw = empty_f32({p.per, p.dims, p.h_pad}, kw);
-      out->kb = empty_f32({k}, kb);
+      out.kw = empty_f32({p.per, p.dims, p.h_pad}, kw);
+      out.kb = empty_f32({k}, kb);
     }
   }
-  const bool pack_w = out->w.defined() && !(plain && p.mlps == 1);
+  const bool pack_w = out.w.defined() && !(plain && p.mlps == 1);
   const bool pack_kernel = kernel && !(plain && p.mlps == 1);
-  if (pack_w || out->wt.defined() || out->w2.defined() || out->w2t.defined() || pack_kernel) {
+  if (pack_w || out.wt.defined() || out.w2.defined() || out.w2t.defined() || pack_kernel) {
     hipStream_t s = current_stream();
     Region t("pack_layer_weights", s);
     check(mccnn_pack_layer_weights(
         s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, (int)first, (int)p.per, (int)p.c_pad,
         (int)p.h_pad, (int)p.g_pad, f32(final_weights), f32(kw), f32(kb),
-        pack_w ? f32(out->w) : nullptr, f32(out->wt), f32(out->w2), f32(out->w2t),
-        pack_kernel ? f32(out->kw) : nullptr, pack_kernel ? f32(out->kb) : nullptr));
+        pack_w ? f32(out.w) : nullptr, f32(out.wt), f32(out.w2), f32(out.w2t),
+        pack_kernel ? f32(out.kw) : nullptr, pack_kernel ? f32(out.kb) : nullptr));
   }
   return out;
+}
+
+// The product of the feature gradient, q w2.
+Tensor transposed_product(const Tensor &q, const Packed &w, const Tensor &out_rows) {
+  if (w.w2t.defined()) return run_product(Product::kTiled, q, Tensor(), w.w2t, out_rows);
+  const bool covered = mccnn_final_product_supported((int)q.size(1), (int)w.w2.size(1));
+  return run_product(covered ? Product::kRegisters : Product::kLibrary, q, w.w2, Tensor(),
+                     out_rows);
 }
 
 Tensor mc_project(const Plan &p, const Packed &w, const Tensor &feats, const Tensor &pin,
@@ -745,19 +760,17 @@ struct McConv : torch::autograd::Function<McConv> {
     const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
     const int64_t n_out = geo->ranges.size(0);
     std::vector<Tensor> outs;
-    c10::List<c10::IValue> packs(c10::AnyType::get());
+    variable_list saved = {feats, kw, kb, final_weights, p.c == p.c_pad ? features : Tensor()};
     for (int64_t first = 0; first < p.mlps; first += p.per) {
-      auto w = pack(p, first, final_weights, kw, kb, n_out, feats.size(0), grads,
-                    grads);
-      const Tensor proj = mc_project(p, *w, feats, geo->points_in, geo->points_out, geo->table,
+      const Packed w = pack(p, first, final_weights, kw, kb, n_out, feats.size(0), grads, grads);
+      const Tensor proj = mc_project(p, w, feats, geo->points_in, geo->points_out, geo->table,
                                      geo->ranges, geo->inv_radii, geo->pdf, geo->centre_rows);
-      outs.push_back(run_product(w->forward, proj, w->w, w->wt, Tensor(), p.cols()));
-      if (grads) packs.push_back(c10::IValue::make_capsule(w));
+      outs.push_back(run_product(w.forward, proj, w.w, w.wt, Tensor(), p.cols()));
+      if (grads) w.save(saved);
     }
     if (grads) {
-      ctx->save_for_backward({feats, kw, kb, final_weights, p.c == p.c_pad ? features : Tensor()});
+      ctx->save_for_backward(std::move(saved));
       ctx->saved_data["geo"] = c10::IValue::make_capsule(geo);
-      ctx->saved_data["packs"] = packs;
       ctx->saved_data["plan"] = std::vector<int64_t>{p.dims, p.c, p.h, p.g, p.mlps, p.c_pad,
                                                      p.h_pad, p.g_pad, p.per, p.act};
     }
@@ -772,7 +785,6 @@ struct McConv : torch::autograd::Function<McConv> {
     const Plan p{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9]};
     const auto geo = c10::static_intrusive_pointer_cast<Geometry>(
         ctx->saved_data["geo"].toCapsule());
-    const auto packs = ctx->saved_data["packs"].toList();
     const Tensor dout = grad_out[0].contiguous();
     const int64_t n_out = geo->ranges.size(0), k = p.k();
     const bool want_feat = ctx->needs_input_grad(0), want_kernel = ctx->needs_input_grad(1) ||
@@ -786,14 +798,13 @@ struct McConv : torch::autograd::Function<McConv> {
     if (want_final) dfinal = at::empty_like(fw);
     hipStream_t s = current_stream();
     for (int64_t first = 0, i = 0; first < p.mlps; first += p.per, ++i) {
-      const auto w = c10::static_intrusive_pointer_cast<Packed>(
-          packs.get(i).toCapsule());
+      const Packed w = Packed::saved(saved, 5 + i * Packed::kTensors);
       const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g || p.per != p.mlps
                             ? gather_upstream(p, dout, geo->centre_rows, first) : dout;
       const bool direct = !p.padded() && p.mlps == 1;      // gradients land in the caller's shapes
       Tensor dkw_pad, dkb_pad, ddense;
       if (want_kernel) {
-        const Tensor dproj = layer_projection_grad(up, w->w);
+        const Tensor dproj = layer_projection_grad(up, w.w);
         Tensor ws = workspace(mccnn_mc_conv_project_grads_workspace_bytes((int)p.dims, (int)k,
                                                                           n_out), feats);
         dkw_pad = direct ? dkw : empty_f32({p.per, p.dims, p.h_pad}, feats);
@@ -802,18 +813,17 @@ struct McConv : torch::autograd::Function<McConv> {
         check(mccnn_mc_conv_project_grads(
             s, (int)p.dims, feats.size(0), f32(geo->points_in), (int)p.c_pad, f32(feats), n_out,
             f32(geo->points_out), geo->table.size(0), i32(geo->table), i32(geo->ranges),
-            f32(geo->inv_radii), (int)k, (int)p.per, (int)p.act, f32(w->kw), f32(w->kb),
+            f32(geo->inv_radii), (int)k, (int)p.per, (int)p.act, f32(w.kw), f32(w.kb),
             f32(geo->pdf), f32(dproj), ws.data_ptr(), ws.numel(), nullptr, nullptr, nullptr,
             nullptr, f32(dkw_pad), f32(dkb_pad)));
       }
       if (want_feat || want_final) {
         const bool in_place = features.defined();
-        const Tensor q = mc_project(p, *w, up, geo->points_out, geo->points_in, geo->table_t,
+        const Tensor q = mc_project(p, w, up, geo->points_out, geo->points_in, geo->table_t,
                                     geo->ranges_t, geo->neg_inv_radii, geo->pdf_t,
                                     in_place ? geo->point_rows : Tensor());
         if (want_feat) {
-          Tensor d = run_product(w->transposed, q, w->w2, w->w2t,
-                                 in_place ? Tensor() : geo->point_rows);
+          Tensor d = transposed_product(q, w, in_place ? Tensor() : geo->point_rows);
           if (dfeat.defined()) dfeat.add_(d);
           else dfeat = d;
         }
@@ -860,17 +870,18 @@ struct KpConv : torch::autograd::Function<KpConv> {
                         const Tensor &kernel_points, const c10::intrusive_ptr<Geometry> &geo,
                         const Plan &p, const KpShape &kp, bool grads) {
     const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
-    auto w = pack(p, 0, weights, Tensor(), Tensor(), geo->ranges.size(0), feats.size(0), false,
-                  grads);
+    const Packed w = pack(p, 0, weights, Tensor(), Tensor(), geo->ranges.size(0), feats.size(0),
+                          false, grads);
     const Tensor proj = kp_project(kp, kernel_points, p.k(), feats, geo->points_in,
                                    geo->points_out, geo->table, geo->ranges, geo->inv_radii,
                                    geo->centre_rows);
-    Tensor out = run_product(w->forward, proj, w->w, w->wt, Tensor(), p.cols());
+    Tensor out = run_product(w.forward, proj, w.w, w.wt, Tensor(), p.cols());
     if (grads) {
       // what the rows of Q are multiplied with: the features where they are, or padded ones
-      ctx->save_for_backward({p.c == p.c_pad ? features : feats, weights, kernel_points});
+      variable_list saved = {p.c == p.c_pad ? features : feats, weights, kernel_points};
+      w.save(saved);
+      ctx->save_for_backward(std::move(saved));
       ctx->saved_data["geo"] = c10::IValue::make_capsule(geo);
-      ctx->saved_data["pack"] = c10::IValue::make_capsule(w);
       ctx->saved_data["plan"] = std::vector<int64_t>{p.dims, p.c, p.h, p.g, p.mlps, p.c_pad,
                                                      p.h_pad, p.g_pad, p.per, p.act, kp.num_kp,
                                                      kp.kind};
@@ -887,7 +898,7 @@ struct KpConv : torch::autograd::Function<KpConv> {
     const KpShape kp{v[10], v[11], ctx->saved_data["sigma"].toDouble()};
     const auto geo = c10::static_intrusive_pointer_cast<Geometry>(
         ctx->saved_data["geo"].toCapsule());
-    const auto w = c10::static_intrusive_pointer_cast<Packed>(ctx->saved_data["pack"].toCapsule());
+    const Packed w = Packed::saved(saved, 3);
     const Tensor dout = grad_out[0].contiguous();
     const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g
                           ? gather_upstream(p, dout, geo->centre_rows, 0) : dout;
@@ -898,8 +909,7 @@ struct KpConv : torch::autograd::Function<KpConv> {
                                   geo->table_t, geo->ranges_t, geo->neg_inv_radii,
                                   in_place ? geo->point_rows : Tensor());
       if (ctx->needs_input_grad(0))
-        dfeat = cut_columns(run_product(w->transposed, q, w->w2, w->w2t,
-                                        in_place ? Tensor() : geo->point_rows), p.c);
+        dfeat = cut_columns(transposed_product(q, w, in_place ? Tensor() : geo->point_rows), p.c);
       if (ctx->needs_input_grad(1)) {
         const Tensor ddense = weight_grad_product(x, q);
         dweights = at::empty_like(weights);

@@ -88,3 +88,33 @@ def test_feature_columns_that_a_layer_does_not_have_are_refused(layer):
     assert out.shape == (50, 64)
     out.sum().backward()
     assert wide.grad.shape == wide.shape
+
+
+@pytest.mark.parametrize("layer", ["mc", "kp"])
+def test_a_kept_output_keeps_no_packed_weights(layer):
+    """After the backward pass an output holds its own memory and the neighbourhood's, whatever
+    forms of the weights the pass made; a second backward pass over the same graph is told so."""
+    from tensorflow_graphics_point_clouds_amd import layers, pc
+    cloud = pc.PointCloud(torch.rand(600, 3, device="cuda"),
+                          torch.zeros(600, dtype=torch.int32, device="cuda"), 1)
+    nbh = pc.Neighborhood(pc.Grid(cloud, 0.2), 0.2, cloud)
+    conv = layers.MCConv(100, 512, 3, num_mlps=1, mlp_size=[16]) if layer == "mc" else \
+        layers.KPConv(100, 512)
+    feats = torch.randn(600, 100, device="cuda", requires_grad=True)
+    held = []
+    for retain in (False, True, False):
+        for p in [feats] + list(conv.parameters()):
+            p.grad = None
+        out = conv(feats, cloud, cloud, 0.2, neighborhood=nbh)
+        out.sum().backward(retain_graph=retain)
+        if retain:
+            once = feats.grad.clone()
+            out.sum().backward()
+            assert torch.allclose(feats.grad, 2 * once)
+        with pytest.raises(RuntimeError, match="second time"):
+            out.sum().backward()
+        with_out = torch.cuda.memory_allocated()
+        shape = out.shape
+        del out
+        held.append(with_out - torch.cuda.memory_allocated())
+    assert max(held) <= 4 * shape[0] * shape[1] + 4096, held
