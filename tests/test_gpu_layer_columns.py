@@ -1,6 +1,8 @@
 """Output columns that are no multiple of 64, on both sides of the sizes from which 64 or 128
 columns take the tiled product: the layer's product and the gradient of its projection against
 float64 on the same operands."""
+import gc
+
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -101,6 +103,10 @@ def test_a_kept_output_keeps_no_packed_weights(layer):
     conv = layers.MCConv(100, 512, 3, num_mlps=1, mlp_size=[16]) if layer == "mc" else \
         layers.KPConv(100, 512)
     feats = torch.randn(600, 100, device="cuda", requires_grad=True)
+
+    def requested():
+        gc.collect()                     # (what other tests left in cycles)
+        return torch.cuda.memory_stats()["requested_bytes.all.current"]
     held = []
     for retain in (False, True, False):
         for p in [feats] + list(conv.parameters()):
@@ -113,8 +119,8 @@ def test_a_kept_output_keeps_no_packed_weights(layer):
             assert torch.allclose(feats.grad, 2 * once)
         with pytest.raises(RuntimeError, match="second time"):
             out.sum().backward()
-        with_out = torch.cuda.memory_allocated()
+        with_out = requested()
         shape = out.shape
         del out
-        held.append(with_out - torch.cuda.memory_allocated())
-    assert max(held) <= 4 * shape[0] * shape[1] + 4096, held
+        held.append(with_out - requested())
+    assert max(held) <= 4 * shape[0] * shape[1] + 4096, held      # (the output itself)
