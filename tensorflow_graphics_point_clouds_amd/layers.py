@@ -414,20 +414,44 @@ class MCConv(torch.nn.Module):
         return _layer_plan(self._num_dims, self._num_features_in, g * self._num_mlps,
                            self._num_mlps, self._hidden, self._act)
 
+    def _convolve_fused(self, g, features, neighborhood, inv_radii):
+        """The single-kernel layer with operands padded as the others' are, or None where it does
+        not cover the sizes: both directions have to be covered (the backward runs it transposed,
+        output channels as its input channels), and several kernel MLPs are better off as
+        sub-layers where they divide into them."""
+        d, c, l, h = self._num_dims, self._num_features_in, self._num_mlps, self._hidden
+        h_pad = next((v // l for v in (16, 32, 64) if v % l == 0 and v // l >= h), None)
+        pad = _layer_padding(c, g * l, l)
+        if h_pad is None or pad is None:
+            return None
+        (c_pad, g_pad), k = pad, l * h_pad
+        per = 16 // h_pad if h_pad <= 16 and 16 % h_pad == 0 else 0
+        if k > 16 and per > 0 and l % per == 0 and per * g_pad % 16 == 0:
+            return None
+        ok = _lib.lib().mccnn_mc_conv_layer_supported
+        if not (ok(cint(d), cint(c_pad), cint(k), cint(g_pad * l)) and
+                ok(cint(d), cint(g_pad * l), cint(k), cint(c_pad))):
+            return None
+        weights, biases, final = self.weights, self.biases.reshape(l, h), self.final_weights
+        pad = torch.nn.functional.pad
+        if h_pad != h:
+            weights, biases = pad(weights, (0, h_pad - h)), pad(biases, (0, h_pad - h))
+        if c_pad != c or g_pad != g or h_pad != h:
+            final = pad(final.reshape(l, c, h, g), (0, g_pad - g, 0, h_pad - h, 0, c_pad - c))
+            final = final.reshape(l, c_pad * h_pad, g_pad)
+            features = pad(features, (0, c_pad - c))
+        out = _MCConvFusedLayer.apply(weights.contiguous(), biases.contiguous(), final, features,
+                                      neighborhood, inv_radii, self._act)
+        return out if g_pad == g else out.reshape(-1, l, g_pad)[:, :, :g].reshape(-1, l * g)
+
     def _convolve_on_view(self, plan, features, neighborhood, radii):
         """The layer on the grid-ordered view (csrc/host.cpp); channel counts its kernels do
         not cover are zero-padded on the way in and the result is cut back."""
         inv_radii = pc._reciprocal(radii)
         if self.fuse_final:
-            c, f, l, h = (self._num_features_in, self._num_features_out, self._num_mlps,
-                          self._hidden)
-            # the backward runs the same single-kernel layer transposed (output channels as its
-            # input channels), so both directions have to be covered
-            d, k, ok = self._num_dims, l * h, _lib.lib().mccnn_mc_conv_layer_supported
-            if ok(cint(d), cint(c), cint(k), cint(f)) and ok(cint(d), cint(f), cint(k), cint(c)):
-                return _MCConvFusedLayer.apply(self.weights, self.biases.reshape(l, h),
-                                               self.final_weights, features, neighborhood,
-                                               inv_radii, self._act)
+            out = self._convolve_fused(plan[3], features, neighborhood, inv_radii)
+            if out is not None:
+                return out
         grads = torch.is_grad_enabled() and (features.requires_grad or
                                              self.weights.requires_grad or
                                              self.final_weights.requires_grad or
