@@ -32,6 +32,11 @@
 
 namespace mccnn {
 
+// Pairs of a table, at most: the kernels step through a centre's pairs in 32 bits and look up to two
+// chunks (128 pairs) past the last of them.
+constexpr int64_t kMostPairs = ((int64_t)1 << 31) - 1024;
+
+// The finalizer "lowbias32" of C. Wellons' hash prospector (public domain).
 __device__ __forceinline__ unsigned hash_id(unsigned x) {
   x ^= x >> 16; x *= 0x7feb352du;
   x ^= x >> 15; x *= 0x846ca68bu;
@@ -502,8 +507,8 @@ extern "C" int mccnn_neighbourhood_order(mccnn_stream_t stream, int64_t num_samp
                                          const int32_t *ranges, void *workspace,
                                          size_t workspace_bytes, int32_t *order_out) {
   MCCNN_REQUIRE(num_samples >= 0 && num_samples < ((int64_t)1 << 31) && num_neighbors >= 0 &&
-                    num_neighbors < ((int64_t)1 << 31),
-                "neighbourhood_order expects sizes in [0, 2^31)");
+                    num_neighbors <= kMostPairs,
+                "neighbourhood_order expects fewer than 2^31 centres and at most 2^31 - 1024 pairs");
   if (num_samples == 0) return MCCNN_OK;
   MCCNN_REQUIRE(ranges && workspace && order_out && (neighbors || num_neighbors == 0),
                 "neighbourhood_order received a null tensor");
@@ -529,7 +534,8 @@ extern "C" int mccnn_neighbourhood_order(mccnn_stream_t stream, int64_t num_samp
 //   22.8 / 16.4, 120 pairs 21.3 / 29.6 ms; 64 x 16 at 30 pairs 2.6 / 2.7 ms).
 extern "C" int mccnn_basis_proj_grads_grouped_pays(int num_features, int num_basis,
                                                    int64_t num_samples, int64_t num_neighbors) {
-  if (group_slices(num_features, num_basis) == 0 || num_samples <= 0) return 0;
+  if (group_slices(num_features, num_basis) == 0 || num_samples <= 0 || num_neighbors > kMostPairs)
+    return 0;
   const int64_t work = num_neighbors * num_features;
   if (!mfma_grads_supported(num_features, num_basis)) return work >= ((int64_t)1 << 20) ? 1 : 0;
   return work >= ((int64_t)1 << 27) && num_features * num_basis >= 2048 &&
@@ -565,8 +571,9 @@ extern "C" int mccnn_basis_proj_grads_grouped(
                 "BasisProjGrads (grouped) supports 8/16/32/64 basis functions and at most 128 "
                 "features (got %d and %d)", num_basis, num_features);
   MCCNN_REQUIRE(num_pts >= 0 && num_samples >= 0 && num_neighbors >= 0 &&
-                    num_neighbors < ((int64_t)1 << 31) && num_samples < ((int64_t)1 << 31),
-                "BasisProjGrads (grouped) expects sizes in [0, 2^31)");
+                    num_neighbors <= kMostPairs && num_samples < ((int64_t)1 << 31),
+                "BasisProjGrads (grouped) expects fewer than 2^31 centres and at most 2^31 - 1024 "
+                "pairs");
   hipStream_t s = as_stream(stream);
   if (num_pts > 0) {
     MCCNN_REQUIRE(feature_grads_out, "BasisProjGrads (grouped) received a null tensor");

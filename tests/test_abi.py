@@ -131,3 +131,18 @@ def test_product_does_not_import_the_oracle():
             if f.endswith((".py", ".hip", ".h", ".cpp")):
                 text = open(os.path.join(base, f)).read()
                 assert "mccnn_oracle" not in text and "from oracle" not in text, f
+
+
+def test_grouped_basis_gradients_stop_short_of_the_last_pair_indices(lib):
+    """The grouped kernels look up to 128 pairs past a centre's last one in 32 bits: tables within
+    that of 2^31 pairs are left to the other kernels and refused."""
+    i64, sz = ctypes.c_int64, ctypes.c_size_t
+    most = 2 ** 31 - 1024
+    pays = lambda m: lib.mccnn_basis_proj_grads_grouped_pays(24, 8, i64(10 ** 7), i64(m))
+    assert pays(most) == 1 and pays(most + 1) == 0 and pays(2 ** 31 - 1) == 0
+    for pairs in (most + 1, 2 ** 31 - 1):
+        rc = lib.mccnn_neighbourhood_order(None, i64(5), i64(pairs), None, None, None, sz(0), None)
+        assert rc == 1 and b"2^31 - 1024" in lib.mccnn_last_error()
+        rc = lib.mccnn_basis_proj_grads_grouped(None, i64(0), 8, None, 24, None, i64(pairs), None,
+                                                i64(5), None, None, None, None, sz(0), None, None)
+        assert rc == 1 and b"2^31 - 1024" in lib.mccnn_last_error()
