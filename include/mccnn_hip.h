@@ -407,7 +407,8 @@ int mccnn_basis_proj_grads_ordered(
  * group instead of once per pair.  For any table and any order; pays where consecutive centres
  * share their points, as in the order mccnn_neighbourhood_order finds from the table itself
  * (centres by the smallest hashes of their points).  Float atomics: the order of the sums is not
- * fixed, as for mccnn_basis_proj_grads.  Supported: up to 128 features and 2^31 - 1024 pairs; basis, in_grads and
+ * fixed, as for mccnn_basis_proj_grads.  Rows of the table behind the last centre's pairs have
+ * zero basis gradients.  Supported: up to 128 features and 2^31 - 1024 pairs; basis, in_grads and
  * basis_grads_out aligned to 16 bytes, features too if their number is a multiple of 16.
  * ..._pays: whether it is the faster one for a table of these sizes. */
 size_t mccnn_neighbourhood_order_workspace_bytes(int64_t num_samples);

@@ -186,7 +186,7 @@ struct GroupInfo {
 __global__ void __launch_bounds__(256) group_rows_kernel(
     int64_t n_out, int group, int max_rows, const int2 *__restrict__ nbrs,
     const int *__restrict__ ranges, const int *__restrict__ order, unsigned short *__restrict__ row_of, int *__restrict__ keys,
-    GroupInfo *__restrict__ info) {
+    GroupInfo *__restrict__ info, int64_t pairs, int num_basis, float *__restrict__ dbasis) {
   __shared__ int key[kHash];
   __shared__ int number[kHash];
   __shared__ unsigned seen[2][kMaxRows];          // centres of the group that list the row's point
@@ -243,6 +243,10 @@ __global__ void __launch_bounds__(256) group_rows_kernel(
   }
   __syncthreads();
   if (t == 0) info[blockIdx.x] = GroupInfo{rows < max_rows ? rows : max_rows, direct};
+  // rows of the table behind the last centre's pairs (a table of more capacity than pairs)
+  for (int64_t i = (int64_t)ranges[n_out - 1] * num_basis + blockIdx.x * 256 + t;
+       i < pairs * num_basis; i += (int64_t)gridDim.x * 256)
+    dbasis[i] = 0.0f;
 }
 
 // W wavefronts of 16 channels each, K basis columns.
@@ -594,7 +598,7 @@ extern "C" int mccnn_basis_proj_grads_grouped(
   GroupInfo *infos = (GroupInfo *)((char *)keys + align256(sizeof(int) * kMaxRows * (size_t)groups));
   hipLaunchKernelGGL(group_rows_kernel, dim3((unsigned)groups), dim3(256), 0, s, num_samples, group,
                      num_basis == 64 ? kRows<64> : kMaxRows, (const int2 *)neighbors, ranges,
-                     centre_order, row_of, keys, infos);
+                     centre_order, row_of, keys, infos, num_neighbors, num_basis, basis_grads_out);
   MCCNN_LAUNCH_CHECK();
   int rc = MCCNN_OK;
 #define MCCNN_GROUP_K(CT_, K_)                                                                   \

@@ -48,3 +48,32 @@ def test_grouped_gradients(c, k, points, centres):
     terms = k * np.bincount(ids, minlength=points)[:, None]
     assert np.all(np.abs(dbasis - db) <= (c + 1) * 2.0 ** -24 * db_mag)
     assert np.all(np.abs(dfeat - df) <= (terms + 1) * 2.0 ** -24 * df_mag)
+
+
+@pytest.mark.parametrize("c,k,spare", [(24, 8, 1), (96, 16, 700), (64, 64, 65)])
+def test_rows_behind_the_last_list_have_zero_gradients(c, k, spare):
+    """A table of more rows than its lists hold (a search into a given capacity): the kernels per
+    pair and channel leave zeros there, the grouped ones write them."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    host, stream, ptr, i64, cint = _lib.host(), _lib.stream, _lib.ptr, _lib.i64, _lib.cint
+    gen = torch.Generator(device="cuda").manual_seed(c)
+    centres, points, per = 300, 200, 20
+    used, rows = centres * per, centres * per + spare
+    pairs = torch.zeros(rows, 2, dtype=torch.int32, device="cuda")
+    pairs[:used, 0] = torch.randint(points, (used,), device="cuda", generator=gen)
+    pairs[:used, 1] = torch.arange(centres, device="cuda").repeat_interleave(per)
+    ranges = torch.arange(per, used + 1, per, device="cuda", dtype=torch.int32)
+    basis, feat, up = (torch.randn(*s, device="cuda", generator=gen)
+                       for s in ((rows, k), (points, c), (centres, c, k)))
+    order = host.neighbourhood_order(pairs, ranges)
+    size = _lib.lib().mccnn_basis_proj_grads_grouped_workspace_bytes
+    size.restype = _lib.csize
+    ws = _lib.workspace(size(i64(centres), i64(rows)), "cuda")
+    dbasis, dfeat = torch.full_like(basis, float("nan")), torch.empty_like(feat)
+    _lib.call("basis_proj_grads_grouped", stream(), i64(points), cint(k), ptr(basis), cint(c),
+              ptr(feat), i64(rows), ptr(pairs), i64(centres), ptr(ranges), ptr(order), ptr(up),
+              ptr(ws), _lib.csize(ws.numel()), ptr(dbasis), ptr(dfeat))
+    assert torch.equal(dbasis[used:], torch.zeros_like(dbasis[used:]))
+    terms = up[pairs[:used, 1].long()].double() * feat[pairs[:used, 0].long()].double()[:, :, None]
+    expect, size = terms.sum(1), terms.abs().sum(1)
+    assert torch.all((dbasis[:used] - expect).abs() <= (c + 1) * 2.0 ** -24 * size)
