@@ -42,13 +42,14 @@ def _bare(module, kind):
 
 def _leaky_slope(activation):
     """The slope for negative inputs of a leaky activation (0: ReLU) that keeps signs, as the
-    gradients of the kernels need it, else None."""
+    gradients of the kernels need it, else None (a LeakyReLU of slope 0 is not a ReLU: infinities
+    and NaN differ)."""
     if activation is torch.relu:
         return 0.0
     if isinstance(activation, torch.nn.ReLU) and _bare(activation, torch.nn.ReLU):
         return 0.0
     if (isinstance(activation, torch.nn.LeakyReLU) and _bare(activation, torch.nn.LeakyReLU) and
-            activation.negative_slope >= 0):
+            activation.negative_slope > 0):
         return activation.negative_slope
     return None
 

@@ -1224,7 +1224,10 @@ struct NormAct : torch::autograd::Function<NormAct> {
         mean = x.mean(0);
         inv = (x.var(0, false) + ctx->saved_data["eps"].toDouble()).rsqrt();
       }
-      const Tensor z = (x - mean) * inv * weight + bias, y = slope == 1.0 ? z : at::where(out > 0, z, z * slope);
+      const Tensor z = (x - mean) * inv * weight + bias;
+      const Tensor y = slope == 1.0   ? z
+                       : slope == 0.0 ? at::where(out <= 0, at::zeros_like(z), z)
+                                      : at::where(out > 0, z, z * slope);
       variable_list wanted;
       std::vector<size_t> slots;
       for (size_t i = 0; i < 3; ++i)

@@ -121,7 +121,8 @@ __device__ __forceinline__ NormCols norm_cols(const NormArgs &a, int c, int C) {
 }
 
 // dz = g act'(z) of a point's four columns, xhat = (x - mean) inv beside it.  The activation
-// keeps signs, so that its result tells on which side of 0 the forward pass saw z.
+// keeps signs, so that its result tells on which side of 0 the forward pass saw z.  NaN takes the
+// side that torch's activations give it: ReLU passes its gradient, a slope applies.
 template <bool kVec>
 __device__ __forceinline__ v4f norm_dz(const NormArgs &a, int64_t i, int c, int C,
                                        const NormCols &p, v4f *xhat) {
@@ -131,7 +132,8 @@ __device__ __forceinline__ v4f norm_dz(const NormArgs &a, int64_t i, int c, int 
     const v4f y = load_cols<kVec>(a.y + i * C, c, C);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (!(y[e] > 0.0f)) dz[e] = a.slope == 0.0f ? 0.0f : a.slope * dz[e];
+      if (a.slope == 0.0f) dz[e] = y[e] <= 0.0f ? 0.0f : dz[e];
+      else if (!(y[e] > 0.0f)) dz[e] = a.slope * dz[e];
   }
   return dz;
 }
@@ -187,7 +189,8 @@ __global__ void __launch_bounds__(256) norm_grads_kernel(
   for (int64_t i = first + threadIdx.x / kLanes; i < last; i += 256 / kLanes) {
     v4f xhat;
     const v4f dz = norm_dz<kVec>(a, i, c, C, p, &xhat);
-    store_cols<kVec>(dx + i * C, c, C, (dz - m1 - xhat * m2) * (p.inv * p.weight));
+    // (with given statistics an infinite point has a finite gradient)
+    store_cols<kVec>(dx + i * C, c, C, (fixed ? dz : dz - m1 - xhat * m2) * (p.inv * p.weight));
   }
 }
 

@@ -139,3 +139,30 @@ def test_transforms_see_torch_operations():
         return [v.detach().cpu() for v in (tangent, gradient, again, many)]
     for got, expect in zip(derivatives("cuda"), derivatives("cpu")):
         assert torch.allclose(got, expect, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("act", [torch.relu, torch.nn.ReLU(), torch.nn.LeakyReLU(0.3),
+                                 torch.nn.LeakyReLU(0.0)])
+@pytest.mark.parametrize("training", [False, True])
+def test_infinities_and_nan_take_the_gradient_of_torch(act, training):
+    """Against torch's own operations on the same float32 values; with given statistics a point
+    that is not finite leaves the gradients of the others alone."""
+    from tensorflow_graphics_point_clouds_amd import blocks
+    x, g = _rand(70, 8, seed=1), _rand(70, 8, seed=2)
+    x[3, 0], x[4, 1], x[5, 2] = float("nan"), float("inf"), -float("inf")
+    norm = blocks.BatchNorm(8)
+    with torch.no_grad():
+        norm.weight.uniform_(0.5, 1.5)
+        norm.running_mean.normal_()
+        norm.running_var.uniform_(0.5, 2.0)
+    plain = torch.nn.BatchNorm1d(8, eps=norm.eps, device="cuda")
+    plain.load_state_dict(norm.state_dict())
+    results = []
+    for module, call in ((norm, lambda v: blocks._norm_act(norm, act, v, training)),
+                         (plain, lambda v: act(plain.train(training)(v)))):
+        a = x.clone().requires_grad_()
+        out = call(a)
+        out.backward(g)
+        results.append((out.detach(), a.grad, module.weight.grad, module.bias.grad))
+    for got, expect in zip(*results):       # sums of 70 terms in float32, elsewhere a few roundings
+        assert torch.allclose(got, expect, rtol=1e-5, atol=1e-4, equal_nan=True)
