@@ -1169,9 +1169,7 @@ class KPConv(torch.nn.Module):
         offsets = None
         if self.deformable:       # KPConv.py:317-392: offsets from a rigid convolution
             if self.transposed_grads and k in (16, 32):
-                offsets = _kp_rigid(self.offset_weights, self._offset_plan, c, features, neighborhood,
-                                    pc._reciprocal(radii), self._kernel_points, k, self._kind,
-                                    sigma)
+                offsets = self._rigid_offsets(features, neighborhood, pc._reciprocal(radii), sigma)
             else:
                 rigid = _KPBasis.apply(None, *geometry, k, self._kind, sigma)
                 offsets = _dense_product(project(rigid).reshape(-1, c * k),
@@ -1182,6 +1180,18 @@ class KPConv(torch.nn.Module):
         basis = _KPBasis.apply(offsets, *geometry, k, self._kind, sigma)
         return _dense_product(project(basis).reshape(-1, c * k), self._padded(self.weights))
 
+    def _rigid_offsets(self, features, neighborhood, inv_radii, sigma):
+        """The rigid convolution that predicts the offsets -> [N_out, KP * D].  Without a plan
+        (more than 128 channels) its columns are padded here: 45 columns have neither a transposed
+        projection nor a product with the weights of their own."""
+        weights, cols = self.offset_weights, self._num_kernel_points * self._num_dims
+        padded = self._offset_plan is None and _offset_columns(cols) != cols
+        if padded:
+            weights = torch.nn.functional.pad(weights, (0, _offset_columns(cols) - cols))
+        out = _kp_rigid(weights, self._offset_plan, self._num_features_in, features, neighborhood,
+                        inv_radii, self._kernel_points, self._num_basis, self._kind, sigma)
+        return out[:, :cols] if padded else out
+
     def _convolve_deformed_on_view(self, features, neighborhood, radii, sigma):
         """KPConv.py:317-392 on the grid-ordered view: a rigid convolution predicts the
         offsets (rows in the caller's centre order, `last_offsets`), which are brought
@@ -1190,9 +1200,7 @@ class KPConv(torch.nn.Module):
         kp, k, d = self._num_kernel_points, self._num_basis, self._num_dims
         view = neighborhood.sorted_view()
         inv_radii = pc._reciprocal(radii)
-        offsets = _kp_rigid(self.offset_weights, self._offset_plan, self._num_features_in, features,
-                            neighborhood, inv_radii, self._kernel_points, k, self._kind, sigma)
-        offsets = offsets.reshape(-1, kp, d)
+        offsets = self._rigid_offsets(features, neighborhood, inv_radii, sigma).reshape(-1, kp, d)
         self.last_offsets = offsets
         on_view = offsets if view.centre_order is None else \
             offsets.index_select(0, view.centre_order)
