@@ -114,9 +114,12 @@ int mccnn_build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims,
 
 /* The same with the host copy of the shape written by the kernel itself into pinned host memory
  * (hipHostMalloc) that stays valid until the call returns.  num_cells_out_pinned and
- * key_bits_out_host may be NULL for up to mccnn_build_grid_single_launch_max() points: the
- * whole grid is then one launch and the call does not wait for the device. */
+ * key_bits_out_host may both be NULL, never one of them, where
+ * mccnn_build_grid_is_single_launch (up to mccnn_build_grid_single_launch_max() points, at least
+ * one, and at most 512 extents batch_size * num_dims): the whole grid is then one launch and the
+ * call does not wait for the device. */
 int64_t mccnn_build_grid_single_launch_max(void);
+int mccnn_build_grid_is_single_launch(int64_t num_pts, int num_dims, int batch_size);
 int mccnn_build_grid_pinned(mccnn_stream_t stream, int64_t num_pts, int num_dims,
                             const float *points, const int32_t *batch_ids, int batch_size,
                             const float *cell_sizes, float *aabb_min_out, float *aabb_max_out,

@@ -56,6 +56,7 @@ def lib():
                      "mccnn_transpose_neighbors_workspace_bytes",
                      "mccnn_weight_grad_product_workspace_bytes"):
             getattr(handle, name).restype = csize
+        handle.mccnn_build_grid_single_launch_max.restype = i64
         _lib = handle
     return _lib
 

@@ -758,7 +758,8 @@ extern "C" int mccnn_invert_order(mccnn_stream_t stream, int64_t count, const in
   return MCCNN_OK;
 }
 
-// The grid of pylib/pc/Grid.py:32-64 in one call.  Up to 16 384 points: one launch, no host
+// The grid of pylib/pc/Grid.py:32-64 in one call.  Up to 16 384 points in clouds whose extents
+// (batch * dims) fit a block's 512: one launch, no host
 // round trip unless the caller asks for the shape.  Beyond that: boxes, shape and keys (three
 // launches), the host copy of the shape -- it sizes the key width of the sort and, for the
 // caller, the grid table --, three launches per digit of the sort, the last of which gathers
@@ -770,6 +771,14 @@ extern "C" size_t mccnn_build_grid_workspace_bytes(int64_t num_pts) {
 }
 
 extern "C" int64_t mccnn_build_grid_single_launch_max(void) { return kSmallMax; }
+
+static bool extents_fit(int num_dims, int batch_size) {
+  return batch_size > 0 && (int64_t)batch_size * num_dims <= kGridLdsExtents;
+}
+
+extern "C" int mccnn_build_grid_is_single_launch(int64_t num_pts, int num_dims, int batch_size) {
+  return num_pts > 0 && num_pts <= kSmallMax && extents_fit(num_dims, batch_size);
+}
 
 static int key_bits_for(int batch, int num_dims, const int32_t *cells) {
   unsigned long long total = (unsigned long long)(batch > 0 ? batch : 1);
@@ -787,15 +796,19 @@ static int build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims, cons
   MCCNN_REQUIRE(num_pts >= 0 && num_pts < ((int64_t)1 << 31), "build_grid expects 0 <= num_pts < 2^31");
   MCCNN_REQUIRE(workspace_bytes >= mccnn_build_grid_workspace_bytes(num_pts),
                 "build_grid workspace too small");
-  hipStream_t s = as_stream(stream);
-  const bool extents_fit = batch_size > 0 && batch_size * num_dims <= kGridLdsExtents;
   const bool want_shape = num_cells_out_host != nullptr;
-  if (num_pts > 0 && extents_fit) {
+  MCCNN_REQUIRE(want_shape == (key_bits_out_host != nullptr),
+                "build_grid expects both host outputs, the grid shape and the key width, or neither");
+  const bool single_launch = mccnn_build_grid_is_single_launch(num_pts, num_dims, batch_size);
+  MCCNN_REQUIRE(want_shape || single_launch,
+                "build_grid needs host outputs for the grid shape and the key width");
+  hipStream_t s = as_stream(stream);
+  if (num_pts > 0 && extents_fit(num_dims, batch_size)) {
     MCCNN_REQUIRE(points && batch_ids && cell_sizes && g.aabb_min && g.aabb_max && g.num_cells &&
                       g.smin && g.inv_cell && g.keys && g.sorted_keys && g.sorted_idx &&
                       g.sorted_pts && g.sorted_bids && workspace,
                   "build_grid received a null tensor");
-    if (num_pts <= kSmallMax) {
+    if (single_launch) {
       int rc = MCCNN_OK;
       MCCNN_DIM_SWITCH(num_dims, rc = (launch_small<D, false>(s, num_pts, batch_size, points, batch_ids,
                                                               cell_sizes, g)));
@@ -806,7 +819,6 @@ static int build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims, cons
       *key_bits_out_host = key_bits_for(batch_size, num_dims, num_cells_out_host);
       return MCCNN_OK;
     }
-    MCCNN_REQUIRE(want_shape, "build_grid needs host outputs for the grid shape and the key width");
     const SortWorkspace w = carve_sort_workspace(workspace, num_pts);
     char *p = (char *)workspace + w.bytes;
     unsigned *keys32 = (unsigned *)p;
@@ -833,8 +845,6 @@ static int build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims, cons
                             out);
     }
   } else {
-    MCCNN_REQUIRE(num_cells_out_host && key_bits_out_host,
-                  "build_grid needs host outputs for the grid shape and the key width");
     int rc = mccnn_grid_setup(stream, num_pts, num_dims, points, batch_ids, batch_size, cell_sizes,
                               g.aabb_min, g.aabb_max, g.num_cells, g.smin, g.inv_cell);
     if (rc != MCCNN_OK) return rc;

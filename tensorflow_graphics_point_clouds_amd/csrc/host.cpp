@@ -217,7 +217,7 @@ GridTensors build_grid(const Tensor &points, const Tensor &bids, int64_t batch,
                                   i64(g.sorted_keys), i32(g.sorted_indices), f32(g.sorted_points),
                                   i32(g.sorted_bids), ws.data_ptr(), ws.numel(), cells, bits));
   };
-  if (n > 0 && n <= mccnn_build_grid_single_launch_max() && batch > 0 && batch * d <= 512) {
+  if (mccnn_build_grid_is_single_launch(n, (int)d, (int)batch)) {
     call(nullptr, nullptr);
     return g;
   }

@@ -13,7 +13,6 @@ import torch
 
 from . import _lib, tfg_custom_ops
 _F32, _I32 = torch.float32, torch.int32
-_SINGLE_LAUNCH = 16384     # points up to which a grid or an order of centres is one launch
 
 
 class KDEMode(enum.Enum):
@@ -508,9 +507,11 @@ class Neighborhood:
             if not cut:
                 tfg_custom_ops._remember_symmetric(self._table)
             return
+        # (an order of few centres is one launch, which does not need the width of the keys)
+        one_launch = s._points.shape[0] <= _lib.lib().mccnn_build_grid_single_launch_max()
         order, pts, bids = _lib.host().order_centres(
             s._points.detach(), s._batch_ids, grid._batch_size, num_cells, smin, inv_cell,
-            0 if s._points.shape[0] <= _SINGLE_LAUNCH else grid._key_bits)
+            0 if one_launch else grid._key_bits)
         ranges, table, _ = _lib.host().search(pts, bids, points, keys, ds, num_cells, smin,
                                               inv_cell, self._inv_radii, self.max_neighbors)
         self._sorted = (order, pts, ranges, table)

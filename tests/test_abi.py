@@ -65,6 +65,30 @@ def test_invalid_arguments_return_status_not_abort(lib):
     assert rc == 1 and b"batch size" in lib.mccnn_last_error()
 
 
+def test_grid_in_one_call_wants_both_host_outputs_or_neither(lib):
+    """The shape without the key width was written through a null pointer; neither is enough only
+    where the grid is one launch (more clouds than a block keeps the extents of are not)."""
+    i64, sz, vp = ctypes.c_int64, ctypes.c_size_t, ctypes.c_void_p
+    cells, bits = (ctypes.c_int32 * 3)(), ctypes.c_int(0)
+    lib.mccnn_build_grid_single_launch_max.restype = i64
+    most = lib.mccnn_build_grid_single_launch_max()
+
+    def status(points, batch, shape, width):
+        rc = lib.mccnn_build_grid_pinned(None, i64(points), 3, None, None, batch, *[None] * 12,
+                                         sz(1 << 40), shape, width)
+        assert rc == 1
+        return lib.mccnn_last_error()
+    for points in (4, most, most + 1):
+        assert b"or neither" in status(points, 2, cells, None)
+        assert b"or neither" in status(points, 2, None, ctypes.byref(bits))
+    single = lib.mccnn_build_grid_is_single_launch
+    for points, batch, expect in ((1, 1, 1), (most, 170, 1), (most, 171, 0), (most + 1, 1, 0),
+                                  (0, 1, 0), (5, 0, 0), (5, 1 << 30, 0)):
+        assert single(i64(points), 3, batch) == expect, (points, batch)
+        message = status(points, batch, None, None)
+        assert (b"null tensor" if expect else b"needs host outputs") in message
+
+
 def test_pointconv_density_entry_points_validate_before_the_device(lib):
     i64, sz = ctypes.c_int64, ctypes.c_size_t
     rc = lib.mccnn_pointconv_density(None, i64(5), None, 2, None, None, None, None, None, None, None)

@@ -165,3 +165,51 @@ def test_clouds_of_other_dimensions_are_refused(points, layer):
     nbh = pc.Neighborhood(pc.Grid(cloud, 0.3), 0.3, cloud)
     with pytest.raises(_lib.InvalidArgumentError):
         conv(torch.ones(100, 4, device="cuda"), cloud, cloud, 0.3, neighborhood=nbh)
+
+
+@pytest.mark.parametrize("n,batch", [(1, 1), (700, 3), (700, 300), (20000, 3)])
+def test_steps_of_the_c_abi_that_the_package_calls_in_one(n, batch):
+    """mccnn_build_grid, mccnn_reorder_neighbors and mccnn_gather_pdf, for callers of the library
+    itself: the same bits as the forms behind the classes."""
+    from ctypes import byref, c_int, c_int32
+    from tensorflow_graphics_point_clouds_amd import _lib, pc
+    from tensorflow_graphics_point_clouds_amd._lib import cint, csize, i64, ptr, stream
+    gen = torch.Generator(device="cuda").manual_seed(n + batch)
+    pts = torch.rand((n, 3), device="cuda", generator=gen)
+    bids = torch.randint(batch, (n,), device="cuda", generator=gen).int()
+    grid = pc.Grid(pc.PointCloud(pts, bids, batch), 0.1)
+    f32 = lambda *s: torch.empty(s, device="cuda")
+    i32 = lambda *s: torch.empty(s, device="cuda", dtype=torch.int32)
+    keys = [torch.empty(n, device="cuda", dtype=torch.int64) for _ in range(2)]
+    got = [f32(batch, 3), f32(batch, 3), i32(3), f32(batch, 3), f32(3), *keys, i32(n), f32(n, 3),
+           i32(n)]
+    cells, bits = (c_int32 * 3)(), c_int(0)
+    ws = _lib.workspace(_lib.lib().mccnn_build_grid_workspace_bytes(i64(n)), "cuda")
+    _lib.call("build_grid", stream(), i64(n), cint(3), ptr(pts), ptr(bids), cint(batch),
+              ptr(grid._cell_sizes), *[ptr(t) for t in got], ptr(ws), csize(ws.numel()), cells,
+              byref(bits))
+    names = ("aabb_min", "aabb_max", "num_cells", "scaled_aabb_min", "inv_cell_sizes", "cur_keys",
+             "sorted_keys", "sorted_indices", "sorted_points", "sorted_batch_ids")
+    for name, t in zip(names, got):
+        assert torch.equal(t, getattr(grid, "_" + name)), name
+    assert (list(cells), bits.value) == (grid._num_cells_host, grid._key_bits)
+
+    nbh = pc.Neighborhood(grid, 0.1)
+    table, ranges = nbh._neighbors, nbh._samples_neigh_ranges
+    m = table.shape[0]
+    order = torch.randperm(n, device="cuda", generator=gen).int()
+    new_ranges, new_table, pdf = i32(n), i32(m, 2), f32(m)
+    ws = _lib.workspace(_lib.lib().mccnn_reorder_neighbors_workspace_bytes(i64(n)), "cuda")
+    _lib.call("reorder_neighbors", stream(), i64(n), ptr(ranges), i64(m), ptr(table), ptr(order),
+              ptr(ws), csize(ws.numel()), ptr(new_ranges), ptr(new_table))
+    ends = ranges.long().cpu()
+    lists = [table[a:b].cpu() for a, b in zip([0] + ends.tolist(), ends.tolist())]
+    picked = [lists[i] for i in order.tolist()]
+    assert torch.equal(new_ranges.cpu().long(),
+                       torch.tensor([len(p) for p in picked]).cumsum(0))
+    assert torch.equal(new_table[:, 0].cpu(), torch.cat(picked)[:, 0])
+    assert torch.equal(new_table[:, 1].cpu().long(),
+                       torch.arange(n).repeat_interleave(torch.tensor([len(p) for p in picked])))
+    values = torch.rand(n, device="cuda", generator=gen)
+    _lib.call("gather_pdf", stream(), i64(m), ptr(table), ptr(values), ptr(pdf))
+    assert torch.equal(pdf, values[table[:, 0].long()])
