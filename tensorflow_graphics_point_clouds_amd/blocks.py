@@ -91,6 +91,8 @@ class BatchNorm(torch.nn.BatchNorm1d):
         out = self._forward(features, training)
         if negative_slope is None:
             return out
+        if negative_slope == 0:                    # (a leaky ReLU of slope 0 makes NaN of -inf)
+            return torch.relu(out)
         return torch.nn.functional.leaky_relu(out, negative_slope)
 
     def _forward(self, features, training):

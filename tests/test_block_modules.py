@@ -50,6 +50,20 @@ def test_forwards_of_subclasses_run(norm, act, expect):
     assert torch.allclose(blocks._norm_act(_norm(norm), act, x, True), expect(_expected(x)), atol=1e-6)
 
 
+@pytest.mark.parametrize("act", [torch.relu, torch.nn.ReLU()])
+def test_relu_of_infinities_without_the_kernels(act):
+    """Where torch's operations run instead of the kernels they are a ReLU's too: 0 at -inf, and
+    the gradient of NaN passes."""
+    norm = _norm().eval()
+    x = torch.tensor([[-float("inf"), -1.0, 2.0], [float("nan"), float("inf"), 0.0]],
+                     requires_grad=True)
+    expect = act(norm(x))
+    got = blocks._norm_act(norm, act, x)
+    assert torch.equal(torch.nan_to_num(got, nan=-7.0), torch.nan_to_num(expect, nan=-7.0))
+    want = torch.autograd.grad(expect.sum(), x)[0]
+    assert torch.equal(torch.autograd.grad(got.sum(), x)[0], want)
+
+
 def test_forward_of_an_instance_runs():
     act = torch.nn.ReLU()
     act.forward = lambda z: z * 2.0
