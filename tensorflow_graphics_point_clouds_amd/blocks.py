@@ -79,12 +79,15 @@ class BatchNorm(torch.nn.BatchNorm1d):
 
     def forward(self, features, training=None, negative_slope=None):
         training = self.training if training is None else bool(training)
+        weight, bias = self.weight, self.bias
         if (_plain_rows(features) and features.shape[1] == self.num_features and
-                features.shape[0] > 1 and self.weight is not None and self.momentum is not None and
-                self.running_mean is not None and self.weight.dtype == _F32 and
-                self.running_mean.dtype == _F32 and self.weight.device == features.device and
+                features.shape[0] > 1 and weight is not None and bias is not None and
+                self.momentum is not None and self.running_mean is not None and
+                weight.dtype == bias.dtype == self.running_mean.dtype == _F32 and
+                weight.device == features.device and
+                weight.is_contiguous() and bias.is_contiguous() and
                 (negative_slope is None or negative_slope >= 0)):
-            return _lib.host().norm_act(features, self.weight, self.bias, self.running_mean,
+            return _lib.host().norm_act(features, weight, bias, self.running_mean,
                                         self.running_var, self.num_batches_tracked, training,
                                         self.momentum, self.eps,
                                         1.0 if negative_slope is None else negative_slope)
