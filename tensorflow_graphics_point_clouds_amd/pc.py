@@ -626,6 +626,8 @@ class Neighborhood:
         grid = self._grid
         inv_bw = _reciprocal(_as_vector(bandwidth, d, dev))
         nbh = self if self._equal_samples else grid.known_self_neighborhood(self._radii)
+        if nbh is None and grid._sorted_points.requires_grad:
+            nbh = grid.self_neighborhood(self._radii)       # (gradients come from the pairs)
         if nbh is None:          # the points' own pairs are not at hand: densities from the grid
             points, ids, keys, ds, num_cells, smin, inv_cell = grid.search_tensors()
             self._pdf_per_point = _lib.host().grid_density(

@@ -213,3 +213,21 @@ def test_steps_of_the_c_abi_that_the_package_calls_in_one(n, batch):
     values = torch.rand(n, device="cuda", generator=gen)
     _lib.call("gather_pdf", stream(), i64(m), ptr(table), ptr(values), ptr(pdf))
     assert torch.equal(pdf, values[table[:, 0].long()])
+
+
+def test_densities_differentiable_in_the_sorted_points():
+    """A neighbourhood with centres of its own takes the densities from the grid, without the
+    points' pairs; with points that require a gradient they come from the pairs."""
+    from tensorflow_graphics_point_clouds_amd import pc
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    pts = torch.rand((500, 3), device="cuda", generator=gen)
+    ids = torch.zeros(500, dtype=torch.int32, device="cuda")
+    grads = []
+    for centres in (pc.PointCloud(pts[::3].contiguous(), ids[::3].contiguous(), 1), None):
+        grid = pc.Grid(pc.PointCloud(pts, ids, 1), 0.2)
+        grid._sorted_points.requires_grad_()
+        pdf = pc.Neighborhood(grid, 0.2, centres).point_pdf(bandwidth=0.2)
+        grads.append(torch.autograd.grad(pdf.square().sum(), grid._sorted_points)[0])
+    assert grads[0].norm() > 0
+    # the same sums of some tens of float32 terms, in another order at most
+    assert (grads[0] - grads[1]).norm() <= 1e-5 * grads[1].norm()
