@@ -531,7 +531,14 @@ extern "C" int mccnn_neighbourhood_order(mccnn_stream_t stream, int64_t num_samp
 // Where the grouped kernels are the faster ones.  Finding the order takes 0.05 ms (0.17 ms for
 // 800 k centres), so a table has to hold work:
 // * shapes without a matrix-core kernel with one atomic per pair and channel: from 2^20 pairs x
-//   channels on (there 0.09 against 0.1 ms, and 3 to 12 times faster from 2^24 on);
+//   channels on, if the other kernels have as much to do as the order and the groups cost.  Those
+//   kernels take about 0.55 ns per pair and 512 elements of C x K (at least one such unit, half
+//   as much again at K = 64, and hardly more for many channels at K = 8), plus about 2 us per pair
+//   of a centre's serial list; the grouped ones 75 to 125 us up to 200 k pairs, the more the
+//   shorter the lists, whose points repeat less.  Other / grouped kernels in us:
+//   96 x 8: 4551 centres of 7 pairs 48 / 125, 5461 of 19 130 / 106;
+//   24 x 8: 9102 of 7 64 / 122, 36 408 of 7 167 / 150; 64 x 64: 3413 of 7 178 / 144;
+//   16 x 8: 13 653 of 7 76 / 119, 109 226 of 7 433 / 186; 3 x 64: 174 762 of 21 3705 / 791.
 // * the others: from 2^27 on, and where the atomics are most of the time (many channels or
 //   columns) and a group of centres shares its points and fits the table: 16 to 80 pairs per
 //   centre (128 x 32: 7.5 pairs per centre 7.9 against 8.7 ms, 20 pairs 11.1 / 9.4, 52 pairs
@@ -541,7 +548,12 @@ extern "C" int mccnn_basis_proj_grads_grouped_pays(int num_features, int num_bas
   if (group_slices(num_features, num_basis) == 0 || num_samples <= 0 || num_neighbors > kMostPairs)
     return 0;
   const int64_t work = num_neighbors * num_features;
-  if (!mfma_grads_supported(num_features, num_basis)) return work >= ((int64_t)1 << 20) ? 1 : 0;
+  if (!mfma_grads_supported(num_features, num_basis)) {
+    const double units = num_features * num_basis * (num_basis == 64 ? 1.5 : 1.0) / 512;
+    const double per_pair = num_basis == 8 ? 0.875 : units > 1 ? units : 1.0;
+    return work >= ((int64_t)1 << 20) &&
+           num_neighbors * per_pair + 14e3 * num_neighbors / num_samples >= 280e3 ? 1 : 0;
+  }
   return work >= ((int64_t)1 << 27) && num_features * num_basis >= 2048 &&
                  num_neighbors >= 16 * num_samples && num_neighbors <= 80 * num_samples
              ? 1 : 0;

@@ -170,3 +170,18 @@ def test_grouped_basis_gradients_stop_short_of_the_last_pair_indices(lib):
         rc = lib.mccnn_basis_proj_grads_grouped(None, i64(0), 8, None, 24, None, i64(pairs), None,
                                                 i64(5), None, None, None, None, sz(0), None, None)
         assert rc == 1 and b"2^31 - 1024" in lib.mccnn_last_error()
+
+
+@pytest.mark.parametrize("c,k,centres,pairs,grouped", [
+    # short lists: the kernels per pair and channel take 0.4 to 0.8 of the time
+    (64, 8, 3413, 23249, 0), (96, 8, 9102, 62418, 0), (24, 16, 9102, 62418, 0),
+    (16, 8, 13653, 94583, 0), (96, 16, 2275, 14775, 0), (128, 8, 4551, 43397, 0),
+    # the grouped ones take 0.1 to 0.9 of it: more pairs, longer lists, more columns
+    (24, 8, 36408, 256794, 1), (16, 32, 27306, 191624, 1), (96, 8, 5461, 106117, 1),
+    (64, 64, 3413, 23249, 1), (128, 64, 1706, 11124, 1), (3, 64, 174762, 3739442, 1),
+    # under 2^20 pairs x channels
+    (3, 64, 3000, 150000, 0)])
+def test_small_tables_of_short_lists_keep_the_ungrouped_basis_gradients(lib, c, k, centres, pairs,
+                                                                        grouped):
+    i64 = ctypes.c_int64
+    assert lib.mccnn_basis_proj_grads_grouped_pays(c, k, i64(centres), i64(pairs)) == grouped
