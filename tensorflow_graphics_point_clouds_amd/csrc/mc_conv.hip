@@ -16,10 +16,36 @@
 
 namespace mccnn {
 
-constexpr int kProjRun = 8;        // consecutive centres per wavefront
+constexpr int kProjRun = 8;        // consecutive centres per wavefront, at most
 constexpr int kGradRun = 8;        // the same in the gradient kernels
 
-// One wavefront per (run of kProjRun consecutive centres, chunk of 16*kCPL channels):
+// Centres per wavefront of the projection: all eight (the table's stretch is then walked in
+// full chunks of 64 pairs) only where the runs still give every SIMD its five wavefronts several
+// times over.  A wavefront walks its run as one chain of dependent loads, so on fewer centres
+// shorter runs on more wavefronts take less time although their chunks are part empty; the sums
+// of a centre keep their order (equal bits).  64 channels, 37 pairs a centre, runs of 8 / 4 / 2 / 1:
+// 25.7 / 16.4 / 13.3 / 14.0 us on 8 k centres, 79 / 46 / 34 / 26 on 16 k, 58 / 46 / 41 / 44 on 33 k,
+// 102 / 86 / 88 / - on 70 k, 182 / 176 on 140 k, 430 / 430 on 300 k.
+static int project_run_len(int64_t num_samples, int chunks) {
+  const int64_t items = num_samples * chunks;
+  if (items >= (int64_t)kProjRun * 20000) return kProjRun;
+  int run = kProjRun / 2;
+  while (run > 1 && items < run * (int64_t)16000) run >>= 1;
+  return run;
+}
+
+// The same for the gradient kernels, whose blocks add a partial sum each: never fewer than two
+// centres, and lists of fewer than 16 pairs keep longer runs.  64 channels, runs of 8 / 4 / 2 / 1:
+// 25 / 17 / 13 / 14 us on 4 k centres of 19 pairs, 87 / 55 / 47 / 45 on 16 k of 31,
+// 74 / 66 / 66 / 77 on 33 k of 30; 43 / 43 / 47 / 58 on 33 k of 8.
+static int grad_run_len(int64_t num_samples, int64_t num_neighbors) {
+  const int64_t waves = num_neighbors >= 16 * num_samples ? 8000 : 4000;
+  int run = kGradRun;
+  while (run > 2 && num_samples < run * waves) run >>= 1;
+  return run;
+}
+
+// One wavefront per (run of up to kProjRun consecutive centres, chunk of 16*kCPL channels):
 // projection of the centres' pairs with the basis evaluated in registers, rows
 // written to out_rows[centre] (or centre).  Lane (quarter, col) owns channels
 // col, col + 16, ... of the chunk, so that each of its kCPL stores lands in one
@@ -41,16 +67,16 @@ __device__ __forceinline__ void project_run_body(
     int64_t n_out, int C, int chunks, const float *__restrict__ feat,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, const McParams<D> &p,
     const Basis &basis, const int *__restrict__ out_rows, float *__restrict__ out,
-    PairStage *stage, bool aux_is_point = false) {
+    PairStage *stage, int run_len, bool aux_is_point = false) {
   constexpr int K = kFusedK * KT;          // basis columns, KT tiles of 16
   constexpr int kCW = 16 * kCPL;
   const int lane = lane_id();
   const int64_t wid = wave_slot_xcd();
   const int64_t run = wid / chunks;
-  const int64_t c0 = run * kProjRun;
+  const int64_t c0 = run * run_len;
   if (c0 >= n_out) return;
   const int chunk = (int)(wid - run * chunks);
-  const int nc = (int)(n_out - c0 < kProjRun ? n_out - c0 : kProjRun);
+  const int nc = (int)(n_out - c0 < run_len ? n_out - c0 : run_len);
   const int quarter = lane >> 4, col = lane & 15;
   // lane i < nc: end offset and output row of centre c0 + i
   int my_end = 0, my_row = 0;
@@ -219,13 +245,13 @@ __device__ __forceinline__ void project_run_body(
 
 template <int kCPL, int D, int kAct, int KT>
 __global__ void __launch_bounds__(256) mc_conv_project16_kernel(
-    int64_t n_out, int C, int chunks, const float *__restrict__ feat,
+    int64_t n_out, int C, int chunks, int run_len, const float *__restrict__ feat,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, McParams<D> p,
     const int *__restrict__ out_rows, float *__restrict__ out) {
   __shared__ PairStage stages[kWavesPerBlock];
   const MlpBasis<D, kAct, KT> basis(p);
   project_run_body<kCPL, D, KT>(n_out, C, chunks, feat, nbrs, ranges, p, basis, out_rows, out,
-                                &stages[threadIdx.x / kWave]);
+                                &stages[threadIdx.x / kWave], run_len);
 }
 
 // The same projection with the kernel-point correlation of KPConv as basis
@@ -233,14 +259,14 @@ __global__ void __launch_bounds__(256) mc_conv_project16_kernel(
 // columns, zero padding beyond the last point).
 template <int kCPL, int D, int kKind, int KT>
 __global__ void __launch_bounds__(256) kp_conv_project16_kernel(
-    int64_t n_out, int C, int chunks, const float *__restrict__ feat,
+    int64_t n_out, int C, int chunks, int run_len, const float *__restrict__ feat,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, McParams<D> p,
     const float *__restrict__ kernel_points, int num_kp, float sigma,
     const int *__restrict__ out_rows, float *__restrict__ out) {
   __shared__ PairStage stages[kWavesPerBlock];
   const KpBasis<D, kKind, KT> basis(kernel_points, num_kp, sigma);
   project_run_body<kCPL, D, KT>(n_out, C, chunks, feat, nbrs, ranges, p, basis, out_rows, out,
-                                &stages[threadIdx.x / kWave]);
+                                &stages[threadIdx.x / kWave], run_len);
 }
 
 // The projection of the deformable kernel-point convolution (KPConv.py:317-392): as
@@ -249,7 +275,7 @@ __global__ void __launch_bounds__(256) kp_conv_project16_kernel(
 // the shifts belong to the gathered side of a pair.
 template <int kCPL, int D, int kKind>
 __global__ void __launch_bounds__(256) kp_deform_project16_kernel(
-    int64_t n_out, int C, int chunks, const float *__restrict__ feat,
+    int64_t n_out, int C, int chunks, int run_len, const float *__restrict__ feat,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, McParams<D> p,
     const float *__restrict__ kernel_points, int num_kp, float sigma,
     const float *__restrict__ offsets, int offsets_follow_points,
@@ -257,7 +283,7 @@ __global__ void __launch_bounds__(256) kp_deform_project16_kernel(
   __shared__ PairStage stages[kWavesPerBlock];
   const KpDeformBasis<D, kKind> basis(kernel_points, num_kp, sigma, offsets);
   project_run_body<kCPL, D, 1>(n_out, C, chunks, feat, nbrs, ranges, p, basis, out_rows, out,
-                               &stages[threadIdx.x / kWave], offsets_follow_points != 0);
+                               &stages[threadIdx.x / kWave], run_len, offsets_follow_points != 0);
 }
 
 // Gradient of the deformable convolution with respect to the kernel-point offsets,
@@ -270,7 +296,7 @@ __global__ void __launch_bounds__(256) kp_deform_project16_kernel(
 // quarter at the end of the centre: fixed order, no atomics.
 template <int C, int D, int kKind>
 __global__ void __launch_bounds__(256) kp_deform_offset_grads16_kernel(
-    int64_t n_out, const float *__restrict__ feat, const int2 *__restrict__ nbrs,
+    int64_t n_out, int run_len, const float *__restrict__ feat, const int2 *__restrict__ nbrs,
     const int *__restrict__ ranges, McParams<D> p, const float *__restrict__ kernel_points,
     int num_kp, float sigma, const float *__restrict__ offsets,
     const float *__restrict__ in_grad, float *__restrict__ doffsets) {
@@ -291,8 +317,8 @@ __global__ void __launch_bounds__(256) kp_deform_offset_grads16_kernel(
       kp[r][d] = (d < D && 4 * quarter + r < num_kp) ? kernel_points[(4 * quarter + r) * D + d]
                                                      : 0.0f;
   const char *feat_lane = reinterpret_cast<const char *>(feat + quarter * kQuarterC);
-  const int64_t first = wave_slot() * kGradRun;
-  const int64_t last = first + kGradRun < n_out ? first + kGradRun : n_out;
+  const int64_t first = wave_slot() * run_len;
+  const int64_t last = first + run_len < n_out ? first + run_len : n_out;
   for (int64_t centre = first; centre < last; ++centre) {
     const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
     float sum[4][3];
@@ -480,15 +506,15 @@ __global__ void __launch_bounds__(256) mc_conv_feature_grads16_kernel(
 // already in flight, and the result is folded in registers into
 //   dW[d][k] += delta_d * dz,  db[k] += dz,  dz = dbasis * act'(z) / pdf.
 
-static int64_t grad_blocks(int64_t num_samples) {
-  const int64_t per_block = (int64_t)kWavesPerBlock * kGradRun;
+static int64_t grad_blocks(int64_t num_samples, int run_len) {
+  const int64_t per_block = (int64_t)kWavesPerBlock * run_len;
   const int64_t b = (num_samples + per_block - 1) / per_block;
   return b < 1 ? 1 : b;
 }
 
 template <int C, int D, int kAct, int KT>
 __global__ void __launch_bounds__(256) mc_conv_weight_grads16_kernel(
-    int64_t n_out, const float *__restrict__ feat, const int2 *__restrict__ nbrs,
+    int64_t n_out, int run_len, const float *__restrict__ feat, const int2 *__restrict__ nbrs,
     const int *__restrict__ ranges, McParams<D> p, const float *__restrict__ in_grad,
     float *__restrict__ partials, float *__restrict__ pair_sums, int64_t pair_stride) {
   constexpr int K = kFusedK;               // a block works on basis columns k0 .. k0 + 15
@@ -526,8 +552,8 @@ __global__ void __launch_bounds__(256) mc_conv_weight_grads16_kernel(
   // on the scene-scale case, for this kernel and the projection: 12 % slower; dealing
   // windows of consecutive blocks to the XCDs in turn leaves the time as it is and
   // cuts the re-fetched feature rows.)
-  const int64_t first = wave_slot_xcd() * kGradRun;
-  const int64_t last = first + kGradRun < n_out ? first + kGradRun : n_out;
+  const int64_t first = wave_slot_xcd() * run_len;
+  const int64_t last = first + run_len < n_out ? first + run_len : n_out;
   for (int64_t centre = first; centre < last; ++centre) {
     const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
     if (b <= a) continue;
@@ -621,9 +647,49 @@ __global__ void __launch_bounds__(256) mc_conv_weight_grads16_kernel(
   }
 }
 
-// weight_grads [L, D, H], bias_grads [L*H] from partials [blocks][(D+1)][K]: one
-// block per output, threads stride over the partials, fixed summation order.
-__global__ void __launch_bounds__(256) mc_conv_reduce_kernel(int64_t blocks, int D, int K, int H,
+// The partial sums of many blocks, `rows` rows of `outs` = (D + 1) K floats, folded in place
+// before the reduction below: block b adds its `per` rows into the first of them.  Lanes run
+// along a row (every read is whole cache lines; the reduction reads 4 bytes of each row per block:
+// 53 us for the 23 846 rows of a 763 k-point layer, 6.3 + 4.6 us with both kernels; at 1907 rows
+// the reduction alone takes 4.7 us, so up to some 4000 rows the second launch does not pay).
+constexpr int kReduceDirect = 4096, kReduceBlocks = 256;
+
+__global__ void __launch_bounds__(256) mc_conv_fold_kernel(int64_t rows, int64_t per, int outs,
+                                                           float *__restrict__ partials) {
+  __shared__ float red[256];
+  const int64_t r0 = blockIdx.x * per;
+  const int64_t r1 = r0 + per < rows ? r0 + per : rows;
+  const int width = outs < 256 ? outs : 256;          // columns at a time; outs >= 48
+  const int groups = 256 / width;
+  const int g = threadIdx.x / width, c = threadIdx.x - g * width;
+  for (int c0 = 0; c0 < outs; c0 += width) {
+    float s = 0.0f;
+    if (g < groups && c0 + c < outs) {
+      const float *p = partials + c0 + c;
+      int64_t r = r0 + g;
+      for (; r + 3 * groups < r1; r += 4 * groups) {  // four rows in flight
+        float v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = p[(r + u * groups) * outs];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s += v[u];
+      }
+      for (; r < r1; r += groups) s += p[r * outs];
+    }
+    red[threadIdx.x] = s;
+    __syncthreads();                                  // (all reads of these columns are done)
+    if (g == 0 && c0 + c < outs) {
+      for (int i = 1; i < groups; ++i) s += red[i * width + c];
+      partials[r0 * outs + c0 + c] = s;
+    }
+    __syncthreads();
+  }
+}
+
+// weight_grads [L, D, H], bias_grads [L*H] from `blocks` partials of [(D+1)][K], `stride` floats
+// apart: one block per output, threads stride over the partials, fixed summation order.
+__global__ void __launch_bounds__(256) mc_conv_reduce_kernel(int64_t blocks, int64_t stride,
+                                                             int D, int K, int H,
                                                              const float *__restrict__ partials,
                                                              float *__restrict__ dweights,
                                                              float *__restrict__ dbiases) {
@@ -631,7 +697,7 @@ __global__ void __launch_bounds__(256) mc_conv_reduce_kernel(int64_t blocks, int
   const int t = blockIdx.x;
   const int q = t / K, j = t - q * K;
   float s = 0.0f;
-  for (int64_t b = threadIdx.x; b < blocks; b += 256) s += partials[b * (D + 1) * K + t];
+  for (int64_t b = threadIdx.x; b < blocks; b += 256) s += partials[b * stride + t];
   s = wave_sum(s);
   if (lane_id() == 0) red[threadIdx.x / kWave] = s;
   __syncthreads();
@@ -652,22 +718,23 @@ static int launch_fused_backward(hipStream_t s, int64_t num_samples, const float
                                  int num_basis, const float *in_grads, float *feature_grads_out,
                                  float *pair_rows, float *workspace, bool want_dfeat,
                                  float *pair_sums, int64_t num_neighbors) {
-  const dim3 grid((unsigned)grad_blocks(num_samples), (unsigned)(num_basis / kFusedK));
+  const int run_len = grad_run_len(num_samples, num_neighbors);
+  const dim3 grid((unsigned)grad_blocks(num_samples, run_len), (unsigned)(num_basis / kFusedK));
   switch (num_basis / kFusedK) {
     case 1:
       hipLaunchKernelGGL((mc_conv_weight_grads16_kernel<C, D, ACT, 1>), grid, dim3(256), 0, s,
-                         num_samples, features, nb, ranges, prm, in_grads, workspace, pair_sums,
-                         num_neighbors);
+                         num_samples, run_len, features, nb, ranges, prm, in_grads, workspace,
+                         pair_sums, num_neighbors);
       break;
     case 2:
       hipLaunchKernelGGL((mc_conv_weight_grads16_kernel<C, D, ACT, 2>), grid, dim3(256), 0, s,
-                         num_samples, features, nb, ranges, prm, in_grads, workspace, pair_sums,
-                         num_neighbors);
+                         num_samples, run_len, features, nb, ranges, prm, in_grads, workspace,
+                         pair_sums, num_neighbors);
       break;
     default:
       hipLaunchKernelGGL((mc_conv_weight_grads16_kernel<C, D, ACT, 4>), grid, dim3(256), 0, s,
-                         num_samples, features, nb, ranges, prm, in_grads, workspace, pair_sums,
-                         num_neighbors);
+                         num_samples, run_len, features, nb, ranges, prm, in_grads, workspace,
+                         pair_sums, num_neighbors);
       break;
   }
   if (want_dfeat)        // the feature half keeps no running sums: one wavefront per centre
@@ -753,7 +820,8 @@ extern "C" int mccnn_mc_conv_project(mccnn_stream_t stream, int num_dims, int64_
   for (int c = 8 / kt; c >= 1; c >>= 1)
     if (num_features % (16 * c) == 0) { cpl = c; break; }
   const int chunks = num_features / (16 * cpl);
-  const dim3 grid(wave_grid((num_samples + kProjRun - 1) / kProjRun * chunks)), block(256);
+  const int run_len = project_run_len(num_samples, chunks);
+  const dim3 grid(wave_grid((num_samples + run_len - 1) / run_len * chunks)), block(256);
   const int2 *nb = (const int2 *)neighbors;
 #define MCCNN_FUSED_FWD(CPL_, D_, KT_)                                                         \
   {                                                                                            \
@@ -762,7 +830,7 @@ extern "C" int mccnn_mc_conv_project(mccnn_stream_t stream, int num_dims, int64_
     MCCNN_ACT_SWITCH(activation,                                                               \
                      hipLaunchKernelGGL((mc_conv_project16_kernel<CPL_, D_, ACT, KT_>), grid,  \
                                         block, 0, s, num_samples, num_features, chunks,        \
-                                        features, nb, ranges, prm, out_rows, out));            \
+                                        run_len, features, nb, ranges, prm, out_rows, out));            \
   }
 #define MCCNN_FUSED_FWD_D(CPL_, KT_) \
   if (num_dims == 3) MCCNN_FUSED_FWD(CPL_, 3, KT_) else MCCNN_FUSED_FWD(CPL_, 2, KT_)
@@ -786,7 +854,9 @@ extern "C" int mccnn_mc_conv_project(mccnn_stream_t stream, int num_dims, int64_
 extern "C" size_t mccnn_mc_conv_project_grads_workspace_bytes(int num_dims, int num_basis,
                                                               int64_t num_samples) {
   if (!valid_dims(num_dims) || num_basis <= 0 || num_samples < 0) return 0;
-  return align256(sizeof(float) * (size_t)grad_blocks(num_samples) * (num_dims + 1) * num_basis);
+  // (the shortest runs that any number of pairs leads to)
+  const int run_len = grad_run_len(num_samples, (int64_t)1 << 40);
+  return align256(sizeof(float) * (size_t)grad_blocks(num_samples, run_len) * (num_dims + 1) * num_basis);
 }
 
 static int project_grads(
@@ -852,9 +922,19 @@ static int project_grads(
   if (rc != MCCNN_OK) return rc;
   MCCNN_LAUNCH_CHECK();
   const int outs = (num_dims + 1) * num_basis;
-  hipLaunchKernelGGL(mc_conv_reduce_kernel, dim3(outs), dim3(256), 0, s,
-                     grad_blocks(num_samples), num_dims, num_basis, num_basis / num_mlps, (const float *)workspace,
-                     weight_grads_out, bias_grads_out);
+  int64_t rows = grad_blocks(num_samples, grad_run_len(num_samples, num_neighbors)), stride = outs;
+  if (rows > kReduceDirect) {
+    const int64_t per = (rows + kReduceBlocks - 1) / kReduceBlocks;
+    const int64_t blocks = (rows + per - 1) / per;
+    hipLaunchKernelGGL(mc_conv_fold_kernel, dim3((unsigned)blocks), dim3(256), 0, s, rows, per,
+                       outs, (float *)workspace);
+    MCCNN_LAUNCH_CHECK();
+    rows = blocks;
+    stride = per * outs;
+  }
+  hipLaunchKernelGGL(mc_conv_reduce_kernel, dim3(outs), dim3(256), 0, s, rows, stride, num_dims,
+                     num_basis, num_basis / num_mlps, (const float *)workspace, weight_grads_out,
+                     bias_grads_out);
   MCCNN_LAUNCH_CHECK();
   if (gathered && num_samples > 0 && num_neighbors > 0)
     return launch_dfeat_gather(s, num_pts, num_features, point_ranges, pair_order, pair_rows,
@@ -926,13 +1006,14 @@ extern "C" int mccnn_kp_conv_project(mccnn_stream_t stream, int num_dims, int64_
   for (int c = 8 / kt; c >= 1; c >>= 1)
     if (num_features % (16 * c) == 0) { cpl = c; break; }
   const int chunks = num_features / (16 * cpl);
-  const dim3 grid(wave_grid((num_samples + kProjRun - 1) / kProjRun * chunks)), block(256);
+  const int run_len = project_run_len(num_samples, chunks);
+  const dim3 grid(wave_grid((num_samples + run_len - 1) / run_len * chunks)), block(256);
   const int2 *nb = (const int2 *)neighbors;
 #define MCCNN_KP_FWD(CPL_, D_, KIND_, KT_)                                                     \
   {                                                                                            \
     McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 1, 0};       \
     hipLaunchKernelGGL((kp_conv_project16_kernel<CPL_, D_, KIND_, KT_>), grid, block, 0, s,    \
-                       num_samples, num_features, chunks, features, nb, ranges, prm,           \
+                       num_samples, num_features, chunks, run_len, features, nb, ranges, prm,           \
                        kernel_points, num_kernel_points, sigma, out_rows, out);                \
   }
 #define MCCNN_KP_FWD_D(CPL_, KT_)                                                  \
@@ -995,13 +1076,14 @@ extern "C" int mccnn_kp_deform_project(mccnn_stream_t stream, int num_dims, int6
   for (int c = 8; c >= 1; c >>= 1)
     if (num_features % (16 * c) == 0) { cpl = c; break; }
   const int chunks = num_features / (16 * cpl);
-  const dim3 grid(wave_grid((num_samples + kProjRun - 1) / kProjRun * chunks)), block(256);
+  const int run_len = project_run_len(num_samples, chunks);
+  const dim3 grid(wave_grid((num_samples + run_len - 1) / run_len * chunks)), block(256);
   const int2 *nb = (const int2 *)neighbors;
 #define MCCNN_KPD(CPL_, D_, KIND_)                                                             \
   {                                                                                            \
     McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 1, 0};       \
     hipLaunchKernelGGL((kp_deform_project16_kernel<CPL_, D_, KIND_>), grid, block, 0, s,       \
-                       num_samples, num_features, chunks, features, nb, ranges, prm,           \
+                       num_samples, num_features, chunks, run_len, features, nb, ranges, prm,           \
                        kernel_points, num_kernel_points, sigma, offsets, offsets_follow_points, \
                        out_rows, out);                                                         \
   }
@@ -1048,13 +1130,14 @@ extern "C" int mccnn_kp_deform_offset_grads(mccnn_stream_t stream, int num_dims,
                                                                    neighbors)),
                 "kp_deform_offset_grads received a null tensor");
   hipStream_t s = as_stream(stream);
-  const dim3 grid((unsigned)grad_blocks(num_samples)), block(256);
+  const int run_len = grad_run_len(num_samples, num_neighbors);
+  const dim3 grid((unsigned)grad_blocks(num_samples, run_len)), block(256);
   const int2 *nb = (const int2 *)neighbors;
 #define MCCNN_KPG(C_, D_, KIND_)                                                               \
   {                                                                                            \
     McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 1, 0};       \
     hipLaunchKernelGGL((kp_deform_offset_grads16_kernel<C_, D_, KIND_>), grid, block, 0, s,    \
-                       num_samples, features, nb, ranges, prm, kernel_points,                  \
+                       num_samples, run_len, features, nb, ranges, prm, kernel_points,         \
                        num_kernel_points, sigma, offsets, in_grads, offset_grads_out);         \
   }
 #define MCCNN_KPG_D(C_)                                                  \
