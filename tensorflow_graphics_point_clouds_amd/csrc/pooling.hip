@@ -33,7 +33,38 @@ __global__ void __launch_bounds__(kPoolThreads) local_pool_kernel(
   }
 }
 
-// One wavefront per centre for C = 4 * 2^q <= 256 channels: a feature row is read
+// Maximum over few channels (C <= 4 with lanes = 1, 2 or 4 of them per centre): sixteen threads
+// share a centre, each a part of its list.  (One thread per centre and channel walks the list as
+// a chain of two dependent loads per pair: 131 us for one channel of 120 k centres x 37 pairs,
+// 19 us with the list shared.)  A maximum does not depend on the order.
+constexpr int kMaxShare = 16;
+
+__global__ void __launch_bounds__(kPoolThreads) local_max_shared_kernel(
+    int64_t n_out, int C, int lanes, const float *__restrict__ feat,
+    const int2 *__restrict__ nbrs, const int *__restrict__ ranges, float *__restrict__ out) {
+  const int64_t centre = (int64_t)blockIdx.x * (kPoolThreads / kMaxShare) + threadIdx.x / kMaxShare;
+  const int t = threadIdx.x % kMaxShare, parts = kMaxShare / lanes;
+  const int part = t / lanes, c = t % lanes;
+  const bool live = centre < n_out && c < C;
+  float acc = -FLT_MAX;
+  if (live) {
+    const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
+    int m = a + part;
+    for (; m + 3 * parts < b; m += 4 * parts) {
+      float v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = feat[(int64_t)nbrs[m + u * parts].x * C + c];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = fmaxf(acc, v[u]);
+    }
+    for (; m < b; m += parts) acc = fmaxf(acc, feat[(int64_t)nbrs[m].x * C + c]);
+  }
+  for (int off = lanes; off < kMaxShare; off <<= 1) acc = fmaxf(acc, __shfl_xor(acc, off, kWave));
+  if (live && part == 0) out[centre * C + c] = acc;
+}
+
+// One wavefront per centre for C = 4 * 2^q <= 256 channels (the maximum: any multiple of 4): a
+// feature row is read
 // by C/4 lanes with 16-byte loads, so one load instruction fetches 256/C rows; the
 // neighbour indices are read 64 at a time and passed around by lane shuffle, four
 // row loads are in flight per lane.  The partial results of the lane groups are
@@ -51,7 +82,8 @@ __global__ void __launch_bounds__(kPoolThreads) local_pool_rows_kernel(
   const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
   const float init = kMax ? -FLT_MAX : 0.0f;
   float4 acc = make_float4(init, init, init, init);
-  const float *fl = feat + 4 * colv;
+  const bool has = 4 * colv < C;                 // lanes past the row's end repeat its start
+  const float *fl = feat + (has ? 4 * colv : 0);
   for (int m0 = a; m0 < b; m0 += kWave) {
     const int cnt = b - m0 < kWave ? b - m0 : kWave;
     const int myidx = nbrs[m0 + (lane < cnt ? lane : 0)].x;
@@ -81,12 +113,85 @@ __global__ void __launch_bounds__(kPoolThreads) local_pool_rows_kernel(
     acc.z = kMax ? fmaxf(acc.z, z) : acc.z + z;
     acc.w = kMax ? fmaxf(acc.w, w) : acc.w + w;
   }
-  if (slot != 0) return;
+  if (slot != 0 || !has) return;
   if (!kMax) {
     const float inv = 1.0f / (float)(b - a > 0 ? b - a : 1);
     acc.x *= inv; acc.y *= inv; acc.z *= inv; acc.w *= inv;
   }
   *reinterpret_cast<float4 *>(out + centre * C + 4 * colv) = acc;
+}
+
+// Gradient of the maximum, C a multiple of 4 up to 256: rows are read as in local_pool_rows_kernel,
+// four in flight.  One pass over the list counts, per channel, the points that hold the maximum
+// and keeps the last one seen; where a channel has one such point in all (the usual case) the
+// lane that saw it adds the gradient, and only centres with ties read their rows again to hand
+// out the shares.  (Every channel on a lane of its own with two passes of dependent loads:
+// 512 us for 64 channels on 38 k centres x 52 pairs, 138 us now.)
+__global__ void __launch_bounds__(kPoolThreads) local_max_grads_rows_kernel(
+    int64_t n_out, int C, int lpr_log2, const float *__restrict__ feat,
+    const int2 *__restrict__ nbrs, const int *__restrict__ ranges, const float *__restrict__ out,
+    const float *__restrict__ out_grads, float *__restrict__ dfeat) {
+  const int64_t centre = (int64_t)blockIdx.x * (kPoolThreads / kWave) + threadIdx.x / kWave;
+  if (centre >= n_out) return;
+  const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
+  if (b <= a) return;
+  const int lane = lane_id();
+  const int lpr = 1 << lpr_log2;
+  const int slot = lane >> lpr_log2, colv = lane & (lpr - 1);
+  const int slots = kWave >> lpr_log2;
+  const bool has = 4 * colv < C;
+  const int c0 = has ? 4 * colv : 0;
+  const float4 top4 = *reinterpret_cast<const float4 *>(out + centre * C + c0);
+  const float4 grad4 = *reinterpret_cast<const float4 *>(out_grads + centre * C + c0);
+  const float top[4] = {top4.x, top4.y, top4.z, top4.w};
+  const float grad[4] = {grad4.x, grad4.y, grad4.z, grad4.w};
+  const float *fl = feat + c0;
+  int ties[4] = {0, 0, 0, 0}, where[4] = {0, 0, 0, 0};
+  auto walk = [&](auto &&visit) {
+    for (int m0 = a; m0 < b; m0 += kWave) {
+      const int cnt = b - m0 < kWave ? b - m0 : kWave;
+      const int myidx = nbrs[m0 + (lane < cnt ? lane : 0)].x;
+      for (int t0 = 0; t0 < cnt; t0 += 4 * slots) {      // uniform trip count: shuffles inside
+        float4 v[4];
+        int idx[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int n = t0 + slot + u * slots;
+          idx[u] = __shfl(myidx, n < cnt ? n : 0, kWave);
+          v[u] = *reinterpret_cast<const float4 *>(fl + (int64_t)idx[u] * C);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (!has || t0 + slot + u * slots >= cnt) continue;
+          visit(0, v[u].x, idx[u]);
+          visit(1, v[u].y, idx[u]);
+          visit(2, v[u].z, idx[u]);
+          visit(3, v[u].w, idx[u]);
+        }
+      }
+    }
+  };
+  walk([&](int j, float v, int idx) {
+    if (v == top[j]) {
+      ++ties[j];
+      where[j] = idx;
+    }
+  });
+  bool again = false;
+  float share[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    int all = ties[j];
+    for (int off = lpr; off < kWave; off <<= 1) all += __shfl_xor(all, off, kWave);
+    share[j] = grad[j] / (float)(all > 0 ? all : 1);
+    if (all == 1 && ties[j] == 1) unsafeAtomicAdd(&dfeat[(int64_t)where[j] * C + c0 + j], share[j]);
+    ties[j] = all;
+    again |= all > 1;
+  }
+  if (__ballot(again) == 0) return;
+  walk([&](int j, float v, int idx) {
+    if (ties[j] > 1 && v == top[j]) unsafeAtomicAdd(&dfeat[(int64_t)idx * C + c0 + j], share[j]);
+  });
 }
 
 template <bool kMax>
@@ -134,6 +239,9 @@ __global__ void global_pool_init_kernel(int count, int batch, bool is_max, unsig
 }
 
 constexpr int kGlobalChunk = 64;   // points walked by one thread
+// ... of which this many are in flight at a time: the walk is a chain of loads otherwise
+// (22 us for [900, 256], 8 us with eight; the same sums in the same order).
+constexpr int kGlobalAhead = 8;
 
 // Thread (chunk of points, channel): running value per run of equal batch ids,
 // flushed with one atomic when the id changes.
@@ -150,19 +258,30 @@ __global__ void __launch_bounds__(256) global_pool_kernel(int64_t n, int C,
   const int64_t i1 = i0 + kGlobalChunk < n ? i0 + kGlobalChunk : n;
   int cur = bids[i0], run = 0;
   float acc = kMax ? -FLT_MAX : 0.0f;
-  for (int64_t i = i0; i < i1; ++i) {
-    const int b = bids[i];
-    if (b != cur) {
-      if (kMax) atomicMax(&out[(int64_t)cur * C + c], enc_order(acc));
-      else unsafeAtomicAdd(reinterpret_cast<float *>(out) + (int64_t)cur * C + c, acc);
-      if (c == 0) atomicAdd(&counts[cur], run);
-      cur = b;
-      run = 0;
-      acc = kMax ? -FLT_MAX : 0.0f;
+  for (int64_t j0 = i0; j0 < i1; j0 += kGlobalAhead) {
+    int ids[kGlobalAhead];
+    float vals[kGlobalAhead];
+#pragma unroll
+    for (int u = 0; u < kGlobalAhead; ++u) {         // past the end: the last point, not counted
+      const int64_t i = j0 + u < i1 ? j0 + u : i1 - 1;
+      ids[u] = bids[i];
+      vals[u] = feat[i * C + c];
     }
-    const float v = feat[i * C + c];
-    acc = kMax ? fmaxf(acc, v) : acc + v;
-    ++run;
+#pragma unroll
+    for (int u = 0; u < kGlobalAhead; ++u) {
+      if (j0 + u >= i1) break;
+      const int b = ids[u];
+      if (b != cur) {
+        if (kMax) atomicMax(&out[(int64_t)cur * C + c], enc_order(acc));
+        else unsafeAtomicAdd(reinterpret_cast<float *>(out) + (int64_t)cur * C + c, acc);
+        if (c == 0) atomicAdd(&counts[cur], run);
+        cur = b;
+        run = 0;
+        acc = kMax ? -FLT_MAX : 0.0f;
+      }
+      acc = kMax ? fmaxf(acc, vals[u]) : acc + vals[u];
+      ++run;
+    }
   }
   if (kMax) atomicMax(&out[(int64_t)cur * C + c], enc_order(acc));
   else unsafeAtomicAdd(reinterpret_cast<float *>(out) + (int64_t)cur * C + c, acc);
@@ -221,6 +340,17 @@ static int lanes_for(int C) {
   return l;
 }
 
+// log2 of the lanes that read a row of C channels 16 bytes at a time; -1 where rows are not whole
+// 16-byte pieces or longer than a wavefront reads at once.
+static int rows_lanes_log2(int C) {
+  if (C % 4 != 0 || C > 256) return -1;
+  int q = 0;
+  while ((4 << q) < C) ++q;
+  return q;
+}
+
+static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 }  // namespace mccnn
 
 using namespace mccnn;
@@ -235,11 +365,10 @@ extern "C" int mccnn_local_pool(mccnn_stream_t stream, int kind, int64_t num_pts
   if (num_samples == 0) return MCCNN_OK;
   MCCNN_REQUIRE(ranges && out && (num_neighbors == 0 || (features && neighbors)),
                 "local_pool received a null tensor");
-  // C = 4 * 2^q <= 256: row-vectorised kernel, one wavefront per centre
-  int lpr_log2 = -1;
-  for (int q = 0; q <= 6; ++q)
-    if (num_features == (4 << q)) lpr_log2 = q;
-  if (lpr_log2 >= 0) {
+  // row-vectorised kernel, one wavefront per centre: the average over C = 4 * 2^q <= 256, the
+  // maximum (whatever its order) over every multiple of 4
+  const int lpr_log2 = rows_lanes_log2(num_features);
+  if (lpr_log2 >= 0 && (num_features == (4 << lpr_log2) || (kind == 0 && aligned16(features) && aligned16(out)))) {
     const unsigned wgrid = blocks_for(num_samples, kPoolThreads / kWave);
     if (kind == 0)
       hipLaunchKernelGGL(local_pool_rows_kernel<true>, dim3(wgrid), dim3(kPoolThreads), 0,
@@ -253,6 +382,13 @@ extern "C" int mccnn_local_pool(mccnn_stream_t stream, int kind, int64_t num_pts
     return MCCNN_OK;
   }
   const int lanes = lanes_for(num_features);
+  if (kind == 0 && lanes <= 4) {
+    hipLaunchKernelGGL(local_max_shared_kernel, dim3(blocks_for(num_samples, kPoolThreads / kMaxShare)),
+                       dim3(kPoolThreads), 0, as_stream(stream), num_samples, num_features, lanes,
+                       features, (const int2 *)neighbors, ranges, out);
+    MCCNN_LAUNCH_CHECK();
+    return MCCNN_OK;
+  }
   const unsigned grid = blocks_for(num_samples, kPoolThreads / lanes);
   if (kind == 0)
     hipLaunchKernelGGL(local_pool_kernel<true>, dim3(grid), dim3(kPoolThreads), 0,
@@ -284,6 +420,14 @@ extern "C" int mccnn_local_pool_grads(mccnn_stream_t stream, int kind, int64_t n
   if (num_samples == 0 || num_neighbors == 0) return MCCNN_OK;
   MCCNN_REQUIRE(ranges && features && neighbors && out && out_grads,
                 "local_pool_grads received a null tensor");
+  const int lpr_log2 = rows_lanes_log2(num_features);
+  if (kind == 0 && lpr_log2 >= 0 && aligned16(features) && aligned16(out) && aligned16(out_grads)) {
+    hipLaunchKernelGGL(local_max_grads_rows_kernel, dim3(blocks_for(num_samples, kPoolThreads / kWave)),
+                       dim3(kPoolThreads), 0, s, num_samples, num_features, lpr_log2, features,
+                       (const int2 *)neighbors, ranges, out, out_grads, feature_grads_out);
+    MCCNN_LAUNCH_CHECK();
+    return MCCNN_OK;
+  }
   const int lanes = lanes_for(num_features);
   const unsigned grid = blocks_for(num_samples, kPoolThreads / lanes);
   if (kind == 0)

@@ -1,0 +1,43 @@
+"""Maximum pooling where its kernels branch: channel counts on either side of the row-wise ones,
+many equal maxima, rows that are not 16-byte aligned, centres without and with long lists."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("c", [1, 2, 3, 4, 5, 12, 48, 100, 256, 260])
+@pytest.mark.parametrize("values", ["distinct", "ties", "unaligned"])
+def test_max_pooling_with_ties(c, values):
+    from tensorflow_graphics_point_clouds_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(c)
+    n, n_out = 500, 301
+    counts = torch.randint(0, 40, (n_out,), device="cuda", generator=gen)
+    counts[::7], counts[5], counts[6] = 0, 200, 64
+    ranges = torch.cumsum(counts, 0).int()
+    seg = torch.repeat_interleave(torch.arange(n_out, device="cuda"), counts)
+    # (a point at most once per list: unequal strides through the points)
+    first = torch.cumsum(counts, 0) - counts
+    ids = (torch.arange(seg.shape[0], device="cuda") - first[seg] + 13 * seg) % n
+    pairs = torch.stack([ids, seg], dim=1).int().contiguous()
+    feat = torch.randn(n, c, device="cuda", generator=gen)
+    if values == "ties":
+        feat = (feat * 2).round() / 2
+    if values == "unaligned":
+        feat = torch.cat([feat.new_zeros(1), feat.reshape(-1)])[1:].reshape(n, c)
+    feat.requires_grad_(True)
+    out = _lib.host().local_pool(feat, pairs, ranges, 0)
+    up = torch.randn(n_out, c, device="cuda", generator=gen)
+    grad, = torch.autograd.grad(out, feat, up)
+    lowest = torch.finfo(torch.float32).min
+    expect = torch.full((n_out, c), lowest, device="cuda").scatter_reduce(
+        0, seg[:, None].expand(-1, c), feat.detach()[ids], "amax")
+    assert torch.equal(out, expect)
+    top = feat.detach()[ids] == expect[seg]
+    ties = torch.zeros(n_out, c, dtype=torch.float64, device="cuda").index_add(0, seg, top.double())
+    share = torch.where(top, (up.double() / ties.clamp(min=1))[seg], 0.0)
+    want = torch.zeros(n, c, dtype=torch.float64, device="cuda").index_add(0, ids, share)
+    mag = torch.zeros(n, c, dtype=torch.float64, device="cuda").index_add(0, ids, share.abs())
+    # a point is in at most 301 lists: as many float32 additions of rounded shares
+    assert bool(((grad.double() - want).abs() <= 302 * 2.0 ** -24 * mag).all())
