@@ -62,13 +62,20 @@ struct SearchGrid {
   }
 };
 
-// The slice of sorted points in cell row r of the neighbourhood of point p (cloud b).  `ds` is
-// the column table, or null: then the whole key array [0, np) is searched.
+// Where a cell row's slice of the sorted points is looked for: in `span` of the keys, from the
+// first key <= maxk up to the first key < mink.  Nothing left to look for where mink > maxk: the
+// slice is `span` itself.
+struct KeyRange {
+  int2 span;
+  int64_t maxk, mink;
+};
+
+// Cell row r of the neighbourhood of point p (cloud b).  `ds` is the column table, or null: then
+// the whole key array [0, np) is searched.
 template <int D>
-__device__ __forceinline__ int2 cell_row_slice(const SearchGrid<D> &sg, const float *p, int b,
-                                               int r, int64_t np, const int64_t *__restrict__ keys,
-                                               const int2 *__restrict__ ds,
-                                               const float *__restrict__ smin) {
+__device__ __forceinline__ KeyRange cell_row_keys(const SearchGrid<D> &sg, const float *p, int b,
+                                                  int r, int64_t np, const int2 *__restrict__ ds,
+                                                  const float *__restrict__ smin) {
   constexpr int OD = OffsetInfo<D>::kDims;
   const GridShape<D> &g = sg.g;
   float m[D];
@@ -106,11 +113,12 @@ __device__ __forceinline__ int2 cell_row_slice(const SearchGrid<D> &sg, const fl
   // dropped here has a scaled distance of at least sqrt(1 + 1e-5) > 1, whatever the
   // rounding of the test itself (a few 1e-7), so the pairs found do not change.
   g2 *= 0.99999f;
-  if (!inside || !(g2 < 1.0f)) return make_int2(0, 0);
+  const KeyRange none = {make_int2(0, 0), 0, 1};
+  if (!inside || !(g2 < 1.0f)) return none;
   int2 span = make_int2(0, (int)np);
   if (ds) span = ds[((int64_t)b * g.n[0] + cell[0]) * g.n[1] + cell[1]];
-  if (span.y <= span.x) return make_int2(0, 0);
-  if (D == 2 && ds) return span;
+  if (span.y <= span.x) return none;
+  if (D == 2 && ds) return KeyRange{span, 0, 1};
   const int64_t aux = key_of_cell<D>(cell, g, b);
   int64_t maxk = aux, mink = aux;
   if (D > 2) {
@@ -125,22 +133,53 @@ __device__ __forceinline__ int2 cell_row_slice(const SearchGrid<D> &sg, const fl
     whi = whi < 0 ? 0 : (whi > nw - 1 ? nw - 1 : whi);
     wlo = wlo > w - 1 ? wlo : (w > 0 ? w - 1 : 0);
     whi = whi < w + 1 ? whi : (w < nw - 1 ? w + 1 : nw - 1);
-    if (whi < wlo) return make_int2(0, 0);
+    if (whi < wlo) return none;
     maxk = aux + (whi - w);
     mink = aux + (wlo - w);
   }
-  int lo = span.x, hi = span.y;
-  while (lo < hi) {                       // first index with key <= maxk
-    const int mid = lo + ((hi - lo) >> 1);
-    if (keys[mid] > maxk) lo = mid + 1; else hi = mid;
+  return KeyRange{span, maxk, mink};
+}
+
+// The slices of kN cell rows.  The two ends of all of them are searched side by side: a binary
+// search is a chain of dependent loads (eleven over 2048 keys), and what one lane has to find is
+// kept to one such chain.
+template <int kN>
+__device__ __forceinline__ void find_slices(const KeyRange *range, const int64_t *__restrict__ keys,
+                                            int2 *slice) {
+  int lo[2 * kN], hi[2 * kN];
+  bool open = false;
+#pragma unroll
+  for (int i = 0; i < kN; ++i) {
+    const bool search = range[i].mink <= range[i].maxk;
+    lo[2 * i] = range[i].span.x;
+    lo[2 * i + 1] = search ? range[i].span.x : range[i].span.y;
+    hi[2 * i] = search ? range[i].span.y : range[i].span.x;
+    hi[2 * i + 1] = range[i].span.y;
+    open |= search;
   }
-  const int first = lo;
-  hi = span.y;
-  while (lo < hi) {                       // first index with key < mink
-    const int mid = lo + ((hi - lo) >> 1);
-    if (keys[mid] >= mink) lo = mid + 1; else hi = mid;
+  while (open) {
+    open = false;
+    int64_t key[2 * kN];
+    int mid[2 * kN];
+#pragma unroll
+    for (int k = 0; k < 2 * kN; ++k) {       // (a search that has ended reads a key it ignores)
+      mid[k] = lo[k] < hi[k] ? lo[k] + ((hi[k] - lo[k]) >> 1) : 0;
+      key[k] = keys[mid[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < 2 * kN; ++k) {
+      // first index with key <= maxk, first index with key < mink
+      const bool up = k % 2 == 0 ? key[k] > range[k / 2].maxk : key[k] >= range[k / 2].mink;
+      if (lo[k] < hi[k]) {
+        lo[k] = up ? mid[k] + 1 : lo[k];
+        hi[k] = up ? hi[k] : mid[k];
+      }
+      open |= lo[k] < hi[k];
+    }
   }
-  return lo > first ? make_int2(first, lo) : make_int2(0, 0);
+#pragma unroll
+  for (int i = 0; i < kN; ++i)
+    slice[i] = lo[2 * i + 1] > lo[2 * i] ? make_int2(lo[2 * i], lo[2 * i + 1]) : make_int2(0, 0);
 }
 
 template <int D>
@@ -159,7 +198,11 @@ __global__ void __launch_bounds__(256) nbr_ranges_kernel(
     float p[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) p[d] = samples[c * D + d];
-    ranges[t] = cell_row_slice<D>(sg, p, sbids[c], (int)(t - c * R), np, keys, ds, smin);
+    const KeyRange range =
+        cell_row_keys<D>(sg, p, sbids[c], (int)(t - c * R), np, ds, smin);
+    int2 slice;
+    find_slices<1>(&range, keys, &slice);
+    ranges[t] = slice;
   }
 }
 
@@ -282,46 +325,81 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
       norm *= bw * 0.39894228f;
     }
   }
-  // the slices of the centre, kGroup at a time: lane `sub` fetches (or finds) one, the group
-  // then takes them in turn (one round trip to memory instead of one per slice)
-  for (int r0 = 0; r0 < R; r0 += kGroup) {
-    int2 mine = make_int2(0, 0);
-    if (r0 + sub < R) {
-      if constexpr (kSearch) {
-        const SearchGrid<D> sg(search.num_cells, search.inv_cell, inv_radii);
-        mine = cell_row_slice<D>(sg, s, search.sbids[c], r0 + sub, search.np, search.keys,
-                                 search.ds, search.smin);
-        if (kVisit == Visit::kCount) ranges[c * R + r0 + sub] = mine;
-      } else {
-        mine = ranges[c * R + r0 + sub];
+  auto load_point = [&](int j, float *q) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) q[d] = pts[(int64_t)j * D + d];
+  };
+  auto visit = [&](bool live, int j, const float *q) {          // kGroup candidates of the centre
+    float diff[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) diff[d] = s[d] - q[d];
+    const bool hit = live && within_radius<D>(diff, ir);
+    if (kVisit == Visit::kFill) {
+      const uint64_t hits = __ballot(hit) & group_mask;
+      const int slot = found + __popcll(hits & below_mask);
+      if (hit && slot < limit && start + slot < capacity)
+        nbrs[start + slot] = make_int2(j, (int)c);
+      found += __popcll(hits);
+    } else if (kVisit == Visit::kCount) {
+      found += hit ? 1 : 0;
+    } else {
+      const unsigned hits = (unsigned)((__ballot(hit) & group_mask) >> (lane & ~(kGroup - 1)));
+      if (hits != 0) {                         // the same for the lanes of a group
+        sums.add(hit ? density_term<D>(diff, scale) : 0.0f, hits, sub, lane & ~(kGroup - 1), found);
+        found += __popc(hits);
       }
     }
-    const int lim = R - r0 < kGroup ? R - r0 : kGroup;
-    for (int r = 0; r < lim; ++r) {
-      const int2 span = make_int2(__shfl(mine.x, r, kGroup), __shfl(mine.y, r, kGroup));
-      for (int j0 = span.x; j0 < span.y; j0 += kGroup) {
-        const int j = j0 + sub;
-        bool hit = false;
-        float diff[D];
-        if (j < span.y) {
+  };
+  // The slices of the centre, nine at a time (their number is a power of three): lane `sub`
+  // fetches or finds one, the first lane the ninth as well, and the group takes them in turn.
+  // The first candidates of kAhead slices are requested together: most slices hold one or two
+  // trips of a group, and slice by slice every one of them waits for memory again (count and
+  // fill of 763 k centres x 37 pairs 390 -> 352 us; with the searches side by side 2 x 1024 points
+  // 21 -> 18 us).
+  constexpr int kSlices = kGroup + 1, kAhead = 3;
+  static_assert(R % kSlices == 0 && kSlices % kAhead == 0, "slices come in nines");
+  for (int r0 = 0; r0 < R; r0 += kSlices) {
+    int2 mine[2] = {make_int2(0, 0), make_int2(0, 0)};          // slices r0 + sub and r0 + kGroup
+    if constexpr (kSearch) {
+      const SearchGrid<D> sg(search.num_cells, search.inv_cell, inv_radii);
+      const int b = search.sbids[c];
+      KeyRange range[2] = {
+          cell_row_keys<D>(sg, s, b, r0 + sub, search.np, search.ds, search.smin),
+          cell_row_keys<D>(sg, s, b, r0 + kGroup, search.np, search.ds, search.smin)};
+      if (sub != 0) range[1] = KeyRange{make_int2(0, 0), 0, 1};
+      find_slices<2>(range, search.keys, mine);
+      if (kVisit == Visit::kCount) {
+        ranges[c * R + r0 + sub] = mine[0];
+        if (sub == 0) ranges[c * R + r0 + kGroup] = mine[1];
+      }
+      mine[1] = make_int2(__shfl(mine[1].x, 0, kGroup), __shfl(mine[1].y, 0, kGroup));
+    } else {
+      mine[0] = ranges[c * R + r0 + sub];
+      mine[1] = ranges[c * R + r0 + kGroup];
+    }
 #pragma unroll
-          for (int d = 0; d < D; ++d) diff[d] = s[d] - pts[(int64_t)j * D + d];
-          hit = within_radius<D>(diff, ir);
-        }
-        if (kVisit == Visit::kFill) {
-          const uint64_t hits = __ballot(hit) & group_mask;
-          const int slot = found + __popcll(hits & below_mask);
-          if (hit && slot < limit && start + slot < capacity)
-            nbrs[start + slot] = make_int2(j, (int)c);
-          found += __popcll(hits);
-        } else if (kVisit == Visit::kCount) {
-          found += hit ? 1 : 0;
-        } else {
-          const unsigned hits = (unsigned)((__ballot(hit) & group_mask) >> (lane & ~(kGroup - 1)));
-          if (hits != 0) {                         // the same for the lanes of a group
-            sums.add(hit ? density_term<D>(diff, scale) : 0.0f, hits, sub, lane & ~(kGroup - 1), found);
-            found += __popc(hits);
-          }
+    for (int rb = 0; rb < kSlices; rb += kAhead) {
+      int2 span[kAhead];
+      float q[kAhead][D];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        span[u] = rb + u < kGroup ? make_int2(__shfl(mine[0].x, (rb + u) % kGroup, kGroup),
+                                              __shfl(mine[0].y, (rb + u) % kGroup, kGroup))
+                                  : mine[1];
+#pragma unroll
+        for (int d = 0; d < D; ++d) q[u][d] = 0.0f;
+        if (span[u].x + sub < span[u].y) load_point(span[u].x + sub, q[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        if (span[u].x >= span[u].y) continue;                   // the same for the lanes of a group
+        visit(span[u].x + sub < span[u].y, span[u].x + sub, q[u]);
+        for (int j0 = span[u].x + kGroup; j0 < span[u].y; j0 += kGroup) {
+          float t[D];
+#pragma unroll
+          for (int d = 0; d < D; ++d) t[d] = 0.0f;
+          if (j0 + sub < span[u].y) load_point(j0 + sub, t);
+          visit(j0 + sub < span[u].y, j0 + sub, t);
         }
       }
     }
@@ -407,8 +485,8 @@ static NbrWorkspace carve_nbr_workspace(void *ws, int d, int64_t ns) {
 }
 
 // Pair table regrouped for another order of the centres: slot q takes the
-// segment of centre order[q].  counts pass, then (after the scan) a copy pass
-// with 16 lanes per slot; the centre column is rewritten to the slot.
+// segment of centre order[q].  counts pass, then (after the scan) a copy pass;
+// the centre column is rewritten to the slot.
 __global__ void __launch_bounds__(256) segment_counts_kernel(int64_t n, const int *__restrict__ ranges,
                                                              const int *__restrict__ order,
                                                              int *__restrict__ counts) {
@@ -419,22 +497,58 @@ __global__ void __launch_bounds__(256) segment_counts_kernel(int64_t n, const in
 }
 
 // `map` (optional) replaces the point index by map[index]; either output may be null, pdf_out
-// takes the density of the pair's point.
+// takes the density of the pair's point.  A wavefront takes `slots` <= 16 consecutive slots, whose
+// pairs are one contiguous stretch of the output, and walks that stretch 64 pairs at a time, four
+// times 64 in flight; a lane finds its pair's slot by a binary search among the slots' ends.
+// (With 16 lanes on one slot the four dependent loads of a slot -- its centre, the segment, the
+// pair, the mapped index -- stood behind each other for every 37 pairs: 174 us per output of 28 M
+// pairs, 121 us now.)
+constexpr int kCopySlots = 16, kCopyAhead = 4;
+
 __global__ void __launch_bounds__(256) segment_copy_kernel(
-    int64_t n, const int *__restrict__ ranges, const int *__restrict__ order,
+    int64_t n, int slots, const int *__restrict__ ranges, const int *__restrict__ order,
     const int2 *__restrict__ pairs, const int *__restrict__ ranges_out,
     const int *__restrict__ map, int2 *__restrict__ pairs_out, const float *__restrict__ pdf,
     float *__restrict__ pdf_out) {
-  const int64_t q = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
-  if (q >= n) return;
-  const int sub = threadIdx.x & 15;
-  const int i = order[q];
-  const int src = i > 0 ? ranges[i - 1] : 0, cnt = ranges[i] - src;
-  const int dst = ranges_out[q] - cnt;
-  for (int t = sub; t < cnt; t += 16) {
-    const int j = pairs[src + t].x;
-    if (pairs_out) pairs_out[dst + t] = make_int2(map ? map[j] : j, (int)q);
-    if (pdf_out) pdf_out[dst + t] = pdf[j];
+  const int lane = lane_id();
+  const int64_t q0 = ((int64_t)blockIdx.x * (256 / kWave) + threadIdx.x / kWave) * slots;
+  if (q0 >= n) return;
+  // lane i < slots: end of slot q0 + i in the output and how far before it its pairs are read
+  int end = 0x7fffffff, shift = 0;
+  const int64_t q = q0 + lane;
+  if (lane < slots && q < n) {
+    const int i = order[q];
+    end = ranges_out[q];
+    shift = (i > 0 ? ranges[i - 1] : 0) - (q > 0 ? ranges_out[q - 1] : 0);
+  }
+  const int first = q0 > 0 ? ranges_out[q0 - 1] : 0;
+  const int last = ranges_out[(q0 + slots < n ? q0 + slots : n) - 1];
+  for (int64_t m0 = first; m0 < last; m0 += kWave * kCopyAhead) {
+    int slot[kCopyAhead], j[kCopyAhead];
+#pragma unroll
+    for (int u = 0; u < kCopyAhead; ++u) {
+      const int64_t m = m0 + u * kWave + lane;
+      slot[u] = 0;                                  // ends up to m: 0 .. 15 of the first 15
+#pragma unroll
+      for (int step = kCopySlots / 2; step > 0; step >>= 1)
+        if (__shfl(end, slot[u] + step - 1, kWave) <= m) slot[u] += step;
+      const int from = __shfl(shift, slot[u], kWave);
+      j[u] = m < last ? pairs[m + from].x : 0;
+    }
+    if (pairs_out) {
+#pragma unroll
+      for (int u = 0; u < kCopyAhead; ++u) {
+        const int64_t m = m0 + u * kWave + lane;
+        if (m < last) pairs_out[m] = make_int2(map ? map[j[u]] : j[u], (int)q0 + slot[u]);
+      }
+    }
+    if (pdf_out) {
+#pragma unroll
+      for (int u = 0; u < kCopyAhead; ++u) {
+        const int64_t m = m0 + u * kWave + lane;
+        if (m < last) pdf_out[m] = pdf[j[u]];
+      }
+    }
   }
 }
 
@@ -860,8 +974,10 @@ extern "C" int mccnn_reorder_pairs(mccnn_stream_t stream, int64_t num_samples,
   MCCNN_REQUIRE(ranges && neighbors && centre_order && ranges_out &&
                     (neighbors_out || pdf_per_pair_out) && (!pdf_per_pair_out || pdf),
                 "reorder_pairs received a null tensor");
-  hipLaunchKernelGGL(segment_copy_kernel, dim3(blocks_for(num_samples * 16, 256)), dim3(256), 0,
-                     as_stream(stream), num_samples, ranges, centre_order,
+  // few slots: a wavefront each for four of them, or the chip is not filled
+  const int slots = num_samples >= 131072 ? kCopySlots : 4;
+  hipLaunchKernelGGL(segment_copy_kernel, dim3(blocks_for(num_samples, slots * (256 / kWave))),
+                     dim3(256), 0, as_stream(stream), num_samples, slots, ranges, centre_order,
                      (const int2 *)neighbors, ranges_out, point_map, (int2 *)neighbors_out, pdf,
                      pdf_per_pair_out);
   MCCNN_LAUNCH_CHECK();
