@@ -10,7 +10,7 @@
 // are gathered.  All element offsets are 64-bit (N*C*K and M*K exceed 2^31 at
 // the benchmark sizes).
 //
-// Generic path (any valid C, K): one wavefront per (centre, chunk of up to
+// Generic gradients (any valid C, K): one wavefront per (centre, chunk of up to
 // 64*kAcc output elements); lane l owns elements l + 64*j, so its basis column
 // k = l % K is fixed and its channel advances by 64/K per j.
 #include "common.h"
@@ -20,42 +20,6 @@
 namespace mccnn {
 
 constexpr int kAcc = 16;   // accumulators per lane in the generic kernels
-
-template <int K>
-__global__ void __launch_bounds__(256) basis_proj_generic_kernel(
-    int64_t n_out, int C, int chunks, const float *__restrict__ basis,
-    const float *__restrict__ feat, const int2 *__restrict__ nbrs,
-    const int *__restrict__ ranges, const int *__restrict__ order, float *__restrict__ out) {
-  constexpr int kChanStep = kWave / K;            // channels covered by one j
-  const int lane = lane_id();
-  const int64_t wid = wave_slot();
-  const int64_t slot_centre = wid / chunks;
-  if (slot_centre >= n_out) return;
-  const int chunk = (int)(wid - slot_centre * chunks);
-  const int64_t centre = centre_of(slot_centre, order);
-  const int c0 = chunk * kAcc * kChanStep + lane / K;
-  const int k = lane % K;
-  const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
-  float acc[kAcc];
-#pragma unroll
-  for (int j = 0; j < kAcc; ++j) acc[j] = 0.0f;
-  for (int m = a; m < b; ++m) {
-    const int64_t nb = nbrs[m].x;
-    const float w = basis[(int64_t)m * K + k];
-    const float *f = feat + nb * C;
-#pragma unroll
-    for (int j = 0; j < kAcc; ++j) {
-      const int c = c0 + j * kChanStep;
-      if (c < C) acc[j] += f[c] * w;
-    }
-  }
-  float *o = out + centre * (int64_t)C * K;
-#pragma unroll
-  for (int j = 0; j < kAcc; ++j) {
-    const int c = c0 + j * kChanStep;
-    if (c < C) o[c * K + k] = acc[j];
-  }
-}
 
 // kAtomicBasis: more than one chunk contributes to dbasis[m,:].
 template <int K>
@@ -245,6 +209,160 @@ __global__ void __launch_bounds__(256) basis_proj_mfma16_kernel(
     float *dst = o + (col * kCPL + j) * K;
     *reinterpret_cast<v4f *>(dst) = acc[j];
   }
+}
+
+// Every other shape (8 basis columns, or channels that do not come in 16s or 32s): tiles of
+// v_mfma_f32_16x16x4f32 with rows = basis, columns = channels and the places past the last channel
+// (or past the eighth basis column) left empty.  A lane owns channels col + 16 j of the chunk and
+// columns col + 16 kt of the basis, so that whole rows are fetched by a quarter of the wavefront
+// and the results of a tile leave as runs of 16 K bytes at least; places without a pair, channel or
+// column read a valid address, and what multiplies a missing pair is set to zero.
+// [66 490 centres, 1.6 M pairs, 24 x 64] 528 us with a wavefront walking the pairs of 16 elements per
+// lane one by one in vector instructions, 185 us; [15 839, 317 k, 24 x 8] 48 and 13 us.
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// kFull: C is a multiple of the chunk, whose tiles are then 64 bytes apart in every row.
+template <int K, int kCPL, bool kFull>
+__global__ void __launch_bounds__(256) basis_proj_tiles_kernel(
+    int64_t n_out, int C, int chunks, const float *__restrict__ basis,
+    const float *__restrict__ feat, const int2 *__restrict__ nbrs,
+    const int *__restrict__ ranges, const int *__restrict__ order, float *__restrict__ out) {
+  constexpr int KT = K < 16 ? 1 : K / 16;
+  const int lane = lane_id();
+  const int64_t wid = wave_slot();
+  const int64_t slot_centre = wid / chunks;
+  if (slot_centre >= n_out) return;
+  const int chunk = (int)(wid - slot_centre * chunks);
+  const int64_t centre = centre_of(slot_centre, order);
+  const int quarter = lane >> 4, col = lane & 15;
+  const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
+  const int c0 = chunk * 16 * kCPL + col;
+  int from[kCPL];                                   // channel read for tile j
+#pragma unroll
+  for (int j = 0; j < kCPL; ++j) from[j] = c0 + 16 * j < C ? c0 + 16 * j : 0;
+  const float *bbase = basis + (K < 16 ? col % K : col);
+  v4f acc[kCPL][KT];
+#pragma unroll
+  for (int j = 0; j < kCPL; ++j)
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) acc[j][kt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+  for (int m0 = a; m0 < b; m0 += kWave) {
+    const int cnt = b - m0 < kWave ? b - m0 : kWave;
+    const int myidx = nbrs[m0 + (lane < cnt ? lane : 0)].x;
+    const int steps = (cnt + 3) >> 2;
+    for (int t = 0; t < steps; t += kUnroll) {
+      float f[kUnroll][kCPL], w[kUnroll][KT];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        if (t + u >= steps) break;                  // the same for the wavefront
+        const int n = 4 * (t + u) + quarter;
+        const bool valid = n < cnt;
+        const int pair = valid ? n : 0;
+        const float *row = feat + (int64_t)__shfl(myidx, pair, kWave) * C + (kFull ? c0 : 0);
+#pragma unroll
+        for (int j = 0; j < kCPL; ++j) {
+          const float v = row[kFull ? 16 * j : from[j]];
+          f[u][j] = valid ? v : 0.0f;
+        }
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+          const float v = bbase[(int64_t)(m0 + pair) * K + 16 * kt];
+          w[u][kt] = valid ? v : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        if (t + u >= steps) break;
+#pragma unroll
+        for (int j = 0; j < kCPL; ++j)
+#pragma unroll
+          for (int kt = 0; kt < KT; ++kt)
+            acc[j][kt] =
+                __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][kt], f[u][j], acc[j][kt], 0, 0, 0);
+      }
+    }
+  }
+  // acc[j][kt][r]: channel c0 + 16 j, basis column 16 kt + 4 quarter + r
+  if (K < 16 && 4 * quarter >= K) return;
+  float *o = out + centre * (int64_t)C * K + 4 * quarter;
+#pragma unroll
+  for (int j = 0; j < kCPL; ++j)
+    if (c0 + 16 * j < C)
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt)
+        __builtin_nontemporal_store(acc[j][kt], reinterpret_cast<v4f_any *>(o + (int64_t)(c0 + 16 * j) * K + 16 * kt));
+}
+
+// Eight basis columns, more than 32 channels: a lane owns whole channels, lane + 64 j, with their eight
+// sums in registers, and a pair is one row fetched by the wavefront and its eight basis values from
+// the scalar cache.  A matrix tile would be half empty (rows = basis), and what counts here is
+// instructions: [219 362 centres, 4.0 M pairs, 64 x 8] 1157 us in the walk named above, 528 us in half
+// empty tiles, 346 us.
+template <int kJ>
+__global__ void __launch_bounds__(256) basis_proj_rows8_kernel(
+    int64_t n_out, int C, int chunks, const float *__restrict__ basis,
+    const float *__restrict__ feat, const int2 *__restrict__ nbrs,
+    const int *__restrict__ ranges, const int *__restrict__ order, float *__restrict__ out) {
+  constexpr int K = 8;
+  const int lane = lane_id();
+  const int64_t wid = wave_slot();
+  const int64_t slot_centre = wid / chunks;
+  if (slot_centre >= n_out) return;
+  const int chunk = (int)(wid - slot_centre * chunks);
+  const int64_t centre = centre_of(slot_centre, order);
+  const int a = __builtin_amdgcn_readfirstlane(centre > 0 ? ranges[centre - 1] : 0);
+  const int b = __builtin_amdgcn_readfirstlane(ranges[centre]);
+  const int c0 = chunk * kWave * kJ + lane;
+  int from[kJ];
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) from[j] = c0 + kWave * j < C ? c0 + kWave * j : 0;
+  float acc[kJ][K];
+#pragma unroll
+  for (int j = 0; j < kJ; ++j)
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc[j][k] = 0.0f;
+  for (int m0 = a; m0 < b; m0 += kWave) {
+    const int cnt = b - m0 < kWave ? b - m0 : kWave;
+    const int myidx = nbrs[m0 + (lane < cnt ? lane : 0)].x;
+    for (int t = 0; t < cnt; t += kUnroll) {
+      float f[kUnroll][kJ];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {           // past the last pair: its row again, not used
+        const int n = t + u < cnt ? t + u : cnt - 1;
+        const float *row = feat + (int64_t)__builtin_amdgcn_readlane(myidx, n) * C;
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) f[u][j] = row[from[j]];
+      }
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        if (t + u >= cnt) break;
+        const float *w = basis + (int64_t)(m0 + t + u) * K;
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) acc[j][k] = fmaf(f[u][j], w[k], acc[j][k]);
+      }
+    }
+  }
+  float *o = out + centre * (int64_t)C * K;
+#pragma unroll
+  for (int j = 0; j < kJ; ++j)
+    if (c0 + kWave * j < C)
+#pragma unroll
+      for (int h = 0; h < K; h += 4) {
+        const v4f v = {acc[j][h], acc[j][h + 1], acc[j][h + 2], acc[j][h + 3]};
+        __builtin_nontemporal_store(v, reinterpret_cast<v4f_any *>(o + (int64_t)(c0 + kWave * j) * K + h));
+      }
+}
+
+// Channel tiles of a wavefront of basis_proj_tiles_kernel: one chunk if up to 64 accumulators hold
+// the row.
+static int tiles_per_wave(int C, int K) {
+  const int most = K <= 16 ? 8 : 4;
+  int cpl = 1;
+  while (cpl < most && 16 * cpl < C) cpl <<= 1;
+  return cpl;
 }
 
 // ---------------------------------------------------------------------------
@@ -548,15 +666,41 @@ extern "C" int mccnn_basis_proj_ordered(mccnn_stream_t stream, int64_t basis_row
     MCCNN_LAUNCH_CHECK();
     return MCCNN_OK;
   }
-  const int chunks = generic_chunks(num_features, num_basis);
+  if (num_basis == 8 && num_features > 32) {
+    const int per_lane = num_features > kWave ? 2 : 1, chunks = (num_features + kWave * per_lane - 1) / (kWave * per_lane);
+    const int64_t waves = num_samples * chunks;
+    MCCNN_REQUIRE(waves < ((int64_t)1 << 31), "BasisProj launch too large");
+    if (per_lane == 2)
+      hipLaunchKernelGGL(basis_proj_rows8_kernel<2>, dim3(wave_grid(waves)), dim3(256), 0, s, num_samples, num_features,
+                         chunks, basis, features, (const int2 *)neighbors, ranges, order, out);
+    else
+      hipLaunchKernelGGL(basis_proj_rows8_kernel<1>, dim3(wave_grid(waves)), dim3(256), 0, s, num_samples, num_features,
+                         chunks, basis, features, (const int2 *)neighbors, ranges, order, out);
+    MCCNN_LAUNCH_CHECK();
+    return MCCNN_OK;
+  }
+  const int tiles = tiles_per_wave(num_features, num_basis);
+  const bool full = num_features % (16 * tiles) == 0;
+  const int chunks = (num_features + 16 * tiles - 1) / (16 * tiles);
   const int64_t waves = num_samples * chunks;
   MCCNN_REQUIRE(waves < ((int64_t)1 << 31), "BasisProj launch too large");
   const unsigned grid = wave_grid(waves);
-  MCCNN_BASIS_SWITCH(num_basis,
-                     hipLaunchKernelGGL(basis_proj_generic_kernel<K>, dim3(grid), dim3(256), 0,
-                                        s, num_samples, num_features, chunks,
-                                        basis, features, (const int2 *)neighbors, ranges, order,
-                                        out));
+#define MCCNN_FWD_TILES(CPL_)                                                                   \
+  if (full)                                                                                     \
+    hipLaunchKernelGGL((basis_proj_tiles_kernel<K, CPL_, true>), dim3(grid), dim3(256), 0, s,   \
+                       num_samples, num_features, chunks, basis, features,                      \
+                       (const int2 *)neighbors, ranges, order, out);                            \
+  else                                                                                          \
+    hipLaunchKernelGGL((basis_proj_tiles_kernel<K, CPL_, false>), dim3(grid), dim3(256), 0, s,  \
+                       num_samples, num_features, chunks, basis, features,                      \
+                       (const int2 *)neighbors, ranges, order, out)
+  MCCNN_BASIS_SWITCH(num_basis, switch (tiles) {
+    case 8: if constexpr (K <= 16) { MCCNN_FWD_TILES(8); } break;
+    case 4: MCCNN_FWD_TILES(4); break;
+    case 2: MCCNN_FWD_TILES(2); break;
+    default: MCCNN_FWD_TILES(1); break;
+  });
+#undef MCCNN_FWD_TILES
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
