@@ -70,12 +70,40 @@ struct MlpBasis {                  // act(delta . W[:, col] + b[col]) / pdf   (M
   }
 };
 
+// The correlation weight of a kernel point at squared distance sq (KPConv.py:29-57).  The linear one
+// takes the square root and the quotient from their approximations with a correction by fused
+// multiply-adds (Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", 1990), which rounds both as sqrtf and the division do -- every mantissa of the root
+// and 6.7e8 quotients compared on this part, none differs -- in a third of the instructions of
+// sqrtf and the division, whose expansions also cover subnormal numbers.  The projection evaluates
+// 16 of them per pair: 120 -> 96 us for 32 channels on 98 765 centres of 37 pairs, 836 -> 813 us for the
+// two passes with shifted kernel points of 64 channels on 200 003.
+// Distances below 1e-15 count as none (the weight is 1 either way).
+template <int kKind>
+struct KpInfluence {
+  float sigma, inv;
+  __device__ __forceinline__ explicit KpInfluence(float s) : sigma(s), inv(1.0f / s) {}
+  __device__ __forceinline__ float operator()(float sq) const {
+    if (kKind != 0) {
+      const float q = sqrtf(sq) / (sigma / 3.0f);
+      return expf(-(q * q));
+    }
+    const float y = __builtin_amdgcn_rsqf(sq), g = sq * y;
+    const float root = fmaf(fmaf(-g, g, sq), 0.5f * y, g);
+    const float dist = sq < 1e-30f ? 0.0f : root;
+    const float q = dist * inv;
+    const float v = 1.0f - fmaf(fmaf(-q, sigma, dist), inv, q);
+    return v > 0.0f ? v : 0.0f;
+  }
+};
+
 template <int D, int kKind, int KT = 1>
 struct KpBasis {                   // kernel-point correlation (KPConv.py:29-57, 193-213)
-  float k[KT][3], sigma;
+  float k[KT][3];
+  KpInfluence<kKind> influence;
   bool live[KT];                   // columns past the last kernel point are zero padding
   __device__ __forceinline__ KpBasis(const float *__restrict__ kernel_points, int num_kp,
-                                     float sigma_) : sigma(sigma_) {
+                                     float sigma) : influence(sigma) {
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
       const int col = 16 * kt + (lane_id() & 15);
@@ -88,41 +116,23 @@ struct KpBasis {                   // kernel-point correlation (KPConv.py:29-57,
   static constexpr bool kUsesAux = false;
   __device__ __forceinline__ float operator()(const float4 &g, int kt = 0, int = 0) const {
     const float dx = g.x - k[kt][0], dy = g.y - k[kt][1], dz = g.z - k[kt][2];
-    const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
-    float wgt;
-    if (kKind == 0) {
-      const float v = 1.0f - dist / sigma;
-      wgt = v > 0.0f ? v : 0.0f;
-    } else {
-      const float q = dist / (sigma / 3.0f);
-      wgt = expf(-(q * q));
-    }
+    const float wgt = influence(dx * dx + dy * dy + dz * dz);
     return live[kt] ? wgt * g.w : 0.0f;
   }
 };
-
-// Correlation weight of the kernel-point convolution for a distance.
-template <int kKind>
-__device__ __forceinline__ float kp_weight(float dist, float sigma) {
-  if (kKind == 0) {
-    const float v = 1.0f - dist / sigma;
-    return v > 0.0f ? v : 0.0f;
-  }
-  const float q = dist / (sigma / 3.0f);
-  return expf(-(q * q));
-}
 
 // Deformable kernel points (KPConv.py:317-392): kernel point `col` of the centre of a
 // pair is shifted by offsets[row, col, :], where `row` (the staged aux value) is the
 // centre's row in the [N_centres, num_kp, D] offset table.  Up to 16 kernel points.
 template <int D, int kKind>
 struct KpDeformBasis {
-  float k[3], sigma;
+  float k[3];
+  KpInfluence<kKind> influence;
   const float *off;                // offsets + col * D, or null for a padding column
   int stride;                      // num_kp * D
   __device__ __forceinline__ KpDeformBasis(const float *__restrict__ kernel_points, int num_kp,
-                                           float sigma_, const float *__restrict__ offsets)
-      : sigma(sigma_), stride(num_kp * D) {
+                                           float sigma, const float *__restrict__ offsets)
+      : influence(sigma), stride(num_kp * D) {
     const int col = lane_id() & 15;
     const bool live = col < num_kp;
     k[0] = k[1] = k[2] = 0.0f;
@@ -141,7 +151,7 @@ struct KpDeformBasis {
       diff[d] -= o[d];
       sq += diff[d] * diff[d];
     }
-    return kp_weight<kKind>(sqrtf(sq), sigma) * g.w;
+    return influence(sq) * g.w;
   }
 };
 

@@ -309,6 +309,7 @@ __global__ void __launch_bounds__(256) kp_deform_offset_grads16_kernel(
   float ir[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) ir[d] = p.inv_radii[d];
+  const float neg_inv_sigma = -1.0f / sigma;
   float kp[4][3];                     // kernel points 4 quarter + r of this lane's rows
 #pragma unroll
   for (int r = 0; r < 4; ++r)
@@ -376,15 +377,20 @@ __global__ void __launch_bounds__(256) kp_deform_offset_grads16_kernel(
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float dx = geo.x - kpo[r][0], dy = geo.y - kpo[r][1], dz = geo.z - kpo[r][2];
-            const float dist = sqrtf(dx * dx + dy * dy + dz * dz);
-            float slope;
+            const float sq = dx * dx + dy * dy + dz * dz;
+            float coef;
             if (kKind == 0) {
-              slope = dist < sigma ? -1.0f / sigma : 0.0f;
+              // root and quotient as in KpInfluence
+              const float y = __builtin_amdgcn_rsqf(sq), g = sq * y;
+              const float dist = fmaf(fmaf(-g, g, sq), 0.5f * y, g);
+              const float top = -acc[r] * geo.w * (dist < sigma ? neg_inv_sigma : 0.0f);
+              const float q = top * y;
+              coef = sq < 1e-30f ? 0.0f : fmaf(fmaf(-q, dist, top), y, q);
             } else {
-              const float sg = sigma / 3.0f, q = dist / sg;
-              slope = -2.0f * q / sg * expf(-(q * q));
+              const float dist = sqrtf(sq), sg = sigma / 3.0f, q = dist / sg;
+              const float slope = -2.0f * q / sg * expf(-(q * q));
+              coef = dist > 0.0f ? -acc[r] * geo.w * slope / dist : 0.0f;
             }
-            const float coef = dist > 0.0f ? -acc[r] * geo.w * slope / dist : 0.0f;
             sum[r][0] += coef * dx;
             sum[r][1] += coef * dy;
             if (D > 2) sum[r][2] += coef * dz;

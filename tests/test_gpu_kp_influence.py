@@ -1,0 +1,39 @@
+"""The linear influence of a kernel point as the projection kernel evaluates it: points on the
+kernel points and next to them, at the edge of the influence, and small and large ones."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sigma", [0.02, 0.3, 1.0 / 3.0, 0.7, 40.0])
+def test_influence_matches_float64(sigma):
+    from tensorflow_graphics_point_clouds_amd import _lib
+    from tensorflow_graphics_point_clouds_amd._lib import cfloat, cint, i64, ptr, stream
+    gen = torch.Generator(device="cuda").manual_seed(int(100 * sigma))
+    n, kp = 4096, 15
+    kpts = (torch.rand(kp, 3, device="cuda", generator=gen) - 0.5) * sigma
+    # around a kernel point at distances from 0 and 1e-12 up to the influence and a last place beyond
+    near = kpts[torch.randint(0, kp, (n,), device="cuda", generator=gen)]
+    way = torch.nn.functional.normalize(torch.randn(n, 3, device="cuda", generator=gen), dim=1)
+    step = sigma * 10.0 ** (-12.0 * torch.rand(n, 1, device="cuda", generator=gen))
+    step[::5], step[1::5] = 0.0, sigma
+    points = (near + way * step).contiguous()
+    centres = torch.zeros(n, 3, device="cuda")
+    pairs = torch.arange(n, device="cuda", dtype=torch.int32)[:, None].expand(-1, 2).contiguous()
+    ranges = torch.arange(1, n + 1, device="cuda", dtype=torch.int32)
+    ones, feat = torch.ones(3, device="cuda"), torch.zeros(n, 16, device="cuda")
+    feat[:, 0] = 1.0
+    out = torch.empty(n, 16, 16, device="cuda")
+    _lib.call("kp_conv_project", stream(), cint(3), i64(n), ptr(points), cint(16), ptr(feat), i64(n),
+              ptr(centres), i64(n), ptr(pairs), ptr(ranges), ptr(ones), cint(kp), ptr(kpts), cint(0),
+              cfloat(sigma), ptr(None), ptr(out))
+    s = torch.tensor(sigma, dtype=torch.float32).double().item()
+    dist = (points.double()[:, None] - kpts.double()[None]).norm(dim=2)
+    want = (1.0 - dist / s).clamp(min=0.0)
+    # rounded: the difference of the coordinates (half a last place of it), three squares and
+    # two sums, root, quotient, 1 - quotient: below 5 of dist / sigma and one of the result
+    bound = 2.0 ** -24 * (10 * dist / s + 2)
+    assert bool(((out[:, 0, :kp].double() - want).abs() <= bound).all())
+    assert float(out[:, 1:].abs().max()) == 0.0 and float(out[:, 0, kp:].abs().max()) == 0.0
