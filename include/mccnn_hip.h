@@ -203,6 +203,13 @@ int mccnn_unpack_layer_grads(mccnn_stream_t stream, int num_dims, int num_featur
                              const float *dense_grads, const float *kernel_weight_grads,
                              const float *kernel_bias_grads, float *final_grads_out,
                              float *weight_grads_out, float *bias_grads_out);
+/* The same with dense_grads as [f, (c,k)], any number of rows f behind the layer's. */
+int mccnn_unpack_layer_grads_wt(mccnn_stream_t stream, int num_dims, int num_features, int hidden,
+                                int group_features, int first_mlp, int num_mlps,
+                                int padded_features, int padded_hidden, int padded_group,
+                                const float *dense_grads, const float *kernel_weight_grads,
+                                const float *kernel_bias_grads, float *final_grads_out,
+                                float *weight_grads_out, float *bias_grads_out);
 
 /* BuildGridDs: build_grid_ds/cc/ops/build_grid_ds_ops.cpp:27-115.
  * ds_out is int32 [batch_size, num_cells[0], num_cells[1], 2]: (first, last+1)
@@ -735,6 +742,31 @@ int mccnn_kp_conv_project(mccnn_stream_t stream, int num_dims, int64_t num_pts,
                           const float *inv_radii, int num_kernel_points,
                           const float *kernel_points, int kind, float sigma,
                           const int32_t *out_rows, float *out);
+
+/* Feature gradient of a convolution layer with few input channels from the gradient of its
+ * projection (MCConv.py:137-194, KPConv.py:165-232):
+ *   out[j, c] = sum over the pairs (i, j) of sum_k basis_k(ij) projection_grads[i, c, k]
+ * over the transposed pair table (rows grouped by point j, neighbors[., 0] = centre i, ranges
+ * over the points; inv_radii negated so that the offsets keep their sign).  projection_grads
+ * [N_centres, padded_features, 16], num_features <= 16 of which are read; out [N_pts,
+ * num_features], row j at out_rows[j] (NULL: j); accumulate != 0 adds to what out holds.
+ * 16 basis columns, D in {2,3}.  No counterpart among the reference's ops. */
+int mccnn_mc_conv_gather_grads(mccnn_stream_t stream, int num_dims, int64_t num_centres,
+                               const float *centres, int num_features, int padded_features,
+                               const float *projection_grads, int64_t num_pts,
+                               const float *points, int64_t num_neighbors,
+                               const int32_t *neighbors, const int32_t *ranges,
+                               const float *inv_radii, int num_mlps, int activation,
+                               const float *weights, const float *biases, const float *pdf,
+                               const int32_t *out_rows, int accumulate, float *out);
+int mccnn_kp_conv_gather_grads(mccnn_stream_t stream, int num_dims, int64_t num_centres,
+                               const float *centres, int num_features, int padded_features,
+                               const float *projection_grads, int64_t num_pts,
+                               const float *points, int64_t num_neighbors,
+                               const int32_t *neighbors, const int32_t *ranges,
+                               const float *inv_radii, int num_kernel_points,
+                               const float *kernel_points, int kind, float sigma,
+                               const int32_t *out_rows, float *out);
 
 /* Projection of the deformable kernel-point convolution (KPConv.py:317-392):
  * mccnn_kp_conv_project with the kernel points of every centre shifted by its row

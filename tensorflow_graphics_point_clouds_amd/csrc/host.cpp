@@ -696,6 +696,28 @@ Packed pack(const Plan &p, int64_t first, const Tensor &final_weights,
   return out;
 }
 
+// Layers of few input and more output channels take their gradients the other way round
+// (feature_grads.hip): from G = dout W^T, which the kernel MLPs' gradients need anyway, instead of
+// the transposed projection Q [N, F, K] of dout,
+//     dfeat[j, c]  = sum_{i in T(j)} sum_k basis[ij, k] G[i, c, k],
+//     dW[c, k, f]  = sum_i proj[i, c, k] dout[i, f],
+// with the projection computed again.  What is written and read then grows with C, not with F.
+// `wide`: the columns that dout and W are padded to for the products, 0 where this does not apply.
+// KPConv 8 -> 96 on 558 617 points of 12 pairs: 3.16 -> 1.76 ms for the pass (transposed projection,
+// its two products: 2.42 ms; gradient of the projection, gather, projection, product: 1.01); MCConv
+// 16 -> 128 on 8726 of 54: 208 -> 184 us of kernels.  At F = C both sides move as much.
+int64_t narrow_columns(const Plan &p, int64_t n_out) {
+  const int64_t f = p.f(), r = p.c_pad * p.k();
+  if (p.k() != 16 || p.c_pad != 16 || f < 2 * p.c_pad || (p.per != 1 && p.g_pad != p.g) ||
+      n_out * r >= (int64_t)1 << 30)
+    return 0;
+  const int64_t wide = f == 32 ? 32 : (f + 63) / 64 * 64;
+  if (wide != f && p.per != 1) return 0;
+  return mccnn_weight_grad_product_supported((int)wide, (int)r) &&
+                 mccnn_projection_grad_product_supported((int)wide, (int)r)
+             ? wide : 0;
+}
+
 // The product of the feature gradient, q w2.
 Tensor transposed_product(const Tensor &q, const Packed &w, const Tensor &out_rows) {
   if (w.w2t.defined()) return run_product(Product::kTiled, q, Tensor(), w.w2t, out_rows);
@@ -738,6 +760,18 @@ Tensor gather_upstream(const Plan &p, const Tensor &dout, const Tensor &rows, in
   return rows.defined() ? gather_rows(cols, rows, 0, p.f(), p.f()) : cols;
 }
 
+// The same with the columns padded to `wide` (one sub-layer of one kernel MLP, or wide as it is).
+Tensor gather_upstream(const Plan &p, const Tensor &dout, const Tensor &rows, int64_t first,
+                       int64_t wide) {
+  return wide > p.f() || p.g_pad != p.g ? gather_rows(dout, rows, first * p.g, p.g, wide)
+                                        : gather_upstream(p, dout, rows, first);
+}
+
+// W [r, f] with its columns padded to `wide`.
+Tensor widen(const Tensor &w, int64_t wide) {
+  return w.size(1) == wide ? w : gather_rows(w, Tensor(), 0, w.size(1), wide);
+}
+
 Tensor cut_columns(const Tensor &x, int64_t cols) {
   return x.size(1) == cols ? x : x.slice(1, 0, cols).contiguous();
 }
@@ -760,9 +794,12 @@ struct McConv : torch::autograd::Function<McConv> {
     const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
     const int64_t n_out = geo->ranges.size(0);
     std::vector<Tensor> outs;
-    variable_list saved = {feats, kw, kb, final_weights, p.c == p.c_pad ? features : Tensor()};
+    const bool narrow = grads && narrow_columns(p, n_out) > 0;
+    variable_list saved = {feats, kw, kb, final_weights,
+                           p.c == p.c_pad && !narrow ? features : Tensor()};
     for (int64_t first = 0; first < p.mlps; first += p.per) {
-      const Packed w = pack(p, first, final_weights, kw, kb, n_out, feats.size(0), grads, grads);
+      const Packed w = pack(p, first, final_weights, kw, kb, n_out, feats.size(0), grads,
+                            grads && !narrow);
       const Tensor proj = mc_project(p, w, feats, geo->points_in, geo->points_out, geo->table,
                                      geo->ranges, geo->inv_radii, geo->pdf, geo->centre_rows);
       outs.push_back(run_product(w.forward, proj, w.w, w.wt, Tensor(), p.cols()));
@@ -796,15 +833,21 @@ struct McConv : torch::autograd::Function<McConv> {
       dkb = at::empty_like(kb);
     }
     if (want_final) dfinal = at::empty_like(fw);
+    const int64_t wide = narrow_columns(p, n_out);
+    if (wide > 0 && want_feat) dfeat = empty_f32({geo->ranges_t.size(0), p.c}, feats);
     hipStream_t s = current_stream();
     for (int64_t first = 0, i = 0; first < p.mlps; first += p.per, ++i) {
       const Packed w = Packed::saved(saved, 5 + i * Packed::kTensors);
-      const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g || p.per != p.mlps
-                            ? gather_upstream(p, dout, geo->centre_rows, first) : dout;
+      const Tensor up =
+          geo->centre_rows.defined() || p.g_pad != p.g || p.per != p.mlps || wide > p.f()
+              ? (wide > 0 ? gather_upstream(p, dout, geo->centre_rows, first, wide)
+                          : gather_upstream(p, dout, geo->centre_rows, first)) : dout;
       const bool direct = !p.padded() && p.mlps == 1;      // gradients land in the caller's shapes
-      Tensor dkw_pad, dkb_pad, ddense;
+      Tensor dkw_pad, dkb_pad, ddense, dproj;
+      if (want_kernel || (wide > 0 && want_feat))
+        dproj = wide > 0 ? projection_grad_product(up, widen(w.w, wide))
+                         : layer_projection_grad(up, w.w);
       if (want_kernel) {
-        const Tensor dproj = layer_projection_grad(up, w.w);
         Tensor ws = workspace(mccnn_mc_conv_project_grads_workspace_bytes((int)p.dims, (int)k,
                                                                           n_out), feats);
         dkw_pad = direct ? dkw : empty_f32({p.per, p.dims, p.h_pad}, feats);
@@ -817,7 +860,23 @@ struct McConv : torch::autograd::Function<McConv> {
             f32(geo->pdf), f32(dproj), ws.data_ptr(), ws.numel(), nullptr, nullptr, nullptr,
             nullptr, f32(dkw_pad), f32(dkb_pad)));
       }
-      if (want_feat || want_final) {
+      if (wide > 0) {
+        if (want_feat) {
+          Region t("mc_conv_gather_grads", s);
+          check(mccnn_mc_conv_gather_grads(
+              s, (int)p.dims, n_out, f32(geo->points_out), (int)p.c, (int)p.c_pad, f32(dproj),
+              geo->ranges_t.size(0), f32(geo->points_in), geo->table_t.size(0),
+              i32(geo->table_t), i32(geo->ranges_t), f32(geo->neg_inv_radii), (int)p.per,
+              (int)p.act, f32(w.kw), f32(w.kb), f32(geo->pdf_t), i32(geo->point_rows),
+              first > 0, f32(dfeat)));
+        }
+        dproj = Tensor();
+        if (want_final)
+          ddense = weight_grad_product(up, mc_project(p, w, feats, geo->points_in, geo->points_out,
+                                                      geo->table, geo->ranges, geo->inv_radii,
+                                                      geo->pdf, Tensor()));
+      } else if (want_feat || want_final) {
+        dproj = Tensor();
         const bool in_place = features.defined();
         const Tensor q = mc_project(p, w, up, geo->points_out, geo->points_in, geo->table_t,
                                     geo->ranges_t, geo->neg_inv_radii, geo->pdf_t,
@@ -832,7 +891,7 @@ struct McConv : torch::autograd::Function<McConv> {
       if (want_final || (want_kernel && !direct)) {
         const bool kernel = want_kernel && !direct;
         Region t("unpack_layer_grads", s);
-        check(mccnn_unpack_layer_grads(
+        check((wide > 0 ? mccnn_unpack_layer_grads_wt : mccnn_unpack_layer_grads)(
             s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, (int)first, (int)p.per, (int)p.c_pad,
             (int)p.h_pad, (int)p.g_pad, f32(ddense), kernel ? f32(dkw_pad) : nullptr,
             kernel ? f32(dkb_pad) : nullptr, f32(dfinal), kernel ? f32(dkw) : nullptr,
@@ -870,15 +929,17 @@ struct KpConv : torch::autograd::Function<KpConv> {
                         const Tensor &kernel_points, const c10::intrusive_ptr<Geometry> &geo,
                         const Plan &p, const KpShape &kp, bool grads) {
     const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
+    const bool narrow = grads && narrow_columns(p, geo->ranges.size(0)) > 0;
     const Packed w = pack(p, 0, weights, Tensor(), Tensor(), geo->ranges.size(0), feats.size(0),
-                          false, grads);
+                          narrow, grads && !narrow);
     const Tensor proj = kp_project(kp, kernel_points, p.k(), feats, geo->points_in,
                                    geo->points_out, geo->table, geo->ranges, geo->inv_radii,
                                    geo->centre_rows);
     Tensor out = run_product(w.forward, proj, w.w, w.wt, Tensor(), p.cols());
     if (grads) {
-      // what the rows of Q are multiplied with: the features where they are, or padded ones
-      variable_list saved = {p.c == p.c_pad ? features : feats, weights, kernel_points};
+      // what the rows of Q are multiplied with (the features where they are, or padded ones), or
+      // what is projected again
+      variable_list saved = {p.c == p.c_pad && !narrow ? features : feats, weights, kernel_points};
       w.save(saved);
       ctx->save_for_backward(std::move(saved));
       ctx->saved_data["geo"] = c10::IValue::make_capsule(geo);
@@ -900,10 +961,34 @@ struct KpConv : torch::autograd::Function<KpConv> {
         ctx->saved_data["geo"].toCapsule());
     const Packed w = Packed::saved(saved, 3);
     const Tensor dout = grad_out[0].contiguous();
-    const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g
-                          ? gather_upstream(p, dout, geo->centre_rows, 0) : dout;
+    const int64_t n_out = geo->ranges.size(0), wide = narrow_columns(p, n_out);
+    const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g || wide > p.f()
+                          ? (wide > 0 ? gather_upstream(p, dout, geo->centre_rows, 0, wide)
+                                      : gather_upstream(p, dout, geo->centre_rows, 0)) : dout;
     Tensor dfeat, dweights;
-    if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1)) {
+    hipStream_t s = current_stream();
+    if (wide > 0) {
+      if (ctx->needs_input_grad(0)) {
+        const Tensor dproj = projection_grad_product(up, widen(w.w, wide));
+        dfeat = empty_f32({geo->ranges_t.size(0), p.c}, x);
+        Region t("kp_conv_gather_grads", s);
+        check(mccnn_kp_conv_gather_grads(
+            s, (int)p.dims, n_out, f32(geo->points_out), (int)p.c, (int)p.c_pad, f32(dproj),
+            geo->ranges_t.size(0), f32(geo->points_in), geo->table_t.size(0), i32(geo->table_t),
+            i32(geo->ranges_t), f32(geo->neg_inv_radii), (int)kp.num_kp, f32(kernel_points),
+            (int)kp.kind, (float)kp.sigma, i32(geo->point_rows), f32(dfeat)));
+      }
+      if (ctx->needs_input_grad(1)) {
+        const Tensor ddense = weight_grad_product(
+            up, kp_project(kp, kernel_points, p.k(), x, geo->points_in, geo->points_out,
+                           geo->table, geo->ranges, geo->inv_radii, Tensor()));
+        dweights = at::empty_like(weights);
+        Region t("unpack_layer_grads", s);
+        check(mccnn_unpack_layer_grads_wt(s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, 0, 1,
+                                          (int)p.c_pad, (int)p.h_pad, (int)p.g_pad, f32(ddense),
+                                          nullptr, nullptr, f32(dweights), nullptr, nullptr));
+      }
+    } else if (ctx->needs_input_grad(0) || ctx->needs_input_grad(1)) {
       const bool in_place = p.c == p.c_pad;
       const Tensor q = kp_project(kp, kernel_points, p.k(), up, geo->points_out, geo->points_in,
                                   geo->table_t, geo->ranges_t, geo->neg_inv_radii,
@@ -913,7 +998,6 @@ struct KpConv : torch::autograd::Function<KpConv> {
       if (ctx->needs_input_grad(1)) {
         const Tensor ddense = weight_grad_product(x, q);
         dweights = at::empty_like(weights);
-        hipStream_t s = current_stream();
         Region t("unpack_layer_grads", s);
         check(mccnn_unpack_layer_grads(s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, 0, 1,
                                        (int)p.c_pad, (int)p.h_pad, (int)p.g_pad, f32(ddense),

@@ -85,18 +85,17 @@ __global__ void __launch_bounds__(256) pack_layer_weights_kernel(
 }
 
 // The gradients back in the caller's shapes: final-weight gradient from the product's
-// [Cp, (f, k)] result, kernel-MLP gradients from [mlps, D, Hp] and [mlps * Hp].
+// [Cp, (f, k)] or [f, (c, k)] result (element (c, f, k) at c c_stride + f f_stride + k), kernel-MLP gradients from [mlps, D, Hp] and [mlps * Hp].
 __global__ void __launch_bounds__(256) unpack_layer_grads_kernel(
-    LayerShapeArgs a, int D, const float *__restrict__ ddense, const float *__restrict__ dkw_src,
-    const float *__restrict__ dkb_src, float *__restrict__ dfinal, float *__restrict__ dkw,
+    LayerShapeArgs a, int D, int c_stride, int f_stride, const float *__restrict__ ddense,
+    const float *__restrict__ dkw_src, const float *__restrict__ dkb_src, float *__restrict__ dfinal, float *__restrict__ dkw,
     float *__restrict__ dkb) {
-  const int K = a.mlps * a.Hp, F = a.mlps * a.Gp;
   const int per = a.C * a.H * a.G, size = a.mlps * per;
   if (dfinal)
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < size; t += gridDim.x * blockDim.x) {
       const int g = t % a.G, h = t / a.G % a.H, c = t / a.G / a.H % a.C, m = t / per;
       dfinal[(int64_t)a.first * per + t] =
-          ddense[((int64_t)c * F + m * a.Gp + g) * K + m * a.Hp + h];
+          ddense[(int64_t)c * c_stride + (int64_t)(m * a.Gp + g) * f_stride + m * a.Hp + h];
     }
   if (blockIdx.x == 0 && dkw) {
     for (int t = threadIdx.x; t < a.mlps * D * a.H; t += blockDim.x) {
@@ -176,6 +175,28 @@ extern "C" int mccnn_pack_layer_weights(mccnn_stream_t stream, int num_dims, int
   return MCCNN_OK;
 }
 
+static int unpack_layer_grads(mccnn_stream_t stream, int num_dims, const LayerShapeArgs &a,
+                              bool by_output, const float *dense_grads,
+                              const float *kernel_weight_grads, const float *kernel_bias_grads,
+                              float *final_grads_out, float *weight_grads_out,
+                              float *bias_grads_out) {
+  int rc = check_shape("unpack_layer_grads", a);
+  if (rc != MCCNN_OK) return rc;
+  MCCNN_REQUIRE((!final_grads_out || dense_grads) &&
+                    (!weight_grads_out || (kernel_weight_grads && kernel_bias_grads &&
+                                           bias_grads_out)),
+                "unpack_layer_grads received a null tensor");
+  const int64_t size = (int64_t)a.mlps * a.C * a.H * a.G;
+  const unsigned grid = blocks_for(size > (1 << 20) ? (1 << 20) : size, 256);
+  const int K = a.mlps * a.Hp, F = a.mlps * a.Gp;
+  hipLaunchKernelGGL(unpack_layer_grads_kernel, dim3(grid), dim3(256), 0, as_stream(stream), a,
+                     num_dims, by_output ? K : F * K, by_output ? a.Cp * K : K, dense_grads,
+                     kernel_weight_grads, kernel_bias_grads, final_grads_out, weight_grads_out,
+                     bias_grads_out);
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
 extern "C" int mccnn_unpack_layer_grads(mccnn_stream_t stream, int num_dims, int num_features,
                                         int hidden, int group_features, int first_mlp,
                                         int num_mlps, int padded_features, int padded_hidden,
@@ -185,17 +206,19 @@ extern "C" int mccnn_unpack_layer_grads(mccnn_stream_t stream, int num_dims, int
                                         float *weight_grads_out, float *bias_grads_out) {
   const LayerShapeArgs a = {num_features, hidden, group_features, first_mlp, num_mlps,
                             padded_features, padded_hidden, padded_group};
-  int rc = check_shape("unpack_layer_grads", a);
-  if (rc != MCCNN_OK) return rc;
-  MCCNN_REQUIRE((!final_grads_out || dense_grads) &&
-                    (!weight_grads_out || (kernel_weight_grads && kernel_bias_grads &&
-                                           bias_grads_out)),
-                "unpack_layer_grads received a null tensor");
-  const int64_t size = (int64_t)a.mlps * a.C * a.H * a.G;
-  const unsigned grid = blocks_for(size > (1 << 20) ? (1 << 20) : size, 256);
-  hipLaunchKernelGGL(unpack_layer_grads_kernel, dim3(grid), dim3(256), 0, as_stream(stream), a,
-                     num_dims, dense_grads, kernel_weight_grads, kernel_bias_grads,
-                     final_grads_out, weight_grads_out, bias_grads_out);
-  MCCNN_LAUNCH_CHECK();
-  return MCCNN_OK;
+  return unpack_layer_grads(stream, num_dims, a, false, dense_grads, kernel_weight_grads,
+                            kernel_bias_grads, final_grads_out, weight_grads_out, bias_grads_out);
+}
+
+extern "C" int mccnn_unpack_layer_grads_wt(mccnn_stream_t stream, int num_dims, int num_features,
+                                           int hidden, int group_features, int first_mlp,
+                                           int num_mlps, int padded_features, int padded_hidden,
+                                           int padded_group, const float *dense_grads,
+                                           const float *kernel_weight_grads,
+                                           const float *kernel_bias_grads, float *final_grads_out,
+                                           float *weight_grads_out, float *bias_grads_out) {
+  const LayerShapeArgs a = {num_features, hidden, group_features, first_mlp, num_mlps,
+                            padded_features, padded_hidden, padded_group};
+  return unpack_layer_grads(stream, num_dims, a, true, dense_grads, kernel_weight_grads,
+                            kernel_bias_grads, final_grads_out, weight_grads_out, bias_grads_out);
 }

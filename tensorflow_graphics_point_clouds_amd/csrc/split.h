@@ -68,6 +68,21 @@ __device__ __forceinline__ v16f mma_split(const Split8 &a, const Split8 &b, v16f
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0], b.p[0], acc, 0, 0, 0);
 }
 
+// The same in two parts, for accumulators that start at zero: the five small products of all steps
+// first, then the large ones, so that the sum is rounded at its own size once per step and not six
+// times (the feature gradient of a 16 -> 128 layer, which is summed from such products: off by
+// 2.3e-7 of the exact sums with one loop, 1.45e-7 with two, at equal speed).
+__device__ __forceinline__ v16f mma_split_small(const Split8 &a, const Split8 &b, v16f acc) {
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[2], b.p[0], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0], b.p[2], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[1], b.p[1], acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[1], b.p[0], acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.p[0], b.p[1], acc, 0, 0, 0);
+}
+__device__ __forceinline__ v16f mma_large(const v8bf &a, const v8bf &b, v16f acc) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+}
+
 // Whether the dense products of the layers run on the bf16 pipe (default) or keep the
 // float32 matrix instructions (mccnn_set_split_products(0), or MCCNN_DENSE_FP32=1 in the
 // environment of the process).

@@ -76,12 +76,17 @@ __global__ void __launch_bounds__(256, 2) nt_split_kernel(int64_t n, int R,
     for (int ct = 0; ct < kCT; ++ct)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[ct][i] = 0.0f;
+    Split8 as[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const Split8 as = split8(a[2 * ks], a[2 * ks + 1]);
+      as[ks] = split8(a[2 * ks], a[2 * ks + 1]);
 #pragma unroll
-      for (int ct = 0; ct < kCT; ++ct) acc[ct] = mma_split(as, b[ct][ks], acc[ct]);
+      for (int ct = 0; ct < kCT; ++ct) acc[ct] = mma_split_small(as[ks], b[ct][ks], acc[ct]);
     }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int ct = 0; ct < kCT; ++ct) acc[ct] = mma_large(as[ks].p[0], b[ct][ks].p[0], acc[ct]);
     // acc[ct][i]: point 32 t + (i / 4) * 8 + 4 h + i % 4, column col0 + 32 ct + p
     constexpr int kPieces = kPairCols / 4;            // 16-byte pieces per row
     constexpr int kRowsPer = kWave / kPieces;         // rows per store instruction
@@ -203,7 +208,13 @@ __global__ void __launch_bounds__(256, 2) nt_split_shared_kernel(int64_t n, int 
 #pragma unroll
       for (int q = 0; q < 3; ++q) a.p[q] = a_lds[cur][((q * KS + ks) * 2 + h) * kLdA + p];
 #pragma unroll
-      for (int ct = 0; ct < kCT; ++ct) acc[ct] = mma_split(a, b[ct][ks], acc[ct]);
+      for (int ct = 0; ct < kCT; ++ct) acc[ct] = mma_split_small(a, b[ct][ks], acc[ct]);
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const v8bf a = a_lds[cur][(ks * 2 + h) * kLdA + p];
+#pragma unroll
+      for (int ct = 0; ct < kCT; ++ct) acc[ct] = mma_large(a, b[ct][ks].p[0], acc[ct]);
     }
     // acc[ct][i]: point 32 t + (i / 4) * 8 + 4 h + i % 4, column wcol + 32 ct + p of the block
 #pragma unroll

@@ -1,0 +1,67 @@
+"""Gradients of layers with few input and more output channels, which go through the gradient of the
+projection: channel counts at the edges of the gathered 4 / 8 / 16, output columns that are padded,
+several kernel MLPs, points without neighbours, runs of every length."""
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("layer", ["mc", "mc_two", "mc_2d", "kp"])
+@pytest.mark.parametrize("c,f", [(1, 32), (3, 64), (4, 48), (5, 96), (8, 128), (9, 112), (16, 32),
+                                 (16, 128)])
+def test_gradients_of_narrow_layers(layer, c, f):
+    from tensorflow_graphics_point_clouds_amd import layers, pc
+    gen = torch.Generator(device="cuda").manual_seed(100 * c + f)
+    rand = lambda *shape: torch.rand(shape, device="cuda", generator=gen)
+    d = 2 if layer == "mc_2d" else 3
+    n_in, n_out, r = 700, 431, 0.16
+    pts, ctr = rand(n_in, d), rand(n_out, d)
+    pts[-20:] += 3.0                                        # points that no centre reaches
+    ids = torch.arange(n_in, device="cuda").mul(2).div(n_in, rounding_mode="floor").int()
+    cids = torch.arange(n_out, device="cuda").mul(2).div(n_out, rounding_mode="floor").int()
+    cin, cout = pc.PointCloud(pts, ids, 2), pc.PointCloud(ctr, cids, 2)
+    nbh = pc.Neighborhood(pc.Grid(cin, r), r, cout)
+    if layer == "kp":
+        conv = layers.KPConv(c, f, num_kernel_points=15, num_dims=3, seed=c)
+    else:
+        mlps = 2 if layer == "mc_two" else 1
+        conv = layers.MCConv(c, f, d, num_mlps=mlps, mlp_size=[16], non_linearity_type="elu", seed=c)
+        with torch.no_grad():
+            conv.biases.add_(rand(*conv.biases.shape) - 0.5)
+    feats = (rand(n_in, c) - 0.5).requires_grad_(True)
+    up = rand(n_out, f) - 0.5
+    out = conv(feats, cin, cout, r, neighborhood=nbh)
+    out.backward(up)
+
+    pairs = nbh._original_neigh_ids.long()
+    delta = (pts.double()[pairs[:, 0]] - ctr.double()[pairs[:, 1]]) / r
+    if layer == "kp":            # linear influence of sigma = 1 radius (KPConv.py:193-213)
+        dist = (delta[:, None, :] - conv._kernel_points.double()[None]).norm(dim=2)
+        basis, finals = [(1.0 - dist).clamp(min=0.0)], [conv.weights.double()]
+    else:
+        pdf = nbh.get_pdf().double().reshape(-1, 1)
+        basis = [torch.nn.functional.elu(delta @ w + b) / pdf
+                 for w, b in zip(conv.weights.double(), conv.biases.double())]
+        finals = list(conv.final_weights.double())
+    g = f // len(finals)
+    dfeat = torch.zeros(n_in, c, dtype=torch.float64, device="cuda")
+    mag = torch.zeros_like(dfeat)
+    for m, (b, w) in enumerate(zip(basis, finals)):
+        k = b.shape[1]
+        dproj = up[:, m * g:(m + 1) * g].double() @ w.detach().t()
+        big = up[:, m * g:(m + 1) * g].double().abs() @ w.detach().t().abs()
+        part = lambda basis, grad: (basis[:, None, :] * grad.reshape(n_out, c, k)[pairs[:, 1]]).sum(2)
+        dfeat.index_add_(0, pairs[:, 0], part(b.detach(), dproj))
+        mag.index_add_(0, pairs[:, 0], part(b.detach().abs(), big))
+        proj = torch.zeros(n_out, c, k, dtype=torch.float64, device="cuda").index_add(
+            0, pairs[:, 1], feats.detach().double()[pairs[:, 0]][:, :, None] * b.detach()[:, None, :])
+        dw = proj.reshape(n_out, c * k).t() @ up[:, m * g:(m + 1) * g].double()
+        got = conv.weights.grad if layer == "kp" else conv.final_weights.grad[m]
+        assert float((got.double().reshape(dw.shape) - dw).norm()) <= 2e-6 * float(dw.norm())
+    # f products per entry of G, 16 basis values and some hundred pairs per sum, a float32 density or
+    # correlation (a few roundings) in each
+    assert bool(((feats.grad.double() - dfeat).abs() <= 400 * 2.0 ** -24 * mag).all())
+    assert feats.grad.shape == (n_in, c) and float(feats.grad[-20:].abs().max()) == 0.0
+
