@@ -181,9 +181,7 @@ __global__ void __launch_bounds__(256) kp_conv_gather_grads_kernel(
 
 // As for the projection (mc_conv.hip): shorter runs on small inputs.
 static int gather_run_len(int64_t n) {
-  int run = kGatherRun;
-  while (run > 1 && n < run * (int64_t)16000) run >>= 1;
-  return run;
+  return n >= 160000 ? kGatherRun : n >= 64000 ? 4 : n >= 20000 ? 2 : 1;
 }
 
 static int check_gather_args(const char *op, int num_dims, int num_features, int padded_features,

@@ -28,21 +28,17 @@ constexpr int kGradRun = 8;        // the same in the gradient kernels
 // 102 / 86 / 88 / - on 70 k, 182 / 176 on 140 k, 430 / 430 on 300 k.
 static int project_run_len(int64_t num_samples, int chunks) {
   const int64_t items = num_samples * chunks;
-  if (items >= (int64_t)kProjRun * 20000) return kProjRun;
-  int run = kProjRun / 2;
-  while (run > 1 && items < run * (int64_t)16000) run >>= 1;
-  return run;
+  return items >= 160000 ? kProjRun : items >= 64000 ? 4 : items >= 20000 ? 2 : 1;
 }
 
 // The same for the gradient kernels, whose blocks add a partial sum each: never fewer than two
 // centres, and lists of fewer than 16 pairs keep longer runs.  64 channels, runs of 8 / 4 / 2 / 1:
 // 25 / 17 / 13 / 14 us on 4 k centres of 19 pairs, 87 / 55 / 47 / 45 on 16 k of 31,
-// 74 / 66 / 66 / 77 on 33 k of 30; 43 / 43 / 47 / 58 on 33 k of 8.
+// 74 / 66 / 66 / 77 on 33 k of 30, 149 / 136 / 147 / - on 70 k of 34; 43 / 43 / 47 / 58 on 33 k of 8.
 static int grad_run_len(int64_t num_samples, int64_t num_neighbors) {
-  const int64_t waves = num_neighbors >= 16 * num_samples ? 8000 : 4000;
-  int run = kGradRun;
-  while (run > 2 && num_samples < run * waves) run >>= 1;
-  return run;
+  if (num_neighbors < 16 * num_samples)
+    return num_samples >= 32000 ? kGradRun : num_samples >= 16000 ? 4 : 2;
+  return num_samples >= 128000 ? kGradRun : num_samples >= 24000 ? 4 : 2;
 }
 
 // One wavefront per (run of up to kProjRun consecutive centres, chunk of 16*kCPL channels):

@@ -16,11 +16,11 @@ def _table(n, mean, gen):
     return torch.stack([ids, centres], dim=1).int().contiguous(), ranges
 
 
-# runs of 1 | 2 | 4 | 8 centres of the projection change at 32 000, 64 000 and 160 000 centres (16 to
-# 128 channels are one chunk), those of the gradients at 16 000 / 32 000 (short lists) and at 32 000 /
-# 64 000; 131 073 centres in runs of 8 are more than 4096 blocks
+# runs of 1 | 2 | 4 | 8 centres of the projection change at 20 000, 64 000 and 160 000 centres (16 to
+# 128 channels are one chunk), those of the gradients at 16 000 / 32 000 (short lists) and at 24 000 /
+# 128 000; 131 073 centres in runs of 8 are more than 4096 blocks
 @pytest.mark.parametrize("n,mean,c", [(1, 20, 16), (9, 3, 64), (15999, 3, 16), (16003, 20, 16),
-                                      (31999, 20, 16), (32001, 3, 16), (64001, 20, 16),
+                                      (20001, 20, 16), (24001, 20, 16), (32001, 3, 16), (64001, 20, 16),
                                       (160001, 3, 16), (131073, 17, 16), (16003, 3, 128)])
 def test_projection_and_gradients_at_changes_of_the_run_length(n, mean, c):
     from tensorflow_graphics_point_clouds_amd import layers, tfg_custom_ops
