@@ -164,12 +164,30 @@ struct Bounds {
       hi[d] = fmaxf(hi[d], p[d]);
     }
   }
-  // The wavefront's bounds into mn[0..D), mx[0..D) (encoded), then start over.
+  // The wavefront's bounds into mn[0..D), mx[0..D) (encoded), then start over.  Inside a row of
+  // sixteen lanes by rotations of the row (vector instructions), between the four rows through the
+  // lane exchange, whose latency six steps in a row would pay six times.
+  template <int kCtrl>
+  static __device__ __forceinline__ float rotated(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kCtrl, 0xf, 0xf, false));
+  }
   __device__ __forceinline__ void flush(unsigned *mn, unsigned *mx) {
+    constexpr int kRor = 0x120;                    // row_ror:n is 0x120 + n
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      lo[d] = fminf(lo[d], rotated<kRor + 8>(lo[d]));
+      hi[d] = fmaxf(hi[d], rotated<kRor + 8>(hi[d]));
+      lo[d] = fminf(lo[d], rotated<kRor + 4>(lo[d]));
+      hi[d] = fmaxf(hi[d], rotated<kRor + 4>(hi[d]));
+      lo[d] = fminf(lo[d], rotated<kRor + 2>(lo[d]));
+      hi[d] = fmaxf(hi[d], rotated<kRor + 2>(hi[d]));
+      lo[d] = fminf(lo[d], rotated<kRor + 1>(lo[d]));
+      hi[d] = fmaxf(hi[d], rotated<kRor + 1>(hi[d]));
+    }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
 #pragma unroll
-      for (int off = kWave / 2; off > 0; off >>= 1) {
+      for (int off = kWave / 2; off >= 16; off >>= 1) {
         lo[d] = fminf(lo[d], __shfl_xor(lo[d], off, kWave));
         hi[d] = fmaxf(hi[d], __shfl_xor(hi[d], off, kWave));
       }
@@ -191,6 +209,10 @@ template <int D, class Flush, class Direct>
 __device__ __forceinline__ void add_points(bool live, int b, const float *p, Bounds<D> &box,
                                            int &cur, Flush &&flush, Direct &&direct) {
   uint64_t todo = __ballot(live);
+  if (todo == __ballot(live && b == cur)) {       // the usual case: all of the cloud at hand
+    if (live) box.add(p);
+    return;
+  }
   for (int runs = 0; todo != 0; ++runs) {
     if (runs == 4) {
       if ((todo >> lane_id()) & 1) direct(b, p);
@@ -413,8 +435,7 @@ __global__ void __launch_bounds__(kSmallThreads) grid_small_kernel(
   int first = small_first(n), last = small_last(n);
   const int cloud = kByCloud ? blockIdx.x : 0;
   if (kByCloud && t == 0) s.lo = s.hi = s.up = s.down = 0;
-  auto find_cloud = [&](int i, int b) {  // point i is of cloud b
-    const int before = i > 0 ? bids[i - 1] : b;
+  auto find_cloud = [&](int i, int b, int before) {  // point i is of cloud b, the one before it
     if (before < b) s.up = 1;
     if (before > b) s.down = 1;
     if (b == cloud && before != b) s.lo = i;
@@ -426,7 +447,21 @@ __global__ void __launch_bounds__(kSmallThreads) grid_small_kernel(
   if (kOrderOnly) {
     if (kByCloud) {
       __syncthreads();
-      for (int i = first + lane; i < last; i += kWave) find_cloud(i, bids[i]);
+      constexpr int kAhead = 4;
+      for (int base = first; base < last; base += kAhead * kWave) {
+        int b[kAhead], before[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          const int i = base + u * kWave + lane < last ? base + u * kWave + lane : last - 1;
+          b[u] = bids[i];
+          before[u] = bids[i > 0 ? i - 1 : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+          if (__any(b[u] != before[u]) || base + (u + 1) * kWave >= n)
+            if (base + u * kWave + lane < last)
+              find_cloud(base + u * kWave + lane, b[u], before[u]);
+      }
       __syncthreads();
     }
 #pragma unroll
@@ -443,23 +478,39 @@ __global__ void __launch_bounds__(kSmallThreads) grid_small_kernel(
     __syncthreads();
     Bounds<D> box;
     int cur = -1;
-    for (int base = first; base < last; base += kWave) {
-      const int i = base + lane;
-      const bool live = i < last;
-      const int b = live ? bids[i] : -1;
-      float p[D];
+    // kAhead times 64 points in flight: every block reads all points, and iteration by iteration
+    // that is a chain of up to sixteen waits (16 clouds of 8659 points in all: 20 -> 14 us, 2 x 1024
+    // 15 -> 12)
+    constexpr int kAhead = 4;
+    for (int base = first; base < last; base += kAhead * kWave) {
+      int b[kAhead], before[kAhead];
+      float p[kAhead][D];
 #pragma unroll
-      for (int d = 0; d < D; ++d) p[d] = live ? pts[(int64_t)i * D + d] : 0.0f;
-      if (kByCloud && live) find_cloud(i, b);
-      add_points<D>(live, b, p, box, cur,
-                    [&](int b, Bounds<D> &box) { box.flush(s.mn + b * D, s.mx + b * D); },
-                    [&](int b, const float *p) {
+      for (int u = 0; u < kAhead; ++u) {            // past the end: the last point again
+        const int i = base + u * kWave + lane < last ? base + u * kWave + lane : last - 1;
+        b[u] = bids[i];
+        if (kByCloud) before[u] = bids[i > 0 ? i - 1 : 0];
 #pragma unroll
-                      for (int d = 0; d < D; ++d) {
-                        atomicMin(&s.mn[b * D + d], enc_float(p[d]));
-                        atomicMax(&s.mx[b * D + d], enc_float(p[d]));
-                      }
-                    });
+        for (int d = 0; d < D; ++d) p[u][d] = pts[(int64_t)i * D + d];
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int i = base + u * kWave + lane;
+        const bool live = i < last;
+        // (nothing to see where the 64 points and the one before them are of one cloud)
+        if (kByCloud && (__any(b[u] != before[u]) || base + (u + 1) * kWave >= n)) {
+          if (live) find_cloud(i, b[u], before[u]);
+        }
+        add_points<D>(live, b[u], p[u], box, cur,
+                      [&](int b, Bounds<D> &box) { box.flush(s.mn + b * D, s.mx + b * D); },
+                      [&](int b, const float *p) {
+#pragma unroll
+                        for (int d = 0; d < D; ++d) {
+                          atomicMin(&s.mn[b * D + d], enc_float(p[d]));
+                          atomicMax(&s.mx[b * D + d], enc_float(p[d]));
+                        }
+                      });
+      }
     }
     if (cur >= 0) box.flush(s.mn + cur * D, s.mx + cur * D);
     __syncthreads();
@@ -504,25 +555,22 @@ __global__ void __launch_bounds__(kSmallThreads) grid_small_kernel(
   const int64_t below = kByCloud && count < n ? (int64_t)cells * cloud : 0;  // keys of the clouds before
   if (count == n) cells *= (uint64_t)(batch > 0 ? batch : 1);
   const int bits = cells > 1 ? 64 - __clzll((long long)(cells - 1)) : 1;
-  for (int r = 0; r < kSmallRounds; ++r) {
-    const int i = first + r * kWave + lane;
-    if (i < last) {
-      const int b = bids[i];
-      float p[D], m[D];
+  for (int i = first + lane; i < last; i += kWave) {
+    const int b = bids[i];
+    float p[D], m[D];
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        p[d] = pts[(int64_t)i * D + d];
-        m[d] = kOrderOnly ? g.smin[(int64_t)b * D + d] : s.smin[b * D + d];
-      }
-      int c[D];
-      cell_of_point<D>(p, m, ic, shape, c);
-      g.keys[i] = key_of_cell<D>(c, shape, b);
+    for (int d = 0; d < D; ++d) {
+      p[d] = pts[(int64_t)i * D + d];
+      m[d] = kOrderOnly ? g.smin[(int64_t)b * D + d] : s.smin[b * D + d];
     }
+    int c[D];
+    cell_of_point<D>(p, m, ic, shape, c);
+    g.keys[i] = key_of_cell<D>(c, shape, b);
   }
   __threadfence_block();
   __syncthreads();                       // the keys are in memory for the whole block
   int item[kSmallRounds];
-  small_sort(count, bits, g.keys + begin, below, item, s.sort);
+  small_sort_any(count, bits, g.keys + begin, below, item, s.sort);
 #pragma unroll
   for (int r = 0; r < kSmallRounds; ++r) {
     if (first + r * kWave + lane < last) {

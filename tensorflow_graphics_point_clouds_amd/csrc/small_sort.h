@@ -44,7 +44,9 @@ __device__ __forceinline__ int small_last(int n) {
 
 // item[r] of a lane becomes the index of the key with rank first + 64 r + lane.  `keys` must be
 // visible to the whole block (a barrier since they were written); the lowest `bits` of keys less
-// `below` tell them apart.
+// `below` tell them apart.  kRounds: n <= 1024 kRounds (the loops over rounds are unrolled and
+// cost their instructions whether a round has items or not).
+template <int kRounds>
 __device__ __forceinline__ void small_sort(int n, int bits, const int64_t *keys, int64_t below,
                                            int *item, SmallSortLds &s) {
   const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
@@ -53,19 +55,19 @@ __device__ __forceinline__ void small_sort(int n, int bits, const int64_t *keys,
   const int width = (bits + passes - 1) / passes;
   const int radix = 1 << width;
 #pragma unroll
-  for (int r = 0; r < kSmallRounds; ++r) item[r] = first + r * kWave + lane;
+  for (int r = 0; r < kRounds; ++r) item[r] = first + r * kWave + lane;
   for (int p = 0; p < passes; ++p) {
     const int shift = p * width;
-    int digit[kSmallRounds];
+    int digit[kRounds];
 #pragma unroll
-    for (int r = 0; r < kSmallRounds; ++r)
+    for (int r = 0; r < kRounds; ++r)
       digit[r] = first + r * kWave + lane < last
                      ? (int)((~(uint64_t)(keys[item[r]] - below) >> shift) & (uint64_t)(radix - 1)) : 0;
     for (int i = t; i < kSmallWaves * radix; i += kSmallThreads) s.start[i] = 0;
     __syncthreads();
     int *mine = s.start + wave * radix;
 #pragma unroll
-    for (int r = 0; r < kSmallRounds; ++r)
+    for (int r = 0; r < kRounds; ++r)
       if (first + r * kWave + lane < last) atomicAdd(&mine[digit[r]], 1);
     __syncthreads();
     // thread t scans digit t over the wavefronts, the block scans the digits
@@ -86,7 +88,7 @@ __device__ __forceinline__ void small_sort(int n, int bits, const int64_t *keys,
       }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSmallRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
       __builtin_amdgcn_sched_barrier(0);                  // rounds one after another: few registers
       if (first + r * kWave < last) {                     // uniform in the wavefront
         const bool live = first + r * kWave + lane < last;
@@ -107,11 +109,18 @@ __device__ __forceinline__ void small_sort(int n, int bits, const int64_t *keys,
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kSmallRounds; ++r) {
+    for (int r = 0; r < kRounds; ++r) {
       const int i = first + r * kWave + lane;
       if (i < last) item[r] = s.exchange[i];
     }
   }
+}
+
+__device__ __forceinline__ void small_sort_any(int n, int bits, const int64_t *keys, int64_t below,
+                                               int *item, SmallSortLds &s) {
+  if (n <= kSmallThreads) small_sort<1>(n, bits, keys, below, item, s);
+  else if (n <= 4 * kSmallThreads) small_sort<4>(n, bits, keys, below, item, s);
+  else small_sort<kSmallRounds>(n, bits, keys, below, item, s);
 }
 
 }  // namespace mccnn

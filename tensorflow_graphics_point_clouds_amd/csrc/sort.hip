@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(kSmallThreads) sort_small_kernel(
   SmallSortLds &s = *reinterpret_cast<SmallSortLds *>(lds_raw);
   const int first = small_first(n), last = small_last(n), lane = lane_id();
   int item[kSmallRounds];
-  small_sort(n, bits, keys, 0, item, s);
+  small_sort_any(n, bits, keys, 0, item, s);
 #pragma unroll
   for (int r = 0; r < kSmallRounds; ++r) {
     const int i = first + r * kWave + lane;
