@@ -141,6 +141,14 @@ int mccnn_order_centres(mccnn_stream_t stream, int64_t num_samples, int num_dims
                         const float *inv_cell_sizes, int key_bits, void *workspace,
                         size_t workspace_bytes, int32_t *order_out, float *points_out,
                         int32_t *batch_ids_out);
+/* The same with the sorted keys (NULL to skip), for a search among the centres. */
+int mccnn_order_centres_keys(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                             const float *samples, const int32_t *sample_batch_ids,
+                             int batch_size, const int32_t *num_cells,
+                             const float *scaled_aabb_min, const float *inv_cell_sizes,
+                             int key_bits, void *workspace, size_t workspace_bytes,
+                             int32_t *order_out, float *points_out, int32_t *batch_ids_out,
+                             int64_t *sorted_keys_out);
 int mccnn_invert_order(mccnn_stream_t stream, int64_t count, const int32_t *order,
                        int32_t *inverse_out);
 
@@ -304,6 +312,15 @@ int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, int num_dims,
                        const float *inv_cell_sizes, const float *inv_radii, int max_neighs,
                        void *workspace, size_t workspace_bytes, int32_t *ranges_out,
                        int64_t *result_pinned);
+/* A whole search whose number of pairs is known beforehand, without a host round trip: both halves
+ * of the search without a limit per centre.  No more than num_neighbors pairs are written. */
+int mccnn_search_known(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                       const float *samples, const int32_t *sample_batch_ids, int64_t num_pts,
+                       const float *points, const int64_t *point_keys, const int32_t *grid_ds,
+                       const int32_t *num_cells, const float *scaled_aabb_min,
+                       const float *inv_cell_sizes, const float *inv_radii, void *workspace,
+                       size_t workspace_bytes, int64_t num_neighbors, int32_t *ranges_out,
+                       int32_t *neighbors_out);
 
 /* Kernel density of a grid's own (sorted) points straight from the grid: mccnn_compute_pdf on the
  * untruncated neighbourhood of the points among themselves, without its pair table.  grid_ds may

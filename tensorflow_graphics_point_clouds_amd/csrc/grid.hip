@@ -576,7 +576,7 @@ __global__ void __launch_bounds__(kSmallThreads) grid_small_kernel(
     if (first + r * kWave + lane < last) {
       const int from = begin + item[r], i = dest + (first - begin) + r * kWave + lane;
       g.sorted_idx[i] = from;
-      if (!kOrderOnly) g.sorted_keys[i] = g.keys[from];
+      if (!kOrderOnly || g.sorted_keys) g.sorted_keys[i] = g.keys[from];
 #pragma unroll
       for (int d = 0; d < D; ++d) g.sorted_pts[(int64_t)i * D + d] = pts[(int64_t)from * D + d];
       g.sorted_bids[i] = bids[from];
@@ -971,6 +971,20 @@ extern "C" int mccnn_order_centres(mccnn_stream_t stream, int64_t num_samples, i
                                    int key_bits, void *workspace, size_t workspace_bytes,
                                    int32_t *order_out, float *points_out,
                                    int32_t *batch_ids_out) {
+  return mccnn_order_centres_keys(stream, num_samples, num_dims, samples, sample_batch_ids,
+                                  batch_size, num_cells, scaled_aabb_min, inv_cell_sizes, key_bits,
+                                  workspace, workspace_bytes, order_out, points_out, batch_ids_out,
+                                  nullptr);
+}
+
+extern "C" int mccnn_order_centres_keys(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                                        const float *samples, const int32_t *sample_batch_ids,
+                                        int batch_size, const int32_t *num_cells,
+                                        const float *scaled_aabb_min,
+                                        const float *inv_cell_sizes, int key_bits,
+                                        void *workspace, size_t workspace_bytes,
+                                        int32_t *order_out, float *points_out,
+                                        int32_t *batch_ids_out, int64_t *sorted_keys_out) {
   MCCNN_REQUIRE(valid_dims(num_dims), "order_centres expects a valid number of dimensions");
   MCCNN_REQUIRE(num_samples >= 0 && num_samples < ((int64_t)1 << 31) && batch_size > 0,
                 "order_centres expects 0 <= num_samples < 2^31 and a positive batch size");
@@ -983,8 +997,8 @@ extern "C" int mccnn_order_centres(mccnn_stream_t stream, int64_t num_samples, i
   hipStream_t s = as_stream(stream);
   if (num_samples <= kSmallMax) {
     const GridArrays g = {nullptr, nullptr, (int *)num_cells, (float *)scaled_aabb_min,
-                          (float *)inv_cell_sizes, (int64_t *)workspace, nullptr, order_out,
-                          points_out, batch_ids_out};
+                          (float *)inv_cell_sizes, (int64_t *)workspace, sorted_keys_out,
+                          order_out, points_out, batch_ids_out};
     int rc = MCCNN_OK;
     MCCNN_DIM_SWITCH(num_dims, rc = (launch_small<D, true>(s, num_samples, batch_size, samples,
                                                            sample_batch_ids, nullptr, g)));
@@ -992,6 +1006,7 @@ extern "C" int mccnn_order_centres(mccnn_stream_t stream, int64_t num_samples, i
   }
   char *p = (char *)workspace;
   int64_t *keys = (int64_t *)p, *sorted = (int64_t *)(p + align256(8 * (size_t)num_samples));
+  if (sorted_keys_out) sorted = sorted_keys_out;
   void *ws = p + 2 * align256(8 * (size_t)num_samples);
   int rc = mccnn_compute_keys(stream, num_samples, num_dims, samples, num_samples,
                               sample_batch_ids, batch_size, num_dims, scaled_aabb_min, num_dims,

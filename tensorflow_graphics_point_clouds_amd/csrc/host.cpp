@@ -232,22 +232,24 @@ GridTensors build_grid(const Tensor &points, const Tensor &bids, int64_t batch,
 void check_search(const Tensor &samples, const Tensor &sbids, const Tensor &num_cells,
                   const Tensor &smin, const Tensor &inv_cell);
 
-// Centres in the order of their cells in a grid -> (order, coordinates, cloud ids).
-std::tuple<Tensor, Tensor, Tensor> order_centres(const Tensor &samples, const Tensor &bids,
+// Centres in the order of their cells in a grid -> (order, coordinates, cloud ids, cell keys).
+std::tuple<Tensor, Tensor, Tensor, Tensor> order_centres(const Tensor &samples, const Tensor &bids,
                                                  int64_t batch, const Tensor &num_cells,
                                                  const Tensor &smin, const Tensor &inv_cell,
                                                  int64_t key_bits) {
   check_search(samples, bids, num_cells, smin, inv_cell);
   const int64_t n = samples.size(0), d = samples.size(1);
   Tensor order = empty_i32({n}, samples), pts = empty_f32({n, d}, samples),
-         out_bids = empty_i32({n}, samples);
+         out_bids = empty_i32({n}, samples),
+         keys = at::empty({n}, samples.options().dtype(at::kLong).requires_grad(false));
   Tensor ws = workspace(mccnn_order_centres_workspace_bytes(n), samples);
   hipStream_t s = current_stream();
   Region r("order_centres", s);
-  check(mccnn_order_centres(s, n, (int)d, f32(samples), i32(bids), (int)batch, i32(num_cells),
-                            f32(smin), f32(inv_cell), (int)key_bits, ws.data_ptr(), ws.numel(),
-                            i32(order), f32(pts), i32(out_bids)));
-  return {order, pts, out_bids};
+  check(mccnn_order_centres_keys(s, n, (int)d, f32(samples), i32(bids), (int)batch,
+                                 i32(num_cells), f32(smin), f32(inv_cell), (int)key_bits,
+                                 ws.data_ptr(), ws.numel(), i32(order), f32(pts), i32(out_bids),
+                                 i64(keys)));
+  return {order, pts, out_bids, keys};
 }
 
 Tensor invert_order(const Tensor &order) {
@@ -371,6 +373,26 @@ std::tuple<Tensor, Tensor, bool> search(const Tensor &samples, const Tensor &sbi
                                   f32(inv_radii), (int)max_neighs, ws.data_ptr(), ws.numel(),
                                   i32(ranges), m, i32(neighbors)));
   return {ranges, neighbors, cut};
+}
+
+// The same where the number of pairs is known: no host round trip -> (ranges, neighbors).
+std::tuple<Tensor, Tensor> search_known(const Tensor &samples, const Tensor &sbids,
+                                        const Tensor &points, const Tensor &keys,
+                                        const Tensor &num_cells, const Tensor &smin,
+                                        const Tensor &inv_cell, const Tensor &inv_radii,
+                                        int64_t pairs) {
+  check_search(samples, sbids, points, keys, num_cells, smin, inv_cell, inv_radii);
+  const int64_t ns = samples.size(0);
+  const int nd = (int)dim(samples, 1);
+  Tensor ws = workspace(mccnn_find_neighbors_workspace_bytes(nd, ns), samples);
+  Tensor ranges = empty_i32({ns}, samples), neighbors = empty_i32({pairs, 2}, samples);
+  hipStream_t s = current_stream();
+  Region r("transpose_neighbors", s);
+  check(mccnn_search_known(s, ns, nd, f32(samples), i32(sbids), points.size(0), f32(points),
+                           i64(keys), nullptr, i32(num_cells), f32(smin), f32(inv_cell),
+                           f32(inv_radii), ws.data_ptr(), ws.numel(), pairs, i32(ranges),
+                           i32(neighbors)));
+  return {ranges, neighbors};
 }
 
 Tensor grid_density(const Tensor &points, const Tensor &bids, const Tensor &keys,
@@ -1427,6 +1449,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("collect_timing", &collect_timing);
   m.def("compute_keys", &compute_keys, release());
   m.def("order_centres", &order_centres, release());
+  m.def("search_known", &search_known, release());
   m.def("invert_order", &invert_order, release());
   m.def("build_grid", &build_grid, release());
   m.def("build_grid_ds", &build_grid_ds, release());

@@ -783,6 +783,34 @@ extern "C" int mccnn_find_neighbors_bounded(
 // The count half of a search by a caller that has the grid in hand (no argument checks beyond
 // sizes and null pointers), with or without the grid's column table, and with the outcome in
 // pinned host memory.
+// Both halves of a count by a caller that has the grid in hand: slices, counts, end offsets and
+// their total in `total` (device or pinned memory).
+static int search_counts(hipStream_t s, int64_t num_samples, int num_dims, const float *samples,
+                         const int32_t *sample_batch_ids, int64_t num_pts, const float *points,
+                         const int64_t *point_keys, const int32_t *grid_ds,
+                         const int32_t *num_cells, const float *scaled_aabb_min,
+                         const float *inv_cell_sizes, const float *inv_radii, int max_neighs,
+                         const NbrWorkspace &w, int32_t *ranges_out, int64_t *total,
+                         int64_t *truncated) {
+  const bool in_visit = num_samples <= kSearchInVisit;
+  const VisitSearch search = {sample_batch_ids, num_pts, (const int64_t *)point_keys,
+                              (const int2 *)grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes};
+  if (!in_visit) {
+    MCCNN_DIM_SWITCH(num_dims,
+                     hipLaunchKernelGGL(nbr_ranges_kernel<D>,
+                                        dim3(blocks_for(num_samples * offsets_for(num_dims), 256)),
+                                        dim3(256), 0, s, num_samples, samples, sample_batch_ids,
+                                        num_pts, (const int64_t *)point_keys, (const int2 *)grid_ds,
+                                        num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
+                                        w.ranges));
+    MCCNN_LAUNCH_CHECK();
+  }
+  int rc = launch_count(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
+                        in_visit ? &search : nullptr, ranges_out, truncated);
+  if (rc != MCCNN_OK) return rc;
+  return inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, total);
+}
+
 extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, int num_dims,
                                   const float *samples, const int32_t *sample_batch_ids,
                                   int64_t num_pts, const float *points, const int64_t *point_keys,
@@ -805,24 +833,10 @@ extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, in
   MCCNN_REQUIRE(workspace_bytes >= w.bytes, "search_count workspace too small (%zu < %zu)",
                 workspace_bytes, w.bytes);
   hipStream_t s = as_stream(stream);
-  const bool in_visit = num_samples <= kSearchInVisit;
-  const VisitSearch search = {sample_batch_ids, num_pts, (const int64_t *)point_keys,
-                              (const int2 *)grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes};
-  if (!in_visit) {
-    MCCNN_DIM_SWITCH(num_dims,
-                     hipLaunchKernelGGL(nbr_ranges_kernel<D>,
-                                        dim3(blocks_for(num_samples * offsets_for(num_dims), 256)),
-                                        dim3(256), 0, s, num_samples, samples, sample_batch_ids,
-                                        num_pts, (const int64_t *)point_keys, (const int2 *)grid_ds,
-                                        num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
-                                        w.ranges));
-    MCCNN_LAUNCH_CHECK();
-  }
-  int rc = launch_count(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
-                        in_visit ? &search : nullptr, ranges_out,
-                        max_neighs > 0 ? result_pinned + 1 : nullptr);
-  if (rc != MCCNN_OK) return rc;
-  rc = inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, result_pinned);
+  int rc = search_counts(s, num_samples, num_dims, samples, sample_batch_ids, num_pts, points,
+                         point_keys, grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
+                         max_neighs, w, ranges_out, result_pinned,
+                         max_neighs > 0 ? result_pinned + 1 : nullptr);
   if (rc != MCCNN_OK) return rc;
   MCCNN_HIP_CHECK(hipStreamSynchronize(s));
   MCCNN_REQUIRE(result_pinned[0] < (((int64_t)1 << 31) - 1),
@@ -830,6 +844,36 @@ extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, in
                 "hold fewer than 2^31 - 1",
                 (long long)result_pinned[0]);
   return MCCNN_OK;
+}
+
+extern "C" int mccnn_search_known(mccnn_stream_t stream, int64_t num_samples, int num_dims,
+                                  const float *samples, const int32_t *sample_batch_ids,
+                                  int64_t num_pts, const float *points, const int64_t *point_keys,
+                                  const int32_t *grid_ds, const int32_t *num_cells,
+                                  const float *scaled_aabb_min, const float *inv_cell_sizes,
+                                  const float *inv_radii, void *workspace, size_t workspace_bytes,
+                                  int64_t num_neighbors, int32_t *ranges_out,
+                                  int32_t *neighbors_out) {
+  MCCNN_REQUIRE(valid_dims(num_dims), "search_known expects a valid number of dimensions");
+  MCCNN_REQUIRE(num_samples >= 0 && num_pts >= 0 && num_samples < ((int64_t)1 << 31) &&
+                    num_pts < ((int64_t)1 << 31) && num_neighbors >= 0 &&
+                    num_neighbors < ((int64_t)1 << 31),
+                "search_known expects sizes in [0, 2^31)");
+  if (num_samples == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(samples && sample_batch_ids && num_cells && scaled_aabb_min && inv_cell_sizes &&
+                    inv_radii && ranges_out && workspace && (num_pts == 0 || (points && point_keys)) &&
+                    (num_neighbors == 0 || neighbors_out),
+                "search_known received a null tensor");
+  const NbrWorkspace w = carve_nbr_workspace(workspace, num_dims, num_samples);
+  MCCNN_REQUIRE(workspace_bytes >= w.bytes, "search_known workspace too small (%zu < %zu)",
+                workspace_bytes, w.bytes);
+  hipStream_t s = as_stream(stream);
+  int rc = search_counts(s, num_samples, num_dims, samples, sample_batch_ids, num_pts, points,
+                         point_keys, grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
+                         0, w, ranges_out, w.total, nullptr);
+  if (rc != MCCNN_OK || num_neighbors == 0) return rc;
+  return launch_fill(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, 0, ranges_out,
+                     neighbors_out, num_neighbors);
 }
 
 struct DensityWorkspace {

@@ -383,6 +383,7 @@ class _SortedView:
         self._symmetric = (nbh._equal_samples or nbh._self_neighborhood is not None) and \
             nbh.max_neighbors == 0
         self._transposed = (self.table, self.ranges) if self._symmetric else None
+        self._search_back = self._search_among_centres(nbh)
         self._pdf_key, self.pdf, self.pdf_t = None, None, None
 
     @property
@@ -399,8 +400,30 @@ class _SortedView:
             self._centre_order = self.centre_rows.long()
         return self._centre_order
 
+    # Up to this many points and centres the transposed table of a search without a limit is the
+    # search from the points among the centres, three launches: the pairs are the same (cells of a
+    # pair are neighbours either way, and the distance test is exact under negation) and so is
+    # their order (ascending slots).  Regrouping the pairs by a sort is nine launches: 35 against
+    # 24 us of kernels for 16 x 1024 points and their cell averages.  Beyond, a search without a
+    # column table of the centres costs more than the sort.
+    _MOST_SEARCHED_BACK = 16384
+
+    def _search_among_centres(self, nbh):
+        """Arguments of that search, or None where it does not apply."""
+        grid = nbh._grid
+        if nbh.max_neighbors != 0 or nbh._sorted_cells is None or self._transposed is not None or \
+                max(self.points_in.shape[0], self.points_out.shape[0]) > self._MOST_SEARCHED_BACK:
+            return None
+        bids, cells = nbh._sorted_cells
+        return (self.points_in.detach(), grid._sorted_batch_ids, self.points_out, cells,
+                grid._num_cells, grid._scaled_aabb_min, grid._inv_cell_sizes, nbh._inv_radii,
+                self.table.shape[0])
+
     def _transpose(self):
         """The pairs grouped by point: needed by gradients only, built on first use."""
+        if self._transposed is None and self._search_back is not None:
+            ranges_t, table_t = _lib.host().search_known(*self._search_back)
+            self._transposed, self._search_back = (table_t, ranges_t), None
         if self._transposed is None:
             ranges_t, pair_order = _lib.host().transpose_neighbors(self.table,
                                                                    self.points_in.shape[0])
@@ -474,7 +497,7 @@ class Neighborhood:
         self._inv_radii = _reciprocal(self._radii)
         s = self._point_cloud_sampled
         self._self_neighborhood = None
-        self._table = self._ranges = self._original = self._sorted = None
+        self._table = self._ranges = self._original = self._sorted = self._sorted_cells = None
         if point_cloud_sample is grid._point_cloud:
             # The centres are the grid's own points in the caller's order: search once
             # from the sorted points (the same search also serves the densities).
@@ -509,12 +532,13 @@ class Neighborhood:
             return
         # (an order of few centres is one launch, which does not need the width of the keys)
         one_launch = s._points.shape[0] <= _lib.lib().mccnn_build_grid_single_launch_max()
-        order, pts, bids = _lib.host().order_centres(
+        order, pts, bids, cells = _lib.host().order_centres(
             s._points.detach(), s._batch_ids, grid._batch_size, num_cells, smin, inv_cell,
             0 if one_launch else grid._key_bits)
         ranges, table, _ = _lib.host().search(pts, bids, points, keys, ds, num_cells, smin,
                                               inv_cell, self._inv_radii, self.max_neighbors)
         self._sorted = (order, pts, ranges, table)
+        self._sorted_cells = (bids, cells)
 
     def _sorted_search(self):
         """(centre order, centres, ranges, pairs) with the centres in the order of their cells."""
