@@ -550,6 +550,17 @@ int mccnn_sampling_count(mccnn_stream_t stream, int mode, int64_t num_pts,
                          int64_t ranges_len, const int32_t *ranges,
                          void *workspace, size_t workspace_bytes,
                          int64_t *num_sampled_out_host);
+/* The same with the number in pinned host memory (hipHostMalloc) that the kernels write. */
+int mccnn_sampling_count_pinned(mccnn_stream_t stream, int mode, int64_t num_pts,
+                         int num_dims, const float *points,
+                         int64_t batch_ids_len, const int32_t *batch_ids,
+                         int64_t point_keys_len, const int64_t *point_keys,
+                         int num_cells_len, const int32_t *num_cells,
+                         int64_t num_neighbors, int neighbors_rank,
+                         int neighbors_cols, const int32_t *neighbors,
+                         int64_t ranges_len, const int32_t *ranges,
+                         void *workspace, size_t workspace_bytes,
+                         int64_t *num_sampled_out_pinned);
 int mccnn_sampling_fill(mccnn_stream_t stream, int mode, int64_t num_pts,
                         int num_dims, const float *points,
                         const int32_t *batch_ids, const int64_t *point_keys,

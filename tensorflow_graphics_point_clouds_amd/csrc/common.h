@@ -37,6 +37,14 @@ inline hipStream_t as_stream(mccnn_stream_t s) { return reinterpret_cast<hipStre
 
 #define MCCNN_LAUNCH_CHECK() MCCNN_HIP_CHECK(hipGetLastError())
 
+// Waits until the kernels on `s` have written `n` values to pinned host memory that held -1 before
+// they were launched (values are never negative), by looking at the memory: what the host asks
+// for is there when the kernel has stored it, which is some 15 us before the stream is known to be
+// idle (a marker is enqueued, its signal waited for).  After a while, or if the values do not
+// arrive that way, the stream is waited for.  Defined in util.hip.
+int wait_for_host_values(hipStream_t s, const volatile int64_t *values, int n);
+int wait_for_host_values(hipStream_t s, const volatile int32_t *values, int n);
+
 // Dispatch on the point dimension (2..6), the template parameter of most kernels.
 #define MCCNN_DIM_SWITCH(D_, ...)                              \
   switch (D_) {                                                \

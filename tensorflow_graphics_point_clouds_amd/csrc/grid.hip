@@ -888,16 +888,22 @@ static int build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims, cons
     int rc = reduce_boxes(s, num_pts, num_dims, points, batch_ids, batch_size, mn, mx);
     if (rc != MCCNN_OK) return rc;
     const int nb = (int)((num_pts + kSortTile - 1) / kSortTile);
+    if (shape_is_pinned)
+      for (int d = 0; d < num_dims; ++d) num_cells_out_host[d] = -1;
     MCCNN_DIM_SWITCH(num_dims,
                      hipLaunchKernelGGL(grid_keys_kernel<D>, dim3(nb), dim3(kSortThreads), 0, s,
                                         num_pts, batch_size, nb, points, batch_ids, cell_sizes, mn,
                                         mx, g, keys32, w.hist,
                                         shape_is_pinned ? num_cells_out_host : (int32_t *)nullptr));
     MCCNN_LAUNCH_CHECK();
-    if (!shape_is_pinned)
+    if (shape_is_pinned) {
+      rc = wait_for_host_values(s, num_cells_out_host, num_dims);
+      if (rc != MCCNN_OK) return rc;
+    } else {
       MCCNN_HIP_CHECK(hipMemcpyAsync(num_cells_out_host, g.num_cells, sizeof(int32_t) * num_dims,
                                      hipMemcpyDeviceToHost, s));
-    MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+      MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+    }
     const int bits = key_bits_for(batch_size, num_dims, num_cells_out_host);
     *key_bits_out_host = bits;
     if (bits <= 32) {

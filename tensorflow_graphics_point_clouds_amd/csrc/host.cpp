@@ -95,7 +95,8 @@ class PinnedBlock {
         pool().pop_back();
       }
     }
-    if (!p_) hip_check(hipHostMalloc(&p_, 256, hipHostMallocDefault));
+    // (coherent: the host reads what a kernel has stored while the kernel still runs)
+    if (!p_) hip_check(hipHostMalloc(&p_, 256, hipHostMallocCoherent));
   }
   ~PinnedBlock() {
     std::lock_guard<std::mutex> lock(mutex());
@@ -520,7 +521,7 @@ std::tuple<Tensor, Tensor, Tensor> sampling(const Tensor &points, const Tensor &
   host.words()[0] = 0;
   {
     Region r("sampling_count", s);
-    check(mccnn_sampling_count(s, (int)mode, n, nd, f32(points), bids.size(0), i32(bids),
+    check(mccnn_sampling_count_pinned(s, (int)mode, n, nd, f32(points), bids.size(0), i32(bids),
                                keys.size(0), i64(keys), (int)num_cells.size(0), i32(num_cells),
                                neighbors.size(0), (int)neighbors.dim(), (int)dim(neighbors, 1),
                                i32(neighbors), ranges.size(0), i32(ranges), ws.data_ptr(),

@@ -833,12 +833,14 @@ extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, in
   MCCNN_REQUIRE(workspace_bytes >= w.bytes, "search_count workspace too small (%zu < %zu)",
                 workspace_bytes, w.bytes);
   hipStream_t s = as_stream(stream);
+  result_pinned[0] = -1;                  // (the flag is written by a kernel before the total's)
   int rc = search_counts(s, num_samples, num_dims, samples, sample_batch_ids, num_pts, points,
                          point_keys, grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
                          max_neighs, w, ranges_out, result_pinned,
                          max_neighs > 0 ? result_pinned + 1 : nullptr);
   if (rc != MCCNN_OK) return rc;
-  MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+  rc = wait_for_host_values(s, result_pinned, 1);
+  if (rc != MCCNN_OK) return rc;
   MCCNN_REQUIRE(result_pinned[0] < (((int64_t)1 << 31) - 1),
                 "FindNeighbors found at least %lld pairs; the int32 offsets of the op contract "
                 "hold fewer than 2^31 - 1",

@@ -302,7 +302,7 @@ extern "C" size_t mccnn_sampling_workspace_bytes(int64_t num_pts) {
   return carve_sampling_workspace(nullptr, num_pts).bytes;
 }
 
-extern "C" int mccnn_sampling_count(mccnn_stream_t stream, int mode, int64_t num_pts, int num_dims,
+static int sampling_count(mccnn_stream_t stream, int mode, int64_t num_pts, int num_dims,
                                     const float *points, int64_t batch_ids_len,
                                     const int32_t *batch_ids, int64_t point_keys_len,
                                     const int64_t *point_keys, int num_cells_len,
@@ -310,7 +310,7 @@ extern "C" int mccnn_sampling_count(mccnn_stream_t stream, int mode, int64_t num
                                     int neighbors_rank, int neighbors_cols,
                                     const int32_t *neighbors, int64_t ranges_len,
                                     const int32_t *ranges, void *workspace,
-                                    size_t workspace_bytes, int64_t *num_sampled_out_host) {
+                                    size_t workspace_bytes, bool pinned, int64_t *num_sampled_out_host) {
   MCCNN_REQUIRE(mode >= 0 && mode < 2, "Sampling requires a valid sampling mode");
   MCCNN_REQUIRE(valid_dims(num_dims), "Sampling expects a valid number of dimensions");
   MCCNN_REQUIRE(batch_ids_len == num_pts,
@@ -340,7 +340,10 @@ extern "C" int mccnn_sampling_count(mccnn_stream_t stream, int mode, int64_t num
   hipLaunchKernelGGL(flag_cell_starts_kernel, dim3(grid), dim3(256), 0, s, num_pts,
                      (const int64_t *)point_keys, w.cell_scan);
   MCCNN_LAUNCH_CHECK();
-  int rc = inclusive_scan_i32(s, num_pts, w.cell_scan, w.scan_scratch, w.num_cells_total);
+  // pinned: the last scan's total goes straight to the host
+  if (pinned) *num_sampled_out_host = -1;
+  int rc = inclusive_scan_i32(s, num_pts, w.cell_scan, w.scan_scratch,
+                              pinned && mode == 1 ? num_sampled_out_host : w.num_cells_total);
   if (rc != MCCNN_OK) return rc;
   hipLaunchKernelGGL(store_cell_starts_kernel, dim3(grid), dim3(256), 0, s, num_pts,
                      (const int64_t *)point_keys, w.cell_scan, w.first_idx);
@@ -371,14 +374,40 @@ extern "C" int mccnn_sampling_count(mccnn_stream_t stream, int mode, int64_t num
     }
     hipLaunchKernelGGL(copy_i32_kernel, dim3(grid), dim3(256), 0, s, num_pts, w.used, w.sel_scan);
     MCCNN_LAUNCH_CHECK();
-    rc = inclusive_scan_i32(s, num_pts, w.sel_scan, w.scan_scratch, w.num_selected);
+    rc = inclusive_scan_i32(s, num_pts, w.sel_scan, w.scan_scratch,
+                            pinned ? num_sampled_out_host : w.num_selected);
     if (rc != MCCNN_OK) return rc;
     result = w.num_selected;
   }
+  if (pinned) return wait_for_host_values(s, num_sampled_out_host, 1);
   MCCNN_HIP_CHECK(hipMemcpyAsync(num_sampled_out_host, result, sizeof(int64_t),
                                  hipMemcpyDeviceToHost, s));
   MCCNN_HIP_CHECK(hipStreamSynchronize(s));
   return MCCNN_OK;
+}
+
+extern "C" int mccnn_sampling_count(
+    mccnn_stream_t stream, int mode, int64_t num_pts, int num_dims, const float *points,
+    int64_t batch_ids_len, const int32_t *batch_ids, int64_t point_keys_len,
+    const int64_t *point_keys, int num_cells_len, const int32_t *num_cells, int64_t num_neighbors,
+    int neighbors_rank, int neighbors_cols, const int32_t *neighbors, int64_t ranges_len,
+    const int32_t *ranges, void *workspace, size_t workspace_bytes, int64_t *num_sampled_out_host) {
+  return sampling_count(stream, mode, num_pts, num_dims, points, batch_ids_len, batch_ids,
+                        point_keys_len, point_keys, num_cells_len, num_cells, num_neighbors,
+                        neighbors_rank, neighbors_cols, neighbors, ranges_len, ranges, workspace,
+                        workspace_bytes, false, num_sampled_out_host);
+}
+
+extern "C" int mccnn_sampling_count_pinned(
+    mccnn_stream_t stream, int mode, int64_t num_pts, int num_dims, const float *points,
+    int64_t batch_ids_len, const int32_t *batch_ids, int64_t point_keys_len,
+    const int64_t *point_keys, int num_cells_len, const int32_t *num_cells, int64_t num_neighbors,
+    int neighbors_rank, int neighbors_cols, const int32_t *neighbors, int64_t ranges_len,
+    const int32_t *ranges, void *workspace, size_t workspace_bytes, int64_t *num_sampled_out_pinned) {
+  return sampling_count(stream, mode, num_pts, num_dims, points, batch_ids_len, batch_ids,
+                        point_keys_len, point_keys, num_cells_len, num_cells, num_neighbors,
+                        neighbors_rank, neighbors_cols, neighbors, ranges_len, ranges, workspace,
+                        workspace_bytes, true, num_sampled_out_pinned);
 }
 
 extern "C" int mccnn_sampling_fill(mccnn_stream_t stream, int mode, int64_t num_pts, int num_dims,

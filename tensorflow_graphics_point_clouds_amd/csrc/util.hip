@@ -1,6 +1,9 @@
 // Error reporting, fill and prefix-sum helpers of libmccnn_hip.so.
 #include <stdarg.h>
 
+#include <atomic>
+#include <chrono>
+
 #include "common.h"
 #include "fill.h"
 
@@ -229,6 +232,31 @@ int inclusive_scan_i32(hipStream_t stream, int64_t n, int *counts, int *block_su
                      counts, block_sums, total_dev);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
+}
+
+template <class T>
+static int wait_for_values(hipStream_t s, const volatile T *values, int n) {
+  const auto start = std::chrono::steady_clock::now();
+  for (int i = 0; i < n;) {
+    if (values[i] != (T)-1) {
+      ++i;
+      continue;
+    }
+    __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() - start > std::chrono::milliseconds(20)) {
+      MCCNN_HIP_CHECK(hipStreamSynchronize(s));
+      return MCCNN_OK;
+    }
+  }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  return MCCNN_OK;
+}
+
+int wait_for_host_values(hipStream_t s, const volatile int64_t *values, int n) {
+  return wait_for_values(s, values, n);
+}
+int wait_for_host_values(hipStream_t s, const volatile int32_t *values, int n) {
+  return wait_for_values(s, values, n);
 }
 
 }  // namespace mccnn

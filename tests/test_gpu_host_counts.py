@@ -1,0 +1,62 @@
+"""Counts that the host reads from pinned memory while the kernels run: behind a stream that is busy
+for longer than the host looks at the memory, and from several threads on streams of their own."""
+import threading
+
+import pytest
+
+torch = pytest.importorskip("torch")
+
+pytestmark = pytest.mark.gpu
+
+
+def _build(points, ids, batch, radius):
+    from tensorflow_graphics_point_clouds_amd import pc
+    cloud = pc.PointCloud(points, ids, batch)
+    nbh = pc.Neighborhood(pc.Grid(cloud, radius), radius, cloud)
+    hierarchy = pc.PointHierarchy(cloud, [radius], "poisson")
+    averages = pc.PointHierarchy(cloud, [radius], "cell average")
+    return (nbh._original_neigh_ids, nbh._samples_neigh_ranges, hierarchy[1]._points,
+            averages[1]._points)
+
+
+def _cloud(n, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    return (torch.rand(n, 3, device="cuda", generator=gen),
+            torch.arange(n, device="cuda").mul(2).div(n, rounding_mode="floor").int())
+
+
+def test_counts_behind_a_busy_stream():
+    points, ids = _cloud(20000, 1)
+    expect = _build(points, ids, 2, 0.06)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(200_000_000)                       # some 80 ms
+    for a, b in zip(_build(points, ids, 2, 0.06), expect):
+        assert torch.equal(a, b)
+
+
+def test_counts_from_several_threads():
+    sizes = [300, 5000, 17000, 40000]
+    clouds = [_cloud(n, n) for n in sizes]
+    expect = [[_build(p, i, 2, r) for r in (0.05, 0.08)] for p, i in clouds]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(k):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                for turn in range(6):
+                    for j, r in enumerate((0.05, 0.08)):
+                        got = _build(*clouds[k], 2, r)
+                        if not all(torch.equal(a, b) for a, b in zip(got, expect[k][j])):
+                            wrong.append((sizes[k], turn, r))
+            stream.synchronize()
+        except Exception as e:                            # (a thread's exception ends the test)
+            wrong.append((sizes[k], e))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
