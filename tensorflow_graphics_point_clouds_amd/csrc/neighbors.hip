@@ -9,14 +9,13 @@
 //   count   8 lanes per centre stride over the slices and test
 //           |(s - p) * inv_radii| < 1 (count_neighbors_kernels.cu.cc:83-86; as the
 //           squared length against 1, which decides identically);
-//   fill    same traversal; the slot of a hit is the centre's start offset plus
-//           a ballot prefix inside the 8-lane group, so the pairs of a centre
-//           come out in ascending sorted-point index without atomics or a sort.
+//   fill    the hits that the count pass has left as bits, one word per lane and window of
+//           trips; the slot of a hit is the centre's start offset plus a ballot prefix inside
+//           the 8-lane group, so the pairs of a centre come out in ascending sorted-point index
+//           without atomics or a sort.
 // Offsets are enumerated so that the slices of a centre ascend in index.
-// (Keeping the count pass's hit masks for the fill pass, so that it need not load
-// and test the candidates again, was measured: what the count pass loses by
-// storing them is what the fill pass gains, and crowded centres, whose masks do
-// not fit a fixed budget, pay for both.)
+// (The bits cost the count pass nothing: instead of a running number of hits a lane shifts each
+// outcome into a word, one add with carry either way, and counts the word's bits at its end.)
 // Small inputs are bound by launches: there the count pass finds its slices itself (every
 // lane of a group searches one or two), and a grid without a column table, which would need
 // the grid's shape on the host first, is searched over all of its keys.
@@ -33,6 +32,11 @@ namespace mccnn {
 constexpr int kGroup = 8;                  // lanes per centre
 constexpr int kNbrThreads = 256;
 constexpr int kCentresPerBlock = kNbrThreads / kGroup;
+constexpr int kTrips = 32;                 // trips of eight candidates listed at a time
+// Windows of 32 trips whose hits the count pass keeps for the fill pass (64 bytes per centre):
+// 21.6 trips on average where a centre has 37 neighbours.  Candidates behind them -- crowded
+// centres, and the slices after the first nine from four dimensions on -- are tested again.
+constexpr int kMaskWindows = 2;
 
 // Offsets act on dims 0..max(D-2,1); the last dim is covered by the key search.
 template <int D>
@@ -206,8 +210,9 @@ __global__ void __launch_bounds__(256) nbr_ranges_kernel(
   }
 }
 
+// Whether a candidate lies inside the radius; `live` false: no candidate at all.
 template <int D>
-__device__ __forceinline__ bool within_radius(const float *diff, const float *ir) {
+__device__ __forceinline__ bool within_radius(bool live, const float *diff, const float *ir) {
   float acc = 0.0f;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
@@ -219,8 +224,8 @@ __device__ __forceinline__ bool within_radius(const float *diff, const float *ir
   // correctly rounded root is monotonic, sqrtf(1) = 1 and the root of the largest
   // float below 1 is again that float, so acc < 1 decides the same for every
   // float, infinities and NaN included, without the twenty instructions of an
-  // IEEE square root per candidate.
-  return acc < 1.0f;
+  // IEEE square root per candidate.  (A sum of squares is never below 0.)
+  return acc < (live ? 1.0f : 0.0f);
 }
 
 // What a visit of a centre's candidates produces.
@@ -294,15 +299,16 @@ struct VisitSearch {                  // for kSearch: the grid to find the slice
 template <int D, Visit kVisit, bool kSearch>
 __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
     int64_t ns, const float *__restrict__ samples, const float *__restrict__ pts,
-    int2 *ranges, const float *__restrict__ inv_radii, int max_neighs, VisitSearch search,
+    int2 *ranges, unsigned *masks, const float *__restrict__ inv_radii, int max_neighs,
+    VisitSearch search,
     int *__restrict__ counts, const int *__restrict__ ends, int2 *__restrict__ nbrs,
     int64_t *__restrict__ truncated, int64_t capacity, const float *__restrict__ inv_bandwidth,
     int mode, float *__restrict__ density /* kDensity: [3, ns], counts: hits per wavefront */) {
   constexpr int R = OffsetInfo<D>::count();
+  constexpr int kAhead = 4;                        // trips in flight
+  __shared__ __align__(16) int2 trips[kCentresPerBlock][kTrips + kAhead];
   const int sub = threadIdx.x & (kGroup - 1);
   const int lane = lane_id();
-  const uint64_t group_mask = ((1ull << kGroup) - 1ull) << (lane & ~(kGroup - 1));
-  const uint64_t below_mask = group_mask & ((1ull << lane) - 1ull);
   float ir[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) ir[d] = inv_radii[d];
@@ -325,39 +331,38 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
       norm *= bw * 0.39894228f;
     }
   }
-  auto load_point = [&](int j, float *q) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) q[d] = pts[(int64_t)j * D + d];
+  const bool upper = lane >= 32;                                // the group's bits in a ballot
+  const int shift = lane & 24;
+  const unsigned below = (1u << sub) - 1u;
+  int2 *const list = nbrs + start;                              // kFill: the centre's pairs,
+  const int64_t space = capacity - start;                       // and how many are stored
+  const int most = (int)(space < limit ? (space > 0 ? space : 0) : limit);
+  auto hits_of = [&](uint64_t ballot) {                         // of the group
+    return ((upper ? (unsigned)(ballot >> 32) : (unsigned)ballot) >> shift) & 0xffu;
   };
-  auto visit = [&](bool live, int j, const float *q) {          // kGroup candidates of the centre
-    float diff[D];
+  auto inside = [&](bool live, const float *q, float *diff) {
 #pragma unroll
     for (int d = 0; d < D; ++d) diff[d] = s[d] - q[d];
-    const bool hit = live && within_radius<D>(diff, ir);
-    if (kVisit == Visit::kFill) {
-      const uint64_t hits = __ballot(hit) & group_mask;
-      const int slot = found + __popcll(hits & below_mask);
-      if (hit && slot < limit && start + slot < capacity)
-        nbrs[start + slot] = make_int2(j, (int)c);
-      found += __popcll(hits);
-    } else if (kVisit == Visit::kCount) {
-      found += hit ? 1 : 0;
-    } else {
-      const unsigned hits = (unsigned)((__ballot(hit) & group_mask) >> (lane & ~(kGroup - 1)));
-      if (hits != 0) {                         // the same for the lanes of a group
-        sums.add(hit ? density_term<D>(diff, scale) : 0.0f, hits, sub, lane & ~(kGroup - 1), found);
-        found += __popc(hits);
-      }
-    }
+    return within_radius<D>(live, diff, ir);
+  };
+  auto store_pair = [&](bool hit, int j) {                      // kGroup candidates of the centre
+    const unsigned hits = hits_of(__ballot(hit));
+    const int slot = found + __popc(hits & below);
+    if (hit && slot < most) list[slot] = make_int2(j, (int)c);
+    found += __popc(hits);
   };
   // The slices of the centre, nine at a time (their number is a power of three): lane `sub`
-  // fetches or finds one, the first lane the ninth as well, and the group takes them in turn.
-  // The first candidates of kAhead slices are requested together: most slices hold one or two
-  // trips of a group, and slice by slice every one of them waits for memory again (count and
-  // fill of 763 k centres x 37 pairs 390 -> 352 us; with the searches side by side 2 x 1024 points
-  // 21 -> 18 us).
-  constexpr int kSlices = kGroup + 1, kAhead = 3;
-  static_assert(R % kSlices == 0 && kSlices % kAhead == 0, "slices come in nines");
+  // fetches or finds one, the first lane the ninth as well.  They are cut into trips of eight
+  // candidates whose bounds go into LDS, and the group walks the list of trips, four in flight,
+  // without a branch but the end of the list.  Both passes are bound by instruction issue (vector
+  // units busy for 98 and 88 % of the time).  Slice by slice a trip took 45 instructions, a third
+  // of them for the exec mask, and a wavefront took in each slice the trips of its fullest centre;
+  // the list takes 24, and 14 in the fill pass, which neither loads nor tests the candidates.
+  // 763 k centres x 37 pairs: count 150 -> 116 us, fill 216 -> 121; densities of 16 384 points
+  // straight from the grid 19.4 -> 16.2.  (Two trips in flight: 125 and 118.)
+  constexpr int kSlices = kGroup + 1;
+  static_assert(R % kSlices == 0, "slices come in nines");
+  int2 *const trip = trips[threadIdx.x / kGroup];
   for (int r0 = 0; r0 < R; r0 += kSlices) {
     int2 mine[2] = {make_int2(0, 0), make_int2(0, 0)};          // slices r0 + sub and r0 + kGroup
     if constexpr (kSearch) {
@@ -377,30 +382,74 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
       mine[0] = ranges[c * R + r0 + sub];
       mine[1] = ranges[c * R + r0 + kGroup];
     }
+    const int n0 = (mine[0].y - mine[0].x + kGroup - 1) / kGroup;
+    const int n1 = (mine[1].y - mine[1].x + kGroup - 1) / kGroup;
+    int upto = n0;                                              // trips of slices r0 .. r0 + sub
 #pragma unroll
-    for (int rb = 0; rb < kSlices; rb += kAhead) {
-      int2 span[kAhead];
-      float q[kAhead][D];
+    for (int off = 1; off < kGroup; off *= 2) {
+      const int o = __shfl_up(upto, off, kGroup);
+      upto += sub >= off ? o : 0;
+    }
+    const int before1 = __shfl(upto, kGroup - 1, kGroup), total = before1 + n1;
+    for (int t0 = 0; t0 < total; t0 += kTrips) {                // a window of the trips
+      wave_lds_sync();                                          // the window before has been read
+      const int first = upto - n0 - t0;
+      for (int k = first < 0 ? -first : 0; k < n0 && first + k < kTrips; ++k)
+        trip[first + k] = make_int2(mine[0].x + kGroup * k, mine[0].y);
+      for (int k = sub; k < n1; k += kGroup)
+        if (before1 + k - t0 >= 0 && before1 + k - t0 < kTrips)
+          trip[before1 + k - t0] = make_int2(mine[1].x + kGroup * k, mine[1].y);
+      const int n = total - t0 < kTrips ? total - t0 : kTrips;
+      if (sub < kAhead) trip[n + sub] = make_int2(0, 0);        // (no candidates)
+      wave_lds_sync();
+      const bool masked = r0 == 0 && t0 < kTrips * kMaskWindows;
+      const int64_t mask_at = ((int64_t)(t0 / kTrips) * ns + c) * kGroup + sub;
+      if (kVisit == Visit::kFill && masked) {
+        unsigned word = masks[mask_at];
+        for (int t = 0; t < n; t += kAhead) {
 #pragma unroll
-      for (int u = 0; u < kAhead; ++u) {
-        span[u] = rb + u < kGroup ? make_int2(__shfl(mine[0].x, (rb + u) % kGroup, kGroup),
-                                              __shfl(mine[0].y, (rb + u) % kGroup, kGroup))
-                                  : mine[1];
-#pragma unroll
-        for (int d = 0; d < D; ++d) q[u][d] = 0.0f;
-        if (span[u].x + sub < span[u].y) load_point(span[u].x + sub, q[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < kAhead; ++u) {
-        if (span[u].x >= span[u].y) continue;                   // the same for the lanes of a group
-        visit(span[u].x + sub < span[u].y, span[u].x + sub, q[u]);
-        for (int j0 = span[u].x + kGroup; j0 < span[u].y; j0 += kGroup) {
-          float t[D];
-#pragma unroll
-          for (int d = 0; d < D; ++d) t[d] = 0.0f;
-          if (j0 + sub < span[u].y) load_point(j0 + sub, t);
-          visit(j0 + sub < span[u].y, j0 + sub, t);
+          for (int u = 0; u < kAhead; ++u) {
+            store_pair((int)word < 0, trip[t + u].x + sub);
+            word <<= 1;
+          }
         }
+        continue;
+      }
+      unsigned word = 0;                                        // kCount: this lane's hits
+      for (int t = 0; t < n; t += kAhead) {
+        int j[kAhead];
+        bool live[kAhead];
+        float q[kAhead][D];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          const int2 span = trip[t + u];
+          j[u] = span.x + sub;
+          live[u] = j[u] < span.y;
+          const int from = live[u] ? j[u] : span.x;             // some point: the trip's first
+#pragma unroll
+          for (int d = 0; d < D; ++d) q[u][d] = pts[(int64_t)from * D + d];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+          float diff[D];
+          const bool hit = inside(live[u], q[u], diff);
+          if (kVisit == Visit::kCount) {
+            word = word + word + (hit ? 1u : 0u);
+          } else if (kVisit == Visit::kFill) {
+            store_pair(hit, j[u]);
+          } else {
+            const unsigned hits = hits_of(__ballot(hit));
+            if (hits != 0) {                   // the same for the lanes of a group
+              sums.add(hit ? density_term<D>(diff, scale) : 0.0f, hits, sub, lane & ~(kGroup - 1),
+                       found);
+              found += __popc(hits);
+            }
+          }
+        }
+      }
+      if (kVisit == Visit::kCount) {
+        found += __popc(word);
+        if (masked) masks[mask_at] = word << (kTrips - (n + kAhead - 1) / kAhead * kAhead);
       }
     }
   }
@@ -459,6 +508,7 @@ constexpr int64_t kSearchInVisit = 16384;
 
 struct NbrWorkspace {
   int2 *ranges;
+  unsigned *masks;       // [kMaskWindows, ns, kGroup]: what the count pass tells the fill pass
   int *scan_scratch;
   int64_t *total;
   size_t bytes;
@@ -476,6 +526,8 @@ static NbrWorkspace carve_nbr_workspace(void *ws, int d, int64_t ns) {
   size_t off = 0;
   w.ranges = (int2 *)(p + off);
   off += align256(sizeof(int2) * (size_t)ns * offsets_for(d));
+  w.masks = (unsigned *)(p + off);
+  off += align256(sizeof(unsigned) * (size_t)ns * kGroup * kMaskWindows);
   w.scan_scratch = (int *)(p + off);
   off += align256(sizeof(int) * scan_scratch_ints(ns));
   w.total = (int64_t *)(p + off);
@@ -562,21 +614,22 @@ extern "C" size_t mccnn_find_neighbors_workspace_bytes(int num_dims, int64_t num
 }
 
 static int launch_count(hipStream_t s, int num_dims, int64_t ns, const float *samples,
-                        const float *points, int2 *slices, const float *inv_radii, int max_neighs,
-                        const VisitSearch *search, int *counts, int64_t *truncated) {
+                        const float *points, const NbrWorkspace &w, const float *inv_radii,
+                        int max_neighs, const VisitSearch *search, int *counts,
+                        int64_t *truncated) {
   const dim3 grid(blocks_for(ns, kCentresPerBlock)), block(kNbrThreads);
   if (search)
     MCCNN_DIM_SWITCH(num_dims,
                      hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kCount, true>), grid, block, 0,
-                                        s, ns, samples, points, slices, inv_radii, max_neighs,
-                                        *search, counts, (const int *)nullptr, (int2 *)nullptr,
+                                        s, ns, samples, points, w.ranges, w.masks, inv_radii,
+                                        max_neighs, *search, counts, (const int *)nullptr, (int2 *)nullptr,
                                         truncated, (int64_t)0, (const float *)nullptr, 0,
                                         (float *)nullptr))
   else
     MCCNN_DIM_SWITCH(num_dims,
                      hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kCount, false>), grid, block,
-                                        0, s, ns, samples, points, slices, inv_radii, max_neighs,
-                                        VisitSearch{}, counts, (const int *)nullptr,
+                                        0, s, ns, samples, points, w.ranges, w.masks, inv_radii,
+                                        max_neighs, VisitSearch{}, counts, (const int *)nullptr,
                                         (int2 *)nullptr, truncated, (int64_t)0,
                                         (const float *)nullptr, 0, (float *)nullptr))
   MCCNN_LAUNCH_CHECK();
@@ -584,13 +637,13 @@ static int launch_count(hipStream_t s, int num_dims, int64_t ns, const float *sa
 }
 
 static int launch_fill(hipStream_t s, int num_dims, int64_t ns, const float *samples,
-                       const float *points, int2 *slices, const float *inv_radii, int max_neighs,
-                       const int *ends, int32_t *neighbors, int64_t capacity) {
+                       const float *points, const NbrWorkspace &w, const float *inv_radii,
+                       int max_neighs, const int *ends, int32_t *neighbors, int64_t capacity) {
   MCCNN_DIM_SWITCH(num_dims,
                    hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kFill, false>),
                                       dim3(blocks_for(ns, kCentresPerBlock)), dim3(kNbrThreads), 0,
-                                      s, ns, samples, points, slices, inv_radii, max_neighs,
-                                      VisitSearch{}, (int *)nullptr, ends, (int2 *)neighbors,
+                                      s, ns, samples, points, w.ranges, w.masks, inv_radii,
+                                      max_neighs, VisitSearch{}, (int *)nullptr, ends, (int2 *)neighbors,
                                       (int64_t *)nullptr, capacity, (const float *)nullptr, 0,
                                       (float *)nullptr));
   MCCNN_LAUNCH_CHECK();
@@ -667,7 +720,7 @@ static int find_neighbors_count_impl(
     int rc0 = fill_zero(s, truncated, sizeof(int64_t));
     if (rc0 != MCCNN_OK) return rc0;
   }
-  int rc = launch_count(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
+  int rc = launch_count(s, num_dims, num_samples, samples, points, w, inv_radii, max_neighs,
                         nullptr, ranges_out, truncated);
   if (rc != MCCNN_OK) return rc;
   rc = inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, w.total);
@@ -739,7 +792,7 @@ extern "C" int mccnn_find_neighbors_fill(
   const NbrWorkspace w = carve_nbr_workspace(workspace, num_dims, num_samples);
   MCCNN_REQUIRE(workspace_bytes >= w.bytes, "FindNeighbors workspace too small (%zu < %zu)",
                 workspace_bytes, w.bytes);
-  return launch_fill(as_stream(stream), num_dims, num_samples, samples, points, w.ranges, inv_radii,
+  return launch_fill(as_stream(stream), num_dims, num_samples, samples, points, w, inv_radii,
                      max_neighs, ranges, neighbors_out, (int64_t)1 << 62);
 }
 
@@ -776,7 +829,7 @@ extern "C" int mccnn_find_neighbors_bounded(
                      count_out_device);
   MCCNN_LAUNCH_CHECK();
   if (capacity == 0) return MCCNN_OK;
-  return launch_fill(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
+  return launch_fill(s, num_dims, num_samples, samples, points, w, inv_radii, max_neighs,
                      ranges_out, neighbors_out, capacity);
 }
 
@@ -805,7 +858,7 @@ static int search_counts(hipStream_t s, int64_t num_samples, int num_dims, const
                                         w.ranges));
     MCCNN_LAUNCH_CHECK();
   }
-  int rc = launch_count(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, max_neighs,
+  int rc = launch_count(s, num_dims, num_samples, samples, points, w, inv_radii, max_neighs,
                         in_visit ? &search : nullptr, ranges_out, truncated);
   if (rc != MCCNN_OK) return rc;
   return inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, total);
@@ -874,7 +927,7 @@ extern "C" int mccnn_search_known(mccnn_stream_t stream, int64_t num_samples, in
                          point_keys, grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
                          0, w, ranges_out, w.total, nullptr);
   if (rc != MCCNN_OK || num_neighbors == 0) return rc;
-  return launch_fill(s, num_dims, num_samples, samples, points, w.ranges, inv_radii, 0, ranges_out,
+  return launch_fill(s, num_dims, num_samples, samples, points, w, inv_radii, 0, ranges_out,
                      neighbors_out, num_neighbors);
 }
 
@@ -933,7 +986,8 @@ extern "C" int mccnn_grid_density(mccnn_stream_t stream, int64_t num_pts, int nu
 #define MCCNN_DENSITY_VISIT(kSearch_, search_)                                                  \
   MCCNN_DIM_SWITCH(num_dims,                                                                    \
                    hipLaunchKernelGGL((nbr_visit_kernel<D, Visit::kDensity, kSearch_>), grid,   \
-                                      block, 0, s, num_pts, points, points, w.slices, inv_radii, \
+                                      block, 0, s, num_pts, points, points, w.slices,            \
+                                      (unsigned *)nullptr, inv_radii,                            \
                                       0, search_, w.counts, (const int *)nullptr,               \
                                       (int2 *)nullptr, (int64_t *)nullptr, (int64_t)0,          \
                                       inv_bandwidth, mode, w.sums))
