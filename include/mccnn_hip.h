@@ -561,6 +561,17 @@ int mccnn_sampling_count_pinned(mccnn_stream_t stream, int mode, int64_t num_pts
                          int64_t ranges_len, const int32_t *ranges,
                          void *workspace, size_t workspace_bytes,
                          int64_t *num_sampled_out_pinned);
+/* Poisson-disk sampling (mode 0) without a pair table, by a caller that has the grid in hand: the
+ * selection that the table of all pairs within the radii (inv_radii [num_dims], the sorted points
+ * among themselves, uncut) would give.  grid_ds as for the search, or null.  The number goes to
+ * pinned host memory; continued by mccnn_sampling_fill on the same workspace. */
+size_t mccnn_sampling_grid_workspace_bytes(int num_dims, int64_t num_pts);
+int mccnn_sampling_grid_count_pinned(mccnn_stream_t stream, int64_t num_pts, int num_dims,
+                                     const float *points, const int32_t *batch_ids,
+                                     const int64_t *point_keys, const int32_t *grid_ds,
+                                     const int32_t *num_cells, const float *inv_radii,
+                                     void *workspace, size_t workspace_bytes,
+                                     int64_t *num_sampled_out_pinned);
 int mccnn_sampling_fill(mccnn_stream_t stream, int mode, int64_t num_pts,
                         int num_dims, const float *points,
                         const int32_t *batch_ids, const int64_t *point_keys,

@@ -508,6 +508,22 @@ Tensor compute_pdf(const Tensor &points, const Tensor &neighbors, const Tensor &
   return pdf;
 }
 
+// The second half: -> (points, batch ids, indices).
+std::tuple<Tensor, Tensor, Tensor> selected_points(int64_t mode, const Tensor &points,
+                                                   const Tensor &bids, const Tensor &keys,
+                                                   const Tensor &num_cells, const Tensor &ws,
+                                                   int64_t k) {
+  const int nd = (int)dim(points, 1);
+  Tensor pts = empty_f32({k, nd}, points), out_bids = empty_i32({k}, points),
+         idx = empty_i32({k}, points);
+  hipStream_t s = current_stream();
+  Region r("sampling_fill", s);
+  check(mccnn_sampling_fill(s, (int)mode, points.size(0), nd, f32(points), i32(bids), i64(keys),
+                            i32(num_cells), ws.data_ptr(), ws.numel(), k, f32(pts), i32(out_bids),
+                            i32(idx)));
+  return {pts, out_bids, idx};
+}
+
 // -> (points, batch ids, indices)
 std::tuple<Tensor, Tensor, Tensor> sampling(const Tensor &points, const Tensor &bids,
                                             const Tensor &keys, const Tensor &num_cells,
@@ -527,14 +543,30 @@ std::tuple<Tensor, Tensor, Tensor> sampling(const Tensor &points, const Tensor &
                                i32(neighbors), ranges.size(0), i32(ranges), ws.data_ptr(),
                                ws.numel(), host.words()));
   }
-  const int64_t k = host.words()[0];
-  Tensor pts = empty_f32({k, nd}, points), out_bids = empty_i32({k}, points),
-         idx = empty_i32({k}, points);
-  Region r("sampling_fill", s);
-  check(mccnn_sampling_fill(s, (int)mode, n, nd, f32(points), i32(bids), i64(keys),
-                            i32(num_cells), ws.data_ptr(), ws.numel(), k, f32(pts), i32(out_bids),
-                            i32(idx)));
-  return {pts, out_bids, idx};
+  return selected_points(mode, points, bids, keys, num_cells, ws, host.words()[0]);
+}
+
+// Poisson-disk sampling of a grid's sorted points without their pair table.
+std::tuple<Tensor, Tensor, Tensor> sampling_grid(const Tensor &points, const Tensor &bids,
+                                                 const Tensor &keys, const OptTensor &ds,
+                                                 const Tensor &num_cells,
+                                                 const Tensor &inv_radii) {
+  const int64_t n = points.size(0);
+  const int nd = (int)dim(points, 1);
+  if (bids.size(0) != n || keys.size(0) != n || num_cells.numel() != nd || inv_radii.numel() != nd)
+    throw InvalidArgument("Sampling expects batch ids and keys per point, numbers of cells and radii "
+                          "per dimension");
+  Tensor ws = workspace(mccnn_sampling_grid_workspace_bytes(nd, n), points);
+  hipStream_t s = current_stream();
+  PinnedBlock host;
+  host.words()[0] = 0;
+  {
+    Region r("sampling_count", s);
+    check(mccnn_sampling_grid_count_pinned(s, n, nd, f32(points), i32(bids), i64(keys),
+                                           i32(opt(ds)), i32(num_cells), f32(inv_radii),
+                                           ws.data_ptr(), ws.numel(), host.words()));
+  }
+  return selected_points(0, points, bids, keys, num_cells, ws, host.words()[0]);
 }
 
 // ------------------------------------------------------------------ dense products ----
@@ -1467,6 +1499,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("gather_i32", &gather_i32, release());
   m.def("compute_pdf", &compute_pdf, release());
   m.def("sampling", &sampling, release());
+  m.def("sampling_grid", &sampling_grid, release());
   m.def("final_product", &final_product, release());
   m.def("weight_grad_product", &weight_grad_product, release());
   m.def("projection_grad_product", &projection_grad_product, release());

@@ -22,6 +22,7 @@
 // Compiled with -ffp-contract=off (the distance test decides integer output).
 #include "common.h"
 #include "fill.h"
+#include "search.h"
 
 namespace mccnn {
 
@@ -38,17 +39,6 @@ constexpr int kTrips = 32;                 // trips of eight candidates listed a
 // centres, and the slices after the first nine from four dimensions on -- are tested again.
 constexpr int kMaskWindows = 2;
 
-// Offsets act on dims 0..max(D-2,1); the last dim is covered by the key search.
-template <int D>
-struct OffsetInfo {
-  static constexpr int kDims = (D - 2 > 1 ? D - 2 : 1) + 1;
-  static constexpr int count() {
-    int c = 1;
-    for (int i = 0; i < kDims; ++i) c *= 3;
-    return c;
-  }
-};
-
 // What a search needs of the grid, per dimension in registers.
 template <int D>
 struct SearchGrid {
@@ -64,14 +54,6 @@ struct SearchGrid {
       rho[d] = inv_radii[d] / ic[d];
     }
   }
-};
-
-// Where a cell row's slice of the sorted points is looked for: in `span` of the keys, from the
-// first key <= maxk up to the first key < mink.  Nothing left to look for where mink > maxk: the
-// slice is `span` itself.
-struct KeyRange {
-  int2 span;
-  int64_t maxk, mink;
 };
 
 // Cell row r of the neighbourhood of point p (cloud b).  `ds` is the column table, or null: then
@@ -146,48 +128,6 @@ __device__ __forceinline__ KeyRange cell_row_keys(const SearchGrid<D> &sg, const
   return KeyRange{span, maxk, mink};
 }
 
-// The slices of kN cell rows.  The two ends of all of them are searched side by side: a binary
-// search is a chain of dependent loads (eleven over 2048 keys), and what one lane has to find is
-// kept to one such chain.
-template <int kN>
-__device__ __forceinline__ void find_slices(const KeyRange *range, const int64_t *__restrict__ keys,
-                                            int2 *slice) {
-  int lo[2 * kN], hi[2 * kN];
-  bool open = false;
-#pragma unroll
-  for (int i = 0; i < kN; ++i) {
-    const bool search = range[i].mink <= range[i].maxk;
-    lo[2 * i] = range[i].span.x;
-    lo[2 * i + 1] = search ? range[i].span.x : range[i].span.y;
-    hi[2 * i] = search ? range[i].span.y : range[i].span.x;
-    hi[2 * i + 1] = range[i].span.y;
-    open |= search;
-  }
-  while (open) {
-    open = false;
-    int64_t key[2 * kN];
-    int mid[2 * kN];
-#pragma unroll
-    for (int k = 0; k < 2 * kN; ++k) {       // (a search that has ended reads a key it ignores)
-      mid[k] = lo[k] < hi[k] ? lo[k] + ((hi[k] - lo[k]) >> 1) : 0;
-      key[k] = keys[mid[k]];
-    }
-#pragma unroll
-    for (int k = 0; k < 2 * kN; ++k) {
-      // first index with key <= maxk, first index with key < mink
-      const bool up = k % 2 == 0 ? key[k] > range[k / 2].maxk : key[k] >= range[k / 2].mink;
-      if (lo[k] < hi[k]) {
-        lo[k] = up ? mid[k] + 1 : lo[k];
-        hi[k] = up ? hi[k] : mid[k];
-      }
-      open |= lo[k] < hi[k];
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kN; ++i)
-    slice[i] = lo[2 * i + 1] > lo[2 * i] ? make_int2(lo[2 * i], lo[2 * i + 1]) : make_int2(0, 0);
-}
-
 // One block per 64 centres and nine slices of each, a wavefront per slice: which cell row it is, and
 // all that follows from it, is then the same for the lanes, and 64 neighbouring centres look
 // for the slice in the same few columns.  Bound by instruction issue (one lane per centre and
@@ -214,24 +154,6 @@ __global__ void __launch_bounds__(kRowWaves * kWave) nbr_ranges_kernel(
   int2 slice;
   find_slices<1>(&range, keys, &slice);
   ranges[r * ns + c] = slice;
-}
-
-// Whether a candidate lies inside the radius; `live` false: no candidate at all.
-template <int D>
-__device__ __forceinline__ bool within_radius(bool live, const float *diff, const float *ir) {
-  float acc = 0.0f;
-#pragma unroll
-  for (int d = 0; d < D; ++d) {
-    const float sc = diff[d] * ir[d];
-    const float sq = sc * sc;
-    acc = acc + sq;
-  }
-  // The reference tests sqrtf(acc) < 1 (count_neighbors_kernels.cu.cc:83-86).  The
-  // correctly rounded root is monotonic, sqrtf(1) = 1 and the root of the largest
-  // float below 1 is again that float, so acc < 1 decides the same for every
-  // float, infinities and NaN included, without the twenty instructions of an
-  // IEEE square root per candidate.  (A sum of squares is never below 0.)
-  return acc < (live ? 1.0f : 0.0f);
 }
 
 // What a visit of a centre's candidates produces.
@@ -519,12 +441,6 @@ struct NbrWorkspace {
   int64_t *total;
   size_t bytes;
 };
-
-static int offsets_for(int d) {
-  int od = (d - 2 > 1 ? d - 2 : 1) + 1, c = 1;
-  for (int i = 0; i < od; ++i) c *= 3;
-  return c;
-}
 
 static NbrWorkspace carve_nbr_workspace(void *ws, int d, int64_t ns) {
   char *p = (char *)ws;

@@ -1,0 +1,93 @@
+// Cell rows of the sorted grid and the distance test, as the neighbour search and the Poisson-disk
+// selection use them.  For files compiled with -ffp-contract=off (the test decides integer output).
+#pragma once
+#include "common.h"
+
+namespace mccnn {
+
+// Offsets act on dims 0..max(D-2,1); the last dim is covered by the key search.
+template <int D>
+struct OffsetInfo {
+  static constexpr int kDims = (D - 2 > 1 ? D - 2 : 1) + 1;
+  static constexpr int count() {
+    int c = 1;
+    for (int i = 0; i < kDims; ++i) c *= 3;
+    return c;
+  }
+};
+
+inline int offsets_for(int d) {
+  int od = (d - 2 > 1 ? d - 2 : 1) + 1, c = 1;
+  for (int i = 0; i < od; ++i) c *= 3;
+  return c;
+}
+
+// Where a cell row's slice of the sorted points is looked for: in `span` of the keys, from the
+// first key <= maxk up to the first key < mink.  Nothing left to look for where mink > maxk: the
+// slice is `span` itself.
+struct KeyRange {
+  int2 span;
+  int64_t maxk, mink;
+};
+
+// The slices of kN cell rows.  The two ends of all of them are searched side by side: a binary
+// search is a chain of dependent loads (eleven over 2048 keys), and what one lane has to find is
+// kept to one such chain.
+template <int kN>
+__device__ __forceinline__ void find_slices(const KeyRange *range, const int64_t *__restrict__ keys,
+                                            int2 *slice) {
+  int lo[2 * kN], hi[2 * kN];
+  bool open = false;
+#pragma unroll
+  for (int i = 0; i < kN; ++i) {
+    const bool search = range[i].mink <= range[i].maxk;
+    lo[2 * i] = range[i].span.x;
+    lo[2 * i + 1] = search ? range[i].span.x : range[i].span.y;
+    hi[2 * i] = search ? range[i].span.y : range[i].span.x;
+    hi[2 * i + 1] = range[i].span.y;
+    open |= search;
+  }
+  while (open) {
+    open = false;
+    int64_t key[2 * kN];
+    int mid[2 * kN];
+#pragma unroll
+    for (int k = 0; k < 2 * kN; ++k) {       // (a search that has ended reads a key it ignores)
+      mid[k] = lo[k] < hi[k] ? lo[k] + ((hi[k] - lo[k]) >> 1) : 0;
+      key[k] = keys[mid[k]];
+    }
+#pragma unroll
+    for (int k = 0; k < 2 * kN; ++k) {
+      // first index with key <= maxk, first index with key < mink
+      const bool up = k % 2 == 0 ? key[k] > range[k / 2].maxk : key[k] >= range[k / 2].mink;
+      if (lo[k] < hi[k]) {
+        lo[k] = up ? mid[k] + 1 : lo[k];
+        hi[k] = up ? hi[k] : mid[k];
+      }
+      open |= lo[k] < hi[k];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kN; ++i)
+    slice[i] = lo[2 * i + 1] > lo[2 * i] ? make_int2(lo[2 * i], lo[2 * i + 1]) : make_int2(0, 0);
+}
+
+// Whether a candidate lies inside the radius; `live` false: no candidate at all.
+template <int D>
+__device__ __forceinline__ bool within_radius(bool live, const float *diff, const float *ir) {
+  float acc = 0.0f;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const float sc = diff[d] * ir[d];
+    const float sq = sc * sc;
+    acc = acc + sq;
+  }
+  // The reference tests sqrtf(acc) < 1 (count_neighbors_kernels.cu.cc:83-86).  The
+  // correctly rounded root is monotonic, sqrtf(1) = 1 and the root of the largest
+  // float below 1 is again that float, so acc < 1 decides the same for every
+  // float, infinities and NaN included, without the twenty instructions of an
+  // IEEE square root per candidate.  (A sum of squares is never below 0.)
+  return acc < (live ? 1.0f : 0.0f);
+}
+
+}  // namespace mccnn

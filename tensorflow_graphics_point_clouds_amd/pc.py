@@ -480,8 +480,8 @@ class Neighborhood:
     own sorted points) inside `grid` (pylib/pc/Neighborhood.py:218-311)."""
 
     def __init__(self, grid, radius, point_cloud_sample=None, max_neighbors=0, lazy=False):
-        """`lazy` puts the search off until the pair table is first read (a cell-average
-        hierarchy keeps a neighbourhood per level that it never reads itself)."""
+        """`lazy` puts the search off until the pair table is first read (a hierarchy keeps a
+        neighbourhood per level that it never reads itself)."""
         d = grid._point_cloud._dimension
         dev = grid._sorted_points.device
         self._radii = _as_vector(radius, d, dev)
@@ -539,6 +539,11 @@ class Neighborhood:
                                               inv_cell, self._inv_radii, self.max_neighbors)
         self._sorted = (order, pts, ranges, table)
         self._sorted_cells = (bids, cells)
+
+    def _unsearched_own(self):
+        """Whether this is the whole neighbourhood of the grid's own points and its search has been
+        put off so far."""
+        return self._equal_samples and self.max_neighbors == 0 and self._table is None
 
     def _sorted_search(self):
         """(centre order, centres, ranges, pairs) with the centres in the order of their cells."""
@@ -700,16 +705,23 @@ def sample(neighborhood, sample_mode="poisson"):
     """pylib/pc/sampling.py:123-150 -> (PointCloud, original indices or None)."""
     mode = _SAMPLE_MODES[sample_mode.lower()]
     g = neighborhood._grid
-    if mode == 1:
-        # cell averages read the keys only: no reason to run the neighbour search that
-        # the (lazily built) pair table of `neighborhood` would cost
-        dev = g._sorted_points.device
-        pairs = torch.empty((0, 2), dtype=_I32, device=dev)
-        ranges = torch.zeros(g._sorted_points.shape[0], dtype=_I32, device=dev)
+    if mode == 0 and neighborhood._unsearched_own():
+        # the selection from the grid itself: as from the pair table, which it does not need
+        points, ids, keys, ds, num_cells, _, _ = g.search_tensors()
+        pts, bids, idx = _lib.host().sampling_grid(points, ids, keys, ds, num_cells,
+                                                   neighborhood._inv_radii)
     else:
-        pairs, ranges = neighborhood._neighbors, neighborhood._samples_neigh_ranges
-    pts, bids, idx = tfg_custom_ops.sampling(
-        g._sorted_points, g._sorted_batch_ids, g._sorted_keys, g._num_cells, pairs, ranges, mode)
+        if mode == 1:
+            # cell averages read the keys only: no reason to run the neighbour search that
+            # the (lazily built) pair table of `neighborhood` would cost
+            dev = g._sorted_points.device
+            pairs = torch.empty((0, 2), dtype=_I32, device=dev)
+            ranges = torch.zeros(g._sorted_points.shape[0], dtype=_I32, device=dev)
+        else:
+            pairs, ranges = neighborhood._neighbors, neighborhood._samples_neigh_ranges
+        pts, bids, idx = tfg_custom_ops.sampling(
+            g._sorted_points, g._sorted_batch_ids, g._sorted_keys, g._num_cells, pairs, ranges,
+            mode)
     original = None
     if mode == 0:
         original = _lib.host().gather_i32(g._sorted_indices, idx)
@@ -724,7 +736,7 @@ def poisson_disk_sampling(point_cloud, radius=None, neighborhood=None, return_id
         raise ValueError("Missing Argument! Either radius or neighborhood must be given!")
     if neighborhood is None:
         radii = _as_vector(radius, point_cloud._dimension, point_cloud._points.device)
-        neighborhood = Neighborhood(Grid(point_cloud, radii), radii)
+        neighborhood = Neighborhood(Grid(point_cloud, radii), radii, lazy=True)
     cloud, ids = sample(neighborhood, "poisson")
     return (cloud, ids) if return_ids else cloud
 
@@ -753,7 +765,7 @@ class PointHierarchy:
             cs = _as_vector(cs, point_cloud._dimension, point_cloud._points.device)
             self._cell_sizes.append(cs)
             grid = Grid(cur, cs)
-            nbh = Neighborhood(grid, cs, lazy=_SAMPLE_MODES[sample_mode.lower()] == 1)
+            nbh = Neighborhood(grid, cs, lazy=True)
             cur, idx = sample(nbh, sample_mode)
             self._neighborhoods.append(nbh)
             self._point_clouds.append(cur)

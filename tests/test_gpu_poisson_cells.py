@@ -24,3 +24,29 @@ def test_poisson_selection_in_crowded_cells(oracle, d, n, cell, radius):
     _, _, got = ops.sampling(dev(g.sorted_points), dev(g.sorted_batch_ids), dev(g.sorted_keys),
                              dev(g.num_cells), dev(nbh.neighbors), dev(nbh.ranges), 0)
     assert np.array_equal(got.cpu().numpy(), expect)
+
+
+@pytest.mark.parametrize("d,n,cell,radius", [
+    (3, 1, 0.3, 0.3), (3, 5, 2.0, 0.05), (3, 3000, 0.3, 0.3), (3, 3000, 0.4, 0.1),
+    (3, 1500, 2.0, 0.07), (3, 3000, 0.4, 0.04), (3, 20000, 0.09, 0.09), (3, 20000, 0.2, 0.05),
+    (3, 3000, 0.1, 0.25), (2, 2500, 0.4, 0.1), (2, 2500, 0.25, 0.25), (2, 30000, 0.02, 0.02),
+    (4, 1500, 0.6, 0.2), (4, 1500, 0.5, 0.5), (5, 800, 0.7, 0.7)])
+def test_selection_from_the_grid_is_that_from_the_table(d, n, cell, radius):
+    """Selected points around a cell that fit the registers, do not, or stop fitting at a point of
+    the cell; with and without a column table; points that coincide or are no numbers."""
+    from tensorflow_graphics_point_clouds_amd import pc
+    gen = torch.Generator(device="cuda").manual_seed(n + d)
+    pts = torch.rand((2 * n, d), device="cuda", generator=gen)
+    pts[n // 2] = pts[0]
+    if n > 1000:
+        pts[n + 3, 0] = float("nan")
+    bids = torch.arange(2, device="cuda").repeat_interleave(n).int()
+    grid = pc.Grid(pc.PointCloud(pts, bids, 2), cell)
+    own = pc.Neighborhood(grid, radius, lazy=True)
+    assert own._unsearched_own()
+    got, ids = pc.sample(own, "poisson")
+    assert own._unsearched_own()
+    expect, expect_ids = pc.sample(pc.Neighborhood(grid, radius), "poisson")
+    assert torch.equal(ids, expect_ids)
+    assert torch.equal(got._points.nan_to_num(7.0), expect._points.nan_to_num(7.0))
+    assert torch.equal(got._batch_ids, expect._batch_ids)
