@@ -188,6 +188,22 @@ int mccnn_gather_rows_padded(mccnn_stream_t stream, int64_t num_rows, const int3
                              const float *src, int64_t src_stride, int first_col, int num_cols,
                              int num_cols_out, float *out);
 
+/* Two sub-layers of 16 basis columns each in one pass over the pairs: num_mlps kernel MLPs over
+ * both, num_features channels each -- the same for both, or with own_features feature rows
+ * [2, num_features].  out [num_samples, 2, num_features, 16]. */
+int mccnn_mc_conv_project_pair(mccnn_stream_t stream, int num_dims, int64_t num_pts,
+                               const float *points_in, int num_features, int own_features,
+                               const float *features, int64_t num_samples,
+                               const float *points_out, int64_t num_neighbors,
+                               const int32_t *neighbors, const int32_t *ranges,
+                               const float *inv_radii, int num_mlps, int activation,
+                               const float *weights, const float *biases, const float *pdf,
+                               const int32_t *out_rows, float *out);
+/* Two products side by side: x [num_rows, 2, num_cols_in], w [2, num_cols_in, num_cols_out],
+ * out [num_rows, 2, num_cols_out]; sums as mccnn_final_product. */
+int mccnn_final_product_pair(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
+                             const float *x, int num_cols_out, const float *w, float *out);
+
 /* The weights of a convolution layer as its kernels read them, one launch: from the final
  * weights [L, num_features * hidden, group_features] (MCConv.py:180-187; L = 1 for
  * kernel-point convolutions) the kernel MLPs first_mlp .. first_mlp + num_mlps - 1 as a dense
@@ -211,6 +227,21 @@ int mccnn_unpack_layer_grads(mccnn_stream_t stream, int num_dims, int num_featur
                              const float *dense_grads, const float *kernel_weight_grads,
                              const float *kernel_bias_grads, float *final_grads_out,
                              float *weight_grads_out, float *bias_grads_out);
+/* Two sub-layers of num_mlps kernel MLPs each: w_out [2, (c,k), f], w2_out [2, (f,k), c], the
+ * kernel MLPs one after the other, and all_out [(c,k), f] over both (NULL to skip).  _unpack_:
+ * dense_grads [padded_features, 2, (f,k)]. */
+int mccnn_pack_layer_weights_pair(mccnn_stream_t stream, int num_dims, int num_features, int hidden,
+                                  int group_features, int num_mlps, int padded_features,
+                                  int padded_hidden, int padded_group, const float *final_weights,
+                                  const float *kernel_weights, const float *kernel_biases,
+                                  float *w_out, float *w2_out, float *kernel_weights_out,
+                                  float *kernel_biases_out, float *all_out);
+int mccnn_unpack_layer_grads_pair(mccnn_stream_t stream, int num_dims, int num_features, int hidden,
+                                  int group_features, int num_mlps, int padded_features,
+                                  int padded_hidden, int padded_group, const float *dense_grads,
+                                  const float *kernel_weight_grads,
+                                  const float *kernel_bias_grads, float *final_grads_out,
+                                  float *weight_grads_out, float *bias_grads_out);
 /* The same with dense_grads as [f, (c,k)], any number of rows f behind the layer's. */
 int mccnn_unpack_layer_grads_wt(mccnn_stream_t stream, int num_dims, int num_features, int hidden,
                                 int group_features, int first_mlp, int num_mlps,

@@ -831,6 +831,62 @@ Tensor cut_columns(const Tensor &x, int64_t cols) {
   return x.size(1) == cols ? x : x.slice(1, 0, cols).contiguous();
 }
 
+// Whether the layer's two sub-layers run side by side, one launch of everything for both: inputs
+// whose products keep the register-resident kernel, where a pass is chains of loads and launches.
+// Per output element the sums are those of the sub-layers on their own.
+// Layer of 6 -> 32 channels, 4 x 8 hidden units, 61 k points of 28 pairs: 592 -> 490 us for the pass, 53 -> 39 launches.
+bool paired(const Plan &p, int64_t n_out, int64_t n_in, bool grads) {
+  const int64_t f = p.f(), r = p.c_pad * p.k();
+  if (p.mlps != 2 * p.per || p.k() != 16 || p.g_pad != p.g || p.cols() != f ||
+      n_in * 2 * std::max(p.c_pad, f) >= (int64_t)1 << 30 || n_out * 2 * f >= (int64_t)1 << 30 ||
+      product_kind(n_out, r, f) != Product::kRegisters)
+    return false;
+  return !grads || (narrow_columns(p, n_out) == 0 &&
+                    product_kind(n_in, f * 16, p.c_pad) == Product::kRegisters &&
+                    product_kind(n_in, 2 * f * 16, p.c_pad) == Product::kRegisters &&
+                    mccnn_projection_grad_product_supported((int)(2 * f), (int)(2 * r)) &&
+                    mccnn_weight_grad_product_supported((int)p.c_pad, (int)(2 * f * 16)));
+}
+
+// Both sub-layers' weights: w [2, r, f] where the forward product reads them, all [2 r, 2 f] as w
+// of the saved ones, w2 [2 f k, c].
+Packed pack_pair(const Plan &p, const Tensor &final_weights, const Tensor &kw, const Tensor &kb,
+                 bool grads, Tensor *forward) {
+  Packed out;
+  const int64_t k = p.k(), f = p.f(), r = p.c_pad * k;
+  *forward = empty_f32({2, r, f}, final_weights);
+  if (grads) {
+    out.w = empty_f32({2 * r, 2 * f}, final_weights);
+    out.w2 = empty_f32({2 * f * k, p.c_pad}, final_weights);
+  }
+  out.kw = empty_f32({p.mlps, p.dims, p.h_pad}, kw);
+  out.kb = empty_f32({2 * k}, kb);
+  hipStream_t s = current_stream();
+  Region t("pack_layer_weights", s);
+  check(mccnn_pack_layer_weights_pair(s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, (int)p.per,
+                                      (int)p.c_pad, (int)p.h_pad, (int)p.g_pad,
+                                      f32(final_weights), f32(kw), f32(kb), f32(*forward),
+                                      f32(out.w2), f32(out.kw), f32(out.kb), f32(out.w)));
+  return out;
+}
+
+// Projections of both sub-layers, [n, 2, channels, 16]; `own`: feats hold channels of each.
+Tensor mc_project_pair(const Plan &p, const Packed &w, const Tensor &feats, bool own,
+                       const Tensor &pin, const Tensor &pout, const Tensor &table,
+                       const Tensor &ranges, const Tensor &inv_radii, const Tensor &pdf,
+                       const Tensor &out_rows) {
+  const int64_t c = own ? feats.size(1) / 2 : feats.size(1);
+  Tensor out = empty_f32({ranges.size(0), 2 * c * p.k()}, feats);
+  hipStream_t s = current_stream();
+  Region t("mc_conv_project", s);
+  check(mccnn_mc_conv_project_pair(s, (int)p.dims, feats.size(0), f32(pin), (int)c, own ? 1 : 0,
+                                   f32(feats), ranges.size(0), f32(pout), table.size(0),
+                                   i32(table), i32(ranges), f32(inv_radii), (int)p.mlps,
+                                   (int)p.act, f32(w.kw), f32(w.kb), f32(pdf), i32(out_rows),
+                                   f32(out)));
+  return out;
+}
+
 // The whole Monte-Carlo convolution (MCConv.py:137-194) on the grid-ordered view.  Forward:
 // fused basis + projection, product with the final weights.  The projection writes its rows (of
 // C K floats) to the centres' original positions, which costs it nothing; the product's rows of
@@ -852,7 +908,22 @@ struct McConv : torch::autograd::Function<McConv> {
     const bool narrow = grads && narrow_columns(p, n_out) > 0;
     variable_list saved = {feats, kw, kb, final_weights,
                            p.c == p.c_pad && !narrow ? features : Tensor()};
-    for (int64_t first = 0; first < p.mlps; first += p.per) {
+    const bool pair = paired(p, n_out, feats.size(0), grads);
+    if (pair) {
+      Tensor forward;
+      const Packed w = pack_pair(p, final_weights, kw, kb, grads, &forward);
+      const Tensor proj = mc_project_pair(p, w, feats, false, geo->points_in, geo->points_out,
+                                          geo->table, geo->ranges, geo->inv_radii, geo->pdf,
+                                          geo->centre_rows);
+      Tensor out = empty_f32({n_out, 2 * p.f()}, feats);
+      hipStream_t s = current_stream();
+      Region t("final_product", s);
+      check(mccnn_final_product_pair(s, n_out, (int)(proj.size(1) / 2), f32(proj), (int)p.f(),
+                                     f32(forward), f32(out)));
+      outs.push_back(out);
+      if (grads) w.save(saved);
+    }
+    for (int64_t first = 0; first < p.mlps && !pair; first += p.per) {
       const Packed w = pack(p, first, final_weights, kw, kb, n_out, feats.size(0), grads,
                             grads && !narrow);
       const Tensor proj = mc_project(p, w, feats, geo->points_in, geo->points_out, geo->table,
@@ -891,7 +962,44 @@ struct McConv : torch::autograd::Function<McConv> {
     const int64_t wide = narrow_columns(p, n_out);
     if (wide > 0 && want_feat) dfeat = empty_f32({geo->ranges_t.size(0), p.c}, feats);
     hipStream_t s = current_stream();
-    for (int64_t first = 0, i = 0; first < p.mlps; first += p.per, ++i) {
+    const bool pair = saved.size() == 5 + Packed::kTensors && p.mlps == 2 * p.per;
+    if (pair) {
+      const Packed w = Packed::saved(saved, 5);
+      const int64_t f2 = 2 * p.f();
+      const Tensor up = geo->centre_rows.defined() ? gather_rows(dout, geo->centre_rows, 0, f2, f2)
+                                                   : dout;
+      Tensor dkw_pad, dkb_pad, ddense;
+      if (want_kernel) {
+        const Tensor dproj = projection_grad_product(up, w.w);
+        Tensor ws = workspace(mccnn_mc_conv_project_grads_workspace_bytes((int)p.dims, (int)(2 * k),
+                                                                          n_out), feats);
+        dkw_pad = empty_f32({p.mlps, p.dims, p.h_pad}, feats);
+        dkb_pad = empty_f32({2 * k}, feats);
+        Region t("mc_conv_project_grads", s);
+        check(mccnn_mc_conv_project_grads(
+            s, (int)p.dims, feats.size(0), f32(geo->points_in), (int)p.c_pad, f32(feats), n_out,
+            f32(geo->points_out), geo->table.size(0), i32(geo->table), i32(geo->ranges),
+            f32(geo->inv_radii), (int)(2 * k), (int)p.mlps, (int)p.act, f32(w.kw), f32(w.kb),
+            f32(geo->pdf), f32(dproj), ws.data_ptr(), ws.numel(), nullptr, nullptr, nullptr,
+            nullptr, f32(dkw_pad), f32(dkb_pad)));
+      }
+      if (want_feat || want_final) {
+        const bool in_place = features.defined();
+        const Tensor q = mc_project_pair(p, w, up, true, geo->points_out, geo->points_in,
+                                         geo->table_t, geo->ranges_t, geo->neg_inv_radii,
+                                         geo->pdf_t, in_place ? geo->point_rows : Tensor());
+        if (want_feat) dfeat = transposed_product(q, w, in_place ? Tensor() : geo->point_rows);
+        if (want_final) ddense = weight_grad_product(in_place ? features : feats, q);
+      }
+      if (want_final || want_kernel) {
+        Region t("unpack_layer_grads", s);
+        check(mccnn_unpack_layer_grads_pair(
+            s, (int)p.dims, (int)p.c, (int)p.h, (int)p.g, (int)p.per, (int)p.c_pad, (int)p.h_pad,
+            (int)p.g_pad, f32(ddense), f32(dkw_pad), f32(dkb_pad), f32(dfinal), f32(dkw),
+            f32(dkb)));
+      }
+    }
+    for (int64_t first = 0, i = 0; first < p.mlps && !pair; first += p.per, ++i) {
       const Packed w = Packed::saved(saved, 5 + i * Packed::kTensors);
       const Tensor up =
           geo->centre_rows.defined() || p.g_pad != p.g || p.per != p.mlps || wide > p.f()

@@ -54,10 +54,25 @@ __global__ void __launch_bounds__(256) pack_layer_weights_kernel(
     LayerShapeArgs a, int D, const float *__restrict__ src, const float *__restrict__ kw_src,
     const float *__restrict__ kb_src, float *__restrict__ w, float *__restrict__ wt,
     float *__restrict__ w2, float *__restrict__ w2t, float *__restrict__ kw,
-    float *__restrict__ kb) {
+    float *__restrict__ kb, float *__restrict__ all) {
   const int K = a.mlps * a.Hp, F = a.mlps * a.Gp, size = a.Cp * K * F;
-  const int which = blockIdx.y;
+  const int which = blockIdx.y, part = blockIdx.z;      // (a part: the next `mlps` kernel MLPs)
+  if (which == 5) {                                     // all of them as one dense matrix [(c,k), f]
+    const int parts = gridDim.z, Fa = parts * F, Ka = parts * K;
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < size * parts;
+         t += gridDim.x * blockDim.x) {
+      const int e = part * size * parts + t;            // a part's share of the size * parts^2
+      all[e] = dense_element(a, src, e / Fa / Ka, e / Fa % Ka, e % Fa);
+    }
+    return;
+  }
+  a.first += part * a.mlps;
   float *dst = which == 0 ? w : which == 1 ? wt : which == 2 ? w2 : which == 3 ? w2t : nullptr;
+  if (dst) dst += (int64_t)part * size;
+  if (kw) {
+    kw += part * D * K;
+    kb += part * K;
+  }
   for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < size; t += gridDim.x * blockDim.x) {
     if (dst == nullptr) break;
     int c, k, f;
@@ -90,7 +105,11 @@ __global__ void __launch_bounds__(256) unpack_layer_grads_kernel(
     LayerShapeArgs a, int D, int c_stride, int f_stride, const float *__restrict__ ddense,
     const float *__restrict__ dkw_src, const float *__restrict__ dkb_src, float *__restrict__ dfinal, float *__restrict__ dkw,
     float *__restrict__ dkb) {
-  const int per = a.C * a.H * a.G, size = a.mlps * per;
+  const int per = a.C * a.H * a.G, size = a.mlps * per, part = blockIdx.z;
+  a.first += part * a.mlps;                    // (f of the parts one after the other)
+  ddense += (int64_t)part * a.mlps * a.Gp * f_stride;
+  dkw_src += part * D * a.mlps * a.Hp;
+  dkb_src += part * a.mlps * a.Hp;
   if (dfinal)
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < size; t += gridDim.x * blockDim.x) {
       const int g = t % a.G, h = t / a.G % a.H, c = t / a.G / a.H % a.C, m = t / per;
@@ -148,6 +167,30 @@ extern "C" int mccnn_gather_rows_padded(mccnn_stream_t stream, int64_t num_rows,
   return MCCNN_OK;
 }
 
+static int pack_layer_weights(mccnn_stream_t stream, int num_dims, const LayerShapeArgs &a,
+                              int parts, const float *final_weights, const float *kernel_weights,
+                              const float *kernel_biases, float *w_out, float *wt_out,
+                              float *w2_out, float *w2t_out, float *kernel_weights_out,
+                              float *kernel_biases_out, float *all_out) {
+  int rc = check_shape("pack_layer_weights", a);
+  if (rc != MCCNN_OK) return rc;
+  const bool kernel = kernel_weights_out != nullptr;
+  MCCNN_REQUIRE(final_weights && (!kernel || (kernel_weights && kernel_biases &&
+                                              kernel_biases_out)),
+                "pack_layer_weights received a null tensor");
+  const int64_t size = (int64_t)a.Cp * a.mlps * a.Hp * a.mlps * a.Gp;
+  MCCNN_REQUIRE(size * parts * parts < ((int64_t)1 << 28),
+                "pack_layer_weights expects fewer than 2^28 weights");
+  const unsigned grid = blocks_for(size > (1 << 20) ? (1 << 20) : size, 256);
+  const unsigned outputs = all_out ? 6 : kernel ? 5 : w2t_out ? 4 : w2_out ? 3 : wt_out ? 2 : 1;
+  hipLaunchKernelGGL(pack_layer_weights_kernel, dim3(grid, outputs, (unsigned)parts), dim3(256), 0,
+                     as_stream(stream), a, num_dims, final_weights, kernel_weights, kernel_biases,
+                     w_out, wt_out, w2_out, w2t_out, kernel_weights_out, kernel_biases_out,
+                     all_out);
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
 extern "C" int mccnn_pack_layer_weights(mccnn_stream_t stream, int num_dims, int num_features,
                                         int hidden, int group_features, int first_mlp,
                                         int num_mlps, int padded_features, int padded_hidden,
@@ -158,28 +201,29 @@ extern "C" int mccnn_pack_layer_weights(mccnn_stream_t stream, int num_dims, int
                                         float *kernel_biases_out) {
   const LayerShapeArgs a = {num_features, hidden, group_features, first_mlp, num_mlps,
                             padded_features, padded_hidden, padded_group};
-  int rc = check_shape("pack_layer_weights", a);
-  if (rc != MCCNN_OK) return rc;
-  const bool kernel = kernel_weights_out != nullptr;
-  MCCNN_REQUIRE(final_weights && (!kernel || (kernel_weights && kernel_biases &&
-                                              kernel_biases_out)),
-                "pack_layer_weights received a null tensor");
-  const int64_t size = (int64_t)a.Cp * a.mlps * a.Hp * a.mlps * a.Gp;
-  const unsigned grid = blocks_for(size > (1 << 20) ? (1 << 20) : size, 256);
-  hipLaunchKernelGGL(pack_layer_weights_kernel, dim3(grid, kernel ? 5 : w2t_out ? 4 : w2_out ? 3
-                                                                        : wt_out ? 2 : 1),
-                     dim3(256), 0, as_stream(stream), a, num_dims, final_weights, kernel_weights,
-                     kernel_biases, w_out, wt_out, w2_out, w2t_out, kernel_weights_out,
-                     kernel_biases_out);
-  MCCNN_LAUNCH_CHECK();
-  return MCCNN_OK;
+  return pack_layer_weights(stream, num_dims, a, 1, final_weights, kernel_weights, kernel_biases,
+                            w_out, wt_out, w2_out, w2t_out, kernel_weights_out, kernel_biases_out,
+                            nullptr);
+}
+
+extern "C" int mccnn_pack_layer_weights_pair(
+    mccnn_stream_t stream, int num_dims, int num_features, int hidden, int group_features,
+    int num_mlps, int padded_features, int padded_hidden, int padded_group,
+    const float *final_weights, const float *kernel_weights, const float *kernel_biases,
+    float *w_out, float *w2_out, float *kernel_weights_out, float *kernel_biases_out,
+    float *all_out) {
+  const LayerShapeArgs a = {num_features, hidden, group_features, 0, num_mlps,
+                            padded_features, padded_hidden, padded_group};
+  return pack_layer_weights(stream, num_dims, a, 2, final_weights, kernel_weights, kernel_biases,
+                            w_out, nullptr, w2_out, nullptr, kernel_weights_out, kernel_biases_out,
+                            all_out);
 }
 
 static int unpack_layer_grads(mccnn_stream_t stream, int num_dims, const LayerShapeArgs &a,
                               bool by_output, const float *dense_grads,
                               const float *kernel_weight_grads, const float *kernel_bias_grads,
                               float *final_grads_out, float *weight_grads_out,
-                              float *bias_grads_out) {
+                              float *bias_grads_out, int parts = 1) {
   int rc = check_shape("unpack_layer_grads", a);
   if (rc != MCCNN_OK) return rc;
   MCCNN_REQUIRE((!final_grads_out || dense_grads) &&
@@ -189,8 +233,8 @@ static int unpack_layer_grads(mccnn_stream_t stream, int num_dims, const LayerSh
   const int64_t size = (int64_t)a.mlps * a.C * a.H * a.G;
   const unsigned grid = blocks_for(size > (1 << 20) ? (1 << 20) : size, 256);
   const int K = a.mlps * a.Hp, F = a.mlps * a.Gp;
-  hipLaunchKernelGGL(unpack_layer_grads_kernel, dim3(grid), dim3(256), 0, as_stream(stream), a,
-                     num_dims, by_output ? K : F * K, by_output ? a.Cp * K : K, dense_grads,
+  hipLaunchKernelGGL(unpack_layer_grads_kernel, dim3(grid, 1, (unsigned)parts), dim3(256), 0,
+                     as_stream(stream), a, num_dims, by_output ? K : parts * F * K, by_output ? a.Cp * K : K, dense_grads,
                      kernel_weight_grads, kernel_bias_grads, final_grads_out, weight_grads_out,
                      bias_grads_out);
   MCCNN_LAUNCH_CHECK();
@@ -221,4 +265,15 @@ extern "C" int mccnn_unpack_layer_grads_wt(mccnn_stream_t stream, int num_dims, 
                             padded_features, padded_hidden, padded_group};
   return unpack_layer_grads(stream, num_dims, a, true, dense_grads, kernel_weight_grads,
                             kernel_bias_grads, final_grads_out, weight_grads_out, bias_grads_out);
+}
+
+extern "C" int mccnn_unpack_layer_grads_pair(
+    mccnn_stream_t stream, int num_dims, int num_features, int hidden, int group_features,
+    int num_mlps, int padded_features, int padded_hidden, int padded_group,
+    const float *dense_grads, const float *kernel_weight_grads, const float *kernel_bias_grads,
+    float *final_grads_out, float *weight_grads_out, float *bias_grads_out) {
+  const LayerShapeArgs a = {num_features, hidden, group_features, 0, num_mlps,
+                            padded_features, padded_hidden, padded_group};
+  return unpack_layer_grads(stream, num_dims, a, false, dense_grads, kernel_weight_grads,
+                            kernel_bias_grads, final_grads_out, weight_grads_out, bias_grads_out, 2);
 }

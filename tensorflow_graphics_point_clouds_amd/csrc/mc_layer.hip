@@ -60,6 +60,10 @@ struct DenseStrides {
   int64_t ldx = 0, ldw = 0, ldo = 0;
   int r_total = 0;       // reduction length of the whole product, walked in blocks of R
   int f_block = 0;       // columns per blockIdx.y
+  // several products side by side: column blocks of each (0: one product), and how far apart
+  // their rows of x, their weights and their columns of out lie
+  int f_blocks = 0, x_step = 0, o_step = 0;
+  int64_t w_step = 0;
 };
 
 template <int kCPL, int FT, int D, class Basis, bool kDense = false>
@@ -86,8 +90,11 @@ __device__ __forceinline__ void layer_body(int64_t n_out, const float *__restric
   const int64_t ldo = kDense && ld.ldo ? ld.ldo : F;
   const int r_total = kDense && ld.r_total ? ld.r_total : R;
   if constexpr (kDense) {           // this block's columns of a wider product
-    w += (int64_t)blockIdx.y * ld.f_block;
-    out += (int64_t)blockIdx.y * ld.f_block;
+    const int product = ld.f_blocks ? blockIdx.y / ld.f_blocks : 0;
+    const int block = blockIdx.y - product * ld.f_blocks;
+    w += product * ld.w_step + (int64_t)block * ld.f_block;
+    out += (int64_t)product * ld.o_step + (int64_t)block * ld.f_block;
+    feat += (int64_t)product * ld.x_step;
   }
   const float *arow = tile + col * S::kTileStride + slice * S::kSliceRows + quarter * kSteps;
   const int64_t tiles = (n_out + kLayerWaves - 1) / kLayerWaves;
@@ -417,6 +424,55 @@ static bool product_blocks(int R, int F, int *rb, int *fb) {
   return false;
 }
 
+// The register-resident product, `products` of them side by side: x [N, products, R],
+// w [products, R, F], out [N, products, F].  What is summed in which order goes by one of them.
+static int launch_final_product(hipStream_t s, int64_t num_rows, int R, const float *x, int F,
+                                int num_cols, const float *w, const int32_t *out_rows, float *out,
+                                int products) {
+  int device = 0, cus = 0, rc = MCCNN_OK;
+  MCCNN_HIP_CHECK(hipGetDevice(&device));
+  MCCNN_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  const int64_t tiles = (num_rows + kLayerWaves - 1) / kLayerWaves;
+  int rb = 0, fb = 0;
+  const bool fits = product_blocks(R, num_cols, &rb, &fb) && F % fb == 0;
+  const int cols = fits ? num_cols : F;
+  if (!fits) product_blocks(R, F, &rb, &fb);
+  // A small input leaves compute units idle: narrower column blocks with longer reduction
+  // blocks then give more blocks of threads, each walking fewer blocks of the reduction
+  // (1500 rows x 4096 x 256: 8 visits of 512 rows of w per block of threads become 4 of 1024)
+  while (fb > 16 && rb < 1024 && R % (2 * rb) == 0 && tiles * (cols / (fb / 2)) <= cus) {
+    fb /= 2;
+    rb *= 2;
+  }
+  // out[:, f0:f0+fb] = sum over the reduction blocks r0 of x[:, r0:r0+rb] W[r0:r0+rb, f0:f0+fb]:
+  // one launch, column block f0 = blockIdx.y * fb, every block walking the reduction blocks
+  // in order for its own tiles
+  DenseStrides ld;
+  ld.ldx = (int64_t)products * R;
+  ld.ldw = F;
+  ld.ldo = (int64_t)products * F;
+  ld.r_total = R;
+  ld.f_block = fb;
+  ld.f_blocks = products > 1 ? cols / fb : 0;
+  ld.x_step = R;
+  ld.o_step = F;
+  ld.w_step = (int64_t)R * F;
+  const int col_blocks = cols / fb * products;
+  // one block per compute unit in all (the register-resident weights and the LDS tile
+  // fill it), shared among the column blocks; never more blocks than tiles
+  int64_t per = cus / col_blocks < 1 ? 1 : cus / col_blocks;
+  if (per > tiles) per = tiles;
+  const unsigned blocks = (unsigned)per;
+  MCCNN_LAYER_SHAPE_SWITCH(rb / kFusedK, fb,
+                           rc = launch_layer(final_product_kernel<CPL, FT>, s,
+                                             dim3(blocks, (unsigned)col_blocks),
+                                             LayerShape<CPL, FT>::kLdsBytes, num_rows, x, w,
+                                             out_rows, out, ld));
+  if (rc != MCCNN_OK) return rc;
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
 extern "C" int mccnn_final_product_supported(int num_cols_in, int num_cols_out) {
   int rb = 0, fb = 0;
   return num_cols_in <= 8192 && num_cols_out <= 1024 &&
@@ -449,11 +505,10 @@ extern "C" int mccnn_final_product_padded(mccnn_stream_t stream, int64_t num_row
   if (num_rows == 0) return MCCNN_OK;
   MCCNN_REQUIRE(x && w && out, "final_product received a null tensor");
   hipStream_t s = as_stream(stream);
-  int device = 0, cus = 0, rc = MCCNN_OK;
+  int device = 0, cus = 0;
   MCCNN_HIP_CHECK(hipGetDevice(&device));
   MCCNN_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   const int R = num_cols_in, F = num_cols_out;
-  const int64_t tiles = (num_rows + kLayerWaves - 1) / kLayerWaves;
   // weights beyond a block's registers: the tiled product, once its 128- or 256-row tiles give
   // every compute unit a block (below that a launch is a few blocks walking the whole
   // reduction alone: 170 us for 400 rows x 4096 x 256 against 20 us for the blocked
@@ -462,40 +517,22 @@ extern "C" int mccnn_final_product_padded(mccnn_stream_t stream, int64_t num_row
       (num_rows + tile_product_rows(F) - 1) / tile_product_rows(F) *
               (F / (F % 128 == 0 ? 128 : 64)) >= cus)
     return launch_tile_product(s, num_rows, R, x, F, w, false, out_rows, out);
-  int rb = 0, fb = 0;
-  const bool fits = product_blocks(R, num_cols, &rb, &fb) && F % fb == 0;
-  const int cols = fits ? num_cols : F;
-  if (!fits) product_blocks(R, F, &rb, &fb);
-  // A small input leaves compute units idle: narrower column blocks with longer reduction
-  // blocks then give more blocks of threads, each walking fewer blocks of the reduction
-  // (1500 rows x 4096 x 256: 8 visits of 512 rows of w per block of threads become 4 of 1024)
-  while (fb > 16 && rb < 1024 && R % (2 * rb) == 0 && tiles * (cols / (fb / 2)) <= cus) {
-    fb /= 2;
-    rb *= 2;
-  }
-  // out[:, f0:f0+fb] = sum over the reduction blocks r0 of x[:, r0:r0+rb] W[r0:r0+rb, f0:f0+fb]:
-  // one launch, column block f0 = blockIdx.y * fb, every block walking the reduction blocks
-  // in order for its own tiles
-  DenseStrides ld;
-  ld.ldx = R;
-  ld.ldw = F;
-  ld.ldo = F;
-  ld.r_total = R;
-  ld.f_block = fb;
-  const int col_blocks = cols / fb;
-  // one block per compute unit in all (the register-resident weights and the LDS tile
-  // fill it), shared among the column blocks; never more blocks than tiles
-  int64_t per = cus / col_blocks < 1 ? 1 : cus / col_blocks;
-  if (per > tiles) per = tiles;
-  const unsigned blocks = (unsigned)per;
-  MCCNN_LAYER_SHAPE_SWITCH(rb / kFusedK, fb,
-                           rc = launch_layer(final_product_kernel<CPL, FT>, s,
-                                             dim3(blocks, (unsigned)col_blocks),
-                                             LayerShape<CPL, FT>::kLdsBytes, num_rows, x, w,
-                                             out_rows, out, ld));
-  if (rc != MCCNN_OK) return rc;
-  MCCNN_LAUNCH_CHECK();
-  return MCCNN_OK;
+  return launch_final_product(s, num_rows, R, x, F, num_cols, w, out_rows, out, 1);
+}
+
+extern "C" int mccnn_final_product_pair(mccnn_stream_t stream, int64_t num_rows, int num_cols_in,
+                                        const float *x, int num_cols_out, const float *w,
+                                        float *out) {
+  MCCNN_REQUIRE(mccnn_final_product_supported(num_cols_in, num_cols_out),
+                "final_product_pair supports a multiple of 256 (at most 8192) input columns and a "
+                "multiple of 16 (at most 1024) output columns (got %d x %d)", num_cols_in,
+                num_cols_out);
+  MCCNN_REQUIRE(num_rows >= 0 && num_rows < ((int64_t)1 << 31),
+                "final_product_pair expects a size in [0, 2^31)");
+  if (num_rows == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(x && w && out, "final_product_pair received a null tensor");
+  return launch_final_product(as_stream(stream), num_rows, num_cols_in, x, num_cols_out,
+                              num_cols_out, w, nullptr, out, 2);
 }
 
 // The same product with the weights given transposed, wt [F, R] (rows of w^T are
