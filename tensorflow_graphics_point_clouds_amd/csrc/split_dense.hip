@@ -283,7 +283,7 @@ int launch_nt_split(hipStream_t s, int64_t n, int F, const float *x, int R, cons
 
 // out[out_rows[n] or n, :] = x[n, :] * w for x [N, R] and the weights given transposed,
 // wt [F, R]: the tiled product on the bf16 pipe.  A block of four wavefronts owns a BM x BN
-// tile of the output (128 x 128, 256 x 128 or 256 x 64), every wavefront 64 x 64 or 128 x 64
+// tile of the output (128 x 128, 256 x 128, 256 x 64 or 128 x 64), every wavefront 64 x 64, 128 x 64 or 32 x 64
 // of it as accumulator tiles of 32 x 32, and walks the reduction in chunks of 32.  The chunk of x and
 // of wt for the next step is fetched into registers while the current one is multiplied;
 // the thread that fetched eight consecutive values splits them once and parks the three
@@ -403,15 +403,24 @@ int launch_tile_split(hipStream_t s, int64_t n, int R, const float *x, int F, co
   int device = 0, cus = 0;
   MCCNN_HIP_CHECK(hipGetDevice(&device));
   MCCNN_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-  const bool tall = bn == 128 && (n + 255) / 256 * (F / 128) >= 2 * (int64_t)cus;
-  const int bm = tall ? 256 : 16384 / bn;
+  // 64 columns: tiles of 256 rows while those of 128 rows would not fill the four places that
+  // compute units have for them one and a half times (98 765 x 512: 62 against 66 us, 120 011 x
+  // 1024: 252 against 259); beyond that four wavefronts per SIMD are worth more than splitting the
+  // weights' chunk once per 128 rows costs (200 003 x 1024: 249 -> 234 us, 763 063 x 1024: 820 -> 783).
+  // (The weights split once for all tiles, by a kernel of their own: 803 us, and 2.29 against 2.33 ms
+  // for 128 columns.)
+  const bool tall = bn == 128 ? (n + 255) / 256 * (F / 128) >= 2 * (int64_t)cus
+                              : (n + 127) / 128 * (F / 64) < 6 * (int64_t)cus;
+  const int bm = tall ? 256 : 128;
   const dim3 block(kSplitThreads), grid((unsigned)((n + bm - 1) / bm * (F / bn)));
-  if (tall)
+  if (bn == 128 && tall)
     hipLaunchKernelGGL((tile_split_kernel<128, 256>), grid, block, 0, s, n, R, F, x, wt, out_rows, out);
   else if (bn == 128)
     hipLaunchKernelGGL((tile_split_kernel<128>), grid, block, 0, s, n, R, F, x, wt, out_rows, out);
+  else if (tall)
+    hipLaunchKernelGGL((tile_split_kernel<64, 256>), grid, block, 0, s, n, R, F, x, wt, out_rows, out);
   else
-    hipLaunchKernelGGL((tile_split_kernel<64>), grid, block, 0, s, n, R, F, x, wt, out_rows, out);
+    hipLaunchKernelGGL((tile_split_kernel<64, 128>), grid, block, 0, s, n, R, F, x, wt, out_rows, out);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
