@@ -78,11 +78,13 @@ struct MlpBasis {                  // act(delta . W[:, col] + b[col]) / pdf   (M
 // sqrtf and the division, whose expansions also cover subnormal numbers.  The projection evaluates
 // 16 of them per pair: 120 -> 96 us for 32 channels on 98 765 centres of 37 pairs, 836 -> 813 us for the
 // two passes with shifted kernel points of 64 channels on 200 003.
-// Distances below 1e-15 count as none (the weight is 1 either way).
+// Distances below 1e-15 count as none (the weight is 1 either way), influences beyond 1e30 as 1e30
+// (likewise; the reciprocal of larger ones is subnormal, that of an infinite one zero).
 template <int kKind>
 struct KpInfluence {
   float sigma, inv;
-  __device__ __forceinline__ explicit KpInfluence(float s) : sigma(s), inv(1.0f / s) {}
+  __device__ __forceinline__ explicit KpInfluence(float s)
+      : sigma(s > 1e30f ? 1e30f : s), inv(1.0f / sigma) {}
   __device__ __forceinline__ float operator()(float sq) const {
     if (kKind != 0) {
       const float q = sqrtf(sq) / (sigma / 3.0f);

@@ -37,3 +37,22 @@ def test_influence_matches_float64(sigma):
     bound = 2.0 ** -24 * (10 * dist / s + 2)
     assert bool(((out[:, 0, :kp].double() - want).abs() <= bound).all())
     assert float(out[:, 1:].abs().max()) == 0.0 and float(out[:, 0, kp:].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("sigma", [1e29, 2e30, 3e38, float("inf")])
+def test_influence_without_an_edge(sigma):
+    from tensorflow_graphics_point_clouds_amd import _lib
+    from tensorflow_graphics_point_clouds_amd._lib import cfloat, cint, i64, ptr, stream
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    n, kp = 64, 15
+    kpts = torch.rand(kp, 3, device="cuda", generator=gen)
+    points = torch.rand(n, 3, device="cuda", generator=gen)
+    points[:kp] = kpts
+    pairs = torch.arange(n, device="cuda", dtype=torch.int32)[:, None].expand(-1, 2).contiguous()
+    ranges = torch.arange(1, n + 1, device="cuda", dtype=torch.int32)
+    out = torch.empty(n, 16, 16, device="cuda")
+    _lib.call("kp_conv_project", stream(), cint(3), i64(n), ptr(points), cint(16),
+              ptr(torch.ones(n, 16, device="cuda")), i64(n), ptr(torch.zeros(n, 3, device="cuda")),
+              i64(n), ptr(pairs), ptr(ranges), ptr(torch.ones(3, device="cuda")), cint(kp),
+              ptr(kpts), cint(0), cfloat(sigma), ptr(None), ptr(out))
+    assert bool((out[:, :, :kp] == 1.0).all())
