@@ -405,9 +405,11 @@ __global__ void __launch_bounds__(256) kp_deform_offset_grads16_kernel(
               // root and quotient as in KpInfluence
               const float y = __builtin_amdgcn_rsqf(sq), g = sq * y;
               const float dist = fmaf(fmaf(-g, g, sq), 0.5f * y, g);
-              const float top = -acc[r] * geo.w * (dist < sigma ? neg_inv_sigma : 0.0f);
+              const bool reached = dist < sigma;      // (not where sq is infinite: dist is NaN)
+              const float top = -acc[r] * geo.w * (reached ? neg_inv_sigma : 0.0f);
               const float q = top * y;
-              coef = sq < 1e-30f ? 0.0f : fmaf(fmaf(-q, dist, top), y, q);
+              // the direction has a length of one down to the smallest normal sq
+              coef = sq < 1.17549435e-38f ? 0.0f : reached ? fmaf(fmaf(-q, dist, top), y, q) : top;
             } else {
               const float dist = sqrtf(sq), sg = sigma / 3.0f, q = dist / sg;
               const float slope = -2.0f * q / sg * expf(-(q * q));

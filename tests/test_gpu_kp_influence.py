@@ -56,3 +56,29 @@ def test_influence_without_an_edge(sigma):
               i64(n), ptr(pairs), ptr(ranges), ptr(torch.ones(3, device="cuda")), cint(kp),
               ptr(kpts), cint(0), cfloat(sigma), ptr(None), ptr(out))
     assert bool((out[:, :, :kp] == 1.0).all())
+
+
+@pytest.mark.parametrize("step,expect", [(1e-12, -2.0), (3e-16, -2.0), (1e-18, -2.0), (0.0, 0.0),
+                                         (0.4, -2.0), (0.6, 0.0), (1e20, 0.0)])
+def test_offset_gradient_of_any_distance(step, expect):
+    """d influence / d distance is -1 / sigma inside the influence, at any distance but none."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    from tensorflow_graphics_point_clouds_amd._lib import cfloat, cint, i64, ptr, stream
+    n, kp, sigma = 40, 15, 0.5
+    zeros = torch.zeros(n, 3, device="cuda")
+    pairs = torch.arange(n, device="cuda", dtype=torch.int32)[:, None].expand(-1, 2).contiguous()
+    ranges = torch.arange(1, n + 1, device="cuda", dtype=torch.int32)
+    offsets = torch.zeros(n, kp, 3, device="cuda")
+    offsets[:, :, 0] = -step                         # the points lie at +step of the kernel points
+    feat = torch.zeros(n, 16, device="cuda")
+    feat[:, 0] = 1.0
+    upstream = torch.ones(n, 16, 16, device="cuda")
+    out = torch.empty(n, kp, 3, device="cuda")
+    _lib.call("kp_deform_offset_grads", stream(), cint(3), i64(n), ptr(zeros), cint(16), ptr(feat),
+              i64(n), ptr(zeros), i64(n), ptr(pairs), ptr(ranges),
+              ptr(torch.ones(3, device="cuda")), cint(kp), ptr(torch.zeros(kp, 3, device="cuda")),
+              cint(0), cfloat(sigma), ptr(offsets), ptr(upstream), ptr(out))
+    # moving a kernel point towards the point (+x) raises the influence by 1 / sigma
+    want = torch.zeros_like(out)
+    want[:, :, 0] = -expect
+    assert torch.allclose(out, want, rtol=4 * 2.0 ** -23, atol=0.0)
