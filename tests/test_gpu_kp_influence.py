@@ -51,10 +51,11 @@ def test_influence_without_an_edge(sigma):
     pairs = torch.arange(n, device="cuda", dtype=torch.int32)[:, None].expand(-1, 2).contiguous()
     ranges = torch.arange(1, n + 1, device="cuda", dtype=torch.int32)
     out = torch.empty(n, 16, 16, device="cuda")
-    _lib.call("kp_conv_project", stream(), cint(3), i64(n), ptr(points), cint(16),
-              ptr(torch.ones(n, 16, device="cuda")), i64(n), ptr(torch.zeros(n, 3, device="cuda")),
-              i64(n), ptr(pairs), ptr(ranges), ptr(torch.ones(3, device="cuda")), cint(kp),
-              ptr(kpts), cint(0), cfloat(sigma), ptr(None), ptr(out))
+    feat, centres = torch.ones(n, 16, device="cuda"), torch.zeros(n, 3, device="cuda")
+    ones = torch.ones(3, device="cuda")
+    _lib.call("kp_conv_project", stream(), cint(3), i64(n), ptr(points), cint(16), ptr(feat), i64(n),
+              ptr(centres), i64(n), ptr(pairs), ptr(ranges), ptr(ones), cint(kp), ptr(kpts), cint(0),
+              cfloat(sigma), ptr(None), ptr(out))
     assert bool((out[:, :, :kp] == 1.0).all())
 
 
@@ -74,9 +75,9 @@ def test_offset_gradient_of_any_distance(step, expect):
     feat[:, 0] = 1.0
     upstream = torch.ones(n, 16, 16, device="cuda")
     out = torch.empty(n, kp, 3, device="cuda")
+    ones, kpts = torch.ones(3, device="cuda"), torch.zeros(kp, 3, device="cuda")
     _lib.call("kp_deform_offset_grads", stream(), cint(3), i64(n), ptr(zeros), cint(16), ptr(feat),
-              i64(n), ptr(zeros), i64(n), ptr(pairs), ptr(ranges),
-              ptr(torch.ones(3, device="cuda")), cint(kp), ptr(torch.zeros(kp, 3, device="cuda")),
+              i64(n), ptr(zeros), i64(n), ptr(pairs), ptr(ranges), ptr(ones), cint(kp), ptr(kpts),
               cint(0), cfloat(sigma), ptr(offsets), ptr(upstream), ptr(out))
     # moving a kernel point towards the point (+x) raises the influence by 1 / sigma
     want = torch.zeros_like(out)
