@@ -261,23 +261,22 @@ extern "C" int mccnn_kp_conv_gather_grads(
                 "kp_conv_gather_grads received a null tensor");
   const int run_len = gather_run_len(num_pts);
   const dim3 grid(wave_grid((num_pts + run_len - 1) / run_len)), block(256);
-#define MCCNN_GATHER(LIVE_, D_, KIND_)                                                          \
+#define MCCNN_GATHER(LIVE_, D_)                                                                 \
   {                                                                                             \
     McParams<D_> prm{centres, points, inv_radii, nullptr, nullptr, nullptr, 1, 0};              \
-    hipLaunchKernelGGL((kp_conv_gather_grads_kernel<LIVE_, D_, KIND_>), grid, block, 0,         \
-                       as_stream(stream), num_pts, run_len, projection_grads,                   \
-                       64u * padded_features, (const int2 *)neighbors, ranges, prm,             \
-                       kernel_points, num_kernel_points, sigma, out_rows, num_features, out);   \
+    MCCNN_INFLUENCE_SWITCH(                                                                     \
+        kind, sigma,                                                                            \
+        hipLaunchKernelGGL((kp_conv_gather_grads_kernel<LIVE_, D_, KIND>), grid, block, 0,      \
+                           as_stream(stream), num_pts, run_len, projection_grads,               \
+                           64u * padded_features, (const int2 *)neighbors, ranges, prm,         \
+                           kernel_points, num_kernel_points, sigma, out_rows, num_features,     \
+                           out));                                                               \
   }
-#define MCCNN_GATHER_D(LIVE_)                                                   \
-  if (num_dims == 3) {                                                          \
-    if (kind == 0) MCCNN_GATHER(LIVE_, 3, 0) else MCCNN_GATHER(LIVE_, 3, 1)     \
-  } else {                                                                      \
-    if (kind == 0) MCCNN_GATHER(LIVE_, 2, 0) else MCCNN_GATHER(LIVE_, 2, 1)     \
-  }
-  if (num_features <= 4) { MCCNN_GATHER_D(4) }
-  else if (num_features <= 8) { MCCNN_GATHER_D(8) }
-  else { MCCNN_GATHER_D(16) }
+#define MCCNN_GATHER_D(LIVE_) \
+  if (num_dims == 3) MCCNN_GATHER(LIVE_, 3) else MCCNN_GATHER(LIVE_, 2)
+  if (num_features <= 4) MCCNN_GATHER_D(4)
+  else if (num_features <= 8) MCCNN_GATHER_D(8)
+  else MCCNN_GATHER_D(16)
 #undef MCCNN_GATHER_D
 #undef MCCNN_GATHER
   MCCNN_LAUNCH_CHECK();

@@ -78,17 +78,36 @@ struct MlpBasis {                  // act(delta . W[:, col] + b[col]) / pdf   (M
 // sqrtf and the division, whose expansions also cover subnormal numbers.  The projection evaluates
 // 16 of them per pair: 120 -> 96 us for 32 channels on 98 765 centres of 37 pairs, 836 -> 813 us for the
 // two passes with shifted kernel points of 64 channels on 200 003.
-// Distances below 1e-15 count as none (the weight is 1 either way), influences beyond 1e30 as 1e30
-// (likewise; the reciprocal of larger ones is subnormal, that of an infinite one zero).
+// Distances below 1e-15 count as none there: the corrections of smaller ones would be subnormal.  With
+// an influence of at least 1e-7 their weight rounds to 1 either way (1e-15 / 1e-7 is below 2^-25);
+// smaller influences, and those beyond 1e30, whose reciprocal is subnormal or zero, go through the
+// root and the division (influence_kind).
+enum : int { kLinear = 0, kGaussian = 1, kLinearByDivision = 2 };
+
+inline int influence_kind(int kind, float sigma) {
+  return kind == kLinear && !(sigma >= 1e-7f && sigma <= 1e30f) ? kLinearByDivision : kind;
+}
+
+// Dispatch on the influence of a kernel point, as the kernels evaluate it.
+#define MCCNN_INFLUENCE_SWITCH(kind_, sigma_, ...)                                  \
+  switch (influence_kind(kind_, sigma_)) {                                          \
+    case kLinear: { constexpr int KIND = kLinear; __VA_ARGS__; } break;             \
+    case kGaussian: { constexpr int KIND = kGaussian; __VA_ARGS__; } break;         \
+    default: { constexpr int KIND = kLinearByDivision; __VA_ARGS__; } break;        \
+  }
+
 template <int kKind>
 struct KpInfluence {
   float sigma, inv;
-  __device__ __forceinline__ explicit KpInfluence(float s)
-      : sigma(s > 1e30f ? 1e30f : s), inv(1.0f / sigma) {}
+  __device__ __forceinline__ explicit KpInfluence(float s) : sigma(s), inv(1.0f / s) {}
   __device__ __forceinline__ float operator()(float sq) const {
-    if (kKind != 0) {
+    if (kKind == kGaussian) {
       const float q = sqrtf(sq) / (sigma / 3.0f);
       return expf(-(q * q));
+    }
+    if (kKind == kLinearByDivision) {
+      const float v = 1.0f - sqrtf(sq) / sigma;
+      return v > 0.0f ? v : 0.0f;
     }
     const float y = __builtin_amdgcn_rsqf(sq), g = sq * y;
     const float root = fmaf(fmaf(-g, g, sq), 0.5f * y, g);

@@ -1092,19 +1092,17 @@ extern "C" int mccnn_kp_conv_project(mccnn_stream_t stream, int num_dims, int64_
   const int run_len = project_run_len(num_samples, chunks);
   const dim3 grid(wave_grid((num_samples + run_len - 1) / run_len * chunks)), block(256);
   const int2 *nb = (const int2 *)neighbors;
-#define MCCNN_KP_FWD(CPL_, D_, KIND_, KT_)                                                     \
-  {                                                                                            \
-    McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 1, 0};       \
-    hipLaunchKernelGGL((kp_conv_project16_kernel<CPL_, D_, KIND_, KT_>), grid, block, 0, s,    \
-                       num_samples, num_features, chunks, run_len, features, nb, ranges, prm,           \
-                       kernel_points, num_kernel_points, sigma, out_rows, out);                \
+#define MCCNN_KP_FWD(CPL_, D_, KT_)                                                             \
+  {                                                                                             \
+    McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 1, 0};        \
+    MCCNN_INFLUENCE_SWITCH(                                                                     \
+        kind, sigma,                                                                            \
+        hipLaunchKernelGGL((kp_conv_project16_kernel<CPL_, D_, KIND, KT_>), grid, block, 0, s,  \
+                           num_samples, num_features, chunks, run_len, features, nb, ranges,    \
+                           prm, kernel_points, num_kernel_points, sigma, out_rows, out));       \
   }
-#define MCCNN_KP_FWD_D(CPL_, KT_)                                                  \
-  if (num_dims == 3) {                                                             \
-    if (kind == 0) MCCNN_KP_FWD(CPL_, 3, 0, KT_) else MCCNN_KP_FWD(CPL_, 3, 1, KT_) \
-  } else {                                                                         \
-    if (kind == 0) MCCNN_KP_FWD(CPL_, 2, 0, KT_) else MCCNN_KP_FWD(CPL_, 2, 1, KT_) \
-  }
+#define MCCNN_KP_FWD_D(CPL_, KT_) \
+  if (num_dims == 3) MCCNN_KP_FWD(CPL_, 3, KT_) else MCCNN_KP_FWD(CPL_, 2, KT_)
   switch (kt * 16 + cpl) {
     case 16 + 8: MCCNN_KP_FWD_D(8, 1); break;
     case 16 + 4: MCCNN_KP_FWD_D(4, 1); break;
@@ -1162,20 +1160,18 @@ extern "C" int mccnn_kp_deform_project(mccnn_stream_t stream, int num_dims, int6
   const int run_len = project_run_len(num_samples, chunks);
   const dim3 grid(wave_grid((num_samples + run_len - 1) / run_len * chunks)), block(256);
   const int2 *nb = (const int2 *)neighbors;
-#define MCCNN_KPD(CPL_, D_, KIND_)                                                             \
-  {                                                                                            \
-    McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 1, 0};       \
-    hipLaunchKernelGGL((kp_deform_project16_kernel<CPL_, D_, KIND_>), grid, block, 0, s,       \
-                       num_samples, num_features, chunks, run_len, features, nb, ranges, prm,           \
-                       kernel_points, num_kernel_points, sigma, offsets, offsets_follow_points, \
-                       out_rows, out);                                                         \
+#define MCCNN_KPD(CPL_, D_)                                                                     \
+  {                                                                                             \
+    McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 1, 0};        \
+    MCCNN_INFLUENCE_SWITCH(                                                                     \
+        kind, sigma,                                                                            \
+        hipLaunchKernelGGL((kp_deform_project16_kernel<CPL_, D_, KIND>), grid, block, 0, s,     \
+                           num_samples, num_features, chunks, run_len, features, nb, ranges,    \
+                           prm, kernel_points, num_kernel_points, sigma, offsets,               \
+                           offsets_follow_points, out_rows, out));                              \
   }
-#define MCCNN_KPD_D(CPL_)                                                  \
-  if (num_dims == 3) {                                                     \
-    if (kind == 0) MCCNN_KPD(CPL_, 3, 0) else MCCNN_KPD(CPL_, 3, 1)        \
-  } else {                                                                 \
-    if (kind == 0) MCCNN_KPD(CPL_, 2, 0) else MCCNN_KPD(CPL_, 2, 1)        \
-  }
+#define MCCNN_KPD_D(CPL_) \
+  if (num_dims == 3) MCCNN_KPD(CPL_, 3) else MCCNN_KPD(CPL_, 2)
   switch (cpl) {
     case 8: MCCNN_KPD_D(8); break;
     case 4: MCCNN_KPD_D(4); break;

@@ -388,20 +388,19 @@ extern "C" int mccnn_kp_conv_layer(mccnn_stream_t stream, int num_dims, int64_t 
   rc = layer_grid(num_samples, &blocks);
   if (rc != MCCNN_OK) return rc;
   const int2 *nb = (const int2 *)neighbors;
-#define MCCNN_LAYER_DK(D_, KIND_)                                                              \
+#define MCCNN_LAYER_D(D_)                                                                      \
   {                                                                                            \
     McParams<D_> prm{points_in, points_out, inv_radii, nullptr, nullptr, nullptr, 0, 0};       \
-    rc = launch_layer(kp_conv_layer16_kernel<CPL, FT, D_, KIND_>, s, blocks,                   \
-                      LayerShape<CPL, FT>::kLdsBytes, num_samples, features, nb, ranges, prm,  \
-                      kernel_points, num_kernel_points, sigma, final_weights, out_rows,        \
-                      proj_out, out);                                                          \
+    MCCNN_INFLUENCE_SWITCH(                                                                    \
+        kind, sigma,                                                                           \
+        rc = launch_layer(kp_conv_layer16_kernel<CPL, FT, D_, KIND>, s, blocks,                \
+                          LayerShape<CPL, FT>::kLdsBytes, num_samples, features, nb, ranges,   \
+                          prm, kernel_points, num_kernel_points, sigma, final_weights,         \
+                          out_rows, proj_out, out));                                           \
   }
-#define MCCNN_LAYER_D(D_) \
-  if (kind == 0) MCCNN_LAYER_DK(D_, 0) else MCCNN_LAYER_DK(D_, 1)
   MCCNN_LAYER_SHAPE_SWITCH(num_features, num_out_features,
                            if (num_dims == 3) MCCNN_LAYER_D(3) else MCCNN_LAYER_D(2));
 #undef MCCNN_LAYER_D
-#undef MCCNN_LAYER_DK
   if (rc != MCCNN_OK) return rc;
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;

@@ -1,5 +1,6 @@
 """The linear influence of a kernel point as the projection kernel evaluates it: points on the
 kernel points and next to them, at the edge of the influence, and small and large ones."""
+import numpy as np
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -83,3 +84,38 @@ def test_offset_gradient_of_any_distance(step, expect):
     want = torch.zeros_like(out)
     want[:, :, 0] = -expect
     assert torch.allclose(out, want, rtol=4 * 2.0 ** -23, atol=0.0)
+
+
+@pytest.mark.parametrize("deformed", [False, True])
+@pytest.mark.parametrize("sigma", [1.0, 1.0 / 3.0, 0.07, 1e30, 2e30, 1.01e-7, 0.99e-7, 1e-8, 1e-15, 1e-16,
+                                   1e-20, 1e-39])
+def test_influence_has_the_bits_of_root_and_quotient(sigma, deformed):
+    """1 - sqrt(sq) / sigma with root and quotient correctly rounded, for random mantissas of the
+    distance and for influences as small as any that is accepted."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    from tensorflow_graphics_point_clouds_amd._lib import cfloat, cint, i64, ptr, stream
+    gen = torch.Generator().manual_seed(7)
+    n = 1 << 16
+    s = torch.tensor(sigma, dtype=torch.float32)
+    x = (s.double() * torch.rand(n, generator=gen, dtype=torch.float64)).float()
+    # down to a millionth of the influence, none, its edge, and fixed small ones
+    x[::3] = (x[::3].double() * 10.0 ** (-6.0 * torch.rand(x[::3].numel(), generator=gen,
+                                                           dtype=torch.float64))).float()
+    x[:6] = torch.tensor([0.0, 5e-16, 1e-15, 1e-18, sigma, 2.0 * sigma])
+    # (numpy: torch's root on the CPU is off by a last place now and then)
+    want = np.maximum(np.float32(1.0) - np.sqrt(x.numpy() * x.numpy()) / s.numpy(), np.float32(0.0))
+    points = torch.zeros(n, 3, device="cuda")
+    points[:, 0] = x.cuda()
+    pairs = torch.arange(n, device="cuda", dtype=torch.int32)[:, None].expand(-1, 2).contiguous()
+    ranges = torch.arange(1, n + 1, device="cuda", dtype=torch.int32)
+    ones, zeros = torch.ones(3, device="cuda"), torch.zeros(n, 3, device="cuda")
+    feat, out = torch.zeros(n, 16, device="cuda"), torch.empty(n, 16, 16, device="cuda")
+    feat[:, 0] = 1.0
+    kernel_point = torch.zeros(1, 3, device="cuda")
+    geometry = (stream(), cint(3), i64(n), ptr(points), cint(16), ptr(feat), i64(n), ptr(zeros), i64(n),
+                ptr(pairs), ptr(ranges), ptr(ones), cint(1), ptr(kernel_point), cint(0), cfloat(sigma))
+    if deformed:
+        _lib.call("kp_deform_project", *geometry, ptr(zeros), cint(0), ptr(None), ptr(out))
+    else:
+        _lib.call("kp_conv_project", *geometry, ptr(None), ptr(out))
+    assert np.array_equal(out[:, 0, 0].cpu().numpy(), want)
