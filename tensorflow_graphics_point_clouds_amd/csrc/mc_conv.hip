@@ -396,29 +396,42 @@ __global__ void __launch_bounds__(256) kp_deform_offset_grads16_kernel(
           for (int s = 0; s < kQuarterC; ++s)
             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(gk[s], f.v[s], acc, 0, 0, 0);
           // acc[r] = dbasis[pair col][k = 4*quarter + r]; geo.w = 1 for a live pair, else 0
+          float diff[4][3], sq[4], coef[4];
+          bool odd = false;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float dx = geo.x - kpo[r][0], dy = geo.y - kpo[r][1], dz = geo.z - kpo[r][2];
-            const float sq = dx * dx + dy * dy + dz * dz;
-            float coef;
-            if (kKind == 0) {
+            diff[r][0] = dx, diff[r][1] = dy, diff[r][2] = dz;
+            sq[r] = dx * dx + dy * dy + dz * dz;
+            const float up = -acc[r] * geo.w;
+            if (kKind == kLinear) {
               // root and quotient as in KpInfluence
-              const float y = __builtin_amdgcn_rsqf(sq), g = sq * y;
-              const float dist = fmaf(fmaf(-g, g, sq), 0.5f * y, g);
+              const float y = __builtin_amdgcn_rsqf(sq[r]), g = sq[r] * y;
+              const float dist = fmaf(fmaf(-g, g, sq[r]), 0.5f * y, g);
               const bool reached = dist < sigma;      // (not where sq is infinite: dist is NaN)
-              const float top = -acc[r] * geo.w * (reached ? neg_inv_sigma : 0.0f);
-              const float q = top * y;
-              // the direction has a length of one down to the smallest normal sq
-              coef = sq < 1.17549435e-38f ? 0.0f : reached ? fmaf(fmaf(-q, dist, top), y, q) : top;
+              const float top = up * (reached ? neg_inv_sigma : 0.0f), q = top * y;
+              const bool apart = sq[r] > 0.0f;        // none, or NaN: no direction
+              coef[r] = !apart ? 0.0f : reached ? fmaf(fmaf(-q, dist, top), y, q) : top;
+              // (an infinite or NaN quotient, or a square of which the residual is subnormal)
+              odd |= apart && !(sq[r] >= 1e-30f && fabsf(q) < __builtin_inff());
             } else {
-              const float dist = sqrtf(sq), sg = sigma / 3.0f, q = dist / sg;
+              const float dist = sqrtf(sq[r]), sg = sigma / 3.0f, q = dist / sg;
               const float slope = -2.0f * q / sg * expf(-(q * q));
-              coef = dist > 0.0f ? -acc[r] * geo.w * slope / dist : 0.0f;
+              coef[r] = dist > 0.0f ? up * slope / dist : 0.0f;
             }
-            sum[r][0] += coef * dx;
-            sum[r][1] += coef * dy;
-            if (D > 2) sum[r][2] += coef * dz;
           }
+          if (kKind == kLinear && odd) {              // what the corrections do not cover
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float dist = sqrtf(sq[r]);
+              const float slope = dist < sigma ? neg_inv_sigma : 0.0f;
+              coef[r] = dist > 0.0f ? -acc[r] * geo.w * slope / dist : 0.0f;
+            }
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int d = 0; d < D; ++d) sum[r][d] += coef[r] * diff[r][d];
           f = fn;
         }
         wave_lds_sync();                      // the stage is free for the next chunk

@@ -86,6 +86,43 @@ def test_offset_gradient_of_any_distance(step, expect):
     assert torch.allclose(out, want, rtol=4 * 2.0 ** -23, atol=0.0)
 
 
+
+@pytest.mark.parametrize("up", [1.0, -3.0, 1e38, float("inf")])
+def test_offset_gradient_beside_the_corrections(up):
+    """Distances whose square is subnormal, and gradients that are infinite or become so by the
+    division: as sqrtf and the division give them."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    from tensorflow_graphics_point_clouds_amd._lib import cfloat, cint, i64, ptr, stream
+    sigma = np.float32(0.5)
+    x = np.float32([0.0, 1e-24, 3e-23, 1e-20, -7e-20, 1e-19, 2e-19, 1e-17, 1e-15, -1.1e-15, 1e-6, -0.3,
+                    0.4, 0.499, 0.5, 0.7, 1e19, 3e19])
+    n, kp = len(x), 15
+    zeros, ones = torch.zeros(n, 3, device="cuda"), torch.ones(3, device="cuda")
+    # each pair sixteen times, which fills a tile (empty places are multiplied by 0)
+    pairs = torch.arange(16 * n, device="cuda").div(16, rounding_mode="floor").int()
+    pairs = pairs[:, None].expand(-1, 2).contiguous()
+    ranges = 16 * torch.arange(1, n + 1, device="cuda", dtype=torch.int32)
+    offsets = torch.zeros(n, kp, 3, device="cuda")
+    offsets[:, :, 0] = -torch.from_numpy(x).cuda()[:, None]
+    feat, kpts = torch.ones(n, 16, device="cuda"), torch.zeros(kp, 3, device="cuda")
+    upstream = torch.zeros(n, 16, 16, device="cuda")
+    upstream[:, 0] = up
+    out = torch.empty(n, kp, 3, device="cuda")
+    _lib.call("kp_deform_offset_grads", stream(), cint(3), i64(n), ptr(zeros), cint(16), ptr(feat),
+              i64(n), ptr(zeros), i64(16 * n), ptr(pairs), ptr(ranges), ptr(ones), cint(kp), ptr(kpts),
+              cint(0), cfloat(sigma), ptr(offsets), ptr(upstream), ptr(out))
+    with np.errstate(all="ignore"):
+        dist = np.sqrt(x * x)
+        slope = np.where(dist < sigma, -1 / sigma, np.float32(0.0))
+        coef = np.where(dist > 0, -np.float32(up) * slope / dist, np.float32(0.0)).astype(np.float32)
+        want = np.broadcast_to((16 * (coef * x))[:, None], (n, kp))
+    got = out[:, :, 0].cpu().numpy()
+    # (a quotient and a product, each rounded once; sixteen times it is exact)
+    assert np.allclose(got, want, rtol=2 * 2.0 ** -23, atol=0.0, equal_nan=True)
+    finite = np.isfinite(coef)                       # (infinite: times 0 in the other coordinates)
+    assert float(out[:, :, 1:].cpu()[finite].abs().max()) == 0.0
+
+
 @pytest.mark.parametrize("deformed", [False, True])
 @pytest.mark.parametrize("sigma", [1.0, 1.0 / 3.0, 0.07, 1e30, 2e30, 1.01e-7, 0.99e-7, 1e-8, 1e-15, 1e-16,
                                    1e-20, 1e-39])
