@@ -818,7 +818,7 @@ int mccnn_kp_conv_project(mccnn_stream_t stream, int num_dims, int64_t num_pts,
  *   out[j, c] = sum over the pairs (i, j) of sum_k basis_k(ij) projection_grads[i, c, k]
  * over the transposed pair table (rows grouped by point j, neighbors[., 0] = centre i, ranges
  * over the points; inv_radii negated so that the offsets keep their sign).  projection_grads
- * [N_centres, padded_features, 16], num_features <= 16 of which are read; out [N_pts,
+ * [N_centres, padded_features, 16] with num_features <= min(padded_features, 16); out [N_pts,
  * num_features], row j at out_rows[j] (NULL: j); accumulate != 0 adds to what out holds.
  * 16 basis columns, D in {2,3}.  No counterpart among the reference's ops. */
 int mccnn_mc_conv_gather_grads(mccnn_stream_t stream, int num_dims, int64_t num_centres,

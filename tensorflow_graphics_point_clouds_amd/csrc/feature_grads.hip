@@ -24,9 +24,10 @@ namespace mccnn {
 constexpr int kGatherRun = 8;      // points per wavefront, at most
 constexpr int kGatherAhead = 2;    // pairs of a quarter in flight
 
-// kLive: channels that are gathered (the rows of G hold `row_bytes` of them, the ones past kLive
-// being padding); columns c < live of `out` are written, `ldo` floats to a row.
-template <int kLive, int D, class Basis>
+// kLive: channels that are gathered, of rows of G of `row_bytes`; columns c < live of `out` are
+// written.  kWhole: a row holds kLive channels or more.  Where it holds fewer the last one is read
+// again in their place (nothing behind the row, or behind G, is).
+template <int kLive, int D, bool kWhole, class Basis>
 __device__ __forceinline__ void gather_grads_body(
     int64_t n_pts, int run_len, const char *__restrict__ grads, unsigned row_bytes,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, const McParams<D> &p,
@@ -51,6 +52,7 @@ __device__ __forceinline__ void gather_grads_body(
   float ir[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) ir[d] = p.inv_radii[d];
+  const unsigned last_channel = row_bytes - 64;
 
   struct Pending {
     int idx;
@@ -136,7 +138,9 @@ __device__ __forceinline__ void gather_grads_body(
           const int at = n < e ? n : s;   // past the point's pairs: its first one, weighted 0
           const char *row = grads + (size_t)stage->row[at] + 4 * col;
 #pragma unroll
-          for (int c = 0; c < kLive; ++c) g[u][c] = *reinterpret_cast<const float *>(row + 64 * c);
+          for (int c = 0; c < kLive; ++c)
+            g[u][c] = *reinterpret_cast<const float *>(
+                row + (kWhole || 64u * c < last_channel ? 64u * c : last_channel));
           w[u] = n < e ? basis(stage->geo[at]) : 0.0f;
         }
 #pragma unroll
@@ -154,19 +158,19 @@ __device__ __forceinline__ void gather_grads_body(
   for (; cur < nc; ++cur) finish_point(cur);      // trailing points without pairs
 }
 
-template <int kLive, int D, int kAct>
+template <int kLive, int D, int kAct, bool kWhole>
 __global__ void __launch_bounds__(256) mc_conv_gather_grads_kernel(
     int64_t n_pts, int run_len, const float *__restrict__ grads, unsigned row_bytes,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, McParams<D> p,
     const int *__restrict__ out_rows, int live, int add, float *__restrict__ out) {
   __shared__ PairStage stages[kWavesPerBlock];
   const MlpBasis<D, kAct> basis(p);
-  gather_grads_body<kLive, D>(n_pts, run_len, reinterpret_cast<const char *>(grads), row_bytes,
-                              nbrs, ranges, p, basis, out_rows, live, add != 0, out,
-                              &stages[threadIdx.x / kWave]);
+  gather_grads_body<kLive, D, kWhole>(n_pts, run_len, reinterpret_cast<const char *>(grads),
+                                      row_bytes, nbrs, ranges, p, basis, out_rows, live, add != 0,
+                                      out, &stages[threadIdx.x / kWave]);
 }
 
-template <int kLive, int D, int kKind>
+template <int kLive, int D, int kKind, bool kWhole>
 __global__ void __launch_bounds__(256) kp_conv_gather_grads_kernel(
     int64_t n_pts, int run_len, const float *__restrict__ grads, unsigned row_bytes,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, McParams<D> p,
@@ -174,9 +178,9 @@ __global__ void __launch_bounds__(256) kp_conv_gather_grads_kernel(
     const int *__restrict__ out_rows, int live, float *__restrict__ out) {
   __shared__ PairStage stages[kWavesPerBlock];
   const KpBasis<D, kKind> basis(kernel_points, num_kp, sigma);
-  gather_grads_body<kLive, D>(n_pts, run_len, reinterpret_cast<const char *>(grads), row_bytes,
-                              nbrs, ranges, p, basis, out_rows, live, false, out,
-                              &stages[threadIdx.x / kWave]);
+  gather_grads_body<kLive, D, kWhole>(n_pts, run_len, reinterpret_cast<const char *>(grads),
+                                      row_bytes, nbrs, ranges, p, basis, out_rows, live, false,
+                                      out, &stages[threadIdx.x / kWave]);
 }
 
 // As for the projection (mc_conv.hip): shorter runs on small inputs.
@@ -220,22 +224,26 @@ extern "C" int mccnn_mc_conv_gather_grads(
                 "mc_conv_gather_grads received a null tensor");
   const int run_len = gather_run_len(num_pts);
   const dim3 grid(wave_grid((num_pts + run_len - 1) / run_len)), block(256);
-#define MCCNN_GATHER(LIVE_, D_)                                                                 \
+#define MCCNN_GATHER(LIVE_, D_, WHOLE_)                                                         \
   {                                                                                             \
     McParams<D_> prm{centres, points, inv_radii, weights, biases, pdf, kFusedK / num_mlps,      \
                      activation};                                                               \
     MCCNN_ACT_SWITCH(activation,                                                                \
-                     hipLaunchKernelGGL((mc_conv_gather_grads_kernel<LIVE_, D_, ACT>), grid,    \
-                                        block, 0, as_stream(stream), num_pts, run_len,          \
+                     hipLaunchKernelGGL((mc_conv_gather_grads_kernel<LIVE_, D_, ACT, WHOLE_>),  \
+                                        grid, block, 0, as_stream(stream), num_pts, run_len,    \
                                         projection_grads, 64u * padded_features,                \
                                         (const int2 *)neighbors, ranges, prm, out_rows,         \
                                         num_features, accumulate, out));                        \
   }
-#define MCCNN_GATHER_D(LIVE_) \
-  if (num_dims == 3) MCCNN_GATHER(LIVE_, 3) else MCCNN_GATHER(LIVE_, 2)
-  if (num_features <= 4) MCCNN_GATHER_D(4)
-  else if (num_features <= 8) MCCNN_GATHER_D(8)
-  else MCCNN_GATHER_D(16)
+#define MCCNN_GATHER_D(LIVE_)                                                                   \
+  if (padded_features >= LIVE_) {                                                               \
+    if (num_dims == 3) MCCNN_GATHER(LIVE_, 3, true) else MCCNN_GATHER(LIVE_, 2, true)           \
+  } else {                                                                                      \
+    if (num_dims == 3) MCCNN_GATHER(LIVE_, 3, false) else MCCNN_GATHER(LIVE_, 2, false)         \
+  }
+  if (num_features <= 4) { MCCNN_GATHER_D(4) }
+  else if (num_features <= 8) { MCCNN_GATHER_D(8) }
+  else { MCCNN_GATHER_D(16) }
 #undef MCCNN_GATHER_D
 #undef MCCNN_GATHER
   MCCNN_LAUNCH_CHECK();
@@ -261,22 +269,26 @@ extern "C" int mccnn_kp_conv_gather_grads(
                 "kp_conv_gather_grads received a null tensor");
   const int run_len = gather_run_len(num_pts);
   const dim3 grid(wave_grid((num_pts + run_len - 1) / run_len)), block(256);
-#define MCCNN_GATHER(LIVE_, D_)                                                                 \
+#define MCCNN_GATHER(LIVE_, D_, WHOLE_)                                                         \
   {                                                                                             \
     McParams<D_> prm{centres, points, inv_radii, nullptr, nullptr, nullptr, 1, 0};              \
     MCCNN_INFLUENCE_SWITCH(                                                                     \
         kind, sigma,                                                                            \
-        hipLaunchKernelGGL((kp_conv_gather_grads_kernel<LIVE_, D_, KIND>), grid, block, 0,      \
-                           as_stream(stream), num_pts, run_len, projection_grads,               \
+        hipLaunchKernelGGL((kp_conv_gather_grads_kernel<LIVE_, D_, KIND, WHOLE_>), grid, block, \
+                           0, as_stream(stream), num_pts, run_len, projection_grads,            \
                            64u * padded_features, (const int2 *)neighbors, ranges, prm,         \
                            kernel_points, num_kernel_points, sigma, out_rows, num_features,     \
                            out));                                                               \
   }
-#define MCCNN_GATHER_D(LIVE_) \
-  if (num_dims == 3) MCCNN_GATHER(LIVE_, 3) else MCCNN_GATHER(LIVE_, 2)
-  if (num_features <= 4) MCCNN_GATHER_D(4)
-  else if (num_features <= 8) MCCNN_GATHER_D(8)
-  else MCCNN_GATHER_D(16)
+#define MCCNN_GATHER_D(LIVE_)                                                                   \
+  if (padded_features >= LIVE_) {                                                               \
+    if (num_dims == 3) MCCNN_GATHER(LIVE_, 3, true) else MCCNN_GATHER(LIVE_, 2, true)           \
+  } else {                                                                                      \
+    if (num_dims == 3) MCCNN_GATHER(LIVE_, 3, false) else MCCNN_GATHER(LIVE_, 2, false)         \
+  }
+  if (num_features <= 4) { MCCNN_GATHER_D(4) }
+  else if (num_features <= 8) { MCCNN_GATHER_D(8) }
+  else { MCCNN_GATHER_D(16) }
 #undef MCCNN_GATHER_D
 #undef MCCNN_GATHER
   MCCNN_LAUNCH_CHECK();
