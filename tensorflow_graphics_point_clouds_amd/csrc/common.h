@@ -41,9 +41,11 @@ inline hipStream_t as_stream(mccnn_stream_t s) { return reinterpret_cast<hipStre
 // they were launched (values are never negative), by looking at the memory: what the host asks
 // for is there when the kernel has stored it, which is some 15 us before the stream is known to be
 // idle (a marker is enqueued, its signal waited for).  After a while, or if the values do not
-// arrive that way, the stream is waited for.  Defined in util.hip.
-int wait_for_host_values(hipStream_t s, const volatile int64_t *values, int n);
-int wait_for_host_values(hipStream_t s, const volatile int32_t *values, int n);
+// arrive that way, the stream is waited for.  Each value is one atomic store of system scope;
+// nothing else that the kernels have written may be read by the host after the wait.  Defined in
+// util.hip.
+int wait_for_host_values(hipStream_t s, const int64_t *values, int n);
+int wait_for_host_values(hipStream_t s, const int32_t *values, int n);
 
 // Dispatch on the point dimension (2..6), the template parameter of most kernels.
 #define MCCNN_DIM_SWITCH(D_, ...)                              \

@@ -379,7 +379,9 @@ __global__ void __launch_bounds__(kSortThreads) grid_keys_kernel(
   if (blockIdx.x == 0 && threadIdx.x < D) {
     g.num_cells[threadIdx.x] = nc[threadIdx.x];
     g.inv_cell[threadIdx.x] = ic[threadIdx.x];
-    if (shape_host) shape_host[threadIdx.x] = nc[threadIdx.x];
+    if (shape_host)
+      __hip_atomic_store(&shape_host[threadIdx.x], nc[threadIdx.x], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
   }
   const int64_t base = (int64_t)blockIdx.x * kSortTile;
 #pragma unroll

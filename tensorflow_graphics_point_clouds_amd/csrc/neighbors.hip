@@ -762,11 +762,8 @@ extern "C" int mccnn_find_neighbors_bounded(
                      ranges_out, neighbors_out, capacity);
 }
 
-// The count half of a search by a caller that has the grid in hand (no argument checks beyond
-// sizes and null pointers), with or without the grid's column table, and with the outcome in
-// pinned host memory.
 // Both halves of a count by a caller that has the grid in hand: slices, counts, end offsets and
-// their total in `total` (device or pinned memory).
+// their total in `total` (device or pinned memory), with kScanFlag where *truncated has been set.
 static int search_counts(hipStream_t s, int64_t num_samples, int num_dims, const float *samples,
                          const int32_t *sample_batch_ids, int64_t num_pts, const float *points,
                          const int64_t *point_keys, const int32_t *grid_ds,
@@ -784,9 +781,12 @@ static int search_counts(hipStream_t s, int64_t num_samples, int num_dims, const
   rc = launch_count(s, num_dims, num_samples, samples, points, w, inv_radii, max_neighs,
                     in_visit ? &search : nullptr, ranges_out, truncated);
   if (rc != MCCNN_OK) return rc;
-  return inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, total);
+  return inclusive_scan_i32(s, num_samples, ranges_out, w.scan_scratch, total, truncated);
 }
 
+// The count half of a search by a caller that has the grid in hand (no argument checks beyond
+// sizes and null pointers), with or without the grid's column table, and with the outcome in
+// pinned host memory.
 extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, int num_dims,
                                   const float *samples, const int32_t *sample_batch_ids,
                                   int64_t num_pts, const float *points, const int64_t *point_keys,
@@ -809,7 +809,7 @@ extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, in
   MCCNN_REQUIRE(workspace_bytes >= w.bytes, "search_count workspace too small (%zu < %zu)",
                 workspace_bytes, w.bytes);
   hipStream_t s = as_stream(stream);
-  result_pinned[0] = -1;                  // (the flag is written by a kernel before the total's)
+  result_pinned[0] = -1;
   int rc = search_counts(s, num_samples, num_dims, samples, sample_batch_ids, num_pts, points,
                          point_keys, grid_ds, num_cells, scaled_aabb_min, inv_cell_sizes, inv_radii,
                          max_neighs, w, ranges_out, result_pinned,
@@ -817,6 +817,10 @@ extern "C" int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, in
   if (rc != MCCNN_OK) return rc;
   rc = wait_for_host_values(s, result_pinned, 1);
   if (rc != MCCNN_OK) return rc;
+  // (the total's word holds the flag: the flag's own is not known to have arrived)
+  const int64_t total = result_pinned[0];
+  result_pinned[0] = total & ~kScanFlag;
+  result_pinned[1] = total & kScanFlag ? 1 : 0;
   MCCNN_REQUIRE(result_pinned[0] < (((int64_t)1 << 31) - 1),
                 "FindNeighbors found at least %lld pairs; the int32 offsets of the op contract "
                 "hold fewer than 2^31 - 1",

@@ -1,7 +1,6 @@
 // Error reporting, fill and prefix-sum helpers of libmccnn_hip.so.
 #include <stdarg.h>
 
-#include <atomic>
 #include <chrono>
 
 #include "common.h"
@@ -129,9 +128,17 @@ __global__ void __launch_bounds__(kScanThreads) scan_tile_sums_kernel(
   if (threadIdx.x == 0) block_sums[blockIdx.x] = saturate_i32(total);
 }
 
+__device__ __forceinline__ void store_total(int64_t *total_dev, long long total,
+                                            const int64_t *flag) {
+  if (flag && __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0)
+    total |= kScanFlag;
+  __hip_atomic_store(total_dev, (int64_t)total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Single block: exclusive scan of block_sums[0..nb) in place, total to *total_dev.
 __global__ void __launch_bounds__(kScanThreads) scan_block_sums_kernel(int nb, int *block_sums,
-                                                                       int64_t *total_dev) {
+                                                                       int64_t *total_dev,
+                                                                       const int64_t *flag) {
   long long carry = 0;
   for (int base = 0; base < nb; base += kScanThreads) {
     const int i = base + threadIdx.x;
@@ -141,7 +148,7 @@ __global__ void __launch_bounds__(kScanThreads) scan_block_sums_kernel(int nb, i
     if (i < nb) block_sums[i] = saturate_i32(carry + ex);
     carry += total;
   }
-  if (threadIdx.x == 0) *total_dev = carry;
+  if (threadIdx.x == 0) store_total(total_dev, carry, flag);
 }
 
 // kOwnPrefix: block_sums are the tile sums themselves and the block adds up those in front of
@@ -149,7 +156,7 @@ __global__ void __launch_bounds__(kScanThreads) scan_block_sums_kernel(int nb, i
 template <bool kOwnPrefix>
 __global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(
     int64_t n, bool vec, int *__restrict__ counts, const int *__restrict__ block_sums,
-    int64_t *total_dev) {
+    int64_t *total_dev, const int64_t *flag) {
   const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
   int v[kScanItems];
   load_items<kScanItems>(counts, base, n, vec, v);
@@ -165,7 +172,8 @@ __global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(
     carry = block_sums[blockIdx.x];
   }
   long long run = carry + block_exclusive_scan_i64<kScanThreads>(s, &total);
-  if (kOwnPrefix && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) *total_dev = carry + total;
+  if (kOwnPrefix && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+    store_total(total_dev, carry + total, flag);
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
     run += v[k];
@@ -181,7 +189,7 @@ constexpr int kScanSingleTile = kScanSingleThreads * kScanSingleItems;
 constexpr int64_t kScanSingleMax = 2 * kScanSingleTile;
 
 __global__ void __launch_bounds__(kScanSingleThreads) scan_single_block_kernel(
-    int64_t n, bool vec, int *counts, int64_t *total_dev) {
+    int64_t n, bool vec, int *counts, int64_t *total_dev, const int64_t *flag) {
   long long carry = 0;
   for (int64_t tile = 0; tile < n; tile += kScanSingleTile) {
     const int64_t base = tile + (int64_t)threadIdx.x * kScanSingleItems;
@@ -200,11 +208,11 @@ __global__ void __launch_bounds__(kScanSingleThreads) scan_single_block_kernel(
     store_items<kScanSingleItems>(counts, base, n, vec, v);
     carry += total;
   }
-  if (threadIdx.x == 0) *total_dev = carry;
+  if (threadIdx.x == 0) store_total(total_dev, carry, flag);
 }
 
 int inclusive_scan_i32(hipStream_t stream, int64_t n, int *counts, int *block_sums,
-                       int64_t *total_dev) {
+                       int64_t *total_dev, const int64_t *flag) {
   const int nb = (int)((n + kScanTile - 1) / kScanTile);
   if (nb == 0) {
     return fill_zero(stream, total_dev, sizeof(int64_t));
@@ -212,7 +220,7 @@ int inclusive_scan_i32(hipStream_t stream, int64_t n, int *counts, int *block_su
   const bool vec = reinterpret_cast<uintptr_t>(counts) % 16 == 0;
   if (n <= kScanSingleMax) {
     hipLaunchKernelGGL(scan_single_block_kernel, dim3(1), dim3(kScanSingleThreads), 0, stream, n,
-                       vec, counts, total_dev);
+                       vec, counts, total_dev, flag);
     MCCNN_LAUNCH_CHECK();
     return MCCNN_OK;
   }
@@ -221,24 +229,24 @@ int inclusive_scan_i32(hipStream_t stream, int64_t n, int *counts, int *block_su
   MCCNN_LAUNCH_CHECK();
   if (nb <= kScanMaxOwnPrefix) {
     hipLaunchKernelGGL(scan_apply_kernel<true>, dim3(nb), dim3(kScanThreads), 0, stream, n, vec,
-                       counts, block_sums, total_dev);
+                       counts, block_sums, total_dev, flag);
     MCCNN_LAUNCH_CHECK();
     return MCCNN_OK;
   }
   hipLaunchKernelGGL(scan_block_sums_kernel, dim3(1), dim3(kScanThreads), 0, stream, nb,
-                     block_sums, total_dev);
+                     block_sums, total_dev, flag);
   MCCNN_LAUNCH_CHECK();
   hipLaunchKernelGGL(scan_apply_kernel<false>, dim3(nb), dim3(kScanThreads), 0, stream, n, vec,
-                     counts, block_sums, total_dev);
+                     counts, block_sums, total_dev, (const int64_t *)nullptr);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
 
 template <class T>
-static int wait_for_values(hipStream_t s, const volatile T *values, int n) {
+static int wait_for_values(hipStream_t s, const T *values, int n) {
   const auto start = std::chrono::steady_clock::now();
   for (int i = 0; i < n;) {
-    if (values[i] != (T)-1) {
+    if (__atomic_load_n(&values[i], __ATOMIC_ACQUIRE) != (T)-1) {
       ++i;
       continue;
     }
@@ -248,14 +256,13 @@ static int wait_for_values(hipStream_t s, const volatile T *values, int n) {
       return MCCNN_OK;
     }
   }
-  std::atomic_thread_fence(std::memory_order_acquire);
   return MCCNN_OK;
 }
 
-int wait_for_host_values(hipStream_t s, const volatile int64_t *values, int n) {
+int wait_for_host_values(hipStream_t s, const int64_t *values, int n) {
   return wait_for_values(s, values, n);
 }
-int wait_for_host_values(hipStream_t s, const volatile int32_t *values, int n) {
+int wait_for_host_values(hipStream_t s, const int32_t *values, int n) {
   return wait_for_values(s, values, n);
 }
 

@@ -60,3 +60,24 @@ def test_counts_from_several_threads():
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("n", [300, 40000, 4300000])
+def test_cut_lists_are_reported_with_the_count(n):
+    """Whether a list was cut comes with the number of pairs, for every form of the scan behind the
+    counts: a limit that cuts none, one that cuts the longest lists only, one that cuts most."""
+    from tensorflow_graphics_point_clouds_amd import _lib, pc
+    points, ids = _cloud(n, 5)
+    grid = pc.Grid(pc.PointCloud(points[:, :2].contiguous(), ids, 2), (2.0 / n) ** 0.5)
+    pts, bids, keys, ds, cells, smin, inv_cell = grid.search_tensors()
+    inv_radii = pc._reciprocal(grid._cell_sizes)
+    search = lambda limit: _lib.host().search(pts, bids, pts, keys, ds, cells, smin, inv_cell,
+                                              inv_radii, limit)
+    ranges, pairs, cut = search(0)
+    counts = torch.diff(ranges, prepend=ranges.new_zeros(1))
+    assert not cut and pairs.shape[0] == int(ranges[-1])
+    most = int(counts.max())
+    for limit in (most, most - 1, most + 5, 2, most - 1, most):
+        ranges, pairs, cut = search(limit)
+        assert cut == (limit < most)
+        assert pairs.shape[0] == int(ranges[-1]) == int(counts.clamp(max=limit).sum())
