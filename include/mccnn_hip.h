@@ -113,7 +113,10 @@ int mccnn_build_grid(mccnn_stream_t stream, int64_t num_pts, int num_dims,
                      int32_t *num_cells_out_host, int *key_bits_out_host);
 
 /* The same with the host copy of the shape written by the kernel itself into pinned host memory
- * (hipHostMalloc) that stays valid until the call returns.  num_cells_out_pinned and
+ * that stays valid until the call returns: memory of hipHostMalloc (its default, coherent
+ * memory).  Here and wherever a name ends in _pinned the host looks at the memory while the
+ * kernels run, without a pause, and waits for the stream if nothing has arrived after 20 ms: the
+ * stream may still be busy with kernels of the call when it returns.  num_cells_out_pinned and
  * key_bits_out_host may both be NULL, never one of them, where
  * mccnn_build_grid_is_single_launch (up to mccnn_build_grid_single_launch_max() points, at least
  * one, and at most 512 extents batch_size * num_dims): the whole grid is then one launch and the
@@ -333,7 +336,7 @@ int mccnn_find_neighbors_fill(
 /* The count half of a search by a caller with a grid in hand: mccnn_find_neighbors_count without
  * the op's shape checks, grid_ds may be NULL (the whole key array is searched: no host copy of
  * the grid's shape is needed, for clouds of a few thousand points), and result_pinned [2] is
- * pinned host memory (hipHostMalloc) that the kernels write: the number of pairs, and 1 if some
+ * pinned host memory (as for mccnn_build_grid_pinned) for the number of pairs, and 1 if some
  * centre lost pairs to max_neighs.  Workspace: mccnn_find_neighbors_workspace_bytes; continued by
  * mccnn_find_neighbors_fill. */
 int mccnn_search_count(mccnn_stream_t stream, int64_t num_samples, int num_dims,
@@ -581,7 +584,7 @@ int mccnn_sampling_count(mccnn_stream_t stream, int mode, int64_t num_pts,
                          int64_t ranges_len, const int32_t *ranges,
                          void *workspace, size_t workspace_bytes,
                          int64_t *num_sampled_out_host);
-/* The same with the number in pinned host memory (hipHostMalloc) that the kernels write. */
+/* The same with the number in pinned host memory (as for mccnn_build_grid_pinned). */
 int mccnn_sampling_count_pinned(mccnn_stream_t stream, int mode, int64_t num_pts,
                          int num_dims, const float *points,
                          int64_t batch_ids_len, const int32_t *batch_ids,
