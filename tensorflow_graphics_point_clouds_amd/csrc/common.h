@@ -132,6 +132,15 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The same among the lanes of a group that shares a piece of LDS with no other lane of the
+// wavefront.  The group's lanes must reach it together; the others may be in another iteration of
+// the loop around it, or gone, and what they have in LDS is not ordered by it.
+__device__ __forceinline__ void group_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Barrier of the block that orders its LDS traffic only: what any thread wrote to LDS
 // before the call is what every thread reads after it.  Unlike __syncthreads() it does not
 // wait for the wavefront's outstanding global loads and stores (a prefetch in flight,

@@ -319,8 +319,9 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
       upto += sub >= off ? o : 0;
     }
     const int before1 = __shfl(upto, kGroup - 1, kGroup), total = before1 + n1;
+    // (as many windows as the group has: the wavefront's other groups have lists of their own)
     for (int t0 = 0; t0 < total; t0 += kTrips) {                // a window of the trips
-      wave_lds_sync();                                          // the window before has been read
+      group_lds_sync();                                         // the window before has been read
       const int first = upto - n0 - t0;
       for (int k = first < 0 ? -first : 0; k < n0 && first + k < kTrips; ++k)
         trip[first + k] = make_int2(mine[0].x + kGroup * k, mine[0].y);
@@ -329,7 +330,7 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
           trip[before1 + k - t0] = make_int2(mine[1].x + kGroup * k, mine[1].y);
       const int n = total - t0 < kTrips ? total - t0 : kTrips;
       if (sub < kAhead) trip[n + sub] = make_int2(0, 0);        // (no candidates)
-      wave_lds_sync();
+      group_lds_sync();
       const bool masked = r0 == 0 && t0 < kTrips * kMaskWindows;
       const int64_t mask_at = ((int64_t)(t0 / kTrips) * ns + c) * kGroup + sub;
       if (kVisit == Visit::kFill && masked) {
