@@ -233,23 +233,24 @@ GridTensors build_grid(const Tensor &points, const Tensor &bids, int64_t batch,
 void check_search(const Tensor &samples, const Tensor &sbids, const Tensor &num_cells,
                   const Tensor &smin, const Tensor &inv_cell);
 
-// Centres in the order of their cells in a grid -> (order, coordinates, cloud ids, cell keys).
-std::tuple<Tensor, Tensor, Tensor, Tensor> order_centres(const Tensor &samples, const Tensor &bids,
-                                                 int64_t batch, const Tensor &num_cells,
-                                                 const Tensor &smin, const Tensor &inv_cell,
-                                                 int64_t key_bits) {
+// Centres in the order of their cells in a grid -> (order, coordinates, cloud ids, cell keys or
+// nothing unless `want_keys`).
+std::tuple<Tensor, Tensor, Tensor, OptTensor> order_centres(
+    const Tensor &samples, const Tensor &bids, int64_t batch, const Tensor &num_cells,
+    const Tensor &smin, const Tensor &inv_cell, int64_t key_bits, bool want_keys) {
   check_search(samples, bids, num_cells, smin, inv_cell);
   const int64_t n = samples.size(0), d = samples.size(1);
   Tensor order = empty_i32({n}, samples), pts = empty_f32({n, d}, samples),
-         out_bids = empty_i32({n}, samples),
-         keys = at::empty({n}, samples.options().dtype(at::kLong).requires_grad(false));
+         out_bids = empty_i32({n}, samples);
+  OptTensor keys;
+  if (want_keys) keys = empty_i64({n}, samples);
   Tensor ws = workspace(mccnn_order_centres_workspace_bytes(n), samples);
   hipStream_t s = current_stream();
   Region r("order_centres", s);
   check(mccnn_order_centres_keys(s, n, (int)d, f32(samples), i32(bids), (int)batch,
                                  i32(num_cells), f32(smin), f32(inv_cell), (int)key_bits,
                                  ws.data_ptr(), ws.numel(), i32(order), f32(pts), i32(out_bids),
-                                 i64(keys)));
+                                 keys ? i64(*keys) : nullptr));
   return {order, pts, out_bids, keys};
 }
 
@@ -1589,7 +1590,9 @@ PYBIND11_MODULE(_host, m) {
   m.def("start_timing", &start_timing);
   m.def("collect_timing", &collect_timing);
   m.def("compute_keys", &compute_keys, release());
-  m.def("order_centres", &order_centres, release());
+  m.def("order_centres", &order_centres, py::arg("samples"), py::arg("batch_ids"),
+        py::arg("batch_size"), py::arg("num_cells"), py::arg("scaled_aabb_min"),
+        py::arg("inv_cell_sizes"), py::arg("key_bits"), py::arg("want_keys") = false, release());
   m.def("search_known", &search_known, release());
   m.def("invert_order", &invert_order, release());
   m.def("build_grid", &build_grid, release());

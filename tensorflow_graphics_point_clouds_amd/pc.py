@@ -400,19 +400,10 @@ class _SortedView:
             self._centre_order = self.centre_rows.long()
         return self._centre_order
 
-    # Up to this many points and centres the transposed table of a search without a limit is the
-    # search from the points among the centres, three launches: the pairs are the same (cells of a
-    # pair are neighbours either way, and the distance test is exact under negation) and so is
-    # their order (ascending slots).  Regrouping the pairs by a sort is nine launches: 35 against
-    # 24 us of kernels for 16 x 1024 points and their cell averages.  Beyond, a search without a
-    # column table of the centres costs more than the sort.
-    _MOST_SEARCHED_BACK = 16384
-
     def _search_among_centres(self, nbh):
         """Arguments of that search, or None where it does not apply."""
         grid = nbh._grid
-        if nbh.max_neighbors != 0 or nbh._sorted_cells is None or self._transposed is not None or \
-                max(self.points_in.shape[0], self.points_out.shape[0]) > self._MOST_SEARCHED_BACK:
+        if nbh._sorted_cells is None or self._transposed is not None:
             return None
         bids, cells = nbh._sorted_cells
         return (self.points_in.detach(), grid._sorted_batch_ids, self.points_out, cells,
@@ -479,6 +470,14 @@ class Neighborhood:
     """Neighbour pairs of the centres `point_cloud_sample` (default: the grid's
     own sorted points) inside `grid` (pylib/pc/Neighborhood.py:218-311)."""
 
+    # Up to this many points and centres the transposed table of a search without a limit is the
+    # search from the points among the centres, three launches: the pairs are the same (cells of a
+    # pair are neighbours either way, and the distance test is exact under negation) and so is
+    # their order (ascending slots).  Regrouping the pairs by a sort is nine launches: 35 against
+    # 24 us of kernels for 16 x 1024 points and their cell averages.  Beyond, a search without a
+    # column table of the centres costs more than the sort, and their cells are not kept.
+    _MOST_SEARCHED_BACK = 16384
+
     def __init__(self, grid, radius, point_cloud_sample=None, max_neighbors=0, lazy=False):
         """`lazy` puts the search off until the pair table is first read (a hierarchy keeps a
         neighbourhood per level that it never reads itself)."""
@@ -532,13 +531,15 @@ class Neighborhood:
             return
         # (an order of few centres is one launch, which does not need the width of the keys)
         one_launch = s._points.shape[0] <= _lib.lib().mccnn_build_grid_single_launch_max()
+        back = self.max_neighbors == 0 and \
+            max(points.shape[0], s._points.shape[0]) <= self._MOST_SEARCHED_BACK
         order, pts, bids, cells = _lib.host().order_centres(
             s._points.detach(), s._batch_ids, grid._batch_size, num_cells, smin, inv_cell,
-            0 if one_launch else grid._key_bits)
+            0 if one_launch else grid._key_bits, back)
         ranges, table, _ = _lib.host().search(pts, bids, points, keys, ds, num_cells, smin,
                                               inv_cell, self._inv_radii, self.max_neighbors)
         self._sorted = (order, pts, ranges, table)
-        self._sorted_cells = (bids, cells)
+        self._sorted_cells = (bids, cells) if back else None
 
     def _unsearched_own(self):
         """Whether this is the whole neighbourhood of the grid's own points and its search has been
