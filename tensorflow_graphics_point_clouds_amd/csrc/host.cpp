@@ -757,15 +757,20 @@ Packed pack(const Plan &p, int64_t first, const Tensor &final_weights,
 // the transposed projection Q [N, F, K] of dout,
 //     dfeat[j, c]  = sum_{i in T(j)} sum_k basis[ij, k] G[i, c, k],
 //     dW[c, k, f]  = sum_i proj[i, c, k] dout[i, f],
-// with the projection computed again.  What is written and read then grows with C, not with F.
+// with the projection computed again.  What is written and read per centre then grows with C, not with
+// F; what is gathered per pair grows with 16 C for the 4, 8 or 16 channels that are gathered, not with F.
 // `wide`: the columns that dout and W are padded to for the products, 0 where this does not apply.
-// KPConv 8 -> 96 on 558 617 points of 12 pairs: 3.16 -> 1.76 ms for the pass (transposed projection,
-// its two products: 2.42 ms; gradient of the projection, gather, projection, product: 1.01); MCConv
-// 16 -> 128 on 8726 of 54: 208 -> 184 us of kernels.  At F = C both sides move as much.
-int64_t narrow_columns(const Plan &p, int64_t n_out) {
-  const int64_t f = p.f(), r = p.c_pad * p.k();
-  if (p.k() != 16 || p.c_pad != 16 || f < 2 * p.c_pad || (p.per != 1 && p.g_pad != p.g) ||
-      n_out * r >= (int64_t)1 << 30)
+// From five columns per gathered channel on it is the faster one whatever the lists (two passes of
+// 500 k points, other way / this way: KPConv 16 -> 96 1.47 with lists of 10, 0.95 with 55, 4 -> 32 1.14
+// and 0.93, 7 -> 48 1.35 and 1.16; MCConv 16 -> 80 1.44 and 1.02, 4 -> 32 1.22 and 1.01); from three
+// on with short lists only (MCConv 16 -> 48 and 64 1.15 and 1.22 with lists of 10, 0.86 with 37,
+// KPConv 1.06 and 1.10, 0.79 and 0.78; 8 -> 32 1.08 and 0.98 with 10, with 25 0.98 and 0.89); with two never
+// (16 -> 32 of 10: 0.89 and 0.78, of 37: 0.62 and 0.53).
+int64_t narrow_columns(const Plan &p, int64_t n_out, int64_t pairs) {
+  const int64_t f = p.f(), r = p.c_pad * p.k(), live = p.c <= 4 ? 4 : p.c <= 8 ? 8 : 16;
+  const bool pays = f >= 5 * live || (f >= 3 * live && pairs <= 16 * n_out);
+  if (p.k() != 16 || p.c_pad != 16 || f < 2 * p.c_pad || !pays ||
+      (p.per != 1 && p.g_pad != p.g) || n_out * r >= (int64_t)1 << 30)
     return 0;
   const int64_t wide = f == 32 ? 32 : (f + 63) / 64 * 64;
   if (wide != f && p.per != 1) return 0;
@@ -836,13 +841,13 @@ Tensor cut_columns(const Tensor &x, int64_t cols) {
 // whose products keep the register-resident kernel, where a pass is chains of loads and launches.
 // Per output element the sums are those of the sub-layers on their own.
 // Layer of 6 -> 32 channels, 4 x 8 hidden units, 61 k points of 28 pairs: 592 -> 490 us for the pass, 53 -> 39 launches.
-bool paired(const Plan &p, int64_t n_out, int64_t n_in, bool grads) {
+bool paired(const Plan &p, int64_t n_out, int64_t n_in, int64_t pairs, bool grads) {
   const int64_t f = p.f(), r = p.c_pad * p.k();
   if (p.mlps != 2 * p.per || p.k() != 16 || p.g_pad != p.g || p.cols() != f ||
       n_in * 2 * std::max(p.c_pad, f) >= (int64_t)1 << 30 || n_out * 2 * f >= (int64_t)1 << 30 ||
       product_kind(n_out, r, f) != Product::kRegisters)
     return false;
-  return !grads || (narrow_columns(p, n_out) == 0 &&
+  return !grads || (narrow_columns(p, n_out, pairs) == 0 &&
                     product_kind(n_in, f * 16, p.c_pad) == Product::kRegisters &&
                     product_kind(n_in, 2 * f * 16, p.c_pad) == Product::kRegisters &&
                     mccnn_projection_grad_product_supported((int)(2 * f), (int)(2 * r)) &&
@@ -906,10 +911,11 @@ struct McConv : torch::autograd::Function<McConv> {
     const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
     const int64_t n_out = geo->ranges.size(0);
     std::vector<Tensor> outs;
-    const bool narrow = grads && narrow_columns(p, n_out) > 0;
+    const int64_t pairs = geo->table.size(0);
+    const bool narrow = grads && narrow_columns(p, n_out, pairs) > 0;
     variable_list saved = {feats, kw, kb, final_weights,
                            p.c == p.c_pad && !narrow ? features : Tensor()};
-    const bool pair = paired(p, n_out, feats.size(0), grads);
+    const bool pair = paired(p, n_out, feats.size(0), pairs, grads);
     if (pair) {
       Tensor forward;
       const Packed w = pack_pair(p, final_weights, kw, kb, grads, &forward);
@@ -960,7 +966,7 @@ struct McConv : torch::autograd::Function<McConv> {
       dkb = at::empty_like(kb);
     }
     if (want_final) dfinal = at::empty_like(fw);
-    const int64_t wide = narrow_columns(p, n_out);
+    const int64_t wide = narrow_columns(p, n_out, geo->table.size(0));
     if (wide > 0 && want_feat) dfeat = empty_f32({geo->ranges_t.size(0), p.c}, feats);
     hipStream_t s = current_stream();
     const bool pair = saved.size() == 5 + Packed::kTensors && p.mlps == 2 * p.per;
@@ -1093,7 +1099,7 @@ struct KpConv : torch::autograd::Function<KpConv> {
                         const Tensor &kernel_points, const c10::intrusive_ptr<Geometry> &geo,
                         const Plan &p, const KpShape &kp, bool grads) {
     const Tensor feats = gather_rows(features, geo->point_rows, 0, p.c, p.c_pad);
-    const bool narrow = grads && narrow_columns(p, geo->ranges.size(0)) > 0;
+    const bool narrow = grads && narrow_columns(p, geo->ranges.size(0), geo->table.size(0)) > 0;
     const Packed w = pack(p, 0, weights, Tensor(), Tensor(), geo->ranges.size(0), feats.size(0),
                           narrow, grads && !narrow);
     const Tensor proj = kp_project(kp, kernel_points, p.k(), feats, geo->points_in,
@@ -1125,7 +1131,8 @@ struct KpConv : torch::autograd::Function<KpConv> {
         ctx->saved_data["geo"].toCapsule());
     const Packed w = Packed::saved(saved, 3);
     const Tensor dout = grad_out[0].contiguous();
-    const int64_t n_out = geo->ranges.size(0), wide = narrow_columns(p, n_out);
+    const int64_t n_out = geo->ranges.size(0);
+    const int64_t wide = narrow_columns(p, n_out, geo->table.size(0));
     const Tensor up = geo->centre_rows.defined() || p.g_pad != p.g || wide > p.f()
                           ? (wide > 0 ? gather_upstream(p, dout, geo->centre_rows, 0, wide)
                                       : gather_upstream(p, dout, geo->centre_rows, 0)) : dout;
