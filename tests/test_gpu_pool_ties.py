@@ -9,11 +9,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("c", [1, 2, 3, 4, 5, 12, 48, 100, 256, 260])
 @pytest.mark.parametrize("values", ["distinct", "ties", "unaligned"])
-def test_max_pooling_with_ties(c, values):
+def test_max_pooling_with_ties(c, values, most=39):
     from tensorflow_graphics_point_clouds_amd import _lib
     gen = torch.Generator(device="cuda").manual_seed(c)
     n, n_out = 500, 301
-    counts = torch.randint(0, 40, (n_out,), device="cuda", generator=gen)
+    counts = torch.randint(0, most + 1, (n_out,), device="cuda", generator=gen)
     counts[::7], counts[5], counts[6] = 0, 200, 64
     ranges = torch.cumsum(counts, 0).int()
     seg = torch.repeat_interleave(torch.arange(n_out, device="cuda"), counts)
@@ -41,3 +41,12 @@ def test_max_pooling_with_ties(c, values):
     mag = torch.zeros(n, c, dtype=torch.float64, device="cuda").index_add(0, ids, share.abs())
     # a point is in at most 301 lists: as many float32 additions of rounded shares
     assert bool(((grad.double() - want).abs() <= 302 * 2.0 ** -24 * mag).all())
+
+
+# lists of 12 pairs on average (20 for up to eight channels) and more go to the kernel that reads whole
+# rows: lists well below and above, and just about, either number
+@pytest.mark.parametrize("c", [4, 8, 12, 64, 256])
+@pytest.mark.parametrize("values", ["distinct", "ties"])
+@pytest.mark.parametrize("most", [2, 26, 46, 90])
+def test_max_pooling_of_short_and_long_lists(c, values, most):
+    test_max_pooling_with_ties(c, values, most)
