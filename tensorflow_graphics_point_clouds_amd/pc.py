@@ -475,8 +475,10 @@ class Neighborhood:
     # pair are neighbours either way, and the distance test is exact under negation) and so is
     # their order (ascending slots).  Regrouping the pairs by a sort is nine launches: 35 against
     # 24 us of kernels for 16 x 1024 points and their cell averages.  Beyond, a search without a
-    # column table of the centres costs more than the sort, and their cells are not kept.
-    _MOST_SEARCHED_BACK = 16384
+    # column table of the centres costs more than the sort, and their cells are not kept.  So does
+    # one of 81 cell rows and more per point, from five dimensions on (5000 points and a third as many
+    # centres, both searches and the transposed table: 174 against 128 us).
+    _MOST_SEARCHED_BACK, _MOST_DIMS_SEARCHED_BACK = 16384, 4
 
     def __init__(self, grid, radius, point_cloud_sample=None, max_neighbors=0, lazy=False):
         """`lazy` puts the search off until the pair table is first read (a hierarchy keeps a
@@ -531,7 +533,7 @@ class Neighborhood:
             return
         # (an order of few centres is one launch, which does not need the width of the keys)
         one_launch = s._points.shape[0] <= _lib.lib().mccnn_build_grid_single_launch_max()
-        back = self.max_neighbors == 0 and \
+        back = self.max_neighbors == 0 and points.shape[1] <= self._MOST_DIMS_SEARCHED_BACK and \
             max(points.shape[0], s._points.shape[0]) <= self._MOST_SEARCHED_BACK
         order, pts, bids, cells = _lib.host().order_centres(
             s._points.detach(), s._batch_ids, grid._batch_size, num_cells, smin, inv_cell,

@@ -45,18 +45,22 @@ def test_search_back_checks_dimensions():
         _lib.host().search_known(f(4, 3), i(4), f(5, 3), keys[:4], i(3), f(1, 3), f(3), f(3), 7)
 
 
-@pytest.mark.parametrize("n,n_out,limit,kept", [(16384, 300, 0, True), (300, 16384, 0, True),
-                                                (16385, 300, 0, False), (300, 16385, 0, False),
-                                                (300, 200, 4, False)])
-def test_cells_of_centres_are_kept_where_they_are_searched(n, n_out, limit, kept):
+@pytest.mark.parametrize("d,n,n_out,limit,kept", [
+    (3, 16384, 300, 0, True), (3, 300, 16384, 0, True), (3, 16385, 300, 0, False),
+    (3, 300, 16385, 0, False), (3, 300, 200, 4, False), (4, 300, 200, 0, True),
+    (5, 300, 200, 0, False), (6, 300, 200, 0, False)])
+def test_cells_of_centres_are_kept_where_they_are_searched(d, n, n_out, limit, kept):
     """Neighbourhoods that are never searched back hold no cell keys or cloud ids of their centres."""
     from tensorflow_graphics_point_clouds_amd import pc
-    cloud = lambda m: pc.PointCloud(torch.rand(m, 3, device="cuda"),
+    cloud = lambda m: pc.PointCloud(torch.rand(m, d, device="cuda"),
                                     torch.zeros(m, dtype=torch.int32, device="cuda"), 1)
-    nbh = pc.Neighborhood(pc.Grid(cloud(n), 0.1), 0.1, cloud(n_out), max_neighbors=limit)
+    r = 0.1 if d == 3 else 0.3
+    nbh = pc.Neighborhood(pc.Grid(cloud(n), r), r, cloud(n_out), max_neighbors=limit)
     assert (nbh._sorted_cells is not None) == kept
     if kept:
         assert nbh._sorted_cells[1].shape == (n_out,)
     view = nbh.sorted_view()
     assert (view._search_back is not None) == kept
-    assert view.table_t.shape == view.table.shape
+    # the pairs by point, each list in ascending slots
+    order = torch.argsort(view.table[:, 0].long() * n_out + view.table[:, 1].long())
+    assert torch.equal(view.table_t, view.table[order][:, [1, 0]])
