@@ -548,6 +548,22 @@ class Neighborhood:
         put off so far."""
         return self._equal_samples and self.max_neighbors == 0 and self._table is None
 
+    # Dimensions up to which a Poisson-disk sample of cells of one radius is selected from the grid.
+    # In more, the cells around one hold more selected points than the registers of a wavefront,
+    # and each point is then compared with all of them from memory: 20 000 points of 40 neighbours
+    # in five dimensions 0.78 ms with the pair table, 3.1 from the grid; in four (30 000) 0.52 and 0.30.
+    _MOST_DIMS_SELECTED_FROM_GRID = 4
+
+    def _selects_from_grid(self):
+        """Whether a Poisson-disk sample is selected faster from the grid than from the pair table, which
+        has to be searched for it.  Radii well below the cell size have the same effect as more
+        dimensions: in four, cells of one radius only (radii of 0.4 cells, as above: 0.44 and 1.8 ms);
+        up to three the grid is 1.2 to 1.5 times faster with those as well, but for hundreds of
+        points in a cell (0.52 and 0.70 ms)."""
+        dims = self._grid._sorted_points.shape[1]
+        one_radius = self._radii.data_ptr() == self._grid._cell_sizes.data_ptr()
+        return dims <= 3 or (dims <= self._MOST_DIMS_SELECTED_FROM_GRID and one_radius)
+
     def _sorted_search(self):
         """(centre order, centres, ranges, pairs) with the centres in the order of their cells."""
         if self._sorted is None:
@@ -708,6 +724,8 @@ def sample(neighborhood, sample_mode="poisson"):
     """pylib/pc/sampling.py:123-150 -> (PointCloud, original indices or None)."""
     mode = _SAMPLE_MODES[sample_mode.lower()]
     g = neighborhood._grid
+    if mode == 0 and neighborhood._unsearched_own() and not neighborhood._selects_from_grid():
+        neighborhood = Neighborhood(g, neighborhood._radii)       # (the caller's stays put off)
     if mode == 0 and neighborhood._unsearched_own():
         # the selection from the grid itself: as from the pair table, which it does not need
         points, ids, keys, ds, num_cells, _, _ = g.search_tensors()
@@ -731,6 +749,13 @@ def sample(neighborhood, sample_mode="poisson"):
     return PointCloud(pts, bids, g._batch_size), original
 
 
+def _sampling_neighborhood(grid, sample_mode):
+    """The grid's own neighbourhood for cells of one radius, searched only if sampling reads its pairs."""
+    reads = _SAMPLE_MODES[sample_mode.lower()] == 0 and \
+        grid._sorted_points.shape[1] > Neighborhood._MOST_DIMS_SELECTED_FROM_GRID
+    return Neighborhood(grid, grid._cell_sizes, lazy=not reads)
+
+
 def poisson_disk_sampling(point_cloud, radius=None, neighborhood=None, return_ids=False):
     """Poisson-disk sample of a point cloud (pylib/pc/sampling.py:31-78) -> PointCloud
     (and the original indices of the kept points).  The reference passes the mode
@@ -739,7 +764,7 @@ def poisson_disk_sampling(point_cloud, radius=None, neighborhood=None, return_id
         raise ValueError("Missing Argument! Either radius or neighborhood must be given!")
     if neighborhood is None:
         radii = _as_vector(radius, point_cloud._dimension, point_cloud._points.device)
-        neighborhood = Neighborhood(Grid(point_cloud, radii), radii, lazy=True)
+        neighborhood = _sampling_neighborhood(Grid(point_cloud, radii), "poisson")
     cloud, ids = sample(neighborhood, "poisson")
     return (cloud, ids) if return_ids else cloud
 
@@ -768,7 +793,7 @@ class PointHierarchy:
             cs = _as_vector(cs, point_cloud._dimension, point_cloud._points.device)
             self._cell_sizes.append(cs)
             grid = Grid(cur, cs)
-            nbh = Neighborhood(grid, cs, lazy=True)
+            nbh = _sampling_neighborhood(grid, sample_mode)
             cur, idx = sample(nbh, sample_mode)
             self._neighborhoods.append(nbh)
             self._point_clouds.append(cur)
