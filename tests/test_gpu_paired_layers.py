@@ -1,6 +1,6 @@
 """Layers whose two sub-layers run side by side give what two layers of half the kernel MLPs give:
 the same bits forward, gradients within the rounding of their sums; channels from one to the
-widest, points without neighbours, runs of one and two centres, single gradients."""
+widest, points without neighbours, runs of one to eight centres and points, single gradients."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -12,11 +12,10 @@ pytestmark = pytest.mark.gpu
     (3, 6, 32, 4, 8, 431), (3, 1, 32, 2, 16, 431), (2, 6, 32, 4, 8, 300), (3, 16, 32, 4, 5, 1),
     (3, 32, 64, 4, 8, 700), (3, 64, 128, 4, 8, 333), (3, 128, 64, 2, 16, 100),
     (3, 100, 32, 4, 8, 250), (3, 8, 32, 4, 8, 21001)])
-def test_paired_sub_layers(d, c, f, mlps, hidden, n_out):
+def test_paired_sub_layers(d, c, f, mlps, hidden, n_out, n_in=900, r=0.16):
     from tensorflow_graphics_point_clouds_amd import layers, pc
     gen = torch.Generator(device="cuda").manual_seed(100 * c + f)
     rand = lambda *shape: torch.rand(shape, device="cuda", generator=gen)
-    n_in, r = 900, 0.16
     pts, ctr = rand(n_in, d), rand(n_out, d)
     pts[-20:] += 3.0                                        # points that no centre reaches
     ids = torch.arange(n_in, device="cuda").mul(2).div(n_in, rounding_mode="floor").int()
@@ -66,3 +65,21 @@ def test_paired_sub_layers(d, c, f, mlps, hidden, n_out):
         p.requires_grad_(False)
     got, = torch.autograd.grad(both(z, cin, cout, r, neighborhood=nbh), z, up)
     assert torch.equal(got, x.grad)
+
+
+# runs of 2 | 4 | 8 centres forward, and points backward, change at 20 000, 64 000 and 160 000; some six
+# pairs a centre, none for one in some hundred, and last runs that are not full
+@pytest.mark.parametrize("d,c,f,mlps,hidden,n_in,n_out,r", [
+    (3, 6, 32, 4, 8, 64003, 64003, 0.036), (2, 16, 32, 4, 8, 64003, 20001, 0.0077),
+    (3, 3, 32, 2, 16, 160005, 64001, 0.0262), (3, 6, 32, 4, 5, 64001, 160003, 0.0355),
+    (3, 32, 64, 4, 8, 160005, 160005, 0.0262)])
+def test_paired_sub_layers_in_longer_runs(d, c, f, mlps, hidden, n_in, n_out, r):
+    from tensorflow_graphics_point_clouds_amd import _lib
+    _lib.start_timing()
+    try:
+        test_paired_sub_layers(d, c, f, mlps, hidden, n_out, n_in, r)
+    finally:
+        timed = _lib.collect_timing()
+    # one product in each of the layer's five forward and two transposed passes, and in those of the two
+    # layers that it is compared with (side by side: not two each)
+    assert len(timed["final_product"]) == 7 + 4
