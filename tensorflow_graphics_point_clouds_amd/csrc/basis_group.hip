@@ -185,7 +185,8 @@ struct GroupInfo {
 // for two blocks, the chain of dependent loads and probes took 5 of 13 ms.
 __global__ void __launch_bounds__(256) group_rows_kernel(
     int64_t n_out, int group, int max_rows, const int2 *__restrict__ nbrs,
-    const int *__restrict__ ranges, const int *__restrict__ order, unsigned short *__restrict__ row_of, int *__restrict__ keys,
+    const int *__restrict__ ranges, const int *__restrict__ order,
+    unsigned short *__restrict__ row_of, int *__restrict__ keys,
     GroupInfo *__restrict__ info, int64_t pairs, int num_basis, float *__restrict__ dbasis) {
   __shared__ int key[kHash];
   __shared__ int number[kHash];

@@ -291,7 +291,9 @@ __global__ void __launch_bounds__(256) basis_proj_tiles_kernel(
     if (c0 + 16 * j < C)
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
-        __builtin_nontemporal_store(acc[j][kt], reinterpret_cast<v4f_any *>(o + (int64_t)(c0 + 16 * j) * K + 16 * kt));
+        __builtin_nontemporal_store(
+            acc[j][kt],
+            reinterpret_cast<v4f_any *>(o + (int64_t)(c0 + 16 * j) * K + 16 * kt));
 }
 
 // Eight basis columns, more than 32 channels: a lane owns whole channels, lane + 64 j, with their eight
@@ -551,15 +553,21 @@ int launch_dfeat_gather(hipStream_t s, int64_t num_pts, int C, const int *point_
   if (num_pts == 0) return MCCNN_OK;
   const int lanes = C / 4;
   const dim3 grid(blocks_for(num_pts, 256 / lanes)), block(256);
+#define MCCNN_GATHER_ROWS(LANES_)                                                               \
+  case LANES_:                                                                                  \
+    hipLaunchKernelGGL(dfeat_gather_kernel<LANES_>, grid, block, 0, s, num_pts, point_ranges,   \
+                       pair_order, pair_rows, dfeat);                                           \
+    break
   switch (lanes) {
-    case 4: hipLaunchKernelGGL(dfeat_gather_kernel<4>, grid, block, 0, s, num_pts, point_ranges, pair_order, pair_rows, dfeat); break;
-    case 8: hipLaunchKernelGGL(dfeat_gather_kernel<8>, grid, block, 0, s, num_pts, point_ranges, pair_order, pair_rows, dfeat); break;
-    case 16: hipLaunchKernelGGL(dfeat_gather_kernel<16>, grid, block, 0, s, num_pts, point_ranges, pair_order, pair_rows, dfeat); break;
-    case 32: hipLaunchKernelGGL(dfeat_gather_kernel<32>, grid, block, 0, s, num_pts, point_ranges, pair_order, pair_rows, dfeat); break;
+    MCCNN_GATHER_ROWS(4);
+    MCCNN_GATHER_ROWS(8);
+    MCCNN_GATHER_ROWS(16);
+    MCCNN_GATHER_ROWS(32);
     default:
       set_error("feature-gradient gather supports C in {16, 32, 64, 128} (got %d)", C);
       return MCCNN_INVALID_ARGUMENT;
   }
+#undef MCCNN_GATHER_ROWS
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
@@ -667,15 +675,18 @@ extern "C" int mccnn_basis_proj_ordered(mccnn_stream_t stream, int64_t basis_row
     return MCCNN_OK;
   }
   if (num_basis == 8 && num_features > 32) {
-    const int per_lane = num_features > kWave ? 2 : 1, chunks = (num_features + kWave * per_lane - 1) / (kWave * per_lane);
+    const int per_lane = num_features > kWave ? 2 : 1;
+    const int chunks = (num_features + kWave * per_lane - 1) / (kWave * per_lane);
     const int64_t waves = num_samples * chunks;
     MCCNN_REQUIRE(waves < ((int64_t)1 << 31), "BasisProj launch too large");
     if (per_lane == 2)
-      hipLaunchKernelGGL(basis_proj_rows8_kernel<2>, dim3(wave_grid(waves)), dim3(256), 0, s, num_samples, num_features,
-                         chunks, basis, features, (const int2 *)neighbors, ranges, order, out);
+      hipLaunchKernelGGL(basis_proj_rows8_kernel<2>, dim3(wave_grid(waves)), dim3(256), 0, s,
+                         num_samples, num_features, chunks, basis, features,
+                         (const int2 *)neighbors, ranges, order, out);
     else
-      hipLaunchKernelGGL(basis_proj_rows8_kernel<1>, dim3(wave_grid(waves)), dim3(256), 0, s, num_samples, num_features,
-                         chunks, basis, features, (const int2 *)neighbors, ranges, order, out);
+      hipLaunchKernelGGL(basis_proj_rows8_kernel<1>, dim3(wave_grid(waves)), dim3(256), 0, s,
+                         num_samples, num_features, chunks, basis, features,
+                         (const int2 *)neighbors, ranges, order, out);
     MCCNN_LAUNCH_CHECK();
     return MCCNN_OK;
   }

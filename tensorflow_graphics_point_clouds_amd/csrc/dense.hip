@@ -217,11 +217,14 @@ __global__ void __launch_bounds__(256) tn_reduce_kernel(int64_t elems, int slice
 static int launch_tn_reduce(hipStream_t s, int64_t elems, int slices, const float *partials,
                             float *out) {
   if (elems <= 16384 && slices >= 64)
-    hipLaunchKernelGGL(tn_reduce_kernel<16>, dim3((unsigned)(elems / 16)), dim3(256), 0, s, elems, slices, partials, out);
+    hipLaunchKernelGGL(tn_reduce_kernel<16>, dim3((unsigned)(elems / 16)), dim3(256), 0, s, elems,
+                       slices, partials, out);
   else if (slices >= 16)
-    hipLaunchKernelGGL(tn_reduce_kernel<4>, dim3((unsigned)(elems / 64)), dim3(256), 0, s, elems, slices, partials, out);
+    hipLaunchKernelGGL(tn_reduce_kernel<4>, dim3((unsigned)(elems / 64)), dim3(256), 0, s, elems,
+                       slices, partials, out);
   else
-    hipLaunchKernelGGL(tn_reduce_kernel<1>, dim3((unsigned)(elems / 256)), dim3(256), 0, s, elems, slices, partials, out);
+    hipLaunchKernelGGL(tn_reduce_kernel<1>, dim3((unsigned)(elems / 256)), dim3(256), 0, s, elems,
+                       slices, partials, out);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }

@@ -840,7 +840,9 @@ Tensor cut_columns(const Tensor &x, int64_t cols) {
 // Whether the layer's two sub-layers run side by side, one launch of everything for both: inputs
 // whose products keep the register-resident kernel, where a pass is chains of loads and launches.
 // Per output element the sums are those of the sub-layers on their own.
-// Layer of 6 -> 32 channels, 4 x 8 hidden units, 61 k points of 28 pairs: 592 -> 490 us for the pass, 53 -> 39 launches.
+// Layer of 6 -> 32 channels, 4 x 8 hidden units, 61 k points of 28 pairs: 592 -> 490 us for the pass, 53 -> 39
+// launches.  Over 4 k to 200 k points, 6 to 128 inputs and 32 to 128 outputs the two apart take 1.0 (from
+// 61 k points and 64 channels on, where the kernels' own time is all) to 1.7 times as long.
 bool paired(const Plan &p, int64_t n_out, int64_t n_in, int64_t pairs, bool grads) {
   const int64_t f = p.f(), r = p.c_pad * p.k();
   if (p.mlps != 2 * p.per || p.k() != 16 || p.g_pad != p.g || p.cols() != f ||

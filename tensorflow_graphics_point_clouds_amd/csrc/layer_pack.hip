@@ -100,11 +100,12 @@ __global__ void __launch_bounds__(256) pack_layer_weights_kernel(
 }
 
 // The gradients back in the caller's shapes: final-weight gradient from the product's
-// [Cp, (f, k)] or [f, (c, k)] result (element (c, f, k) at c c_stride + f f_stride + k), kernel-MLP gradients from [mlps, D, Hp] and [mlps * Hp].
+// [Cp, (f, k)] or [f, (c, k)] result (element (c, f, k) at c c_stride + f f_stride + k), kernel-MLP
+// gradients from [mlps, D, Hp] and [mlps * Hp].
 __global__ void __launch_bounds__(256) unpack_layer_grads_kernel(
     LayerShapeArgs a, int D, int c_stride, int f_stride, const float *__restrict__ ddense,
-    const float *__restrict__ dkw_src, const float *__restrict__ dkb_src, float *__restrict__ dfinal, float *__restrict__ dkw,
-    float *__restrict__ dkb) {
+    const float *__restrict__ dkw_src, const float *__restrict__ dkb_src,
+    float *__restrict__ dfinal, float *__restrict__ dkw, float *__restrict__ dkb) {
   const int per = a.C * a.H * a.G, size = a.mlps * per, part = blockIdx.z;
   a.first += part * a.mlps;                    // (f of the parts one after the other)
   ddense += (int64_t)part * a.mlps * a.Gp * f_stride;
@@ -234,9 +235,9 @@ static int unpack_layer_grads(mccnn_stream_t stream, int num_dims, const LayerSh
   const unsigned grid = blocks_for(size > (1 << 20) ? (1 << 20) : size, 256);
   const int K = a.mlps * a.Hp, F = a.mlps * a.Gp;
   hipLaunchKernelGGL(unpack_layer_grads_kernel, dim3(grid, 1, (unsigned)parts), dim3(256), 0,
-                     as_stream(stream), a, num_dims, by_output ? K : parts * F * K, by_output ? a.Cp * K : K, dense_grads,
-                     kernel_weight_grads, kernel_bias_grads, final_grads_out, weight_grads_out,
-                     bias_grads_out);
+                     as_stream(stream), a, num_dims, by_output ? K : parts * F * K,
+                     by_output ? a.Cp * K : K, dense_grads, kernel_weight_grads,
+                     kernel_bias_grads, final_grads_out, weight_grads_out, bias_grads_out);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }

@@ -7,9 +7,9 @@
 // cell list and both outputs keep the sorted order (the reference compacts with
 // a global atomic counter and leaves the order to chance).  Poisson disk keeps
 // the reference's 2^D cell-parity launches; inside a launch one wavefront owns a
-// cell and decides its points in order (details at the kernel).  Cell averages are summed serially in sorted order so that the
-// result is bit-reproducible (later hierarchy levels derive integer keys from
-// these points).
+// cell and decides its points in order (details at the kernel).  Cell averages are
+// summed serially in sorted order so that the result is bit-reproducible (later
+// hierarchy levels derive integer keys from these points).
 #include "common.h"
 #include "fill.h"
 #include "search.h"

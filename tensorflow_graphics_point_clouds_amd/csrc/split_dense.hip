@@ -587,9 +587,18 @@ int launch_tn_split(hipStream_t s, int64_t n, int C, const float *x, int R, cons
   const int groups = R / kTnCols;
   const dim3 grid((unsigned)(groups * ((slices + 7) / 8) * 8)), block(kSplitThreads);
   switch (C) {
-    case 128: hipLaunchKernelGGL((tn_split_kernel<128, kTnCols, 3>), grid, block, 0, s, n, R, x, y, slices, partials); break;
-    case 64: hipLaunchKernelGGL((tn_split_kernel<64, kTnCols, 4>), grid, block, 0, s, n, R, x, y, slices, partials); break;
-    default: hipLaunchKernelGGL((tn_split_kernel<32, kTnCols, 4>), grid, block, 0, s, n, R, x, y, slices, partials); break;
+    case 128:
+      hipLaunchKernelGGL((tn_split_kernel<128, kTnCols, 3>), grid, block, 0, s, n, R, x, y, slices,
+                         partials);
+      break;
+    case 64:
+      hipLaunchKernelGGL((tn_split_kernel<64, kTnCols, 4>), grid, block, 0, s, n, R, x, y, slices,
+                         partials);
+      break;
+    default:
+      hipLaunchKernelGGL((tn_split_kernel<32, kTnCols, 4>), grid, block, 0, s, n, R, x, y, slices,
+                         partials);
+      break;
   }
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;

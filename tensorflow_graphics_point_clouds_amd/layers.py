@@ -913,8 +913,8 @@ def _kp_project(features, points_in, points_out, neighbors, ranges, inv_radii, k
 class _KPConvRigidLayer(torch.autograd.Function):
     """Rigid kernel-point convolution (KPConv.py:165-232) on the neighbourhood's
     grid-ordered view, for the shapes that KpConv of csrc/host.cpp does not cover (more than 32
-    kernel points, other dimensions or channel counts: through the op).  As for the Monte-Carlo convolution, the feature gradient is
-    the same convolution run from the centres back to the points over the
+    kernel points, other dimensions or channel counts: through the op).  As for the
+    Monte-Carlo convolution, the feature gradient is the same convolution run from the centres back to the points over the
     transposed pair table, with the kernel-point weights re-evaluated there
     (offset negated), and the weight gradient is feat^T Q; nothing is scattered and
     the basis gradient, which a rigid kernel does not need, is never formed."""
