@@ -282,8 +282,8 @@ __global__ void __launch_bounds__(kNbrThreads) nbr_visit_kernel(
   // The slices of the centre, nine at a time (their number is a power of three): lane `sub`
   // fetches or finds one, the first lane the ninth as well.  They are cut into trips of eight
   // candidates whose bounds go into LDS, and the group walks the list of trips, four in flight,
-  // without a branch but the end of the list.  Both passes are bound by instruction issue (vector
-  // units busy for 98 and 88 % of the time).  Slice by slice a trip took 45 instructions, a third
+  // without a branch but the end of the list.  The count pass is bound by instruction issue (its vector
+  // instructions, at four cycles each, fill the time), the fill pass for three quarters.  Slice by slice a trip took 45 instructions, a third
   // of them for the exec mask, and a wavefront took in each slice the trips of its fullest centre;
   // the list takes 24, and 14 in the fill pass, which neither loads nor tests the candidates.
   // 763 k centres x 37 pairs: count 150 -> 116 us, fill 216 -> 121; densities of 16 384 points
