@@ -127,6 +127,13 @@ __global__ void __launch_bounds__(kPoolThreads) local_pool_rows_kernel(
 // lane that saw it adds the gradient, and only centres with ties read their rows again to hand
 // out the shares.  (Every channel on a lane of its own with two passes of dependent loads:
 // 512 us for 64 channels on 38 k centres x 52 pairs, 138 us now.)
+// Short lists of 32 channels and more: a channel per lane, whose additions to a point are whole cache
+// lines where a few points hold the maxima of all channels, while those of a lane with four
+// channels are four times as many.  Decided per centre: samples of uneven clouds have lists of a few and
+// of hundreds.  32 channels of 213 k centres, 6.4 pairs on average, 18 as a pair sees it: 222 us by rows, 254
+// with a lane per channel for all, 129; 64 of 60 k centres of 3: 1.96 and 1 to 0.72.
+constexpr int kShortList = 12, kShortListChannels = 32;
+
 __global__ void __launch_bounds__(kPoolThreads) local_max_grads_rows_kernel(
     int64_t n_out, int C, int lpr_log2, const float *__restrict__ feat,
     const int2 *__restrict__ nbrs, const int *__restrict__ ranges, const float *__restrict__ out,
@@ -136,6 +143,36 @@ __global__ void __launch_bounds__(kPoolThreads) local_max_grads_rows_kernel(
   const int a = centre > 0 ? ranges[centre - 1] : 0, b = ranges[centre];
   if (b <= a) return;
   const int lane = lane_id();
+  if (C >= kShortListChannels && b - a < kShortList) {   // the same for the wavefront
+    const int cnt = b - a;
+    const int myidx = nbrs[a + (lane < cnt ? lane : 0)].x;
+    for (int c = lane; c < C; c += kWave) {
+      const float top = out[centre * C + c], grad = out_grads[centre * C + c];
+      int ties = 0, where = 0;
+      for (int m = 0; m < cnt; m += 4) {
+        float v[4];
+        int idx[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          idx[u] = __builtin_amdgcn_readlane(myidx, m + u < cnt ? m + u : cnt - 1);
+          v[u] = feat[(int64_t)idx[u] * C + c];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (m + u < cnt && v[u] == top) {
+            ++ties;
+            where = idx[u];
+          }
+      }
+      const float share = grad / (float)(ties > 0 ? ties : 1);
+      if (ties == 1) unsafeAtomicAdd(&dfeat[(int64_t)where * C + c], share);
+      for (int m = 0; m < cnt && __any(ties > 1); ++m) {
+        const int64_t at = (int64_t)__builtin_amdgcn_readlane(myidx, m) * C + c;
+        if (ties > 1 && feat[at] == top) unsafeAtomicAdd(&dfeat[at], share);
+      }
+    }
+    return;
+  }
   const int lpr = 1 << lpr_log2;
   const int slot = lane >> lpr_log2, colv = lane & (lpr - 1);
   const int slots = kWave >> lpr_log2;
@@ -421,13 +458,12 @@ extern "C" int mccnn_local_pool_grads(mccnn_stream_t stream, int kind, int64_t n
   MCCNN_REQUIRE(ranges && features && neighbors && out && out_grads,
                 "local_pool_grads received a null tensor");
   const int lpr_log2 = rows_lanes_log2(num_features);
-  // Short lists: a lane per channel, whose additions to a row are whole cache lines where a few points
-  // hold the maxima of all channels, while those of a lane with four channels are four times as many
-  // (64 channels on 60 k centres, lane per channel / rows: lists of 3 0.51, of 8 0.73, of 12 0.92, of 20
-  // 1.28; 4 channels on 250 k: 0.33, 0.53, 0.67, 0.96).
-  const int64_t long_list = num_features <= 8 ? 20 : 12;
-  if (kind == 0 && lpr_log2 >= 0 && num_neighbors >= long_list * num_samples &&
-      aligned16(features) && aligned16(out) && aligned16(out_grads)) {
+  // (few channels: several centres per wavefront where many short lists fill the chip either way; 4
+  // channels on 250 k centres of 5 0.43 of the time of rows, but 8 on 28 k of 5 1.8 times)
+  const bool packed = num_features < kShortListChannels && num_samples >= 128000 &&
+                      num_neighbors < 6 * num_samples;
+  if (kind == 0 && lpr_log2 >= 0 && !packed && aligned16(features) && aligned16(out) &&
+      aligned16(out_grads)) {
     hipLaunchKernelGGL(local_max_grads_rows_kernel, dim3(blocks_for(num_samples, kPoolThreads / kWave)),
                        dim3(kPoolThreads), 0, s, num_samples, num_features, lpr_log2, features,
                        (const int2 *)neighbors, ranges, out, out_grads, feature_grads_out);

@@ -43,10 +43,34 @@ def test_max_pooling_with_ties(c, values, most=39):
     assert bool(((grad.double() - want).abs() <= 302 * 2.0 ** -24 * mag).all())
 
 
-# lists of 12 pairs on average (20 for up to eight channels) and more go to the kernel that reads whole
-# rows: lists well below and above, and just about, either number
-@pytest.mark.parametrize("c", [4, 8, 12, 64, 256])
+# lists of fewer than 12 pairs are walked by a lane per channel from 32 channels on: nothing but such
+# lists, lists on either side, mostly longer ones; the last 64 channels not full
+@pytest.mark.parametrize("c", [4, 12, 28, 32, 64, 96, 256])
 @pytest.mark.parametrize("values", ["distinct", "ties"])
-@pytest.mark.parametrize("most", [2, 26, 46, 90])
+@pytest.mark.parametrize("most", [2, 11, 24, 90])
 def test_max_pooling_of_short_and_long_lists(c, values, most):
     test_max_pooling_with_ties(c, values, most)
+
+
+@pytest.mark.parametrize("c", [4, 16, 32])
+@pytest.mark.parametrize("n_out,k", [(127999, 5), (128000, 5), (128000, 6)])
+def test_max_pooling_of_many_short_lists(c, n_out, k):
+    """Either side of the number of centres from which short lists of few channels are packed."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(c + k)
+    seg = torch.repeat_interleave(torch.arange(n_out, device="cuda"), k)
+    ids = (7 * seg + torch.arange(k, device="cuda").repeat(n_out)) % n_out
+    pairs = torch.stack([ids, seg], dim=1).int().contiguous()
+    ranges = (k * torch.arange(1, n_out + 1, device="cuda")).int()
+    feat = torch.randint(0, 40, (n_out, c), device="cuda", generator=gen).float().requires_grad_(True)
+    up = torch.randn(n_out, c, device="cuda", generator=gen)
+    out = _lib.host().local_pool(feat, pairs, ranges, 0)
+    grad, = torch.autograd.grad(out, feat, up)
+    rows = feat.detach()[ids].reshape(n_out, k, c)
+    assert torch.equal(out, rows.amax(1))
+    top = rows == rows.amax(1, keepdim=True)
+    share = (top * (up / top.sum(1)).double()[:, None, :]).reshape(-1, c)
+    want = torch.zeros(n_out, c, dtype=torch.float64, device="cuda").index_add(0, ids, share)
+    mag = torch.zeros_like(want).index_add(0, ids, share.abs())
+    # a point is in at most k lists: as many float32 additions of rounded shares
+    assert bool(((grad.double() - want).abs() <= (k + 2) * 2.0 ** -24 * mag).all())
