@@ -177,6 +177,13 @@ struct GroupInfo {
   int direct;                        // a pair of the group has none
 };
 
+// The centres of a group that have pairs, from its first place in the order on (in a group without
+// pairs one centre of none).
+struct __align__(16) GroupCentre {
+  int centre, begin, count;          // its pairs
+  int flags;                         // 1: the group's last, 2: GroupInfo::direct, 4 x GroupInfo::rows
+};
+
 // The rows of a group: its points are numbered through a hash table, keys[kMaxRows g ..] are the
 // points by number and row_of[m] is the number of pair m.  A pair goes without a row when the
 // table is full or when its centre has listed its point before (the products of one centre are
@@ -187,7 +194,8 @@ __global__ void __launch_bounds__(256) group_rows_kernel(
     int64_t n_out, int group, int max_rows, const int2 *__restrict__ nbrs,
     const int *__restrict__ ranges, const int *__restrict__ order,
     unsigned short *__restrict__ row_of, int *__restrict__ keys,
-    GroupInfo *__restrict__ info, int64_t pairs, int num_basis, float *__restrict__ dbasis) {
+    GroupInfo *__restrict__ info, GroupCentre *__restrict__ listed /* optional */, int64_t pairs,
+    int num_basis, float *__restrict__ dbasis) {
   __shared__ int key[kHash];
   __shared__ int number[kHash];
   __shared__ unsigned seen[2][kMaxRows];          // centres of the group that list the row's point
@@ -243,7 +251,17 @@ __global__ void __launch_bounds__(256) group_rows_kernel(
     }
   }
   __syncthreads();
-  if (t == 0) info[blockIdx.x] = GroupInfo{rows < max_rows ? rows : max_rows, direct};
+  const int used = rows < max_rows ? rows : max_rows;
+  if (t == 0) info[blockIdx.x] = GroupInfo{used, direct};
+  if (listed && wave == 0) {                      // (n <= 64: a lane each)
+    const int count = lane < n ? end[lane] - begin[lane] : 0;
+    const unsigned long long any = __ballot(count > 0);
+    const int flags = (direct ? 2 : 0) + 4 * used;
+    if (count > 0)
+      listed[g0 + __popcll(any & ((1ull << lane) - 1ull))] =
+          GroupCentre{order[g0 + lane], begin[lane], count, flags + ((any >> lane) == 1 ? 1 : 0)};
+    if (any == 0 && lane == 0) listed[g0] = GroupCentre{order[g0], begin[0], 0, flags + 1};
+  }
   // rows of the table behind the last centre's pairs (a table of more capacity than pairs)
   for (int64_t i = (int64_t)ranges[n_out - 1] * num_basis + blockIdx.x * 256 + t;
        i < pairs * num_basis; i += (int64_t)gridDim.x * 256)
@@ -418,7 +436,9 @@ __global__ void __launch_bounds__(64 * W, 2) feature_grads_group_kernel(
         for (int u = 0; u < tiles; ++u)
           acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(gk[q], w[u][q], acc[u], 0, 0, 0);
     };
-    if (kTiles == 4 && c.left > 32) multiply(std::integral_constant<int, kTiles>{});
+    // (tiles of 16 without pairs are left out: 15.1 -> 14.8 ms where half of the centres have 49 or more)
+    if (kTiles == 4 && c.left > 48) multiply(std::integral_constant<int, kTiles>{});
+    else if (kTiles == 4 && c.left > 32) multiply(std::integral_constant<int, kTiles < 4 ? 2 : 3>{});
     else if (c.left > 16) multiply(std::integral_constant<int, 2>{});
     else multiply(std::integral_constant<int, 1>{});
     // acc[u][r]: channel ch0 + 4 quarter + r of pair 16 u + col
@@ -465,6 +485,289 @@ __global__ void __launch_bounds__(64 * W, 2) feature_grads_group_kernel(
   }
 }
 
+// ----------------------------------------------------------- both gradients at once ----
+
+// For 128 channels and 32 basis columns, where a centre's upstream gradient is 16 KB, one kernel
+// forms both gradients.
+constexpr int kBothTiles = 8, kBothC = 16 * kBothTiles, kBothK = 32;
+constexpr int kBothWaves = 8, kBothThreads = 64 * kBothWaves;
+constexpr int kBothChunk = 64;        // pairs of one centre that are worked on at a time
+constexpr int kBothRows = 192;        // rows of its table: what 160 KB leave beside a chunk's operands
+
+struct BothLds {
+  static constexpr int kLdF = kBothC / 4 + 1;     // 16-byte pieces of a feature row and one of padding
+  static constexpr int kLdG = kBothK + 4;         // floats of a channel's upstream gradient, padded
+  v4f acc[(kBothRows + 1) * kBothC / 4];          // as in GroupLds
+  v4f feat[kBothChunk * kLdF];                    // feature rows of the chunk's pairs
+  v4f basis[kBothChunk * kBothK / 4];             // their basis rows
+  float grad[kBothC * kLdG];                      // upstream gradient of the centre
+  int key[2][kBothRows];                          // points of the group and of the one after
+  unsigned short row[kBothChunk];
+  int point[kBothChunk];
+};
+static_assert(sizeof(BothLds) <= 160 * 1024, "one block per compute unit");
+
+// dbasis^T [k x pair] = G^T [k x c] F^T [c x pair] and dfeat^T [c x pair] = G [c x k] B^T [k x pair]
+// by one block per compute unit, which walks groups of centres chunk by chunk: the upstream
+// gradient, by far the largest operand, comes from memory once for both.  Per chunk the eight
+// wavefronts fetch its operands together in runs of consecutive lanes, one chunk ahead and across
+// the ends of the groups, and share them through LDS; a wavefront multiplies 16 channels of
+// dfeat and a 16 x 16 tile of dbasis.  What is summed in which order is as in the two kernels above.
+// 800 k x 52 pairs: 14.2 -> 12.6 ms against the two (2.31 -> 2.08 ms with the numbering of the rows for
+// 200 k x 20, 2.50 -> 2.37 for 100 k x 75, clustered clouds of 200 k x 37 3.24 -> 3.13, 100 k x 70 2.35
+// both).  Bound by the phases of a chunk one after the other: multiplying 6 ms of it (matrix
+// cores 5.3), parking the operands between two barriers 4, and what of the fetch they do
+// not cover.  Sixteen wavefronts: 13.0 ms; feature rows from memory straight into the operands and
+// two buffers for the rest 13.5; both with 16 basis columns or 64 channels: up to 18 % slower
+// than the two kernels, whose upstream gradient is half as large there.
+__global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
+    int64_t n_out, int last_pair, int group, int groups, const float *__restrict__ feat,
+    const float *__restrict__ basis, const int2 *__restrict__ nbrs,
+    const GroupCentre *__restrict__ listed, const unsigned short *__restrict__ row_of,
+    const int *__restrict__ keys, const float *__restrict__ in_grad, float *__restrict__ dbasis,
+    float *__restrict__ dfeat) {
+  constexpr int C = kBothC, K = kBothK;
+  constexpr int kRun = K / 4, kPieces = K / 4;
+  constexpr int kFetchG = C * kPieces / kBothThreads;
+  constexpr int kFetchF = kBothChunk * (C / 4) / kBothThreads;
+  constexpr int kNoPair = kBothRows;
+  static_assert(kBothChunk * kPieces == kBothThreads, "a piece of the basis rows per thread");
+  static_assert(kBothChunk / 16 * (K / 16) == kBothWaves && kBothTiles == kBothWaves &&
+                    kRun == kBothTiles, "a tile of either product per wavefront, steps side by side");
+  extern __shared__ __align__(16) char lds_raw[];
+  BothLds &s = *reinterpret_cast<BothLds *>(lds_raw);
+  const int t = threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int quarter = lane >> 4, col = lane & 15;
+  const int ch0 = 16 * wave;                                // its channels of dfeat
+  const int pair0 = 16 * (wave / 2), k0 = 16 * (wave % 2);  // its pairs and columns of dbasis
+
+  struct Chunk {
+    int centre, begin, left;          // left: pairs of the centre from begin on
+    int group;                        // its group, or -1 past the last chunk
+    int rows, direct, odd;            // of the group
+    bool first, last;                 // of the group
+  };
+  // The reader walks the chunks three ahead of the multiplication.  The centre after the one
+  // being read is fetched by every lane and looked at after the wait for a chunk's operands: a
+  // wait of its own would be one for all loads before it, and one for the scalar cache a wait
+  // of the LDS accesses.
+  const int per_xcd = gridDim.x / 8;              // groups side by side share points: one XCD, one L2
+  int at_group = (int)((blockIdx.x % 8) * per_xcd + blockIdx.x / 8);
+  int64_t at = (int64_t)at_group * group;         // the centre after the one being read
+  GroupCentre after = {0, 0, 0, 1};
+  auto fetch_centre = [&]() __attribute__((always_inline)) {
+    int64_t place = at < n_out ? at : n_out - 1;
+    asm volatile("" : "+v"(place));               // (a vector load, though the same for all lanes)
+    after = listed[place];
+  };
+  int centre = 0, begin = 0, left = 0, flags = 0, group_read = 0, odd = 0;
+  bool fresh = true;                              // the next centre starts a group
+  auto read = [&]() __attribute__((always_inline)) {
+    Chunk c{0, 0, 0, -1, 0, 0, 0, false, false};
+    while (left <= 0) {                           // the next centre (twice: groups without pairs)
+      if (at_group >= groups) return c;
+      centre = __builtin_amdgcn_readfirstlane(after.centre);
+      begin = __builtin_amdgcn_readfirstlane(after.begin);
+      left = __builtin_amdgcn_readfirstlane(after.count);
+      flags = __builtin_amdgcn_readfirstlane(after.flags);
+      group_read = at_group;
+      if (fresh) {
+        c.first = true;
+        odd ^= 1;
+      }
+      fresh = flags & 1;
+      at = fresh ? (int64_t)(at_group += (int)gridDim.x) * group : at + 1;
+      if (left <= 0) fetch_centre();
+    }
+    c.centre = centre;
+    c.begin = begin;
+    c.left = left;
+    c.group = group_read;
+    c.rows = flags >> 2;
+    c.direct = flags & 2;
+    c.odd = odd;
+    begin += kBothChunk;
+    left -= kBothChunk;
+    c.last = left <= 0 && (flags & 1);
+    return c;
+  };
+  auto pair_of = [&](const Chunk &c) {            // this lane's; some valid one past the last
+    const int m = c.begin + lane;
+    return m < last_pair ? m : last_pair;
+  };
+
+  v4f fb, fg[kFetchG], ff[kFetchF];
+  int frow = kNoPair, fkey = 0, fpoint = 0;
+  // (nothing that is fetched is looked at here: the wait for it would be one for every load before)
+  auto fetch = [&](const Chunk &c, int ids) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < kFetchF; ++x) {
+      const int idx = x * kBothThreads + t;
+      ff[x] = *reinterpret_cast<const v4f *>(
+          feat + (int64_t)__shfl(ids, idx / (C / 4), kWave) * C + 4 * (idx % (C / 4)));
+    }
+#pragma unroll
+    for (int x = 0; x < kFetchG; ++x)
+      fg[x] = __builtin_nontemporal_load(reinterpret_cast<const v4f *>(
+          in_grad + (int64_t)c.centre * C * K + 4 * (x * kBothThreads + t)));
+    const int m = c.begin + t / kPieces;
+    fb = __builtin_nontemporal_load(reinterpret_cast<const v4f *>(
+        basis + (int64_t)(m < last_pair ? m : last_pair) * K + 4 * (t % kPieces)));
+    if (wave == 0) {
+      frow = row_of[pair_of(c)];
+      fpoint = ids;
+    }
+    if (c.first && t < c.rows) fkey = keys[(int64_t)c.group * kMaxRows + t];
+  };
+  auto park = [&](const Chunk &c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < kFetchF; ++x) {
+      const int idx = x * kBothThreads + t;
+      s.feat[idx / (C / 4) * BothLds::kLdF + idx % (C / 4)] = ff[x];
+    }
+#pragma unroll
+    for (int x = 0; x < kFetchG; ++x) {
+      const int idx = x * kBothThreads + t;
+      *reinterpret_cast<v4f *>(s.grad + idx / kPieces * BothLds::kLdG + 4 * (idx % kPieces)) = fg[x];
+    }
+    const int slot = t / kPieces;
+    s.basis[slot * kPieces + ((t % kPieces) ^ (slot & (kPieces - 1)))] = fb;
+    if (wave == 0) {
+      s.row[lane] = (unsigned short)(lane < c.left ? frow : kNoPair);
+      s.point[lane] = fpoint;
+    }
+    if (c.first && t < c.rows) s.key[c.odd][t] = fkey;
+  };
+  // The wavefront's tiles of dfeat go into the table, its tile of dbasis is returned.  With both to
+  // multiply it does so in turn: the latter is a chain of dependent instructions.
+  auto multiply = [&](const Chunk &c, auto tiles, auto with_basis) __attribute__((always_inline)) {
+    constexpr int T = tiles;
+    v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    int at[T];
+    bool direct[T];
+    float gk[kRun], w[T][kRun];
+    v4f have[T], acc[T];
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int r = s.row[16 * u + col];
+      direct[u] = r == kNoRow;
+      at[u] = place<kBothTiles>(ch0 / 4 + quarter, direct[u] ? kNoPair : r);
+    }
+#pragma unroll
+    for (int x = 0; x < kRun / 4; ++x) {
+      const v4f q = *reinterpret_cast<const v4f *>(s.grad + (ch0 + col) * BothLds::kLdG +
+                                                   quarter * kRun + 4 * x);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) gk[4 * x + e] = q[e];
+    }
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int slot = 16 * u + col;
+#pragma unroll
+      for (int x = 0; x < kRun / 4; ++x) {
+        const v4f q = s.basis[slot * kPieces + ((quarter * (kRun / 4) + x) ^ (slot & (kPieces - 1)))];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[u][4 * x + e] = q[e];
+      }
+    }
+    // The pairs of a centre have distinct rows (or that of no pair): the rows are all read
+    // before the products and written back after them.
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      have[u] = s.acc[at[u]];
+      acc[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int q = 0; q < kRun; ++q) {
+#pragma unroll
+      for (int u = 0; u < T; ++u)
+        acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(gk[q], w[u][q], acc[u], 0, 0, 0);
+      if constexpr (with_basis) {                 // channels 16 q .. 16 q + 15
+        const v4f f = s.feat[(pair0 + col) * BothLds::kLdF + 4 * q + quarter];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          sum = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              s.grad[(16 * q + 4 * quarter + e) * BothLds::kLdG + k0 + col], f[e], sum, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < T; ++u) s.acc[at[u]] = have[u] + acc[u];
+    if (c.direct) {                               // pairs without a row
+#pragma unroll
+      for (int u = 0; u < T; ++u) {
+        if (!direct[u]) continue;
+        float *dst = dfeat + (int64_t)s.point[16 * u + col] * C + ch0 + 4 * quarter;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) unsafeAtomicAdd(dst + r, acc[u][r]);
+      }
+    }
+    return sum;
+  };
+  auto products = [&](const Chunk &c) __attribute__((always_inline)) {
+    auto by_basis = [&](auto tiles) __attribute__((always_inline)) {
+      return pair0 < c.left ? multiply(c, tiles, std::true_type{})
+                            : multiply(c, tiles, std::false_type{});
+    };
+    if (c.left > 48) return by_basis(std::integral_constant<int, 4>{});
+    if (c.left > 32) return by_basis(std::integral_constant<int, 3>{});
+    if (c.left > 16) return by_basis(std::integral_constant<int, 2>{});
+    return by_basis(std::integral_constant<int, 1>{});
+  };
+  // sum[r]: basis column k0 + 4 quarter + r of pair pair0 + col
+  auto store = [&](const Chunk &c, const v4f &sum) __attribute__((always_inline)) {
+    if (pair0 + col < c.left)
+      __builtin_nontemporal_store(sum, reinterpret_cast<v4f *>(
+          dbasis + (int64_t)(c.begin + pair0 + col) * K + k0 + 4 * quarter));
+  };
+  // the rows leave, consecutive floats each, and the table is empty again
+  auto send = [&](const Chunk &c) __attribute__((always_inline)) {
+    const int *key = s.key[c.odd];
+    for (int i = t; i < c.rows * C; i += kBothThreads) {
+      const int row = i / C, ch = i - row * C;
+      float &sum = reinterpret_cast<float *>(s.acc + place<kBothTiles>(ch >> 2, row))[ch & 3];
+      unsafeAtomicAdd(dfeat + (int64_t)key[row] * C + ch, sum);
+      sum = 0.0f;
+    }
+  };
+
+  for (int i = t; i < kBothRows * C / 4; i += kBothThreads) s.acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  fetch_centre();
+  Chunk c = read();
+  if (c.group < 0) return;
+  fetch_centre();
+  Chunk next = read();
+  fetch_centre();
+  Chunk ahead = read();
+  fetch_centre();
+  fetch(c, nbrs[pair_of(c)].x);
+  int ids = nbrs[pair_of(next)].x;
+  park(c);
+  asm volatile("" : "+v"(ids));                   // (waited for here)
+  while (true) {                                  // ends: every step takes a chunk off the list
+    block_lds_sync();                             // the chunk is in LDS, the rows before have left
+    if (next.group >= 0) {
+      fetch(next, ids);
+      ids = nbrs[pair_of(ahead)].x;
+    }
+    const v4f sum = products(c);
+    block_lds_sync();                             // the chunk has been read
+    // What has been fetched is waited for before anything is written: a wait behind the stores
+    // and atomics would be one for them as well.
+    if (next.group >= 0) park(next);
+    asm volatile("" : "+v"(ids), "+v"(after.centre), "+v"(after.begin), "+v"(after.count),
+                 "+v"(after.flags));
+    const Chunk third = read();
+    fetch_centre();
+    store(c, sum);
+    if (c.last) send(c);
+    if (next.group < 0) break;
+    c = next;
+    next = ahead;
+    ahead = third;
+  }
+}
+
 // Blocks of 16 channels, or 0 if the shape has no grouped kernel.
 static int group_slices(int C, int K) {
   if (K != 8 && K != 16 && K != 32 && K != 64) return 0;
@@ -493,6 +796,26 @@ static int launch_group(hipStream_t s, int64_t n, int64_t pairs, int C, int grou
   auto dbasis_kernel = full ? basis_grads_kernel<CT, K, true> : basis_grads_kernel<CT, K, false>;
   hipLaunchKernelGGL(dbasis_kernel, dim3(wave_grid(n)), dim3(256), 0, s, n, C, feat, nbrs, ranges,
                      order, in_grad, dbasis);
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
+static int launch_both(hipStream_t s, int64_t n, int64_t pairs, int group, const float *basis,
+                       const float *feat, const int2 *nbrs, const GroupCentre *listed,
+                       const unsigned short *row_of, const int *keys, const float *in_grad,
+                       float *dbasis, float *dfeat) {
+  int device = 0, cus = 0;
+  MCCNN_HIP_CHECK(hipGetDevice(&device));
+  MCCNN_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  // a block per compute unit, in eights (blocks are numbered per XCD)
+  const int64_t groups = blocks_for(n, group), wanted = (groups + 7) / 8 * 8;
+  const int64_t most = cus < 8 ? 8 : cus / 8 * 8;
+  MCCNN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(both_grads_group_kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)sizeof(BothLds)));
+  hipLaunchKernelGGL(both_grads_group_kernel, dim3((unsigned)(wanted < most ? wanted : most)),
+                     dim3(kBothThreads), sizeof(BothLds), s, n, (int)(pairs - 1), group, (int)groups,
+                     feat, basis, nbrs, listed, row_of, keys, in_grad, dbasis, dfeat);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }
@@ -563,19 +886,23 @@ extern "C" int mccnn_basis_proj_grads_grouped_pays(int num_features, int num_bas
 // Centres per group: about 400 pairs, which list some 140 points where lists overlap as they do in
 // space.  Fewer pairs per point than in larger groups, but hardly a group that overflows the
 // table's 192 or 224 rows: 800 k x 52 pairs, 128 x 32 take 10.9 / 9.9 / 10.0 / 11.2 ms at 560 /
-// 440 / 340 / 240 pairs.
-static int group_centres(int64_t num_samples, int64_t num_neighbors) {
+// 440 / 340 / 240 pairs; both gradients at once (192 rows) 13.8 / 13.3 / 13.2 ms at 460 / 400 / 350,
+// clustered clouds of 200 k x 37 3.29 / 3.30 / 3.13.
+constexpr double kGroupPairs = 400.0, kBothPairs = 350.0;
+static int group_centres(int64_t num_samples, int64_t num_neighbors, double pairs) {
   const double mean = (double)num_neighbors / (double)(num_samples > 0 ? num_samples : 1);
-  const int group = (int)(400.0 / (mean > 1.0 ? mean : 1.0));
+  const int group = (int)(pairs / (mean > 1.0 ? mean : 1.0));
   return group < 4 ? 4 : (group > kMaxGroup ? kMaxGroup : group);
 }
 
 extern "C" size_t mccnn_basis_proj_grads_grouped_workspace_bytes(int64_t num_samples,
                                                                  int64_t num_neighbors) {
   if (num_samples <= 0 || num_neighbors <= 0) return 0;
-  const int64_t groups = blocks_for(num_samples, group_centres(num_samples, num_neighbors));
+  const int64_t groups = blocks_for(num_samples, group_centres(num_samples, num_neighbors, kBothPairs));
   return align256(sizeof(unsigned short) * (size_t)num_neighbors) +
-         align256(sizeof(int) * kMaxRows * (size_t)groups) + align256(sizeof(GroupInfo) * (size_t)groups);
+         align256(sizeof(int) * kMaxRows * (size_t)groups) +
+         align256(sizeof(GroupInfo) * (size_t)groups) +
+         align256(sizeof(GroupCentre) * (size_t)num_samples);
 }
 
 extern "C" int mccnn_basis_proj_grads_grouped(
@@ -604,16 +931,24 @@ extern "C" int mccnn_basis_proj_grads_grouped(
   MCCNN_REQUIRE(workspace && workspace_bytes >= mccnn_basis_proj_grads_grouped_workspace_bytes(
                                                      num_samples, num_neighbors),
                 "BasisProjGrads (grouped) workspace too small");
-  const int group = group_centres(num_samples, num_neighbors);
+  const bool both = num_features == kBothC && num_basis == kBothK;
+  const int group = group_centres(num_samples, num_neighbors, both ? kBothPairs : kGroupPairs);
   const int64_t groups = blocks_for(num_samples, group);
   unsigned short *row_of = (unsigned short *)workspace;
   int *keys = (int *)((char *)workspace + align256(sizeof(unsigned short) * (size_t)num_neighbors));
   GroupInfo *infos = (GroupInfo *)((char *)keys + align256(sizeof(int) * kMaxRows * (size_t)groups));
+  GroupCentre *listed =
+      both ? (GroupCentre *)((char *)infos + align256(sizeof(GroupInfo) * (size_t)groups)) : nullptr;
   hipLaunchKernelGGL(group_rows_kernel, dim3((unsigned)groups), dim3(256), 0, s, num_samples, group,
-                     num_basis == 64 ? kRows<64> : kMaxRows, (const int2 *)neighbors, ranges,
-                     centre_order, row_of, keys, infos, num_neighbors, num_basis, basis_grads_out);
+                     both ? kBothRows : num_basis == 64 ? kRows<64> : kMaxRows,
+                     (const int2 *)neighbors, ranges, centre_order, row_of, keys, infos,
+                     listed, num_neighbors, num_basis, basis_grads_out);
   MCCNN_LAUNCH_CHECK();
   int rc = MCCNN_OK;
+  if (both)
+    return launch_both(s, num_samples, num_neighbors, group, basis, features,
+                       (const int2 *)neighbors, listed, row_of, keys, in_grads, basis_grads_out,
+                       feature_grads_out);
 #define MCCNN_GROUP_K(CT_, K_)                                                                   \
   rc = launch_group<CT_, K_>(s, num_samples, num_neighbors, num_features, group, basis, features, \
                              (const int2 *)neighbors, ranges, centre_order, row_of, keys, infos, \

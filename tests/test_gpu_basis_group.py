@@ -14,7 +14,7 @@ LENGTHS = [0, 1, 16, 17, 64, 65, 31, 33, 700, 5]
 @pytest.mark.parametrize("c,k,points,centres", [
     (3, 8, 40, 1), (7, 64, 900, 37), (16, 16, 64, 10), (24, 32, 4000, 83), (64, 8, 300, 21),
     (64, 64, 5000, 64), (96, 16, 500, 129), (104, 32, 2000, 50), (128, 64, 1000, 33),
-    (128, 32, 3000, 260)])
+    (128, 32, 3000, 260), (128, 32, 40, 1), (128, 16, 40, 1), (64, 32, 700, 130)])
 def test_grouped_gradients(c, k, points, centres):
     from tensorflow_graphics_point_clouds_amd import _lib
     host = _lib.host()
@@ -77,3 +77,38 @@ def test_rows_behind_the_last_list_have_zero_gradients(c, k, spare):
     terms = up[pairs[:used, 1].long()].double() * feat[pairs[:used, 0].long()].double()[:, :, None]
     expect, size = terms.sum(1), terms.abs().sum(1)
     assert torch.all((dbasis[:used] - expect).abs() <= (c + 1) * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("c,k,longest,window", [(64, 32, 40, 60), (128, 32, 66, 80), (128, 32, 130, 2000)])
+def test_gradients_of_more_groups_than_blocks(c, k, longest, window):
+    """The block that forms both gradients of 128 x 32 walks several groups: more of them than the
+    device takes blocks, with runs of centres without pairs, lists that share their points and
+    groups whose points overflow the table."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    host = _lib.host()
+    gen = torch.Generator(device="cuda").manual_seed(c + k)
+    rand = lambda high, n: torch.randint(high, (n,), device="cuda", generator=gen)
+    centres = 10 * 400 * 256 // longest
+    points = centres
+    lengths = rand(longest + 1, centres)
+    lengths[5000:5400] = 0
+    lengths[-1] = 0
+    ranges = torch.cumsum(lengths, 0).int()
+    owner = torch.repeat_interleave(torch.arange(centres, device="cuda"), lengths)
+    ids = (owner + rand(window, len(owner))) % points        # (a point twice in a list among them)
+    pairs = torch.stack([ids, owner], 1).int().contiguous()
+    basis, feat, up = (torch.randn(*s, device="cuda", generator=gen)
+                       for s in ((len(ids), k), (points, c), (centres, c, k)))
+    dbasis, dfeat = host.basis_proj_grads_grouped(basis, feat, pairs, ranges, up,
+                                                  host.neighbourhood_order(pairs, ranges))
+    df, df_mag = (torch.zeros(points, c, device="cuda", dtype=torch.float64) for _ in range(2))
+    for part in torch.arange(len(ids), device="cuda").split(16384):
+        g, b, i = up[owner[part]].double(), basis[part].double(), ids[part]
+        terms = g * feat[i].double()[:, :, None]
+        assert torch.all((dbasis[part] - terms.sum(1)).abs() <=
+                         (c + 1) * 2.0 ** -24 * terms.abs().sum(1))
+        terms = g * b[:, None, :]
+        df.index_add_(0, i, terms.sum(2))
+        df_mag.index_add_(0, i, terms.abs().sum(2))
+    terms = k * torch.bincount(ids, minlength=points)[:, None]
+    assert torch.all((dfeat - df).abs() <= (terms + 1) * 2.0 ** -24 * df_mag)
