@@ -35,6 +35,57 @@ __global__ void __launch_bounds__(256) store_cell_starts_kernel(int64_t n,
     if (i == 0 || keys[i] != keys[i - 1]) first_idx[cell_scan[i] - 1] = (int)i;
 }
 
+// The three steps -- flags, their prefix sum and the list of cells -- of up to 16 384 points in one
+// launch of one block, with the number of cells in *total: launches cost more than the work there (4
+// or 16 rounds of 1024 keys, all in flight; three levels of 16 x 1024 points 28 us and the gaps of nine
+// launches, 17 and those of three).  Beyond, one compute unit is too few.
+constexpr int kStartThreads = 1024, kStartWaves = kStartThreads / kWave;
+constexpr int64_t kStartMax = 16 * kStartThreads;
+
+template <int kStartRounds>
+__global__ void __launch_bounds__(kStartThreads) cell_starts_block_kernel(
+    int n, const int64_t *__restrict__ keys, int *__restrict__ first_idx, int64_t *total) {
+  constexpr int kParts = kStartRounds * kStartWaves;
+  __shared__ int before[kParts];                 // cells that start in (round, wavefront), then before it
+  const int t = threadIdx.x, lane = lane_id(), wave = t / kWave;
+  int64_t key[kStartRounds], prev[kStartRounds];
+#pragma unroll
+  for (int r = 0; r < kStartRounds; ++r) {       // (past the end: the last point again)
+    const int i = r * kStartThreads + t < n ? r * kStartThreads + t : n - 1;
+    key[r] = keys[i];
+    prev[r] = keys[i > 0 ? i - 1 : 0];
+  }
+  uint64_t starts[kStartRounds];
+#pragma unroll
+  for (int r = 0; r < kStartRounds; ++r) {
+    const int i = r * kStartThreads + t;
+    starts[r] = __ballot(i < n && (i == 0 || key[r] != prev[r]));
+    if (lane == 0) before[r * kStartWaves + wave] = __popcll(starts[r]);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    constexpr int kEach = kParts / kWave;
+    int count[kEach], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) sum += count[k] = before[kEach * lane + k];
+    const int incl = wave_inclusive_scan(sum);
+    int run = incl - sum;
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+      before[kEach * lane + k] = run;
+      run += count[k];
+    }
+    if (lane == kWave - 1)
+      __hip_atomic_store(total, (int64_t)incl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kStartRounds; ++r)
+    if ((starts[r] >> lane) & 1)
+      first_idx[before[r * kStartWaves + wave] + __popcll(starts[r] & ((1ull << lane) - 1ull))] =
+          r * kStartThreads + t;
+}
+
 // Parity class of every occupied cell (bit d = parity of the cell index in dim d), and how many
 // cells every class has.
 constexpr int kMaxClasses = 1 << kMaxDims;
@@ -541,17 +592,26 @@ static int sampling_count(mccnn_stream_t stream, int mode, int64_t num_pts, int 
                 workspace_bytes, w.bytes);
   hipStream_t s = as_stream(stream);
   const unsigned grid = blocks_for(num_pts, 256);
-  hipLaunchKernelGGL(flag_cell_starts_kernel, dim3(grid), dim3(256), 0, s, num_pts,
-                     (const int64_t *)point_keys, w.cell_scan);
-  MCCNN_LAUNCH_CHECK();
-  // pinned: the last scan's total goes straight to the host
+  // pinned: the last count goes straight to the host
   if (pinned) *num_sampled_out_host = -1;
-  int rc = inclusive_scan_i32(s, num_pts, w.cell_scan, w.scan_scratch,
-                              pinned && mode == 1 ? num_sampled_out_host : w.num_cells_total);
-  if (rc != MCCNN_OK) return rc;
-  hipLaunchKernelGGL(store_cell_starts_kernel, dim3(grid), dim3(256), 0, s, num_pts,
-                     (const int64_t *)point_keys, w.cell_scan, w.first_idx);
-  MCCNN_LAUNCH_CHECK();
+  int64_t *cells = pinned && mode == 1 ? num_sampled_out_host : w.num_cells_total;
+  int rc = MCCNN_OK;
+  if (num_pts <= kStartMax) {
+    auto kernel = num_pts <= 4 * kStartThreads ? cell_starts_block_kernel<4>
+                                               : cell_starts_block_kernel<16>;
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kStartThreads), 0, s, (int)num_pts,
+                       (const int64_t *)point_keys, w.first_idx, cells);
+    MCCNN_LAUNCH_CHECK();
+  } else {
+    hipLaunchKernelGGL(flag_cell_starts_kernel, dim3(grid), dim3(256), 0, s, num_pts,
+                       (const int64_t *)point_keys, w.cell_scan);
+    MCCNN_LAUNCH_CHECK();
+    rc = inclusive_scan_i32(s, num_pts, w.cell_scan, w.scan_scratch, cells);
+    if (rc != MCCNN_OK) return rc;
+    hipLaunchKernelGGL(store_cell_starts_kernel, dim3(grid), dim3(256), 0, s, num_pts,
+                       (const int64_t *)point_keys, w.cell_scan, w.first_idx);
+    MCCNN_LAUNCH_CHECK();
+  }
   const int64_t *result = w.num_cells_total;
   if (mode == 0) {
     rc = fill_zero(s, w.used, (char *)(w.cursors + kMaxClasses) - (char *)w.used);

@@ -91,3 +91,26 @@ def test_which_samples_are_selected_from_the_grid(d, from_grid, monkeypatch):
     assert len(searched) == (0 if d <= 3 else 1 if d == 4 else 4)
     pc.PointHierarchy(cloud, [0.3], "cell average")
     assert len(searched) == (0 if d <= 3 else 1 if d == 4 else 4)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, 4096, 4097, 16383, 16384, 16385])
+@pytest.mark.parametrize("cell", [0.04, 0.4, 3.0])
+def test_cells_of_points_on_either_side_of_one_block(n, cell):
+    """One point per occupied cell: cells of one point, of tens and of all, as many as a block lists in
+    one launch and one more."""
+    from tensorflow_graphics_point_clouds_amd import pc
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    pts = torch.rand((n, 3), device="cuda", generator=gen)
+    bids = (torch.arange(n, device="cuda") * 3 // n).int()
+    grid = pc.Grid(pc.PointCloud(pts, bids, 3), cell)
+    got = pc.cell_average_sampling(None, grid=grid)
+    _, owner, counts = torch.unique_consecutive(grid._sorted_keys, return_inverse=True,
+                                                return_counts=True)
+    sums = torch.zeros(len(counts), 3, device="cuda", dtype=torch.float64)
+    sums.index_add_(0, owner, grid._sorted_points.double())
+    want = sums / counts[:, None]
+    # n - 1 float32 additions of values up to 1 and a division
+    assert got._points.shape == want.shape
+    assert bool(((got._points.double() - want).abs() <= (counts[:, None] + 1) * 2.0 ** -24).all())
+    firsts = torch.cumsum(counts, 0) - counts
+    assert torch.equal(got._batch_ids, grid._sorted_batch_ids[firsts])
