@@ -179,6 +179,11 @@ int mccnn_swapped_pairs(mccnn_stream_t stream, int64_t num_neighbors,
 int mccnn_gather_pdf_column(mccnn_stream_t stream, int64_t num_neighbors,
                             const int32_t *neighbors, int column, const float *pdf,
                             float *pdf_per_pair_out);
+/* column 0 of a table and column 1 of its transpose, of as many pairs, at once */
+int mccnn_gather_pdf_both(mccnn_stream_t stream, int64_t num_neighbors,
+                          const int32_t *neighbors, const int32_t *transposed,
+                          const float *pdf, float *pdf_per_pair_out,
+                          float *pdf_per_transposed_out);
 int mccnn_gather_i32(mccnn_stream_t stream, int64_t count, const int32_t *src,
                      const int32_t *indices, int32_t *out);
 int mccnn_gather_rows(mccnn_stream_t stream, int64_t num_rows, int num_cols, const float *src,

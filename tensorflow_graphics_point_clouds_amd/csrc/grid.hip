@@ -86,6 +86,20 @@ __global__ void __launch_bounds__(256) gather_pdf_kernel(int64_t m, const int2 *
   }
 }
 
+// Both tables of a neighbourhood at once, column 0 of one and column 1 of the other: small clouds pay for
+// launches (three levels of 16 x 1024 points 15.2 us and the gaps of six, 8.7 and those of three;
+// 61 k points x 28 pairs 13.0 -> 9.1, 763 k x 37 168 -> 139).
+__global__ void __launch_bounds__(256) gather_pdf_both_kernel(
+    int64_t m, const int2 *__restrict__ nbrs, const int2 *__restrict__ transposed,
+    const float *__restrict__ pdf, float *__restrict__ out, float *__restrict__ out_transposed) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < m;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int p = nbrs[i].x, q = transposed[i].y;
+    out[i] = pdf[p];
+    out_transposed[i] = pdf[q];
+  }
+}
+
 __global__ void __launch_bounds__(256) gather_i32_kernel(int64_t n, const int *__restrict__ src,
                                                          const int *__restrict__ idx,
                                                          int *__restrict__ out) {
@@ -785,6 +799,21 @@ extern "C" int mccnn_gather_pdf_column(mccnn_stream_t stream, int64_t num_neighb
   hipLaunchKernelGGL(gather_pdf_kernel, dim3(capped_grid(num_neighbors)), dim3(256), 0,
                      as_stream(stream), num_neighbors, (const int2 *)neighbors, column, pdf,
                      pdf_per_pair_out);
+  MCCNN_LAUNCH_CHECK();
+  return MCCNN_OK;
+}
+
+extern "C" int mccnn_gather_pdf_both(mccnn_stream_t stream, int64_t num_neighbors,
+                                     const int32_t *neighbors, const int32_t *transposed,
+                                     const float *pdf, float *pdf_per_pair_out,
+                                     float *pdf_per_transposed_out) {
+  MCCNN_REQUIRE(num_neighbors >= 0, "gather_pdf expects a non-negative size");
+  if (num_neighbors == 0) return MCCNN_OK;
+  MCCNN_REQUIRE(neighbors && transposed && pdf && pdf_per_pair_out && pdf_per_transposed_out,
+                "gather_pdf received a null tensor");
+  hipLaunchKernelGGL(gather_pdf_both_kernel, dim3(capped_grid(num_neighbors)), dim3(256), 0,
+                     as_stream(stream), num_neighbors, (const int2 *)neighbors,
+                     (const int2 *)transposed, pdf, pdf_per_pair_out, pdf_per_transposed_out);
   MCCNN_LAUNCH_CHECK();
   return MCCNN_OK;
 }

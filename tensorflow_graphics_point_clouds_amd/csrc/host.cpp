@@ -479,6 +479,18 @@ Tensor swapped_pairs(const Tensor &neighbors, const Tensor &order) {
   return out;
 }
 
+// Column 0 of a pair table and column 1 of its transpose -> (densities, densities).
+std::pair<Tensor, Tensor> gather_pdf_both(const Tensor &neighbors, const Tensor &transposed,
+                                          const Tensor &pdf) {
+  const int64_t m = neighbors.size(0);
+  if (transposed.size(0) != m) throw InvalidArgument("gather_pdf expects tables of equal length");
+  Tensor out = empty_f32({m}, pdf), out_t = empty_f32({m}, pdf);
+  hipStream_t s = current_stream();
+  Region r("gather_pdf", s);
+  check(mccnn_gather_pdf_both(s, m, i32(neighbors), i32(transposed), f32(pdf), f32(out), f32(out_t)));
+  return {out, out_t};
+}
+
 Tensor gather_pdf(const Tensor &neighbors, int64_t column, const Tensor &pdf) {
   Tensor out = empty_f32({neighbors.size(0)}, neighbors);
   hipStream_t s = current_stream();
@@ -1616,6 +1628,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("transpose_neighbors", &transpose_neighbors, release());
   m.def("swapped_pairs", &swapped_pairs, release());
   m.def("gather_pdf", &gather_pdf, release());
+  m.def("gather_pdf_both", &gather_pdf_both, release());
   m.def("gather_i32", &gather_i32, release());
   m.def("compute_pdf", &compute_pdf, release());
   m.def("sampling", &sampling, release());

@@ -445,6 +445,9 @@ class _SortedView:
         key = nbh._pdf_generation
         if key != self._pdf_key:
             self._pdf_key, self.pdf, self.pdf_t = key, None, None
+        if transposed and self.pdf is None and per_point is not None and not nbh._pdf_normalize:
+            self.pdf, self.pdf_t = _lib.host().gather_pdf_both(self.table, self.table_t,
+                                                               per_point.detach())
         if self.pdf is None:
             self.pdf = self._pair_values(nbh, per_point, self.table, 0)
         if transposed and self.pdf_t is None:

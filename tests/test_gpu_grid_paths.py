@@ -246,3 +246,15 @@ def test_densities_differentiable_in_the_sorted_points():
     assert grads[0].norm() > 0
     # the same sums of some tens of float32 terms, in another order at most
     assert (grads[0] - grads[1]).norm() <= 1e-5 * grads[1].norm()
+
+
+@pytest.mark.parametrize("m", [0, 1, 255, 257, 70001])
+def test_pair_densities_of_both_tables_at_once(m):
+    from tensorflow_graphics_point_clouds_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    pdf = torch.rand(999, device="cuda", generator=gen)
+    table, transposed = (torch.randint(999, (m, 2), device="cuda", generator=gen).int()
+                         for _ in range(2))
+    got, got_t = _lib.host().gather_pdf_both(table, transposed, pdf)
+    assert torch.equal(got, pdf[table[:, 0].long()])
+    assert torch.equal(got_t, pdf[transposed[:, 1].long()])
