@@ -287,20 +287,28 @@ __global__ void __launch_bounds__(kAabbThreads) aabb_reduce_kernel(
   };
   Bounds<D> box;
   int cur = -1;                     // cloud of the running minima / maxima (wave-uniform)
-  for (int64_t base = first; base < last; base += kWave) {
-    const int64_t i = base + lane_id();
-    const bool live = i < last;
-    const int b = live ? bids[i] : -1;
-    float p[D];
+  // Four times 64 points in flight: one after the other they are a chain of waits (eight: the same).
+  constexpr int kAhead = 4;
+  for (int64_t base = first; base < last; base += kAhead * kWave) {
+    int b[kAhead];
+    float p[kAhead][D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) p[d] = live ? pts[i * D + d] : 0.f;
-    add_points<D>(live, b, p, batch >= kWave ? 3 : kWave, box, cur, flush, [&](int b, const float *p) {
+    for (int u = 0; u < kAhead; ++u) {            // past the end: the last point again
+      const int64_t at = base + u * kWave + lane_id(), i = at < last ? at : last - 1;
+      b[u] = bids[i];
 #pragma unroll
-      for (int d = 0; d < D; ++d) {
-        atomicMin(&mn[(int64_t)b * D + d], enc_float(p[d]));
-        atomicMax(&mx[(int64_t)b * D + d], enc_float(p[d]));
-      }
-    });
+      for (int d = 0; d < D; ++d) p[u][d] = pts[i * D + d];
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      add_points<D>(base + u * kWave + lane_id() < last, b[u], p[u], batch >= kWave ? 3 : kWave, box,
+                    cur, flush, [&](int b, const float *p) {
+#pragma unroll
+                      for (int d = 0; d < D; ++d) {
+                        atomicMin(&mn[(int64_t)b * D + d], enc_float(p[d]));
+                        atomicMax(&mx[(int64_t)b * D + d], enc_float(p[d]));
+                      }
+                    });
   }
   if (cur >= 0) flush(cur, box);
   __syncthreads();
@@ -644,7 +652,11 @@ static int reduce_boxes(hipStream_t s, int64_t n, int num_dims, const float *poi
   MCCNN_LAUNCH_CHECK();
   if (n == 0) return MCCNN_OK;
   // stretches of at least 1024 points, at most 1024 blocks
-  int64_t per_block = (n + 1023) / 1024;
+  // Stretches of at least 1024 points, at most 256 blocks: every block ends in a few minima and
+  // maxima of the same words of memory, one after the other, which were most of the time of 745
+  // blocks (763 k points in 8 clouds 11.9 -> 8.2 us, 800 k in 4 13.7 -> 8.4, 98 k in one 4.6 -> 3.7,
+  // 3 M 17.3 -> 14.2; 128 blocks: 10.6, 10.2, 4.0 and 22.6).
+  int64_t per_block = (n + 255) / 256;
   per_block = (per_block < 1024 ? 1024 : per_block + 255) / 256 * 256;
   MCCNN_DIM_SWITCH(num_dims,
                    hipLaunchKernelGGL(aabb_reduce_kernel<D>, dim3(blocks_for(n, (int)per_block)),
