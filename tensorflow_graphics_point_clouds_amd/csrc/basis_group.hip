@@ -592,9 +592,11 @@ __global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
     c.last = left <= 0 && (flags & 1);
     return c;
   };
-  auto pair_of = [&](const Chunk &c) {            // this lane's; some valid one past the last
-    const int m = c.begin + lane;
-    return m < last_pair ? m : last_pair;
+  // The point of this lane's pair; past the last one that of the last, since rows behind the lists of
+  // a table with spare capacity may hold anything (past the last chunk: of the first row).
+  auto point_of = [&](const Chunk &c) {
+    const int last = c.left > 0 ? c.left - 1 : 0;
+    return nbrs[c.begin + (lane < last ? lane : last)].x;
   };
 
   v4f fb, fg[kFetchG], ff[kFetchF];
@@ -615,7 +617,8 @@ __global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
     fb = __builtin_nontemporal_load(reinterpret_cast<const v4f *>(
         basis + (int64_t)(m < last_pair ? m : last_pair) * K + 4 * (t % kPieces)));
     if (wave == 0) {
-      frow = row_of[pair_of(c)];
+      const int own = c.begin + lane;
+      frow = row_of[own < last_pair ? own : last_pair];
       fpoint = ids;
     }
     if (c.first && t < c.rows) fkey = keys[(int64_t)c.group * kMaxRows + t];
@@ -740,15 +743,15 @@ __global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
   fetch_centre();
   Chunk ahead = read();
   fetch_centre();
-  fetch(c, nbrs[pair_of(c)].x);
-  int ids = nbrs[pair_of(next)].x;
+  fetch(c, point_of(c));
+  int ids = point_of(next);
   park(c);
   asm volatile("" : "+v"(ids));                   // (waited for here)
   while (true) {                                  // ends: every step takes a chunk off the list
     block_lds_sync();                             // the chunk is in LDS, the rows before have left
     if (next.group >= 0) {
       fetch(next, ids);
-      ids = nbrs[pair_of(ahead)].x;
+      ids = point_of(ahead);
     }
     const v4f sum = products(c);
     block_lds_sync();                             // the chunk has been read

@@ -50,7 +50,7 @@ def test_grouped_gradients(c, k, points, centres):
     assert np.all(np.abs(dfeat - df) <= (terms + 1) * 2.0 ** -24 * df_mag)
 
 
-@pytest.mark.parametrize("c,k,spare", [(24, 8, 1), (96, 16, 700), (64, 64, 65)])
+@pytest.mark.parametrize("c,k,spare", [(24, 8, 1), (96, 16, 700), (64, 64, 65), (128, 32, 70)])
 def test_rows_behind_the_last_list_have_zero_gradients(c, k, spare):
     """A table of more rows than its lists hold (a search into a given capacity): the kernels per
     pair and channel leave zeros there, the grouped ones write them."""
