@@ -27,6 +27,7 @@
 
 #include "common.h"
 #include "fill.h"
+#include "group_walk.h"
 #include "mfma.h"
 #include "sort.h"
 
@@ -175,13 +176,6 @@ constexpr int kProbes = 32;          // places tried for a point before it goes 
 struct GroupInfo {
   int rows;                          // points of the group that have a row
   int direct;                        // a pair of the group has none
-};
-
-// The centres of a group that have pairs, from its first place in the order on (in a group without
-// pairs one centre of none).
-struct __align__(16) GroupCentre {
-  int centre, begin, count;          // its pairs
-  int flags;                         // 1: the group's last, 2: GroupInfo::direct, 4 x GroupInfo::rows
 };
 
 // The rows of a group: its points are numbered through a hash table, keys[kMaxRows g ..] are the
@@ -542,56 +536,13 @@ __global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
   const int ch0 = 16 * wave;                                // its channels of dfeat
   const int pair0 = 16 * (wave / 2), k0 = 16 * (wave % 2);  // its pairs and columns of dbasis
 
-  struct Chunk {
-    int centre, begin, left;          // left: pairs of the centre from begin on
-    int group;                        // its group, or -1 past the last chunk
-    int rows, direct, odd;            // of the group
-    bool first, last;                 // of the group
-  };
-  // The reader walks the chunks three ahead of the multiplication.  The centre after the one
-  // being read is fetched by every lane and looked at after the wait for a chunk's operands: a
-  // wait of its own would be one for all loads before it, and one for the scalar cache a wait
-  // of the LDS accesses.
+  // The reader walks the chunks three ahead of the multiplication.  What it fetches is looked at
+  // after the wait for a chunk's operands: a wait of its own would be one for all loads before it,
+  // and one for the scalar cache a wait of the LDS accesses.
+  using Chunk = GroupChunk;
   const int per_xcd = gridDim.x / 8;              // groups side by side share points: one XCD, one L2
-  int at_group = (int)((blockIdx.x % 8) * per_xcd + blockIdx.x / 8);
-  int64_t at = (int64_t)at_group * group;         // the centre after the one being read
-  GroupCentre after = {0, 0, 0, 1};
-  auto fetch_centre = [&]() __attribute__((always_inline)) {
-    int64_t place = at < n_out ? at : n_out - 1;
-    asm volatile("" : "+v"(place));               // (a vector load, though the same for all lanes)
-    after = listed[place];
-  };
-  int centre = 0, begin = 0, left = 0, flags = 0, group_read = 0, odd = 0;
-  bool fresh = true;                              // the next centre starts a group
-  auto read = [&]() __attribute__((always_inline)) {
-    Chunk c{0, 0, 0, -1, 0, 0, 0, false, false};
-    while (left <= 0) {                           // the next centre (twice: groups without pairs)
-      if (at_group >= groups) return c;
-      centre = __builtin_amdgcn_readfirstlane(after.centre);
-      begin = __builtin_amdgcn_readfirstlane(after.begin);
-      left = __builtin_amdgcn_readfirstlane(after.count);
-      flags = __builtin_amdgcn_readfirstlane(after.flags);
-      group_read = at_group;
-      if (fresh) {
-        c.first = true;
-        odd ^= 1;
-      }
-      fresh = flags & 1;
-      at = fresh ? (int64_t)(at_group += (int)gridDim.x) * group : at + 1;
-      if (left <= 0) fetch_centre();
-    }
-    c.centre = centre;
-    c.begin = begin;
-    c.left = left;
-    c.group = group_read;
-    c.rows = flags >> 2;
-    c.direct = flags & 2;
-    c.odd = odd;
-    begin += kBothChunk;
-    left -= kBothChunk;
-    c.last = left <= 0 && (flags & 1);
-    return c;
-  };
+  GroupWalk<kBothChunk> walk(listed, n_out, group, groups, (int)gridDim.x,
+                             (int)((blockIdx.x % 8) * per_xcd + blockIdx.x / 8));
   // The point of this lane's pair; past the last one that of the last, since rows behind the lists of
   // a table with spare capacity may hold anything (past the last chunk: of the first row).
   auto point_of = [&](const Chunk &c) {
@@ -735,14 +686,14 @@ __global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
   };
 
   for (int i = t; i < kBothRows * C / 4; i += kBothThreads) s.acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-  fetch_centre();
-  Chunk c = read();
+  walk.fetch();
+  Chunk c = walk.read();
   if (c.group < 0) return;
-  fetch_centre();
-  Chunk next = read();
-  fetch_centre();
-  Chunk ahead = read();
-  fetch_centre();
+  walk.fetch();
+  Chunk next = walk.read();
+  walk.fetch();
+  Chunk ahead = walk.read();
+  walk.fetch();
   fetch(c, point_of(c));
   int ids = point_of(next);
   park(c);
@@ -758,10 +709,10 @@ __global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
     // What has been fetched is waited for before anything is written: a wait behind the stores
     // and atomics would be one for them as well.
     if (next.group >= 0) park(next);
-    asm volatile("" : "+v"(ids), "+v"(after.centre), "+v"(after.begin), "+v"(after.count),
-                 "+v"(after.flags));
-    const Chunk third = read();
-    fetch_centre();
+    asm volatile("" : "+v"(ids), "+v"(walk.after.centre), "+v"(walk.after.begin),
+                 "+v"(walk.after.count), "+v"(walk.after.flags));
+    const Chunk third = walk.read();
+    walk.fetch();
     store(c, sum);
     if (c.last) send(c);
     if (next.group < 0) break;

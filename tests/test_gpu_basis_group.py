@@ -112,3 +112,46 @@ def test_gradients_of_more_groups_than_blocks(c, k, longest, window):
         df_mag.index_add_(0, i, terms.abs().sum(2))
     terms = k * torch.bincount(ids, minlength=points)[:, None]
     assert torch.all((dfeat - df).abs() <= (terms + 1) * 2.0 ** -24 * df_mag)
+
+
+@pytest.mark.parametrize("order", ["index", "random"])
+def test_groups_without_pairs_between_others(order):
+    """Orders of the caller's own, by which a block that forms both gradients comes to one, two and three
+    groups without pairs in a row between two others (the order of the table's own has them last)."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    host = _lib.host()
+    c, k, group, window = 128, 32, 8, 60
+    gen = torch.Generator().manual_seed(3)
+    rand = lambda high, n: torch.randint(high, (n,), generator=gen)
+    blocks = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
+    rounds = 9
+    centres = rounds * blocks * group - 5
+    slot = torch.arange(centres) // group                    # group of the centre by its place in the order
+    empty = torch.tensor([[0, 0, 0, 0, 0, 0, 0, 0, 0], [0, 1, 0, 1, 0, 1, 0, 0, 0],
+                          [0, 1, 1, 0, 1, 1, 0, 0, 1], [1, 0, 1, 1, 1, 0, 1, 0, 0]], dtype=torch.bool)
+    lengths = torch.where(empty[slot % blocks % 4, slot // blocks], 0, rand(131, centres))
+    mean = int(lengths.sum()) / centres
+    assert int(350 / mean) == group                          # what the library makes of these sizes
+    by_order = torch.arange(centres) if order == "index" else torch.randperm(centres, generator=gen)
+    lengths = torch.empty_like(lengths).scatter_(0, by_order, lengths)
+    owner = torch.repeat_interleave(torch.arange(centres), lengths)
+    place = torch.empty_like(by_order).scatter_(0, by_order, torch.arange(centres))
+    ids = (place[owner] + rand(window, len(owner))) % centres      # (centres of a group share points)
+    pairs = torch.stack([ids, owner], 1).int().cuda()
+    ranges = torch.cumsum(lengths, 0).int().cuda()
+    ids, owner = ids.cuda(), owner.cuda()
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    basis, feat, up = (torch.randn(*s, device="cuda", generator=gen)
+                       for s in ((len(ids), k), (centres, c), (centres, c, k)))
+    dbasis, dfeat = host.basis_proj_grads_grouped(basis, feat, pairs, ranges, up, by_order.int().cuda())
+    df, df_mag = (torch.zeros(centres, c, device="cuda", dtype=torch.float64) for _ in range(2))
+    for part in torch.arange(len(ids), device="cuda").split(16384):
+        g, b, i = up[owner[part]].double(), basis[part].double(), ids[part]
+        terms = g * feat[i].double()[:, :, None]
+        assert torch.all((dbasis[part] - terms.sum(1)).abs() <=
+                         (c + 1) * 2.0 ** -24 * terms.abs().sum(1))
+        terms = g * b[:, None, :]
+        df.index_add_(0, i, terms.sum(2))
+        df_mag.index_add_(0, i, terms.abs().sum(2))
+    terms = k * torch.bincount(ids, minlength=centres)[:, None]
+    assert torch.all((dfeat - df).abs() <= (terms + 1) * 2.0 ** -24 * df_mag)

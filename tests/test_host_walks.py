@@ -1,0 +1,25 @@
+"""Index arithmetic of the kernels, compiled for the CPU from their headers."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "tensorflow_graphics_point_clouds_amd", "csrc")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("walks") / "host_walks")
+    subprocess.run([HIPCC, "-x", "hip", "--offload-arch=gfx950", "-O1", "-std=c++17", "-Xclang",
+                    "-target-feature", "-Xclang", "-packed-fp32-ops", "-I", CSRC,
+                    os.path.join(HERE, "host_walks.cpp"), "-o", path], check=True,
+                   capture_output=True, text=True)
+    return path
+
+
+@pytest.mark.parametrize("walk", ["groups"])
+def test_walk(program, walk):
+    run = subprocess.run([program, walk], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0 and run.stdout == "ok\n", run.stderr
