@@ -37,15 +37,15 @@ struct KeyRange {
 // of each end's own took 30 (763 k centres x 37 pairs 82 -> 79 us; the searches inside the visits
 // of a three-level network of 16 x 1024 points 122 -> 108).
 template <int kN>
-__device__ __forceinline__ void find_slices(const KeyRange *range, const int64_t *__restrict__ keys,
-                                            int2 *slice) {
+__host__ __device__ __forceinline__ void find_slices(const KeyRange *range,
+                                                     const int64_t *__restrict__ keys, int2 *slice) {
   int at[2 * kN], step[kN];
   int open = 0;
 #pragma unroll
   for (int i = 0; i < kN; ++i) {
     const int length = range[i].span.y - range[i].span.x;
     const bool search = range[i].mink <= range[i].maxk;
-    step[i] = search && length > 0 ? 1 << (31 - __clz(length)) : 0;
+    step[i] = search && length > 0 ? 1 << (31 - __builtin_clz(length)) : 0;
     at[2 * i] = range[i].span.x;
     at[2 * i + 1] = search ? range[i].span.x : range[i].span.y;
     open |= step[i];
@@ -56,9 +56,9 @@ __device__ __forceinline__ void find_slices(const KeyRange *range, const int64_t
     bool live[2 * kN];
 #pragma unroll
     for (int k = 0; k < 2 * kN; ++k) {       // (a step past the end reads a key it ignores)
-      const int to = at[k] + step[k / 2];
-      live[k] = to <= range[k / 2].span.y && step[k / 2] > 0;
-      key[k] = keys[live[k] ? to - 1 : 0];
+      // (not the sum against the end: it may pass 2^31 - 1)
+      live[k] = step[k / 2] <= range[k / 2].span.y - at[k] && step[k / 2] > 0;
+      key[k] = keys[live[k] ? at[k] + step[k / 2] - 1 : 0];
     }
 #pragma unroll
     for (int k = 0; k < 2 * kN; ++k) {

@@ -2,12 +2,14 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <random>
 #include <vector>
 
 #include "group_walk.h"
+#include "search.h"
 
 using namespace mccnn;
 
@@ -96,8 +98,47 @@ static void test_groups() {
   }
 }
 
+// Slices of descending keys against the definition: of short tables for all pairs of bounds and spans,
+// and of 2^31 - 1 keys, whose last positions a step must not run past.
+static void test_slices() {
+  auto expect = [](int x, int y, int64_t maxk, int64_t mink, const int64_t *keys, int first, int last) {
+    KeyRange range{make_int2(x, y), maxk, mink};
+    int2 got;
+    find_slices<1>(&range, keys, &got);
+    EXPECT(last > first ? got.x == first && got.y == last : got.x == 0 && got.y == 0,
+           "keys %ld .. %ld of [%d, %d): [%d, %d), not [%d, %d)", (long)maxk, (long)mink, x, y, got.x,
+           got.y, first, last);
+  };
+  const int64_t keys[] = {9, 9, 7, 7, 7, 6, 4, 3, 3, 1, 0};
+  for (int x = 0; x <= 11; ++x)
+    for (int y = x; y <= 11; ++y)
+      for (int64_t mink = -1; mink <= 10; ++mink)
+        for (int64_t maxk = mink; maxk <= 10; ++maxk) {
+          int first = x, last = x;
+          while (first < y && keys[first] > maxk) ++first;
+          while (last < y && keys[last] >= mink) ++last;
+          expect(x, y, maxk, mink, keys, first, last);
+        }
+  const int64_t n = ((int64_t)1 << 31) - 1;      // (pages that nothing is written to take no memory)
+  int64_t *many = (int64_t *)mmap(nullptr, n * sizeof(int64_t), PROT_READ | PROT_WRITE,
+                                  MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  EXPECT(many != MAP_FAILED, "no address space for 2^31 keys");
+  for (int i = 0; i < 50; ++i) many[i] = 2, many[n - 1 - i] = -2;
+  for (int begin : {0, 7, 50, 100, 1 << 30, (1 << 30) + 1, (int)n - 60, (int)n - 20})
+    for (int end : {(int)n, (int)n - 1, (int)n - 3, (int)n - 9}) {
+      const int zeros = begin < 50 ? 50 : begin, low = (int)n - 50;
+      expect(begin, end, 0, 0, many, zeros, low);
+      expect(begin, end, -1, -2, many, low > begin ? low : begin, end);
+      expect(begin, end, 2, -2, many, begin, end);
+      expect(begin, end, 2, 1, many, begin, zeros);
+      expect(begin, end, -3, -4, many, end, end);
+    }
+  munmap(many, n * sizeof(int64_t));
+}
+
 int main(int argc, char **argv) {
   if (argc == 2 && !strcmp(argv[1], "groups")) test_groups();
+  else if (argc == 2 && !strcmp(argv[1], "slices")) test_slices();
   else return 2;
   printf("ok\n");
   return 0;

@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return path
 
 
-@pytest.mark.parametrize("walk", ["groups"])
+@pytest.mark.parametrize("walk", ["groups", "slices"])
 def test_walk(program, walk):
     run = subprocess.run([program, walk], capture_output=True, text=True, timeout=120)
     assert run.returncode == 0 and run.stdout == "ok\n", run.stderr
