@@ -223,7 +223,9 @@ struct Bounds {
 // 8000 points in 5 shuffled clouds 52 us, 91 with four clouds taken together first, in strips of 23 points 64
 // and 77) or to as many clouds as there are lanes (from the fourth on: 600 points in 300 clouds 40 and
 // 54 us, 30 k in 64 113 and 117); fewer addresses in memory are worth sparing (100 k points in 5
-// shuffled clouds 1460 and 733).
+// shuffled clouds 1460 and 733).  How long a stretch is hardly matters there: the boxes of 763 k points in
+// 8 shuffled clouds take 5.67 ms with 256 blocks and 5.70 with 745, those of 300 k points in 20 000
+// clouds one after another 77 and 89 us.
 template <int D, class Flush, class Direct>
 __device__ __forceinline__ void add_points(bool live, int b, const float *p, int together,
                                            Bounds<D> &box, int &cur, Flush &&flush,
@@ -651,12 +653,15 @@ static int reduce_boxes(hipStream_t s, int64_t n, int num_dims, const float *poi
   hipLaunchKernelGGL(aabb_init_kernel, dim3(blocks_for(count, 256)), dim3(256), 0, s, count, mn, mx);
   MCCNN_LAUNCH_CHECK();
   if (n == 0) return MCCNN_OK;
-  // stretches of at least 1024 points, at most 1024 blocks
-  // Stretches of at least 1024 points, at most 256 blocks: every block ends in a few minima and
+  // Stretches of at least 1024 points, at most 256 or 512 blocks.  Every block ends in a few minima and
   // maxima of the same words of memory, one after the other, which were most of the time of 745
-  // blocks (763 k points in 8 clouds 11.9 -> 8.2 us, 800 k in 4 13.7 -> 8.4, 98 k in one 4.6 -> 3.7,
-  // 3 M 17.3 -> 14.2; 128 blocks: 10.6, 10.2, 4.0 and 22.6).
-  int64_t per_block = (n + 255) / 256;
+  // blocks; the words of many clouds are others, and long stretches are better read by more blocks.
+  // us at 256 / 512 / 1024 blocks, 1, 8, 16 and 64 clouds: 763 k points 7.6 / 10.6 / 11.4,
+  // 7.5 / 8.5 / 9.7, 7.3 / 7.0 / 8.1, 7.0 / 6.4 / 6.4; 3 M 14.8 / 13.6 / 17.9, 14.1 / 12.2 / 15.2,
+  // 14.1 / 11.6 / 13.3, 14.0 / 10.4 / 10.3; 8 M 30 / 22 / 21 to 28; 300 k 6 to 7 all.  (64 points in
+  // flight and up to 1024 blocks: 763 k 12.7, 10.7, 9.3, 6.8; 3 M 19.9, 17.2, 15.2, 11.9.)
+  const int64_t most = batch >= 16 || n >= (int64_t)1 << 21 ? 512 : 256;
+  int64_t per_block = (n + most - 1) / most;
   per_block = (per_block < 1024 ? 1024 : per_block + 255) / 256 * 256;
   MCCNN_DIM_SWITCH(num_dims,
                    hipLaunchKernelGGL(aabb_reduce_kernel<D>, dim3(blocks_for(n, (int)per_block)),

@@ -94,6 +94,25 @@ def test_boxes_of_clouds_in_strips(oracle, n, strip, batch):
                 oracle.Grid(pts, bids, batch, np.float32(0.1)))
 
 
+@pytest.mark.parametrize("n,batch", [(262145, 1), (600001, 15), (600001, 16), (524289, 70),
+                                     ((1 << 21) - 1, 3), (1 << 21, 3)])
+@pytest.mark.parametrize("even", [True, False])
+def test_boxes_of_long_stretches(n, batch, even):
+    """More points than blocks of the shortest stretches take, with 256 and 512 blocks; clouds of one size,
+    and one large cloud with clouds of ten points behind it, of which a stretch meets more than a block
+    keeps bounds of."""
+    from tensorflow_graphics_point_clouds_amd import pc
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    pts = torch.rand((n, 3), device="cuda", generator=gen) - 0.5
+    index = torch.arange(n, device="cuda")
+    bids = (index * batch // n if even else (index - (n - 10 * batch)).clamp(min=0) // 10).int()
+    grid = pc.Grid(pc.PointCloud(pts, bids, batch), 0.5)
+    bids = bids.long()[:, None].expand(-1, 3)
+    low, high = (torch.zeros(batch, 3, device="cuda").scatter_reduce(0, bids, pts, how, include_self=False)
+                 for how in ("amin", "amax"))
+    assert torch.equal(grid._aabb_min, low - 1e-9) and torch.equal(grid._aabb_max, high + 1e-9)
+
+
 @pytest.mark.parametrize("d", [2, 3, 4])
 @pytest.mark.parametrize("n,n_out,max_neighbors", [(700, 700, 0), (16384, 300, 0), (300, 16385, 0),
                                                    (16385, 16384, 0), (5000, 4000, 3)])
