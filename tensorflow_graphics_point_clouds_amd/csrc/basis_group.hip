@@ -20,9 +20,10 @@
 // centres of 52 pairs, against 4.3 in the order of the grid's cells).
 //
 // Measured (both gradients, order of the centres included), one atomic per pair and channel ->
-// grouped: 800 k points x 52 pairs, 128 channels x 32: 22.8 -> 16.4 ms (dbasis 6.0, dfeat 9.9);
-// shapes without a matrix-core kernel in basis_proj.hip: 200 k x 30, 128 x 64: 66 -> 5.2 ms;
-// 400 k x 30, 96 x 16: 19.1 -> 3.8 ms; 100 k x 20, 24 x 8 and 3 x 32: 1.16 -> 0.34, 1.81 -> 0.36 ms.
+// grouped: 800 k points x 52 pairs, 128 channels x 32: 22.8 -> 13.3 ms by one kernel for both (15.1 by
+// one for either, dbasis 5.3 and dfeat 9.4); shapes without a matrix-core kernel in
+// basis_proj.hip: 200 k x 30, 128 x 64: 66 -> 5.2 ms; 400 k x 30, 96 x 16: 19.1 -> 3.8 ms; 100 k x
+// 20, 24 x 8 and 3 x 32: 1.16 -> 0.34, 1.81 -> 0.36 ms.
 #include <type_traits>
 
 #include "common.h"
@@ -430,7 +431,9 @@ __global__ void __launch_bounds__(64 * W, 2) feature_grads_group_kernel(
         for (int u = 0; u < tiles; ++u)
           acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(gk[q], w[u][q], acc[u], 0, 0, 0);
     };
-    // (tiles of 16 without pairs are left out: 15.1 -> 14.8 ms where half of the centres have 49 or more)
+    // (tiles of 16 without pairs are left out: both gradients of 200 k centres x 36 pairs, 96 x 32 2.52 ->
+    // 2.44 ms, 128 x 16 2.10 -> 2.07, 64 x 32 1.60 -> 1.57; 300 k x 50 4.73 -> 4.68, 4.43 -> 4.35, 2.99 ->
+    // 2.97; clustered clouds and shorter lists the same as before)
     if (kTiles == 4 && c.left > 48) multiply(std::integral_constant<int, kTiles>{});
     else if (kTiles == 4 && c.left > 32) multiply(std::integral_constant<int, kTiles < 4 ? 2 : 3>{});
     else if (c.left > 16) multiply(std::integral_constant<int, 2>{});
@@ -513,7 +516,8 @@ static_assert(sizeof(BothLds) <= 160 * 1024, "one block per compute unit");
 // cores 5.3), parking the operands between two barriers 4, and what of the fetch they do
 // not cover.  Sixteen wavefronts: 13.0 ms; feature rows from memory straight into the operands and
 // two buffers for the rest 13.5; both with 16 basis columns or 64 channels: up to 18 % slower
-// than the two kernels, whose upstream gradient is half as large there.
+// than the two kernels, whose upstream gradient is half as large there.  Other shapes have not been
+// tried.
 __global__ void __launch_bounds__(kBothThreads, 2) both_grads_group_kernel(
     int64_t n_out, int last_pair, int group, int groups, const float *__restrict__ feat,
     const float *__restrict__ basis, const int2 *__restrict__ nbrs,
@@ -819,8 +823,12 @@ extern "C" int mccnn_neighbourhood_order(mccnn_stream_t stream, int64_t num_samp
 //   16 x 8: 13 653 of 7 76 / 119, 109 226 of 7 433 / 186; 3 x 64: 174 762 of 21 3705 / 791.
 // * the others: from 2^27 on, and where the atomics are most of the time (many channels or
 //   columns) and a group of centres shares its points and fits the table: 16 to 80 pairs per
-//   centre (128 x 32: 7.5 pairs per centre 7.9 against 8.7 ms, 20 pairs 11.1 / 9.4, 52 pairs
-//   22.8 / 16.4, 120 pairs 21.3 / 29.6 ms; 64 x 16 at 30 pairs 2.6 / 2.7 ms).
+//   centre (64 x 16 at 30 pairs 2.6 against 2.7 ms).  128 x 32, centres x pairs of uniform and of
+//   clustered clouds: 66 k x 17 0.73 / 0.79 and 0.92 / 0.82; 130 k x 18 1.46 / 1.50 and 1.90 / 1.55; 200 k x
+//   20 2.43 / 2.20 and 2.99 / 2.30; 100 k x 73 and 47 3.37 / 2.54 and 2.73 / 2.02; 100 k x 88 and 78
+//   4.03 / 3.21 and 4.12 / 4.51; 100 k x 115 and 99 5.11 / 6.42 and 5.09 / 6.82.  (Below 16 pairs the
+//   line is that of the kernels that form one gradient each, 800 k x 8 7.8 / 8.3; both at once are
+//   the faster ones from some 2 M pairs on, 7.8 / 7.5, 400 k x 12 4.16 / 3.85 and 4.50 / 4.04.)
 extern "C" int mccnn_basis_proj_grads_grouped_pays(int num_features, int num_basis,
                                                    int64_t num_samples, int64_t num_neighbors) {
   if (group_slices(num_features, num_basis) == 0 || num_samples <= 0 || num_neighbors > kMostPairs)
@@ -843,6 +851,17 @@ extern "C" int mccnn_basis_proj_grads_grouped_pays(int num_features, int num_bas
 // 440 / 340 / 240 pairs; both gradients at once (192 rows) 13.8 / 13.3 / 13.2 ms at 460 / 400 / 350,
 // clustered clouds of 200 k x 37 3.29 / 3.30 / 3.13.
 constexpr double kGroupPairs = 400.0, kBothPairs = 350.0;
+
+// Where both gradients are formed at once.  A block per compute unit walks its share of the groups, and
+// with few of them uneven ones do not even out: time of the two kernels over that of the one at
+// 1.1 .. 2.2 M pairs of 17 to 57 per centre 0.98 to 1.05 in uniform clouds but 0.94 to 1.00 in
+// clustered ones, 2.5 .. 3.2 M 1.02 to 1.04 and 0.97 to 1.01, from 3.9 M on 1.03 to 1.13 and 1.00 to
+// 1.07.  (Clustered clouds of more than 64 pairs per centre: 0.95 to 1.03, uniform ones 1.07 to 1.10.)
+constexpr int64_t kBothLeast = (int64_t)9 << 18;
+static bool both_at_once(int C, int K, int64_t pairs) {
+  return C == kBothC && K == kBothK && pairs >= kBothLeast;
+}
+
 static int group_centres(int64_t num_samples, int64_t num_neighbors, double pairs) {
   const double mean = (double)num_neighbors / (double)(num_samples > 0 ? num_samples : 1);
   const int group = (int)(pairs / (mean > 1.0 ? mean : 1.0));
@@ -852,11 +871,14 @@ static int group_centres(int64_t num_samples, int64_t num_neighbors, double pair
 extern "C" size_t mccnn_basis_proj_grads_grouped_workspace_bytes(int64_t num_samples,
                                                                  int64_t num_neighbors) {
   if (num_samples <= 0 || num_neighbors <= 0) return 0;
-  const int64_t groups = blocks_for(num_samples, group_centres(num_samples, num_neighbors, kBothPairs));
+  // one size for all shapes: groups as small as any, centres listed where one may have them listed
+  const bool both = both_at_once(kBothC, kBothK, num_neighbors);
+  const int64_t groups = blocks_for(num_samples, group_centres(num_samples, num_neighbors,
+                                                               both ? kBothPairs : kGroupPairs));
   return align256(sizeof(unsigned short) * (size_t)num_neighbors) +
          align256(sizeof(int) * kMaxRows * (size_t)groups) +
          align256(sizeof(GroupInfo) * (size_t)groups) +
-         align256(sizeof(GroupCentre) * (size_t)num_samples);
+         (both ? align256(sizeof(GroupCentre) * (size_t)num_samples) : 0);
 }
 
 extern "C" int mccnn_basis_proj_grads_grouped(
@@ -885,7 +907,7 @@ extern "C" int mccnn_basis_proj_grads_grouped(
   MCCNN_REQUIRE(workspace && workspace_bytes >= mccnn_basis_proj_grads_grouped_workspace_bytes(
                                                      num_samples, num_neighbors),
                 "BasisProjGrads (grouped) workspace too small");
-  const bool both = num_features == kBothC && num_basis == kBothK;
+  const bool both = both_at_once(num_features, num_basis, num_neighbors);
   const int group = group_centres(num_samples, num_neighbors, both ? kBothPairs : kGroupPairs);
   const int64_t groups = blocks_for(num_samples, group);
   unsigned short *row_of = (unsigned short *)workspace;

@@ -114,6 +114,22 @@ def test_gradients_of_more_groups_than_blocks(c, k, longest, window):
     assert torch.all((dfeat - df).abs() <= (terms + 1) * 2.0 ** -24 * df_mag)
 
 
+def _check(dbasis, dfeat, basis, feat, ids, owner, up):
+    """Against the sums in 64 bits; the bounds are those of test_grouped_gradients."""
+    c, k = up.shape[1:]
+    df, df_mag = (torch.zeros(feat.shape, device="cuda", dtype=torch.float64) for _ in range(2))
+    for part in torch.arange(len(ids), device="cuda").split(16384):
+        g, b, i = up[owner[part]].double(), basis[part].double(), ids[part]
+        terms = g * feat[i].double()[:, :, None]
+        assert torch.all((dbasis[part] - terms.sum(1)).abs() <=
+                         (c + 1) * 2.0 ** -24 * terms.abs().sum(1))
+        terms = g * b[:, None, :]
+        df.index_add_(0, i, terms.sum(2))
+        df_mag.index_add_(0, i, terms.abs().sum(2))
+    terms = k * torch.bincount(ids, minlength=len(feat))[:, None]
+    assert torch.all((dfeat - df).abs() <= (terms + 1) * 2.0 ** -24 * df_mag)
+
+
 @pytest.mark.parametrize("order", ["index", "random"])
 def test_groups_without_pairs_between_others(order):
     """Orders of the caller's own, by which a block that forms both gradients comes to one, two and three
@@ -124,14 +140,14 @@ def test_groups_without_pairs_between_others(order):
     gen = torch.Generator().manual_seed(3)
     rand = lambda high, n: torch.randint(high, (n,), generator=gen)
     blocks = torch.cuda.get_device_properties(0).multi_processor_count // 8 * 8
-    rounds = 9
+    rounds = (30 * 256 + blocks - 1) // blocks
     centres = rounds * blocks * group - 5
     slot = torch.arange(centres) // group                    # group of the centre by its place in the order
     empty = torch.tensor([[0, 0, 0, 0, 0, 0, 0, 0, 0], [0, 1, 0, 1, 0, 1, 0, 0, 0],
                           [0, 1, 1, 0, 1, 1, 0, 0, 1], [1, 0, 1, 1, 1, 0, 1, 0, 0]], dtype=torch.bool)
-    lengths = torch.where(empty[slot % blocks % 4, slot // blocks], 0, rand(131, centres))
-    mean = int(lengths.sum()) / centres
-    assert int(350 / mean) == group                          # what the library makes of these sizes
+    lengths = torch.where(empty[slot % blocks % 4, slot // blocks % 9], 0, rand(131, centres))
+    # what the library makes of these sizes
+    assert lengths.sum() >= 9 << 18 and int(350 / (int(lengths.sum()) / centres)) == group
     by_order = torch.arange(centres) if order == "index" else torch.randperm(centres, generator=gen)
     lengths = torch.empty_like(lengths).scatter_(0, by_order, lengths)
     owner = torch.repeat_interleave(torch.arange(centres), lengths)
@@ -139,19 +155,35 @@ def test_groups_without_pairs_between_others(order):
     ids = (place[owner] + rand(window, len(owner))) % centres      # (centres of a group share points)
     pairs = torch.stack([ids, owner], 1).int().cuda()
     ranges = torch.cumsum(lengths, 0).int().cuda()
-    ids, owner = ids.cuda(), owner.cuda()
     gen = torch.Generator(device="cuda").manual_seed(4)
     basis, feat, up = (torch.randn(*s, device="cuda", generator=gen)
                        for s in ((len(ids), k), (centres, c), (centres, c, k)))
     dbasis, dfeat = host.basis_proj_grads_grouped(basis, feat, pairs, ranges, up, by_order.int().cuda())
-    df, df_mag = (torch.zeros(centres, c, device="cuda", dtype=torch.float64) for _ in range(2))
-    for part in torch.arange(len(ids), device="cuda").split(16384):
-        g, b, i = up[owner[part]].double(), basis[part].double(), ids[part]
-        terms = g * feat[i].double()[:, :, None]
-        assert torch.all((dbasis[part] - terms.sum(1)).abs() <=
-                         (c + 1) * 2.0 ** -24 * terms.abs().sum(1))
-        terms = g * b[:, None, :]
-        df.index_add_(0, i, terms.sum(2))
-        df_mag.index_add_(0, i, terms.abs().sum(2))
-    terms = k * torch.bincount(ids, minlength=centres)[:, None]
-    assert torch.all((dfeat - df).abs() <= (terms + 1) * 2.0 ** -24 * df_mag)
+    _check(dbasis, dfeat, basis, feat, ids.cuda(), owner.cuda(), up)
+
+
+@pytest.mark.parametrize("rows,spare,longest,window", [
+    ((9 << 18) - 1, 0, 40, 60), (9 << 18, 0, 40, 60), (9 << 18, 70, 66, 80), ((9 << 18) + 1, 1, 130, 2000),
+    ((9 << 18) + 77, 700, 700, 900)])
+def test_tables_on_either_side_of_both_gradients_at_once(rows, spare, longest, window):
+    """Lists of 0, 1, .. `longest` pairs with points listed twice among them, groups that overflow
+    their table, rows behind the last list; and one pair fewer than are worked on by one kernel."""
+    from tensorflow_graphics_point_clouds_amd import _lib
+    host = _lib.host()
+    c, k, used = 128, 32, rows - spare
+    gen = torch.Generator(device="cuda").manual_seed(longest)
+    rand = lambda high, n: torch.randint(high, (n,), device="cuda", generator=gen)
+    lengths = rand(longest + 1, 3 * used // longest)
+    lengths[1000:1400] = 0
+    centres = int((torch.cumsum(lengths, 0) < used).sum()) + 1
+    ranges = torch.cumsum(lengths[:centres], 0).clamp(max=used).int()
+    owner = torch.searchsorted(ranges, torch.arange(used, device="cuda", dtype=torch.int32), right=True)
+    ids = (owner + rand(window, used)) % centres
+    pairs = torch.zeros(rows, 2, dtype=torch.int32, device="cuda")
+    pairs[:used] = torch.stack([ids, owner], 1).int()
+    basis, feat, up = (torch.randn(*s, device="cuda", generator=gen)
+                       for s in ((rows, k), (centres, c), (centres, c, k)))
+    dbasis, dfeat = host.basis_proj_grads_grouped(basis, feat, pairs, ranges, up,
+                                                  host.neighbourhood_order(pairs, ranges))
+    assert not dbasis[used:].any()
+    _check(dbasis, dfeat, basis, feat, ids, owner, up)
