@@ -476,7 +476,8 @@ int mccnn_basis_proj_grads_ordered(
  * fixed, as for mccnn_basis_proj_grads.  Rows of the table behind the last centre's pairs have
  * zero basis gradients.  Supported: up to 128 features and 2^31 - 1024 pairs; basis, in_grads and
  * basis_grads_out aligned to 16 bytes, features too if their number is a multiple of 16.
- * ..._pays: whether it is the faster one for a table of these sizes. */
+ * ..._pays: whether it is the faster one for a table of these sizes; ..._workspace_bytes: enough
+ * for any number of features and basis functions. */
 size_t mccnn_neighbourhood_order_workspace_bytes(int64_t num_samples);
 int mccnn_neighbourhood_order(mccnn_stream_t stream, int64_t num_samples, int64_t num_neighbors,
                               const int32_t *neighbors, const int32_t *ranges, void *workspace,

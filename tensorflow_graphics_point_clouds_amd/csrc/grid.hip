@@ -659,7 +659,8 @@ static int reduce_boxes(hipStream_t s, int64_t n, int num_dims, const float *poi
   // us at 256 / 512 / 1024 blocks, 1, 8, 16 and 64 clouds: 763 k points 7.6 / 10.6 / 11.4,
   // 7.5 / 8.5 / 9.7, 7.3 / 7.0 / 8.1, 7.0 / 6.4 / 6.4; 3 M 14.8 / 13.6 / 17.9, 14.1 / 12.2 / 15.2,
   // 14.1 / 11.6 / 13.3, 14.0 / 10.4 / 10.3; 8 M 30 / 22 / 21 to 28; 300 k 6 to 7 all.  (64 points in
-  // flight and up to 1024 blocks: 763 k 12.7, 10.7, 9.3, 6.8; 3 M 19.9, 17.2, 15.2, 11.9.)
+  // flight and up to 1024 blocks: 763 k 12.7, 10.7, 9.3, 6.8; 3 M 19.9, 17.2, 15.2, 11.9.  All of one
+  // grid after another; 800 k points in 4 clouds between the kernels of a whole pass 9.3, 11.8 before.)
   const int64_t most = batch >= 16 || n >= (int64_t)1 << 21 ? 512 : 256;
   int64_t per_block = (n + most - 1) / most;
   per_block = (per_block < 1024 ? 1024 : per_block + 255) / 256 * 256;

@@ -41,8 +41,9 @@ __device__ __forceinline__ PdfScale<D> load_pdf_scale(const float *__restrict__ 
 // 4 x 200k points, 7.5 / 52 / 170 pairs per point: 0.027 / 0.134 / 0.486 ms with 4 lanes,
 // 0.041 / 0.115 / 0.355 ms with 8, 0.074 / 0.133 / 0.315 ms with 16.  The indices of the next
 // trip are fetched before the coordinates of this one, which takes a link out of the chain of
-// every trip but the first (clustered clouds, 763 k points x 38 pairs 75.6 -> 66.8 us, x 9
-// 29.5 -> 26.7; 400 k x 55 54.5 -> 48.2; 200 k x 20 17.0 -> 15.5).
+// every trip but the first (the kernel over and over on one table, clustered clouds: 763 k points x 38
+// pairs 75.6 -> 66.8 us, x 9 29.5 -> 26.7; 400 k x 55 54.5 -> 48.2; 200 k x 20 17.0 -> 15.5; the
+// first of these behind the search that has written the table 100.9 -> 85.6).
 template <int D, int G>
 __global__ void __launch_bounds__(kPdfThreads) compute_pdf_kernel(
     int64_t n, const float *__restrict__ pts, const int2 *__restrict__ nbrs,
